@@ -166,7 +166,7 @@ int smat_plan_attach_values(smat_plan *plan, const uint16_t *vals, const int32_t
  * called by the SpMM itself.  No counterpart in the reference, which keeps no copy. */
 int smat_plan_values_current(const smat_plan *plan, const uint16_t *vals, int *current);
 int smat_plan_destroy(smat_plan *plan);
-/* Opt-in check that `plan` was made from this block pattern: M, K, nnzb and a 64-bit FNV-1a hash of
+/* Opt-in check that `plan` was made from this block pattern: M, K, nnzb and a 64-bit hash of
  * row_ptr_host (and of col_idx_host if the plan was made with one; then it must be passed).  One pass over
  * the host arrays; SMAT_ERR_INVALID when they differ.  No counterpart in the reference. */
 int smat_plan_check(const smat_plan *plan, const int32_t *row_ptr_host, const int32_t *col_idx_host,

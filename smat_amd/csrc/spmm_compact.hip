@@ -71,9 +71,37 @@ constexpr int LIST_PAD = 640; // entries readable past the end of the list (the 
 
 // ---- census of nonzero block columns ----
 
-__global__ __launch_bounds__(256) void colmask_kernel(const uint16_t *__restrict__ vals, long nnzb,
-                                                      uint16_t *__restrict__ mask, int32_t *__restrict__ count)
+// Order-independent 64-bit checksum of the block values: sum over all dwords of value * (2 * index + 1).  A workgroup
+// adds its part to one of CHECKSUM_SLOTS words, 128 bytes apart: additions to one word queue up at 12 ns each, which
+// for one word and every wavefront of a pass over 121 MB is 200 us of a 25 us pass.
+constexpr int CHECKSUM_SLOTS = 32, CHECKSUM_STRIDE = 16;
+constexpr size_t CHECKSUM_BYTES = CHECKSUM_SLOTS * CHECKSUM_STRIDE * sizeof(unsigned long long);
+__device__ __forceinline__ unsigned long long checksum_term(uint32_t v, long i)
 {
+    return (unsigned long long)v * (2ull * (unsigned long long)i + 1ull);
+}
+__device__ __forceinline__ void add_checksum(unsigned long long sum, unsigned long long *__restrict__ sums)
+{
+    __shared__ unsigned long long part[4];
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(&sums[(blockIdx.x % CHECKSUM_SLOTS) * CHECKSUM_STRIDE], part[0] + part[1] + part[2] + part[3]);
+}
+uint64_t total_checksum(const std::vector<unsigned long long> &sums)
+{
+    uint64_t h = 0;
+    for (int i = 0; i < CHECKSUM_SLOTS; i++) h += sums[(size_t)i * CHECKSUM_STRIDE];
+    return h;
+}
+
+// The checksum of the block values (values_checksum_kernel) is taken on the way.
+__global__ __launch_bounds__(256) void colmask_kernel(const uint16_t *__restrict__ vals, long nnzb,
+                                                      uint16_t *__restrict__ mask, int32_t *__restrict__ count,
+                                                      unsigned long long *__restrict__ sums)
+{
+    unsigned long long sum = 0;
     const int lane = threadIdx.x & 63;
     const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const long n_waves = ((long)gridDim.x * blockDim.x) >> 6;
@@ -82,6 +110,8 @@ __global__ __launch_bounds__(256) void colmask_kernel(const uint16_t *__restrict
         // lane % 32 = row * 2 + half: 8 values of one row
         u32x4 w = {0u, 0u, 0u, 0u};
         if (blk < nnzb) w = *reinterpret_cast<const u32x4 *>(vals + blk * 256 + (lane & 31) * 8);
+#pragma unroll
+        for (int q = 0; q < 4; q++) sum += checksum_term(w[q], blk * 128 + (lane & 31) * 4 + q);
         w &= 0x7fff7fffu; // -0.0 is a zero
 #pragma unroll
         for (int d = 2; d <= 16; d <<= 1) { // OR over the 16 rows (lane bits 1..4)
@@ -103,18 +133,18 @@ __global__ __launch_bounds__(256) void colmask_kernel(const uint16_t *__restrict
             count[blk] = __popc(m);
         }
     }
+    add_checksum(sum, sums);
 }
 
-// Order-independent 64-bit checksum of the block values: sum over all dwords of value * (2 * index + 1).
-__global__ __launch_bounds__(256) void values_checksum_kernel(const uint32_t *__restrict__ vals, long n_dwords,
-                                                              unsigned long long *__restrict__ out)
+__global__ __launch_bounds__(256) void values_checksum_kernel(const u32x4 *__restrict__ vals, long n_quads, unsigned long long *__restrict__ sums)
 {
     unsigned long long sum = 0;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n_dwords; i += (long)gridDim.x * blockDim.x)
-        sum += (unsigned long long)vals[i] * (2ull * (unsigned long long)i + 1ull);
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n_quads; i += (long)gridDim.x * blockDim.x) {
+        const u32x4 v = vals[i];
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
-    if ((threadIdx.x & 63) == 0) atomicAdd(out, sum);
+        for (int q = 0; q < 4; q++) sum += checksum_term(v[q], 4 * i + q);
+    }
+    add_checksum(sum, sums);
 }
 
 // One thread per block: its nonzero columns go to positions padded_start[br] + (offset[p] -
@@ -538,11 +568,7 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
-struct Scratch {
-    void *p = nullptr;
-    ~Scratch() { if (p) (void)dev_free(p); }
-    hipError_t alloc(size_t bytes) { return dev_malloc(&p, bytes ? bytes : 16); }
-};
+using Scratch = DevScratch;
 
 } // namespace
 
@@ -649,20 +675,17 @@ hipError_t values_checksum(const uint16_t *vals, size_t nnzb, uint64_t *out)
 {
     *out = 0;
     if (!nnzb) return hipSuccess;
-    unsigned long long *d = nullptr;
-    hipError_t e = dev_malloc(&d, sizeof(unsigned long long));
+    DevScratch d;
+    hipError_t e = d.alloc(CHECKSUM_BYTES);
+    if (e == hipSuccess) e = hipMemsetAsync(d.p, 0, CHECKSUM_BYTES, nullptr);
     if (e != hipSuccess) return e;
-    e = hipMemset(d, 0, sizeof(unsigned long long));
-    if (e == hipSuccess) {
-        const long n_dwords = (long)nnzb * 128;
-        const unsigned blocks = (unsigned)std::min<long>((n_dwords + 255) / 256, 256L * 16);
-        hipLaunchKernelGGL(values_checksum_kernel, dim3(blocks), dim3(256), 0, 0, reinterpret_cast<const uint32_t *>(vals), n_dwords, d);
-        e = hipGetLastError();
-    }
-    unsigned long long h = 0;
-    if (e == hipSuccess) e = hipMemcpy(&h, d, sizeof h, hipMemcpyDeviceToHost);
-    (void)dev_free(d);
-    *out = h;
+    const long n_quads = (long)nnzb * 32;
+    const unsigned blocks = (unsigned)std::min<long>((n_quads + 255) / 256, 256L * 8);
+    hipLaunchKernelGGL(values_checksum_kernel, dim3(blocks), dim3(256), 0, 0, reinterpret_cast<const u32x4 *>(vals), n_quads, (unsigned long long *)d.p);
+    e = hipGetLastError();
+    std::vector<unsigned long long> sums(CHECKSUM_BYTES / sizeof(unsigned long long));
+    if (e == hipSuccess) e = hipMemcpy(sums.data(), d.p, CHECKSUM_BYTES, hipMemcpyDeviceToHost);
+    if (e == hipSuccess) *out = total_checksum(sums);
     return e;
 }
 
@@ -699,7 +722,7 @@ hipError_t compact_build(const uint16_t *vals, const int32_t *row_ptr, const int
     CompactPlan *p = new (std::nothrow) CompactPlan();
     if (!p) return hipErrorOutOfMemory;
     hipError_t e = hipSuccess;
-    Scratch mask, count, offset, tmp, cc;
+    Scratch mask, count, offset, tmp, cc, sums;
 #define SMAT_STEP(call)                                                                            \
     do {                                                                                           \
         if (e == hipSuccess) e = (call);                                                           \
@@ -708,12 +731,14 @@ hipError_t compact_build(const uint16_t *vals, const int32_t *row_ptr, const int
     SMAT_STEP(count.alloc(nnzb * 4));
     SMAT_STEP(offset.alloc(nnzb * 4));
     SMAT_STEP(cc.alloc((mb + 1) * 4));
+    SMAT_STEP(sums.alloc(CHECKSUM_BYTES));
+    SMAT_STEP(hipMemsetAsync(sums.p, 0, CHECKSUM_BYTES, nullptr));
     int64_t n_cols = 0;
     std::vector<int32_t> raw(mb + 1, 0), padded(mb + 1, 0);
     if (e == hipSuccess && nnzb) {
         const long waves = std::min<long>((long)(nnzb + 1) / 2, 256L * 32);
         hipLaunchKernelGGL(colmask_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, 0, vals, (long)nnzb,
-                           (uint16_t *)mask.p, (int32_t *)count.p);
+                           (uint16_t *)mask.p, (int32_t *)count.p, (unsigned long long *)sums.p);
         e = hipGetLastError();
         if (block_cols) { // nonzero columns of every block, for the caller's choice of a split
             std::vector<int32_t> cnt(nnzb);
@@ -824,7 +849,9 @@ hipError_t compact_build(const uint16_t *vals, const int32_t *row_ptr, const int
         SMAT_STEP(hipMemcpy(p->d_split, split.data(), split.size() * sizeof(SplitRow), hipMemcpyHostToDevice));
         SMAT_STEP(dev_malloc(&p->d_workspace, (size_t)slot * 16 * n_cap * sizeof(float)));
     }
-    SMAT_STEP(values_checksum(vals, nnzb, &p->values_checksum));
+    std::vector<unsigned long long> parts(CHECKSUM_BYTES / sizeof(unsigned long long));
+    SMAT_STEP(hipMemcpy(parts.data(), sums.p, CHECKSUM_BYTES, hipMemcpyDeviceToHost));
+    p->values_checksum = total_checksum(parts);
     SMAT_STEP(hipDeviceSynchronize());
 #undef SMAT_STEP
     if (e != hipSuccess) {
