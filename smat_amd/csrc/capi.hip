@@ -161,7 +161,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
     a.vals = vals; a.row_ptr = row_ptr; a.col_idx = col_idx; a.B = B; a.C = C;
     a.M = M; a.N = N; a.K = K; a.nnzb = nnzb;
     a.c_f32 = o.c_dtype == SMAT_C_F32;
-    a.n_items = (int)(M / 16);
+    a.n_items = a.rule_items = (int)(M / 16);
     if (plan) {
         if (plan->M != M || plan->K != K || plan->nnzb != nnzb)
             return set_error(SMAT_ERR_INVALID, "plan was built for another matrix (M/K/nnzb differ)");
@@ -172,7 +172,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         a.items = plan->d_items; a.n_items = plan->n_items;
         a.split_rows = plan->d_split; a.n_split_rows = plan->n_split_rows;
         a.workspace = plan->d_workspace;
-        a.panel_tiles = plan->panel_tiles;
+        a.rule_items = plan->n_items;
         a.max_item_blocks = plan->max_item_blocks;
         a.deal = &plan->deal;
         if (plan->d_bpack && N <= plan->n_cap && o.kernel != SMAT_KERNEL_ROWWISE_DIRECT) a.b_packed = plan->d_bpack;
@@ -305,7 +305,7 @@ extern "C" int smat_spmm_bcsr_f16_static(const uint16_t *vals, const int32_t *ro
     a.vals = vals; a.row_ptr = row_ptr; a.col_idx = col_idx; a.B = B; a.C = C;
     a.M = M; a.N = N; a.K = K; a.nnzb = nnzb;
     a.c_f32 = false;
-    a.n_items = (int)(M / 16); // whole block rows, one wavefront each: no work list, no partial tiles
+    a.n_items = a.rule_items = (int)(M / 16); // whole block rows: no work list, no partial tiles
     a.b_packed = static_cast<uint16_t *>(ptr); // every element the kernel reads is rewritten by the repack first
     hipError_t e = launch_rowwise(a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return set_error(SMAT_ERR_HIP, "SpMM launch failed: %s", hipGetErrorString(e));
@@ -457,7 +457,7 @@ static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
     p->n_items = (int)items.size();
     rowwise_costs(items, p->deal);
     for (const WorkItem &wi : items) p->max_item_blocks = std::max(p->max_item_blocks, wi.end - wi.begin);
-    p->panel_tiles = rowwise_panel_tiles(n_hint, 0, items.size());
+    p->panel_tiles = rowwise_panel_tiles(n_hint, items.size(), items.empty() ? 0 : nnzb / items.size(), !split.empty());
     p->n_split_rows = (int)split.size();
     p->n_slots = slot;
 

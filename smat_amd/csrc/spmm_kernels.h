@@ -56,7 +56,7 @@ struct SpmmArgs {
     void *C;
     size_t M, N, K, nnzb;
     bool c_f32;
-    int panel_tiles;       // 0 = choose from N; else 1, 2, 4, 8 or 16 n-tiles of 16 per wavefront
+    int rule_items;        // work items of the whole matrix: with nnzb, what the choice of the kernel's shape looks at
     const WorkItem *items; // device; nullptr = one item per block row
     int n_items;
     const SplitRow *split_rows; // device
@@ -140,7 +140,7 @@ hipError_t launch_compact(const CompactArgs &a, hipStream_t st);
 hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t K, bool b_row_major, bool accumulate);
 hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, size_t N, size_t K, hipStream_t st);
 
-int rowwise_panel_tiles(size_t N, int requested, size_t n_items);
+int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, bool split_rows);
 hipError_t launch_sweep(const SweepArgs &a, hipStream_t st);
 hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st);
 

@@ -57,6 +57,51 @@ __device__ __forceinline__ int ncol_of(int t, int i)
     return 16 * TG * (t / TG) + 4 * TG * (i >> 2) + 4 * (t % TG) + (i & 3);
 }
 
+// acc[t][r] = C[br*16 + i16][n0 + ncol_of(t, 4*g + r)], to C or (dst >= 0) to workspace slot dst.
+template <int TN, bool C_F32>
+__device__ __forceinline__ void store_tile(const f32x4 (&acc)[TN], int br, int dst, int n0, int i16, int g, void *__restrict__ Cout,
+                                           float *__restrict__ workspace, int N)
+{
+    constexpr int TG = TN < 4 ? TN : 4;
+    const long m = (long)br * 16 + i16;
+#pragma unroll
+    for (int u = 0; u < TN / TG; u++) {
+        const int nbase = n0 + 16 * TG * u + 4 * TG * g; // first of 4*TG consecutive columns
+        if (dst >= 0) {
+            // fp32 partial tile: slot-major, then the same row-major M x N addressing
+            float *wrow = workspace + ((long)dst * 16 + i16) * (long)N;
+#pragma unroll
+            for (int tt = 0; tt < TG; tt++) {
+                int n = nbase + 4 * tt;
+                if (n < N) *reinterpret_cast<f32x4 *>(wrow + n) = acc[u * TG + tt];
+            }
+        } else if (C_F32) {
+            float *crow = reinterpret_cast<float *>(Cout) + m * (long)N;
+#pragma unroll
+            for (int tt = 0; tt < TG; tt++) {
+                int n = nbase + 4 * tt;
+                if (n < N) *reinterpret_cast<f32x4 *>(crow + n) = acc[u * TG + tt];
+            }
+        } else {
+            uint16_t *crow = reinterpret_cast<uint16_t *>(Cout) + m * (long)N;
+            if constexpr (TG == 1) {
+                f32x4 v = acc[u];
+                f16x4 h = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+                if (nbase < N) *reinterpret_cast<f16x4 *>(crow + nbase) = h;
+            } else {
+#pragma unroll
+                for (int tt = 0; tt < TG; tt += 2) {
+                    f32x4 v0 = acc[u * TG + tt], v1 = acc[u * TG + tt + 1];
+                    f16x8 h = {(_Float16)v0[0], (_Float16)v0[1], (_Float16)v0[2], (_Float16)v0[3],
+                               (_Float16)v1[0], (_Float16)v1[1], (_Float16)v1[2], (_Float16)v1[3]};
+                    int n = nbase + 4 * tt;
+                    if (n < N) *reinterpret_cast<f16x8 *>(crow + n) = h;
+                }
+            }
+        }
+    }
+}
+
 // One wavefront per work item x N panel.  blockDim = 256 (4 wavefronts).
 //   items == nullptr : item w is the whole block row w (no work list)
 //   items != nullptr : items[w] = {block row, first block, end block, dst}
@@ -83,7 +128,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
     float *__restrict__ workspace, const WorkItem *__restrict__ items, int n_items, int N, long K,
     int n_panels, unsigned xcd_run)
 {
-    constexpr int TG = TN < 4 ? TN : 4;
     constexpr int PANEL = 16 * TN;
     const int lane = threadIdx.x & 63;
     // wavefront-uniform values are forced into scalar registers
@@ -179,44 +223,109 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
         if (j < npair) multiply(j, a0, b0); // odd number of pairs: the last one is already in set 0
     }
 
-    // Epilogue.  acc[t][r] = C[br*16 + i16][n0 + ncol_of(t, 4*g + r)].
-    const long m = (long)br * 16 + i16;
+    store_tile<TN, C_F32>(acc, br, dst, n0, i16, g, Cout, workspace, N);
+}
+
+// Launches of few (item, panel) pairs with long items: the four wavefronts of a workgroup share one, each takes a run of
+// the item's block pairs with the operands of NP pairs in flight, and the partial tiles are added in LDS in the order of
+// the runs.  Bound by the chain item -> column indices -> operands of a wavefront and by too few of them: 8192^2 with 10 %
+// of the blocks and N = 16 (512 items) takes 6.3 us where one wavefront per item takes 9.1; 1024 x 8192 with 30 % and
+// N = 64 (64 items of 154 blocks) 13.8 against 39.8.  Eight wavefronts per item are no faster than four.
+template <int TN, bool C_F32, bool PACKED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void spmm_rowwise_split_kernel(
+    const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_idx,
+    const uint16_t *__restrict__ B, void *__restrict__ Cout, float *__restrict__ workspace, const WorkItem *__restrict__ items,
+    int n_items, int N, long K, int n_panels)
+{
+    constexpr int SPLIT = 4, PANEL = 16 * TN;
+    constexpr int NP = TN <= 2 ? 4 : 3;
+    __shared__ f32x4 part[SPLIT][TN][64];
+    const int lane = threadIdx.x & 63;
+    const int run = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // an XCD takes an eighth of the panel-major (panel, item) space: few panels of B in its L2
+    const long total = (long)n_items * n_panels, per_xcd = (total + 7) / 8;
+    const long w = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= per_xcd || w >= total) return; // the whole workgroup
+    const int panel = (int)(w / n_items);
+    const int it = (int)(w - (long)panel * n_items);
+    int br, p0, p1, dst;
+    if (items) {
+        const WorkItem wi = items[it];
+        br = wi.block_row; p0 = wi.begin; p1 = wi.end; dst = wi.dst;
+    } else {
+        br = it; p0 = row_ptr[it]; p1 = row_ptr[it + 1]; dst = -1;
+    }
+    br = __builtin_amdgcn_readfirstlane(br);
+    p0 = __builtin_amdgcn_readfirstlane(p0);
+    p1 = __builtin_amdgcn_readfirstlane(p1);
+    dst = __builtin_amdgcn_readfirstlane(dst);
+
+    const int i16 = lane & 15, g = lane >> 4, sel = g >> 1, kh = g & 1;
+    const int n0 = panel * PANEL;
+    f32x4 acc[TN];
 #pragma unroll
-    for (int u = 0; u < TN / TG; u++) {
-        const int nbase = n0 + 16 * TG * u + 4 * TG * g; // first of 4*TG consecutive columns
-        if (dst >= 0) {
-            // fp32 partial tile: slot-major, then the same row-major M x N addressing
-            float *wrow = workspace + ((long)dst * 16 + i16) * (long)N;
+    for (int t = 0; t < TN; t++) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int npair = (p1 - p0 + 1) >> 1, per = (npair + SPLIT - 1) / SPLIT;
+    const int j0 = run * per, j1 = j0 + per < npair ? j0 + per : npair;
+    if (j0 < j1) { // uniform over the wavefront
+        long boff[TN];
 #pragma unroll
-            for (int tt = 0; tt < TG; tt++) {
-                int n = nbase + 4 * tt;
-                if (n < N) *reinterpret_cast<f32x4 *>(wrow + n) = acc[u * TG + tt];
-            }
-        } else if (C_F32) {
-            float *crow = reinterpret_cast<float *>(Cout) + m * (long)N;
+        for (int t = 0; t < TN; t++) {
+            const int n = n0 + ncol_of<TN>(t, i16);
+            boff[t] = PACKED ? (long)(n < N ? n : 0) * 16 + kh * 8 : (long)(n < N ? n : 0) * K + kh * 8; // past N: column 0, never stored
+        }
+        const uint16_t *abase = vals + i16 * 16 + kh * 8;
+        const f16x8 zero8 = zero_f16x8();
+        for (int jw = j0; jw < j1; jw += 32) { // a window of 64 column indices
+            const int first = p0 + 2 * jw, last = p1 - 1;
+            const int myc = col_idx[first + lane < last ? first + lane : last];
+            const int jend = jw + 32 < j1 ? jw + 32 : j1;
+            auto blocks = [&](int j, int &q0, int &q1) {
+                const int jj = j < jend ? j : jend - 1; // past the end: the last pair again, multiplied by zeros
+                q0 = p0 + 2 * jj;
+                q1 = q0 < last ? q0 + 1 : q0; // a single block pairs with itself
+            };
+            auto multiply = [&](int j, f16x8 a, const f16x8 (&b)[TN]) {
+                if (j >= jend) a = zero8;
+                else if (p0 + 2 * j >= last) a = sel ? zero8 : a; // single block: the upper K half contributes nothing
 #pragma unroll
-            for (int tt = 0; tt < TG; tt++) {
-                int n = nbase + 4 * tt;
-                if (n < N) *reinterpret_cast<f32x4 *>(crow + n) = acc[u * TG + tt];
-            }
-        } else {
-            uint16_t *crow = reinterpret_cast<uint16_t *>(Cout) + m * (long)N;
-            if constexpr (TG == 1) {
-                f32x4 v = acc[u];
-                f16x4 h = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-                if (nbase < N) *reinterpret_cast<f16x4 *>(crow + nbase) = h;
-            } else {
+                for (int t = 0; t < TN; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[t], a, acc[t], 0, 0, 0);
+            };
+            for (int j = jw; j < jend; j += NP) { // the operands of NP pairs at once; a run is seldom more than one batch
+                f16x8 a[NP], b[NP][TN];
 #pragma unroll
-                for (int tt = 0; tt < TG; tt += 2) {
-                    f32x4 v0 = acc[u * TG + tt], v1 = acc[u * TG + tt + 1];
-                    f16x8 h = {(_Float16)v0[0], (_Float16)v0[1], (_Float16)v0[2], (_Float16)v0[3],
-                               (_Float16)v1[0], (_Float16)v1[1], (_Float16)v1[2], (_Float16)v1[3]};
-                    int n = nbase + 4 * tt;
-                    if (n < N) *reinterpret_cast<f16x8 *>(crow + n) = h;
+                for (int u = 0; u < NP; u++) { // the values first: they do not wait for the column indices
+                    int q0, q1;
+                    blocks(j + u, q0, q1);
+                    a[u] = load_f16x8(abase + (long)(sel ? q1 : q0) * 256);
                 }
+                SMAT_ORDER_FENCE();
+#pragma unroll
+                for (int u = 0; u < NP; u++) {
+                    int q0, q1;
+                    blocks(j + u, q0, q1);
+                    const int c0 = __builtin_amdgcn_readlane(myc, q0 - first), c1 = __builtin_amdgcn_readlane(myc, q1 - first);
+                    const int bc = sel ? c1 : c0;
+                    const long boffs = PACKED ? (long)bc * N : (long)bc;
+#pragma unroll
+                    for (int t = 0; t < TN; t++) b[u][t] = load_f16x8(B + boff[t] + boffs);
+                }
+                SMAT_ORDER_FENCE();
+#pragma unroll
+                for (int u = 0; u < NP; u++) multiply(j + u, a[u], b[u]);
             }
         }
     }
+    if (run > 0)
+#pragma unroll
+        for (int t = 0; t < TN; t++) part[run][t][lane] = acc[t];
+    __syncthreads();
+    if (run > 0) return;
+#pragma unroll
+    for (int s = 1; s < SPLIT; s++)
+#pragma unroll
+        for (int t = 0; t < TN; t++) acc[t] += part[s][t][lane];
+    store_tile<TN, C_F32>(acc, br, dst, n0, i16, g, Cout, workspace, N);
 }
 
 // Small problems with short block rows (a band matrix: 9 blocks per row, 256 rows): the kernel above keeps the
@@ -453,18 +562,29 @@ unsigned XcdDeal::run(size_t n_items, int n_panels) const
     return r;
 }
 
-int rowwise_panel_tiles(size_t N, int requested, size_t n_items)
+// Panel width of the row-wise kernel in tiles of 16 columns: as wide as leaves the chip enough wavefronts, since every
+// panel reads the blocks again.  Enough are 768 to 1000 with long items; items of fewer than 32 blocks are over so soon
+// that a panel wider than 64 columns wants 4000 (measured: 512 items of 115 blocks, N = 256 / 512: 128 / 256 columns win, 45
+// against 51 and 73 against 80 us; 1250 items of 14 blocks, N = 256: 64 columns, 19.7 against 21.6 us; 48 items of 51
+// blocks, N = 1024: 64 columns, 9.9 against 31 us for 256).  Lists with split rows are uneven in more than their
+// items' lengths: 64 columns (R-MAT scale 16, N = 512: 618 against 944 us; scale 20, N = 128: 13.8 against 18.2 ms).
+int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, bool split_rows)
 {
-    if (requested == 1 || requested == 2 || requested == 4 || requested == 8 || requested == 16) return requested;
-    if (N >= 1024) return 16; // 256 columns per wavefront: every A block is read once per 256 columns of C
-    if (N >= 512) return 8;
-    // Below that, 64-column panels: measured faster than 128-column ones even where the work
-    // list alone fills the chip (R-MAT scale 20, N = 128: 13.8 ms against 18.2 ms), more
-    // wavefronts in flight outweighing the second pass over A.
-    (void)n_items;
-    if (N >= 64) return 4;
-    if (N >= 32) return 2;
-    return 1;
+    if (N < 32) return 1;
+    if (N < 64) return 2;
+    if (split_rows) return 4;
+    const size_t few = 768, many = avg_blocks < 32 ? 4000 : 1000;
+    if (N >= 256 && n_items * ((N + 255) / 256) >= (N >= 1024 ? few : many)) return 16;
+    if (N >= 128 && n_items * ((N + 127) / 128) >= (N >= 512 ? few : many)) return 8;
+    return 4;
+}
+
+// Four wavefronts per (item, panel of 64 columns): up to 512 of those, of 12 blocks and more.  (256 items of 26 blocks,
+// N = 64: 6.0 against 9.7 us; 512 items of 51 blocks, N = 64: 11.7 against 17.0; with 1024 the two are level, with more
+// the shared items lose.)  The rule knows nothing about the layout of B: in place and repacked give the same bits.
+static bool rowwise_shares_items(size_t N, size_t n_items, size_t avg_blocks)
+{
+    return n_items * ((N + 63) / 64) <= 512 && avg_blocks >= 12;
 }
 
 // The short-row kernel: rows of at most 2 * SHORT_NP blocks, no split rows, B in place, few wavefronts.
@@ -487,6 +607,27 @@ static hipError_t launch_rowwise_short(const SpmmArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
+template <int TN>
+static hipError_t launch_rowwise_split(const SpmmArgs &a, hipStream_t st)
+{
+    const int n_panels = (int)((a.N + 16 * TN - 1) / (16 * TN));
+    const long wgs = (long)a.n_items * n_panels;
+    if (wgs == 0) return hipSuccess;
+    dim3 grid((unsigned)((wgs + 7) / 8 * 8)), block(256);
+#define SMAT_LAUNCH_SPLIT(F32, PK)                                                                                         \
+    hipLaunchKernelGGL((spmm_rowwise_split_kernel<TN, F32, PK>), grid, block, 0, st, a.vals, a.row_ptr, a.col_idx, \
+                       a.b_packed ? a.b_packed : a.B, a.C, a.workspace, a.items, a.n_items, (int)a.N, (long)a.K, n_panels)
+    if (a.b_packed) {
+        if (a.c_f32) SMAT_LAUNCH_SPLIT(true, true);
+        else SMAT_LAUNCH_SPLIT(false, true);
+    } else {
+        if (a.c_f32) SMAT_LAUNCH_SPLIT(true, false);
+        else SMAT_LAUNCH_SPLIT(false, false);
+    }
+#undef SMAT_LAUNCH_SPLIT
+    return hipGetLastError();
+}
+
 hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st)
 {
     hipError_t e;
@@ -502,12 +643,19 @@ hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st)
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    switch (rowwise_panel_tiles(a.N, a.panel_tiles, (size_t)a.n_items)) {
-    case 16: e = launch_rowwise_tn<16>(a, st); break;
-    case 8: e = launch_rowwise_tn<8>(a, st); break;
-    case 4: e = launch_rowwise_tn<4>(a, st); break;
-    case 2: e = launch_rowwise_tn<2>(a, st); break;
-    default: e = launch_rowwise_tn<1>(a, st); break;
+    const size_t n_items = (size_t)a.rule_items, avg = n_items ? a.nnzb / n_items : 0;
+    if (rowwise_shares_items(a.N, n_items, avg)) {
+        if (a.N < 32) e = launch_rowwise_split<1>(a, st);
+        else if (a.N < 64) e = launch_rowwise_split<2>(a, st);
+        else e = launch_rowwise_split<4>(a, st);
+    } else {
+        switch (rowwise_panel_tiles(a.N, n_items, avg, a.n_split_rows > 0)) {
+        case 16: e = launch_rowwise_tn<16>(a, st); break;
+        case 8: e = launch_rowwise_tn<8>(a, st); break;
+        case 4: e = launch_rowwise_tn<4>(a, st); break;
+        case 2: e = launch_rowwise_tn<2>(a, st); break;
+        default: e = launch_rowwise_tn<1>(a, st); break;
+        }
     }
     if (e != hipSuccess) return e;
     if (a.n_split_rows > 0) e = launch_reduce(a.workspace, a.split_rows, a.n_split_rows, a.C, a.N, a.c_f32, st);
