@@ -258,18 +258,39 @@ class Plan:
             pass
 
 
+_launch, _launch_drop_in = lib.smat_spmm_bcsr_f16_ex, lib.smat_spmm_bcsr_f16
+_opts_of = {}  # options that were used before, ready to pass; never written again
+
+
+def _opts(key):
+    if len(_opts_of) >= 256:  # one per stream, so a program could go on making them
+        _opts_of.clear()
+    b_row_major, c_f32, kernel, stream = key
+    o = SpmmOpts(1 if b_row_major else 0, C_F32 if c_f32 else C_F16, kernel, 0, C.c_void_p(stream) if stream else None)
+    r = _opts_of[key] = C.byref(o)  # keeps o alive
+    return r
+
+
 def spmm(vals, row_ptr, col_idx, B, C_out, M, N, K, nnzb, plan=None, c_f32=False, kernel=KERNEL_AUTO,
          stream=None, drop_in=False, b_row_major=False):
     """Launch the SpMM on device tensors (anything with .data_ptr()).
 
     drop_in=True calls the positional drop-in entry point (smat_spmm_bcsr_f16) with
     NULL block_info / rel_map; otherwise the options entry point."""
-    ptr = lambda t: C.c_void_p(t.data_ptr()) if t is not None else None  # noqa: E731
+    # A small product is over sooner than the call that launches it: addresses go to ctypes as plain integers and the
+    # options are not made anew (1.1 us of Python per call when they were).
+    v = vals.data_ptr() if vals is not None else None
+    rp = row_ptr.data_ptr() if row_ptr is not None else None
+    ci = col_idx.data_ptr() if col_idx is not None else None
+    b = B.data_ptr() if B is not None else None
+    c = C_out.data_ptr() if C_out is not None else None
     if drop_in:
-        check(lib.smat_spmm_bcsr_f16(ptr(vals), ptr(row_ptr), ptr(col_idx), ptr(B), ptr(C_out), M, N, K, nnzb,
-                                     None, None))
-        return
-    opts = SpmmOpts(1 if b_row_major else 0, C_F32 if c_f32 else C_F16, kernel, 0,
-                    C.c_void_p(stream) if stream else None)
-    check(lib.smat_spmm_bcsr_f16_ex(ptr(vals), ptr(row_ptr), ptr(col_idx), ptr(B), ptr(C_out), M, N, K, nnzb,
-                                    C.byref(opts), plan.handle if plan is not None else None))
+        rc = _launch_drop_in(v, rp, ci, b, c, M, N, K, nnzb, None, None)
+    else:
+        key = (b_row_major, c_f32, kernel, stream)
+        o = _opts_of.get(key)
+        if o is None:
+            o = _opts(key)
+        rc = _launch(v, rp, ci, b, c, M, N, K, nnzb, o, plan._h if plan is not None else None)
+    if rc:
+        check(rc)
