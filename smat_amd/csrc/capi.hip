@@ -560,11 +560,19 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     // per block (27-point stencil) 53 us compact against 86 us row-wise; 16 per block (dense blocks, N = 4096)
     // 326 us against 180 us.  This is the per-block classification of the reference (matrix.h:400-419: blocks
     // without / with 2:4 / with dense rows) put to use per block row.
-    std::vector<uint8_t> dense, block_cols;
+    CompactCensus census;
     CompactPlan *c = nullptr;
-    hipError_t e = compact_build(vals, row_ptr, col_idx, row_ptr_host, mb, p->nnzb, p->n_cap, may_mix ? 0.6 : 0.0,
-                                 may_mix ? &dense : nullptr, &c, nullptr, may_mix ? &block_cols : nullptr);
+    hipError_t e = compact_census(vals, row_ptr, mb, p->nnzb, census);
     if (e != hipSuccess) return fail(e);
+    std::vector<uint8_t> dense(mb, 0);
+    int64_t dense_cols_all = 0;
+    for (size_t i = 0; may_mix && i < mb; i++) {
+        const int64_t blocks = row_ptr_host[i + 1] - row_ptr_host[i], cols = census.cols_of_row(i);
+        if (blocks > 0 && (double)cols >= 0.6 * 16.0 * (double)blocks) {
+            dense[i] = 1;
+            dense_cols_all += cols;
+        }
+    }
     int64_t blocks_dense = 0;
     for (size_t i = 0; may_mix && i < mb; i++)
         if (dense[i]) blocks_dense += row_ptr_host[i + 1] - row_ptr_host[i];
@@ -583,7 +591,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
         // operand bytes, the row-wise kernel on B in place 7.6 TB/s, the row-wise kernel on repacked B 20 TB/s; a
         // pass over B moves 4*K*N bytes at 4 TB/s; a launch costs 3 us.  (27-point stencil on 64^3 after the reorder,
         // N = 64: a sixth of the blocks sit in dense rows, 10 us of compact kernel against 20 us for the repack alone.)
-        const double dense_cols = (double)(c->n_cols_all - c->n_cols);
+        const double dense_cols = (double)dense_cols_all;
         const double t_compact = dense_cols * (double)p->n_cap * 2.0 / 10e6;
         const double gather = (double)blocks_dense * 16.0 * (double)p->n_cap * 2.0;
         const double t_direct = gather / 7.6e6 + 3.0;
@@ -603,61 +611,49 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     // (10 % dense blocks with as many blocks again of one nonzero: estimate 179 us, measured 180; sweep kernel alone
     // 201 us, compact kernel alone 252 us).
     bool block_split = false;
-    std::vector<uint8_t> skip;
-    int64_t n_split_blocks = 0;
+    const int64_t n_split_blocks = census.full_blocks;
     const double n_est = (double)p->n_cap, n_rg_est = (double)((mb + SWEEP_G - 1) / SWEEP_G);
     auto t_sweep = [&](double blocks) { return n_rg_est * (double)p->K * n_est * 2.0 / 13.4e6 + blocks * n_est * 512.0 / 1.04e9; };
     auto t_compact = [&](double cols) { return cols * n_est * 2.0 / 10e6; };
     const double t_pass = 3.0 + (double)p->K * n_est / 1e6;
     // one kernel for everything: the sweep kernel (when the plan has its work list) or the compact kernel
     const double t_sweep_all = p->sweep.d_ops ? t_sweep((double)p->nnzb) : 1e30;
-    const double t_compact_all = t_compact((double)c->n_cols_all) + t_pass;
-    if (may_mix && !mixed && !p->col_idx_host.empty() && block_cols.size() == p->nnzb && p->nnzb < ((size_t)1 << 23) &&
+    const double t_compact_all = t_compact((double)census.n_cols_all) + t_pass;
+    if (may_mix && !mixed && !p->col_idx_host.empty() && p->nnzb < ((size_t)1 << 23) &&
         p->K < ((size_t)1 << 28) && sweep_fills_device(mb, p->n_cap)) {
-        int64_t cols_rest = 0;
-        skip.assign(p->nnzb, 0);
-        for (size_t q = 0; q < p->nnzb; q++) {
-            if (block_cols[q] >= 10) { skip[q] = 1; n_split_blocks++; }
-            else cols_rest += block_cols[q];
-        }
         const int64_t n_rest = (int64_t)p->nnzb - n_split_blocks;
         if (n_split_blocks >= 2 && n_split_blocks * 10 >= (int64_t)p->nnzb && n_rest * 10 >= (int64_t)p->nnzb) {
-            const double t_split = t_sweep((double)n_split_blocks) + t_compact((double)cols_rest) + t_pass;
+            const double t_split = t_sweep((double)n_split_blocks) + t_compact((double)census.cols_rest) + t_pass;
             block_split = want == SMAT_KERNEL_MIXED || t_split < 0.95 * std::min(t_sweep_all, t_compact_all);
         }
     }
-    if (block_split) { // the list without the blocks that the sweep kernel takes
-        compact_destroy(c);
-        c = nullptr;
-        e = compact_build(vals, row_ptr, col_idx, row_ptr_host, mb, p->nnzb, p->n_cap, 0.0, nullptr, &c, skip.data(), nullptr);
+    std::vector<uint8_t> skip; // the blocks that the sweep kernel takes
+    if (block_split) { // the list without them
+        e = compact_full_blocks(census, skip);
+        if (e == hipSuccess) e = compact_build(census, vals, row_ptr, col_idx, p->K, p->n_cap, nullptr, true, &c);
         if (e != hipSuccess) return fail(e);
         if (c->n_split_rows > 0) { // partial tiles through the workspace cannot be added to C: one kernel for everything
             block_split = false;
             compact_destroy(c);
             c = nullptr;
-            e = compact_build(vals, row_ptr, col_idx, row_ptr_host, mb, p->nnzb, p->n_cap, 0.0, nullptr, &c);
+            e = compact_census(vals, row_ptr, mb, p->nnzb, census);
             if (e != hipSuccess) return fail(e);
         }
     }
     if (want == SMAT_KERNEL_MIXED && !block_split) mixed = true;
-    if (may_mix && !mixed && !block_split && blocks_dense > 0) { // the list left dense rows out: make it whole again
-        compact_destroy(c);
-        c = nullptr;
-        e = compact_build(vals, row_ptr, col_idx, row_ptr_host, mb, p->nnzb, p->n_cap, 0.0, nullptr, &c);
-        if (e != hipSuccess) return fail(e);
-    }
     if (p->compact) { compact_destroy(p->compact); p->compact = nullptr; }
     drop_mixed();
     // the compact kernel for everything: few nonzero columns per block - unless the plan has the sweep kernel's work
     // list and the same estimate says that one is faster (blocks of both kinds in a matrix that is dense enough)
     const bool take = mixed || block_split || want == SMAT_KERNEL_COMPACT ||
-                      (want == SMAT_KERNEL_AUTO && (double)c->n_cols_all < 0.6 * 16.0 * (double)p->nnzb &&
+                      (want == SMAT_KERNEL_AUTO && (double)census.n_cols_all < 0.6 * 16.0 * (double)p->nnzb &&
                        !(dense_kernel == SMAT_KERNEL_SWEEP && t_sweep_all < t_compact_all));
-    if (!take) { // nothing will use the list: the plan keeps (or goes back to) a dense kernel
-        compact_destroy(c);
+    if (!take) { // nothing would use the list: the plan keeps (or goes back to) a dense kernel
         if (p->kernel == SMAT_KERNEL_COMPACT || p->kernel == SMAT_KERNEL_MIXED) p->kernel = dense_kernel;
         return SMAT_OK;
     }
+    if (!c) e = compact_build(census, vals, row_ptr, col_idx, p->K, p->n_cap, mixed ? &dense : nullptr, false, &c);
+    if (e != hipSuccess) return fail(e);
     if (!p->d_bt) e = dev_malloc(&p->d_bt, p->bt_bytes());
     std::vector<int32_t> dense_list;
     for (size_t i = 0; mixed && i < mb; i++)

@@ -14,35 +14,21 @@
 //                       list into work items (whole block rows, long ones in chunks whose fp32
 //                       partial tiles are summed afterwards);
 //      gather_kernel    writes, for every nonzero column, its row of B (absolute column index)
-//                       and a COPY of its 16 values in MFMA operand order:
+//                       and a COPY of its values: either all 16 in MFMA operand order,
 //                       acol[((step*4 + g)*16 + m)*8 + j] = A[m][column 32*step + 8*g + j],
-//                       so that the A operand of a step is one coalesced 16-byte load per lane.
+//                       so that the A operand of a step is one coalesced 16-byte load per lane; or, where
+//                       columns hold few nonzeros, the nonzeros alone with their places in that operand.
 //    The SpMM then does not read the block values any more: they must be attached again when
 //    they change.
 //  * transpose_b_kernel: column-major B (B[n*K + k]) -> Bt at the start of every launch, so that
 //    the row of B under a nonzero column is contiguous.  Bt holds the panels of 64*TQ columns one
 //    after the other, each a row-major K x 64*TQ matrix: the pass over a panel gathers from one
 //    contiguous K * 128*TQ bytes.
-//  * spmm_compact_kernel<TQ>: one wavefront per (work item, panel of 64*TQ columns).  A step takes
-//    32 columns = K of one v_mfma_f32_16x16x32_f16.  The product is formed as
-//    C^T = B^T * A^T like in the other kernels:
-//      A operand   lane (m = lane % 16, g = lane / 16): one 16-byte load from acol;
-//      B operand   lane (i = lane % 16, g) needs, for each of its 8 entries (listed columns 8g .. 8g+7 of the
-//                  step), the columns of C its tiles own.  Every gather is 16 bytes per lane: a CU keeps a
-//                  limited number of vector memory instructions (and of cache lines) in flight, so an
-//                  instruction should bring as much as it can (8-byte gathers: 12 % slower on every config).
-//                  TQ = 2: 8 columns 8i .. 8i+7 of the 128-column panel per entry (16 lanes read 256
-//                  contiguous bytes); one v_perm_b32 per word merges the t-th halves of two consecutive
-//                  entries into the operand word of n-tile t, so tile t of the group owns columns 8i + t.
-//                  TQ = 1 (rows of 128 bytes): lanes i < 8 gather the even entries of the group, lanes
-//                  i >= 8 the odd ones, 8 columns 8 (i & 7) .. + 7 each (4 instructions, not 8); lane i and
-//                  lane i ^ 8 then trade halves (one DPP row rotation per word), so that each has 4 columns
-//                  of all 8 entries: tile t owns columns 8 (i & 7) + 4 (i >> 3) + t.
-//                  The index list keeps, inside every group of 8, the even entries first and then the odd
-//                  ones, so the four indices such a lane needs are 16 contiguous bytes; one load instruction
-//                  fetches them for 8 steps at a time (lane i16 & 7 = step) and DPP row broadcasts hand them round.
-//      result      TQ = 2: lane (m, g) holds 32 consecutive columns of C row m;
-//                  TQ = 1: after one v_permlane32_swap per value, 16 consecutive columns.
+//  * spmm_compact_kernel<TQ>: one wavefront per (run of work items, panel of 64*TQ columns).  A step takes
+//    32 columns = K of one v_mfma_f32_16x16x32_f16.  The product is formed as C^T = B^T * A^T like in the other
+//    kernels; every gather is 16 bytes per lane (a CU keeps a limited number of vector memory instructions and of
+//    cache lines in flight, so an instruction should bring as much as it can).  The index list keeps, inside every
+//    group of 8, the even entries first and then the odd ones: the four indices a lane needs are 16 contiguous bytes.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <stdint.h>
@@ -67,41 +53,61 @@ int g_tune = 1; // test hook: 0 = attaching values measures nothing, the estimat
 int g_last_run = 0; // test hook: the run length of the latest launch
 int g_force_tq = 0; // test hook: 1 or 2 = panels of 64 or 128 columns whatever the sizes say, 0 = the launcher decides
 
-constexpr int LIST_PAD = 640; // entries readable past the end of the list (the index loads of the 64-column panel run up to 16 steps ahead)
+constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts as full (of 16)
+constexpr int TASK_STEPS = 12;     // short items are put together up to this many steps (8 to 24: level; one item each: 9 % slower on R-MAT)
+constexpr int MAX_TASK_STEPS = 56; // of a task of the product kernel: the entry ranges of 64 steps come in at once, some of them read ahead
+constexpr int LIST_PAD = 2304; // entries readable past the end of the list (the index loads of the 64-column panel run up to 16 steps ahead)
 
 // ---- census of nonzero block columns ----
 
-// Order-independent 64-bit checksum of the block values: sum over all dwords of value * (2 * index + 1).  A workgroup
-// adds its part to one of CHECKSUM_SLOTS words, 128 bytes apart: additions to one word queue up at 12 ns each, which
-// for one word and every wavefront of a pass over 121 MB is 200 us of a 25 us pass.
-constexpr int CHECKSUM_SLOTS = 32, CHECKSUM_STRIDE = 16;
-constexpr size_t CHECKSUM_BYTES = CHECKSUM_SLOTS * CHECKSUM_STRIDE * sizeof(unsigned long long);
+// Sums over a whole pass: a workgroup adds its part to one of SUM_SLOTS groups of words, 128 bytes apart.  Additions to
+// one word queue up at 12 ns each, which for one word and every wavefront of a pass over 121 MB is 200 us of a 25 us pass.
+constexpr int SUM_SLOTS = 32, SUM_STRIDE = 16;
+constexpr size_t SUM_BYTES = SUM_SLOTS * SUM_STRIDE * sizeof(unsigned long long);
+template <int N>
+__device__ __forceinline__ void add_totals(const unsigned long long (&mine)[N], unsigned long long *__restrict__ sums)
+{
+    __shared__ unsigned long long part[4][N];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        unsigned long long v = mine[i];
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6][i] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < N) {
+        const unsigned long long v = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
+        if (v) atomicAdd(&sums[(blockIdx.x % SUM_SLOTS) * SUM_STRIDE + threadIdx.x], v);
+    }
+}
+// sums[i] of the pass, from the words that add_totals added to (synchronous)
+hipError_t fetch_totals(const void *d_sums, unsigned long long *out, int n)
+{
+    std::vector<unsigned long long> all(SUM_BYTES / sizeof(unsigned long long));
+    const hipError_t e = hipMemcpy(all.data(), d_sums, SUM_BYTES, hipMemcpyDeviceToHost);
+    for (int i = 0; i < n; i++) {
+        out[i] = 0;
+        for (int s = 0; s < SUM_SLOTS; s++) out[i] += all[(size_t)(s * SUM_STRIDE + i)];
+    }
+    return e;
+}
+// Order-independent 64-bit checksum of the block values: sum over all dwords of value * (2 * index + 1).
 __device__ __forceinline__ unsigned long long checksum_term(uint32_t v, long i)
 {
     return (unsigned long long)v * (2ull * (unsigned long long)i + 1ull);
 }
-__device__ __forceinline__ void add_checksum(unsigned long long sum, unsigned long long *__restrict__ sums)
-{
-    __shared__ unsigned long long part[4];
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(&sums[(blockIdx.x % CHECKSUM_SLOTS) * CHECKSUM_STRIDE], part[0] + part[1] + part[2] + part[3]);
-}
-uint64_t total_checksum(const std::vector<unsigned long long> &sums)
-{
-    uint64_t h = 0;
-    for (int i = 0; i < CHECKSUM_SLOTS; i++) h += sums[(size_t)i * CHECKSUM_STRIDE];
-    return h;
-}
 
-// The checksum of the block values (values_checksum_kernel) is taken on the way.
+// What a pass over the blocks counts besides the masks, summed over all blocks (add_totals): the checksum of the values,
+// blocks with at least FULL_BLOCK_COLS nonzero columns, nonzero columns of the others, nonzeros.
+enum { SUM_CHECK, SUM_FULL, SUM_COLS_REST, SUM_NNZ, N_SUMS };
+
+// Per block: mask of its nonzero columns; their number in the lower half of count, the number of nonzeros in the upper.
 __global__ __launch_bounds__(256) void colmask_kernel(const uint16_t *__restrict__ vals, long nnzb,
-                                                      uint16_t *__restrict__ mask, int32_t *__restrict__ count,
+                                                      uint16_t *__restrict__ mask, unsigned long long *__restrict__ count,
                                                       unsigned long long *__restrict__ sums)
 {
-    unsigned long long sum = 0;
+    unsigned long long total[N_SUMS] = {0, 0, 0, 0};
     const int lane = threadIdx.x & 63;
     const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const long n_waves = ((long)gridDim.x * blockDim.x) >> 6;
@@ -110,15 +116,22 @@ __global__ __launch_bounds__(256) void colmask_kernel(const uint16_t *__restrict
         // lane % 32 = row * 2 + half: 8 values of one row
         u32x4 w = {0u, 0u, 0u, 0u};
         if (blk < nnzb) w = *reinterpret_cast<const u32x4 *>(vals + blk * 256 + (lane & 31) * 8);
+        int nz = 0;
 #pragma unroll
-        for (int q = 0; q < 4; q++) sum += checksum_term(w[q], blk * 128 + (lane & 31) * 4 + q);
-        w &= 0x7fff7fffu; // -0.0 is a zero
+        for (int q = 0; q < 4; q++) {
+            total[SUM_CHECK] += checksum_term(w[q], blk * 128 + (lane & 31) * 4 + q);
+            w[q] &= 0x7fff7fffu; // -0.0 is a zero
+            nz += ((w[q] & 0xffffu) != 0) + ((w[q] >> 16) != 0);
+        }
 #pragma unroll
-        for (int d = 2; d <= 16; d <<= 1) { // OR over the 16 rows (lane bits 1..4)
-            w[0] |= __shfl_xor(w[0], d);
-            w[1] |= __shfl_xor(w[1], d);
-            w[2] |= __shfl_xor(w[2], d);
-            w[3] |= __shfl_xor(w[3], d);
+        for (int d = 1; d <= 16; d <<= 1) {
+            if (d >= 2) { // OR over the 16 rows (lane bits 1..4)
+                w[0] |= __shfl_xor(w[0], d);
+                w[1] |= __shfl_xor(w[1], d);
+                w[2] |= __shfl_xor(w[2], d);
+                w[3] |= __shfl_xor(w[3], d);
+            }
+            nz += __shfl_xor(nz, d);
         }
         uint32_t bits = 0;
 #pragma unroll
@@ -129,11 +142,15 @@ __global__ __launch_bounds__(256) void colmask_kernel(const uint16_t *__restrict
         const uint32_t other = __shfl_xor(bits, 1); // the other half of the row
         if ((lane & 31) == 0 && blk < nnzb) {
             const uint32_t m = bits | (other << 8);
+            const int cols = __popc(m);
             mask[blk] = (uint16_t)m;
-            count[blk] = __popc(m);
+            count[blk] = (unsigned long long)nz << 32 | (unsigned)cols;
+            total[SUM_NNZ] += nz;
+            if (cols >= FULL_BLOCK_COLS) total[SUM_FULL]++;
+            else total[SUM_COLS_REST] += cols;
         }
     }
-    add_checksum(sum, sums);
+    add_totals<N_SUMS>(total, sums);
 }
 
 __global__ __launch_bounds__(256) void values_checksum_kernel(const u32x4 *__restrict__ vals, long n_quads, unsigned long long *__restrict__ sums)
@@ -144,27 +161,36 @@ __global__ __launch_bounds__(256) void values_checksum_kernel(const u32x4 *__res
 #pragma unroll
         for (int q = 0; q < 4; q++) sum += checksum_term(v[q], 4 * i + q);
     }
-    add_checksum(sum, sums);
+    const unsigned long long total[1] = {sum};
+    add_totals<1>(total, sums);
 }
 
-// One thread per block: its nonzero columns go to positions padded_start[br] + (offset[p] -
-// offset[row_ptr[br]]) .. of the padded list.
+// One thread per block: its nonzero columns go to positions padded_start[br] + (columns of the block row in the blocks
+// before it) .. of the padded list, and
+//   acol != NULL: their 16 values each to acol, in MFMA operand order;
+//   else: their nonzeros to entries from entry_start[br] + (nonzeros of the block row before) on, column by column,
+//         each with its place in the operand of its step, and the range of entries of every step to step_range.
 __global__ void gather_kernel(const uint16_t *__restrict__ vals, const uint16_t *__restrict__ mask,
-                              const int32_t *__restrict__ offset, const int32_t *__restrict__ row_ptr,
-                              const int32_t *__restrict__ col_idx, const int32_t *__restrict__ padded_start,
-                              long mb, long nnzb, int32_t *__restrict__ cols, uint16_t *__restrict__ acol)
+                              const unsigned long long *__restrict__ offset, const int32_t *__restrict__ row_ptr,
+                              const int32_t *__restrict__ col_idx, const unsigned long long *__restrict__ raw,
+                              const int2 *__restrict__ start, long mb, long nnzb, bool drop_full, int32_t *__restrict__ cols,
+                              uint16_t *__restrict__ acol, uint32_t *__restrict__ entries, int2 *__restrict__ step_range)
 {
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= nnzb) return;
     uint32_t m = mask[p];
-    if (!m) return;
+    if (!m || (drop_full && __popc(m) >= FULL_BLOCK_COLS)) return;
     long lo = 0, hi = mb; // block row of p: largest br with row_ptr[br] <= p
     while (hi - lo > 1) {
         const long mid = (lo + hi) >> 1;
         if (row_ptr[mid] <= p) lo = mid; else hi = mid;
     }
-    if (padded_start[lo] < 0) return; // a block row that another kernel multiplies
-    long o = (long)padded_start[lo] + (offset[p] - offset[row_ptr[lo]]);
+    const int2 first = start[lo]; // of the columns and of the entries
+    if (first.x < 0) return; // a block row that another kernel multiplies
+    const unsigned long long before = offset[p] - raw[lo]; // no borrow: both halves of offset[p] are at least those of raw
+    const long row_end = (long)first.x + (long)(uint32_t)(raw[lo + 1] - raw[lo]);
+    long o = (long)first.x + (long)(uint32_t)before;
+    int32_t at = first.y + (int32_t)(before >> 32);
     const int32_t c0 = col_idx[p];
     const uint16_t *blk = vals + p * 256;
     while (m) {
@@ -173,16 +199,57 @@ __global__ void gather_kernel(const uint16_t *__restrict__ vals, const uint16_t 
         // inside its group of 8 the even entries come first, then the odd ones: the lanes of the product kernel that
         // gather the even (odd) entries of a group read their four indices with one 16-byte load
         cols[(o & ~7L) + ((o & 1) << 2) + ((o & 7) >> 1)] = c0 + k;
-        uint16_t *dst = acol + ((o >> 3) * 16) * 8 + (o & 7); // (step*4 + g) = o / 8
+        if (acol) {
+            uint16_t *dst = acol + ((o >> 3) * 16) * 8 + (o & 7); // (step*4 + g) = o / 8
 #pragma unroll
-        for (int r = 0; r < 16; r++) dst[r * 8] = blk[r * 16 + k];
+            for (int r = 0; r < 16; r++) dst[r * 8] = blk[r * 16 + k];
+        } else {
+            if ((o & 31) == 0) step_range[o >> 5].x = at;
+            const uint32_t place = (uint32_t)((o & 31) >> 3) * 128u + (uint32_t)(o & 7); // half of the step's operand, row 0; the entry holds it in bytes
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const uint32_t v = blk[r * 16 + k];
+                if (v & 0x7fffu) entries[at++] = v << 16 | (place + r * 8) * 2;
+            }
+            if ((o & 31) == 31 || o + 1 == row_end) step_range[o >> 5].y = at;
+        }
         o++;
     }
 }
 
-// raw[br] = first (unpadded) list position of block row br; raw[mb] = total
-__global__ void row_offsets_kernel(const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ offset,
-                                   const int32_t *__restrict__ count, long mb, long nnzb, int32_t *__restrict__ raw)
+// Steps of every group of 32 listed columns: one for each `most` of its entries, at least one.
+__global__ void count_steps_kernel(const int2 *__restrict__ group_range, int n_groups, int most, int32_t *__restrict__ steps)
+{
+    const int g = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (g >= n_groups) return;
+    const int n = group_range[g].y - group_range[g].x;
+    steps[g] = n > most ? (n + most - 1) / most : 1;
+}
+// The groups that take several steps are listed once for each, with another part of their entries.  32 threads a group.
+__global__ __launch_bounds__(256) void expand_steps_kernel(const int2 *__restrict__ group_range, const int32_t *__restrict__ group_cols,
+                                                           const int32_t *__restrict__ steps, const int32_t *__restrict__ first_step, int n_groups,
+                                                           int most, int2 *__restrict__ step_range, int32_t *__restrict__ cols)
+{
+    const int g = (int)(blockIdx.x * 8 + threadIdx.x / 32), i = threadIdx.x & 31;
+    if (g >= n_groups) return;
+    const int2 r = group_range[g];
+    const int32_t col = group_cols[(long)g * 32 + i];
+    for (int k = 0; k < steps[g]; k++) {
+        const int s = first_step[g] + k;
+        cols[(long)s * 32 + i] = col;
+        if (i == 0) step_range[s] = int2{r.x + k * most, min(r.x + (k + 1) * most, r.y)};
+    }
+}
+// first_step of the first group of every block row (starts: its first listed column, and the end)
+__global__ void row_steps_kernel(const int32_t *__restrict__ starts, const int32_t *__restrict__ first_step, long n, int32_t *__restrict__ out)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = first_step[starts[i] / 32];
+}
+
+// raw[br] = what the blocks before block row br hold: columns in the lower, nonzeros in the upper half; raw[mb] = total
+__global__ void row_offsets_kernel(const int32_t *__restrict__ row_ptr, const unsigned long long *__restrict__ offset,
+                                   const unsigned long long *__restrict__ count, long mb, long nnzb, unsigned long long *__restrict__ raw)
 {
     const long br = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (br > mb) return;
@@ -190,14 +257,11 @@ __global__ void row_offsets_kernel(const int32_t *__restrict__ row_ptr, const in
     raw[br] = p < nnzb ? offset[p] : (nnzb ? offset[nnzb - 1] + count[nnzb - 1] : 0);
 }
 
-// Blocks that another kernel multiplies (per-block split of a mixed plan): no listed columns.
-__global__ void drop_blocks_kernel(const uint8_t *__restrict__ skip, long nnzb, uint16_t *__restrict__ mask, int32_t *__restrict__ count)
+// Blocks that another kernel multiplies (per-block split of a mixed plan): nothing of theirs is listed.
+__global__ void drop_full_kernel(const uint16_t *__restrict__ mask, long nnzb, unsigned long long *__restrict__ count)
 {
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < nnzb && skip[p]) {
-        mask[p] = 0;
-        count[p] = 0;
-    }
+    if (p < nnzb && __popc((uint32_t)mask[p]) >= FULL_BLOCK_COLS) count[p] = 0;
 }
 
 // out[j] = block ids[j] of vals (512 bytes each; 32 lanes x 16 bytes per block).
@@ -255,277 +319,246 @@ __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__rest
 
 // ---- the product ----
 
+// A wavefront takes a task x a panel of 64 TQ columns.  A task is a run of items of the list, worked off as one stream of
+// steps, so that the loads of the next step are under way across the end of an item.
+//
+// What bounds a step of 32 columns x 64 columns of C on a CU is the return path of the vector L1 (4 KiB of rows of B and
+// 0.3 to 1 KiB of A at 64 bytes a clock) and, close behind, the LDS and the VALU.  Hence:
+//   * Rows of B go from the registers they were gathered into through 4 KiB of LDS, [entry][64 columns], and come back as
+//     MFMA operands through transposing reads (ds_read_b64_tr_b16): no VALU work, where exchanging and merging halves
+//     between lanes took 56 VALU instructions of 130 a step.  Lane (octet o = lane / 8, c = lane & 7) gathers columns
+//     8c .. 8c + 7 of the entries k = 8 (o / 2) + 2j + (o & 1), j = 0 .. 3; the 16-byte pieces of the rows k with k & 2 are
+//     swapped in pairs, so that neither side has bank conflicts.  In lane (i = lane % 16, g = lane / 16) n-tile t of the
+//     operand reads columns 16 (i & 3) + 4t .. + 3 of the rows 8g + i / 4 and + 4; the lane ends up with the 16
+//     consecutive columns 16g .. of row i of the tile of C.
+//   * The address of a gathered row is one multiply-add of 32 bits from its index (BIG: 64 bits, for copies of B of 4 GiB
+//     and more).
+//   * The A operand (AF): 0: acol, 1 KiB a step.  1, 2: entries, 4 bytes per nonzero; the at most 64 * AF of a step are put
+//     to their places in 1 KiB of LDS that is zero otherwise, read back as the operand and cleared again (LDS operations
+//     of a wavefront complete in order: nothing is waited for in between).
+//   * Every load of a step is unconditional and nothing in the loop uses scalar loads, so that what is in flight can be
+//     counted; the gathers asked for past the end of the task read row 0.
+// Whole products with all of it (before: operands merged in the VALU, A in whole columns, an item per wavefront): R-MAT
+// scale 20, N = 128, 703 -> 595 us; Erdos-Renyi 16384^2, 0.1 %, N = 256, 17.3 -> 16.3 us.  A third copy of the step's code
+// costs more than it saves: kernels of 10 us wait for their instructions.
+//
 // C_ACC: the result is added to what C holds (the per-block split of a mixed plan: a dense kernel has written the
 // part of the blocks it multiplies); work items that go through the workspace are not made for such plans.
-template <int TQ, bool C_F32, bool C_ACC>
+template <int TQ, bool C_F32, bool C_ACC, int AF, bool BIG>
 __global__ __launch_bounds__(256) void spmm_compact_kernel(
-    const uint16_t *__restrict__ acol, const int32_t *__restrict__ cols, const uint16_t *__restrict__ Bt,
-    void *__restrict__ Cout, float *__restrict__ workspace, const WorkItem *__restrict__ items, int n_items, int N,
-    int n_panels, long panel_stride, long row_stride, unsigned xcd_run)
+    const uint16_t *__restrict__ acol, const uint32_t *__restrict__ entries, const int2 *__restrict__ step_range, const int32_t *__restrict__ cols,
+    const uint16_t *__restrict__ Bt, void *__restrict__ Cout, float *__restrict__ workspace, const WorkItem *__restrict__ items,
+    const int4 *__restrict__ tasks, int n_tasks, int N, int n_panels, long panel_stride, long row_stride, unsigned xcd_run)
 {
-    constexpr int PANEL = 64 * TQ;
+    constexpr int A_BYTES = 1024, B_BYTES = 4096 * TQ, I_BYTES = 2048;
+    __shared__ __align__(1024) unsigned char lds[4][A_BYTES + B_BYTES + I_BYTES];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // Panel-major order of the (panel, item) space.  An XCD gets the workgroup ids that are equal modulo 8, whatever
+    // Panel-major order of the (panel, task) space.  An XCD gets the workgroup ids that are equal modulo 8, whatever
     // their work costs; here the XCDs take runs of xcd_run consecutive workgroups of that order in turn (gridDim.x is a
     // multiple of 8 * xcd_run).  One run per XCD keeps neighbouring block rows, which share rows of B, on one L2;
-    // short runs even out a list whose cost per item changes along it (R-MAT: 60 to 70 % of the steps are in the first
+    // short runs even out a list whose cost per task changes along it (R-MAT: 60 to 70 % of the steps are in the first
     // quarter of the items, and the launch took as long as the XCD that got them).
-    const long total = (long)n_items * n_panels;
+    const long total = (long)n_tasks * n_panels;
     const unsigned slot = blockIdx.x >> 3;
     const unsigned run = __builtin_amdgcn_readfirstlane(slot / xcd_run);
     const long wg = ((long)run * 8 + (blockIdx.x & 7)) * xcd_run + (slot - run * xcd_run);
     const long w = wg * 4 + wave;
     if (w >= total) return;
-    const int panel = (int)(w / n_items);
-    const int it = (int)(w - (long)panel * n_items);
-    const WorkItem wi = items[it];
-    const int br = __builtin_amdgcn_readfirstlane(wi.block_row);
-    const int e0 = __builtin_amdgcn_readfirstlane(wi.begin);
-    const int e1 = __builtin_amdgcn_readfirstlane(wi.end);
-    const int dst = __builtin_amdgcn_readfirstlane(wi.dst);
+    const int panel = __builtin_amdgcn_readfirstlane((int)(w / n_tasks));
+    const int task = __builtin_amdgcn_readfirstlane((int)(w - (long)panel * n_tasks));
+    const int4 tk = tasks[task]; // first item, items (at most 64), first and last column of the stream
+    int e = tk.z;
+    const int e_last = tk.w;
+    // Scalar loads share a counter with the LDS operations below, which would wait for them at every step: the items of
+    // the task and the entry ranges of its steps come in through vector loads, one per lane, and are read from the lanes.
+    const WorkItem mine = items[tk.x + (lane < tk.y ? lane : tk.y - 1)];
+    int it = 0, item_end, br, dst;
+    auto enter = [&] {
+        br = __builtin_amdgcn_readlane(mine.block_row, it);
+        item_end = __builtin_amdgcn_readlane(mine.end, it);
+        dst = __builtin_amdgcn_readlane(mine.dst, it);
+    };
+    enter();
 
     const int i16 = lane & 15, g = lane >> 4;
-    const int n0 = panel * PANEL;
-    // Row `col` of this panel of B starts at Bp + col * row_stride (B in place: panel_stride = PANEL,
-    // row_stride = N; the transposed copy: panels one after the other, row_stride = PANEL).
+    const int n0 = panel * 64 * TQ;
+    // Row `col` of this panel of B starts at Bp + col * row_stride (B in place: panel_stride = 64 TQ, row_stride = N; the
+    // transposed copy: panels one after the other, row_stride = 64 TQ).
     const uint16_t *Bp = Bt + (long)panel * panel_stride;
-    // Every gather is 16 bytes per lane: what a CU can keep in flight is a number of vector memory instructions
-    // and of cache lines, so an instruction should bring as much as it can.
-    //   WIDE (TQ = 2): a lane takes 8 columns of the 128-column panel, for each of its 8 entries.
-    //   PAIRED (TQ = 1, rows of 128 bytes): lanes i16 < 8 take the even entries, lanes i16 >= 8 the odd ones, 8
-    //   columns each (4 instructions instead of 8); the two lanes then trade halves, so that each has 4 columns of
-    //   all 8 entries again.
-    constexpr bool WIDE = TQ % 2 == 0, PAIRED = TQ == 1;
-    static_assert(TQ == 1 || TQ == 2, "panels of 64 or 128 columns");
-    constexpr int NG = WIDE ? TQ / 2 : 1; // groups of 128 columns (WIDE)
-    const bool odd_entries = (i16 & 8) != 0; // PAIRED
-    int boff[NG]; // element offset of this lane's 8 columns inside the panel row (its column 0 when out of range)
+    int boff[TQ]; // N % 8 == 0: all of the lane's columns or none (then its column 0)
 #pragma unroll
-    for (int q = 0; q < NG; q++) {
-        const int n = WIDE ? 128 * q + 8 * i16 : 8 * (i16 & 7);
-        boff[q] = n0 + n < N ? n : 0; // N % 8 == 0: all of the lane's columns or none
-    }
+    for (int q = 0; q < TQ; q++) boff[q] = n0 + 64 * q + 8 * (lane & 7) < N ? 64 * q + 8 * (lane & 7) : 0;
+
+    unsigned char *const a_tile = lds[wave], *const b_tile = lds[wave] + A_BYTES;
+    const uint32_t a_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)a_tile; // a multiple of 1024
+    const int oct = lane >> 3, c8 = lane & 7, row0 = (8 * (oct >> 1) + (oct & 1)) * 128;
+    unsigned char *const put_even = b_tile + row0 + c8 * 16, *const put_odd = b_tile + row0 + (c8 ^ 1) * 16; // entry j: + j * 256
+    const int swap = (i16 >> 3) & 1;
+    const unsigned char *const get = b_tile + (8 * g + (i16 >> 2)) * 128 + (i16 & 3) * 32;
+    const unsigned char *const get01 = get + 16 * swap, *const get23 = get - 16 * swap; // tiles 0, 1 and 2, 3: + t * 8
 
     f32x4 acc[TQ][4];
+    auto clear_acc = [&] {
 #pragma unroll
-    for (int q = 0; q < TQ; q++)
+        for (int q = 0; q < TQ; q++)
 #pragma unroll
-        for (int t = 0; t < 4; t++) acc[q][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < 4; t++) acc[q][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    };
+    clear_acc();
 
-    // Software pipeline over steps of 32 columns (items start and end on multiples of 32): the
-    // column indices of step s+2, then the operands of step s+1 (whose indices arrived a step
-    // ago) are requested before the MFMAs of step s.  Loads past the end of the item read the
-    // next item's data or the padding behind the arrays: always valid addresses, never used.
-    struct Entries { u32x4 r[PAIRED ? 1 : 2]; }; // the indices of a group of 8: entries 0, 2, 4, 6, then 1, 3, 5, 7
-    struct Operands { u32x4 aw; u32x4 L[NG][PAIRED ? 4 : 8]; };
-    auto load_entries = [&](int e, Entries &x) {
-        const u32x4 *lp = reinterpret_cast<const u32x4 *>(cols + e + 8 * g); // the 128-column panel; the other has its own loop
-        x.r[0] = lp[0];
-        if constexpr (!PAIRED) x.r[1] = lp[1];
+    struct Operands {
+        u32x4 aw;                  // AF = 0
+        uint32_t ent[AF ? AF : 1]; // AF > 0
+        int n;                     // the step's entries
+        u32x4 L[TQ][4];
     };
-    auto load_operands = [&](int e, const Entries &x, Operands &o) {
-        o.aw = *reinterpret_cast<const u32x4 *>(acol + ((long)(e >> 3) + g) * 128 + i16 * 8);
-        if constexpr (PAIRED) {
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                o.L[0][j] = *reinterpret_cast<const u32x4 *>(Bp + (long)x.r[0][j] * row_stride + boff[0]); // entry 2j or 2j + 1
-        } else {
-#pragma unroll
-            for (int q = 0; q < NG; q++)
-#pragma unroll
-                for (int j = 0; j < 8; j++)
-                    o.L[q][j] = *reinterpret_cast<const u32x4 *>(Bp + (long)x.r[j & 1][j >> 1] * row_stride + boff[q]);
-        }
-    };
-    auto multiply = [&](const Operands &o) {
-        const f16x8 av = __builtin_bit_cast(f16x8, o.aw);
-        if constexpr (WIDE) {
-#pragma unroll
-            for (int q = 0; q < NG; q++)
-#pragma unroll
-                for (int t = 0; t < 8; t++) { // tile t of the group takes the t-th of the lane's eight columns
-                    u32x4 b;
-#pragma unroll
-                    for (int p = 0; p < 4; p++)
-                        b[p] = __builtin_amdgcn_perm(o.L[q][2 * p + 1][t >> 1], o.L[q][2 * p][t >> 1], (t & 1) ? 0x07060302u : 0x05040100u);
-                    acc[2 * q + (t >> 2)][t & 3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, b), av, acc[2 * q + (t >> 2)][t & 3], 0, 0, 0);
-                }
-        } else {
-            // Lane i16 < 8 holds columns 8 i16 .. + 7 of the even entries, lane i16 + 8 the same columns of the odd
-            // entries.  Each sends the half the other needs (row rotation by 8 lanes) and ends up with 4 columns of
-            // both entries of every pair: columns 8 (i16 & 7) + 4 (i16 >> 3) + t, t = tile.
-            u32x4 b[4];
-#pragma unroll
-            for (int p = 0; p < 4; p++) {
-                const u32x4 x = o.L[0][p];
-                const uint32_t s0 = odd_entries ? x[0] : x[2], s1 = odd_entries ? x[1] : x[3];
-                const uint32_t k0 = odd_entries ? x[2] : x[0], k1 = odd_entries ? x[3] : x[1];
-                const uint32_t r0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)s0, 0x128, 0xf, 0xf, false); // row_ror:8
-                const uint32_t r1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)s1, 0x128, 0xf, 0xf, false);
-                const uint32_t ev0 = odd_entries ? r0 : k0, ev1 = odd_entries ? r1 : k1; // entry 2p
-                const uint32_t od0 = odd_entries ? k0 : r0, od1 = odd_entries ? k1 : r1; // entry 2p + 1
-                b[0][p] = __builtin_amdgcn_perm(od0, ev0, 0x05040100u);
-                b[1][p] = __builtin_amdgcn_perm(od0, ev0, 0x07060302u);
-                b[2][p] = __builtin_amdgcn_perm(od1, ev1, 0x05040100u);
-                b[3][p] = __builtin_amdgcn_perm(od1, ev1, 0x07060302u);
-            }
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-                acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, b[t]), av, acc[0][t], 0, 0, 0);
-        }
-    };
-    if constexpr (PAIRED) {
-        // The index loads of 8 steps in one instruction (an instruction that brings 128 bytes costs the vector memory
-        // path as much as one that brings 1 KiB): lane (i16, g) asks for the four indices that its kind of lane (group g,
-        // even or odd entries) needs at step i16 & 7 of a block of 8 steps; at step k of the block every lane takes them
-        // from the lane that holds step k, with one DPP row broadcast per half of the 16-lane row and word.  Blocks are
-        // asked for one block ahead; what lies past the end of the item is the next item's list or the padding.
-        if (e0 < e1) {
-            auto load_block = [&](int e, u32x4 &x) {
-                x = *reinterpret_cast<const u32x4 *>(cols + e + 32 * (i16 & 7) + 8 * g + (odd_entries ? 4 : 0));
-            };
-            auto indices = [&](const u32x4 &x, auto kc, Entries &out) {
-                constexpr int K = decltype(kc)::value;
-#pragma unroll
-                for (int w = 0; w < 4; w++) {
-                    int r = __builtin_amdgcn_update_dpp(0, (int)x[w], 0x150 + K, 0xf, 0x3, false); // row_newbcast:K     -> lanes 0-7 of the row
-                    r = __builtin_amdgcn_update_dpp(r, (int)x[w], 0x150 + 8 + K, 0xf, 0xc, false); // row_newbcast:8 + K -> lanes 8-15
-                    out.r[0][w] = (uint32_t)r;
-                }
-            };
-            u32x4 blk_a, blk_b;
-            Entries ent;
-            Operands op_a, op_b;
-            load_block(e0, blk_a);
-            load_block(e0 + 256, blk_b);
-            indices(blk_a, std::integral_constant<int, 0>{}, ent);
-            load_operands(e0, ent, op_a);
-            int e = e0;
-            while (true) {
-#define SMAT_TWO_STEPS(KA, KB, BLK_B)                                                                  \
-                indices(blk_a, std::integral_constant<int, KA>{}, ent);                                \
-                load_operands(e + 32, ent, op_b);                                                      \
-                multiply(op_a);                                                                        \
-                e += 32;                                                                               \
-                if (e >= e1) break;                                                                    \
-                indices(BLK_B, std::integral_constant<int, KB>{}, ent);                                \
-                load_operands(e + 32, ent, op_a);                                                      \
-                multiply(op_b);                                                                        \
-                e += 32;                                                                               \
-                if (e >= e1) break;
-                SMAT_TWO_STEPS(1, 2, blk_a)
-                SMAT_TWO_STEPS(3, 4, blk_a)
-                SMAT_TWO_STEPS(5, 6, blk_a)
-                SMAT_TWO_STEPS(7, 0, blk_b)
-#undef SMAT_TWO_STEPS
-                blk_a = blk_b;
-                load_block(e + 256, blk_b);
-            }
-        }
-    } else if (e0 < e1) {
-        Entries ent_a, ent_b;
-        Operands op_a, op_b;
-        load_entries(e0, ent_a);
-        load_entries(e0 + 32, ent_b);
-        load_operands(e0, ent_a, op_a);
-        int e = e0;
-        while (true) {
-            load_entries(e + 64, ent_a);
-            load_operands(e + 32, ent_b, op_b);
-            multiply(op_a);
-            e += 32;
-            if (e >= e1) break;
-            load_entries(e + 64, ent_b);
-            load_operands(e + 32, ent_a, op_a);
-            multiply(op_b);
-            e += 32;
-            if (e >= e1) break;
-        }
+    int2 ranges = {0, 0}; // entries of the steps from range_base + lane on: a task has at most MAX_TASK_STEPS
+    const int range_base = e >> 5;
+    if constexpr (AF > 0) {
+        *reinterpret_cast<u32x4 *>(a_tile + lane * 16) = (u32x4){0u, 0u, 0u, 0u};
+        ranges = step_range[range_base + lane];
     }
-
-    const long m = (long)br * 16 + i16;
-    if constexpr (WIDE) {
-        // tile t8 = 4 * (q & 1) + t of group q / 2: acc[q][t][r] = C[br*16 + i16][n0 + 128 (q/2) + 32g + 8r + t8]
-#pragma unroll
-        for (int q2 = 0; q2 < NG; q2++) {
-            const int c0 = n0 + 128 * q2 + 32 * g;
-            float o[32];
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-#pragma unroll
-                for (int t = 0; t < 8; t++) o[8 * r + t] = acc[2 * q2 + (t >> 2)][t & 3][r];
-            if (dst >= 0 || C_F32) {
-                float *row = dst >= 0 ? workspace + ((long)dst * 16 + i16) * (long)N
-                                      : reinterpret_cast<float *>(Cout) + m * (long)N;
-#pragma unroll
-                for (int h = 0; h < 8; h++)
-                    if (c0 + 4 * h < N) {
-                        f32x4 v = {o[4 * h], o[4 * h + 1], o[4 * h + 2], o[4 * h + 3]};
-                        if (C_ACC && dst < 0) v += *reinterpret_cast<const f32x4 *>(row + c0 + 4 * h);
-                        *reinterpret_cast<f32x4 *>(row + c0 + 4 * h) = v;
-                    }
-            } else {
-                uint16_t *row = reinterpret_cast<uint16_t *>(Cout) + m * (long)N;
-#pragma unroll
-                for (int h = 0; h < 4; h++) {
-                    if (c0 + 8 * h >= N) continue;
-                    f16x8 v;
-                    if (C_ACC) {
-                        const f16x8 old = *reinterpret_cast<const f16x8 *>(row + c0 + 8 * h);
-#pragma unroll
-                        for (int j = 0; j < 8; j++) v[j] = (_Float16)(o[8 * h + j] + (float)old[j]);
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 8; j++) v[j] = (_Float16)o[8 * h + j];
-                    }
-                    *reinterpret_cast<f16x8 *>(row + c0 + 8 * h) = v;
-                }
-            }
-        }
-    } else {
-        // acc[0][t][r] = C[br*16 + i16][n0 + cb + t] with cb = 32 g + 8 r (g < 2) or 32 (g - 2) + 8 r + 4 (g >= 2): lane
-        // (i16, g) and lane (i16, g + 2) hold the two halves of the same 8-column groups.  One swap per value between
-        // the halves of the wavefront (the lower lanes hand over r = 2, 3 and get r = 0, 1) leaves every lane with 16
-        // consecutive columns, starting at 32 (g & 1) + 16 (g >> 1).
-        float o[16];
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int rr = 0; rr < 2; rr++) {
-                const float lo = acc[0][t][rr], hi = acc[0][t][rr + 2]; // scalars first: a bit cast of a vector element reads element 0
-                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
-                o[8 * rr + t] = __uint_as_float((uint32_t)sw[0]);
-                o[8 * rr + 4 + t] = __uint_as_float((uint32_t)sw[1]);
-            }
-        const int c0 = n0 + 32 * (g & 1) + 16 * (g >> 1);
-        if (dst >= 0 || C_F32) {
-            float *row = dst >= 0 ? workspace + ((long)dst * 16 + i16) * (long)N
-                                  : reinterpret_cast<float *>(Cout) + m * (long)N;
-#pragma unroll
-            for (int h = 0; h < 4; h++)
-                if (c0 + 4 * h < N) {
-                    f32x4 v = {o[4 * h], o[4 * h + 1], o[4 * h + 2], o[4 * h + 3]};
-                    if (C_ACC && dst < 0) v += *reinterpret_cast<const f32x4 *>(row + c0 + 4 * h);
-                    *reinterpret_cast<f32x4 *>(row + c0 + 4 * h) = v;
-                }
+    // The indices of 8 steps are 1 KiB, one load, and go to one half of 2 KiB of LDS, from where each lane takes the four of
+    // its octet (an instruction that brings 128 bytes costs the vector memory path as much as one that brings 1 KiB).
+    unsigned char *const i_tile = lds[wave] + A_BYTES + B_BYTES;
+    auto load_block = [&](int s) { return reinterpret_cast<const u32x4 *>(cols + s)[lane]; };
+    auto put_block = [&](int s, u32x4 x) { *reinterpret_cast<u32x4 *>(i_tile + (((s >> 5) - range_base) & 8) * 128 + lane * 16) = x; };
+    auto indices = [&](int s) { return *reinterpret_cast<const u32x4 *>(i_tile + (((s >> 5) - range_base) & 15) * 128 + oct * 16); };
+    auto request = [&](int s, const u32x4 x, Operands &o) {
+        if constexpr (AF == 0) {
+            o.aw = *reinterpret_cast<const u32x4 *>(acol + ((long)(s >> 3) + g) * 128 + i16 * 8);
         } else {
-            uint16_t *row = reinterpret_cast<uint16_t *>(Cout) + m * (long)N;
+            const int first = __builtin_amdgcn_readlane(ranges.x, (s >> 5) - range_base);
+            o.n = __builtin_amdgcn_readlane(ranges.y, (s >> 5) - range_base) - first;
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                if (c0 + 8 * h >= N) continue;
-                f16x8 v;
-                if (C_ACC) {
-                    const f16x8 old = *reinterpret_cast<const f16x8 *>(row + c0 + 8 * h);
-#pragma unroll
-                    for (int j = 0; j < 8; j++) v[j] = (_Float16)(o[8 * h + j] + (float)old[j]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 8; j++) v[j] = (_Float16)o[8 * h + j];
-                }
-                *reinterpret_cast<f16x8 *>(row + c0 + 8 * h) = v;
-            }
+            for (int u = 0; u < AF; u++) o.ent[u] = (entries + (long)first + 64 * u)[lane]; // past the step's end: the next step's, unused
         }
+        if constexpr (BIG) {
+            const long stride = s < e_last ? row_stride : 0;
+#pragma unroll
+            for (int q = 0; q < TQ; q++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) o.L[q][j] = *reinterpret_cast<const u32x4 *>(Bp + (long)x[j] * stride + boff[q]);
+        } else {
+            const uint32_t stride = s < e_last ? (uint32_t)row_stride * 2u : 0u;
+#pragma unroll
+            for (int q = 0; q < TQ; q++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    o.L[q][j] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const unsigned char *>(Bp) +
+                                                                 (size_t)(uint32_t)(__umul24(x[j], stride) + (uint32_t)boff[q] * 2u));
+        }
+    };
+    auto a_operand = [&](const Operands &o) {
+        if constexpr (AF == 0) return __builtin_bit_cast(f16x8, o.aw);
+        typedef __attribute__((address_space(3))) uint16_t lds_half;
+        auto put = [&](bool clear) {
+#pragma unroll
+            for (int u = 0; u < AF; u++)
+                if (64 * u + lane < o.n) *(lds_half *)(uintptr_t)((o.ent[u] & 0x3ffu) | a_base) = clear ? (uint16_t)0 : (uint16_t)(o.ent[u] >> 16);
+        };
+        put(false);
+        asm volatile("" ::: "memory");
+        const f16x8 av = *reinterpret_cast<const f16x8 *>(a_tile + lane * 16);
+        asm volatile("" ::: "memory");
+        put(true);
+        return av;
+    };
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    auto multiply = [&](const Operands &o) {
+        const f16x8 av = a_operand(o);
+#pragma unroll
+        for (int q = 0; q < TQ; q++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) *reinterpret_cast<u32x4 *>((j & 1 ? put_odd : put_even) + q * 4096 + j * 256) = o.L[q][j];
+        asm volatile("" ::: "memory");
+        f16x8 b[TQ][4];
+#pragma unroll
+        for (int q = 0; q < TQ; q++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const unsigned char *p = (t < 2 ? get01 : get23) + q * 4096 + t * 8;
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p);
+                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(p + 512));
+                b[q][t] = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int q = 0; q < TQ; q++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[q][t], av, acc[q][t], 0, 0, 0);
+    };
+    // The tile of item `it` goes out (acc[q][t][r] = C[16 br + i16][n0 + 64 q + 16 g + 4 t + r]); the next item that has
+    // steps is the current one afterwards.
+    auto finish = [&] {
+        do {
+            const long m = (long)br * 16 + i16;
+#pragma unroll
+            for (int q = 0; q < TQ; q++) {
+                const int c0 = n0 + 64 * q + 16 * g;
+                if (dst >= 0 || C_F32) {
+                    float *row = dst >= 0 ? workspace + ((long)dst * 16 + i16) * (long)N
+                                          : reinterpret_cast<float *>(Cout) + m * (long)N;
+#pragma unroll
+                    for (int t = 0; t < 4; t++)
+                        if (c0 + 4 * t < N) {
+                            f32x4 v = acc[q][t];
+                            if (C_ACC && dst < 0) v += *reinterpret_cast<const f32x4 *>(row + c0 + 4 * t);
+                            *reinterpret_cast<f32x4 *>(row + c0 + 4 * t) = v;
+                        }
+                } else {
+                    uint16_t *row = reinterpret_cast<uint16_t *>(Cout) + m * (long)N;
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        if (c0 + 8 * h >= N) continue;
+                        f16x8 v;
+                        if (C_ACC) {
+                            const f16x8 old = *reinterpret_cast<const f16x8 *>(row + c0 + 8 * h);
+#pragma unroll
+                            for (int j = 0; j < 8; j++) v[j] = (_Float16)(acc[q][2 * h + j / 4][j % 4] + (float)old[j]);
+                        } else {
+#pragma unroll
+                            for (int j = 0; j < 8; j++) v[j] = (_Float16)acc[q][2 * h + j / 4][j % 4];
+                        }
+                        *reinterpret_cast<f16x8 *>(row + c0 + 8 * h) = v;
+                    }
+                }
+            }
+            clear_acc();
+            if (++it < tk.y) enter();
+        } while (it < tk.y && item_end == e);
+    };
+    if (item_end == e) finish(); // block rows without a step: zeros
+    if (it >= tk.y) return;
+
+    Operands op_a, op_b;
+    u32x4 block = load_block(e); // of the 8 steps after those in LDS
+    put_block(e, block);
+    block = load_block(e + 256);
+    asm volatile("" ::: "memory");
+    request(e, indices(e), op_a);
+    int next = e + 32; // the step whose operands are asked for
+    u32x4 x = indices(next); // read from LDS a step before they are used
+    while (true) {
+#define SMAT_STEP_OF(CUR, NEW)                                                                         \
+        if (((next + 32 - tk.z) & 255) == 0) {                                                         \
+            put_block(next + 32, block);                                                               \
+            block = load_block(next + 288);                                                            \
+        }                                                                                              \
+        asm volatile("" ::: "memory");                                                                 \
+        request(next, x, NEW);                                                                         \
+        x = indices(next + 32);                                                                        \
+        multiply(CUR);                                                                                 \
+        e = next;                                                                                      \
+        next += 32;                                                                                    \
+        if (e == item_end) {                                                                           \
+            finish();                                                                                  \
+            if (it >= tk.y) break;                                                                     \
+        }
+        SMAT_STEP_OF(op_a, op_b)
+        SMAT_STEP_OF(op_b, op_a)
+#undef SMAT_STEP_OF
     }
 }
 
@@ -544,10 +577,10 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
         panel_stride = (long)a.K * PANEL;
         row_stride = PANEL;
     }
-    const long total = (long)p.n_items * n_panels;
+    const long total = (long)p.n_tasks * n_panels;
     long wgs = (total + 3) / 4;
     if (wgs == 0) return hipSuccess;
-    long xcd_run = p.deal.run((size_t)p.n_items, n_panels);
+    long xcd_run = p.deal.run((size_t)p.n_tasks, n_panels);
     if (p.tuned_run > 0 && p.tuned_n == a.N) xcd_run = p.tuned_run;
     if (a.xcd_run > 0) xcd_run = a.xcd_run;
     if (g_force_run > 0) xcd_run = g_force_run;
@@ -556,15 +589,28 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
     wgs = (wgs + 8 * xcd_run - 1) / (8 * xcd_run) * (8 * xcd_run);
     if (wgs > 0x7fffffffL) return hipErrorInvalidValue;
     if (a.accumulate && p.n_split_rows > 0) return hipErrorInvalidValue; // partial tiles through the workspace overwrite C
-#define SMAT_LAUNCH_COMPACT(F32, ACC)                                                                                           \
-    hipLaunchKernelGGL((spmm_compact_kernel<TQ, F32, ACC>), dim3((unsigned)wgs), dim3(256), 0, st, p.d_acol, p.d_cols, a.Bt, a.C, \
-                       p.d_workspace, p.d_items, p.n_items, (int)a.N, n_panels, panel_stride, row_stride, (unsigned)xcd_run)
-    if (a.c_f32) {
-        if (a.accumulate) SMAT_LAUNCH_COMPACT(true, true); else SMAT_LAUNCH_COMPACT(true, false);
-    } else {
-        if (a.accumulate) SMAT_LAUNCH_COMPACT(false, true); else SMAT_LAUNCH_COMPACT(false, false);
-    }
-#undef SMAT_LAUNCH_COMPACT
+    // 32-bit byte offsets from indices of 24 bits
+    const bool big = a.K > ((size_t)1 << 24) || a.K * (size_t)row_stride * 2 >= ((size_t)1 << 32) || row_stride >= (1L << 23);
+    auto launch = [&](auto af, auto f32, auto acc, auto wide) {
+        hipLaunchKernelGGL((spmm_compact_kernel<TQ, decltype(f32)::value, decltype(acc)::value, decltype(af)::value, decltype(wide)::value>),
+                           dim3((unsigned)wgs), dim3(256), 0, st, p.d_acol, p.d_entries, p.d_step_range, p.d_cols, a.Bt, a.C, p.d_workspace,
+                           p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, (unsigned)xcd_run);
+    };
+    using std::false_type;
+    using std::true_type;
+    auto by_output = [&](auto af, auto wide) {
+        if (a.c_f32) {
+            if (a.accumulate) launch(af, true_type{}, true_type{}, wide); else launch(af, true_type{}, false_type{}, wide);
+        } else {
+            if (a.accumulate) launch(af, false_type{}, true_type{}, wide); else launch(af, false_type{}, false_type{}, wide);
+        }
+    };
+    auto by_entries = [&](auto wide) {
+        if (p.d_acol) by_output(std::integral_constant<int, 0>{}, wide);
+        else if (p.entries_ahead == 1) by_output(std::integral_constant<int, 1>{}, wide);
+        else by_output(std::integral_constant<int, 2>{}, wide);
+    };
+    if (big) by_entries(true_type{}); else by_entries(false_type{});
     return hipGetLastError();
 }
 
@@ -645,9 +691,9 @@ hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t
     // the run length of an untuned launch, as launch_compact_tq computes it for this N
     const int tq = compact_panel_width(p, N, K);
     const int n_panels = (int)((N + 64 * tq - 1) / (64 * tq));
-    const long wgs = ((long)p.n_items * n_panels + 3) / 4;
+    const long wgs = ((long)p.n_tasks * n_panels + 3) / 4;
     const unsigned eighth = (unsigned)std::max<long>((wgs + 7) / 8, 1);
-    const unsigned base = std::min(eighth, p.deal.run((size_t)p.n_items, n_panels));
+    const unsigned base = std::min(eighth, p.deal.run((size_t)p.n_tasks, n_panels));
     float t_base = 0.f;
     if (e == hipSuccess) e = time_of(base, 1, &t_base);
     if (e == hipSuccess && t_base <= 20.f) {
@@ -655,7 +701,7 @@ hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t
         if (base * 4 >= eighth) // a list that the estimate finds even: the longer runs are worth a try
             for (unsigned r : {eighth, eighth / 2, eighth / 4})
                 if (r >= 4 && std::find(runs.begin(), runs.end(), r) == runs.end()) runs.push_back(r);
-        const int launches = t_base < 0.2f ? 20 : t_base < 2.f ? 6 : 3;
+        const int launches = t_base < 0.2f ? 6 : 3;
         unsigned best_run = base;
         float best = 0.f;
         for (size_t i = 0; i < runs.size() && e == hipSuccess; i++) {
@@ -676,16 +722,16 @@ hipError_t values_checksum(const uint16_t *vals, size_t nnzb, uint64_t *out)
     *out = 0;
     if (!nnzb) return hipSuccess;
     DevScratch d;
-    hipError_t e = d.alloc(CHECKSUM_BYTES);
-    if (e == hipSuccess) e = hipMemsetAsync(d.p, 0, CHECKSUM_BYTES, nullptr);
+    hipError_t e = d.alloc(SUM_BYTES);
+    if (e == hipSuccess) e = hipMemsetAsync(d.p, 0, SUM_BYTES, nullptr);
     if (e != hipSuccess) return e;
     const long n_quads = (long)nnzb * 32;
     const unsigned blocks = (unsigned)std::min<long>((n_quads + 255) / 256, 256L * 8);
     hipLaunchKernelGGL(values_checksum_kernel, dim3(blocks), dim3(256), 0, 0, reinterpret_cast<const u32x4 *>(vals), n_quads, (unsigned long long *)d.p);
     e = hipGetLastError();
-    std::vector<unsigned long long> sums(CHECKSUM_BYTES / sizeof(unsigned long long));
-    if (e == hipSuccess) e = hipMemcpy(sums.data(), d.p, CHECKSUM_BYTES, hipMemcpyDeviceToHost);
-    if (e == hipSuccess) *out = total_checksum(sums);
+    unsigned long long sum = 0;
+    if (e == hipSuccess) e = fetch_totals(d.p, &sum, 1);
+    if (e == hipSuccess) *out = sum;
     return e;
 }
 
@@ -694,7 +740,10 @@ void compact_destroy(CompactPlan *p)
     if (!p) return;
     if (p->d_cols) (void)dev_free(p->d_cols);
     if (p->d_acol) (void)dev_free(p->d_acol);
+    if (p->d_entries) (void)dev_free(p->d_entries);
+    if (p->d_step_range) (void)dev_free(p->d_step_range);
     if (p->d_items) (void)dev_free(p->d_items);
+    if (p->d_tasks) (void)dev_free(p->d_tasks);
     if (p->d_split) (void)dev_free(p->d_split);
     if (p->d_workspace) (void)dev_free(p->d_workspace);
     delete p;
@@ -713,98 +762,184 @@ hipError_t copy_blocks(const uint16_t *vals, const int32_t *ids_host, size_t n, 
     return e;
 }
 
-hipError_t compact_build(const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx,
-                         const int32_t *row_ptr_host, size_t mb, size_t nnzb, size_t n_cap, double dense_share,
-                         std::vector<uint8_t> *dense_rows, CompactPlan **out, const uint8_t *skip_blocks_host,
-                         std::vector<uint8_t> *block_cols)
-{
-    *out = nullptr;
-    CompactPlan *p = new (std::nothrow) CompactPlan();
-    if (!p) return hipErrorOutOfMemory;
-    hipError_t e = hipSuccess;
-    Scratch mask, count, offset, tmp, cc, sums;
 #define SMAT_STEP(call)                                                                            \
     do {                                                                                           \
         if (e == hipSuccess) e = (call);                                                           \
     } while (0)
-    SMAT_STEP(mask.alloc(nnzb * 2));
-    SMAT_STEP(count.alloc(nnzb * 4));
-    SMAT_STEP(offset.alloc(nnzb * 4));
-    SMAT_STEP(cc.alloc((mb + 1) * 4));
-    SMAT_STEP(sums.alloc(CHECKSUM_BYTES));
-    SMAT_STEP(hipMemsetAsync(sums.p, 0, CHECKSUM_BYTES, nullptr));
-    int64_t n_cols = 0;
-    std::vector<int32_t> raw(mb + 1, 0), padded(mb + 1, 0);
-    if (e == hipSuccess && nnzb) {
+
+// count -> offset (exclusive sums), rows (what the blocks before every block row hold) and raw, its copy on the host
+static hipError_t census_offsets(CompactCensus &s, const int32_t *row_ptr)
+{
+    hipError_t e = hipSuccess;
+    Scratch tmp;
+    size_t bytes = 0;
+    auto *count = static_cast<unsigned long long *>(s.count.p), *offset = static_cast<unsigned long long *>(s.offset.p);
+    SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, count, offset, (int)s.nnzb));
+    SMAT_STEP(tmp.alloc(bytes));
+    SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, count, offset, (int)s.nnzb));
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(row_offsets_kernel, dim3((unsigned)((s.mb + 1 + 255) / 256)), dim3(256), 0, 0, row_ptr, offset, count, (long)s.mb,
+                           (long)s.nnzb, (unsigned long long *)s.rows.p);
+        e = hipGetLastError();
+    }
+    SMAT_STEP(hipMemcpy(s.raw.data(), s.rows.p, (s.mb + 1) * 8, hipMemcpyDeviceToHost));
+    return e;
+}
+
+hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t mb, size_t nnzb, CompactCensus &s)
+{
+    hipError_t e = hipSuccess;
+    s.mb = mb;
+    s.nnzb = nnzb;
+    s.raw.assign(mb + 1, 0);
+    if (!nnzb) return e;
+    Scratch sums;
+    for (Scratch *q : {&s.mask, &s.count, &s.offset, &s.rows}) q->release();
+    s.dropped = false;
+    SMAT_STEP(s.mask.alloc(nnzb * 2));
+    SMAT_STEP(s.count.alloc(nnzb * 8));
+    SMAT_STEP(s.offset.alloc(nnzb * 8));
+    SMAT_STEP(s.rows.alloc((mb + 1) * 8));
+    SMAT_STEP(sums.alloc(SUM_BYTES));
+    SMAT_STEP(hipMemsetAsync(sums.p, 0, SUM_BYTES, nullptr));
+    if (e == hipSuccess) {
         const long waves = std::min<long>((long)(nnzb + 1) / 2, 256L * 32);
         hipLaunchKernelGGL(colmask_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, 0, vals, (long)nnzb,
-                           (uint16_t *)mask.p, (int32_t *)count.p, (unsigned long long *)sums.p);
+                           (uint16_t *)s.mask.p, (unsigned long long *)s.count.p, (unsigned long long *)sums.p);
         e = hipGetLastError();
-        if (block_cols) { // nonzero columns of every block, for the caller's choice of a split
-            std::vector<int32_t> cnt(nnzb);
-            SMAT_STEP(hipMemcpy(cnt.data(), count.p, nnzb * 4, hipMemcpyDeviceToHost));
-            block_cols->resize(nnzb);
-            for (size_t i = 0; i < nnzb; i++) (*block_cols)[i] = (uint8_t)cnt[i];
-        }
-        if (skip_blocks_host && e == hipSuccess) {
-            Scratch skip;
-            SMAT_STEP(skip.alloc(nnzb));
-            SMAT_STEP(hipMemcpy(skip.p, skip_blocks_host, nnzb, hipMemcpyHostToDevice));
-            if (e == hipSuccess) {
-                hipLaunchKernelGGL(drop_blocks_kernel, dim3((unsigned)((nnzb + 255) / 256)), dim3(256), 0, 0, (const uint8_t *)skip.p,
-                                   (long)nnzb, (uint16_t *)mask.p, (int32_t *)count.p);
-                e = hipGetLastError();
-            }
-            SMAT_STEP(hipDeviceSynchronize()); // skip goes out of scope
-        }
-        size_t bytes = 0;
-        SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, (int32_t *)count.p, (int32_t *)offset.p, (int)nnzb));
-        SMAT_STEP(tmp.alloc(bytes));
-        SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, (int32_t *)count.p, (int32_t *)offset.p, (int)nnzb));
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(row_offsets_kernel, dim3((unsigned)((mb + 1 + 255) / 256)), dim3(256), 0, 0, row_ptr,
-                               (const int32_t *)offset.p, (const int32_t *)count.p, (long)mb, (long)nnzb, (int32_t *)cc.p);
-            e = hipGetLastError();
-        }
-        SMAT_STEP(hipMemcpy(raw.data(), cc.p, (mb + 1) * 4, hipMemcpyDeviceToHost));
-        n_cols = raw[mb];
     }
-    // Block rows whose blocks are mostly full (at least dense_share of their 16 x blocks columns are nonzero) are
-    // left to a dense kernel when the caller asks for the split: they get no list and no work item here.
-    std::vector<uint8_t> dense(mb, 0);
-    p->n_cols_all = n_cols;
-    if (dense_rows && dense_share > 0.0)
-        for (size_t i = 0; i < mb; i++) {
-            const int64_t blocks = row_ptr_host[i + 1] - row_ptr_host[i];
-            if (blocks > 0 && (double)(raw[i + 1] - raw[i]) >= dense_share * 16.0 * (double)blocks) {
-                dense[i] = 1;
-                n_cols -= raw[i + 1] - raw[i];
-            }
-        }
-    p->n_cols = n_cols;
-    // every block row is padded to a multiple of 32 columns (one MFMA step); padding = zero columns
-    int64_t total = 0;
-    std::vector<int32_t> padded_dev(mb + 1, 0); // what the gather kernel sees: -1 for rows without a list
+    SMAT_STEP(census_offsets(s, row_ptr));
+    unsigned long long total[N_SUMS] = {0};
+    SMAT_STEP(fetch_totals(sums.p, total, N_SUMS));
+    s.values_checksum = total[SUM_CHECK];
+    s.full_blocks = (int64_t)total[SUM_FULL];
+    s.cols_rest = (int64_t)total[SUM_COLS_REST];
+    s.nnz = (int64_t)total[SUM_NNZ];
+    s.n_cols_all = (int64_t)(uint32_t)s.raw[mb];
+    return e;
+}
+
+hipError_t compact_full_blocks(const CompactCensus &s, std::vector<uint8_t> &full)
+{
+    std::vector<uint16_t> mask(s.nnzb);
+    full.assign(s.nnzb, 0);
+    if (!s.nnzb) return hipSuccess;
+    const hipError_t e = hipMemcpy(mask.data(), s.mask.p, s.nnzb * 2, hipMemcpyDeviceToHost);
+    for (size_t i = 0; i < s.nnzb; i++) full[i] = __builtin_popcount(mask[i]) >= FULL_BLOCK_COLS;
+    return e;
+}
+
+hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx, size_t K, size_t n_cap,
+                         const std::vector<uint8_t> *leave_rows, bool drop_full, CompactPlan **out)
+{
+    *out = nullptr;
+    const size_t mb = s.mb, nnzb = s.nnzb;
+    CompactPlan *p = new (std::nothrow) CompactPlan();
+    if (!p) return hipErrorOutOfMemory;
+    hipError_t e = hipSuccess;
+    if (drop_full && nnzb && !s.dropped) {
+        hipLaunchKernelGGL(drop_full_kernel, dim3((unsigned)((nnzb + 255) / 256)), dim3(256), 0, 0, (const uint16_t *)s.mask.p, (long)nnzb,
+                           (unsigned long long *)s.count.p);
+        e = hipGetLastError();
+        SMAT_STEP(census_offsets(s, row_ptr));
+        s.dropped = true;
+    }
+    p->values_checksum = s.values_checksum;
+    p->n_cols_all = s.n_cols_all;
+    std::vector<uint8_t> none;
+    const std::vector<uint8_t> &dense = leave_rows ? *leave_rows : (none.assign(mb, 0), none);
+    // Block rows left to a dense kernel get no list and no work item here; the others are padded to a multiple of 32
+    // columns (one MFMA step) with zero columns.
+    int64_t total = 0, n_cols = 0, nnz = 0;
+    std::vector<int32_t> padded(mb + 1, 0);
+    std::vector<int2> start(mb + 1); // what the gather kernel sees: list and entries of the row, -1 for rows without a list
     for (size_t i = 0; i < mb; i++) {
         padded[i] = (int32_t)total;
-        padded_dev[i] = dense[i] ? -1 : (int32_t)total;
-        if (!dense[i]) total += ((int64_t)(raw[i + 1] - raw[i]) + 31) / 32 * 32;
+        start[i] = dense[i] ? int2{-1, 0} : int2{(int32_t)total, (int32_t)nnz};
+        if (!dense[i]) {
+            const uint64_t d = s.raw[i + 1] - s.raw[i];
+            total += ((int64_t)(uint32_t)d + 31) / 32 * 32;
+            n_cols += (int64_t)(uint32_t)d;
+            nnz += (int64_t)(d >> 32);
+        }
         if (total > 0x7fffff00) e = hipErrorInvalidValue;
     }
     padded[mb] = (int32_t)total;
-    padded_dev[mb] = (int32_t)total;
+    start[mb] = int2{(int32_t)total, (int32_t)nnz};
+    p->n_cols = n_cols;
+    // The nonzeros one by one (4 bytes each, and 8 per step) while that is at most half of the 32 bytes per column that
+    // whole columns take: about one nonzero per column in random sparse matrices (a step of 36 entries: 152 bytes for
+    // 1024), 2.8 in the 27-point stencil (368 bytes).  Where the panels of B are small enough to stay in the L2 (K up to
+    // 4096) it is the LDS that binds, and whole columns, which do not go through it, win (24352 x 1376, 22 a row, N = 72:
+    // 13.7 against 14.5 us; 16384^2, N = 256, the other way round: 18.9 against 16.3).
+    const bool by_entry = nnz <= 4 * n_cols && K > 4096 && s.nnz < 0x7fffff00;
     const size_t cap = (size_t)total + LIST_PAD;
     SMAT_STEP(dev_malloc(&p->d_cols, cap * sizeof(int32_t)));
-    SMAT_STEP(hipMemset(p->d_cols, 0, cap * sizeof(int32_t))); // padding: row 0 of B
-    SMAT_STEP(dev_malloc(&p->d_acol, cap * 16 * sizeof(uint16_t)));
-    SMAT_STEP(hipMemset(p->d_acol, 0, cap * 16 * sizeof(uint16_t)));
+    SMAT_STEP(hipMemsetAsync(p->d_cols, 0, cap * sizeof(int32_t), nullptr)); // padding: row 0 of B
+    if (by_entry) {
+        const size_t steps = cap / 32;
+        p->entries_ahead = nnz <= 48 * (total / 32) ? 1 : 2; // most steps have no more than 64 a load
+        SMAT_STEP(dev_malloc(&p->d_entries, ((size_t)nnz + 128) * sizeof(uint32_t)));
+        SMAT_STEP(dev_malloc(&p->d_step_range, steps * sizeof(int2)));
+        SMAT_STEP(hipMemsetAsync(p->d_step_range, 0, steps * sizeof(int2), nullptr)); // the steps read ahead of the last one have no entries
+    } else {
+        SMAT_STEP(dev_malloc(&p->d_acol, cap * 16 * sizeof(uint16_t)));
+        SMAT_STEP(hipMemsetAsync(p->d_acol, 0, cap * 16 * sizeof(uint16_t), nullptr));
+    }
+    Scratch starts;
+    SMAT_STEP(starts.alloc((mb + 1) * sizeof(int2)));
     if (e == hipSuccess && nnzb) {
-        SMAT_STEP(hipMemcpy(cc.p, padded_dev.data(), (mb + 1) * 4, hipMemcpyHostToDevice));
+        SMAT_STEP(hipMemcpy(starts.p, start.data(), (mb + 1) * sizeof(int2), hipMemcpyHostToDevice));
         if (e == hipSuccess) {
-            hipLaunchKernelGGL(gather_kernel, dim3((unsigned)((nnzb + 255) / 256)), dim3(256), 0, 0, vals,
-                               (const uint16_t *)mask.p, (const int32_t *)offset.p, row_ptr, col_idx,
-                               (const int32_t *)cc.p, (long)mb, (long)nnzb, p->d_cols, p->d_acol);
+            hipLaunchKernelGGL(gather_kernel, dim3((unsigned)((nnzb + 255) / 256)), dim3(256), 0, 0, vals, (const uint16_t *)s.mask.p,
+                               (const unsigned long long *)s.offset.p, row_ptr, col_idx, (const unsigned long long *)s.rows.p, (const int2 *)starts.p,
+                               (long)mb, (long)nnzb, drop_full, p->d_cols, p->d_acol, p->d_entries, p->d_step_range);
             e = hipGetLastError();
+        }
+    }
+    if (by_entry && total > 0) { // no step with more entries than the product kernel asks for
+        const int n_groups = (int)(total / 32), most = 64 * p->entries_ahead;
+        const size_t padded_groups = cap / 32;
+        Scratch steps, first, tmp, starts_dev, row_first;
+        size_t bytes = 0;
+        SMAT_STEP(steps.alloc(((size_t)n_groups + 1) * sizeof(int32_t)));
+        SMAT_STEP(first.alloc(((size_t)n_groups + 1) * sizeof(int32_t)));
+        SMAT_STEP(hipMemsetAsync(steps.p, 0, ((size_t)n_groups + 1) * sizeof(int32_t), nullptr));
+        if (e == hipSuccess) {
+            hipLaunchKernelGGL(count_steps_kernel, dim3((unsigned)((n_groups + 255) / 256)), dim3(256), 0, 0, p->d_step_range, n_groups, most, (int32_t *)steps.p);
+            e = hipGetLastError();
+        }
+        SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, (int32_t *)steps.p, (int32_t *)first.p, n_groups + 1));
+        SMAT_STEP(tmp.alloc(bytes));
+        SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, (int32_t *)steps.p, (int32_t *)first.p, n_groups + 1));
+        int32_t n_steps = 0;
+        SMAT_STEP(hipMemcpy(&n_steps, (int32_t *)first.p + n_groups, sizeof n_steps, hipMemcpyDeviceToHost));
+        if (e == hipSuccess && n_steps > n_groups) {
+            if ((int64_t)n_steps * 32 > 0x7fffff00) e = hipErrorInvalidValue;
+            const size_t step_cap = (size_t)n_steps + (padded_groups - (size_t)n_groups);
+            int32_t *cols = nullptr;
+            int2 *range = nullptr;
+            SMAT_STEP(dev_malloc(&cols, step_cap * 32 * sizeof(int32_t)));
+            SMAT_STEP(dev_malloc(&range, step_cap * sizeof(int2)));
+            SMAT_STEP(hipMemsetAsync(cols + (size_t)n_steps * 32, 0, (step_cap - (size_t)n_steps) * 32 * sizeof(int32_t), nullptr));
+            SMAT_STEP(hipMemsetAsync(range + n_steps, 0, (step_cap - (size_t)n_steps) * sizeof(int2), nullptr));
+            SMAT_STEP(starts_dev.alloc((mb + 1) * sizeof(int32_t)));
+            SMAT_STEP(row_first.alloc((mb + 1) * sizeof(int32_t)));
+            SMAT_STEP(hipMemcpy(starts_dev.p, padded.data(), (mb + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
+            if (e == hipSuccess) {
+                hipLaunchKernelGGL(expand_steps_kernel, dim3((unsigned)((n_groups + 7) / 8)), dim3(256), 0, 0, p->d_step_range, p->d_cols,
+                                   (const int32_t *)steps.p, (const int32_t *)first.p, n_groups, most, range, cols);
+                hipLaunchKernelGGL(row_steps_kernel, dim3((unsigned)((mb + 1 + 255) / 256)), dim3(256), 0, 0, (const int32_t *)starts_dev.p,
+                                   (const int32_t *)first.p, (long)mb + 1, (int32_t *)row_first.p);
+                e = hipGetLastError();
+            }
+            SMAT_STEP(hipMemcpy(padded.data(), row_first.p, (mb + 1) * sizeof(int32_t), hipMemcpyDeviceToHost));
+            for (int32_t &v : padded) v *= 32;
+            total = (int64_t)n_steps * 32;
+            (void)dev_free_idle(p->d_cols); // the copy back has waited for the kernels
+            (void)dev_free_idle(p->d_step_range);
+            p->d_cols = cols;
+            p->d_step_range = range;
         }
     }
     // work items: whole block rows; rows much longer than the average in chunks of 32-column steps
@@ -814,7 +949,7 @@ hipError_t compact_build(const uint16_t *vals, const int32_t *row_ptr, const int
     const double avg = nonempty ? (double)total / (double)nonempty : 0.0;
     long chunk = (long)(4.0 * avg + 0.5);
     chunk = std::max(chunk, 512L);
-    chunk = (chunk + 31) / 32 * 32;
+    chunk = std::min((chunk + 31) / 32 * 32, 32L * MAX_TASK_STEPS);
     std::vector<WorkItem> items;
     std::vector<SplitRow> split;
     int slot = 0;
@@ -832,14 +967,29 @@ hipError_t compact_build(const uint16_t *vals, const int32_t *row_ptr, const int
         if (len > chunk || dense[i]) continue;
         items.push_back(WorkItem{(int32_t)i, cc_host[i], cc_host[i + 1], -1});
     }
-    if (dense_rows) *dense_rows = dense;
-    // what an item costs, for the deal of the items to the XCDs: its steps, and two more for fetching the item, the
-    // first indices and the stores of its tile
-    std::vector<uint64_t> cost_prefix(items.size() + 1, 0);
-    for (size_t i = 0; i < items.size(); i++)
-        cost_prefix[i + 1] = cost_prefix[i] + (uint64_t)((items[i].end - items[i].begin + 31) / 32) + 2;
+    // Tasks: whole items that follow each other in the list, TASK_STEPS steps together at most and fewer where that leaves
+    // less than 16 wavefronts a CU (chunks of split rows and longer items are a task each).  Their costs, for the deal to the XCDs: the steps, two more for what is fetched first,
+    // and one per item for the stores of its tile.
+    const long task_steps = std::min<long>(TASK_STEPS, (long)(total / 32 * (int64_t)((n_cap + 63) / 64) / 4096));
+    std::vector<int4> tasks;
+    std::vector<uint64_t> cost_prefix(1, 0);
+    for (size_t i = 0; i < items.size();) {
+        size_t j = i + 1;
+        long steps = (items[i].end - items[i].begin) / 32;
+        while (j < items.size() && j - i < 64 && items[i].dst < 0 && items[j].begin == items[j - 1].end &&
+               steps + (items[j].end - items[j].begin) / 32 <= task_steps) {
+            steps += (items[j].end - items[j].begin) / 32;
+            j++;
+        }
+        tasks.push_back(int4{(int)i, (int)(j - i), items[i].begin, items[j - 1].end});
+        cost_prefix.push_back(cost_prefix.back() + (uint64_t)steps + 2 + (uint64_t)(j - i));
+        i = j;
+    }
     p->deal.set_costs(std::move(cost_prefix));
     p->n_items = (int)items.size();
+    p->n_tasks = (int)tasks.size();
+    SMAT_STEP(dev_malloc(&p->d_tasks, std::max<size_t>(tasks.size(), 1) * sizeof(int4)));
+    if (!tasks.empty()) SMAT_STEP(hipMemcpy(p->d_tasks, tasks.data(), tasks.size() * sizeof(int4), hipMemcpyHostToDevice));
     p->n_split_rows = (int)split.size();
     p->n_slots = slot;
     SMAT_STEP(dev_malloc(&p->d_items, std::max<size_t>(items.size(), 1) * sizeof(WorkItem)));
@@ -849,9 +999,6 @@ hipError_t compact_build(const uint16_t *vals, const int32_t *row_ptr, const int
         SMAT_STEP(hipMemcpy(p->d_split, split.data(), split.size() * sizeof(SplitRow), hipMemcpyHostToDevice));
         SMAT_STEP(dev_malloc(&p->d_workspace, (size_t)slot * 16 * n_cap * sizeof(float)));
     }
-    std::vector<unsigned long long> parts(CHECKSUM_BYTES / sizeof(unsigned long long));
-    SMAT_STEP(hipMemcpy(parts.data(), sums.p, CHECKSUM_BYTES, hipMemcpyDeviceToHost));
-    p->values_checksum = total_checksum(parts);
     SMAT_STEP(hipDeviceSynchronize());
 #undef SMAT_STEP
     if (e != hipSuccess) {

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "devmem.h"
 #include "sweep_format.h"
 #include <mutex>
 #include <utility>
@@ -92,29 +93,46 @@ hipError_t launch_reduce(const float *workspace, const SplitRow *split_rows, int
 // row are listed once (from the zero pattern of the values) and multiplied 32 at a time.
 struct CompactPlan {
     int32_t *d_cols = nullptr;   // row of B (absolute column of A) of every listed column; block rows padded to 32
-    uint16_t *d_acol = nullptr;  // the 16 values of every listed column, in MFMA operand order (32 bytes per column)
+    uint16_t *d_acol = nullptr;  // the 16 values of every listed column, in MFMA operand order (32 bytes per column), or
+    uint32_t *d_entries = nullptr;  // their nonzeros: value << 16 | byte in the step's operand
+    int2 *d_step_range = nullptr;   // entries [x, y) of every step of 32 listed columns
+    int entries_ahead = 0;          // loads of 64 entries that the product kernel asks for ahead: 1 or 2
     WorkItem *d_items = nullptr; // begin/end index the padded list
+    int4 *d_tasks = nullptr;     // runs of items: first item, items, first and last column of the list
     SplitRow *d_split = nullptr;
     float *d_workspace = nullptr; // n_slots * 16 * n_cap floats
-    int n_items = 0, n_split_rows = 0, n_slots = 0;
+    int n_items = 0, n_tasks = 0, n_split_rows = 0, n_slots = 0;
     int64_t n_cols = 0;           // nonzero block columns listed (without padding)
     int64_t n_cols_all = 0;       // nonzero block columns of the whole matrix
     uint64_t values_checksum = 0; // of the block values the lists were made from
-    XcdDeal deal;                 // cost of an item: its steps of 32 columns, and two more
+    XcdDeal deal;                 // of the tasks
     // Measured once, when the values are attached (compact_tune): the run length of the deal to the XCDs for
     // launches of tuned_n columns; 0 = not measured, the estimate from the costs decides.
     size_t tuned_n = 0;
     unsigned tuned_run = 0;
 };
-// vals / row_ptr / col_idx: device BCSR arrays; row_ptr_host: host copy of row_ptr.
-// dense_rows != NULL and dense_share > 0: block rows with at least that share of nonzero columns get no list and no
-// work item (a dense kernel multiplies them); *dense_rows receives one flag per block row.
-// skip_blocks_host != NULL: one flag per block; flagged blocks get no listed columns (another kernel multiplies them).
-// block_cols != NULL: receives the number of nonzero columns of every block.
-hipError_t compact_build(const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx,
-                         const int32_t *row_ptr_host, size_t mb, size_t nnzb, size_t n_cap, double dense_share,
-                         std::vector<uint8_t> *dense_rows, CompactPlan **out, const uint8_t *skip_blocks_host = nullptr,
-                         std::vector<uint8_t> *block_cols = nullptr);
+// What one pass over the block values tells: which columns of the blocks are nonzero, and the sums that the choice of
+// the kernels looks at.
+struct CompactCensus {
+    size_t mb = 0, nnzb = 0;
+    DevScratch mask;          // uint16 per block: its nonzero columns
+    DevScratch count, offset; // uint64 per block: nonzero columns | nonzeros << 32, and their exclusive sums
+    DevScratch rows;          // the same sums at the block rows (mb + 1)
+    std::vector<uint64_t> raw; // rows on the host
+    bool dropped = false;     // count, offset, rows and raw are those of the blocks that are not full
+    uint64_t values_checksum = 0;
+    int64_t n_cols_all = 0, nnz = 0;
+    int64_t full_blocks = 0, cols_rest = 0; // blocks with at least 10 of their 16 columns nonzero, nonzero columns of the others
+    int64_t cols_of_row(size_t br) const { return (int64_t)(uint32_t)(raw[br + 1] - raw[br]); }
+};
+// vals / row_ptr / col_idx here and below: device BCSR arrays.  Synchronous.
+hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t mb, size_t nnzb, CompactCensus &s);
+hipError_t compact_full_blocks(const CompactCensus &s, std::vector<uint8_t> &full); // one flag per block
+// The lists of a plan.  leave_rows != NULL: flagged block rows get no list and no work item (a dense kernel multiplies
+// them).  drop_full: full blocks get no listed columns (another kernel multiplies them); from then on the census is
+// that of the other blocks.
+hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx, size_t K, size_t n_cap,
+                         const std::vector<uint8_t> *leave_rows, bool drop_full, CompactPlan **out);
 // out[j * 256 ..] = block ids_host[j] of vals (device to device, synchronous).
 hipError_t copy_blocks(const uint16_t *vals, const int32_t *ids_host, size_t n, uint16_t *out);
 void compact_destroy(CompactPlan *p);
