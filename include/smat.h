@@ -280,7 +280,7 @@ int smat_csr_to_bcsr_device(size_t M, size_t K, const int32_t *row_ptr, const in
  *             VBR_nzblocks_count, VBR_longest_row (utilities.cpp:217-224,
  *             blocking.cpp:562-614); may be NULL
  *
- * Matrices of 16,384 rows and more are scanned on several threads (the hardware's
+ * Matrices of 262,144 rows and more are scanned on several threads (the hardware's
  * count, at most 16; SMAT_REORDER_THREADS in the environment sets it, 1 = none):
  * the output does not depend on the number of threads.
  */

@@ -41,6 +41,7 @@
 #include <atomic>
 #include <chrono>
 #include <functional>
+#include <limits>
 #include <numeric>
 #include <thread>
 #include <utility>
@@ -129,13 +130,14 @@ public:
         insert_fixup(z);
     }
 
-    // True if insert(dist, row) followed by trim_from_end(steps) with an odd `steps` would leave the tree as it is:
-    // a key above the largest one becomes the right child of the largest node; under a black parent nothing is
-    // rebalanced; the new node, a red leaf without a left child, is then the only one the trim removes (cycle of
-    // two, odd step count), and removing a red leaf rebalances nothing either.
-    bool insert_then_trim_is_noop(float dist, int64_t row) const
+    // insert(dist, row) followed by trim_from_end(steps) with an odd `steps` leaves the tree as it is for every
+    // dist >= keeps_below() of a row behind all rows in the set: a key above the largest one becomes the right child
+    // of the largest node; under a black parent nothing is rebalanced; the new node, a red leaf without a left child,
+    // is then the only one the trim removes (cycle of two, odd step count), and removing a red leaf rebalances
+    // nothing either.
+    float keeps_below() const
     {
-        return rightmost_ && !nodes_[rightmost_].red && !key_less(dist, row, nodes_[rightmost_]);
+        return rightmost_ && !nodes_[rightmost_].red ? nodes_[rightmost_].dist : std::numeric_limits<float>::infinity();
     }
 
     // Emulates `it = end(); advance(it, steps); erase(it, end());`.
@@ -369,11 +371,12 @@ Pattern build_block_patterns(int64_t rows, const int64_t *row_ptr, const int64_t
     Pattern p;
     p.ptr.resize(rows + 1);
     p.blk.reserve((size_t)row_ptr[rows]);
+    const int shift = col_block & (col_block - 1) ? -1 : __builtin_ctzll((unsigned long long)col_block); // a division takes as long as the rest
     for (int64_t r = 0; r < rows; r++) {
         p.ptr[r] = (int64_t)p.blk.size();
         int64_t last = -1;
         for (int64_t k = row_ptr[r]; k < row_ptr[r + 1]; k++) {
-            const int64_t b = col_idx[k] / col_block;
+            const int64_t b = shift >= 0 ? col_idx[k] >> shift : col_idx[k] / col_block;
             if (b != last) { p.blk.push_back((int32_t)b); last = b; }
         }
     }
@@ -383,13 +386,16 @@ Pattern build_block_patterns(int64_t rows, const int64_t *row_ptr, const int64_t
 
 // get_permutation (utilities.cpp:8-20): unstable sort of row ids by group id,
 // comparator arguments narrowed to int exactly as in the reference.
+// Group ids are below twice the rows, so id and row travel together in 8 bytes.
 std::vector<int64_t> permutation_by_group(const std::vector<int64_t> &grouping)
 {
-    auto comp = [&](int i, int j) { return grouping[i] < grouping[j]; };
-    std::vector<int64_t> v(grouping.size());
-    std::iota(v.begin(), v.end(), 0);
-    std::sort(v.begin(), v.end(), comp);
-    return v;
+    struct Entry { uint32_t group; int32_t row; };
+    std::vector<Entry> v(grouping.size());
+    for (size_t r = 0; r < v.size(); r++) v[r] = Entry{(uint32_t)grouping[r], (int32_t)r};
+    std::sort(v.begin(), v.end(), [](const Entry &a, const Entry &b) { return a.group < b.group; });
+    std::vector<int64_t> perm(v.size());
+    for (size_t i = 0; i < v.size(); i++) perm[i] = v[i].row;
+    return perm;
 }
 
 // Helper threads for the row scan of keeper_grouping.  A job is a function of the thread index that every
@@ -473,164 +479,382 @@ int scan_threads()
     return (int)std::min(std::max(hw, 1u), 16u);
 }
 
-// What looking at a row needs, by value: the helper threads take a copy per job, so that they read nothing that
-// the scanning thread writes while it applies results (its locals share cache lines with these fields otherwise).
-struct RowView {
-    static constexpr float PRUNED = -1.0f, TAKEN = -2.0f; // marks next to the distances (which are >= 0)
-    const int64_t *row_ptr, *pat_ptr, *stamp, *grouping;
-    const int32_t *pat_blk;
-    const float *dist_cache;
-    int64_t seed, pattern_blocks, group_size;
-    float seed_cached, tau;
-    bool pattern_empty;
-
-    // what the reference does with row j before it touches any state: skipped by the cached distances,
-    // already in a group, or compared with the pattern
-    float look(int64_t j) const
+// The `room` smallest keys (distance, position) of those offered so far, positions ascending.
+//
+// That is what the reference's trimmed set holds at its front.  A trim of a set of more than `room` keys takes away
+// the largest one, or the two largest if `room` is 1 modulo 3 and the shape of the tree has it so, and `room` only
+// ever falls (by one per merge).  With room % 3 != 1 at the end of a scan the smallest `room` keys are therefore
+// still in the set, and they are all that the group takes from it: the tree is built only for the other scans.
+// (On an Erdos-Renyi matrix the set grows to hundreds of rows, and half of the rows compared go through it.)
+//
+// Keys are collected below a limit, and whenever half as many again as needed are there, the nearest ones stay and the
+// last of them becomes the limit.
+class NearestRows {
+public:
+    void clear()
     {
-        if (seed_cached != -1 && dist_cache[j] != -1 && std::fabs(seed_cached - dist_cache[j]) > tau) return PRUNED;
-        if (grouping[j] != -1) return TAKEN;
-        const int64_t nb = pat_ptr[j + 1] - pat_ptr[j];
-        const bool b_empty = row_ptr[j + 1] == row_ptr[j];
-        if (pattern_empty && b_empty) return 0.0f;
-        if (pattern_empty || b_empty) return 1.0f;
-        int64_t common = 0;
-        for (int64_t k = pat_ptr[j]; k < pat_ptr[j + 1]; k++) common += stamp[pat_blk[k]] == seed;
-        const int64_t na = pattern_blocks;
-        // count_zeros weighting: blocks only in the group count once, blocks
-        // only in the row count group_size times (blocking.cpp:912-917)
-        const int64_t count = (na - common) + (nb - common) * group_size;
-        return (float)((2.0 * (double)count) / (double)(na * group_size + nb + count));
+        keys_.clear();
+        limit_ = std::numeric_limits<float>::infinity();
+    }
+    float limit() const { return limit_; } // keys from this distance on would not stay
+    void offer(float dist, int64_t pos, size_t room) // 0 <= dist < limit()
+    {
+        keys_.push_back(key(dist, pos));
+        if (keys_.size() >= room + room / 2 + 8) {
+            keep(room);
+            const uint32_t bits = (uint32_t)(*std::max_element(keys_.begin(), keys_.end()) >> 32);
+            memcpy(&limit_, &bits, 4);
+        }
+    }
+    template <class F> void for_each_ascending(size_t room, F f)
+    {
+        if (keys_.size() > room) keep(room);
+        std::sort(keys_.begin(), keys_.end());
+        for (uint64_t k : keys_) f((int64_t)(uint32_t)k);
+    }
+
+private:
+    // ascending like the pair: a float that is not negative orders like its bits
+    static uint64_t key(float dist, int64_t pos)
+    {
+        uint32_t bits;
+        memcpy(&bits, &dist, 4);
+        return (uint64_t)bits << 32 | (uint32_t)pos;
+    }
+    void keep(size_t room)
+    {
+        std::nth_element(keys_.begin(), keys_.begin() + (room - 1), keys_.end());
+        keys_.resize(room);
+    }
+    std::vector<uint64_t> keys_;
+    float limit_ = std::numeric_limits<float>::infinity();
+};
+
+// The rows that are in no group yet (and, until the next compaction, some that are), in row order, as the scan reads
+// them, and for every block column the ones that have it.
+struct LiveRows {
+    static constexpr int32_t TAKEN = -1; // in place of `blocks`
+    std::vector<int32_t> row, blocks, common; // row number, its block columns, those it shares with the pattern
+    std::vector<float> cached;                // the reference's distance cache
+    std::vector<int64_t> list_ptr;            // per block column: positions of the rows that have it, ascending
+    std::vector<int32_t> list;
+    int64_t n = 0, left = 0; // positions; those not taken
+
+    void start(int64_t rows, const Pattern &pat, int64_t nblk_cols)
+    {
+        row.resize((size_t)rows);
+        std::iota(row.begin(), row.end(), 0);
+        cached.assign((size_t)rows, 0.0f);
+        if (rows > 0) cached[0] = -1.0f;
+        blocks.assign((size_t)rows, 0);
+        list_ptr.resize((size_t)nblk_cols + 1);
+        list.resize(pat.blk.size());
+        n = left = rows;
+        index(pat);
+    }
+    void take(int64_t x)
+    {
+        blocks[x] = TAKEN;
+        left--;
+    }
+    // Taken rows leave.  A scan and a list walk pass over at most two thirds more rows than are there, and all
+    // compactions together cost four passes over the pattern.
+    void compact(const Pattern &pat)
+    {
+        int64_t to = 0;
+        for (int64_t x = 0; x < n; x++)
+            if (blocks[x] != TAKEN) {
+                row[to] = row[x];
+                cached[to++] = cached[x];
+            }
+        n = to;
+        index(pat);
+    }
+    int64_t list_length(int32_t b) const { return list_ptr[b + 1] - list_ptr[b]; }
+
+private:
+    void index(const Pattern &pat)
+    {
+        std::fill(list_ptr.begin(), list_ptr.end(), 0);
+        for (int64_t x = 0; x < n; x++) {
+            const int64_t r = row[x];
+            blocks[x] = (int32_t)(pat.ptr[r + 1] - pat.ptr[r]);
+            for (int64_t k = pat.ptr[r]; k < pat.ptr[r + 1]; k++) list_ptr[pat.blk[k] + 1]++;
+        }
+        for (size_t b = 1; b < list_ptr.size(); b++) list_ptr[b] += list_ptr[b - 1];
+        std::vector<int64_t> fill(list_ptr.begin(), list_ptr.end() - 1);
+        for (int64_t x = 0; x < n; x++)
+            for (int64_t k = pat.ptr[row[x]]; k < pat.ptr[row[x] + 1]; k++) list[fill[pat.blk[k]]++] = (int32_t)x;
+        common.assign((size_t)n, 0);
     }
 };
 
+// What looking at rows needs, by value: the helper threads take a copy per job, so that they read nothing that the
+// scanning thread writes while it applies results (its locals share cache lines with these fields otherwise).
+struct RowView {
+    static constexpr float PRUNED = -1.0f, TAKEN = -2.0f; // marks next to the distances (which are >= 0)
+    const int32_t *blocks, *common;
+    const float *cached;
+    int64_t pattern_blocks, group_size;
+    float seed_cached, tau;
+};
+
+// What the reference does with the rows at [first, first + count) before it touches any state: skipped by the cached
+// distances, already in a group, or compared with the pattern.  count_zeros weighting of the distance: blocks only in
+// the group count once, blocks only in the row count group_size times (blocking.cpp:912-917).
+//
+// The reference divides in double precision and rounds to float.  Where numerator and denominator are below 2^24 a
+// division in single precision gives the same float (both operands exact, and 53 bits are more than twice 24, so the
+// second rounding of the double quotient changes nothing), eight to an AVX2 instruction: 5.6 -> 0.7 ns a row.
+template <class Int, class Real>
+static inline __attribute__((always_inline)) void look_at(const RowView &v, const int32_t *__restrict blocks, const int32_t *__restrict common, const float *__restrict cached, int64_t count, float *__restrict res)
+{
+    const float seed_cached = v.seed_cached, tau = v.tau;
+    const Int na = (Int)v.pattern_blocks, group_size = (Int)v.group_size;
+    if (na == 0)
+        for (int64_t x = 0; x < count; x++) res[x] = blocks[x] == 0 ? 0.0f : 1.0f;
+    else
+        for (int64_t x = 0; x < count; x++) {
+            const Int nb = blocks[x], apart = (na - common[x]) + (nb - common[x]) * group_size;
+            res[x] = (float)((Real)(2 * apart) / (Real)(na * group_size + nb + apart));
+        }
+    if (na != 0) // in a loop of its own: a condition in the one above would keep the compiler from vectors
+        for (int64_t x = 0; x < count; x++) res[x] = blocks[x] == 0 ? 1.0f : res[x];
+    if (seed_cached != -1)
+        for (int64_t x = 0; x < count; x++)
+            res[x] = (cached[x] != -1) & (std::fabs(seed_cached - cached[x]) > tau) ? RowView::PRUNED : res[x];
+    for (int64_t x = 0; x < count; x++) res[x] = blocks[x] == LiveRows::TAKEN ? RowView::TAKEN : res[x];
+}
+
+#if defined(__x86_64__)
+__attribute__((target_clones("avx2", "default")))
+#endif
+void look_narrow(const RowView &v, int64_t first, int64_t count, float *res)
+{
+    look_at<int32_t, float>(v, v.blocks + first, v.common + first, v.cached + first, count, res);
+}
+void look_wide(const RowView &v, int64_t first, int64_t count, float *res)
+{
+    look_at<int64_t, double>(v, v.blocks + first, v.common + first, v.cached + first, count, res);
+}
+
+// Of the next RUN (or count) results: how many are distances; near[y] = 1 for one that is below `limit` or at most tau.
+constexpr int64_t RUN = 64;
+#if defined(__x86_64__)
+__attribute__((target_clones("avx2", "default")))
+#endif
+int32_t mark_near(const float *__restrict res, int64_t count, float limit, float tau, uint8_t *__restrict near)
+{
+    int32_t distances = 0;
+    for (int64_t y = 0; y < count; y++) distances += res[y] >= 0;
+    int32_t wide[RUN]; // float to byte in one step stays scalar code
+    for (int64_t y = 0; y < count; y++) wide[y] = (res[y] >= 0) & ((res[y] < limit) | (res[y] <= tau));
+    for (int64_t y = 0; y < count; y++) near[y] = (uint8_t)wide[y];
+    return distances;
+}
+
 // IterativeBlockingKeeper with use_pattern = 1 and the Jaccard group distance.
 //
-// The scan over the later rows j of one seed row i is sequential in the reference: the distance of row j is
-// taken against the pattern as the merges before j left it.  Here the scan runs in batches.  What happens to
-// row j depends on the scan so far only through the pattern and the group size, which change at a merge and
-// nowhere else (at most row_block - 1 times per seed): the rows of a batch are therefore evaluated in
-// parallel against the current pattern, and their results are applied in row order up to and including the
-// first merge; what was evaluated behind it is thrown away and the next batch starts there.  Every write
-// (distance cache, grouping, candidate set, counters) happens in that ordered pass, so the output is the one
-// of the sequential scan whatever the number of threads.
+// The scan over the later rows of one seed row is sequential in the reference: the distance of a row is taken
+// against the pattern as the merges before it left it.  It depends on the scan so far only through the pattern and
+// the group size, which change at a merge and nowhere else (at most row_block - 1 times per seed).  So between two
+// merges the rows are looked at in batches, and their results are applied in row order up to and including the first
+// merge; what was looked at behind it is thrown away.  Every write (distance cache, grouping, candidate set,
+// counters) happens in that ordered pass, so the output is the one of the sequential scan.
+//
+// What a row shares with the pattern is counted from the pattern's side: for every block column of the pattern the
+// rows that have it are counted up (a pattern of 16 blocks on 256 block columns: 4096 increments), instead of
+// looking up every block of every row (65,536 look-ups).  Right behind a merge the next one is often near: rows are
+// compared block by block until that has cost as much as bringing the counts up to date would.
+//
+// Both passes over a 4096 x 4096 matrix with 16 nonzeros per row: 47 -> 4.6 ms (10^6 comparisons; the counts 1 ms,
+// distances and the search for near ones 3 ms); R-MAT scale 17, 8.7 * 10^8 comparisons: 14.5 s on eight threads -> 3.5 s.
+// Helper threads pay from batches of 65,536 rows on (45 us): below, the scanning thread alone is faster.
 std::vector<int64_t> keeper_grouping(int64_t rows, const int64_t *row_ptr, const int64_t *col_idx,
                                      const Pattern &pat, int64_t nblk_cols, int64_t col_block,
                                      int64_t max_rows, float tau, int64_t &comparisons,
                                      int64_t &merges)
 {
     std::vector<int64_t> grouping((size_t)rows, -1);
-    std::vector<float> dist_cache((size_t)rows, 0.0f);
-    if (rows > 0) dist_cache[0] = -1.0f;
-
     std::vector<int64_t> stamp((size_t)nblk_cols + 1, -1); // stamp[b] == seed  <=>  b in pattern
     std::vector<int32_t> pattern, scratch;
     std::vector<int64_t> merged_rows;
+    std::vector<int64_t> merged_at; // positions of the rows merged during a scan
+    NearestRows nearest;
     CandidateTree candidates;
+    LiveRows live;
+    live.start(rows, pat, nblk_cols);
 
-    constexpr float TAKEN = RowView::TAKEN;
-    // Row by row for SERIAL_ROWS rows behind a change of the pattern, then batches that grow with the distance
-    // from it.  The two environment variables exist for the tests, which run small matrices through the batches.
+    // Batches grow with the distance from the last change of the pattern.  The environment variables exist for the
+    // tests, which run small matrices through the helper threads.
     auto tunable = [](const char *name, int64_t fallback) {
         const char *e = getenv(name);
         const long long v = e ? atoll(e) : 0;
         return v >= 1 ? (int64_t)v : fallback;
     };
-    const int64_t SERIAL_ROWS = tunable("SMAT_REORDER_SERIAL_ROWS", 512), FIRST_BATCH = tunable("SMAT_REORDER_FIRST_BATCH", 4096);
-    const int64_t MAX_BATCH = std::max<int64_t>(131072, FIRST_BATCH), GRAIN = std::max<int64_t>(1, std::min<int64_t>(512, FIRST_BATCH / 8));
+    const int64_t SERIAL_ROWS = tunable("SMAT_REORDER_SERIAL_ROWS", 512), FIRST_BATCH = tunable("SMAT_REORDER_FIRST_BATCH", 65536);
+    const int64_t MAX_BATCH = std::max<int64_t>(524288, FIRST_BATCH), GRAIN = std::max<int64_t>(1, std::min<int64_t>(4096, FIRST_BATCH / 8));
+    const int64_t ALONE = 512; // rows per batch of the scanning thread alone
     const int want_threads = rows >= 4 * FIRST_BATCH ? scan_threads() : 1;
     ScanPool pool(want_threads);
     // Three result buffers: one being applied, one being filled for the rows behind it, one whose distances
     // are being copied into the cache.
     std::vector<float> results[3];
+    results[0].resize((size_t)ALONE);
     if (pool.size() > 1)
-        for (std::vector<float> &r : results) r.resize((size_t)std::min<int64_t>(rows, MAX_BATCH));
+        for (std::vector<float> &r : results) r.resize((size_t)std::max(ALONE, std::min<int64_t>(rows, MAX_BATCH)));
     struct Span { int buf; int64_t first, count; };
     std::atomic<int64_t> next_store{0}, next_look{0};
+    // 2 * apart and the denominator are at most 2 * nblk_cols * (max_rows + 1)
+    const auto look = max_rows < ((int64_t)1 << 23) / std::max<int64_t>(nblk_cols, 1) - 1 ? look_narrow : look_wide;
 
-    for (int64_t i = 0; i < rows; i++) {
-        if (grouping[i] != -1) continue;
-        candidates.clear();
-        merged_rows.clear();
+    // block columns whose counts the pattern's last changes have not reached yet, and the step (+1 or -1)
+    std::vector<std::pair<int32_t, int32_t>> behind;
+    std::vector<int32_t> counted; // block columns that `common` has heard of since it was last zero
+
+    for (int64_t p = 0; p < live.n; p++) {
+        if (live.blocks[p] == LiveRows::TAKEN) continue;
+        if (live.left * 5 < live.n * 3) {
+            live.compact(pat);
+            p = 0;
+        }
+        const int64_t i = live.row[p];
         const int64_t group_number = i + rows;
         int64_t group_size = 1;
         grouping[i] = group_number;
+        nearest.clear();
+        merged_at.clear();
+        merged_rows.clear();
         merged_rows.push_back(i);
+        live.take(p);
 
         pattern.assign(pat.blk.begin() + pat.ptr[i], pat.blk.begin() + pat.ptr[i + 1]);
-        for (int32_t b : pattern) stamp[b] = i;
-        bool pattern_empty = row_ptr[i + 1] == row_ptr[i];
-        int64_t pattern_max = pattern_empty ? -1 : col_idx[row_ptr[i + 1] - 1];
-        const float seed_cached = dist_cache[i];
+        behind.clear();
+        int64_t behind_cost = 0, spent = 0;
+        auto will_count = [&](int32_t b, int32_t step) {
+            behind.emplace_back(b, step);
+            behind_cost += live.list_length(b);
+        };
+        for (int32_t b : pattern) {
+            stamp[b] = i;
+            will_count(b, 1);
+        }
+        int64_t pattern_max = pattern.empty() ? -1 : col_idx[row_ptr[i + 1] - 1];
+        const float seed_cached = live.cached[p];
         auto view = [&] {
-            return RowView{row_ptr, pat.ptr.data(), stamp.data(), grouping.data(), pat.blk.data(), dist_cache.data(),
-                           i, (int64_t)pattern.size(), group_size, seed_cached, tau, pattern_empty};
+            return RowView{live.blocks.data(), live.common.data(), live.cached.data(), (int64_t)pattern.size(), group_size, seed_cached, tau};
         };
-
-        auto look = [&](int64_t j) { return view().look(j); };
-        // a compared row that is not merged competes for the places left in the group
-        auto keep_candidate = [&](int64_t j, float dist) {
-            const size_t room = (size_t)(max_rows - (int64_t)merged_rows.size());
-            // most rows are farther than every candidate kept so far: see insert_then_trim_is_noop
-            if (candidates.size() >= room && (room & 1) && candidates.insert_then_trim_is_noop(dist, j)) return;
-            candidates.insert(dist, j);
-            if (candidates.size() > room) candidates.trim_from_end(room);
+        // brings the counts of the rows from position x on up to date
+        auto catch_up = [&](int64_t x) {
+            for (const auto &[b, step] : behind) {
+                const int32_t *at = live.list.data() + live.list_ptr[b], *end = live.list.data() + live.list_ptr[b + 1];
+                for (at = std::lower_bound(at, end, (int32_t)x); at < end; at++) live.common[*at] += step;
+                counted.push_back(b);
+            }
+            behind.clear();
+            behind_cost = 0;
         };
-        auto merge = [&](int64_t j) {
+        auto merge = [&](int64_t x) {
+            const int64_t j = live.row[x];
             merges++;
             grouping[j] = group_number;
             merged_rows.push_back(j);
+            merged_at.push_back(x);
+            live.take(x);
             // merge_rows(pattern, row j): row j's columns, plus the pattern's
             // columns below the largest column of row j that is <= max(pattern).
             // An empty row j therefore empties the pattern.
             const bool b_empty = row_ptr[j + 1] == row_ptr[j];
             int64_t cut = -1; // pattern blocks with id < cut survive
-            if (!b_empty && !pattern_empty) {
+            if (!b_empty && !pattern.empty()) {
                 const int64_t *bb = col_idx + row_ptr[j], *be = col_idx + row_ptr[j + 1];
                 const int64_t *ub = std::upper_bound(bb, be, pattern_max);
                 if (ub != bb) cut = *(ub - 1) / col_block;
             }
+            // both ascending: what stays of the pattern and row j, and where the two differ
             scratch.clear();
-            for (int32_t b : pattern) {
-                if (b < cut) scratch.push_back(b);
-                else stamp[b] = -1;
-            }
-            pattern.clear();
             size_t a = 0;
             int64_t k = pat.ptr[j];
-            while (a < scratch.size() || k < pat.ptr[j + 1]) {
-                if (k >= pat.ptr[j + 1] || (a < scratch.size() && scratch[a] < pat.blk[k])) {
-                    pattern.push_back(scratch[a++]);
+            const int64_t k_end = pat.ptr[j + 1];
+            while (a < pattern.size() || k < k_end) {
+                if (k >= k_end || (a < pattern.size() && pattern[a] < pat.blk[k])) {
+                    const int32_t b = pattern[a++];
+                    if (b < cut) {
+                        scratch.push_back(b);
+                    } else {
+                        stamp[b] = -1;
+                        will_count(b, -1);
+                    }
                 } else {
-                    if (a < scratch.size() && scratch[a] == pat.blk[k]) a++;
-                    pattern.push_back(pat.blk[k++]);
+                    const int32_t b = pat.blk[k++];
+                    if (a < pattern.size() && pattern[a] == b) {
+                        a++;
+                    } else {
+                        stamp[b] = i;
+                        will_count(b, 1);
+                    }
+                    scratch.push_back(b);
                 }
             }
-            for (int32_t b : pattern) stamp[b] = i;
-            pattern_empty = b_empty;
+            pattern.swap(scratch);
             pattern_max = b_empty ? -1 : col_idx[row_ptr[j + 1] - 1];
             group_size++;
+            spent = 0;
         };
-        // one row, start to end; true if it was merged
-        auto scan_row = [&](int64_t j) -> bool {
-            const float r = look(j);
-            if (r == TAKEN) return false;
-            dist_cache[j] = r; // PRUNED is the cache's own mark for "unknown"
-            if (r < 0) return false;
-            comparisons++;
-            if (r > tau) {
-                keep_candidate(j, r);
-                return false;
+        // Results of looked-at rows in row order, up to and including the first row that is to be merged: the number
+        // of rows gone through; `merged` tells whether the last of them is such a row.
+        bool merged = false;
+        auto apply = [&](const float *res, int64_t first, int64_t count) {
+            // a compared row that is not merged competes for the places left in the group; no merge inside the loop:
+            // the room for them stays what it is
+            const size_t room = (size_t)(max_rows - group_size);
+            for (int64_t x = 0; x < count; x += RUN) {
+                uint8_t near[RUN] = {};
+                const int32_t distances = mark_near(res + x, std::min(count - x, RUN), nearest.limit(), tau, near);
+                for (int64_t word = 0; word < RUN; word += 8) {
+                    uint64_t marks;
+                    memcpy(&marks, near + word, 8);
+                    for (; marks; marks &= marks - 1) { // little endian, as everywhere here
+                        const int64_t y = x + word + (__builtin_ctzll(marks) >> 3);
+                        const float r = res[y];
+                        if (r <= tau) {
+                            merged = true;
+                            comparisons += std::count_if(res + x, res + y + 1, [](float d) { return d >= 0; });
+                            return y + 1;
+                        }
+                        if (r < nearest.limit()) nearest.offer(r, first + y, room); // the limit may have fallen within the run
+                    }
+                }
+                comparisons += distances;
             }
-            merge(j);
-            return true;
+            return count;
         };
 
-        int64_t j = i + 1;
-        int64_t since_change = 0; // rows scanned since the pattern last changed
-        if (pool.size() == 1) {
-            for (; j < rows && group_size != max_rows; j++) scan_row(j);
-        }
+        int64_t x = p + 1;            // next position
+        int64_t since_change = 0;     // positions gone through since the pattern last changed
+        // Looks at rows block by block until that has cost as much as catching up with the counts would (a look-up
+        // with its loop takes as long as four to eight increments, and most seeds have no merge); true when the counts are up to date.
+        auto near_rows = [&] {
+            while (x < live.n && group_size != max_rows && 16 * spent < behind_cost) {
+                const int32_t nb = live.blocks[x];
+                if (nb != LiveRows::TAKEN) {
+                    const int64_t j = live.row[x];
+                    int32_t shared = 0;
+                    for (int64_t k = pat.ptr[j]; k < pat.ptr[j + 1]; k++) shared += stamp[pat.blk[k]] == i;
+                    float r;
+                    look_at<int64_t, double>(view(), &nb, &shared, &live.cached[x], 1, &r);
+                    live.cached[x] = r;
+                    spent += nb;
+                    merged = false;
+                    apply(&r, x, 1);
+                    if (merged) merge(x);
+                    since_change = merged ? 0 : since_change + 1;
+                }
+                spent++;
+                x++;
+            }
+            if (x < live.n && group_size != max_rows) catch_up(x);
+        };
         // ---- with helpers: `looked` = rows whose results are in a buffer, `stored` = rows applied whose distances
         // still have to go into the cache (the helpers do that on their next job) ----
         Span looked{0, 0, 0}, stored{0, 0, 0}, ahead{0, 0, 0};
@@ -645,25 +869,21 @@ std::vector<int64_t> keeper_grouping(int64_t rows, const int64_t *row_ptr, const
         const std::function<void(int)> job = [&](int) {
             const RowView v = job_view;
             const Span st = job_store, lk = job_look;
-            float *cache = dist_cache.data();
+            float *cache = live.cached.data();
             for (;;) {
                 const int64_t g0 = next_store.fetch_add(GRAIN, std::memory_order_relaxed);
                 if (g0 >= st.count) break;
                 const int64_t g1 = std::min(st.count, g0 + GRAIN);
-                const float *res = results[st.buf].data();
-                for (int64_t x = g0; x < g1; x++)
-                    if (res[x] != TAKEN) cache[st.first + x] = res[x];
+                std::copy(results[st.buf].data() + g0, results[st.buf].data() + g1, cache + st.first + g0);
             }
             for (;;) {
                 const int64_t g0 = next_look.fetch_add(GRAIN, std::memory_order_relaxed);
                 if (g0 >= lk.count) break;
-                const int64_t g1 = std::min(lk.count, g0 + GRAIN);
-                float *res = results[lk.buf].data();
-                for (int64_t x = g0; x < g1; x++) res[x] = v.look(lk.first + x);
+                look(v, lk.first + g0, std::min(lk.count, g0 + GRAIN) - g0, results[lk.buf].data() + g0);
             }
         };
         auto batch_rows = [&](int64_t first, int64_t since) {
-            return std::min(std::min<int64_t>(rows - first, MAX_BATCH), std::max(FIRST_BATCH, since));
+            return std::min(std::min<int64_t>(live.n - first, MAX_BATCH), std::max(FIRST_BATCH, since));
         };
         auto set_job = [&](Span st, Span lk) {
             job_view = view();
@@ -672,85 +892,108 @@ std::vector<int64_t> keeper_grouping(int64_t rows, const int64_t *row_ptr, const
             next_store.store(0, std::memory_order_relaxed);
             next_look.store(0, std::memory_order_relaxed);
         };
-        while (pool.size() > 1 && j < rows && group_size != max_rows) {
-            if (since_change < SERIAL_ROWS || rows - j < FIRST_BATCH) {
-                // right behind a merge the next one is often near: row by row (rows >= j are in no buffer)
-                const int64_t stop = std::min(rows, j + std::max<int64_t>(SERIAL_ROWS - since_change, rows - j < FIRST_BATCH ? rows - j : 0));
-                for (; j < stop && group_size != max_rows; j++) since_change = scan_row(j) ? 0 : since_change + 1;
+        auto store = [&](Span s) { // what is written for a taken row is never read
+            if (s.count) std::copy(results[s.buf].data(), results[s.buf].data() + s.count, live.cached.data() + s.first);
+        };
+        while (x < live.n && group_size != max_rows) {
+            if (!looked.count && !behind.empty()) {
+                near_rows();
                 continue;
             }
-            if (!looked.count) { // nothing looked at yet from j on: everybody looks
-                looked = Span{free_buffer(), j, batch_rows(j, since_change)};
+            merged = false;
+            if (pool.size() == 1 || since_change < SERIAL_ROWS || live.n - x < FIRST_BATCH) { // rows from x on are in no buffer
+                if (!looked.count) {
+                    store(stored);
+                    stored.count = 0;
+                    Span s{0, x, std::min(live.n - x, ALONE)};
+                    look(view(), s.first, s.count, results[0].data());
+                    s.count = apply(results[0].data(), s.first, s.count);
+                    store(s);
+                    x += s.count;
+                    since_change = merged ? 0 : since_change + s.count;
+                    if (merged) merge(x - 1);
+                    continue;
+                }
+            }
+            if (!looked.count) { // nothing looked at yet from x on: everybody looks
+                looked = Span{free_buffer(), x, batch_rows(x, since_change)};
                 set_job(stored, looked);
                 pool.run(job);
                 stored.count = 0;
             }
             // the helpers look at the rows behind this batch while its results are applied here
-            const int64_t behind = looked.first + looked.count;
-            ahead = Span{free_buffer(), behind, behind < rows ? batch_rows(behind, since_change + looked.count) : 0};
+            const int64_t next = looked.first + looked.count;
+            ahead = Span{free_buffer(), next, next < live.n ? batch_rows(next, since_change + looked.count) : 0};
             set_job(stored, ahead);
             pool.start(job);
             // whatever ends this iteration (an insertion that runs out of memory throws), the helpers have left the
             // job before the buffers and the job itself go away
             struct WaitOnExit { ScanPool &p; ~WaitOnExit() { p.wait(); } } wait_on_exit{pool};
-            const float *res = results[looked.buf].data();
-            int64_t x = 0;
-            bool merged = false;
-            // no merge inside the loop: the room for candidates stays what it is
-            const size_t room = (size_t)(max_rows - (int64_t)merged_rows.size());
-            const bool odd_room = room & 1;
-            int64_t compared = 0;
-            for (; x < looked.count; x++) {
-                const float r = res[x];
-                if (r < 0) continue;
-                compared++;
-                if (r > tau) {
-                    const int64_t row = looked.first + x;
-                    // most rows are farther than every candidate kept so far: see insert_then_trim_is_noop
-                    if (odd_room && candidates.size() >= room && candidates.insert_then_trim_is_noop(r, row)) continue;
-                    candidates.insert(r, row);
-                    if (candidates.size() > room) candidates.trim_from_end(room);
-                    continue;
-                }
-                merged = true; // applied below, when the helpers no longer read the pattern
-                x++;
-                break;
-            }
-            comparisons += compared;
+            const int64_t done = apply(results[looked.buf].data(), looked.first, looked.count);
             pool.wait();
-            stored = Span{looked.buf, looked.first, x};
-            j = looked.first + x;
-            if (merged) {
-                merge(j - 1);
+            stored = Span{looked.buf, looked.first, done};
+            x = looked.first + done;
+            if (merged) { // now that the helpers no longer read the pattern
+                merge(x - 1);
                 since_change = 0;
                 looked.count = 0; // what was looked at behind the merge saw the old pattern
             } else {
-                since_change += x;
+                since_change += done;
                 looked = ahead;
             }
         }
-        if (stored.count) { // distances of the last rows applied
-            const float *res = results[stored.buf].data();
-            for (int64_t x = 0; x < stored.count; x++)
-                if (res[x] != TAKEN) dist_cache[stored.first + x] = res[x];
-        }
+        store(stored); // distances of the last rows applied
 
-        if (group_size < max_rows) {
+        auto take = [&](int64_t pos) {
+            const int64_t j = live.row[pos];
+            grouping[j] = group_number;
+            merged_rows.push_back(j);
+            live.take(pos);
+            group_size++;
+        };
+        if (group_size < max_rows && (max_rows - group_size) % 3 != 1) {
+            nearest.for_each_ascending((size_t)(max_rows - group_size), take);
+        } else if (group_size < max_rows) {
+            // the set as the reference keeps it, from the distances the scan has left in the cache
+            candidates.clear();
+            merged_at.push_back(live.n);
+            int64_t y = p + 1;
+            size_t room = (size_t)max_rows - 1;
+            for (int64_t end : merged_at) {
+                auto keeps_below = [&] { return (room & 1) && candidates.size() >= room ? candidates.keeps_below() : std::numeric_limits<float>::infinity(); };
+                float limit = keeps_below();
+                for (; y < end; y++) {
+                    const float r = live.cached[y];
+                    if (r < 0 || r >= limit || live.blocks[y] == LiveRows::TAKEN) continue;
+                    candidates.insert(r, y);
+                    if (candidates.size() > room) candidates.trim_from_end(room);
+                    limit = keeps_below();
+                }
+                y++;
+                room--;
+            }
             candidates.for_each_ascending([&](const CandidateTree::Node &n) {
                 if (group_size == max_rows) return false;
-                grouping[n.row] = group_number;
-                merged_rows.push_back(n.row);
-                group_size++;
+                take(n.row);
                 return true;
             });
         }
         if (group_size == max_rows)
             for (int64_t r : merged_rows) grouping[r] -= rows; // complete groups sort first
         for (int32_t b : pattern) stamp[b] = -1;
+        // counts back to zero, by whichever way touches less
+        int64_t touched = 0;
+        for (int32_t b : counted) touched += live.list_length(b);
+        if (4 * touched < live.n) {
+            for (int32_t b : counted)
+                for (int64_t k = live.list_ptr[b]; k < live.list_ptr[b + 1]; k++) live.common[live.list[k]] = 0;
+        } else if (!counted.empty()) {
+            std::fill(live.common.begin(), live.common.begin() + live.n, 0);
+        }
+        counted.clear();
     }
     return grouping;
 }
-
 
 // CollectBlockingInfo (blocking.cpp:562-614) restricted to the two integer
 // statistics that do not depend on timers: number of nonzero blocks and the
@@ -866,7 +1109,8 @@ static int smat_reorder_csr_impl(size_t M, size_t K, const int32_t *row_ptr, con
             ci[k] = col_idx[k];
             cols_eff = std::max<int64_t>(cols_eff, (int64_t)col_idx[k] + 1);
         }
-        std::sort(ci.begin() + row_ptr[r], ci.begin() + row_ptr[r + 1]);
+        if (!std::is_sorted(ci.begin() + row_ptr[r], ci.begin() + row_ptr[r + 1]))
+            std::sort(ci.begin() + row_ptr[r], ci.begin() + row_ptr[r + 1]);
     }
     rp[rows_eff] = rows_eff ? row_ptr[rows_eff] : 0;
 

@@ -62,6 +62,20 @@ def test_fixtures_through_the_batched_scan(smat, monkeypatch, path, env):
     check_fixture(smat, path)
 
 
+@pytest.mark.parametrize("row_block", [2, 5, 16])
+def test_distances_in_single_and_in_double_precision_agree(smat, row_block):
+    """Distances are divided in fp32 while counts stay below 2^24.  The same rows with the block columns drawn apart
+    have the same distances but too many block columns for that."""
+    d = gen.rmat(10, 16)
+    rows, cols = int(np.flatnonzero(np.diff(d["row_ptr"]))[-1]) + 1, d["col_idx"].astype(np.int64)
+    args = (d["row_ptr"].astype(np.int64)[:rows + 1],)
+    want = smat.reorder_rows(rows, int(d["K"]), *args, cols, 16, row_block, 0.5)
+    apart = (cols >> 4 << 18) + (cols & 15)  # 2^14 times as many block columns
+    got = smat.reorder_rows(rows, int(d["K"]) << 14, *args, apart, 16, row_block, 0.5)
+    for a, b in zip(want, got):
+        assert np.array_equal(a, b)
+
+
 def run_reference(tmp_path, r, c, cb, rb, tau):
     binary = ref_binary("Matrix_Blocking")
     el = tmp_path / "case.el"
