@@ -136,6 +136,7 @@ extern "C" int smat_plan_cache_clear(void)
     for (Entry &en : g_cache.entries)
         if (en.plan) smat_plan_destroy(en.plan);
     g_cache.entries.clear();
+    dev_trim();
     return SMAT_OK;
 }
 
