@@ -570,10 +570,12 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
     const int n_panels = (int)((a.N + PANEL - 1) / PANEL);
     long panel_stride = PANEL, row_stride = (long)a.N;
     if (!a.b_row_major) {
-        dim3 grid((unsigned)((a.K + 63) / 64), (unsigned)((a.N + 63) / 64));
-        hipLaunchKernelGGL(transpose_b_kernel, grid, dim3(256), 0, st, a.B, a.Bt, (int)a.N, (long)a.K, PANEL, (long)PANEL);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+        if (!a.bt_ready) {
+            dim3 grid((unsigned)((a.K + 63) / 64), (unsigned)((a.N + 63) / 64));
+            hipLaunchKernelGGL(transpose_b_kernel, grid, dim3(256), 0, st, a.B, a.Bt, (int)a.N, (long)a.K, PANEL, (long)PANEL);
+            hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
         panel_stride = (long)a.K * PANEL;
         row_stride = PANEL;
     }
@@ -664,28 +666,37 @@ hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t
     p.tuned_n = 0;
     p.tuned_run = 0;
     if (!g_tune || p.n_items == 0 || N == 0 || !Bt) return hipSuccess;
+    // What the deal is about is the product kernel: with column-major B it is timed on a zeroed copy Bt, without the
+    // transposition.  (24 launches of 20 us each with it, and a synchronisation for every run length, were 0.5 of the
+    // 1.25 ms that blocking, planning and attaching a 16384^2 matrix with 0.1 % nonzeros and its first product took.)
     Scratch B, C;
-    if (B.alloc(K * N * sizeof(uint16_t)) != hipSuccess || C.alloc(M * N * sizeof(uint16_t)) != hipSuccess) {
+    if ((b_row_major && B.alloc(K * N * sizeof(uint16_t)) != hipSuccess) || C.alloc(M * N * sizeof(uint16_t)) != hipSuccess) {
         (void)hipGetLastError(); // no room for the trial: not an error of the plan
         return hipSuccess;
     }
-    hipError_t e = hipMemset(B.p, 0, K * N * sizeof(uint16_t));
+    hipError_t e = b_row_major ? hipMemset(B.p, 0, K * N * sizeof(uint16_t)) : hipMemset(Bt, 0, K * ((N + 255) / 256 * 256) * sizeof(uint16_t));
     if (e == hipSuccess) e = hipMemset(C.p, 0, M * N * sizeof(uint16_t));
-    hipEvent_t t0 = nullptr, t1 = nullptr;
-    if (e == hipSuccess) e = hipEventCreate(&t0);
-    if (e == hipSuccess) e = hipEventCreate(&t1);
+    constexpr int MAX_RUNS = 4;
+    hipEvent_t mark[MAX_RUNS + 1] = {};
+    for (int i = 0; i <= MAX_RUNS && e == hipSuccess; i++) e = hipEventCreate(&mark[i]);
     CompactArgs a{};
-    a.B = static_cast<const uint16_t *>(B.p); a.b_row_major = b_row_major; a.Bt = Bt; a.C = C.p;
+    a.B = static_cast<const uint16_t *>(B.p); a.b_row_major = b_row_major; a.Bt = Bt; a.bt_ready = true; a.C = C.p;
     a.M = M; a.N = N; a.K = K; a.c_f32 = false; a.plan = &p; a.accumulate = accumulate;
-    auto time_of = [&](unsigned run, int launches, float *ms) {
-        a.xcd_run = run;
-        hipError_t r = launch_compact(a, nullptr); // warm-up
-        if (r == hipSuccess) r = hipEventRecord(t0, nullptr);
-        for (int i = 0; i < launches && r == hipSuccess; i++) r = launch_compact(a, nullptr);
-        if (r == hipSuccess) r = hipEventRecord(t1, nullptr);
-        if (r == hipSuccess) r = hipEventSynchronize(t1);
-        if (r == hipSuccess) r = hipEventElapsedTime(ms, t0, t1);
-        *ms /= (float)launches;
+    // the run lengths one after the other without a gap between them, `launches` times each after one more of the first
+    auto time_all = [&](const unsigned *runs, int n, int launches, float *ms) {
+        a.xcd_run = runs[0];
+        hipError_t r = launch_compact(a, nullptr);
+        if (r == hipSuccess) r = hipEventRecord(mark[0], nullptr);
+        for (int k = 0; k < n; k++) {
+            a.xcd_run = runs[k];
+            for (int i = 0; i < launches && r == hipSuccess; i++) r = launch_compact(a, nullptr);
+            if (r == hipSuccess) r = hipEventRecord(mark[k + 1], nullptr);
+        }
+        if (r == hipSuccess) r = hipEventSynchronize(mark[n]);
+        for (int k = 0; k < n && r == hipSuccess; k++) {
+            r = hipEventElapsedTime(&ms[k], mark[k], mark[k + 1]);
+            ms[k] /= (float)launches;
+        }
         return r;
     };
     // the run length of an untuned launch, as launch_compact_tq computes it for this N
@@ -695,25 +706,25 @@ hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t
     const unsigned eighth = (unsigned)std::max<long>((wgs + 7) / 8, 1);
     const unsigned base = std::min(eighth, p.deal.run((size_t)p.n_tasks, n_panels));
     float t_base = 0.f;
-    if (e == hipSuccess) e = time_of(base, 1, &t_base);
+    if (e == hipSuccess) e = time_all(&base, 1, 1, &t_base);
     if (e == hipSuccess && t_base <= 20.f) {
-        std::vector<unsigned> runs{base};
+        unsigned runs[MAX_RUNS] = {base};
+        int n = 1;
         if (base * 4 >= eighth) // a list that the estimate finds even: the longer runs are worth a try
             for (unsigned r : {eighth, eighth / 2, eighth / 4})
-                if (r >= 4 && std::find(runs.begin(), runs.end(), r) == runs.end()) runs.push_back(r);
-        const int launches = t_base < 0.2f ? 6 : 3;
+                if (r >= 4 && std::find(runs, runs + n, r) == runs + n) runs[n++] = r;
         unsigned best_run = base;
-        float best = 0.f;
-        for (size_t i = 0; i < runs.size() && e == hipSuccess; i++) {
-            float ms = 0.f;
-            e = time_of(runs[i], launches, &ms);
-            if (i == 0) best = ms * 0.97f; // another run length has to be 3 % faster than the estimate's choice
-            else if (ms < best) best = ms, best_run = runs[i];
+        if (n > 1) {
+            float ms[MAX_RUNS] = {};
+            e = time_all(runs, n, t_base < 0.2f ? 5 : 3, ms);
+            float best = ms[0] * 0.97f; // another run length has to be 3 % faster than the estimate's choice
+            for (int k = 1; k < n && e == hipSuccess; k++)
+                if (ms[k] < best) best = ms[k], best_run = runs[k];
         }
         if (e == hipSuccess) p.tuned_n = N, p.tuned_run = best_run;
     }
-    if (t0) (void)hipEventDestroy(t0);
-    if (t1) (void)hipEventDestroy(t1);
+    for (hipEvent_t m : mark)
+        if (m) (void)hipEventDestroy(m);
     return e;
 }
 

@@ -142,6 +142,7 @@ struct CompactArgs {
     const uint16_t *B; // column-major, or row-major with b_row_major
     bool b_row_major;  // B is already B[k*N + n]: no copy is made
     uint16_t *Bt;      // scratch, K * (N rounded up to 256) halves: the copy of B in panels of rows made at the start of the launch
+    bool bt_ready = false; // the copy is there already
     void *C;
     size_t M, N, K;
     bool c_f32;
@@ -151,7 +152,7 @@ struct CompactArgs {
 };
 hipError_t launch_compact(const CompactArgs &a, hipStream_t st);
 // Times launches of M x N x K with a few run lengths of the deal to the XCDs (the estimate's choice, an eighth of the
-// launch, a half and a quarter of that) on zeros in temporary buffers and keeps the fastest for launches of N columns
+// launch, a half and a quarter of that) on zeros (a column-major B: without the launch that makes Bt, which is overwritten) and keeps the fastest for launches of N columns
 // (tuned_n, tuned_run).  The deal decides where an item runs, not what it computes: the results do not depend on
 // it.  Synchronous, default stream; a plan too large for the temporary buffers, or whose single launch takes
 // longer than 20 ms, keeps the estimate's choice.
