@@ -53,6 +53,8 @@ struct smat_plan {
         }
     };
     SweepDev sweep;       // all block rows (SMAT_KERNEL_SWEEP)
+    bool sweep_few_tiles = false; // its row groups were chosen by sweep_estimate_us
+    size_t sweep_chunks = 0;      // chunks its row groups list
     SweepDev sweep_dense; // mixed dispatch: the block rows with mostly full blocks, when they fill the device
     // mixed dispatch per block (rows that hold both kinds of blocks): the blocks with mostly nonzero columns, copied one
     // behind the other into d_vals_dense, go through the sweep kernel; the compact kernel adds the other blocks' columns
@@ -141,6 +143,40 @@ static bool sweep_fills_device(size_t mb, size_t n)
     return n_rg * n_panels >= 256;
 }
 
+// Time of a product through the sweep kernel, from the tiles (row groups x panels of 64 columns, one workgroup of a compute unit
+// each), the chunks that the row groups list together and the ops of a wavefront per chunk.  Measured: a tile costs 2.5 us of
+// entry and stores, a chunk 0.25 us and 0.115 us per op (the plan fills up to four), a third more where every compute unit
+// has a tile and they share the L2.  Row groups of 16 / 32 / 64 block rows, estimate (measured), us:
+//   3088 x 4112, 15 %, N = 1000: 19.5 (23.9) / 18.8 (24.8) / 24.5 (34.9); 30 %: 21.3 (21.4) / 28.1 (27.1) / 39.8 (42.8)
+//   8192 x 8192, 10 %, N = 640:  67.8 (51.2) / 31.7 (29.5) / 41.5 (37.9); N = 1536: 101 (82) / 68 (56) / 46.7 (43.1)
+//   768 x 3072, 10 %, N = 4096:  14.8 (14.2) / 14.0 (15.0) / 15.3 (16.8)
+static double sweep_estimate_us(size_t n_rg, size_t listed_chunks, size_t nnzb, size_t N)
+{
+    if (n_rg == 0 || listed_chunks == 0) return 1e30;
+    const size_t tiles = n_rg * ((N + 16 * SWEEP_TN - 1) / (16 * SWEEP_TN)), rounds = (tiles + 255) / 256;
+    const double ops = 0.525 * (double)nnzb / ((double)listed_chunks * SWEEP_WAVES) + 0.3;
+    const double chunk = (0.25 + 0.115 * std::max(4.0, ops)) * (1.0 + 0.35 * (double)std::min<size_t>(tiles, 256) / 256.0);
+    return 1.5 + (double)rounds * (2.5 + (double)listed_chunks / (double)n_rg * chunk);
+}
+// The same through the row-wise kernel: 20 TB/s of operands from repacked B, behind the repack, 7.6 TB/s from B in place.
+// (3088 x 4112, 15 %, N = 1000: 24.0, measured 26.2; 8192 x 8192, 10 %, N = 640: 40.1 (44.9), N = 128: 14.4 (13.0).)
+static double rowwise_estimate_us(size_t K, size_t N, size_t nnzb, bool packed)
+{
+    const double gather = (double)nnzb * 16.0 * (double)N * 2.0;
+    return packed ? 8.0 + 4.0 * (double)K * (double)N / 4e6 + gather / 20e6 : 4.0 + gather / 7.6e6;
+}
+static size_t sweep_listed_chunks(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t group_rows)
+{
+    std::vector<size_t> seen((kb + SWEEP_S - 1) / SWEEP_S, 0); // the last row group that listed the chunk, from 1
+    size_t n = 0;
+    for (size_t i = 0; i < mb; i++)
+        for (int32_t q = row_ptr[i]; q < row_ptr[i + 1]; q++) {
+            size_t &s = seen[(size_t)col_idx[q] / (16 * SWEEP_S)];
+            if (s != i / group_rows + 1) s = i / group_rows + 1, n++;
+        }
+    return n;
+}
+
 extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_ptr,
                                       const int32_t *col_idx, const uint16_t *B, void *C, size_t M,
                                       size_t N, size_t K, size_t nnzb, const smat_spmm_opts *opts,
@@ -191,7 +227,9 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         kernel = SMAT_KERNEL_ROWWISE;
     }
     // a plan made for a wide N, used with a narrow one: too few workgroups for the sweep kernel
-    if (kernel == SMAT_KERNEL_SWEEP && o.kernel == SMAT_KERNEL_AUTO && !sweep_fills_device(M / 16, N))
+    if (kernel == SMAT_KERNEL_SWEEP && o.kernel == SMAT_KERNEL_AUTO &&
+        (plan->sweep_few_tiles ? sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, N) > rowwise_estimate_us(K, N, nnzb, a.b_packed != nullptr)
+                               : !sweep_fills_device(M / 16, N)))
         kernel = SMAT_KERNEL_ROWWISE;
     const uint16_t *B_as_given = B;
     if (kernel == SMAT_KERNEL_MIXED && (!plan || !plan->compact || (!plan->d_items_dense && !plan->sweep_dense.d_ops && !plan->sweep_blocks.d_ops) || !plan->d_bt || N > plan->n_cap))
@@ -522,6 +560,40 @@ extern "C" int smat_plan_create(smat_plan **out, const int32_t *row_ptr_host,
     return smat::guarded("smat_plan_create", [&] { return smat_plan_create_impl(out, row_ptr_host, col_idx_host, M, K, nnzb, n_hint, opts); });
 }
 
+// A matrix of mostly full blocks whose tiles of 64 block rows x 64 columns are fewer than the compute units: the sweep kernel
+// all the same, on row groups of 64, 32 or 16 block rows, where the estimates say that it is 15 % faster than the row-wise
+// kernel.  (Measured, us, before and after: 8192^2, 10 %, N = 640: 44.9 -> 29.0, N = 1536: 71.2 -> 42.6; 3088 x 4112, 15 %,
+// N = 2000: 40.6 -> 22.7; 768 x 3072, 30 %, N = 4096: 31.9 -> 15.6; 1040 x 16384, 35 %, N = 1000, which the estimate leaves
+// with the row-wise kernel: 85 against 57.)  Below 3 % of the blocks even four ops a chunk are mostly fillers (4096^2, 3 %,
+// N = 512: 16.2 against 9.6).  A K of one or two chunks, less than the entry fetches, stays with the row-wise kernel as it was.
+// The streams take about 0.7 us a block to build on the host, so they are built once the values are known to be dense.
+static hipError_t sweep_small_groups(smat_plan &p)
+{
+    const size_t mb = p.M / 16, kb = p.K / 16, nnzb = p.nnzb;
+    if (p.col_idx_host.size() != nnzb || nnzb < 2 || nnzb >= (size_t)1 << 23 || p.K >= (size_t)1 << 28 || kb <= 2 * SWEEP_S ||
+        sweep_fills_device(mb, p.n_cap) || (double)nnzb < 0.03 * (double)mb * (double)kb)
+        return hipSuccess;
+    const int32_t *row_ptr = p.row_ptr_host.data(), *col_idx = p.col_idx_host.data();
+    double best = rowwise_estimate_us(p.K, p.n_cap, nnzb, p.d_bpack != nullptr) / 1.15;
+    size_t group_rows = 0;
+    for (size_t rows : {(size_t)SWEEP_G, (size_t)SWEEP_G / 2, (size_t)SWEEP_G / 4}) {
+        const double t = sweep_estimate_us((mb + rows - 1) / rows, sweep_listed_chunks(row_ptr, col_idx, mb, kb, rows), nnzb, p.n_cap);
+        if (t < best) best = t, group_rows = rows;
+    }
+    if (!group_rows) return hipSuccess;
+    SweepPlanHost h;
+    build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 1e7);
+    const hipError_t e = p.sweep.upload(h);
+    if (e != hipSuccess) {
+        p.sweep.release();
+        return e;
+    }
+    p.sweep_chunks = (size_t)h.rg_chunk_ptr.back();
+    p.sweep_few_tiles = true;
+    p.kernel = SMAT_KERNEL_SWEEP;
+    return hipSuccess;
+}
+
 static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, const int32_t *row_ptr,
                                         const int32_t *col_idx, const int32_t *row_ptr_host)
 {
@@ -617,7 +689,9 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     auto t_compact = [&](double cols) { return cols * n_est * 2.0 / 10e6; };
     const double t_pass = 3.0 + (double)p->K * n_est / 1e6;
     // one kernel for everything: the sweep kernel (when the plan has its work list) or the compact kernel
-    const double t_sweep_all = p->sweep.d_ops ? t_sweep((double)p->nnzb) : 1e30;
+    const double t_sweep_all = !p->sweep.d_ops ? 1e30
+                               : p->sweep_few_tiles ? sweep_estimate_us((size_t)p->sweep.n_rg, p->sweep_chunks, p->nnzb, p->n_cap)
+                                                    : t_sweep((double)p->nnzb);
     const double t_compact_all = t_compact((double)census.n_cols_all) + t_pass;
     if (may_mix && !mixed && !p->col_idx_host.empty() && p->nnzb < ((size_t)1 << 23) &&
         p->K < ((size_t)1 << 28) && sweep_fills_device(mb, p->n_cap)) {
@@ -650,7 +724,8 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
                        !(dense_kernel == SMAT_KERNEL_SWEEP && t_sweep_all < t_compact_all));
     if (!take) { // nothing would use the list: the plan keeps (or goes back to) a dense kernel
         if (p->kernel == SMAT_KERNEL_COMPACT || p->kernel == SMAT_KERNEL_MIXED) p->kernel = dense_kernel;
-        return SMAT_OK;
+        if (want == SMAT_KERNEL_AUTO && dense_kernel == SMAT_KERNEL_ROWWISE) e = sweep_small_groups(*p);
+        return e == hipSuccess ? SMAT_OK : fail(e);
     }
     if (!c) e = compact_build(census, vals, row_ptr, col_idx, p->K, p->n_cap, mixed ? &dense : nullptr, false, &c);
     if (e != hipSuccess) return fail(e);

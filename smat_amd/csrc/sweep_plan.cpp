@@ -23,11 +23,12 @@ constexpr int VM_MARK = MIN_OPS; // a chunk boundary waits until at most this ma
 } // namespace
 
 void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, SweepPlanHost &out,
-                      const int32_t *rows, size_t n_rows)
+                      const int32_t *rows, size_t n_rows, size_t group_rows, double search)
 {
     if (!rows) n_rows = mb;
-    const size_t n_rg = (n_rows + G - 1) / G;
-    // Row groups: G block rows of the list each, in list order - unless that leaves one group with far more blocks
+    const size_t GR = std::min<size_t>(std::max<size_t>(group_rows, 1), G); // block rows that share a group's 64 places
+    const size_t n_rg = (n_rows + GR - 1) / GR;
+    // Row groups: GR block rows of the list each, in list order - unless that leaves one group with far more blocks
     // than the average.  A workgroup multiplies one row group under several panels, so the launch takes as long as
     // the heaviest group; then the rows are dealt out instead: in descending block count, each to the group with the
     // fewest blocks so far that still has room (the group sizes stay what they were).  Which rows share a group
@@ -39,10 +40,10 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
         int64_t total = 0, heaviest = 0;
         for (size_t i = 0; i < n_rows; i++) {
             const size_t br = rows ? (size_t)rows[i] : i;
-            blocks_of[i / G] += row_ptr[br + 1] - row_ptr[br];
+            blocks_of[i / GR] += row_ptr[br + 1] - row_ptr[br];
         }
         for (size_t rg = 0; rg < n_rg; rg++) total += blocks_of[rg], heaviest = std::max(heaviest, blocks_of[rg]);
-        if (n_rg > 1 && (double)heaviest * (double)n_rows > 1.08 * (double)total * (double)G) {
+        if (n_rg > 1 && (double)heaviest * (double)n_rows > 1.08 * (double)total * (double)GR) {
             std::vector<int32_t> by_count(n_rows);
             for (size_t i = 0; i < n_rows; i++) by_count[i] = rows ? rows[i] : (int32_t)i;
             std::stable_sort(by_count.begin(), by_count.end(), [&](int32_t x, int32_t y) {
@@ -57,7 +58,7 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
                 lightest.pop();
                 const size_t rg = l.second;
                 members[rg].push_back(br);
-                if (members[rg].size() < std::min(n_rows, (rg + 1) * G) - rg * G)
+                if (members[rg].size() < std::min(n_rows, (rg + 1) * GR) - rg * GR)
                     lightest.push(Load(l.first + (row_ptr[br + 1] - row_ptr[br]), rg));
             }
             order.reserve(n_rows);
@@ -80,7 +81,7 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
     struct Ranked { int rank; int row; int32_t hi; SweepOpHost op; };
     std::vector<std::vector<Ranked>> by_chunk;
     for (size_t rg = 0; rg < n_rg; rg++) {
-        const size_t r_begin = rg * G, r_end = std::min(n_rows, (rg + 1) * G);
+        const size_t r_begin = rg * GR, r_end = std::min(n_rows, (rg + 1) * GR);
         // the chunks this row group touches, ascending
         const size_t first_chunk = out.chunk_ids.size();
         for (size_t i = r_begin; i < r_end; i++)
@@ -209,8 +210,8 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
                 return sum;
             };
             long best = sum_of_caps(nullptr);
-            // work bound: about 2e8 counter updates per plan, shared evenly by the row groups
-            long budget = (long)(2e8 / (double)(n * WAVES * 3) / (double)n_rg);
+            // work bound: so many counter updates per plan, shared evenly by the row groups
+            long budget = (long)(search / (double)(n * WAVES * 3) / (double)n_rg);
             for (int pass = 0; pass < 4 && budget > 0; pass++) {
                 bool improved = false;
                 for (int i = 0; i < G && budget > 0; i++)

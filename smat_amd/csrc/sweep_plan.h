@@ -26,7 +26,9 @@ struct SweepPlanHost {
 // at least two blocks.  rows != NULL: only these n_rows block rows (ascending) are multiplied and stored, packed
 // 64 to a row group; the others belong to another kernel.  The rows go to the row groups in list order, or, where
 // that leaves one group with over 1.08 x the blocks of an average one, by their block count (row_map says where).
+// Row groups of group_rows (at most 64) block rows each; search: counter updates that the assignment of rows to wavefronts
+// may cost.
 void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, SweepPlanHost &out,
-                      const int32_t *rows = nullptr, size_t n_rows = 0);
+                      const int32_t *rows = nullptr, size_t n_rows = 0, size_t group_rows = SWEEP_G, double search = 2e8);
 
 } // namespace smat

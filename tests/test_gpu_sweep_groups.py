@@ -1,0 +1,37 @@
+"""Sweep kernel on row groups of fewer than 64 block rows: what a plan takes where groups of 64 would leave compute units idle."""
+import numpy as np
+import pytest
+
+from smat_amd import generators as gen
+
+pytestmark = pytest.mark.gpu
+
+
+def to_dev(torch, a, cuda):
+    return torch.from_numpy(np.ascontiguousarray(a).view(np.int16) if a.dtype == np.uint16 else np.ascontiguousarray(a)).to(cuda)
+
+
+# block rows around one, two and four groups of 16 and 32, a last group of one row, K not a multiple of a chunk
+@pytest.mark.parametrize("mb,kb,density,N", [(48, 64, 0.3, 4096), (49, 33, 0.5, 2048), (17, 64, 0.4, 8192), (65, 49, 0.4, 2504), (193, 64, 0.1, 1608)])
+@pytest.mark.parametrize("c_f32", [False, True])
+def test_small_row_groups_match_the_oracle(smat, cuda, oracle, mb, kb, density, N, c_f32):
+    import torch
+    A = gen.random_bcsr(mb, kb, density, seed=mb + kb)
+    M, K, nnzb = A["M"], A["K"], A["nnzb"]
+    B = gen.dense_b(K, N, seed=N)
+    vals, rp, ci, Bd = (to_dev(torch, x, cuda) for x in (A["b_val"], A["b_row_ptr"].astype(np.int32), A["b_col_idx"].astype(np.int32), B))
+    plan = smat.Plan(A["b_row_ptr"], M, K, nnzb, N, col_idx_host=A["b_col_idx"])
+    plan.attach_values(vals, rp, ci)
+    assert plan.info()["kernel"] == smat.KERNEL_SWEEP
+    want = oracle.spmm_bcsr(M, N, K, A["b_row_ptr"], A["b_col_idx"], A["b_val"], B, threads=4)
+    C = torch.full((M, N), float("nan"), dtype=torch.float32 if c_f32 else torch.float16, device=cuda)
+    smat.spmm(vals, rp, ci, Bd, C, M, N, K, nnzb, plan=plan, c_f32=c_f32)
+    torch.cuda.synchronize()
+    assert oracle.compare(C.half().cpu().numpy().view(np.uint16), want)[0] <= 1e-3
+    # the same plan at another width: the first columns of the same product, through whichever kernel that width takes
+    n = 64
+    C2 = torch.full((M, n), float("nan"), dtype=C.dtype, device=cuda)
+    smat.spmm(vals, rp, ci, Bd, C2, M, n, K, nnzb, plan=plan, c_f32=c_f32)
+    torch.cuda.synchronize()
+    first = oracle.spmm_bcsr(M, n, K, A["b_row_ptr"], A["b_col_idx"], A["b_val"], B[:n * K], threads=4)
+    assert oracle.compare(C2.half().cpu().numpy().view(np.uint16), first)[0] <= 1e-3
