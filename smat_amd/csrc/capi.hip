@@ -63,7 +63,7 @@ struct smat_plan {
     int64_t n_blocks_split = 0;
     std::vector<int32_t> row_ptr_host; // the block row pointer the plan was made from: smat_plan_attach_values works from this copy
     std::vector<int32_t> col_idx_host; // kept for the split of a mixed plan (plans made with col_idx_host for AUTO / MIXED)
-    uint64_t fingerprint = 0; // FNV-1a over row_ptr_host and, when given, col_idx_host
+    uint64_t fingerprint = 0; // hash of row_ptr_host and, when given, col_idx_host
     bool fingerprint_has_cols = false;
     // compacted-column kernel (present after smat_plan_attach_values)
     CompactPlan *compact = nullptr;
