@@ -93,9 +93,9 @@ int smat_plan_cache_clear(void);
 #define SMAT_KERNEL_SWEEP 2   /* workgroup sweeps K for a group of 64 block rows x 64 columns, B staged in LDS
                                * in chunks of 16 block columns; needs a plan made with col_idx_host, between 2
                                * and 2^23 - 1 blocks and K below 2^28.  SMAT_KERNEL_AUTO takes it when at least
-                               * 5% of the blocks exist and (M/1024) x (N/64) workgroups fill the 256 CUs; with
-                               * fewer workgroups, from 3% on, once the attached values are mostly full blocks
-                               * and an estimate finds it faster (on groups of 64, 32 or 16 block rows).
+                               * 5% of the blocks exist and (M/1024) x (N/64) workgroups fill the 256 CUs, or
+                               * once the attached values are mostly full blocks and an estimate finds it
+                               * faster (on groups of 64, 32 or 16 block rows).
                                * It works from the plan's op list, NOT from the row_ptr / col_idx passed at
                                * launch: the plan must have been made from the same block pattern
                                * (smat_plan_check verifies that on request)                                 */

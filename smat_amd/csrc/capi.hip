@@ -560,21 +560,24 @@ extern "C" int smat_plan_create(smat_plan **out, const int32_t *row_ptr_host,
     return smat::guarded("smat_plan_create", [&] { return smat_plan_create_impl(out, row_ptr_host, col_idx_host, M, K, nnzb, n_hint, opts); });
 }
 
-// A matrix of mostly full blocks whose tiles of 64 block rows x 64 columns are fewer than the compute units: the sweep kernel
-// all the same, on row groups of 64, 32 or 16 block rows, where the estimates say that it is 15 % faster than the row-wise
-// kernel.  (Measured, us, before and after: 8192^2, 10 %, N = 640: 44.9 -> 29.0, N = 1536: 71.2 -> 42.6; 3088 x 4112, 15 %,
-// N = 2000: 40.6 -> 22.7; 768 x 3072, 30 %, N = 4096: 31.9 -> 15.6; 1040 x 16384, 35 %, N = 1000, which the estimate leaves
-// with the row-wise kernel: 85 against 57.)  Below 3 % of the blocks even four ops a chunk are mostly fillers (4096^2, 3 %,
-// N = 512: 16.2 against 9.6).  A K of one or two chunks, less than the entry fetches, stays with the row-wise kernel as it was.
-// The streams take about 0.7 us a block to build on the host, so they are built once the values are known to be dense.
+// A matrix of mostly full blocks that plan creation left with the row-wise kernel, because its tiles of 64 block rows x 64
+// columns are fewer than the compute units or because fewer than 5 % of its blocks exist: the sweep kernel all the same, on
+// row groups of 64, 32 or 16 block rows, where the estimates say that it is 15 % faster than the row-wise kernel (half as fast
+// again where every compute unit has a tile: there the estimate is up to 30 % low, 68 for 87 us on 8192^2, 3 %, N = 4096).
+// Measured, us, before and after: 8192^2, 10 %, N = 640: 44.9 -> 29.0, N = 1536: 71.2 -> 42.6; 3088 x 4112, 15 %, N = 2000:
+// 40.6 -> 22.7; 768 x 3072, 30 %, N = 4096: 31.9 -> 15.6; bands, whose row groups list few chunks: 16384 rows, bandwidth 64,
+// N = 1024 42.5 -> 19.3; 65536, 256, N = 512 146 -> 77; 4096, 30, N = 1024 14.4 -> 8.7.  Left alone by the estimate: 4096^2, 3 %,
+// N = 512 (9.6 against 16.2); 1040 x 16384, 35 %, N = 1000, wrongly (85 against 57).  A K of one or two chunks, less than
+// the entry fetches, stays with the row-wise kernel as it was.
+// The streams take 0.1 to 0.2 us a block to build on the host, so they are built once the values are known to be dense; the
+// search for a better deal of the rows to the wavefronts is cut short (ten times the work: 5.5 against 1.8 ms, same kernel times).
 static hipError_t sweep_small_groups(smat_plan &p)
 {
     const size_t mb = p.M / 16, kb = p.K / 16, nnzb = p.nnzb;
-    if (p.col_idx_host.size() != nnzb || nnzb < 2 || nnzb >= (size_t)1 << 23 || p.K >= (size_t)1 << 28 || kb <= 2 * SWEEP_S ||
-        sweep_fills_device(mb, p.n_cap) || (double)nnzb < 0.03 * (double)mb * (double)kb)
+    if (p.col_idx_host.size() != nnzb || nnzb < 2 || nnzb >= (size_t)1 << 23 || p.K >= (size_t)1 << 28 || kb <= 2 * SWEEP_S)
         return hipSuccess;
     const int32_t *row_ptr = p.row_ptr_host.data(), *col_idx = p.col_idx_host.data();
-    double best = rowwise_estimate_us(p.K, p.n_cap, nnzb, p.d_bpack != nullptr) / 1.15;
+    double best = rowwise_estimate_us(p.K, p.n_cap, nnzb, p.d_bpack != nullptr) / (sweep_fills_device(mb, p.n_cap) ? 1.5 : 1.15);
     size_t group_rows = 0;
     for (size_t rows : {(size_t)SWEEP_G, (size_t)SWEEP_G / 2, (size_t)SWEEP_G / 4}) {
         const double t = sweep_estimate_us((mb + rows - 1) / rows, sweep_listed_chunks(row_ptr, col_idx, mb, kb, rows), nnzb, p.n_cap);
@@ -582,7 +585,7 @@ static hipError_t sweep_small_groups(smat_plan &p)
     }
     if (!group_rows) return hipSuccess;
     SweepPlanHost h;
-    build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 1e7);
+    build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 1e6);
     const hipError_t e = p.sweep.upload(h);
     if (e != hipSuccess) {
         p.sweep.release();

@@ -35,3 +35,21 @@ def test_small_row_groups_match_the_oracle(smat, cuda, oracle, mb, kb, density, 
     torch.cuda.synchronize()
     first = oracle.spmm_bcsr(M, n, K, A["b_row_ptr"], A["b_col_idx"], A["b_val"], B[:n * K], threads=4)
     assert oracle.compare(C2.half().cpu().numpy().view(np.uint16), first)[0] <= 1e-3
+
+
+# bands: few blocks of the matrix, few chunks for a row group; a last group of one block row, edges cut off
+@pytest.mark.parametrize("m,bandwidth,N", [(4096, 30, 1024), (4112, 64, 1000), (8192, 100, 520)])
+def test_bands_match_the_oracle(smat, cuda, oracle, m, bandwidth, N):
+    import torch
+    d = gen.band(m, bandwidth)
+    A = smat.csr_to_bcsr(d["M"], d["K"], d["row_ptr"], d["col_idx"], d["val"])
+    B = gen.dense_b(A.K, N, seed=m)
+    vals, rp, ci, Bd = (to_dev(torch, x, cuda) for x in (A.val, A.row_ptr, A.col_idx, B))
+    plan = smat.Plan(A.row_ptr, A.M, A.K, A.nnzb, N, col_idx_host=A.col_idx)
+    plan.attach_values(vals, rp, ci)
+    assert plan.info()["kernel"] == smat.KERNEL_SWEEP
+    C = torch.full((A.M, N), float("nan"), dtype=torch.float16, device=cuda)
+    smat.spmm(vals, rp, ci, Bd, C, A.M, N, A.K, A.nnzb, plan=plan)
+    torch.cuda.synchronize()
+    want = oracle.spmm_bcsr(A.M, N, A.K, A.row_ptr, A.col_idx, A.val, B, threads=4)
+    assert oracle.compare(C.cpu().numpy().view(np.uint16), want)[0] <= 1e-3
