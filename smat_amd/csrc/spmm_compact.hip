@@ -880,10 +880,11 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     p->n_cols = n_cols;
     // The nonzeros one by one (4 bytes each, and 8 per step) while that is at most half of the 32 bytes per column that
     // whole columns take: about one nonzero per column in random sparse matrices (a step of 36 entries: 152 bytes for
-    // 1024), 2.8 in the 27-point stencil (368 bytes).  Where the panels of B are small enough to stay in the L2 (K up to
+    // 1024), 2.8 in the 27-point stencil (368 bytes).  Where the panels of B are small enough to stay in the L2 (K below
     // 4096) it is the LDS that binds, and whole columns, which do not go through it, win (24352 x 1376, 22 a row, N = 72:
-    // 13.7 against 14.5 us; 16384^2, N = 256, the other way round: 18.9 against 16.3).
-    const bool by_entry = nnz <= 4 * n_cols && K > 4096 && s.nnz < 0x7fffff00;
+    // 13.7 against 14.5 us; 16384^2, N = 256, the other way round: 18.9 against 16.3; 65536 x 4096, 8 a row, N = 512: 50.3 against
+    // 43.7, 16384 x 4096, 16 a row, N = 256: 14.5 against 14.7).
+    const bool by_entry = nnz <= 4 * n_cols && K >= 4096 && s.nnz < 0x7fffff00;
     const size_t cap = (size_t)total + LIST_PAD;
     SMAT_STEP(dev_malloc(&p->d_cols, cap * sizeof(int32_t)));
     SMAT_STEP(hipMemsetAsync(p->d_cols, 0, cap * sizeof(int32_t), nullptr)); // padding: row 0 of B
@@ -979,9 +980,10 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         items.push_back(WorkItem{(int32_t)i, cc_host[i], cc_host[i + 1], -1});
     }
     // Tasks: whole items that follow each other in the list, TASK_STEPS steps together at most and fewer where that leaves
-    // less than 16 wavefronts a CU (chunks of split rows and longer items are a task each).  Their costs, for the deal to the XCDs: the steps, two more for what is fetched first,
+    // less than 28 wavefronts a CU (65536 x 4096, 8 a row, N = 96: 16.0 us, with 16 a CU 17.8; chunks of split rows and longer
+    // items are a task each).  Their costs, for the deal to the XCDs: the steps, two more for what is fetched first,
     // and one per item for the stores of its tile.
-    const long task_steps = std::min<long>(TASK_STEPS, (long)(total / 32 * (int64_t)((n_cap + 63) / 64) / 4096));
+    const long task_steps = std::min<long>(TASK_STEPS, (long)(total / 32 * (int64_t)((n_cap + 63) / 64) / 7168));
     std::vector<int4> tasks;
     std::vector<uint64_t> cost_prefix(1, 0);
     for (size_t i = 0; i < items.size();) {
