@@ -37,10 +37,14 @@ namespace {
 constexpr int LONG_ROW = 512;
 
 constexpr int HELD = 8;               // entries that a thread of emit_held keeps in registers
-constexpr int BITMAP_COLS = 1 << 17;  // block columns per pass over the entries (16 KiB per bitmap; K above 2^21 takes more passes)
+// Block columns per pass over the entries: three words of LDS per 32 of them beside the blocks that are put together, in
+// the 64 KiB that a launch may ask for without more ado (12 KiB a bitmap; K above 1.5 * 2^20 takes more passes).
+constexpr int BITMAP_COLS = 3 << 15;
 constexpr int LIGHT_THREADS = 256, HEAVY_THREADS = 1024, HEAVY_GRID = 256;
 constexpr int HEAVY_ROW = HELD * LIGHT_THREADS; // entries of a block row above which it goes to the workgroups of 1024
 constexpr int CHUNK = 32;             // blocks that emit_held puts together in LDS at a time (16 KiB)
+constexpr int STATIC_LDS = 256;       // at most: row_ptr of a block row and one word per wavefront
+static_assert(BITMAP_COLS % 32 == 0 && BITMAP_COLS / 32 * 12 + CHUNK * 512 + STATIC_LDS <= 65536, "LDS of the emitting kernels");
 
 struct State { // zeroed before the first kernel
     int32_t bad;      // a column index is outside the matrix

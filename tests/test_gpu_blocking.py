@@ -88,3 +88,27 @@ def test_rejects_bad_column(smat, cuda):
     rp = np.array([0, 1] + [1] * 15, np.int32)
     with pytest.raises(smat.SmatError):
         device_blocking(smat, cuda, 16, 16, rp, np.array([16], np.int32), np.array([1], np.uint16))
+
+
+# K around one, two and three passes over the entries (98304 block columns each), with a light block row, one whose entries
+# are counted by the larger workgroups, and one of more entries than those hold
+@pytest.mark.parametrize("K", [98304 * 16, 98304 * 16 + 16, 1 << 21, (1 << 21) + 16, 98304 * 32 + 4096])
+@pytest.mark.parametrize("ordered", [True, False])
+def test_wide_matrices_in_several_passes(smat, cuda, K, ordered):
+    rng = np.random.default_rng(K % 1009)
+    edges = np.array([0, 15, 16, 98304 * 16 - 1, 98304 * 16, K - 17, K - 1])
+    edges = np.unique(edges[edges < K])
+    rows = []
+    for r in range(64):
+        n = (40, 300, 900, 5)[r // 16]  # entries of a block row: 640, 4,800, 14,400 and 80
+        cols = np.unique(np.concatenate([rng.integers(0, K, n), edges]))
+        if r % 5 == 0:
+            cols = np.unique(np.concatenate([cols, cols[:20] + 1, cols[:20] + 2]))
+            cols = cols[cols < K]
+        if not ordered and r % 16 == 3:
+            cols = rng.permutation(cols)
+        rows.append(cols)
+    rp = np.concatenate([[0], np.cumsum([len(c) for c in rows])]).astype(np.int32)
+    ci = np.concatenate(rows).astype(np.int32)
+    v = rng.integers(1, 0x3C00, len(ci)).astype(np.uint16)
+    check_same(smat, cuda, 64, K, rp, ci, v)
