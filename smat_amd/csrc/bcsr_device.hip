@@ -518,13 +518,14 @@ static int smat_csr_to_bcsr_device_impl(size_t M, size_t K, const int32_t *row_p
     step(heavy.alloc((nnz / HEAVY_ROW + 1) * sizeof(int32_t)));
     State *st = static_cast<State *>(state.p);
     const int32_t words = (int32_t)((std::min<size_t>(kb, BITMAP_COLS) + 31) / 32);
+    const int32_t kb32 = (int32_t)std::min<size_t>(kb, (size_t)1 << 27); // the block columns that an int32 column index can name
     if (e == hipSuccess) {
         step(hipMemsetAsync(st, 0, sizeof(State), nullptr));
         if (nnz) {
             hipLaunchKernelGGL(count_blocks_kernel, dim3((unsigned)mb), dim3(LIGHT_THREADS), words * 4, 0, row_ptr, col_idx, (int64_t)K,
-                               (int32_t)kb, st, (int32_t *)heavy.p, (int32_t *)count.p);
+                               kb32, st, (int32_t *)heavy.p, (int32_t *)count.p);
             hipLaunchKernelGGL(count_heavy_kernel, dim3(HEAVY_GRID), dim3(HEAVY_THREADS), words * 4, 0, row_ptr, col_idx, (int64_t)K,
-                               (int32_t)kb, st, (const int32_t *)heavy.p, (int32_t *)count.p);
+                               kb32, st, (const int32_t *)heavy.p, (int32_t *)count.p);
         } else {
             step(hipMemsetAsync(count.p, 0, mb * sizeof(int32_t), nullptr));
         }
@@ -542,10 +543,10 @@ static int smat_csr_to_bcsr_device_impl(size_t M, size_t K, const int32_t *row_p
     if (e == hipSuccess && nnzb) {
         const unsigned lds = (unsigned)(words * 12 + CHUNK * 512);
         hipLaunchKernelGGL(emit_blocks_kernel, dim3((unsigned)mb), dim3(LIGHT_THREADS), lds, 0, row_ptr, col_idx, val, (int64_t)K,
-                           (int32_t)kb, words, !h.unsorted, (int32_t *)count.p, orp, oci, ov);
+                           kb32, words, !h.unsorted, (int32_t *)count.p, orp, oci, ov);
         if (h.n_heavy)
             hipLaunchKernelGGL(emit_heavy_kernel, dim3(HEAVY_GRID), dim3(HEAVY_THREADS), lds, 0, row_ptr, col_idx, val, (int64_t)K,
-                               (int32_t)kb, words, st, !h.unsorted, (int32_t *)count.p, (const int32_t *)heavy.p, orp, oci, ov);
+                               kb32, words, st, !h.unsorted, (int32_t *)count.p, (const int32_t *)heavy.p, orp, oci, ov);
         if (!h.unsorted && counts)
             hipLaunchKernelGGL(sum_dense_kernel, dim3((unsigned)std::min<size_t>((mb + 1023) / 1024, 64)), dim3(256), 0, 0,
                                (const int32_t *)count.p, (int64_t)mb, st);

@@ -112,3 +112,16 @@ def test_wide_matrices_in_several_passes(smat, cuda, K, ordered):
     ci = np.concatenate(rows).astype(np.int32)
     v = rng.integers(1, 0x3C00, len(ci)).astype(np.uint16)
     check_same(smat, cuda, 64, K, rp, ci, v)
+
+
+def test_more_block_columns_than_an_int32_column_can_name(smat, cuda):
+    """K beyond 2^31: the passes end behind the last block column that an int32 column index reaches."""
+    rng = np.random.default_rng(4)
+    ci = np.unique(np.concatenate([rng.integers(0, 2**31 - 1, 300), [0, 2**31 - 1]])).astype(np.int32)
+    rp = np.array([0] + [len(ci)] * 16, np.int32)
+    v = rng.integers(1, 0x3C00, len(ci)).astype(np.uint16)
+    got = device_blocking(smat, cuda, 16, 16 * (2**31 - 1), rp, ci, v)
+    assert np.array_equal(got.col_idx, np.unique(ci // 16) * 16)
+    want = np.zeros((len(got.col_idx), 256), np.uint16)
+    want[np.searchsorted(got.col_idx, ci // 16 * 16), ci % 16] = v
+    assert np.array_equal(got.val.reshape(-1, 256), want)
