@@ -115,6 +115,9 @@ extern "C" void smat_internal_alloc_counts(int64_t *out)
     out[1] = g_dev_frees.load();
 }
 
+// Test hook (not part of smat.h): the library's n-th device allocation from now on (0 = the next) fails; < 0: none does.
+extern "C" void smat_internal_fail_alloc(int64_t n) { g_dev_fail_in.store(n); }
+
 extern "C" const char *smat_version(void) { return "smat-amd 0.1 gfx950"; }
 
 static int check_shapes(const void *vals, const void *row_ptr, const void *col_idx, const void *B,

@@ -13,6 +13,7 @@
 
 namespace smat {
 extern std::atomic<long long> g_dev_mallocs, g_dev_frees;
+extern std::atomic<long long> g_dev_fail_in; // test hook: so many allocations from now on succeed, the next fails; < 0: none
 
 constexpr size_t DEV_KEEP_BYTES = (size_t)1 << 30, DEV_KEEP_BLOCK = (size_t)1 << 29;
 

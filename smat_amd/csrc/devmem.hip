@@ -9,7 +9,7 @@
 
 namespace smat {
 
-std::atomic<long long> g_dev_mallocs{0}, g_dev_frees{0};
+std::atomic<long long> g_dev_mallocs{0}, g_dev_frees{0}, g_dev_fail_in{-1};
 
 namespace {
 
@@ -124,8 +124,9 @@ hipError_t release(void *p, bool idle)
 
 hipError_t dev_malloc_bytes(void **p, size_t bytes)
 {
-    g_dev_mallocs.fetch_add(1, std::memory_order_relaxed);
     *p = nullptr;
+    if (g_dev_fail_in.load(std::memory_order_relaxed) >= 0 && g_dev_fail_in.fetch_sub(1) == 0) return hipErrorOutOfMemory;
+    g_dev_mallocs.fetch_add(1, std::memory_order_relaxed);
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     if (e != hipSuccess) return e;

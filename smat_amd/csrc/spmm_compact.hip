@@ -946,12 +946,17 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
                 e = hipGetLastError();
             }
             SMAT_STEP(hipMemcpy(padded.data(), row_first.p, (mb + 1) * sizeof(int32_t), hipMemcpyDeviceToHost));
-            for (int32_t &v : padded) v *= 32;
-            total = (int64_t)n_steps * 32;
-            (void)dev_free_idle(p->d_cols); // the copy back has waited for the kernels
-            (void)dev_free_idle(p->d_step_range);
-            p->d_cols = cols;
-            p->d_step_range = range;
+            if (e == hipSuccess) { // the copy back has waited for the kernels, so the old lists are idle
+                for (int32_t &v : padded) v *= 32;
+                total = (int64_t)n_steps * 32;
+                std::swap(p->d_cols, cols);
+                std::swap(p->d_step_range, range);
+                (void)dev_free_idle(cols);
+                (void)dev_free_idle(range);
+            } else { // kernels may still be at work on either
+                if (cols) (void)dev_free(cols);
+                if (range) (void)dev_free(range);
+            }
         }
     }
     // work items: whole block rows; rows much longer than the average in chunks of 32-column steps
