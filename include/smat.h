@@ -72,7 +72,8 @@ const char *smat_version(void);
 int smat_spmm_bcsr_f16(const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx,
                        const uint16_t *B, uint16_t *C, size_t M, size_t N, size_t K, size_t nnzb,
                        const int32_t *block_info, const int32_t *rel_map);
-/* Drops every plan that smat_spmm_bcsr_f16 keeps (synchronous).  No counterpart in the reference. */
+/* Drops every plan that smat_spmm_bcsr_f16 keeps and gives the device memory that the library holds in reserve, on
+ * every GPU, back to the driver (synchronous): see smat_plan_destroy.  No counterpart in the reference. */
 int smat_plan_cache_clear(void);
 
 /* ---- SpMM with options / explicit stream / plan -------------------------- */
@@ -167,6 +168,11 @@ int smat_plan_attach_values(smat_plan *plan, const uint16_t *vals, const int32_t
  * 8-byte copy back (synchronous): 3 us for 13 MB of values, 1.3 ms for the 5.7 GB of R-MAT scale 20.  Not
  * called by the SpMM itself.  No counterpart in the reference, which keeps no copy. */
 int smat_plan_values_current(const smat_plan *plan, const uint16_t *vals, int *current);
+/* Device memory released by the library (by this call, smat_free, a replaced list of smat_plan_attach_values, scratch of
+ * smat_csr_to_bcsr_device) is kept for the next plan or matrix: at most 1 GiB per GPU, in blocks of at most 512 MiB, the
+ * oldest given back first.  Kept blocks count as used memory for everyone else in the process and on the GPU: an allocator next to
+ * the library that runs out of memory gets them back after smat_plan_cache_clear(); an allocation of the library itself
+ * that fails gives them back and tries again. */
 int smat_plan_destroy(smat_plan *plan);
 /* Opt-in check that `plan` was made from this block pattern: M, K, nnzb and a 64-bit hash of
  * row_ptr_host (and of col_idx_host if the plan was made with one; then it must be passed).  One pass over

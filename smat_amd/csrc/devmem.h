@@ -26,8 +26,8 @@ template <class T> inline hipError_t dev_malloc(T **p, size_t bytes)
 hipError_t dev_free(void *p);
 // The same for a caller that has waited since the last use of the block.
 hipError_t dev_free_idle(void *p);
-// Gives the kept blocks of the current device back to the driver.
-void dev_trim();
+// Gives the kept blocks, of the current device or of all, back to the driver.
+void dev_trim(bool all_devices);
 
 // Scratch memory of one call; the call has waited for its kernels when it goes out of scope.
 struct DevScratch {

@@ -147,7 +147,7 @@ hipError_t dev_malloc_bytes(void **p, size_t bytes)
     e = hipMalloc(p, cls ? cls : bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        dev_trim();
+        dev_trim(false);
         e = hipMalloc(p, cls ? cls : bytes);
     }
     if (e == hipSuccess && cls) {
@@ -160,17 +160,20 @@ hipError_t dev_malloc_bytes(void **p, size_t bytes)
 hipError_t dev_free(void *p) { return release(p, false); }
 hipError_t dev_free_idle(void *p) { return release(p, true); }
 
-void dev_trim()
+void dev_trim(bool all_devices)
 {
     int device = 0;
-    if (hipGetDevice(&device) != hipSuccess) return;
+    if (!all_devices && hipGetDevice(&device) != hipSuccess) return;
     Keeper &k = keeper();
     std::vector<void *> all;
     {
         std::lock_guard<std::mutex> lock(k.mutex);
-        Keeper::PerDevice &d = k.devices[device];
-        all = take_oldest(k, d, 0);
-        d.order.clear();
+        for (auto &d : k.devices) {
+            if (!all_devices && d.first != device) continue;
+            const std::vector<void *> some = take_oldest(k, d.second, 0);
+            all.insert(all.end(), some.begin(), some.end());
+            d.second.order.clear();
+        }
     }
     for (void *q : all) (void)hipFree(q);
 }

@@ -136,7 +136,7 @@ extern "C" int smat_plan_cache_clear(void)
     for (Entry &en : g_cache.entries)
         if (en.plan) smat_plan_destroy(en.plan);
     g_cache.entries.clear();
-    dev_trim();
+    dev_trim(true); // its plans may be on any device
     return SMAT_OK;
 }
 

@@ -66,3 +66,18 @@ def test_attach_values_survives_every_failing_allocation(smat, cuda, oracle):
         assert held(smat) <= before + 1, f"device blocks lost by failing allocation {n}"  # the copy of B may stay for the next attempt
     assert failures >= 15 and plan.info()["kernel"] == smat.KERNEL_COMPACT
     plan.close()
+
+
+def test_clearing_the_plan_cache_gives_kept_memory_back(smat, cuda):
+    import torch
+    torch.cuda.synchronize()
+    smat.lib.smat_plan_cache_clear()
+    free = torch.cuda.mem_get_info()[0]
+    big = 256 << 20
+    p = C.c_void_p()
+    assert smat.lib.smat_malloc(C.byref(p), big) == 0
+    assert torch.cuda.mem_get_info()[0] <= free - big
+    assert smat.lib.smat_free(p) == 0
+    assert torch.cuda.mem_get_info()[0] <= free - big  # kept
+    assert smat.lib.smat_plan_cache_clear() == 0
+    assert torch.cuda.mem_get_info()[0] >= free
