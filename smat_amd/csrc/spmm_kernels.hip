@@ -281,15 +281,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
             const int myc = col_idx[first + lane < last ? first + lane : last];
             const int jend = jw + 32 < j1 ? jw + 32 : j1;
             auto blocks = [&](int j, int &q0, int &q1) {
-                const int jj = j < jend ? j : jend - 1; // past the end: the last pair again, multiplied by zeros
+                const int jj = j < jend ? j : jend - 1; // past the end: the last pair again, not used
                 q0 = p0 + 2 * jj;
                 q1 = q0 < last ? q0 + 1 : q0; // a single block pairs with itself
             };
             auto multiply = [&](int j, f16x8 a, const f16x8 (&b)[TN]) {
-                if (j >= jend) a = zero8;
-                else if (p0 + 2 * j >= last) a = sel ? zero8 : a; // single block: the upper K half contributes nothing
+                const bool past = j >= jend; // zeros times zeros: an Inf or NaN in the B of the last pair must not meet a zero
+                a = past || (sel && p0 + 2 * j >= last) ? zero8 : a; // single block: the upper K half contributes nothing
 #pragma unroll
-                for (int t = 0; t < TN; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[t], a, acc[t], 0, 0, 0);
+                for (int t = 0; t < TN; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(past ? zero8 : b[t], a, acc[t], 0, 0, 0);
             };
             for (int j = jw; j < jend; j += NP) { // the operands of NP pairs at once; a run is seldom more than one batch
                 f16x8 a[NP], b[NP][TN];
@@ -332,7 +332,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
 // operands of two block pairs in flight, so a row of five pairs costs four memory latencies one after the other
 // and the launch is over before the chip is busy.  Here a wavefront asks for the operands of all its pairs
 // (at most NP) at once: work item -> column indices -> operands, three latencies, then NP x TN MFMAs (pairs past
-// the end of the row multiply zeros).  Whole block rows only (dst < 0), B in place.
+// the end of the row are zeros times zeros).  Whole block rows only (dst < 0), B in place.
 template <int TN, bool C_F32, int NP>
 __global__ __launch_bounds__(256) void spmm_rowwise_short_kernel(
     const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_idx,
@@ -378,7 +378,7 @@ __global__ __launch_bounds__(256) void spmm_rowwise_short_kernel(
         f16x8 a[NP], b[NP][TN];
 #pragma unroll
         for (int j = 0; j < NP; j++) {
-            const int jj = j < npair ? j : npair - 1; // past the end: the last pair again, multiplied by zeros below
+            const int jj = j < npair ? j : npair - 1; // past the end: the last pair again, not used
             const int second = (2 * jj + 1 < cnt) ? 2 * jj + 1 : 2 * jj; // a single block pairs with itself
             const int c0 = __builtin_amdgcn_readlane(myc, 2 * jj);
             const int c1 = __builtin_amdgcn_readlane(myc, second);
@@ -392,10 +392,10 @@ __global__ __launch_bounds__(256) void spmm_rowwise_short_kernel(
 #pragma unroll
         for (int j = 0; j < NP; j++) {
             f16x8 aj = a[j];
-            if (j >= npair) aj = zero8;
-            else if (2 * j + 1 >= cnt) aj = sel ? zero8 : aj; // single block: the upper K half contributes nothing
+            const bool past = j >= npair; // zeros times zeros: an Inf or NaN in the B of the last pair must not meet a zero
+            aj = past || (sel && 2 * j + 1 >= cnt) ? zero8 : aj; // single block: the upper K half contributes nothing
 #pragma unroll
-            for (int t = 0; t < TN; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[j][t], aj, acc[t], 0, 0, 0);
+            for (int t = 0; t < TN; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(past ? zero8 : b[j][t], aj, acc[t], 0, 0, 0);
         }
     }
     // acc[t][r] = C[br*16 + i16][n0 + ncol_of(t, 4*g + r)]: 4*TN consecutive columns per lane, as in the kernel above

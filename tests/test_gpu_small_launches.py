@@ -37,3 +37,25 @@ def test_shared_items_match_the_oracle(smat, cuda, oracle, N, kernel, c_f32):
         torch.cuda.synchronize()
         if plan.info()["split_rows"] == 0:
             assert torch.equal(C, C2)
+
+
+# even numbers of blocks: every pair is complete, so a column of B that is Inf gives Inf (the values of A are positive)
+@pytest.mark.parametrize("lengths", [[2, 4, 6, 8, 10, 0, 4, 2] * 8, [2, 4, 14, 24, 26, 30, 46, 64, 66, 126, 128, 140]])
+@pytest.mark.parametrize("N", [8, 40, 72, 200])
+@pytest.mark.parametrize("kernel", [3, 4])
+def test_infinities_under_complete_pairs_stay_infinities(smat, cuda, lengths, N, kernel):
+    import torch
+    A = gen.random_bcsr(len(lengths), 144, 0.0, seed=N, row_lengths=lengths)
+    M, K, nnzb = A["M"], A["K"], A["nnzb"]
+    val = np.full(nnzb * 256, np.float16(0.5)).view(np.uint16)
+    B = np.full((N, K), np.float16(0.25))
+    B[3] = np.inf
+    vals, rp, ci, Bd = (to_dev(torch, x, cuda) for x in (val, A["b_row_ptr"].astype(np.int32), A["b_col_idx"].astype(np.int32), B.view(np.uint16)))
+    plan = smat.Plan(A["b_row_ptr"], M, K, nnzb, N, col_idx_host=A["b_col_idx"], kernel=kernel)
+    want = np.repeat(2.0 * np.array(lengths, np.float32), 16)[:, None].repeat(N, 1)  # 16 products of 0.5 * 0.25 a block
+    want[:, 3] = np.where(np.repeat(lengths, 16) > 0, np.inf, 0)
+    for p in (plan, None) if kernel == 3 else (plan,):
+        C = torch.full((M, N), float("nan"), dtype=torch.float32, device=cuda)
+        smat.spmm(vals, rp, ci, Bd, C, M, N, K, nnzb, plan=p, kernel=kernel, c_f32=True)
+        torch.cuda.synchronize()
+        assert np.array_equal(C.cpu().numpy(), want)
