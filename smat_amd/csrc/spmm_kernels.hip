@@ -566,16 +566,23 @@ unsigned XcdDeal::run(size_t n_items, int n_panels) const
 // panel reads the blocks again.  Enough are 768 to 1000 with long items; items of fewer than 32 blocks are over so soon
 // that a panel wider than 64 columns wants 4000 (measured: 512 items of 115 blocks, N = 256 / 512: 128 / 256 columns win, 45
 // against 51 and 73 against 80 us; 1250 items of 14 blocks, N = 256: 64 columns, 19.7 against 21.6 us; 48 items of 51
-// blocks, N = 1024: 64 columns, 9.9 against 31 us for 256).  Lists with split rows are uneven in more than their
-// items' lengths: 64 columns (R-MAT scale 16, N = 512: 618 against 944 us; scale 20, N = 128: 13.8 against 18.2 ms).
-int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, bool split_rows)
+// blocks, N = 1024: 64 columns, 9.9 against 31 us for 256).  Below that go
+//   SPLIT    lists with split rows, uneven in more than their items' lengths: 64 columns (R-MAT scale 16, N = 512: 618
+//            against 944 us; scale 20, N = 128: 13.8 against 18.2 ms);
+//   UNKNOWN  whole block rows without a plan: the heaviest row may be many times the average and is one wavefront per
+//            panel, so no wider than 64 columns below N = 512 and 128 below 1024 (R-MAT scale 16, 16 a row: N = 128 1,406
+//            against 2,609 us with 128, N = 256 1,584 against 3,307 with 256; scale 14, N = 512 806 against 975 with 256);
+//   in place no wider than 4 MiB of B, an L2, unless N alone allows it (16384^2, 15 %, N = 384: 270, 257, 344 us with 64, 128,
+//            256 columns; 16384^2, 5 %, N = 256: 66.5, 64.9, 68.2; 8192^2, 10 %, N = 256, where 256 columns fit: 37.2, -, 36.3).
+int rowwise_panel_tiles(size_t N, size_t K, size_t n_items, size_t avg_blocks, RowLengths lengths, bool packed)
 {
     if (N < 32) return 1;
     if (N < 64) return 2;
-    if (split_rows) return 4;
+    if (lengths == RowLengths::SPLIT) return 4;
     const size_t few = 768, many = avg_blocks < 32 ? 4000 : 1000;
-    if (N >= 256 && n_items * ((N + 255) / 256) >= (N >= 1024 ? few : many)) return 16;
-    if (N >= 128 && n_items * ((N + 127) / 128) >= (N >= 512 ? few : many)) return 8;
+    auto fits = [&](size_t tiles) { return lengths != RowLengths::UNKNOWN && (packed || K * 32 * tiles <= (size_t)4 << 20); };
+    if (N >= 256 && (N >= 1024 || fits(16)) && n_items * ((N + 255) / 256) >= (N >= 1024 ? few : many)) return 16;
+    if (N >= 128 && (N >= 512 || fits(8)) && n_items * ((N + 127) / 128) >= (N >= 512 ? few : many)) return 8;
     return 4;
 }
 
@@ -649,7 +656,8 @@ hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st)
         else if (a.N < 64) e = launch_rowwise_split<2>(a, st);
         else e = launch_rowwise_split<4>(a, st);
     } else {
-        switch (rowwise_panel_tiles(a.N, n_items, avg, a.n_split_rows > 0)) {
+        const RowLengths lengths = a.n_split_rows > 0 ? RowLengths::SPLIT : a.items ? RowLengths::EVEN : RowLengths::UNKNOWN;
+        switch (rowwise_panel_tiles(a.N, a.K, n_items, avg, lengths, a.b_packed != nullptr)) {
         case 16: e = launch_rowwise_tn<16>(a, st); break;
         case 8: e = launch_rowwise_tn<8>(a, st); break;
         case 4: e = launch_rowwise_tn<4>(a, st); break;
@@ -679,3 +687,9 @@ hipError_t launch_reduce(const float *workspace, const SplitRow *split_rows, int
 }
 
 } // namespace smat
+
+// Test hook (not part of smat.h): the panel width of the row-wise kernel in tiles of 16 columns; lengths as in RowLengths.
+extern "C" int smat_internal_rowwise_panel(size_t N, size_t K, size_t n_items, size_t avg_blocks, int lengths, int packed)
+{
+    return smat::rowwise_panel_tiles(N, K, n_items, avg_blocks, static_cast<smat::RowLengths>(lengths), packed != 0);
+}
