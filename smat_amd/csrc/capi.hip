@@ -118,6 +118,9 @@ extern "C" void smat_internal_alloc_counts(int64_t *out)
 // Test hook (not part of smat.h): the library's n-th device allocation from now on (0 = the next) fails; < 0: none does.
 extern "C" void smat_internal_fail_alloc(int64_t n) { g_dev_fail_in.store(n); }
 
+// Test hook (not part of smat.h): block rows that the compact kernel's list of this plan splits, -1 without a list.
+extern "C" int smat_internal_compact_split_rows(const smat_plan *p) { return p->compact ? p->compact->n_split_rows : -1; }
+
 extern "C" const char *smat_version(void) { return "smat-amd 0.1 gfx950"; }
 
 static int check_shapes(const void *vals, const void *row_ptr, const void *col_idx, const void *B,

@@ -55,7 +55,7 @@ int g_force_tq = 0; // test hook: 1 or 2 = panels of 64 or 128 columns whatever 
 
 constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts as full (of 16)
 constexpr int TASK_STEPS = 12;     // short items are put together up to this many steps (8 to 24: level; one item each: 9 % slower on R-MAT)
-constexpr int MAX_TASK_STEPS = 56; // of a task of the product kernel: the entry ranges of 64 steps come in at once, some of them read ahead
+constexpr int LONG_ROW_STEPS = 56; // steps from which a block row is split where a launch has few wavefronts
 constexpr int LIST_PAD = 2304; // entries readable past the end of the list (the index loads of the 64-column panel run up to 16 steps ahead)
 
 // ---- census of nonzero block columns ----
@@ -413,24 +413,25 @@ __global__ __launch_bounds__(256) void spmm_compact_kernel(
         int n;                     // the step's entries
         u32x4 L[TQ][4];
     };
-    int2 ranges = {0, 0}; // entries of the steps from range_base + lane on: a task has at most MAX_TASK_STEPS
-    const int range_base = e >> 5;
+    int2 ranges = {0, 0}; // entries of the step range_from + lane
+    const int first_step = e >> 5;
+    int range_from = first_step;
     if constexpr (AF > 0) {
         *reinterpret_cast<u32x4 *>(a_tile + lane * 16) = (u32x4){0u, 0u, 0u, 0u};
-        ranges = step_range[range_base + lane];
+        ranges = step_range[range_from + lane];
     }
     // The indices of 8 steps are 1 KiB, one load, and go to one half of 2 KiB of LDS, from where each lane takes the four of
     // its octet (an instruction that brings 128 bytes costs the vector memory path as much as one that brings 1 KiB).
     unsigned char *const i_tile = lds[wave] + A_BYTES + B_BYTES;
     auto load_block = [&](int s) { return reinterpret_cast<const u32x4 *>(cols + s)[lane]; };
-    auto put_block = [&](int s, u32x4 x) { *reinterpret_cast<u32x4 *>(i_tile + (((s >> 5) - range_base) & 8) * 128 + lane * 16) = x; };
-    auto indices = [&](int s) { return *reinterpret_cast<const u32x4 *>(i_tile + (((s >> 5) - range_base) & 15) * 128 + oct * 16); };
+    auto put_block = [&](int s, u32x4 x) { *reinterpret_cast<u32x4 *>(i_tile + (((s >> 5) - first_step) & 8) * 128 + lane * 16) = x; };
+    auto indices = [&](int s) { return *reinterpret_cast<const u32x4 *>(i_tile + (((s >> 5) - first_step) & 15) * 128 + oct * 16); };
     auto request = [&](int s, const u32x4 x, Operands &o) {
         if constexpr (AF == 0) {
             o.aw = *reinterpret_cast<const u32x4 *>(acol + ((long)(s >> 3) + g) * 128 + i16 * 8);
         } else {
-            const int first = __builtin_amdgcn_readlane(ranges.x, (s >> 5) - range_base);
-            o.n = __builtin_amdgcn_readlane(ranges.y, (s >> 5) - range_base) - first;
+            const int first = __builtin_amdgcn_readlane(ranges.x, (s >> 5) - range_from);
+            o.n = __builtin_amdgcn_readlane(ranges.y, (s >> 5) - range_from) - first;
 #pragma unroll
             for (int u = 0; u < AF; u++) o.ent[u] = (entries + (long)first + 64 * u)[lane]; // past the step's end: the next step's, unused
         }
@@ -540,11 +541,21 @@ __global__ __launch_bounds__(256) void spmm_compact_kernel(
     request(e, indices(e), op_a);
     int next = e + 32; // the step whose operands are asked for
     u32x4 x = indices(next); // read from LDS a step before they are used
+    // Before the first step that `ranges` does not reach (every 64 steps): the ranges of 64 steps from there on.  The wait for
+    // them is inside, so that no other step has one; a task of up to 62 steps never gets here.
+    auto more_ranges = [&] {
+        if (AF > 0 && (next >> 5) - range_from >= 60) {
+            range_from = next >> 5;
+            ranges = step_range[range_from + lane];
+            asm volatile("" : "+v"(ranges.x), "+v"(ranges.y));
+        }
+    };
     while (true) {
 #define SMAT_STEP_OF(CUR, NEW)                                                                         \
         if (((next + 32 - tk.z) & 255) == 0) {                                                         \
             put_block(next + 32, block);                                                               \
             block = load_block(next + 288);                                                            \
+            more_ranges();                                                                             \
         }                                                                                              \
         asm volatile("" ::: "memory");                                                                 \
         request(next, x, NEW);                                                                         \
@@ -959,14 +970,19 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
             }
         }
     }
-    // work items: whole block rows; rows much longer than the average in chunks of 32-column steps
+    // Work items: whole block rows; rows much longer than the average in chunks of 32-column steps, all of a row's about
+    // as long.  Long rows that are all alike stay whole: their partial tiles are 2 * 16 * N floats to write and read again
+    // for each (32768 x 65536, 131 a row, N = 256: 138 us whole, 191 in chunks of 1792 columns; 8192 x 65536, 140 a row,
+    // N = 1024: 175 against 241) - except where whole rows would be fewer than four wavefronts a CU (2048 x 65536, 140 a row,
+    // N = 256, 512 wavefronts: 43 us whole, 34 in halves; 512 x 65536, 300 a row, N = 1024, 512 of them: 96 against 75).
     const std::vector<int32_t> &cc_host = padded;
     size_t nonempty = 0;
     for (size_t i = 0; i < mb; i++) nonempty += cc_host[i + 1] > cc_host[i];
     const double avg = nonempty ? (double)total / (double)nonempty : 0.0;
     long chunk = (long)(4.0 * avg + 0.5);
     chunk = std::max(chunk, 512L);
-    chunk = std::min((chunk + 31) / 32 * 32, 32L * MAX_TASK_STEPS);
+    chunk = (chunk + 31) / 32 * 32;
+    if (nonempty * ((n_cap + 63) / 64) < 1024) chunk = std::min(chunk, 32L * LONG_ROW_STEPS);
     std::vector<WorkItem> items;
     std::vector<SplitRow> split;
     int slot = 0;
@@ -974,8 +990,9 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         const long len = cc_host[i + 1] - cc_host[i];
         if (len <= chunk || dense[i]) continue;
         SplitRow sr{(int32_t)i, slot, slot, 0};
-        for (long b = cc_host[i]; b < cc_host[i + 1]; b += chunk)
-            items.push_back(WorkItem{(int32_t)i, (int32_t)b, (int32_t)std::min<long>(b + chunk, cc_host[i + 1]), slot++});
+        const long pieces = (len + chunk - 1) / chunk, piece = (len / 32 + pieces - 1) / pieces * 32;
+        for (long b = cc_host[i]; b < cc_host[i + 1]; b += piece)
+            items.push_back(WorkItem{(int32_t)i, (int32_t)b, (int32_t)std::min<long>(b + piece, cc_host[i + 1]), slot++});
         sr.slot_end = slot;
         split.push_back(sr);
     }

@@ -112,6 +112,16 @@ class Oracle:
         self.h.orc_compare_f16_vs_f32(_p(c), _p(r), r.shape[0], r.shape[1], _p(out))
         return tuple(out)
 
+    def assert_fp32_close(self, C, want, N, K, A, B):
+        """An fp32 result against the oracle's, element by element.  Products of two halves are exact in fp32; a sum of n
+        of them is off by at most n roundings of partial sums, each no larger than the sum of the magnitudes: 2^-24 of it
+        each in the oracle, 2^-23 in a matrix unit, which may cut off instead of rounding."""
+        mag = self.spmm_bcsr(A["M"], N, K, A["b_row_ptr"], A["b_col_idx"], A["b_val"] & 0x7FFF, B & 0x7FFF, threads=4)
+        n = 16 * np.diff(A["b_row_ptr"]).repeat(16)
+        bound = n[:, None] * (2.0 ** -24 + 2.0 ** -23) * mag.astype(np.float64)
+        err = np.abs(C.astype(np.float64) - want)
+        assert C.dtype == np.float32 and (err <= bound).all(), (err - bound).max()
+
     def max_threads(self):
         return self.h.orc_max_threads()
 

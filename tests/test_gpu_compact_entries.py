@@ -54,3 +54,43 @@ def test_lists_of_nonzeros_match_the_oracle(smat, cuda, oracle, fill, N, c_f32, 
         finally:
             smat.lib.smat_internal_compact_panel(0)
         assert oracle.compare(C.half().cpu().numpy().view(np.uint16), want)[0] <= 1e-3
+
+
+# block rows of up to 260 steps: around what one load of entry ranges covers (64 steps), and around two
+STEPS = [1, 7, 60, 61, 62, 63, 64, 65, 66, 71, 126, 127, 128, 129, 130, 131, 191, 193, 260]
+
+
+@pytest.mark.parametrize("fill", [1, 2])
+@pytest.mark.parametrize("K", [8448, 4080])
+@pytest.mark.parametrize("N", [64, 200])
+@pytest.mark.parametrize("n_hint", [0, 4096])
+def test_long_even_block_rows(smat, cuda, oracle, fill, K, N, n_hint):
+    """K = 8448: lists of nonzeros; K = 4080: whole columns.  A plan for a wide product has wavefronts enough and leaves the
+    rows whole, one for N columns splits them."""
+    import torch
+    rng = np.random.default_rng(fill)
+    lengths = [min(2 * s, K // 16) for s in STEPS]  # blocks with all their columns: two a step
+    A = gen.random_bcsr(len(lengths), K // 16, 0.0, seed=fill, row_lengths=lengths)
+    M, nnzb = A["M"], A["nnzb"]
+    v = A["b_val"].reshape(-1, 16, 16).copy()
+    keep = np.zeros((nnzb, 16, 16), bool)
+    for _ in range(fill):
+        keep[np.arange(nnzb)[:, None], rng.integers(0, 16, (nnzb, 16)), np.arange(16)[None, :]] = True
+    v[~keep] = 0
+    A["b_val"] = v.reshape(-1)
+    B = gen.dense_b(K, N, seed=N)
+    vals, rp, ci, Bd = (to_dev(torch, x, cuda) for x in (A["b_val"], A["b_row_ptr"].astype(np.int32), A["b_col_idx"].astype(np.int32), B))
+    want = oracle.spmm_bcsr(M, N, K, A["b_row_ptr"], A["b_col_idx"], A["b_val"], B, threads=4)
+    for tq in (1, 2):
+        smat.lib.smat_internal_compact_panel(tq)
+        try:
+            C = torch.full((M, N), float("nan"), dtype=torch.float32, device=cuda)
+            plan = smat.Plan(A["b_row_ptr"], M, K, nnzb, n_hint or N, col_idx_host=A["b_col_idx"], kernel=5)
+            plan.attach_values(vals, rp, ci)
+            split = smat.lib.smat_internal_compact_split_rows(plan.handle)
+            assert split == 0 if n_hint else split == sum(min(s, K // 32) > 56 for s in STEPS)
+            smat.spmm(vals, rp, ci, Bd, C, M, N, K, nnzb, plan=plan, kernel=5, c_f32=True)
+            torch.cuda.synchronize()
+        finally:
+            smat.lib.smat_internal_compact_panel(0)
+        oracle.assert_fp32_close(C.cpu().numpy(), want, N, K, A, B)
