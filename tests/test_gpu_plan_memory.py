@@ -74,10 +74,11 @@ def test_clearing_the_plan_cache_gives_kept_memory_back(smat, cuda):
     smat.lib.smat_plan_cache_clear()
     free = torch.cuda.mem_get_info()[0]
     big = 256 << 20
+    slack = 16 << 20  # the runtime holds chunks of 2 MiB of its own that an allocation may come out of in part
     p = C.c_void_p()
     assert smat.lib.smat_malloc(C.byref(p), big) == 0
-    assert torch.cuda.mem_get_info()[0] <= free - big
+    assert torch.cuda.mem_get_info()[0] <= free - big + slack
     assert smat.lib.smat_free(p) == 0
-    assert torch.cuda.mem_get_info()[0] <= free - big  # kept
+    assert torch.cuda.mem_get_info()[0] <= free - big + slack  # kept
     assert smat.lib.smat_plan_cache_clear() == 0
-    assert torch.cuda.mem_get_info()[0] >= free
+    assert torch.cuda.mem_get_info()[0] >= free - slack
