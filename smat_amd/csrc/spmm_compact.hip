@@ -51,6 +51,7 @@ namespace {
 int g_force_run = 0;
 int g_tune = 1; // test hook: 0 = attaching values measures nothing, the estimate decides the deal
 int g_last_run = 0; // test hook: the run length of the latest launch
+int g_force_list = 0; // test hook: 1 = lists of whole columns, 2 = of nonzeros, 0 = compact_build decides
 int g_force_tq = 0; // test hook: 1 or 2 = panels of 64 or 128 columns whatever the sizes say, 0 = the launcher decides
 
 constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts as full (of 16)
@@ -863,6 +864,23 @@ hipError_t compact_full_blocks(const CompactCensus &s, std::vector<uint8_t> &ful
     return e;
 }
 
+// Whether the nonzeros are listed one by one (4 bytes each, and 8 per step) instead of whole columns (32 bytes each): a step of
+// random sparse columns, one nonzero each, is then 152 bytes of A instead of 1024, of the 4 to 5 KiB that the vector L1
+// returns for it, but its operand takes two trips through LDS.  Over 250 drawn random matrices (rows 1,024 to 65,536, K 512 to
+// 32,768, 3 to 90 nonzeros a row, N 32 to 2,048, either layout of B) this rule is 0.6 % from the better of the two in the
+// mean, a rule by K alone (>= 4096) 2.5 %:
+//   * the trips through LDS are what a wavefront waits for where there are fewer than five on a CU (whole columns / nonzeros, us:
+//     8192 x 4096, 40 a row, N = 128 10.4 / 11.6; R-MAT scale 12, N = 64 11.5 / 13.5);
+//   * with more, the nonzeros win while they are few per column (65536 x 512, 8 a row, N = 512 43.4 / 38.9; 59328 x 27344, 17.5 a
+//     row, N = 288 76 / 55; at 2.3 per column 4096 x 512, 64 a row, N = 1024 they lose, 15.2 / 17.0);
+//   * columns with more nonzeros pay while the list of whole columns stays in the eight L2s of 4 MiB (27-point stencil, 2.8 per
+//     column: 32^3, 300 k columns, N = 256 22.5 / 23.9; 48^3, 1.05 M, 70.8 / 62.8; 64^3, 2.5 M, N = 64 47.8 / 42.5).
+static bool lists_nonzeros(int64_t nnz, int64_t n_cols, size_t n_rows, size_t N)
+{
+    if (n_rows * ((N + 63) / 64) < 5 * 256) return false;
+    return 2 * nnz <= 3 * n_cols || (n_cols >= 1000000 && nnz <= 4 * n_cols);
+}
+
 hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx, size_t K, size_t n_cap,
                          const std::vector<uint8_t> *leave_rows, bool drop_full, CompactPlan **out)
 {
@@ -885,6 +903,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     // Block rows left to a dense kernel get no list and no work item here; the others are padded to a multiple of 32
     // columns (one MFMA step) with zero columns.
     int64_t total = 0, n_cols = 0, nnz = 0;
+    size_t n_rows = 0; // block rows with listed columns
     std::vector<int32_t> padded(mb + 1, 0);
     std::vector<int2> start(mb + 1); // what the gather kernel sees: list and entries of the row, -1 for rows without a list
     for (size_t i = 0; i < mb; i++) {
@@ -894,6 +913,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
             const uint64_t d = s.raw[i + 1] - s.raw[i];
             total += ((int64_t)(uint32_t)d + 31) / 32 * 32;
             n_cols += (int64_t)(uint32_t)d;
+            n_rows += (uint32_t)d != 0;
             nnz += (int64_t)(d >> 32);
         }
         if (total > 0x7fffff00) e = hipErrorInvalidValue;
@@ -901,13 +921,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     padded[mb] = (int32_t)total;
     start[mb] = int2{(int32_t)total, (int32_t)nnz};
     p->n_cols = n_cols;
-    // The nonzeros one by one (4 bytes each, and 8 per step) while that is at most half of the 32 bytes per column that
-    // whole columns take: about one nonzero per column in random sparse matrices (a step of 36 entries: 152 bytes for
-    // 1024), 2.8 in the 27-point stencil (368 bytes).  Where the panels of B are small enough to stay in the L2 (K below
-    // 4096) it is the LDS that binds, and whole columns, which do not go through it, win (24352 x 1376, 22 a row, N = 72:
-    // 13.7 against 14.5 us; 16384^2, N = 256, the other way round: 18.9 against 16.3; 65536 x 4096, 8 a row, N = 512: 50.3 against
-    // 43.7, 16384 x 4096, 16 a row, N = 256: 14.5 against 14.7).
-    const bool by_entry = nnz <= 4 * n_cols && K >= 4096 && s.nnz < 0x7fffff00;
+    const bool by_entry = s.nnz < 0x7fffff00 && (g_force_list ? g_force_list == 2 : lists_nonzeros(nnz, n_cols, n_rows, n_cap));
     const size_t cap = (size_t)total + LIST_PAD;
     SMAT_STEP(dev_malloc(&p->d_cols, cap * sizeof(int32_t)));
     SMAT_STEP(hipMemsetAsync(p->d_cols, 0, cap * sizeof(int32_t), nullptr)); // padding: row 0 of B
@@ -1061,6 +1075,8 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
 // Test hook (not part of smat.h): 1 or 2 = the compact kernel works on panels of 64 or 128 columns whatever the sizes
 // say (each width has its own way of gathering the rows of B), 0 = the launcher decides (the default).
 extern "C" void smat_internal_compact_panel(int tq) { smat::g_force_tq = tq; }
+// Test hook: 1 = lists of whole columns, 2 = of nonzeros (where their number allows it), 0 = as the sizes say (the default).
+extern "C" void smat_internal_compact_list(int what) { smat::g_force_list = what; }
 // Test hooks for the deal of the compact kernel's workgroups to the XCDs: a run length that every launch uses
 // (0 = chosen per plan and number of panels), the run length of the latest launch, and the choice itself for a list
 // of item costs (host only).

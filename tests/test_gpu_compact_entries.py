@@ -12,8 +12,15 @@ def to_dev(torch, a, cuda):
     return torch.from_numpy(np.ascontiguousarray(a).view(np.int16) if a.dtype == np.uint16 else np.ascontiguousarray(a)).to(cuda)
 
 
+@pytest.fixture
+def lists(smat):
+    """lists(1): plans list whole columns; lists(2): nonzeros one by one (how many wavefronts and nonzeros decides otherwise)."""
+    yield smat.lib.smat_internal_compact_list
+    smat.lib.smat_internal_compact_list(0)
+
+
 def matrix(fill, seed):
-    """Block rows of 0 .. 70 blocks, K above 4096 (lists of nonzeros), fill nonzeros per nonzero column on average:
+    """Block rows of 0 .. 70 blocks, fill nonzeros per nonzero column on average:
     one row or several of a column; some block rows hold full columns, so that a step has up to 512 entries."""
     rng = np.random.default_rng(seed)
     mb, kb = 40, 300
@@ -34,8 +41,9 @@ def matrix(fill, seed):
 @pytest.mark.parametrize("fill", [1.0, 2.5])
 @pytest.mark.parametrize("N", [8, 64, 136])
 @pytest.mark.parametrize("c_f32,row_major", [(False, False), (True, False), (False, True)])
-def test_lists_of_nonzeros_match_the_oracle(smat, cuda, oracle, fill, N, c_f32, row_major):
+def test_lists_of_nonzeros_match_the_oracle(smat, cuda, oracle, lists, fill, N, c_f32, row_major):
     import torch
+    lists(2)
     A = matrix(fill, 7 + N)
     M, K, nnzb = A["M"], A["K"], A["nnzb"]
     B = gen.dense_b(K, N, seed=N + 1)
@@ -61,13 +69,14 @@ STEPS = [1, 7, 60, 61, 62, 63, 64, 65, 66, 71, 126, 127, 128, 129, 130, 131, 191
 
 
 @pytest.mark.parametrize("fill", [1, 2])
-@pytest.mark.parametrize("K", [8448, 4080])
+@pytest.mark.parametrize("what,K", [(2, 8448), (1, 8448), (1, 4080)])
 @pytest.mark.parametrize("N", [64, 200])
 @pytest.mark.parametrize("n_hint", [0, 4096])
-def test_long_even_block_rows(smat, cuda, oracle, fill, K, N, n_hint):
-    """K = 8448: lists of nonzeros; K = 4080: whole columns.  A plan for a wide product has wavefronts enough and leaves the
+def test_long_even_block_rows(smat, cuda, oracle, lists, fill, what, K, N, n_hint):
+    """Lists of nonzeros and of whole columns.  A plan for a wide product has wavefronts enough and leaves the
     rows whole, one for N columns splits them."""
     import torch
+    lists(what)
     rng = np.random.default_rng(fill)
     lengths = [min(2 * s, K // 16) for s in STEPS]  # blocks with all their columns: two a step
     A = gen.random_bcsr(len(lengths), K // 16, 0.0, seed=fill, row_lengths=lengths)

@@ -21,7 +21,7 @@ def held(smat):
 
 
 def split_in_steps(seed):
-    """K for lists of nonzeros, columns with up to 16 of them: groups of 32 columns that take several steps."""
+    """Columns with up to 16 nonzeros: in lists of nonzeros, groups of 32 columns that take several steps."""
     rng = np.random.default_rng(seed)
     A = gen.random_bcsr(24, 300, 0.1, seed=seed)
     v = A["b_val"].reshape(-1, 16, 16).copy()
@@ -38,6 +38,7 @@ def test_attach_values_survives_every_failing_allocation(smat, cuda, oracle):
     import torch
     lib = smat.lib
     lib.smat_internal_fail_alloc.argtypes = [C.c_int64]
+    lib.smat_internal_compact_list(2)  # the lists with the most allocations
     A = split_in_steps(3)
     M, K, nnzb, N = A["M"], A["K"], A["nnzb"], 72
     B = gen.dense_b(K, N, seed=1)
@@ -64,6 +65,7 @@ def test_attach_values_survives_every_failing_allocation(smat, cuda, oracle):
         failures += 1
         assert plan.info()["kernel"] == smat.KERNEL_ROWWISE
         assert held(smat) <= before + 1, f"device blocks lost by failing allocation {n}"  # the copy of B may stay for the next attempt
+    lib.smat_internal_compact_list(0)
     assert failures >= 15 and plan.info()["kernel"] == smat.KERNEL_COMPACT
     plan.close()
 
