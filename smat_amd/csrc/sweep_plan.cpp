@@ -234,6 +234,14 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
             sum_of_caps(&caps);
         }
 
+        // where the rows of C are: also those of a group without a block, which the kernel fills with zeros
+        for (int w = 0; w < WAVES; w++)
+            for (int lr = 0, r = 0; lr < G; lr++)
+                if (wave_of[lr] == w) {
+                    if (r_begin + (size_t)lr < r_end) out.row_map[(rg * WAVES + (size_t)w) * RW + (size_t)r] = (int32_t)row_at(r_begin + (size_t)lr);
+                    r++;
+                }
+
         struct Pending { int32_t last, first, seq, row, hi; SweepOpHost op; };
         std::vector<std::vector<std::vector<Ranked>>> schedule((size_t)WAVES, std::vector<std::vector<Ranked>>(n_chunks));
         if (n_chunks > 0) {
@@ -242,7 +250,6 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
                 int r = 0;
                 for (int lr = 0; lr < G; lr++) {
                     if (wave_of[lr] != w) continue;
-                    if (r_begin + (size_t)lr < r_end) out.row_map[(rg * WAVES + (size_t)w) * RW + (size_t)r] = (int32_t)row_at(r_begin + (size_t)lr);
                     for (const RowOp &ro : row_ops[lr]) todo.push_back(Pending{ro.last, ro.first, (int32_t)todo.size(), r, ro.hi, ro.op});
                     r++;
                 }
@@ -375,14 +382,14 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
 // allocated with malloc; release each with smat_host_free.  row_map: n_rg * 64 block rows (-1 = none).  counts[0..5] = row groups, listed
 // chunks, stream entries (ops, fillers, ends; without padding), pairs, singles, fillers.
 static int smat_internal_sweep_plan_impl(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K,
-                                         const int32_t *rows, size_t n_rows, int32_t **rg_chunk_ptr, int32_t **chunk_ids, int32_t **op_ptr,
+                                         const int32_t *rows, size_t n_rows, size_t group_rows, int32_t **rg_chunk_ptr, int32_t **chunk_ids, int32_t **op_ptr,
                                          uint32_t **ops, int32_t **row_map, int64_t *counts)
 {
     if (!row_ptr || !col_idx || !rg_chunk_ptr || !chunk_ids || !op_ptr || !ops || !row_map || !counts) return SMAT_ERR_INVALID;
     if (M == 0 || M % 16 || K % 16 || row_ptr[M / 16] < 2) return SMAT_ERR_INVALID;
     smat::SweepPlanHost p;
     try {
-        smat::build_sweep_plan(row_ptr, col_idx, M / 16, K / 16, p, rows, n_rows);
+        smat::build_sweep_plan(row_ptr, col_idx, M / 16, K / 16, p, rows, n_rows, group_rows);
     } catch (...) {
         return SMAT_ERR_NOMEM;
     }
@@ -416,5 +423,16 @@ extern "C" int smat_internal_sweep_plan(const int32_t *row_ptr, const int32_t *c
                                          const int32_t *rows, size_t n_rows, int32_t **rg_chunk_ptr, int32_t **chunk_ids, int32_t **op_ptr,
                                          uint32_t **ops, int32_t **row_map, int64_t *counts)
 {
-    return smat::guarded("smat_internal_sweep_plan", [&] { return smat_internal_sweep_plan_impl(row_ptr, col_idx, M, K, rows, n_rows, rg_chunk_ptr, chunk_ids, op_ptr, ops, row_map, counts); });
+    return smat::guarded("smat_internal_sweep_plan", [&] {
+        return smat_internal_sweep_plan_impl(row_ptr, col_idx, M, K, rows, n_rows, smat::SWEEP_G, rg_chunk_ptr, chunk_ids, op_ptr, ops, row_map, counts);
+    });
+}
+// The same on row groups of group_rows (at most 64) block rows.
+extern "C" int smat_internal_sweep_plan_groups(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t group_rows,
+                                               int32_t **rg_chunk_ptr, int32_t **chunk_ids, int32_t **op_ptr, uint32_t **ops,
+                                               int32_t **row_map, int64_t *counts)
+{
+    return smat::guarded("smat_internal_sweep_plan_groups", [&] {
+        return smat_internal_sweep_plan_impl(row_ptr, col_idx, M, K, nullptr, 0, group_rows, rg_chunk_ptr, chunk_ids, op_ptr, ops, row_map, counts);
+    });
 }

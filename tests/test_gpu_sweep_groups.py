@@ -53,3 +53,23 @@ def test_bands_match_the_oracle(smat, cuda, oracle, m, bandwidth, N):
     torch.cuda.synchronize()
     want = oracle.spmm_bcsr(A.M, N, A.K, A.row_ptr, A.col_idx, A.val, B, threads=4)
     assert oracle.compare(C.cpu().numpy().view(np.uint16), want)[0] <= 1e-3
+
+
+@pytest.mark.parametrize("c_f32", [False, True])
+def test_row_groups_without_a_block_give_zeros(smat, cuda, oracle, c_f32):
+    import torch
+    lengths = [0 if 64 <= r < 128 else 3 for r in range(16 * 64)]  # the second of 16 groups of 64 block rows is empty
+    A = gen.random_bcsr(len(lengths), 33, 0.0, seed=5, row_lengths=lengths)
+    M, K, nnzb, N = A["M"], A["K"], A["nnzb"], 136
+    B = gen.dense_b(K, N, seed=N)
+    vals, rp, ci, Bd = (to_dev(torch, x, cuda) for x in (A["b_val"], A["b_row_ptr"].astype(np.int32), A["b_col_idx"].astype(np.int32), B))
+    plan = smat.Plan(A["b_row_ptr"], M, K, nnzb, N, col_idx_host=A["b_col_idx"], kernel=smat.KERNEL_SWEEP)
+    C = torch.full((M, N), float("nan"), dtype=torch.float32 if c_f32 else torch.float16, device=cuda)
+    smat.spmm(vals, rp, ci, Bd, C, M, N, K, nnzb, plan=plan, kernel=smat.KERNEL_SWEEP, c_f32=c_f32)
+    torch.cuda.synchronize()
+    want = oracle.spmm_bcsr(M, N, K, A["b_row_ptr"], A["b_col_idx"], A["b_val"], B, threads=4)
+    assert (C[64 * 16:128 * 16] == 0).all()
+    if c_f32:
+        oracle.assert_fp32_close(C.cpu().numpy(), want, N, K, A, B)
+    else:
+        assert oracle.compare(C.cpu().numpy().view(np.uint16), want)[0] <= 1e-3

@@ -27,18 +27,25 @@ LDS_MASK = 0x1C0E0
 PAD, CHUNK_PAD = 16, 4
 
 
-def sweep_plan(row_ptr, col_idx, M, K, rows=None):
-    """rows: the ascending block rows the plan is made for (what mixed dispatch hands to the sweep kernel); None = all."""
-    fn = lib.smat_internal_sweep_plan
-    fn.restype = C.c_int
-    fn.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_size_t, C.c_void_p, C.c_size_t] + [C.POINTER(C.c_void_p)] * 5 + [C.POINTER(C.c_int64)]
+def sweep_plan(row_ptr, col_idx, M, K, rows=None, group_rows=G):
+    """rows: the ascending block rows the plan is made for (what mixed dispatch hands to the sweep kernel); None = all.
+    group_rows: block rows to a row group (all rows only)."""
+    fn, fn_groups = lib.smat_internal_sweep_plan, lib.smat_internal_sweep_plan_groups
+    fn.restype = fn_groups.restype = C.c_int
+    outputs = [C.POINTER(C.c_void_p)] * 5 + [C.POINTER(C.c_int64)]
+    fn.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_size_t, C.c_void_p, C.c_size_t] + outputs
+    fn_groups.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t] + outputs
     row_ptr = np.ascontiguousarray(row_ptr, np.int32)
     col_idx = np.ascontiguousarray(col_idx, np.int32)
     rows_arr = None if rows is None else np.ascontiguousarray(rows, np.int32)
     out = [C.c_void_p() for _ in range(5)]
     counts = (C.c_int64 * 6)()
-    rc = fn(row_ptr.ctypes.data, col_idx.ctypes.data, M, K, None if rows is None else rows_arr.ctypes.data,
-            0 if rows is None else rows_arr.size, *[C.byref(o) for o in out], counts)
+    if group_rows == G:
+        rc = fn(row_ptr.ctypes.data, col_idx.ctypes.data, M, K, None if rows is None else rows_arr.ctypes.data,
+                0 if rows is None else rows_arr.size, *[C.byref(o) for o in out], counts)
+    else:
+        assert rows is None
+        rc = fn_groups(row_ptr.ctypes.data, col_idx.ctypes.data, M, K, group_rows, *[C.byref(o) for o in out], counts)
     assert rc == 0
     n_rg, n_chunks, n_ops = counts[0], counts[1], counts[2]
 
@@ -75,9 +82,9 @@ def slot_of(off):
     return slot // S, slot % S
 
 
-def replay(plan, A, Bd, rows=None):
+def replay(plan, A, Bd, rows=None, group_rows=G):
     """Runs the streams on dense numpy operands. A: dict from gen (BCSR), Bd: K x N float64.  rows: the block rows
-    the plan was made for (None = all): only their blocks may be used, 64 of them to a row group in this order."""
+    the plan was made for (None = all): only their blocks may be used, group_rows of them to a row group in this order."""
     M, K, rp, ci = A["M"], A["K"], A["b_row_ptr"], A["b_col_idx"]
     blocks = A["b_val"].view(np.float16).astype(np.float64).reshape(-1, 16, 16)
     nnzb = ci.size
@@ -183,21 +190,21 @@ def replay(plan, A, Bd, rows=None):
     assert n_fill == plan["fillers"] and n_real == plan["pairs"] + plan["singles"]
     mapped = plan["row_map"][plan["row_map"] >= 0]
     assert np.array_equal(np.sort(mapped), np.sort(subset)), "row_map is not a partition of the plan's block rows"
-    # Row group rg holds the rows subset[64 rg : 64 rg + 64] (the slots that are left say -1) - unless that grouping
+    # Row group rg holds the rows subset[g rg : g rg + g], g = group_rows (the slots that are left say -1) - unless that grouping
     # leaves one group with more than 1.08 x the blocks of an average one: then the rows are dealt out by their block
     # count, heaviest first to the lightest group with room, and every group keeps its size
     groups = [plan["row_map"][rg * G:(rg + 1) * G] for rg in range(n_rg)]
     groups = [g[g >= 0] for g in groups]
-    in_order = [row_len[subset[rg * G:(rg + 1) * G]].sum() for rg in range(n_rg)]
-    skewed = n_rg > 1 and max(in_order) * subset.size > 1.08 * sum(in_order) * G
+    in_order = [row_len[subset[rg * group_rows:(rg + 1) * group_rows]].sum() for rg in range(n_rg)]
+    skewed = n_rg > 1 and max(in_order) * subset.size > 1.08 * sum(in_order) * group_rows
     plan["dealt"] = bool(skewed)
     for rg in range(n_rg):
-        assert groups[rg].size == subset[rg * G:(rg + 1) * G].size
+        assert groups[rg].size == subset[rg * group_rows:(rg + 1) * group_rows].size
         if not skewed:
-            assert np.array_equal(np.sort(groups[rg]), np.sort(subset[rg * G:(rg + 1) * G]))
+            assert np.array_equal(np.sort(groups[rg]), np.sort(subset[rg * group_rows:(rg + 1) * group_rows]))
     if skewed:
         dealt = np.array([row_len[g].sum() for g in groups])
-        full = [rg for rg in range(n_rg) if groups[rg].size == G]
+        full = [rg for rg in range(n_rg) if groups[rg].size == group_rows]
         # no full group is heavier than the lightest full group by more than one row (what dealing heaviest-first gives)
         assert dealt[full].max() - dealt[full].min() <= row_len[subset].max()
         assert dealt.max() <= max(in_order)
@@ -272,6 +279,52 @@ def test_replay_of_a_row_subset(mb, kb, density, seed, pick):
     assert np.allclose(Cd, D @ Bd, rtol=1e-12, atol=1e-12)
     row_blocks = np.diff(A["b_row_ptr"])[rows].sum()
     assert plan["pairs"] * 2 + plan["singles"] == row_blocks
+
+
+@pytest.mark.parametrize("group_rows", [32, 16, 1])
+@pytest.mark.parametrize("mb,kb,density,seed", [(64, 64, 0.10, 1), (65, 40, 0.30, 2), (17, 200, 0.5, 4), (130, 33, 0.02, 6), (3, 3, 1.0, 7)])
+def test_replay_of_smaller_row_groups(group_rows, mb, kb, density, seed):
+    """Row groups that leave places of their 64 empty: a last group of one row, an empty and a full row, groups that list
+    one chunk only (3 x 3 blocks)."""
+    A = random_mask_matrix(mb, kb, density, seed, empty_rows=(1,) if mb > 3 else (), long_rows=(2,) if mb > 3 else ())
+    plan = sweep_plan(A["b_row_ptr"], A["b_col_idx"], A["M"], A["K"], group_rows=group_rows)
+    assert plan["rg_chunk_ptr"].size - 1 == -(-mb // group_rows)
+    Bd = np.random.default_rng(seed + 100).normal(size=(A["K"], 8))
+    Cd = replay(plan, A, Bd, group_rows=group_rows)
+    assert np.allclose(Cd, dense_of(A) @ Bd, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("group_rows", [64, 16])
+def test_row_groups_without_a_block_are_stored_too(group_rows):
+    """C is overwritten: the rows of an empty row group are in the plan, with no op and no chunk."""
+    n_groups, kb = 16, 33  # as many groups that they stay in order: the others are hardly above the average
+    empty = range(group_rows, 2 * group_rows)
+    lengths = [0 if r in empty else 3 for r in range(n_groups * group_rows)]
+    A = gen.random_bcsr(len(lengths), kb, 0.0, seed=9, row_lengths=lengths)
+    plan = sweep_plan(A["b_row_ptr"], A["b_col_idx"], A["M"], A["K"], group_rows=group_rows)
+    chunks = np.diff(plan["rg_chunk_ptr"])
+    assert chunks.tolist().count(0) == 1
+    rg = int(np.argmin(chunks))
+    rows = plan["row_map"][rg * G:(rg + 1) * G]
+    assert sorted(rows[rows >= 0]) == list(empty)
+    Bd = np.random.default_rng(1).normal(size=(A["K"], 4))
+    assert np.allclose(replay(plan, A, Bd, group_rows=group_rows), dense_of(A) @ Bd, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("group_rows", [32, 16])
+def test_uneven_rows_are_dealt_to_even_smaller_row_groups(group_rows):
+    """Density falling from 18 % to 2 %: the first groups would be far above the average, the plan deals the rows out."""
+    A = gen.block_pruned_skewed(2048, 0.18, 0.02)
+    lens = np.diff(A["b_row_ptr"])
+    in_order = lens.reshape(-1, group_rows).sum(1)
+    assert in_order.max() > 1.5 * in_order.mean()
+    plan = sweep_plan(A["b_row_ptr"], A["b_col_idx"], A["M"], A["K"], group_rows=group_rows)
+    Bd = np.random.default_rng(3).normal(size=(A["K"], 4))
+    Cd = replay(plan, A, Bd, group_rows=group_rows)
+    assert plan["dealt"]
+    assert np.allclose(Cd, dense_of(A) @ Bd, rtol=1e-12, atol=1e-12)
+    dealt = np.array([lens[g[g >= 0]].sum() for g in plan["row_map"].reshape(-1, G)])
+    assert dealt.max() < 1.03 * dealt.mean()
 
 
 def test_single_last_block_is_listed_as_second_half():
