@@ -149,27 +149,29 @@ static bool sweep_fills_device(size_t mb, size_t n)
     return n_rg * n_panels >= 256;
 }
 
-// Time of a product through the sweep kernel, from the tiles (row groups x panels of 64 columns, one workgroup of a compute unit
-// each), the chunks that the row groups list together and the ops of a wavefront per chunk.  Measured: a tile costs 2.5 us of
-// entry and stores, a chunk 0.25 us and 0.115 us per op (the plan fills up to four), a third more where every compute unit
-// has a tile and they share the L2.  Row groups of 16 / 32 / 64 block rows, estimate (measured), us:
-//   3088 x 4112, 15 %, N = 1000: 19.5 (23.9) / 18.8 (24.8) / 24.5 (34.9); 30 %: 21.3 (21.4) / 28.1 (27.1) / 39.8 (42.8)
-//   8192 x 8192, 10 %, N = 640:  67.8 (51.2) / 31.7 (29.5) / 41.5 (37.9); N = 1536: 101 (82) / 68 (56) / 46.7 (43.1)
-//   768 x 3072, 10 %, N = 4096:  14.8 (14.2) / 14.0 (15.0) / 15.3 (16.8)
-static double sweep_estimate_us(size_t n_rg, size_t listed_chunks, size_t nnzb, size_t N)
+// Time of a product with fp16 results through the sweep kernel, from the tiles (row groups x panels of 64 columns, one
+// workgroup of a compute unit each), the chunks that the row groups list together and the ops of a wavefront per chunk: a
+// tile costs 0.65 us, a chunk 0.32 us and 0.111 us per op (the plan fills up to four), C 0.66 us per 10^6 elements.  Fitted
+// to 153 matrices (random blocks 768^2 to 16384^2 at 3 to 36 %, bands; N = 64 to 4096) on row groups of 16, 32 and 64, three
+// products on their own inputs in turn: 8 % standard deviation, all but a few within 25 %.  Estimate (measured), us:
+//   3088 x 4112, 15 %, N = 1000:  18.1 (19.9) / 19.3 (19.9) / 25.0 (27.3)
+//   8192 x 8192, 10 %, N = 640:   55.2 (50.7) / 30.8 (28.9) / 42.3 (37.6); N = 1536: 84.5 (78.7) / 60.1 (56.3) / 47.1 (41.9)
+//   768 x 3072, 10 %, N = 4096:   14.6 (14.0) / 14.6 (15.0) / 16.7 (17.0)
+static double sweep_estimate_us(size_t n_rg, size_t listed_chunks, size_t nnzb, size_t M, size_t N)
 {
     if (n_rg == 0 || listed_chunks == 0) return 1e30;
     const size_t tiles = n_rg * ((N + 16 * SWEEP_TN - 1) / (16 * SWEEP_TN)), rounds = (tiles + 255) / 256;
     const double ops = 0.525 * (double)nnzb / ((double)listed_chunks * SWEEP_WAVES) + 0.3;
-    const double chunk = (0.25 + 0.115 * std::max(4.0, ops)) * (1.0 + 0.35 * (double)std::min<size_t>(tiles, 256) / 256.0);
-    return 1.5 + (double)rounds * (2.5 + (double)listed_chunks / (double)n_rg * chunk);
+    const double chunk = 0.32 + 0.111 * std::max(3.8, ops);
+    return 3.0 + (double)rounds * (0.65 + (double)listed_chunks / (double)n_rg * chunk) + 0.66e-6 * (double)M * (double)N;
 }
-// The same through the row-wise kernel: 20 TB/s of operands from repacked B, behind the repack, 7.6 TB/s from B in place.
-// (3088 x 4112, 15 %, N = 1000: 24.0, measured 26.2; 8192 x 8192, 10 %, N = 640: 40.1 (44.9), N = 128: 14.4 (13.0).)
-static double rowwise_estimate_us(size_t K, size_t N, size_t nnzb, bool packed)
+// The same through the row-wise kernel, fitted to the same products: 17.8 TB/s of operands from repacked B, behind the
+// repack, 4.9 TB/s from B in place.  18 % standard deviation; too high for bands, whose rows share B (16384, 64, N = 1024: 68,
+// measured 43), too low for few or long rows (1040 x 16384, 35 %, N = 1000: 63, measured 85).
+static double rowwise_estimate_us(size_t M, size_t K, size_t N, size_t nnzb, bool packed)
 {
-    const double gather = (double)nnzb * 16.0 * (double)N * 2.0;
-    return packed ? 8.0 + 4.0 * (double)K * (double)N / 4e6 + gather / 20e6 : 4.0 + gather / 7.6e6;
+    const double gather = (double)nnzb * 16.0 * (double)N * 2.0e-6, c = 0.14e-6 * (double)M * (double)N;
+    return c + (packed ? 8.0 + 0.8e-6 * (double)K * (double)N + gather / 17.8 : 4.0 + gather / 4.9);
 }
 static size_t sweep_listed_chunks(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t group_rows)
 {
@@ -234,7 +236,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
     }
     // a plan made for a wide N, used with a narrow one: too few workgroups for the sweep kernel
     if (kernel == SMAT_KERNEL_SWEEP && o.kernel == SMAT_KERNEL_AUTO &&
-        (plan->sweep_few_tiles ? sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, N) > rowwise_estimate_us(K, N, nnzb, a.b_packed != nullptr)
+        (plan->sweep_few_tiles ? sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N) > rowwise_estimate_us(M, K, N, nnzb, a.b_packed != nullptr)
                                : !sweep_fills_device(M / 16, N)))
         kernel = SMAT_KERNEL_ROWWISE;
     const uint16_t *B_as_given = B;
@@ -569,30 +571,52 @@ extern "C" int smat_plan_create(smat_plan **out, const int32_t *row_ptr_host,
 
 // A matrix of mostly full blocks that plan creation left with the row-wise kernel, because its tiles of 64 block rows x 64
 // columns are fewer than the compute units or because fewer than 5 % of its blocks exist: the sweep kernel all the same, on
-// row groups of 64, 32 or 16 block rows, where the estimates say that it is 15 % faster than the row-wise kernel (half as fast
-// again where every compute unit has a tile: there the estimate is up to 30 % low, 68 for 87 us on 8192^2, 3 %, N = 4096).
-// Measured, us, before and after: 8192^2, 10 %, N = 640: 44.9 -> 29.0, N = 1536: 71.2 -> 42.6; 3088 x 4112, 15 %, N = 2000:
-// 40.6 -> 22.7; 768 x 3072, 30 %, N = 4096: 31.9 -> 15.6; bands, whose row groups list few chunks: 16384 rows, bandwidth 64,
-// N = 1024 42.5 -> 19.3; 65536, 256, N = 512 146 -> 77; 4096, 30, N = 1024 14.4 -> 8.7.  Left alone by the estimate: 4096^2, 3 %,
-// N = 512 (9.6 against 16.2); 1040 x 16384, 35 %, N = 1000, wrongly (85 against 57).  A K of one or two chunks, less than
-// the entry fetches, stays with the row-wise kernel as it was.
-// The streams take 0.1 to 0.2 us a block to build on the host, so they are built once the values are known to be dense; the
-// search for a better deal of the rows to the wavefronts is cut short (ten times the work: 5.5 against 1.8 ms, same kernel times).
+// row groups of 64, 32 or 16 block rows, where
+//   * the estimate is below that of the row-wise kernel by more than the two are off, a quarter.  Of the 153 matrices above it
+//     takes 64, all of them faster than row-wise with fp16 results (by 5 to 62 %; what the rule leaves would gain another 3 %
+//     in the mean), four up to 10 % slower with fp32 ones, whose stores cost the sweep kernel more;
+//   * a thousand products make up for the building, 0.11 us a block (one core).  The products that it took to do so, as
+//     measured: 10 to 200 for most, 990 for 8192^2, 30 %, N = 256 (38.1 -> 29.4 us), at most 1,760 (a band of 16384 rows and 250,
+//     N = 128, 12.4 -> 10.3).
+// Measured, us, before and after: 8192^2, 10 %, N = 640: 45.6 -> 28.9, N = 1536: 72.1 -> 41.9; 3088 x 4112, 15 %, N = 2000:
+// 39.6 -> 22.4, N = 1000 24.2 -> 19.9; 768 x 3072, 30 %, N = 4096: 31.9 -> 15.4; bands, whose row groups list few chunks: 16384 rows,
+// bandwidth 64, N = 1024 43.1 -> 19.4; 65536, 256, N = 512 146 -> 78.  A K of one or two chunks, less than the entry fetches, stays
+// with the row-wise kernel.  Returns the block rows of a group, 0 = row-wise.
+static int g_force_group_rows = 0; // test hook: 64, 32 or 16 whatever the estimates say
+static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, bool packed)
+{
+    const size_t mb = M / 16, kb = K / 16;
+    if (nnzb < 2 || nnzb >= (size_t)1 << 23 || K >= (size_t)1 << 28 || kb <= 2 * SWEEP_S) return 0;
+    if (g_force_group_rows) return (size_t)g_force_group_rows;
+    const double row_wise = rowwise_estimate_us(M, K, N, nnzb, packed);
+    double best = std::min(row_wise / 1.25, row_wise - 0.11e-3 * (double)nnzb);
+    size_t group_rows = 0;
+    for (size_t rows : {(size_t)SWEEP_G, (size_t)SWEEP_G / 2, (size_t)SWEEP_G / 4}) {
+        const double t = sweep_estimate_us((mb + rows - 1) / rows, sweep_listed_chunks(row_ptr, col_idx, mb, kb, rows), nnzb, M, N);
+        if (t < best) best = t, group_rows = rows;
+    }
+    return group_rows;
+}
+// Test hooks (not part of smat.h): row groups of 64, 32 or 16 wherever the sweep kernel may be taken at all (0 = the
+// choice, the default), and the choice itself.
+extern "C" void smat_internal_sweep_force_groups(int rows) { g_force_group_rows = rows; }
+extern "C" int smat_internal_sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, int packed)
+{
+    return (int)sweep_group_rows(row_ptr, col_idx, M, K, nnzb, N, packed != 0);
+}
+
+// The streams are built once the values are known to be dense.  The search for a better deal of the rows to the wavefronts
+// takes a tenth of the time (16 counter updates a block: 3088 x 4112, 15 % 0.84 ms for all, without the search 0.75, with a
+// million updates, 0.5 % fewer ops in the busiest wavefronts, 1.8; same kernel times).
 static hipError_t sweep_small_groups(smat_plan &p)
 {
     const size_t mb = p.M / 16, kb = p.K / 16, nnzb = p.nnzb;
-    if (p.col_idx_host.size() != nnzb || nnzb < 2 || nnzb >= (size_t)1 << 23 || p.K >= (size_t)1 << 28 || kb <= 2 * SWEEP_S)
-        return hipSuccess;
+    if (p.col_idx_host.size() != nnzb) return hipSuccess;
     const int32_t *row_ptr = p.row_ptr_host.data(), *col_idx = p.col_idx_host.data();
-    double best = rowwise_estimate_us(p.K, p.n_cap, nnzb, p.d_bpack != nullptr) / (sweep_fills_device(mb, p.n_cap) ? 1.5 : 1.15);
-    size_t group_rows = 0;
-    for (size_t rows : {(size_t)SWEEP_G, (size_t)SWEEP_G / 2, (size_t)SWEEP_G / 4}) {
-        const double t = sweep_estimate_us((mb + rows - 1) / rows, sweep_listed_chunks(row_ptr, col_idx, mb, kb, rows), nnzb, p.n_cap);
-        if (t < best) best = t, group_rows = rows;
-    }
+    const size_t group_rows = sweep_group_rows(row_ptr, col_idx, p.M, p.K, nnzb, p.n_cap, p.d_bpack != nullptr);
     if (!group_rows) return hipSuccess;
     SweepPlanHost h;
-    build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 1e6);
+    build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 16.0 * (double)nnzb);
     const hipError_t e = p.sweep.upload(h);
     if (e != hipSuccess) {
         p.sweep.release();
@@ -700,7 +724,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     const double t_pass = 3.0 + (double)p->K * n_est / 1e6;
     // one kernel for everything: the sweep kernel (when the plan has its work list) or the compact kernel
     const double t_sweep_all = !p->sweep.d_ops ? 1e30
-                               : p->sweep_few_tiles ? sweep_estimate_us((size_t)p->sweep.n_rg, p->sweep_chunks, p->nnzb, p->n_cap)
+                               : p->sweep_few_tiles ? sweep_estimate_us((size_t)p->sweep.n_rg, p->sweep_chunks, p->nnzb, p->M, p->n_cap)
                                                     : t_sweep((double)p->nnzb);
     const double t_compact_all = t_compact((double)census.n_cols_all) + t_pass;
     if (may_mix && !mixed && !p->col_idx_host.empty() && p->nnzb < ((size_t)1 << 23) &&
