@@ -866,19 +866,19 @@ hipError_t compact_full_blocks(const CompactCensus &s, std::vector<uint8_t> &ful
 
 // Whether the nonzeros are listed one by one (4 bytes each, and 8 per step) instead of whole columns (32 bytes each): a step of
 // random sparse columns, one nonzero each, is then 152 bytes of A instead of 1024, of the 4 to 5 KiB that the vector L1
-// returns for it, but its operand takes two trips through LDS.  Over 250 drawn random matrices (rows 1,024 to 65,536, K 512 to
-// 32,768, 3 to 90 nonzeros a row, N 32 to 2,048, either layout of B) this rule is 0.6 % from the better of the two in the
-// mean, a rule by K alone (>= 4096) 2.5 %:
+// returns for it, but its operand takes two trips through LDS.  Over 260 drawn matrices (random, R-MAT, 27-point stencils; rows
+// 1,024 to 262,144, N 8 to 1,024, either layout of B, three products on their own inputs in turn) this rule is 0.8 % from the
+// better of the two in the mean, always listing nonzeros 3.3 %, a rule by K alone (>= 4096) 3.2 %:
 //   * the trips through LDS are what a wavefront waits for where there are fewer than five on a CU (whole columns / nonzeros, us:
 //     8192 x 4096, 40 a row, N = 128 10.4 / 11.6; R-MAT scale 12, N = 64 11.5 / 13.5);
 //   * with more, the nonzeros win while they are few per column (65536 x 512, 8 a row, N = 512 43.4 / 38.9; 59328 x 27344, 17.5 a
 //     row, N = 288 76 / 55; at 2.3 per column 4096 x 512, 64 a row, N = 1024 they lose, 15.2 / 17.0);
-//   * columns with more nonzeros pay while the list of whole columns stays in the eight L2s of 4 MiB (27-point stencil, 2.8 per
-//     column: 32^3, 300 k columns, N = 256 22.5 / 23.9; 48^3, 1.05 M, 70.8 / 62.8; 64^3, 2.5 M, N = 64 47.8 / 42.5).
+//   * whole columns with more nonzeros pay while their list takes no more than half of the eight L2s of 4 MiB (27-point stencil,
+//     2.8 per column: 32^3, 300 k columns, N = 256 22.5 / 23.9; 48^3, 1.05 M, 70.8 / 62.8; 64^3, 2.5 M, N = 64 47.8 / 42.5).
 static bool lists_nonzeros(int64_t nnz, int64_t n_cols, size_t n_rows, size_t N)
 {
     if (n_rows * ((N + 63) / 64) < 5 * 256) return false;
-    return 2 * nnz <= 3 * n_cols || (n_cols >= 1000000 && nnz <= 4 * n_cols);
+    return 2 * nnz <= 3 * n_cols || (n_cols >= 500000 && nnz <= 4 * n_cols);
 }
 
 hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx, size_t K, size_t n_cap,
