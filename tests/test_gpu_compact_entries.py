@@ -61,7 +61,10 @@ def test_lists_of_nonzeros_match_the_oracle(smat, cuda, oracle, lists, fill, N, 
             torch.cuda.synchronize()
         finally:
             smat.lib.smat_internal_compact_panel(0)
-        assert oracle.compare(C.half().cpu().numpy().view(np.uint16), want)[0] <= 1e-3
+        if c_f32:
+            oracle.assert_fp32_close(C.cpu().numpy(), want, N, K, A, B)
+        else:
+            assert oracle.compare(C.cpu().numpy().view(np.uint16), want)[0] <= 1e-3
 
 
 # block rows of up to 260 steps: around what one load of entry ranges covers (64 steps), and around two
@@ -103,3 +106,44 @@ def test_long_even_block_rows(smat, cuda, oracle, lists, fill, what, K, N, n_hin
         finally:
             smat.lib.smat_internal_compact_panel(0)
         oracle.assert_fp32_close(C.cpu().numpy(), want, N, K, A, B)
+
+
+# copies of B of 4 GiB and more, K above 2^24: row addresses in 64 bits
+@pytest.mark.parametrize("what", [1, 2])
+@pytest.mark.parametrize("K,N,row_major", [((1 << 24) + 160, 136, True), ((1 << 24) + 160, 8, False), (1 << 20, 2056, True)])
+@pytest.mark.parametrize("c_f32", [False, True])
+def test_wide_row_addresses_match_the_oracle(smat, cuda, oracle, lists, what, K, N, row_major, c_f32):
+    import torch
+    lists(what)
+    rng = np.random.default_rng(N)
+    mb, kb = 6, K // 16
+    # block columns all over K, the first and the last among them, and around 2^32 bytes of B
+    edge = min(kb - 2, (1 << 32) // (N * 2) // 16)
+    per_row = [np.unique(np.concatenate([rng.integers(0, kb, n), [0, edge - 1, edge, edge + 1, kb - 1]])) for n in (3, 20, 60, 0, 40, 9)]
+    rp = np.concatenate([[0], np.cumsum([len(c) for c in per_row])]).astype(np.int32)
+    ci = (np.concatenate(per_row) * 16).astype(np.int32)
+    v = np.zeros((len(ci), 16, 16), np.float16)
+    for p in range(len(ci)):
+        for c in rng.choice(16, 3, replace=False):
+            v[p, rng.choice(16, 2, replace=False), c] = rng.normal(size=2)
+    M, nnzb, val = mb * 16, len(ci), v.view(np.uint16).reshape(-1)
+    g = torch.Generator("cuda").manual_seed(3)
+    B = torch.randn(K * N, generator=g, device=cuda, dtype=torch.float16) if K * N < 1 << 31 else \
+        torch.cat([torch.randn(K // 2 * N, generator=g, device=cuda, dtype=torch.float16) for _ in range(2)])
+    used = np.unique(ci).astype(np.int64)
+    rows = (torch.as_tensor(used)[:, None] + torch.arange(16)).reshape(-1).to(cuda)
+    small = B.view(K, N)[rows].t() if row_major else B.view(N, K)[:, rows]  # the rows of B that are used, column-major
+    small = np.ascontiguousarray(small.cpu().numpy().view(np.uint16)).reshape(-1)
+    A = {"M": M, "b_row_ptr": rp, "b_col_idx": (np.searchsorted(used, ci) * 16).astype(np.int32), "b_val": val}
+    want = oracle.spmm_bcsr(M, N, len(used) * 16, rp, A["b_col_idx"], val, small, threads=4)
+    vals, rpd, cid = (to_dev(torch, x, cuda) for x in (val, rp, ci))
+    C = torch.full((M, N), float("nan"), dtype=torch.float32 if c_f32 else torch.float16, device=cuda)
+    plan = smat.Plan(rp, M, K, nnzb, N, col_idx_host=ci, kernel=5, b_row_major=row_major)
+    plan.attach_values(vals, rpd, cid)
+    smat.spmm(vals, rpd, cid, B, C, M, N, K, nnzb, plan=plan, kernel=5, c_f32=c_f32, b_row_major=row_major)
+    torch.cuda.synchronize()
+    plan.close()
+    if c_f32:
+        oracle.assert_fp32_close(C.cpu().numpy(), want, N, len(used) * 16, A, small)
+    else:
+        assert oracle.compare(C.cpu().numpy().view(np.uint16), want)[0] <= 1e-3
