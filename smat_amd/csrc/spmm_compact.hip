@@ -594,12 +594,10 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
     const int n_panels = (int)((a.N + PANEL - 1) / PANEL);
     long panel_stride = PANEL, row_stride = (long)a.N;
     if (!a.b_row_major) {
-        if (!a.bt_ready) {
-            dim3 grid((unsigned)((a.K + 63) / 64), (unsigned)((a.N + 63) / 64));
-            hipLaunchKernelGGL(transpose_b_kernel, grid, dim3(256), 0, st, a.B, a.Bt, (int)a.N, (long)a.K, PANEL, (long)PANEL);
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-        }
+        dim3 grid((unsigned)((a.K + 63) / 64), (unsigned)((a.N + 63) / 64));
+        hipLaunchKernelGGL(transpose_b_kernel, grid, dim3(256), 0, st, a.B, a.Bt, (int)a.N, (long)a.K, PANEL, (long)PANEL);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
         panel_stride = (long)a.K * PANEL;
         row_stride = PANEL;
     }
@@ -690,62 +688,56 @@ hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t
     p.tuned_n = 0;
     p.tuned_run = 0;
     if (!g_tune || p.n_items == 0 || N == 0 || !Bt) return hipSuccess;
-    // What the deal is about is the product kernel: with column-major B it is timed on a zeroed copy Bt, without the
-    // transposition.  (24 launches of 20 us each with it, and a synchronisation for every run length, were 0.5 of the
-    // 1.25 ms that blocking, planning and attaching a 16384^2 matrix with 0.1 % nonzeros and its first product took.)
-    Scratch B, C;
-    if ((b_row_major && B.alloc(K * N * sizeof(uint16_t)) != hipSuccess) || C.alloc(M * N * sizeof(uint16_t)) != hipSuccess) {
-        (void)hipGetLastError(); // no room for the trial: not an error of the plan
-        return hipSuccess;
-    }
-    hipError_t e = b_row_major ? hipMemset(B.p, 0, K * N * sizeof(uint16_t)) : hipMemset(Bt, 0, K * ((N + 255) / 256 * 256) * sizeof(uint16_t));
-    if (e == hipSuccess) e = hipMemset(C.p, 0, M * N * sizeof(uint16_t));
-    constexpr int MAX_RUNS = 4;
-    hipEvent_t mark[MAX_RUNS + 1] = {};
-    for (int i = 0; i <= MAX_RUNS && e == hipSuccess; i++) e = hipEventCreate(&mark[i]);
-    CompactArgs a{};
-    a.B = static_cast<const uint16_t *>(B.p); a.b_row_major = b_row_major; a.Bt = Bt; a.bt_ready = true; a.C = C.p;
-    a.M = M; a.N = N; a.K = K; a.c_f32 = false; a.plan = &p; a.accumulate = accumulate;
-    // the run lengths one after the other without a gap between them, `launches` times each after one more of the first
-    auto time_all = [&](const unsigned *runs, int n, int launches, float *ms) {
-        a.xcd_run = runs[0];
-        hipError_t r = launch_compact(a, nullptr);
-        if (r == hipSuccess) r = hipEventRecord(mark[0], nullptr);
-        for (int k = 0; k < n; k++) {
-            a.xcd_run = runs[k];
-            for (int i = 0; i < launches && r == hipSuccess; i++) r = launch_compact(a, nullptr);
-            if (r == hipSuccess) r = hipEventRecord(mark[k + 1], nullptr);
-        }
-        if (r == hipSuccess) r = hipEventSynchronize(mark[n]);
-        for (int k = 0; k < n && r == hipSuccess; k++) {
-            r = hipEventElapsedTime(&ms[k], mark[k], mark[k + 1]);
-            ms[k] /= (float)launches;
-        }
-        return r;
-    };
-    // the run length of an untuned launch, as launch_compact_tq computes it for this N
+    // Timed as a program launches it, the transposition of a column-major B included: the copy is written over what the
+    // launch before left in the L2s, and how many of them hold a line of it follows from the deal (16384^2, 0.1 %, N = 256: the
+    // product kernel alone is fastest in runs of 128, 10.9 against 11.9 us; launch after launch it is 64, 19.8 against 21.4.
+    // 8192 x 16384, 24 a row, N = 512: 24.2 against 27.1 in runs of 32 and 128).
     const int tq = compact_panel_width(p, N, K);
     const int n_panels = (int)((N + 64 * tq - 1) / (64 * tq));
     const long wgs = ((long)p.n_tasks * n_panels + 3) / 4;
     const unsigned eighth = (unsigned)std::max<long>((wgs + 7) / 8, 1);
+    // the run length of an untuned launch, as launch_compact_tq computes it for this N
     const unsigned base = std::min(eighth, p.deal.run((size_t)p.n_tasks, n_panels));
-    float t_base = 0.f;
-    if (e == hipSuccess) e = time_all(&base, 1, 1, &t_base);
-    if (e == hipSuccess && t_base <= 20.f) {
-        unsigned runs[MAX_RUNS] = {base};
-        int n = 1;
-        if (base * 4 >= eighth) // a list that the estimate finds even: the longer runs are worth a try
-            for (unsigned r : {eighth, eighth / 2, eighth / 4})
-                if (r >= 4 && std::find(runs, runs + n, r) == runs + n) runs[n++] = r;
-        unsigned best_run = base;
-        if (n > 1) {
-            float ms[MAX_RUNS] = {};
-            e = time_all(runs, n, t_base < 0.2f ? 5 : 3, ms);
-            float best = ms[0] * 0.97f; // another run length has to be 3 % faster than the estimate's choice
-            for (int k = 1; k < n && e == hipSuccess; k++)
-                if (ms[k] < best) best = ms[k], best_run = runs[k];
-        }
-        if (e == hipSuccess) p.tuned_n = N, p.tuned_run = best_run;
+    constexpr int MAX_RUNS = 4;
+    unsigned runs[MAX_RUNS] = {base};
+    int n = 1;
+    if (base * 4 >= eighth) // a list that the estimate finds even: the longer runs are worth a try
+        for (unsigned r : {eighth, eighth / 2, eighth / 4})
+            if (r >= 4 && std::find(runs, runs + n, r) == runs + n) runs[n++] = r;
+    // R-MAT scale 20 has 10^6 steps and takes 0.5 ms: a launch of over 20 ms is not worth trying several times
+    if (n == 1 || p.n_steps * n_panels > 40000000) return hipSuccess;
+    Scratch B, C;
+    if (B.alloc(K * N * sizeof(uint16_t)) != hipSuccess || C.alloc(M * N * sizeof(uint16_t)) != hipSuccess) {
+        (void)hipGetLastError(); // no room for the trial: not an error of the plan
+        return hipSuccess;
+    }
+    hipError_t e = hipMemset(B.p, 0, K * N * sizeof(uint16_t));
+    if (e == hipSuccess) e = hipMemset(C.p, 0, M * N * sizeof(uint16_t));
+    hipEvent_t mark[MAX_RUNS + 1] = {};
+    for (int i = 0; i <= MAX_RUNS && e == hipSuccess; i++) e = hipEventCreate(&mark[i]);
+    CompactArgs a{};
+    a.B = static_cast<const uint16_t *>(B.p); a.b_row_major = b_row_major; a.Bt = Bt; a.C = C.p;
+    a.M = M; a.N = N; a.K = K; a.c_f32 = false; a.plan = &p; a.accumulate = accumulate;
+    // one after the other without a gap between them, three launches each, the first after one more (the choice is the same twelve times out of
+    // twelve on these matrices)
+    constexpr int LAUNCHES = 3;
+    a.xcd_run = runs[0];
+    if (e == hipSuccess) e = launch_compact(a, nullptr);
+    if (e == hipSuccess) e = hipEventRecord(mark[0], nullptr);
+    for (int k = 0; k < n; k++) {
+        a.xcd_run = runs[k];
+        for (int i = 0; i < LAUNCHES && e == hipSuccess; i++) e = launch_compact(a, nullptr);
+        if (e == hipSuccess) e = hipEventRecord(mark[k + 1], nullptr);
+    }
+    if (e == hipSuccess) e = hipEventSynchronize(mark[n]);
+    float ms[MAX_RUNS] = {};
+    for (int k = 0; k < n && e == hipSuccess; k++) e = hipEventElapsedTime(&ms[k], mark[k], mark[k + 1]);
+    if (e == hipSuccess) {
+        p.tuned_n = N;
+        p.tuned_run = base;
+        float best = ms[0] * 0.97f; // another run length has to be 3 % faster than the estimate's choice
+        for (int k = 1; k < n; k++)
+            if (ms[k] < best) best = ms[k], p.tuned_run = runs[k];
     }
     for (hipEvent_t m : mark)
         if (m) (void)hipEventDestroy(m);
@@ -1049,6 +1041,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     p->deal.set_costs(std::move(cost_prefix));
     p->n_items = (int)items.size();
     p->n_tasks = (int)tasks.size();
+    p->n_steps = total / 32;
     SMAT_STEP(dev_malloc(&p->d_tasks, std::max<size_t>(tasks.size(), 1) * sizeof(int4)));
     if (!tasks.empty()) SMAT_STEP(hipMemcpy(p->d_tasks, tasks.data(), tasks.size() * sizeof(int4), hipMemcpyHostToDevice));
     p->n_split_rows = (int)split.size();

@@ -102,6 +102,7 @@ struct CompactPlan {
     SplitRow *d_split = nullptr;
     float *d_workspace = nullptr; // n_slots * 16 * n_cap floats
     int n_items = 0, n_tasks = 0, n_split_rows = 0, n_slots = 0;
+    int64_t n_steps = 0;          // of 32 columns, of all block rows listed
     int64_t n_cols = 0;           // nonzero block columns listed (without padding)
     int64_t n_cols_all = 0;       // nonzero block columns of the whole matrix
     uint64_t values_checksum = 0; // of the block values the lists were made from
@@ -142,7 +143,6 @@ struct CompactArgs {
     const uint16_t *B; // column-major, or row-major with b_row_major
     bool b_row_major;  // B is already B[k*N + n]: no copy is made
     uint16_t *Bt;      // scratch, K * (N rounded up to 256) halves: the copy of B in panels of rows made at the start of the launch
-    bool bt_ready = false; // the copy is there already
     void *C;
     size_t M, N, K;
     bool c_f32;
@@ -152,10 +152,10 @@ struct CompactArgs {
 };
 hipError_t launch_compact(const CompactArgs &a, hipStream_t st);
 // Times launches of M x N x K with a few run lengths of the deal to the XCDs (the estimate's choice, an eighth of the
-// launch, a half and a quarter of that) on zeros (a column-major B: without the launch that makes Bt, which is overwritten) and keeps the fastest for launches of N columns
-// (tuned_n, tuned_run).  The deal decides where an item runs, not what it computes: the results do not depend on
-// it.  Synchronous, default stream; a plan too large for the temporary buffers, or whose single launch takes
-// longer than 20 ms, keeps the estimate's choice.
+// launch, a half and a quarter of that) on zeros and keeps the fastest for launches of N columns (tuned_n, tuned_run);
+// Bt is overwritten.  The deal decides where an item runs, not what it computes: the results do not depend on it.
+// Synchronous, default stream; a plan too large for the temporary buffers, or whose single launch would take longer than
+// 20 ms, keeps the estimate's choice.
 hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t K, bool b_row_major, bool accumulate);
 hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, size_t N, size_t K, hipStream_t st);
 
