@@ -323,13 +323,15 @@ __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__rest
 // A wavefront takes a task x a panel of 64 TQ columns.  A task is a run of items of the list, worked off as one stream of
 // steps, so that the loads of the next step are under way across the end of an item.
 //
-// What bounds a step of 32 columns x 64 columns of C on a CU is the return path of the vector L1 (4 KiB of rows of B and
-// 0.3 to 1 KiB of A at 64 bytes a clock) and, close behind, the LDS and the VALU.  Hence:
+// What a step of 32 columns x 64 columns of C waits for is the vector memory path: 4 KiB of rows of B and 0.15 to 1 KiB of A.
+// Counted on R-MAT scale 20 (stencil 64^3): its data unit is busy 92 (65) % of the time, the vector L1 waits for the L2 62
+// (23) %, LDS is active 30 (37) %, and a step has 21 (30) VALU instructions, 16 (19) of LDS and 6 (7) loads.  Operands merged in
+// the VALU took 130 VALU instructions a step, of which 56 exchanged and merged halves between lanes.  Hence:
 //   * Rows of B go from the registers they were gathered into through 4 KiB of LDS, [entry][64 columns], and come back as
-//     MFMA operands through transposing reads (ds_read_b64_tr_b16): no VALU work, where exchanging and merging halves
-//     between lanes took 56 VALU instructions of 130 a step.  Lane (octet o = lane / 8, c = lane & 7) gathers columns
-//     8c .. 8c + 7 of the entries k = 8 (o / 2) + 2j + (o & 1), j = 0 .. 3; the 16-byte pieces of the rows k with k & 2 are
-//     swapped in pairs, so that neither side has bank conflicts.  In lane (i = lane % 16, g = lane / 16) n-tile t of the
+//     MFMA operands through transposing reads (ds_read_b64_tr_b16): no VALU work.  Lane (octet o = lane / 8, c = lane & 7)
+//     gathers columns 8c .. 8c + 7 of the entries k = 8 (o / 2) + 2j + (o & 1), j = 0 .. 3; the 16-byte pieces of the rows k
+//     with k & 2 are swapped in pairs, which leaves 16 of the 71 clocks that a step keeps LDS active to bank conflicts (AF = 0,
+//     counted).  In lane (i = lane % 16, g = lane / 16) n-tile t of the
 //     operand reads columns 16 (i & 3) + 4t .. + 3 of the rows 8g + i / 4 and + 4; the lane ends up with the 16
 //     consecutive columns 16g .. of row i of the tile of C.
 //   * The address of a gathered row is one multiply-add of 32 bits from its index (BIG: 64 bits, for copies of B of 4 GiB
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__rest
 //   * Every load of a step is unconditional and nothing in the loop uses scalar loads, so that what is in flight can be
 //     counted; the gathers asked for past the end of the task read row 0.
 // Whole products with all of it (before: operands merged in the VALU, A in whole columns, an item per wavefront): R-MAT
-// scale 20, N = 128, 703 -> 595 us; Erdos-Renyi 16384^2, 0.1 %, N = 256, 17.3 -> 16.3 us.  A third copy of the step's code
+// scale 20, N = 128, 703 -> 590 us; Erdos-Renyi 16384^2, 0.1 %, N = 256, 17.3 -> 16.0 us.  A third copy of the step's code
 // costs more than it saves: kernels of 10 us wait for their instructions.
 //
 // C_ACC: the result is added to what C holds (the per-block split of a mixed plan: a dense kernel has written the
