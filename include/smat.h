@@ -96,7 +96,8 @@ int smat_plan_cache_clear(void);
                                * and 2^23 - 1 blocks and K below 2^28.  SMAT_KERNEL_AUTO takes it when at least
                                * 5% of the blocks exist and (M/1024) x (N/64) workgroups fill the 256 CUs, or
                                * once the attached values are mostly full blocks and an estimate finds it
-                               * faster (on groups of 64, 32 or 16 block rows).
+                               * a quarter faster (on groups of 64, 32 or 16 block rows; 0.11 us of host time
+                               * a block for its streams, which a thousand products have to make up for).
                                * It works from the plan's op list, NOT from the row_ptr / col_idx passed at
                                * launch: the plan must have been made from the same block pattern
                                * (smat_plan_check verifies that on request)                                 */
@@ -150,13 +151,13 @@ int smat_plan_create(smat_plan **plan, const int32_t *row_ptr_host, const int32_
                      size_t M, size_t K, size_t nnzb, size_t n_hint, const smat_spmm_opts *opts);
 /* Optional: lets the plan look at the block values (DEVICE arrays of the matrix the plan was
  * made for; row_ptr_host must equal the array given to smat_plan_create, else SMAT_ERR_INVALID).  The plan lists the nonzero columns of every
- * block and keeps a COPY of them (32 bytes per nonzero column, in MFMA operand order), so that
+ * block and keeps a COPY of them (32 bytes per nonzero column, in MFMA operand order, or 4 bytes per nonzero), so that
  * SMAT_KERNEL_COMPACT multiplies only those and touches only the rows of B under them; with
  * SMAT_KERNEL_AUTO the plan switches to that kernel when fewer than 60% of the block columns
  * are nonzero.  The compact kernel works from the copy: attach again after the values change.
  * The new list is built before the old one is dropped; if the call fails the plan has no list and
  * SMAT_KERNEL_AUTO goes back to the sweep or row-wise kernel.  When the plan takes the compact kernel, the call also
- * times a few launches of it on zeros (temporary device buffers of K x n_hint and M x n_hint halves, freed before it
+ * times ten or so launches of it on zeros (temporary device buffers of K x n_hint and M x n_hint halves, freed before it
  * returns; skipped if they do not fit) to choose how the work is dealt to the GPU's eight XCDs: a choice that moves
  * no bit of any result.  Synchronous.  No counterpart in the reference, which multiplies every block as a dense
  * 16x16 (mmaCBT.cu:44-66). */

@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
 // Launches of few (item, panel) pairs with long items: the four wavefronts of a workgroup share one, each takes a run of
 // the item's block pairs with the operands of NP pairs in flight, and the partial tiles are added in LDS in the order of
 // the runs.  Bound by the chain item -> column indices -> operands of a wavefront and by too few of them: 8192^2 with 10 %
-// of the blocks and N = 16 (512 items) takes 6.3 us where one wavefront per item takes 9.1; 1024 x 8192 with 30 % and
+// of the blocks and N = 16 (512 items) takes 6.6 us where one wavefront per item takes 9.1; 1024 x 8192 with 30 % and
 // N = 64 (64 items of 154 blocks) 13.8 against 39.8.  Eight wavefronts per item are no faster than four.
 template <int TN, bool C_F32, bool PACKED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void spmm_rowwise_split_kernel(
