@@ -527,7 +527,7 @@ static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
             (gain_us > 1.5 * cost_us || want == SMAT_KERNEL_ROWWISE_PACKED))
             e = dev_malloc(&p->d_bpack, K * n_hint * sizeof(uint16_t));
     }
-    p->panel_tiles = rowwise_panel_tiles(n_hint, K, items.size(), items.empty() ? 0 : nnzb / items.size(),
+    p->panel_tiles = rowwise_panel_tiles(n_hint, items.size(), items.empty() ? 0 : nnzb / items.size(),
                                          split.empty() ? RowLengths::EVEN : RowLengths::SPLIT, p->d_bpack != nullptr);
     // The sweep kernel pays one pass over the B panel per group of 32 block rows,
     // whatever the sparsity, and shares each staged slab between the blocks of the group

@@ -162,7 +162,7 @@ hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, siz
 // What a launch of the row-wise kernel knows about the lengths of its items: no block row is much longer than the average
 // (a plan found none to split), some were (and are split), or nothing (no plan).
 enum class RowLengths { EVEN, SPLIT, UNKNOWN };
-int rowwise_panel_tiles(size_t N, size_t K, size_t n_items, size_t avg_blocks, RowLengths lengths, bool packed);
+int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, RowLengths lengths, bool packed);
 hipError_t launch_sweep(const SweepArgs &a, hipStream_t st);
 hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st);
 

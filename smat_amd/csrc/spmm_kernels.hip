@@ -508,9 +508,11 @@ static hipError_t launch_rowwise_tn(const SpmmArgs &a, hipStream_t st)
     if (a.b_packed) {
         if (a.c_f32) SMAT_LAUNCH_ROWWISE(true, true);
         else SMAT_LAUNCH_ROWWISE(false, true);
-    } else {
+    } else if constexpr (TN < 16) { // the rule takes 256 columns on repacked B only
         if (a.c_f32) SMAT_LAUNCH_ROWWISE(true, false);
         else SMAT_LAUNCH_ROWWISE(false, false);
+    } else {
+        return hipErrorInvalidValue;
     }
 #undef SMAT_LAUNCH_ROWWISE
     return hipGetLastError();
@@ -562,28 +564,41 @@ unsigned XcdDeal::run(size_t n_items, int n_panels) const
     return r;
 }
 
-// Panel width of the row-wise kernel in tiles of 16 columns: as wide as leaves the chip enough wavefronts, since every
-// panel reads the blocks again.  Enough are 768 to 1000 with long items; items of fewer than 32 blocks are over so soon
-// that a panel wider than 64 columns wants 4000 (measured: 512 items of 115 blocks, N = 256 / 512: 128 / 256 columns win, 45
-// against 51 and 73 against 80 us; 1250 items of 14 blocks, N = 256: 64 columns, 19.7 against 21.6 us; 48 items of 51
-// blocks, N = 1024: 64 columns, 9.9 against 31 us for 256).  Below that go
-//   SPLIT    lists with split rows, uneven in more than their items' lengths: 64 columns (R-MAT scale 16, N = 512: 618
-//            against 944 us; scale 20, N = 128: 13.8 against 18.2 ms);
-//   UNKNOWN  whole block rows without a plan: the heaviest row may be many times the average and is one wavefront per
-//            panel, so no wider than 64 columns below N = 512 and 128 below 1024 (R-MAT scale 16, 16 a row: N = 128 1,406
-//            against 2,609 us with 128, N = 256 1,584 against 3,307 with 256; scale 14, N = 512 806 against 975 with 256);
-//   in place no wider than 4 MiB of B, an L2, unless N alone allows it (16384^2, 15 %, N = 384: 270, 257, 344 us with 64, 128,
-//            256 columns; 16384^2, 5 %, N = 256: 66.5, 64.9, 68.2; 8192^2, 10 %, N = 256, where 256 columns fit: 37.2, -, 36.3).
-int rowwise_panel_tiles(size_t N, size_t K, size_t n_items, size_t avg_blocks, RowLengths lengths, bool packed)
+// Panel width of the row-wise kernel in tiles of 16 columns, from 513 timed products (random blocks 768^2 to 16384^2 at 3 to
+// 36 %, bands; N = 96 to 4096, every width):
+//   repacked B  the launch runs in rounds of 1024 wavefronts, one per SIMD, and a column of a round costs 0.85 in a panel of
+//               128 and 0.8 in one of 256 of what it costs in one of 64, which reads the blocks more often: the width with the
+//               lowest product.  Of 285 launches 0.3 % slower than the best width in the mean, at most 8 %.  64, 128, 256
+//               columns, us: 640 items of 59 blocks, N = 384 39.4, 35.9, 54.6, N = 512 51.3, 48.2, 56.9; 512 of 113, N = 512
+//               60.2, 51.3, 47.9; 284 of 122, N = 888 69.9, 60.5, 96.1; 651 of 155, N = 136 42.6, 62.2, -;
+//   in place    64 columns, 128 where that still leaves 8000 wavefronts, or 2000 with items of 32 blocks and more.  Of 228
+//               launches 1 % slower than the best width in the mean, at most 12 %; 256 columns win by 4 % at most.
+//               120 items of 66 blocks, N = 2344 102.5, 121.1, 174.2; 2913 of 5, N = 2224 195.8, 168.0, 189.1; 1024 of 51, N = 384
+//               100.8, 96.2, 133.6;
+//   UNKNOWN     whole block rows without a plan, in place: the heaviest row may be many times the average and is one
+//               wavefront per panel, so 64 columns below N = 512 (R-MAT scale 16, 16 a row: N = 256 1,595, 2,686, 3,315;
+//               scale 14, N = 1024 730, 839, 986);
+//   SPLIT       lists with split rows, uneven in more than their items' lengths: 64 columns (R-MAT scale 16, N = 512: 618
+//               against 944 us; scale 20, N = 128: 13.8 against 18.2 ms).
+int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, RowLengths lengths, bool packed)
 {
     if (N < 32) return 1;
     if (N < 64) return 2;
-    if (lengths == RowLengths::SPLIT) return 4;
-    const size_t few = 768, many = avg_blocks < 32 ? 4000 : 1000;
-    auto fits = [&](size_t tiles) { return lengths != RowLengths::UNKNOWN && (packed || K * 32 * tiles <= (size_t)4 << 20); };
-    if (N >= 256 && (N >= 1024 || fits(16)) && n_items * ((N + 255) / 256) >= (N >= 1024 ? few : many)) return 16;
-    if (N >= 128 && (N >= 512 || fits(8)) && n_items * ((N + 127) / 128) >= (N >= 512 ? few : many)) return 8;
-    return 4;
+    if (lengths == RowLengths::SPLIT || N < 128) return 4;
+    if (!packed) {
+        const size_t wavefronts = n_items * ((N + 127) / 128);
+        return N >= (lengths == RowLengths::UNKNOWN ? 512 : 128) && wavefronts >= (avg_blocks < 32 ? 8000 : 2000) ? 8 : 4;
+    }
+    static const struct { int tiles; double column; } widths[] = {{4, 1.0}, {8, 0.85}, {16, 0.8}};
+    int best_tiles = 4;
+    double best = 1e30;
+    for (const auto &w : widths) {
+        if (N < (size_t)w.tiles * 16) break;
+        const size_t panels = (N + 16 * w.tiles - 1) / (16 * w.tiles);
+        const double cost = w.tiles * w.column * (double)((n_items * panels + 1023) / 1024);
+        if (cost < best) best = cost, best_tiles = w.tiles;
+    }
+    return best_tiles;
 }
 
 // Four wavefronts per (item, panel of 64 columns): up to 512 of those, of 12 blocks and more.  (256 items of 26 blocks,
@@ -657,7 +672,7 @@ hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st)
         else e = launch_rowwise_split<4>(a, st);
     } else {
         const RowLengths lengths = a.n_split_rows > 0 ? RowLengths::SPLIT : a.items ? RowLengths::EVEN : RowLengths::UNKNOWN;
-        switch (rowwise_panel_tiles(a.N, a.K, n_items, avg, lengths, a.b_packed != nullptr)) {
+        switch (rowwise_panel_tiles(a.N, n_items, avg, lengths, a.b_packed != nullptr)) {
         case 16: e = launch_rowwise_tn<16>(a, st); break;
         case 8: e = launch_rowwise_tn<8>(a, st); break;
         case 4: e = launch_rowwise_tn<4>(a, st); break;
@@ -689,7 +704,7 @@ hipError_t launch_reduce(const float *workspace, const SplitRow *split_rows, int
 } // namespace smat
 
 // Test hook (not part of smat.h): the panel width of the row-wise kernel in tiles of 16 columns; lengths as in RowLengths.
-extern "C" int smat_internal_rowwise_panel(size_t N, size_t K, size_t n_items, size_t avg_blocks, int lengths, int packed)
+extern "C" int smat_internal_rowwise_panel(size_t N, size_t n_items, size_t avg_blocks, int lengths, int packed)
 {
-    return smat::rowwise_panel_tiles(N, K, n_items, avg_blocks, static_cast<smat::RowLengths>(lengths), packed != 0);
+    return smat::rowwise_panel_tiles(N, n_items, avg_blocks, static_cast<smat::RowLengths>(lengths), packed != 0);
 }
