@@ -564,11 +564,11 @@ unsigned XcdDeal::run(size_t n_items, int n_panels) const
     return r;
 }
 
-// Panel width of the row-wise kernel in tiles of 16 columns, from 513 timed products (random blocks 768^2 to 16384^2 at 3 to
+// Panel width of the row-wise kernel in tiles of 16 columns, from 842 timed products (random blocks 768^2 to 16384^2 at 3 to
 // 36 %, bands; N = 96 to 4096, every width):
-//   repacked B  the launch runs in rounds of 1024 wavefronts, one per SIMD, and a column of a round costs 0.85 in a panel of
+//   repacked B  the launch runs in rounds of 1024 wavefronts, one per SIMD, and a column of a round costs 0.83 in a panel of
 //               128 and 0.8 in one of 256 of what it costs in one of 64, which reads the blocks more often: the width with the
-//               lowest product.  Of 285 launches 0.3 % slower than the best width in the mean, at most 8 %.  64, 128, 256
+//               lowest product.  Of 614 launches 0.5 % slower than the best width in the mean, at most 14 %.  64, 128, 256
 //               columns, us: 640 items of 59 blocks, N = 384 39.4, 35.9, 54.6, N = 512 51.3, 48.2, 56.9; 512 of 113, N = 512
 //               60.2, 51.3, 47.9; 284 of 122, N = 888 69.9, 60.5, 96.1; 651 of 155, N = 136 42.6, 62.2, -;
 //   in place    64 columns, 128 where that still leaves 8000 wavefronts, or 2000 with items of 32 blocks and more.  Of 228
@@ -589,7 +589,7 @@ int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, RowLengths 
         const size_t wavefronts = n_items * ((N + 127) / 128);
         return N >= (lengths == RowLengths::UNKNOWN ? 512 : 128) && wavefronts >= (avg_blocks < 32 ? 8000 : 2000) ? 8 : 4;
     }
-    static const struct { int tiles; double column; } widths[] = {{4, 1.0}, {8, 0.85}, {16, 0.8}};
+    static const struct { int tiles; double column; } widths[] = {{4, 1.0}, {8, 0.83}, {16, 0.8}};
     int best_tiles = 4;
     double best = 1e30;
     for (const auto &w : widths) {
