@@ -165,13 +165,22 @@ static double sweep_estimate_us(size_t n_rg, size_t listed_chunks, size_t nnzb, 
     const double chunk = 0.32 + 0.111 * std::max(3.8, ops);
     return 3.0 + (double)rounds * (0.65 + (double)listed_chunks / (double)n_rg * chunk) + 0.66e-6 * (double)M * (double)N;
 }
-// The same through the row-wise kernel, fitted to the same products: 17.8 TB/s of operands from repacked B, behind the
-// repack, 4.9 TB/s from B in place.  18 % standard deviation; too high for bands, whose rows share B (16384, 64, N = 1024: 68,
-// measured 43), too low for few or long rows (1040 x 16384, 35 %, N = 1000: 63, measured 85).
-static double rowwise_estimate_us(size_t M, size_t K, size_t N, size_t nnzb, bool packed)
+// The same through the row-wise kernel, fitted to those of 239 products that it can lose: the rounds of 1024 wavefronts that
+// rowwise_panel_tiles counts and the blocks of an item, or the blocks of all where four wavefronts share an item, behind the
+// repack of B.  Standard deviation 7 % on repacked B, 12 % in place, 20 % with shared items.  Estimate (measured), us: 8192^2, 10 %,
+// N = 640 40.1 (41.7); 5008 x 3008, 20 %, N = 800 25.9 (25.2); 1040 x 16384, 35 %, N = 1000 83.4 (78.4); 768 x 3072, 10 %,
+// N = 4096, in place 21.7 (20.7); too high for narrow bands, whose rows share B (16384, 64, N = 1024: 55, measured 44.6).
+static double rowwise_estimate_us(size_t M, size_t K, size_t N, size_t nnzb, size_t n_items, RowLengths lengths, bool packed)
 {
-    const double gather = (double)nnzb * 16.0 * (double)N * 2.0e-6, c = 0.14e-6 * (double)M * (double)N;
-    return c + (packed ? 8.0 + 0.8e-6 * (double)K * (double)N + gather / 17.8 : 4.0 + gather / 4.9);
+    n_items = std::max<size_t>(n_items, 1);
+    const size_t avg = nnzb / n_items;
+    const double start = 0.6e-6 * (double)M * (double)N + (packed ? 5.6 + 0.6e-6 * (double)K * (double)N : 2.7);
+    if (rowwise_shares_items(N, n_items, avg))
+        return start + (double)nnzb * (double)((N + 63) / 64) / 256.0 * (packed ? 0.047 : 0.14);
+    const size_t tiles = (size_t)rowwise_panel_tiles(N, n_items, avg, lengths, packed);
+    const size_t rounds = (n_items * ((N + 16 * tiles - 1) / (16 * tiles)) + 1023) / 1024;
+    const double column = !packed || tiles <= 4 ? 1.0 : tiles == 8 ? 0.83 : 0.8;
+    return start + (double)rounds * (double)tiles * (double)nnzb / (double)n_items * (packed ? 0.0274 * column : 0.074);
 }
 static size_t sweep_listed_chunks(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t group_rows)
 {
@@ -236,7 +245,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
     }
     // a plan made for a wide N, used with a narrow one: too few workgroups for the sweep kernel
     if (kernel == SMAT_KERNEL_SWEEP && o.kernel == SMAT_KERNEL_AUTO &&
-        (plan->sweep_few_tiles ? sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N) > rowwise_estimate_us(M, K, N, nnzb, a.b_packed != nullptr)
+        (plan->sweep_few_tiles ? sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N) > rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, plan->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, a.b_packed != nullptr)
                                : !sweep_fills_device(M / 16, N)))
         kernel = SMAT_KERNEL_ROWWISE;
     const uint16_t *B_as_given = B;
@@ -572,24 +581,26 @@ extern "C" int smat_plan_create(smat_plan **out, const int32_t *row_ptr_host,
 // A matrix of mostly full blocks that plan creation left with the row-wise kernel, because its tiles of 64 block rows x 64
 // columns are fewer than the compute units or because fewer than 5 % of its blocks exist: the sweep kernel all the same, on
 // row groups of 64, 32 or 16 block rows, where
-//   * the estimate is below that of the row-wise kernel by more than the two are off, a quarter.  Of the 153 matrices above it
-//     takes 64, all of them faster than row-wise with fp16 results (by 5 to 62 %; what the rule leaves would gain another 3 %
-//     in the mean), four up to 10 % slower with fp32 ones, whose stores cost the sweep kernel more;
+//   * the estimate is below that of the row-wise kernel by more than the two are off, 10 % on repacked B and 20 % in place.  Of
+//     239 products that creation leaves to the choice (random blocks 768^2 to 16384^2 at 3 to 36 %, bands; N = 64 to 4096) it
+//     takes 96, all but a band of 8192 rows (8.7 -> 9.1 us) faster than row-wise with fp16 results (by up to 60 %; what the rule
+//     leaves would gain another 1.7 % in the mean), seven up to 10 % slower with fp32 ones, whose stores cost the sweep kernel more;
 //   * a thousand products make up for the building, 0.11 us a block (one core).  The products that it took to do so, as
-//     measured: 10 to 200 for most, 990 for 8192^2, 30 %, N = 256 (38.1 -> 29.4 us), at most 1,760 (a band of 16384 rows and 250,
-//     N = 128, 12.4 -> 10.3).
-// Measured, us, before and after: 8192^2, 10 %, N = 640: 45.6 -> 28.9, N = 1536: 72.1 -> 41.9; 3088 x 4112, 15 %, N = 2000:
-// 39.6 -> 22.4, N = 1000 24.2 -> 19.9; 768 x 3072, 30 %, N = 4096: 31.9 -> 15.4; bands, whose row groups list few chunks: 16384 rows,
-// bandwidth 64, N = 1024 43.1 -> 19.4; 65536, 256, N = 512 146 -> 78.  A K of one or two chunks, less than the entry fetches, stays
+//     measured: 109 in the middle, 958 for 2336 x 2192, 20 %, N = 896 (12.9 -> 12.4 us), 1,740 for a band of 16384 rows and 250,
+//     N = 128 (12.4 -> 10.3), and that band of 8192 rows never does.
+// Measured, us, before and after: 8192^2, 10 %, N = 640: 41.7 -> 28.9, N = 1536: 71.4 -> 41.9; 3088 x 4112, 15 %, N = 2000:
+// 40.0 -> 22.1, N = 1000 24.5 -> 19.9; 768 x 3072, 30 %, N = 4096: 29.6 -> 15.4; bands, whose row groups list few chunks: 16384 rows,
+// bandwidth 64, N = 1024 44.6 -> 19.4; 65536, 256, N = 512 146 -> 78.  A K of one or two chunks, less than the entry fetches, stays
 // with the row-wise kernel.  Returns the block rows of a group, 0 = row-wise.
 static int g_force_group_rows = 0; // test hook: 64, 32 or 16 whatever the estimates say
-static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, bool packed)
+static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, size_t n_items,
+                               RowLengths lengths, bool packed)
 {
     const size_t mb = M / 16, kb = K / 16;
     if (nnzb < 2 || nnzb >= (size_t)1 << 23 || K >= (size_t)1 << 28 || kb <= 2 * SWEEP_S) return 0;
     if (g_force_group_rows) return (size_t)g_force_group_rows;
-    const double row_wise = rowwise_estimate_us(M, K, N, nnzb, packed);
-    double best = std::min(row_wise / 1.25, row_wise - 0.11e-3 * (double)nnzb);
+    const double row_wise = rowwise_estimate_us(M, K, N, nnzb, n_items, lengths, packed);
+    double best = std::min(row_wise / (packed ? 1.1 : 1.2), row_wise - 0.11e-3 * (double)nnzb);
     size_t group_rows = 0;
     for (size_t rows : {(size_t)SWEEP_G, (size_t)SWEEP_G / 2, (size_t)SWEEP_G / 4}) {
         const double t = sweep_estimate_us((mb + rows - 1) / rows, sweep_listed_chunks(row_ptr, col_idx, mb, kb, rows), nnzb, M, N);
@@ -602,7 +613,7 @@ static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, s
 extern "C" void smat_internal_sweep_force_groups(int rows) { g_force_group_rows = rows; }
 extern "C" int smat_internal_sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, int packed)
 {
-    return (int)sweep_group_rows(row_ptr, col_idx, M, K, nnzb, N, packed != 0);
+    return (int)sweep_group_rows(row_ptr, col_idx, M, K, nnzb, N, M / 16, RowLengths::EVEN, packed != 0);
 }
 
 // The streams are built once the values are known to be dense.  The search for a better deal of the rows to the wavefronts
@@ -613,7 +624,8 @@ static hipError_t sweep_small_groups(smat_plan &p)
     const size_t mb = p.M / 16, kb = p.K / 16, nnzb = p.nnzb;
     if (p.col_idx_host.size() != nnzb) return hipSuccess;
     const int32_t *row_ptr = p.row_ptr_host.data(), *col_idx = p.col_idx_host.data();
-    const size_t group_rows = sweep_group_rows(row_ptr, col_idx, p.M, p.K, nnzb, p.n_cap, p.d_bpack != nullptr);
+    const size_t group_rows = sweep_group_rows(row_ptr, col_idx, p.M, p.K, nnzb, p.n_cap, (size_t)p.n_items,
+                                               p.n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, p.d_bpack != nullptr);
     if (!group_rows) return hipSuccess;
     SweepPlanHost h;
     build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 16.0 * (double)nnzb);

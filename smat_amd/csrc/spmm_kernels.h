@@ -163,6 +163,7 @@ hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, siz
 // (a plan found none to split), some were (and are split), or nothing (no plan).
 enum class RowLengths { EVEN, SPLIT, UNKNOWN };
 int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, RowLengths lengths, bool packed);
+bool rowwise_shares_items(size_t N, size_t n_items, size_t avg_blocks);
 hipError_t launch_sweep(const SweepArgs &a, hipStream_t st);
 hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st);
 

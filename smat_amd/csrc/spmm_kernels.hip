@@ -604,7 +604,7 @@ int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, RowLengths 
 // Four wavefronts per (item, panel of 64 columns): up to 512 of those, of 12 blocks and more.  (256 items of 26 blocks,
 // N = 64: 6.0 against 9.7 us; 512 items of 51 blocks, N = 64: 11.7 against 17.0; with 1024 the two are level, with more
 // the shared items lose.)  The rule knows nothing about the layout of B: in place and repacked give the same bits.
-static bool rowwise_shares_items(size_t N, size_t n_items, size_t avg_blocks)
+bool rowwise_shares_items(size_t N, size_t n_items, size_t avg_blocks)
 {
     return n_items * ((N + 63) / 64) <= 512 && avg_blocks >= 12;
 }

@@ -14,22 +14,25 @@ _fn.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_
 # m, k, n, share of the blocks (or bandwidth), whether the row-wise kernel repacks B, times of the row-wise kernel and of
 # the sweep kernel on row groups of 64, 32, 16
 MEASURED = [
-    (3088, 4112, 1000, 0.15, 1, 24.25, 27.34, 19.91, 19.92),
-    (3088, 4112, 2000, 0.15, 1, 39.61, 28.05, 22.38, 34.45),
-    (3088, 4112, 504, 0.15, 1, 15.76, 26.98, 19.12, 17.91),
-    (1600, 2000, 512, 0.2, 0, 9.92, 20.14, 13.59, 10.87),
-    (4096, 4096, 512, 0.03, 0, 9.80, 18.81, 16.93, 16.16),
-    (8192, 8192, 640, 0.04, 1, 22.75, 29.83, 28.51, 49.34),
-    (8192, 8192, 640, 0.10, 1, 45.57, 37.60, 28.88, 50.74),
-    (8192, 8192, 128, 0.10, 0, 13.59, 36.98, 27.89, 26.16),
-    (8192, 8192, 256, 0.30, 1, 38.10, 78.52, 45.01, 29.39),
-    (8192, 8192, 1536, 0.10, 1, 72.10, 41.90, 56.30, 78.70),
-    (768, 3072, 4096, 0.10, 1, 27.70, 16.98, 14.98, 14.04),
-    (2048, 1024, 2048, 0.20, 1, 13.30, 14.40, 10.30, 9.20),
-    (16384, 16384, 1024, 0.04, 1, 106.0, 61.41, 100.1, 188.7),
-    (4096, 64, 128, "band", 0, 3.80, 11.27, 7.66, 6.00),
-    (16384, 64, 1024, "band", 1, 43.10, 19.40, 22.80, 25.00),
-    (4096, 30, 1024, "band", 1, 14.90, 12.10, 9.60, 8.90),
+    (3088, 4112, 1000, 0.15, 1, 24.54, 27.29, 19.91, 19.61),
+    (3088, 4112, 2000, 0.15, 1, 40.03, 28.34, 22.08, 34.54),
+    (3088, 4112, 504, 0.15, 1, 15.27, 26.95, 19.10, 17.95),
+    (1600, 2000, 512, 0.2, 0, 9.88, 19.71, 13.48, 11.01),
+    (4096, 4096, 512, 0.03, 0, 9.61, 18.88, 17.03, 16.34),
+    (8192, 8192, 640, 0.04, 1, 23.74, 29.95, 28.66, 49.66),
+    (8192, 8192, 640, 0.10, 1, 41.69, 37.57, 29.48, 50.61),
+    (8192, 8192, 128, 0.10, 1, 13.62, 37.10, 28.07, 26.41),
+    (8192, 8192, 256, 0.30, 1, 37.49, 78.71, 45.07, 29.89),
+    (8192, 8192, 1536, 0.10, 1, 71.40, 42.11, 55.74, 77.76),
+    (5008, 3008, 800, 0.20, 1, 25.22, 26.35, 17.95, 25.66),
+    (10240, 14640, 384, 0.0647, 1, 35.56, 53.32, 51.30, 51.10),
+    (4560, 944, 168, 0.216, 0, 5.43, 10.76, 7.85, 6.94),
+    (768, 3072, 4096, 0.10, 0, 20.66, 16.88, 15.17, 14.20),
+    (2048, 1024, 2048, 0.20, 1, 13.36, 15.13, 10.91, 9.30),
+    (16384, 16384, 1024, 0.04, 1, 106.17, 60.19, 99.11, 183.55),
+    (4096, 64, 128, "band", 0, 3.82, 11.22, 7.63, 6.00),
+    (16384, 64, 1024, "band", 0, 44.59, 19.63, 23.30, 25.51),
+    (4096, 30, 1024, "band", 0, 14.96, 12.81, 10.11, 9.15),
 ]
 
 
@@ -53,7 +56,8 @@ def test_choice_is_worth_its_building(m, k, n, share, packed, row_wise, t64, t32
     if group:  # faster, and a thousand products pay for the streams (0.11 us a block)
         assert times[group] < 0.9 * row_wise
         assert 0.11 * ci.size <= 1000 * (row_wise - times[group])
-    assert times[group] <= 1.15 * min(times.values())
+    worth = [t for g, t in times.items() if not g or 0.11 * ci.size <= 1000 * (row_wise - t)]
+    assert times[group] <= 1.15 * min(worth)
 
 
 @pytest.mark.parametrize("m,k,n,nnzb", [(1024, 512, 4096, 600), (1024, 256, 4096, 300), (64, 1024, 4096, 1), (8192, 8192, 8, 26000)])
