@@ -95,7 +95,9 @@ hipError_t smat_plan::SweepDev::upload(const SweepPlanHost &h)
     up((void **)&d_chunk_ids, h.chunk_ids.data(), h.chunk_ids.size() * sizeof(int32_t));
     up((void **)&d_op_ptr, h.op_ptr.data(), h.op_ptr.size() * sizeof(int32_t));
     up((void **)&d_row_map, h.row_map.data(), h.row_map.size() * sizeof(int32_t));
-    up((void **)&d_ops, h.ops.data(), h.ops.size() * sizeof(SweepOp));
+    std::vector<SweepOp> streams;
+    encode_sweep_streams(h.rg_chunk_ptr, h.op_ptr, h.ops.data(), streams);
+    up((void **)&d_ops, streams.data(), streams.size() * sizeof(SweepOp));
     if (e != hipSuccess) release();
     return e;
 }

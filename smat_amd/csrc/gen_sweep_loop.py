@@ -9,6 +9,8 @@ to the block of the next descriptor.  A block is specialised for
     r  the block row of the wavefront the op adds to (which accumulators),
     v  whether the copies of a chunk boundary were issued between the load of its A operand and now (which s_waitcnt vmcnt),
 
+and a chunk boundary for the ops of the chunk it ends (4, 5, 6, 7 or more: again an s_waitcnt),
+
 so the run-time choices cost no instruction besides the jump.  It is written by hand because a
 wavefront issues in order: every instruction next to its MFMAs adds to its run time.  Blocks have a
 fixed size (the host computes their offsets; .org fails the build if one outgrows its slot).
@@ -16,18 +18,19 @@ Run after changing:
 
     python3 gen_sweep_loop.py > spmm_sweep_loop.inc
 
-Stream position i, J = i % 8.  Block of op i (AHEAD = 4):
+Stream position i, J = i % 8.  Block of op i (AHEAD = 7):
     even position: LDS reads of the B operands of op i + 1 (into set (J + 1) % 2), then a wait until only those
     four are left: LDS reads return in order, so the reads of op i are in registers.  Scalar loads share the
     counter and return in any order; with one of them under way the same wait holds for the reads of op i
     (it then also waits for the first read of op i + 1 or for the scalar load, whichever comes first)
     odd position: wait for everything (the reads of op i, and the descriptors that the odd position before it
     asked for), scalar load of the descriptors of ops i + 7 and i + 8 (32 bytes), LDS reads of op i + 1
-    load of the A operand of op i + AHEAD (into slot (J + AHEAD) % 8)
+    load of the A operand of op i + AHEAD (into slot (J + AHEAD) % 8 = (J - 1) % 8); its address is in the entry of op i + 1,
+    as that of op i may be overwritten already
     wait for the A operand of op i, 4 MFMAs, jump to op i + 1
     The set that the reads of op i + 1 land in is the one the MFMAs of op i - 1 took their operands from a few
-    instructions earlier: an MFMA reads its A and B sources when it starts, LDS data arrives 64 clocks later
-    at the earliest.
+    instructions earlier, and so is the slot of the A load: an MFMA reads its A and B sources when it starts, LDS data
+    arrives 64 clocks later at the earliest, global data later still.
 Chunk boundary (before the first op of every chunk but the first): the descriptor of that op names a trampoline
 instead of its block; the trampoline notes the block's offset and branches to the boundary code: own copies of
 the next chunk have landed, barrier, copies of the chunk after next, then on to the op's block.  The boundary is
@@ -37,9 +40,11 @@ Registers (fixed, all listed as clobbers):
     v40-v71    B operands, two sets of 4 tiles x 4 registers
     v72-v103   A operands, ring of eight
     v104-v106  temporaries
+    v107       what the entry code's touches of A return (never read)
     s40-s71    descriptor ring, op i in slot i % 8: w0 w1 w2 w3
     s72-s86    state: descriptor pointer, code base, chunk counter, next chunk id, chunk list pointer,
                temporaries, jump target, the block a chunk boundary continues with
+    s88-s95    the head of the stream (entry code)
     a0-a127    accumulators (block row r, tile t in a[16r + 4t .. + 3])
 """
 
@@ -48,30 +53,31 @@ import sys
 if len(sys.argv) > 1:
     sys.exit("gen_sweep_loop.py takes no arguments: it writes the one loop the library ships")
 
-AHEAD = 4                                # SWEEP_AHEAD: A operands are loaded this many stream positions ahead (ring of eight)
+AHEAD = 7                                # SWEEP_DEV_AHEAD: A operands are loaded this many stream positions ahead (ring of eight)
 BSETS, ARING = 2, 8                      # B operands are read from LDS one position ahead (two register sets)
 
 RING = 8
 BLOCK_BYTES = 128                        # SWEEP_BLOCK_BYTES
 N_BLOCKS = 8 * 8 * 2                     # SWEEP_N_BLOCKS: stream position % 8 x block row x v
-TRAMP_BASE = N_BLOCKS * BLOCK_BYTES      # SWEEP_TRAMP_BASE: after the op blocks
+TRAMP_BASE = N_BLOCKS * BLOCK_BYTES      # SWEEP_DEV_TRAMP_BASE: after the op blocks
 TRAMP_BYTES = 8                          # SWEEP_TRAMP_BYTES
-MARK_OFF = TRAMP_BASE + N_BLOCKS * TRAMP_BYTES   # SWEEP_MARK_OFF
-MARK_BYTES = 512                         # SWEEP_MARK_BYTES
-END_OFF = MARK_OFF + MARK_BYTES          # SWEEP_END_OFF
+MIN_OPS, MARKS = 4, 4                    # SWEEP_MIN_OPS, SWEEP_DEV_MARKS: boundaries after chunks of 4, 5, 6, 7 and more ops
+MARK_OFF = TRAMP_BASE + MARKS * N_BLOCKS * TRAMP_BYTES   # SWEEP_DEV_MARK_OFF
+MARK_BYTES = 512
+END_OFF = MARK_OFF + MARK_BYTES          # SWEEP_DEV_END_OFF
 COPIES = 4
-MIN_OPS = AHEAD            # SWEEP_MIN_OPS
-VM_MARK = MIN_OPS          # a boundary's copies of one boundary ago are older than the A loads of the MIN_OPS positions since
+TOUCHES = 2                              # loads of the entry code that bring A into the caches
 
 S_RING0 = 40
 DESC_AHEAD = 7   # an odd position loads the descriptors of ops i + DESC_AHEAD and the one after
 S_DP, S_BASE, S_CUR, S_NEXTK, S_CP, S_T0, S_T1, S_JMP = 72, 74, 76, 77, 78, 80, 81, 84
 S_RET = 86
-S_LAST = 86
+S_HEAD = 88
+S_LAST = S_HEAD + 7
 V_B0 = 40
 V_A0 = V_B0 + 16 * BSETS
 V_T0 = V_A0 + 4 * ARING
-V_T1, V_COPY = V_T0 + 1, V_T0 + 2
+V_T1, V_COPY, V_TOUCH = V_T0 + 1, V_T0 + 2, V_T0 + 3
 
 
 def ring(slot, word):
@@ -109,8 +115,8 @@ def b_reads(dst_set, desc_slot):
         emit(f"ds_read_b128 {bset(dst_set, t)}, v{V_T1}{off}")
 
 
-def a_load(slot):
-    emit(f"buffer_load_dwordx4 {aslot(slot)}, %[a_voff], %[rsrc], {ring(slot, 0)} offen")
+def a_load(slot, offset):
+    emit(f"buffer_load_dwordx4 {aslot(slot)}, %[a_voff], %[rsrc], {offset} offen")
 
 
 def top_wait(J):
@@ -139,7 +145,7 @@ def op_block(J, r, v):
     k = (J * 8 + r) * 2 + v
     label(f"Lb{k}")
     top_wait(J)
-    a_load(J + AHEAD)
+    a_load(J + AHEAD, ring(J + 1, 0))
     emit(f"s_waitcnt vmcnt({AHEAD + COPIES * v})")
     for t in range(4):
         acc = f"a[{16 * r + 4 * t}:{16 * r + 4 * t + 3}]"
@@ -148,16 +154,21 @@ def op_block(J, r, v):
     emit(f".org Lb0_%= + {(k + 1) * BLOCK_BYTES}")
 
 
-def trampoline(k):
-    label(f"Lt{k}")
+def trampoline(m, k):
     emit(f"s_movk_i32 s{S_RET}, {k * BLOCK_BYTES}")
-    emit("s_branch Lmark_%=")
-    emit(f".org Lb0_%= + {TRAMP_BASE + (k + 1) * TRAMP_BYTES}")
+    emit(f"s_branch Lmark{m}_%=")
+    emit(f".org Lb0_%= + {TRAMP_BASE + (m * N_BLOCKS + k + 1) * TRAMP_BYTES}")
 
 
 def boundary_code():
+    # Own copies of the chunk after the one being entered (issued one boundary ago) have landed: since then the chunk that
+    # ends here has issued MIN_OPS + m A loads or more.
+    for m in reversed(range(MARKS)):
+        label(f"Lmark{m}")
+        emit(f"s_waitcnt vmcnt({MIN_OPS + m})")
+        if m:
+            emit("s_branch Lmark_%=")
     label("Lmark")
-    emit(f"s_waitcnt vmcnt({VM_MARK})")               # own copies of the chunk after the one being entered (issued one boundary ago) have landed
     emit("s_barrier")
     emit(f"s_add_u32 s{S_CUR}, s{S_CUR}, 1")          # chunk (position in the row group's list) being entered
     emit(f"s_add_u32 s{S_T0}, s{S_CUR}, 2")
@@ -184,12 +195,15 @@ def boundary_code():
     emit(f".org Lb0_%= + {MARK_OFF + MARK_BYTES}")
 
 
-# ---- entry: descriptors of ops 0..5, A operands of ops 0..AHEAD-1, B operands of ops 0 and 1 ----
+# ---- entry: A operands of ops 0 .. AHEAD - 1 (their offsets stand in front of the stream), descriptors of ops 0 .. 7, B
+# operands of op 0.  The touches ask for a part of A that other workgroups, or this one later, will want: nobody waits for
+# them but the operands asked for after them. ----
 emit(f"s_mov_b32 s{S_DP}, %[op_lo]")
 emit(f"s_mov_b32 s{S_DP + 1}, %[op_hi]")
-emit(f"s_load_dwordx16 s[{S_RING0}:{S_RING0 + 15}], s[{S_DP}:{S_DP + 1}], 0x0")
-emit(f"s_load_dwordx16 s[{S_RING0 + 16}:{S_RING0 + 31}], s[{S_DP}:{S_DP + 1}], 0x40")
-emit(f"s_add_u32 s{S_DP}, s{S_DP}, 128")
+emit(f"s_load_dwordx8 s[{S_HEAD}:{S_HEAD + 7}], s[{S_DP}:{S_DP + 1}], 0x0")
+emit(f"s_load_dwordx16 s[{S_RING0}:{S_RING0 + 15}], s[{S_DP}:{S_DP + 1}], 0x20")
+emit(f"s_load_dwordx16 s[{S_RING0 + 16}:{S_RING0 + 31}], s[{S_DP}:{S_DP + 1}], 0x60")
+emit(f"s_add_u32 s{S_DP}, s{S_DP}, {32 + 128}")
 emit(f"s_addc_u32 s{S_DP + 1}, s{S_DP + 1}, 0")
 emit(f"s_mov_b32 s{S_CP}, %[chunk_lo]")
 emit(f"s_mov_b32 s{S_CP + 1}, %[chunk_hi]")
@@ -199,8 +213,10 @@ emit(f"s_addc_u32 s{S_CP + 1}, s{S_CP + 1}, 0")
 emit(f"s_mov_b32 s{S_CUR}, 0")
 emit("s_waitcnt lgkmcnt(0)")
 for k in range(AHEAD):
-    a_load(k)
-emit(f"s_waitcnt vmcnt({AHEAD})")                     # the copies of chunks 0, 1, 2 (issued before these loads) have landed
+    a_load(k, f"s{S_HEAD + k}")
+for t in range(TOUCHES):
+    emit(f"buffer_load_dword v{V_TOUCH}, %[touch{t}], %[rsrc], 0 offen")
+emit(f"s_waitcnt vmcnt({AHEAD + TOUCHES})")  # the copies of chunks 0, 1, 2 (issued before these loads) have landed
 emit("s_barrier")
 b_reads(0, 0)
 emit(f"s_getpc_b64 s[{S_BASE}:{S_BASE + 1}]")
@@ -213,23 +229,25 @@ for J in range(8):
     for r in range(8):
         for v in range(2):
             op_block(J, r, v)
-for k in range(N_BLOCKS):
-    trampoline(k)
+for m in range(MARKS):
+    for k in range(N_BLOCKS):
+        trampoline(m, k)
 boundary_code()
 label("Lend")                                         # offset END_OFF: the descriptor after the last op jumps here
 emit("s_waitcnt vmcnt(0) lgkmcnt(0)")
 
-clob = ([f'"v{i}"' for i in range(V_B0, V_COPY + 1)] + [f'"s{i}"' for i in range(S_RING0, S_LAST + 2)] +
+clob = ([f'"v{i}"' for i in range(V_B0, V_TOUCH + 1)] + [f'"s{i}"' for i in range(S_RING0, S_LAST + 1)] +
         [f'"a{i}"' for i in range(128)] + ['"vcc"', '"scc"', '"memory"'])
 print("// generated by gen_sweep_loop.py; do not edit")
-print(f"static_assert(SWEEP_AHEAD == {AHEAD} && SWEEP_MIN_OPS == {MIN_OPS} && SWEEP_BLOCK_BYTES == {BLOCK_BYTES} && SWEEP_TRAMP_BASE == {TRAMP_BASE} && "
-      f"SWEEP_TRAMP_BYTES == {TRAMP_BYTES} && SWEEP_MARK_OFF == {MARK_OFF} && SWEEP_END_OFF == {END_OFF}, \"regenerate spmm_sweep_loop.inc\");")
+print(f"static_assert(SWEEP_DEV_AHEAD == {AHEAD} && SWEEP_MIN_OPS == {MIN_OPS} && SWEEP_DEV_MARKS == {MARKS} && SWEEP_BLOCK_BYTES == {BLOCK_BYTES} && "
+      f"SWEEP_DEV_TRAMP_BASE == {TRAMP_BASE} && SWEEP_TRAMP_BYTES == {TRAMP_BYTES} && SWEEP_DEV_MARK_OFF == {MARK_OFF} && SWEEP_DEV_END_OFF == {END_OFF}, "
+      f"\"regenerate spmm_sweep_loop.inc\");")
 print("asm volatile(")
 for line in out:
     end = "\\n" if line.endswith(":") else "\\n\\t"
     print(f'    "{line}{end}"')
 print("    :")
-print('    : [sel01] "v"(sel01), [lane_xor] "v"(lane_xor), [rd_lane] "v"(rd_addr), [a_voff] "v"(a_voff), [rsrc] "s"(vals_rsrc),')
+print('    : [sel01] "v"(sel01), [lane_xor] "v"(lane_xor), [rd_lane] "v"(rd_addr), [a_voff] "v"(a_voff), [rsrc] "s"(vals_rsrc), [touch0] "v"(touch[0]), [touch1] "v"(touch[1]),')
 print('      [copy_off] "v"(copy_off), [copy_lim] "v"(copy_lim), [dst_wave] "s"(dst_wave), [n_chunks] "s"(n_chunks_u),')
 print('      [sb0] "s"(sb0), [sb1] "s"(sb1), [sb2] "s"(sb2), [sb3] "s"(sb3),')
 print('      [op_lo] "s"(op_lo), [op_hi] "s"(op_hi), [chunk_lo] "s"(chunk_lo), [chunk_hi] "s"(chunk_hi)')

@@ -22,9 +22,12 @@
 //    loads, two at a time, seven positions ahead.
 //  * Pipeline.  The B operands of an op are read from LDS one position ahead (two register sets), its A
 //    operand (two neighbouring 512-byte blocks, one load straight into MFMA layout) comes from global memory
-//    four positions ahead (ring of eight).  Vector memory operations complete in order, so the number of
-//    younger ones at every wait is known when the plan is built: 4, or 8 when a chunk boundary issued its copies in
-//    between.  A half of an MFMA that must not contribute (unpaired block) reads a 16 KiB region of zeros.
+//    seven positions ahead (ring of eight).  Vector memory operations complete in order, so the number of
+//    younger ones at every wait is known when the plan is uploaded: 7, or 11 when a chunk boundary issued its copies in
+//    between.  In order also means that an A operand asked for behind the copies of a boundary waits for them: four
+//    positions were 0.7 us for copies that come from HBM.  Four -> seven, 8192^2, 10 %, N = 4096: 104.4 -> 101.5 us with
+//    inputs that change from launch to launch, 89 -> 86 with the same ones again.  A half of an MFMA that must not
+//    contribute (unpaired block) reads a 16 KiB region of zeros.
 //  * Accumulators live in a[0:127] and are touched by inline assembly only.
 //  * Synchronisation.  One barrier per chunk, in the boundary code that the first op of the chunk runs through
 //    before its own block (it is no stream position: no descriptor, no operand load is spent on it).  Boundary of
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(THREADS) void spmm_sweep_kernel(
     const uint16_t *__restrict__ vals, const uint16_t *__restrict__ B, void *__restrict__ Cout,
     const int32_t *__restrict__ rg_chunk_ptr, const int32_t *__restrict__ chunk_ids,
     const int32_t *__restrict__ op_ptr, const SweepOp *__restrict__ ops, const int32_t *__restrict__ row_map, int N, long K, int n_rg, int n_panels,
-    uint32_t vals_bytes, int n_vb)
+    uint32_t vals_bytes, uint32_t touch_bytes, int n_vb)
 {
     extern __shared__ __align__(16) unsigned char lds[];
 
@@ -211,11 +214,19 @@ __global__ __launch_bounds__(THREADS) void spmm_sweep_kernel(
         const uint32_t a_voff = (uint32_t)sel * 512u + a_lane_bytes; // lanes 32-63 take the second block of the pair
         const uint32_t sel01 = (uint32_t)sel;
         const uint32_t n_chunks_u = __builtin_amdgcn_readfirstlane((uint32_t)n_chunks);
-        const SweepOp *op_base = ops + op_begin;
+        const SweepOp *op_base = ops + op_begin + SWEEP_DEV_HEAD * (rg * W + wave);
         const uint32_t op_lo = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)op_base);
         const uint32_t op_hi = __builtin_amdgcn_readfirstlane((uint32_t)((uintptr_t)op_base >> 32));
         const uint32_t chunk_lo = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)chunk_ptr);
         const uint32_t chunk_hi = __builtin_amdgcn_readfirstlane((uint32_t)((uintptr_t)chunk_ptr >> 32));
+        // Touches: every lane of the launch asks for one word of a 128-byte line of A, twice, so that A is on its way from HBM
+        // before the wavefronts get to it; lines behind touch_bytes are outside the buffer and cost no access.
+        uint32_t touch[2];
+        const uint64_t line = ((uint64_t)blockIdx.x * THREADS + (uint64_t)tid) * 128u;
+        for (int t = 0; t < 2; t++) {
+            const uint64_t at = line + t * ((uint64_t)gridDim.x * THREADS * 128u);
+            touch[t] = vb == (int)blockIdx.x && at < touch_bytes ? (uint32_t)at : 0xffffffffu;
+        }
 #include "spmm_sweep_loop.inc"
     }
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); // the last MFMAs retire before their results are read
@@ -292,15 +303,21 @@ hipError_t launch_sweep(const SweepArgs &a, hipStream_t st)
             if (launched > resident) launched = resident;
         }
     }
+    // A is touched ahead where the launch before has displaced it: where A, B and C are more than half of the 256 MiB of the
+    // memory-side cache.  8192^2, 10 %, N = 4096, inputs changing: 101.5 -> 97.2 us.  With A still in that cache the touches only
+    // cost (the same with N = 2048: 42.1 -> 43.2 us; 3088 x 4112, 15 %, N = 1000: 22.7 -> 23.0), and so they do where two per
+    // lane do not reach the end of A (8192^2, 30 %, N = 4096: 202.5 -> 204.6).
+    const size_t vals_bytes = a.nnzb * 512, traffic = vals_bytes + a.K * a.N * 2 + a.M * a.N * (a.c_f32 ? 4 : 2);
+    const uint32_t touch_bytes = traffic >= ((size_t)128 << 20) && vals_bytes <= (size_t)launched * THREADS * 128 * 2 ? (uint32_t)vals_bytes : 0;
     dim3 grid((unsigned)launched), block(THREADS);
     if (a.c_f32)
         hipLaunchKernelGGL((spmm_sweep_kernel<true>), grid, block, lds_bytes, st, a.vals, a.B, a.C,
                            a.rg_chunk_ptr, a.chunk_ids, a.op_ptr, a.ops, a.row_map, (int)a.N, (long)a.K,
-                           a.n_rg, n_panels, (uint32_t)(a.nnzb * 512), (int)wgs);
+                           a.n_rg, n_panels, (uint32_t)(a.nnzb * 512), touch_bytes, (int)wgs);
     else
         hipLaunchKernelGGL((spmm_sweep_kernel<false>), grid, block, lds_bytes, st, a.vals, a.B, a.C,
                            a.rg_chunk_ptr, a.chunk_ids, a.op_ptr, a.ops, a.row_map, (int)a.N, (long)a.K,
-                           a.n_rg, n_panels, (uint32_t)(a.nnzb * 512), (int)wgs);
+                           a.n_rg, n_panels, (uint32_t)(a.nnzb * 512), touch_bytes, (int)wgs);
     return hipGetLastError();
 }
 

@@ -1,5 +1,7 @@
 // Stream format of the sweep kernel (spmm_sweep.hip), shared by the kernel, its generated interpreter
 // (gen_sweep_loop.py) and the host-side plan builder (sweep_plan.cpp).  No HIP types.
+// build_sweep_plan makes the streams as described first; encode_sweep_streams turns them into what the kernel runs (end of
+// this file), which asks for A earlier than the 4 positions that the streams of the plan are numbered for.
 #pragma once
 #include <stdint.h>
 
@@ -49,6 +51,25 @@ constexpr uint32_t SWEEP_TRAMP_BYTES = 8;
 constexpr uint32_t SWEEP_MARK_OFF = SWEEP_TRAMP_BASE + SWEEP_N_BLOCKS * SWEEP_TRAMP_BYTES; // 17408: the chunk boundary code
 constexpr uint32_t SWEEP_MARK_BYTES = 512;
 constexpr uint32_t SWEEP_END_OFF = SWEEP_MARK_OFF + SWEEP_MARK_BYTES;               // 17920
+
+// The streams as the kernel runs them.  Each starts with SWEEP_DEV_HEAD entries that hold, one uint32 after the other, the A
+// offsets of its first AHEAD ops (0 behind the last op), where AHEAD = SWEEP_DEV_AHEAD; then come the entries of the plan with
+//   w0  the A offset of op i + AHEAD - 1 (0 behind the last op): the position in front asks for it
+//   w1, w2 as in the plan
+//   w3  op      its block, v = 1 when the copies of a chunk boundary were issued after the load of this op's A operand; the
+//               block waits until AHEAD + 4 v vector memory operations are under way, with the copies of two boundaries in
+//               between (chunks of less than AHEAD ops) for a little more than it has to
+//       first op of every chunk but the first:  SWEEP_DEV_TRAMP_BASE + (m * SWEEP_N_BLOCKS + the op's block index) *
+//               SWEEP_TRAMP_BYTES, m = min(ops of the chunk before, AHEAD) - SWEEP_MIN_OPS: so many more A loads than
+//               SWEEP_MIN_OPS may be under way when the boundary's own copies have landed
+//       end     SWEEP_DEV_END_OFF
+constexpr int SWEEP_DEV_AHEAD = 7; // with a ring of eight operands the most there is room for
+constexpr int SWEEP_DEV_HEAD = 2;
+constexpr int SWEEP_DEV_MARKS = SWEEP_DEV_AHEAD - SWEEP_MIN_OPS + 1;
+constexpr uint32_t SWEEP_DEV_TRAMP_BASE = SWEEP_TRAMP_BASE;
+constexpr uint32_t SWEEP_DEV_MARK_OFF = SWEEP_DEV_TRAMP_BASE + SWEEP_DEV_MARKS * SWEEP_N_BLOCKS * SWEEP_TRAMP_BYTES;
+constexpr uint32_t SWEEP_DEV_END_OFF = SWEEP_DEV_MARK_OFF + SWEEP_MARK_BYTES;
+static_assert(SWEEP_DEV_AHEAD <= 4 * SWEEP_DEV_HEAD && SWEEP_DEV_AHEAD > SWEEP_MIN_OPS, "the head holds the offsets of the first ops");
 
 inline uint32_t sweep_lds_offset(int32_t chunk_pos, int32_t slab)
 {

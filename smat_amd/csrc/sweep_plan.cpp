@@ -376,7 +376,64 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
     out.chunk_ids.resize(out.chunk_ids.size() + SWEEP_CHUNK_PAD, 0);
 }
 
+void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::vector<int32_t> &op_ptr, const SweepOpHost *ops,
+                          std::vector<SweepOpHost> &dev)
+{
+    constexpr int DEV_AHEAD = SWEEP_DEV_AHEAD, HEAD = SWEEP_DEV_HEAD;
+    const size_t n_streams = op_ptr.size() - 1;
+    dev.assign((size_t)op_ptr.back() + HEAD * n_streams + SWEEP_OP_PAD, SweepOpHost{0, SWEEP_ZERO_OFF, 0, SWEEP_DEV_END_OFF});
+    std::vector<long> a_issue;
+    for (size_t s = 0; s < n_streams; s++) {
+        const SweepOpHost *op = ops + op_ptr[s];
+        SweepOpHost *out = dev.data() + op_ptr[s] + HEAD * s;
+        const size_t len = (size_t)(op_ptr[s + 1] - op_ptr[s]), n_ops = len ? len - 1 : 0; // the end is no op
+        const long n_chunks = rg_chunk_ptr[s / WAVES + 1] - rg_chunk_ptr[s / WAVES];
+        auto a_offset = [&](size_t i) { return i < n_ops ? op[i].w0 : 0u; };
+        uint32_t head[4 * HEAD] = {0};
+        for (int k = 0; k < DEV_AHEAD; k++) head[k] = a_offset((size_t)k);
+        memcpy(out, head, sizeof head);
+        out += HEAD;
+        // vector memory operations in issue order: what is younger than the load of an op's A operand when the op needs it
+        a_issue.assign(len + DEV_AHEAD + 1, 0);
+        long seq = 0, cur = 0, in_chunk = 0;
+        for (int k = 0; k < DEV_AHEAD; k++) a_issue[(size_t)k] = ++seq;
+        for (size_t i = 0; i < n_ops; i++) {
+            const bool opens = op[i].w3 >= SWEEP_TRAMP_BASE;
+            const uint32_t block = opens ? (op[i].w3 - SWEEP_TRAMP_BASE) / SWEEP_TRAMP_BYTES : op[i].w3 / SWEEP_BLOCK_BYTES;
+            uint32_t m = 0;
+            if (opens) {
+                if (in_chunk < MIN_OPS) throw std::logic_error("sweep plan: chunk boundaries closer than the copies' wait allows");
+                m = (uint32_t)(std::min<long>(in_chunk, DEV_AHEAD) - MIN_OPS);
+                in_chunk = 0;
+                if (++cur + 2 < n_chunks) seq += COPIES;
+            }
+            in_chunk++;
+            a_issue[i + DEV_AHEAD] = ++seq;
+            const uint32_t v = seq - a_issue[i] > DEV_AHEAD ? 1u : 0u;
+            const uint32_t code = (block & ~1u) | v;
+            out[i].w0 = a_offset(i + DEV_AHEAD - 1);
+            out[i].w1 = op[i].w1;
+            out[i].w2 = op[i].w2;
+            out[i].w3 = opens ? SWEEP_DEV_TRAMP_BASE + (m * SWEEP_N_BLOCKS + code) * SWEEP_TRAMP_BYTES : code * SWEEP_BLOCK_BYTES;
+        }
+        // the end stays what dev was filled with
+    }
+}
+
 } // namespace smat
+
+// Test hook (not part of smat.h): the streams of a plan that smat_internal_sweep_plan handed out as the kernel runs them, in
+// out[0 .. op_ptr[8 n_rg] + 2 * 8 n_rg + 16).
+extern "C" int smat_internal_sweep_encode(const int32_t *rg_chunk_ptr, int64_t n_rg, const int32_t *op_ptr, const uint32_t *ops, uint32_t *out)
+{
+    return smat::guarded("smat_internal_sweep_encode", [&] {
+        const std::vector<int32_t> chunk_ptr(rg_chunk_ptr, rg_chunk_ptr + n_rg + 1), ptr(op_ptr, op_ptr + n_rg * smat::SWEEP_WAVES + 1);
+        std::vector<smat::SweepOpHost> dev;
+        smat::encode_sweep_streams(chunk_ptr, ptr, reinterpret_cast<const smat::SweepOpHost *>(ops), dev);
+        memcpy(out, dev.data(), dev.size() * sizeof(smat::SweepOpHost));
+        return (int)SMAT_OK;
+    });
+}
 
 // Test hook (not part of smat.h): builds the work list on the host (rows != NULL: of these block rows only) and hands it out.  Arrays are
 // allocated with malloc; release each with smat_host_free.  row_map: n_rg * 64 block rows (-1 = none).  counts[0..5] = row groups, listed

@@ -31,4 +31,9 @@ struct SweepPlanHost {
 void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, SweepPlanHost &out,
                       const int32_t *rows = nullptr, size_t n_rows = 0, size_t group_rows = SWEEP_G, double search = 2e8);
 
+// The plan's streams as the kernel runs them (second part of sweep_format.h): stream s from dev[op_ptr[s] + SWEEP_DEV_HEAD * s] on,
+// and SWEEP_OP_PAD entries after the last.
+void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::vector<int32_t> &op_ptr, const SweepOpHost *ops,
+                          std::vector<SweepOpHost> &dev);
+
 } // namespace smat
