@@ -44,11 +44,13 @@ struct smat_plan {
         int n_rg = 0, n_records = 0, n_ops = 0;
         int32_t *d_rg_chunk_ptr = nullptr, *d_chunk_ids = nullptr, *d_op_ptr = nullptr, *d_row_map = nullptr;
         SweepOp *d_ops = nullptr;
-        hipError_t upload(const SweepPlanHost &h);
+        SweepOp *d_ops_row_major = nullptr; // the streams for row-major B (plans made for SMAT_B_ROW_MAJOR)
+        hipError_t upload(const SweepPlanHost &h, bool b_row_major);
         void release();
-        void fill(SweepArgs &w) const
+        void fill(SweepArgs &w, bool b_row_major) const
         {
-            w.rg_chunk_ptr = d_rg_chunk_ptr; w.chunk_ids = d_chunk_ids; w.op_ptr = d_op_ptr; w.ops = d_ops;
+            w.rg_chunk_ptr = d_rg_chunk_ptr; w.chunk_ids = d_chunk_ids; w.op_ptr = d_op_ptr;
+            w.b_row_major = b_row_major; w.ops = b_row_major ? d_ops_row_major : d_ops;
             w.row_map = d_row_map; w.n_rg = n_rg;
         }
     };
@@ -79,7 +81,7 @@ struct smat_plan {
     uint16_t *d_bcol = nullptr; // column-major copy of a row-major B, K * n_cap halves (plans made for SMAT_B_ROW_MAJOR)
 };
 
-hipError_t smat_plan::SweepDev::upload(const SweepPlanHost &h)
+hipError_t smat_plan::SweepDev::upload(const SweepPlanHost &h, bool b_row_major)
 {
     release();
     n_rg = (int)h.rg_chunk_ptr.size() - 1;
@@ -96,17 +98,21 @@ hipError_t smat_plan::SweepDev::upload(const SweepPlanHost &h)
     up((void **)&d_op_ptr, h.op_ptr.data(), h.op_ptr.size() * sizeof(int32_t));
     up((void **)&d_row_map, h.row_map.data(), h.row_map.size() * sizeof(int32_t));
     std::vector<SweepOp> streams;
-    encode_sweep_streams(h.rg_chunk_ptr, h.op_ptr, h.ops.data(), streams);
+    encode_sweep_streams(h.rg_chunk_ptr, h.op_ptr, h.ops.data(), false, streams);
     up((void **)&d_ops, streams.data(), streams.size() * sizeof(SweepOp));
+    if (b_row_major) {
+        encode_sweep_streams(h.rg_chunk_ptr, h.op_ptr, h.ops.data(), true, streams);
+        up((void **)&d_ops_row_major, streams.data(), streams.size() * sizeof(SweepOp));
+    }
     if (e != hipSuccess) release();
     return e;
 }
 void smat_plan::SweepDev::release()
 {
-    for (void *q : {(void *)d_rg_chunk_ptr, (void *)d_chunk_ids, (void *)d_op_ptr, (void *)d_row_map, (void *)d_ops})
+    for (void *q : {(void *)d_rg_chunk_ptr, (void *)d_chunk_ids, (void *)d_op_ptr, (void *)d_row_map, (void *)d_ops, (void *)d_ops_row_major})
         if (q) (void)dev_free(q);
     d_rg_chunk_ptr = d_chunk_ids = d_op_ptr = d_row_map = nullptr;
-    d_ops = nullptr;
+    d_ops = d_ops_row_major = nullptr;
     n_rg = n_records = n_ops = 0;
 }
 
@@ -184,6 +190,11 @@ static double rowwise_estimate_us(size_t M, size_t K, size_t N, size_t nnzb, siz
     const double column = !packed || tiles <= 4 ? 1.0 : tiles == 8 ? 0.83 : 0.8;
     return start + (double)rounds * (double)tiles * (double)nnzb / (double)n_items * (packed ? 0.0274 * column : 0.074);
 }
+// A row-major B into column-major order, for the kernels that do not read it in place (8192 x 4096 23 us, 4112 x 504 3 us beside
+// the launch that follows); and what the sweep kernel takes longer on a row-major B in place (8192^2, 10 %, N = 4096 103 against 97 us,
+// with N = 2040, rows that straddle cache lines, 50 against 43).
+static double to_col_major_us(size_t K, size_t N) { return 2.0 + 0.6e-6 * (double)K * (double)N; }
+static double sweep_in_place_factor(size_t N) { return N % 64 == 0 ? 1.05 : 1.13; }
 static size_t sweep_listed_chunks(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t group_rows)
 {
     std::vector<size_t> seen((kb + SWEEP_S - 1) / SWEEP_S, 0); // the last row group that listed the chunk, from 1
@@ -246,24 +257,37 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         kernel = SMAT_KERNEL_ROWWISE;
     }
     // a plan made for a wide N, used with a narrow one: too few workgroups for the sweep kernel
-    if (kernel == SMAT_KERNEL_SWEEP && o.kernel == SMAT_KERNEL_AUTO &&
-        (plan->sweep_few_tiles ? sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N) > rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, plan->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, a.b_packed != nullptr)
-                               : !sweep_fills_device(M / 16, N)))
-        kernel = SMAT_KERNEL_ROWWISE;
+    if (kernel == SMAT_KERNEL_SWEEP && o.kernel == SMAT_KERNEL_AUTO) {
+        const bool in_place = o.b_layout == SMAT_B_ROW_MAJOR && plan->sweep.d_ops_row_major && sweep_takes_row_major(N, K, plan->sweep.n_rg);
+        const double row_wise = rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, plan->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN,
+                                                    a.b_packed != nullptr) + (in_place ? to_col_major_us(K, N) : 0.0);
+        const double factor = in_place ? sweep_in_place_factor(N) : 1.0;
+        if (plan->sweep_few_tiles ? factor * sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N) > row_wise
+                                  : !sweep_fills_device(M / 16, N))
+            kernel = SMAT_KERNEL_ROWWISE;
+    }
     const uint16_t *B_as_given = B;
+    bool sweep_row_major = false;
     if (kernel == SMAT_KERNEL_MIXED && (!plan || !plan->compact || (!plan->d_items_dense && !plan->sweep_dense.d_ops && !plan->sweep_blocks.d_ops) || !plan->d_bt || N > plan->n_cap))
         return set_error(SMAT_ERR_INVALID, "SMAT_KERNEL_MIXED needs a plan that split the block rows when the values were "
                                            "attached (smat_plan_attach_values) and n_hint >= N");
     if (o.b_layout == SMAT_B_ROW_MAJOR && kernel != SMAT_KERNEL_COMPACT) {
-        // the row-wise and sweep kernels want 8 consecutive k of one column in a lane: B is first brought into the
-        // reference layout in plan scratch, then they run as for column-major B (same bits in C)
+        // the row-wise kernel wants 8 consecutive k of one column in a lane: B is first brought into the reference layout in
+        // plan scratch, then it runs as for column-major B; the sweep kernel reads B in place (same bits in C either way)
         if (!plan || !plan->d_bcol || N > plan->n_cap)
             return set_error(SMAT_ERR_UNSUPPORTED,
                              "row-major B (B[k*N+n]) with the row-wise or sweep kernel needs a plan created with "
                              "b_layout = SMAT_B_ROW_MAJOR and n_hint >= N; the compact kernel reads it in place");
-        e = launch_b_to_col_major(B, plan->d_bcol, N, K, static_cast<hipStream_t>(o.stream));
-        if (e != hipSuccess) return set_error(SMAT_ERR_HIP, "SpMM launch failed: %s", hipGetErrorString(e));
-        a.B = B = plan->d_bcol;
+        const smat_plan::SweepDev *sweep = kernel == SMAT_KERNEL_SWEEP ? &plan->sweep
+                                         : kernel != SMAT_KERNEL_MIXED ? nullptr
+                                         : plan->sweep_blocks.d_ops    ? &plan->sweep_blocks
+                                                                       : &plan->sweep_dense;
+        sweep_row_major = sweep && sweep->d_ops_row_major && sweep_takes_row_major(N, K, sweep->n_rg);
+        if (!sweep_row_major) {
+            e = launch_b_to_col_major(B, plan->d_bcol, N, K, static_cast<hipStream_t>(o.stream));
+            if (e != hipSuccess) return set_error(SMAT_ERR_HIP, "SpMM launch failed: %s", hipGetErrorString(e));
+            a.B = B = plan->d_bcol;
+        }
     }
     if (kernel == SMAT_KERNEL_MIXED) {
         // the block rows with mostly full blocks through the row-wise kernel, the others (and the empty ones) through
@@ -273,12 +297,12 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
             // written), then the compact kernel adds the columns of the other blocks
             SweepArgs w{};
             w.vals = plan->d_vals_dense; w.B = B; w.C = C; w.M = M; w.N = N; w.K = K; w.nnzb = (size_t)plan->n_blocks_split; w.c_f32 = a.c_f32;
-            plan->sweep_blocks.fill(w);
+            plan->sweep_blocks.fill(w, sweep_row_major);
             e = launch_sweep(w, static_cast<hipStream_t>(o.stream));
         } else if (plan->sweep_dense.d_ops) {
             SweepArgs w{};
             w.vals = vals; w.B = B; w.C = C; w.M = M; w.N = N; w.K = K; w.nnzb = nnzb; w.c_f32 = a.c_f32;
-            plan->sweep_dense.fill(w);
+            plan->sweep_dense.fill(w, sweep_row_major);
             e = launch_sweep(w, static_cast<hipStream_t>(o.stream));
         } else {
             SpmmArgs d = a;
@@ -310,7 +334,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
             return set_error(SMAT_ERR_INVALID, "SMAT_KERNEL_SWEEP needs a plan built for it (with col_idx_host)");
         SweepArgs w{};
         w.vals = vals; w.B = B; w.C = C; w.M = M; w.N = N; w.K = K; w.nnzb = nnzb; w.c_f32 = a.c_f32;
-        plan->sweep.fill(w);
+        plan->sweep.fill(w, sweep_row_major);
         e = launch_sweep(w, static_cast<hipStream_t>(o.stream));
     } else {
         e = launch_rowwise(a, static_cast<hipStream_t>(o.stream));
@@ -561,7 +585,7 @@ static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
         build_sweep_plan(row_ptr_host, col_idx_host, mb, kb, h);
         p->kernel = SMAT_KERNEL_SWEEP;
         static_assert(sizeof(SweepOpHost) == sizeof(SweepOp), "host and device op layouts");
-        e = p->sweep.upload(h);
+        e = p->sweep.upload(h, p->d_bcol != nullptr);
         if (p->d_bpack && want != SMAT_KERNEL_ROWWISE_PACKED) { // the sweep kernel reads B in place
             (void)dev_free(p->d_bpack);
             p->d_bpack = nullptr;
@@ -596,16 +620,20 @@ extern "C" int smat_plan_create(smat_plan **out, const int32_t *row_ptr_host,
 // with the row-wise kernel.  Returns the block rows of a group, 0 = row-wise.
 static int g_force_group_rows = 0; // test hook: 64, 32 or 16 whatever the estimates say
 static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, size_t n_items,
-                               RowLengths lengths, bool packed)
+                               RowLengths lengths, bool packed, bool b_row_major)
 {
     const size_t mb = M / 16, kb = K / 16;
     if (nnzb < 2 || nnzb >= (size_t)1 << 23 || K >= (size_t)1 << 28 || kb <= 2 * SWEEP_S) return 0;
     if (g_force_group_rows) return (size_t)g_force_group_rows;
-    const double row_wise = rowwise_estimate_us(M, K, N, nnzb, n_items, lengths, packed);
+    const double to_col_major = b_row_major ? to_col_major_us(K, N) : 0.0;
+    const double row_wise = rowwise_estimate_us(M, K, N, nnzb, n_items, lengths, packed) + to_col_major;
     double best = std::min(row_wise / (packed ? 1.1 : 1.2), row_wise - 0.11e-3 * (double)nnzb);
     size_t group_rows = 0;
     for (size_t rows : {(size_t)SWEEP_G, (size_t)SWEEP_G / 2, (size_t)SWEEP_G / 4}) {
-        const double t = sweep_estimate_us((mb + rows - 1) / rows, sweep_listed_chunks(row_ptr, col_idx, mb, kb, rows), nnzb, M, N);
+        const size_t n_rg = (mb + rows - 1) / rows;
+        const double sweep = sweep_estimate_us(n_rg, sweep_listed_chunks(row_ptr, col_idx, mb, kb, rows), nnzb, M, N);
+        const bool in_place = b_row_major && sweep_takes_row_major(N, K, (int)n_rg);
+        const double t = in_place ? sweep_in_place_factor(N) * sweep : sweep + to_col_major;
         if (t < best) best = t, group_rows = rows;
     }
     return group_rows;
@@ -615,7 +643,7 @@ static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, s
 extern "C" void smat_internal_sweep_force_groups(int rows) { g_force_group_rows = rows; }
 extern "C" int smat_internal_sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, int packed)
 {
-    return (int)sweep_group_rows(row_ptr, col_idx, M, K, nnzb, N, M / 16, RowLengths::EVEN, packed != 0);
+    return (int)sweep_group_rows(row_ptr, col_idx, M, K, nnzb, N, M / 16, RowLengths::EVEN, packed != 0, false);
 }
 
 // The streams are built once the values are known to be dense.  The search for a better deal of the rows to the wavefronts
@@ -627,11 +655,11 @@ static hipError_t sweep_small_groups(smat_plan &p)
     if (p.col_idx_host.size() != nnzb) return hipSuccess;
     const int32_t *row_ptr = p.row_ptr_host.data(), *col_idx = p.col_idx_host.data();
     const size_t group_rows = sweep_group_rows(row_ptr, col_idx, p.M, p.K, nnzb, p.n_cap, (size_t)p.n_items,
-                                               p.n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, p.d_bpack != nullptr);
+                                               p.n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, p.d_bpack != nullptr, p.d_bcol != nullptr);
     if (!group_rows) return hipSuccess;
     SweepPlanHost h;
     build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 16.0 * (double)nnzb);
-    const hipError_t e = p.sweep.upload(h);
+    const hipError_t e = p.sweep.upload(h, p.d_bcol != nullptr);
     if (e != hipSuccess) {
         p.sweep.release();
         return e;
@@ -802,7 +830,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
             try { // the list and the copies made so far are released by fail() below
                 SweepPlanHost h;
                 build_sweep_plan(rp_d.data(), ci_d.data(), mb, p->K / 16, h, nullptr, 0);
-                e = p->sweep_blocks.upload(h);
+                e = p->sweep_blocks.upload(h, p->d_bcol != nullptr);
             } catch (...) {
                 e = hipErrorOutOfMemory;
             }
@@ -813,7 +841,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
         try {
             SweepPlanHost h;
             build_sweep_plan(row_ptr_host, p->col_idx_host.data(), mb, p->K / 16, h, dense_list.data(), dense_list.size());
-            e = p->sweep_dense.upload(h);
+            e = p->sweep_dense.upload(h, p->d_bcol != nullptr);
         } catch (...) {
             e = hipErrorOutOfMemory;
         }

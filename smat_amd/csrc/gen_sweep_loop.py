@@ -1,5 +1,6 @@
 #!/usr/bin/env python3
-"""Writes spmm_sweep_loop.inc: the op interpreter of the sweep kernel as one inline-assembly statement.
+"""Writes spmm_sweep_loop.inc: the op interpreter of the sweep kernel as one inline-assembly statement, for column-major
+B and, where SMAT_SWEEP_ROW_MAJOR is defined, for row-major B.
 
 The stream of one wavefront (see spmm_sweep.hip for the scheme) is threaded code: every 16-byte
 descriptor ends in the byte offset of the code block that executes it, and every block ends in a jump
@@ -36,11 +37,16 @@ instead of its block; the trampoline notes the block's offset and branches to th
 the next chunk have landed, barrier, copies of the chunk after next, then on to the op's block.  The boundary is
 no stream position: no operand load and no descriptor slot is spent on it.
 
+Row-major B: rows of 64 columns, 128 bytes, as they lie in B; the operands come out of LDS through transposing reads of
+8 bytes a lane (ds_read_b64_tr_b16: the four rows that 16 lanes read come back as four k of one column each), eight instead
+of four an op; tile t is at the address of tile 0 with 8 t xor-ed to it.  LDS operations under way are counted in four bits, so an even position waits for op i when half of the
+reads of op i + 1 are on their way.
+
 Registers (fixed, all listed as clobbers):
     v40-v71    B operands, two sets of 4 tiles x 4 registers
     v72-v103   A operands, ring of eight
-    v104-v106  temporaries
-    v107       what the entry code's touches of A return (never read)
+    v104-v108  temporaries
+    v109       what the entry code's touches of A return (never read)
     s40-s71    descriptor ring, op i in slot i % 8: w0 w1 w2 w3
     s72-s86    state: descriptor pointer, code base, chunk counter, next chunk id, chunk list pointer,
                temporaries, jump target, the block a chunk boundary continues with
@@ -57,14 +63,10 @@ AHEAD = 7                                # SWEEP_DEV_AHEAD: A operands are loade
 BSETS, ARING = 2, 8                      # B operands are read from LDS one position ahead (two register sets)
 
 RING = 8
-BLOCK_BYTES = 128                        # SWEEP_BLOCK_BYTES
 N_BLOCKS = 8 * 8 * 2                     # SWEEP_N_BLOCKS: stream position % 8 x block row x v
-TRAMP_BASE = N_BLOCKS * BLOCK_BYTES      # SWEEP_DEV_TRAMP_BASE: after the op blocks
 TRAMP_BYTES = 8                          # SWEEP_TRAMP_BYTES
 MIN_OPS, MARKS = 4, 4                    # SWEEP_MIN_OPS, SWEEP_DEV_MARKS: boundaries after chunks of 4, 5, 6, 7 and more ops
-MARK_OFF = TRAMP_BASE + MARKS * N_BLOCKS * TRAMP_BYTES   # SWEEP_DEV_MARK_OFF
-MARK_BYTES = 512
-END_OFF = MARK_OFF + MARK_BYTES          # SWEEP_DEV_END_OFF
+MARK_BYTES = 512                         # SWEEP_MARK_BYTES
 COPIES = 4
 TOUCHES = 2                              # loads of the entry code that bring A into the caches
 
@@ -77,7 +79,22 @@ S_LAST = S_HEAD + 7
 V_B0 = 40
 V_A0 = V_B0 + 16 * BSETS
 V_T0 = V_A0 + 4 * ARING
-V_T1, V_COPY, V_TOUCH = V_T0 + 1, V_T0 + 2, V_T0 + 3
+V_T1, V_COPY, V_TOUCH = V_T0 + 1, V_T0 + 4, V_T0 + 5
+
+
+ROW_MAJOR = False                        # the loop being written; what follows depends on it
+
+
+def block_bytes():
+    return 192 if ROW_MAJOR else 128     # sweep_block_bytes
+
+
+def tramp_base():
+    return N_BLOCKS * block_bytes()      # sweep_tramp_base: after the op blocks
+
+
+def mark_off():
+    return tramp_base() + MARKS * N_BLOCKS * TRAMP_BYTES
 
 
 def ring(slot, word):
@@ -105,14 +122,29 @@ def label(name):
     emit(f"{name}_%=:")
 
 
-def b_reads(dst_set, desc_slot):
-    """B operands of the op in ring slot desc_slot: lanes 0-31 at w1, lanes 32-63 at w1 + w2."""
+def b_reads(dst_set, desc_slot, wait=None):
+    """B operands of the op in ring slot desc_slot: lanes 0-31 at w1, lanes 32-63 at w1 + w2.  wait: how many of these reads may
+    be under way when those before them have to be back, 4 at most."""
+    if ROW_MAJOR:
+        emit(f"v_mad_i32_i24 v{V_T0}, {ring(desc_slot, 2)}, %[sel01], %[rd_lane]")
+        emit(f"v_add_u32 v{V_T0}, {ring(desc_slot, 1)}, v{V_T0}")
+        for t in range(1, 4):
+            emit(f"v_xor_b32 v{V_T0 + t}, {8 * t}, v{V_T0}")
+        for t in range(4):
+            b = V_B0 + 16 * (dst_set % BSETS) + 4 * t
+            for h in range(2):
+                emit(f"ds_read_b64_tr_b16 v[{b + 2 * h}:{b + 2 * h + 1}], v{V_T0 + t}" + (" offset:512" if h else ""))
+            if t == 1 and wait is not None:
+                emit(f"s_waitcnt lgkmcnt({wait})")
+        return
     emit(f"v_mul_i32_i24 v{V_T0}, {ring(desc_slot, 2)}, %[sel01]")
     emit(f"v_add_u32 v{V_T0}, {ring(desc_slot, 1)}, v{V_T0}")
     emit(f"v_xad_u32 v{V_T1}, v{V_T0}, %[lane_xor], %[rd_lane]")
     for t in range(4):
         off = f" offset:{1024 * t}" if t else ""
         emit(f"ds_read_b128 {bset(dst_set, t)}, v{V_T1}{off}")
+    if wait is not None:
+        emit(f"s_waitcnt lgkmcnt({wait})")
 
 
 def a_load(slot, offset):
@@ -124,8 +156,7 @@ def top_wait(J):
     only they are left; an odd position waits for everything (reads of op i, descriptors asked for two positions
     ago), asks for two descriptors and then for the reads of op i + 1."""
     if J % 2 == 0:
-        b_reads(J + 1, J + 1)
-        emit("s_waitcnt lgkmcnt(4)")
+        b_reads(J + 1, J + 1, wait=4)
         return
     emit("s_waitcnt lgkmcnt(0)")
     s0 = S_RING0 + 4 * ((J + DESC_AHEAD) % RING)
@@ -151,13 +182,13 @@ def op_block(J, r, v):
         acc = f"a[{16 * r + 4 * t}:{16 * r + 4 * t + 3}]"
         emit(f"v_mfma_f32_16x16x32_f16 {acc}, {bset(J, t)}, {aslot(J)}, {acc}")
     jump(J + 1)
-    emit(f".org Lb0_%= + {(k + 1) * BLOCK_BYTES}")
+    emit(f".org Lb0_%= + {(k + 1) * block_bytes()}")
 
 
 def trampoline(m, k):
-    emit(f"s_movk_i32 s{S_RET}, {k * BLOCK_BYTES}")
+    emit(f"s_movk_i32 s{S_RET}, {k * block_bytes()}")
     emit(f"s_branch Lmark{m}_%=")
-    emit(f".org Lb0_%= + {TRAMP_BASE + (m * N_BLOCKS + k + 1) * TRAMP_BYTES}")
+    emit(f".org Lb0_%= + {tramp_base() + (m * N_BLOCKS + k + 1) * TRAMP_BYTES}")
 
 
 def boundary_code():
@@ -175,16 +206,26 @@ def boundary_code():
     emit(f"s_cmp_ge_u32 s{S_T0}, %[n_chunks]")
     emit("s_cbranch_scc1 Lmn_%=")
     # copies of chunk cur + 2 into stage (cur + 2) % 4: rows of B from k = 256 * id (the id was loaded by the previous boundary)
-    emit(f"s_lshl_b32 s{S_T1}, s{S_NEXTK}, 9")
-    emit(f"v_add_u32 v{V_COPY}, s{S_T1}, %[copy_off]")
-    emit(f"v_min_u32 v{V_COPY}, v{V_COPY}, %[copy_lim]")
+    if ROW_MAJOR:
+        emit(f"s_mul_i32 s{S_T1}, s{S_NEXTK}, %[chunk_bytes]")
+        emit(f"v_add_u32 v{V_T0}, s{S_T1}, %[copy_off]")
+        emit(f"v_add_u32 v{V_T1}, s{S_T1}, %[copy_off1]")
+    else:
+        emit(f"s_lshl_b32 s{S_T1}, s{S_NEXTK}, 9")
+        emit(f"v_add_u32 v{V_COPY}, s{S_T1}, %[copy_off]")
+        emit(f"v_min_u32 v{V_COPY}, v{V_COPY}, %[copy_lim]")
     emit(f"s_and_b32 s{S_T0}, s{S_T0}, 3")
     emit(f"s_lshl_b32 s{S_T0}, s{S_T0}, 15")
     emit(f"s_add_u32 s{S_T0}, s{S_T0}, %[dst_wave]")
     for it in range(COPIES):
         emit(f"s_add_u32 m0, s{S_T0}, {1024 * it}")
-        emit("s_nop 0")
-        emit(f"global_load_lds_dwordx4 v{V_COPY}, %[sb{it}]")
+        if ROW_MAJOR:  # eight rows of B each
+            emit(f"v_min_u32 v{V_COPY}, v{V_T0 + it % 2}, %[copy_lim{'1' if it % 2 else ''}]")
+            emit(f"v_add_u32 v{V_T0 + it % 2}, %[rows16_bytes], v{V_T0 + it % 2}")
+            emit(f"global_load_lds_dwordx4 v{V_COPY}, %[sb0]")
+        else:
+            emit("s_nop 0")
+            emit(f"global_load_lds_dwordx4 v{V_COPY}, %[sb{it}]")
     label("Lmn")
     emit(f"s_load_dword s{S_NEXTK}, s[{S_CP}:{S_CP + 1}], 0x0")   # id of chunk cur + 3, for the next boundary
     emit(f"s_add_u32 s{S_CP}, s{S_CP}, 4")
@@ -192,63 +233,73 @@ def boundary_code():
     emit(f"s_add_u32 s{S_JMP}, s{S_BASE}, s{S_RET}")             # on to the block of the op that opens the chunk
     emit(f"s_addc_u32 s{S_JMP + 1}, s{S_BASE + 1}, 0")
     emit(f"s_setpc_b64 s[{S_JMP}:{S_JMP + 1}]")
-    emit(f".org Lb0_%= + {MARK_OFF + MARK_BYTES}")
+    emit(f".org Lb0_%= + {mark_off() + MARK_BYTES}")
 
 
-# ---- entry: A operands of ops 0 .. AHEAD - 1 (their offsets stand in front of the stream), descriptors of ops 0 .. 7, B
-# operands of op 0.  The touches ask for a part of A that other workgroups, or this one later, will want: nobody waits for
-# them but the operands asked for after them. ----
-emit(f"s_mov_b32 s{S_DP}, %[op_lo]")
-emit(f"s_mov_b32 s{S_DP + 1}, %[op_hi]")
-emit(f"s_load_dwordx8 s[{S_HEAD}:{S_HEAD + 7}], s[{S_DP}:{S_DP + 1}], 0x0")
-emit(f"s_load_dwordx16 s[{S_RING0}:{S_RING0 + 15}], s[{S_DP}:{S_DP + 1}], 0x20")
-emit(f"s_load_dwordx16 s[{S_RING0 + 16}:{S_RING0 + 31}], s[{S_DP}:{S_DP + 1}], 0x60")
-emit(f"s_add_u32 s{S_DP}, s{S_DP}, {32 + 128}")
-emit(f"s_addc_u32 s{S_DP + 1}, s{S_DP + 1}, 0")
-emit(f"s_mov_b32 s{S_CP}, %[chunk_lo]")
-emit(f"s_mov_b32 s{S_CP + 1}, %[chunk_hi]")
-emit(f"s_load_dword s{S_NEXTK}, s[{S_CP}:{S_CP + 1}], 0xc")      # id of chunk 3, for the first marker
-emit(f"s_add_u32 s{S_CP}, s{S_CP}, 16")
-emit(f"s_addc_u32 s{S_CP + 1}, s{S_CP + 1}, 0")
-emit(f"s_mov_b32 s{S_CUR}, 0")
-emit("s_waitcnt lgkmcnt(0)")
-for k in range(AHEAD):
-    a_load(k, f"s{S_HEAD + k}")
-for t in range(TOUCHES):
-    emit(f"buffer_load_dword v{V_TOUCH}, %[touch{t}], %[rsrc], 0 offen")
-emit(f"s_waitcnt vmcnt({AHEAD + TOUCHES})")  # the copies of chunks 0, 1, 2 (issued before these loads) have landed
-emit("s_barrier")
-b_reads(0, 0)
-emit(f"s_getpc_b64 s[{S_BASE}:{S_BASE + 1}]")
-label("Lpc")
-emit(f"s_add_u32 s{S_BASE}, s{S_BASE}, Lb0_%=-Lpc_%=")
-emit(f"s_addc_u32 s{S_BASE + 1}, s{S_BASE + 1}, 0")
-jump(0)
-emit(".p2align 7")
-for J in range(8):
-    for r in range(8):
-        for v in range(2):
-            op_block(J, r, v)
-for m in range(MARKS):
-    for k in range(N_BLOCKS):
-        trampoline(m, k)
-boundary_code()
-label("Lend")                                         # offset END_OFF: the descriptor after the last op jumps here
-emit("s_waitcnt vmcnt(0) lgkmcnt(0)")
+def loop():
+    # ---- entry: A operands of ops 0 .. AHEAD - 1 (their offsets stand in front of the stream), descriptors of ops 0 .. 7, B
+    # operands of op 0.  The touches ask for a part of A that other workgroups, or this one later, will want: nobody waits for
+    # them but the operands asked for after them. ----
+    emit(f"s_mov_b32 s{S_DP}, %[op_lo]")
+    emit(f"s_mov_b32 s{S_DP + 1}, %[op_hi]")
+    emit(f"s_load_dwordx8 s[{S_HEAD}:{S_HEAD + 7}], s[{S_DP}:{S_DP + 1}], 0x0")
+    emit(f"s_load_dwordx16 s[{S_RING0}:{S_RING0 + 15}], s[{S_DP}:{S_DP + 1}], 0x20")
+    emit(f"s_load_dwordx16 s[{S_RING0 + 16}:{S_RING0 + 31}], s[{S_DP}:{S_DP + 1}], 0x60")
+    emit(f"s_add_u32 s{S_DP}, s{S_DP}, {32 + 128}")
+    emit(f"s_addc_u32 s{S_DP + 1}, s{S_DP + 1}, 0")
+    emit(f"s_mov_b32 s{S_CP}, %[chunk_lo]")
+    emit(f"s_mov_b32 s{S_CP + 1}, %[chunk_hi]")
+    emit(f"s_load_dword s{S_NEXTK}, s[{S_CP}:{S_CP + 1}], 0xc")      # id of chunk 3, for the first marker
+    emit(f"s_add_u32 s{S_CP}, s{S_CP}, 16")
+    emit(f"s_addc_u32 s{S_CP + 1}, s{S_CP + 1}, 0")
+    emit(f"s_mov_b32 s{S_CUR}, 0")
+    emit("s_waitcnt lgkmcnt(0)")
+    for k in range(AHEAD):
+        a_load(k, f"s{S_HEAD + k}")
+    for t in range(TOUCHES):
+        emit(f"buffer_load_dword v{V_TOUCH}, %[touch{t}], %[rsrc], 0 offen")
+    emit(f"s_waitcnt vmcnt({AHEAD + TOUCHES})")  # the copies of chunks 0, 1, 2 (issued before these loads) have landed
+    emit("s_barrier")
+    b_reads(0, 0)
+    emit(f"s_getpc_b64 s[{S_BASE}:{S_BASE + 1}]")
+    label("Lpc")
+    emit(f"s_add_u32 s{S_BASE}, s{S_BASE}, Lb0_%=-Lpc_%=")
+    emit(f"s_addc_u32 s{S_BASE + 1}, s{S_BASE + 1}, 0")
+    jump(0)
+    emit(".p2align 7")
+    for J in range(8):
+        for r in range(8):
+            for v in range(2):
+                op_block(J, r, v)
+    for m in range(MARKS):
+        for k in range(N_BLOCKS):
+            trampoline(m, k)
+    boundary_code()
+    label("Lend")                                         # offset END_OFF: the descriptor after the last op jumps here
+    emit("s_waitcnt vmcnt(0) lgkmcnt(0)")
+
 
 clob = ([f'"v{i}"' for i in range(V_B0, V_TOUCH + 1)] + [f'"s{i}"' for i in range(S_RING0, S_LAST + 1)] +
         [f'"a{i}"' for i in range(128)] + ['"vcc"', '"scc"', '"memory"'])
 print("// generated by gen_sweep_loop.py; do not edit")
-print(f"static_assert(SWEEP_DEV_AHEAD == {AHEAD} && SWEEP_MIN_OPS == {MIN_OPS} && SWEEP_DEV_MARKS == {MARKS} && SWEEP_BLOCK_BYTES == {BLOCK_BYTES} && "
-      f"SWEEP_DEV_TRAMP_BASE == {TRAMP_BASE} && SWEEP_TRAMP_BYTES == {TRAMP_BYTES} && SWEEP_DEV_MARK_OFF == {MARK_OFF} && SWEEP_DEV_END_OFF == {END_OFF}, "
-      f"\"regenerate spmm_sweep_loop.inc\");")
-print("asm volatile(")
-for line in out:
-    end = "\\n" if line.endswith(":") else "\\n\\t"
-    print(f'    "{line}{end}"')
-print("    :")
-print('    : [sel01] "v"(sel01), [lane_xor] "v"(lane_xor), [rd_lane] "v"(rd_addr), [a_voff] "v"(a_voff), [rsrc] "s"(vals_rsrc), [touch0] "v"(touch[0]), [touch1] "v"(touch[1]),')
-print('      [copy_off] "v"(copy_off), [copy_lim] "v"(copy_lim), [dst_wave] "s"(dst_wave), [n_chunks] "s"(n_chunks_u),')
-print('      [sb0] "s"(sb0), [sb1] "s"(sb1), [sb2] "s"(sb2), [sb3] "s"(sb3),')
-print('      [op_lo] "s"(op_lo), [op_hi] "s"(op_hi), [chunk_lo] "s"(chunk_lo), [chunk_hi] "s"(chunk_hi)')
-print("    : " + ", ".join(clob) + ");")
+print(f"static_assert(SWEEP_DEV_AHEAD == {AHEAD} && SWEEP_MIN_OPS == {MIN_OPS} && SWEEP_DEV_MARKS == {MARKS} && SWEEP_N_BLOCKS == {N_BLOCKS} && "
+      f"SWEEP_TRAMP_BYTES == {TRAMP_BYTES} && SWEEP_MARK_BYTES == {MARK_BYTES}, \"regenerate spmm_sweep_loop.inc\");")
+for ROW_MAJOR in (True, False):
+    out.clear()
+    loop()
+    b = "true" if ROW_MAJOR else "false"
+    print("#ifdef SMAT_SWEEP_ROW_MAJOR" if ROW_MAJOR else "#else")
+    print(f"static_assert(sweep_block_bytes({b}) == {block_bytes()} && sweep_tramp_base({b}) == {tramp_base()} && sweep_end_off({b}) == {mark_off() + MARK_BYTES}, "
+          f"\"regenerate spmm_sweep_loop.inc\");")
+    print("asm volatile(")
+    for line in out:
+        end = "\\n" if line.endswith(":") else "\\n\\t"
+        print(f'    "{line}{end}"')
+    print("    :")
+    print('    : [sel01] "v"(sel01), [rd_lane] "v"(rd_addr), [a_voff] "v"(a_voff), [rsrc] "s"(vals_rsrc), [touch0] "v"(touch[0]), [touch1] "v"(touch[1]),')
+    print('      [copy_off] "v"(copy_off), [copy_lim] "v"(copy_lim), [dst_wave] "s"(dst_wave), [n_chunks] "s"(n_chunks_u),')
+    print('      [sb0] "s"(sb0), [chunk_bytes] "s"(chunk_bytes), [rows16_bytes] "s"(rows16_bytes), [copy_off1] "v"(copy_off1), [copy_lim1] "v"(copy_lim1),' if ROW_MAJOR else
+          '      [lane_xor] "v"(lane_xor), [sb0] "s"(sb0), [sb1] "s"(sb1), [sb2] "s"(sb2), [sb3] "s"(sb3),')
+    print('      [op_lo] "s"(op_lo), [op_hi] "s"(op_hi), [chunk_lo] "s"(chunk_lo), [chunk_hi] "s"(chunk_hi)')
+    print("    : " + ", ".join(clob) + ");")
+print("#endif")

@@ -76,6 +76,7 @@ struct SweepArgs {
     void *C;
     size_t M, N, K, nnzb;
     bool c_f32;
+    bool b_row_major;            // B[k*N + n]; ops are the streams for it
     const int32_t *rg_chunk_ptr; // device, n_rg + 1: range of the row group in chunk_ids
     const int32_t *chunk_ids;    // device: the K chunks in which the row group has blocks, ascending (+ SWEEP_CHUNK_PAD entries)
     const int32_t *op_ptr;       // device, n_rg * SWEEP_WAVES + 1: range of (row group, wavefront) in ops
@@ -165,6 +166,13 @@ enum class RowLengths { EVEN, SPLIT, UNKNOWN };
 int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, RowLengths lengths, bool packed);
 bool rowwise_shares_items(size_t N, size_t n_items, size_t avg_blocks);
 hipError_t launch_sweep(const SweepArgs &a, hipStream_t st);
+// Whether the sweep kernel reads a row-major B of this size in place; otherwise B is brought into column-major order first, one
+// read and one write of it.  In place a row group reads 128 bytes of every row of B where it reads 512 of every column of the
+// other order, which costs it more the more row groups there are and the less of B the caches hold, twice as much where the
+// pieces straddle cache lines.  Of 39 products the rule takes the slower way in four, by 1 to 6 %; in place / column-major
+// first, us: 8192^2, 10 %, N = 4096 105 / 119, N = 2048 46 / 72; 4096^2, N = 4088 30 / 50; 12288 x 8192, 8 %, N = 4096 132 / 145;
+// 16384 rows, 16 row groups: K = 8192, N = 2048 96 / 101, N = 3072 153 / 140; K = 16384, N = 2040 185 / 155.
+bool sweep_takes_row_major(size_t N, size_t K, int n_rg);
 hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st);
 
 } // namespace smat

@@ -102,7 +102,14 @@ __device__ __forceinline__ f32x4 read_acc()
 
 } // namespace
 
-template <bool C_F32>
+// B_ROW: B is row-major.  A stage is then [16 slabs][16 k][64 columns] as it lies in B, 128 bytes a row, 16-byte piece p of row k
+// at place p ^ s(k), s(k) = bit 1 of k + 2 * bit 3 of k.  In a transposing read of tile t lane (i16, g) takes 8 bytes of row
+// 8 (g & 1) + i16 / 4 (and, in a second one, of 4 rows on): with c = i16 % 4 the columns 16 c + 4 (t ^ (c & 1)) .. + 3, half
+// (t ^ c) & 1 of piece 2c + t / 2.  So 32 lanes read one half of four pieces in each of eight rows, 32 places in different
+// banks (with the columns 16 c + 4t, the halves all alike, every read took twice as long: 8192^2, 10 %, N = 4032 101 against
+// 94 us).  Everything else, the order of the sums included, is the same; the lanes of odd g find the tiles t and t ^ 1 swapped
+// in the end.
+template <bool C_F32, bool B_ROW>
 __global__ __launch_bounds__(THREADS) void spmm_sweep_kernel(
     const uint16_t *__restrict__ vals, const uint16_t *__restrict__ B, void *__restrict__ Cout,
     const int32_t *__restrict__ rg_chunk_ptr, const int32_t *__restrict__ chunk_ids,
@@ -131,8 +138,13 @@ __global__ __launch_bounds__(THREADS) void spmm_sweep_kernel(
     gb = gb < n_blk - 1 ? gb : n_blk - 1;
     const int rem = tile - gb * RGB * n_panels;
     const int rgs_here = n_rg - gb * RGB < RGB ? n_rg - gb * RGB : RGB;
-    const int panel = rem / rgs_here;
-    const int rg = gb * RGB + rem - panel * rgs_here;
+    const int pos = rem / rgs_here;
+    const int rg = gb * RGB + rem - pos * rgs_here;
+    // Row-major B: the panels that an XCD has at a time are every other one of 16.  What the device reads at a time is then 128
+    // of every 256 bytes of the rows and comes from all memory channels; neighbouring panels would leave out a half of them
+    // where the rows are a power of two apart (8192^2, 10 %, N = 4096: 113 -> 103 us, with N = 4032 102 either way).
+    int panel = pos;
+    if (B_ROW && N % 64 == 0 && (pos | 15) < n_panels) panel = (pos & ~15) | (pos & 7) << 1 | ((pos >> 3) & 1);
     const int n0 = panel * NT;
 
     const int i16 = lane & 15, g = lane >> 4, sel = g >> 1, kh = g & 1;
@@ -169,31 +181,58 @@ __global__ __launch_bounds__(THREADS) void spmm_sweep_kernel(
                          : "v"(voff), "s"(sbase), "s"(dst)
                          : "memory");
         };
-        // ---- B panel copies: this wavefront fills rows ((wave & 3) * 4 + it) * 4 .. + 3 of slab group wave / 4 ----
-        // lane -> (row q = lane / 16, physical slot ps = lane % 16); logical slot = ps ^ swizzle(n),
-        // swizzle(n) = (n & 3) | ((n >> 2) & 12) = q | (wave & 3) << 2 for these rows.
-        const int q = lane >> 4;
-        const uint32_t ls = (uint32_t)((lane & 15) ^ (q | ((wave & 3) << 2)));
-        const uint32_t k_lane = (uint32_t)(wave >> 2) * 128u + ls * 8u;  // k inside the chunk
-        const uint32_t col_bytes = (uint32_t)q * (uint32_t)K * 2u;       // the launcher checks K < 2^28
-        const uint32_t copy_off = col_bytes + k_lane * 2u;               // byte offset of this lane's 16 bytes for chunk id 0
-        const uint32_t copy_lim = col_bytes + ((uint32_t)K - 8u) * 2u;   // slabs past K are referenced by no op: the read stays inside the matrix
         const uint32_t dst_wave = lbase + (uint32_t)(wave * COPIES) * 1024u;
-        // the four copy instructions of a chunk: scalar base = first of their four columns of B.  Columns past N
-        // (last panel, N % 8 == 0) are replaced by the last four: what lands in their rows is never stored, and
-        // every wavefront issues the same number of copies (the plan counts them).
-        const int col0 = n0 + (wave & 3) * 16;
-        auto col_base = [&](int c) { return B + (long)(c + 4 <= N ? c : N - 4) * K; };
-        const uint16_t *sb0 = col_base(col0), *sb1 = col_base(col0 + 4), *sb2 = col_base(col0 + 8), *sb3 = col_base(col0 + 12);
         const int32_t *chunk_ptr = chunk_ids + c_begin;
+        // column-major B: see below
+        uint32_t copy_off, copy_lim;
+        const uint16_t *sb0, *sb1, *sb2, *sb3;
+        // row-major B: rows 8 (COPIES * wave + it) .. + 7 of a chunk for copy it; lane -> (row lane / 8, physical piece lane % 8)
+        const uint32_t row_bytes = (uint32_t)N * 2u, rows8_bytes = 8u * row_bytes, rows16_bytes = 16u * row_bytes, chunk_bytes = (uint32_t)(S * 16) * row_bytes;
+        uint32_t copy_off1 = 0, copy_lim1 = 0; // of the copies of odd it, whose rows have bit 3 set
+        if constexpr (B_ROW) {
+            auto place = [&](int it, uint32_t &off, uint32_t &lim) {
+                const int piece = (lane & 7) ^ (((lane >> 4) & 1) | (it & 1) << 1);
+                const int col = n0 + 8 * piece < N ? n0 + 8 * piece : N - 8; // past N: never stored
+                off = (uint32_t)(wave * COPIES * 8 + (lane >> 3)) * row_bytes + (uint32_t)it * rows8_bytes + (uint32_t)col * 2u;
+                lim = ((uint32_t)K - 1u) * row_bytes + (uint32_t)col * 2u; // rows past K are referenced by no op: the read stays inside B
+            };
+            place(0, copy_off, copy_lim);
+            place(1, copy_off1, copy_lim1);
+            sb0 = sb1 = sb2 = sb3 = B;
+        } else {
+            // ---- B panel copies: this wavefront fills rows ((wave & 3) * 4 + it) * 4 .. + 3 of slab group wave / 4 ----
+            // lane -> (row q = lane / 16, physical slot ps = lane % 16); logical slot = ps ^ swizzle(n),
+            // swizzle(n) = (n & 3) | ((n >> 2) & 12) = q | (wave & 3) << 2 for these rows.
+            const int q = lane >> 4;
+            const uint32_t ls = (uint32_t)((lane & 15) ^ (q | ((wave & 3) << 2)));
+            const uint32_t k_lane = (uint32_t)(wave >> 2) * 128u + ls * 8u;  // k inside the chunk
+            const uint32_t col_bytes = (uint32_t)q * (uint32_t)K * 2u;       // the launcher checks K < 2^28
+            copy_off = col_bytes + k_lane * 2u;               // byte offset of this lane's 16 bytes for chunk id 0
+            copy_lim = col_bytes + ((uint32_t)K - 8u) * 2u;   // slabs past K are referenced by no op: the read stays inside the matrix
+            // the four copy instructions of a chunk: scalar base = first of their four columns of B.  Columns past N
+            // (last panel, N % 8 == 0) are replaced by the last four: what lands in their rows is never stored, and
+            // every wavefront issues the same number of copies (the plan counts them).
+            const int col0 = n0 + (wave & 3) * 16;
+            auto col_base = [&](int c) { return B + (long)(c + 4 <= N ? c : N - 4) * K; };
+            sb0 = col_base(col0); sb1 = col_base(col0 + 4); sb2 = col_base(col0 + 8); sb3 = col_base(col0 + 12);
+        }
         auto issue_copies = [&](int cl) { // chunk cl of the row group's list into stage cl % NS
-            uint32_t voff = (uint32_t)chunk_ptr[cl] * (uint32_t)(S * 16 * 2) + copy_off;
-            voff = voff < copy_lim ? voff : copy_lim;
             const uint32_t dst0 = dst_wave + (uint32_t)(cl % NS) * STAGE_BYTES;
-            lds_copy(voff, sb0, dst0);
-            lds_copy(voff, sb1, dst0 + 1024u);
-            lds_copy(voff, sb2, dst0 + 2048u);
-            lds_copy(voff, sb3, dst0 + 3072u);
+            if constexpr (B_ROW) {
+                const uint32_t base = (uint32_t)chunk_ptr[cl] * chunk_bytes;
+#pragma unroll
+                for (uint32_t it = 0; it < COPIES; it++) {
+                    const uint32_t at = base + (it & 1 ? copy_off1 : copy_off) + it / 2 * rows16_bytes, lim = it & 1 ? copy_lim1 : copy_lim;
+                    lds_copy(at < lim ? at : lim, sb0, dst0 + 1024u * it);
+                }
+            } else {
+                uint32_t voff = (uint32_t)chunk_ptr[cl] * (uint32_t)(S * 16 * 2) + copy_off;
+                voff = voff < copy_lim ? voff : copy_lim;
+                lds_copy(voff, sb0, dst0);
+                lds_copy(voff, sb1, dst0 + 1024u);
+                lds_copy(voff, sb2, dst0 + 2048u);
+                lds_copy(voff, sb3, dst0 + 3072u);
+            }
         };
         // ---- entry: chunks 0, 1, 2 on their way, the region of zeros written ----
         if (zeros_written) __syncthreads(); // a later tile of this workgroup: everybody has left the stages of the tile before
@@ -210,7 +249,10 @@ __global__ __launch_bounds__(THREADS) void spmm_sweep_kernel(
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
         // ---- the interpreter: see gen_sweep_loop.py ----
-        const uint32_t rd_addr = lbase + (uint32_t)(16 * (i16 >> 2) + (i16 & 3)) * ROW_BYTES; // LDS address of this lane's column in stage 0
+        // LDS address in stage 0 that this lane reads from.  Column-major B: its column.  Row-major B: tile 0, see above.
+        const int c4 = i16 & 3, row = 8 * kh + (i16 >> 2);
+        const uint32_t rd_addr = lbase + (B_ROW ? (uint32_t)(row * 128 + ((2 * c4) ^ (((row >> 1) & 1) | (row >> 3) << 1)) * 16 + (c4 & 1) * 8)
+                                                : (uint32_t)(16 * (i16 >> 2) + (i16 & 3)) * ROW_BYTES);
         const uint32_t a_voff = (uint32_t)sel * 512u + a_lane_bytes; // lanes 32-63 take the second block of the pair
         const uint32_t sel01 = (uint32_t)sel;
         const uint32_t n_chunks_u = __builtin_amdgcn_readfirstlane((uint32_t)n_chunks);
@@ -227,7 +269,13 @@ __global__ __launch_bounds__(THREADS) void spmm_sweep_kernel(
             const uint64_t at = line + t * ((uint64_t)gridDim.x * THREADS * 128u);
             touch[t] = vb == (int)blockIdx.x && at < touch_bytes ? (uint32_t)at : 0xffffffffu;
         }
+        if constexpr (B_ROW) {
+#define SMAT_SWEEP_ROW_MAJOR
 #include "spmm_sweep_loop.inc"
+#undef SMAT_SWEEP_ROW_MAJOR
+        } else {
+#include "spmm_sweep_loop.inc"
+        }
     }
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); // the last MFMAs retire before their results are read
 
@@ -238,7 +286,11 @@ __global__ __launch_bounds__(THREADS) void spmm_sweep_kernel(
         if (br < 0) return;
         const long m = (long)br * 16 + i16;
         const int nbase = n0 + 16 * g;
-        const f32x4 v0 = read_acc<R, 0>(), v1 = read_acc<R, 1>(), v2 = read_acc<R, 2>(), v3 = read_acc<R, 3>();
+        f32x4 v0 = read_acc<R, 0>(), v1 = read_acc<R, 1>(), v2 = read_acc<R, 2>(), v3 = read_acc<R, 3>();
+        if (B_ROW && (g & 1)) { // tiles t and t ^ 1
+            const f32x4 w0 = v0, w2 = v2;
+            v0 = v1; v1 = w0; v2 = v3; v3 = w2;
+        }
         if (C_F32) {
             float *crow = reinterpret_cast<float *>(Cout) + m * (long)N + nbase;
             if (nbase < N) { *reinterpret_cast<f32x4 *>(crow) = v0; *reinterpret_cast<f32x4 *>(crow + 4) = v1; }
@@ -275,17 +327,23 @@ __global__ __launch_bounds__(THREADS) void spmm_sweep_kernel(
   }
 }
 
+bool sweep_takes_row_major(size_t N, size_t K, int n_rg)
+{
+    if ((K + 256) * N * sizeof(uint16_t) >= ((size_t)1 << 32)) return false; // 32-bit offsets into B
+    const bool whole_lines = N % 64 == 0;
+    return n_rg <= (whole_lines ? 12 : 8) || K * N * sizeof(uint16_t) <= (size_t)(whole_lines ? 40 : 24) << 20;
+}
+
 hipError_t launch_sweep(const SweepArgs &a, hipStream_t st)
 {
     const int lds_bytes = NS * STAGE_BYTES + ZERO_BYTES;
     // dynamic LDS above 64 KiB has to be allowed once per kernel and device; the call is cheap and idempotent
-    hipError_t e = a.c_f32
-        ? hipFuncSetAttribute(reinterpret_cast<const void *>(&spmm_sweep_kernel<true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes)
-        : hipFuncSetAttribute(reinterpret_cast<const void *>(&spmm_sweep_kernel<false>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    const auto kernel = a.b_row_major ? (a.c_f32 ? spmm_sweep_kernel<true, true> : spmm_sweep_kernel<false, true>)
+                                      : (a.c_f32 ? spmm_sweep_kernel<true, false> : spmm_sweep_kernel<false, false>);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (e != hipSuccess) return e;
     if (a.K >= ((size_t)1 << 28)) return hipErrorInvalidValue; // copy offsets: (3 * K + k) * 2 in 32 bits
+    if (a.b_row_major && (!a.ops || !sweep_takes_row_major(a.N, a.K, a.n_rg))) return hipErrorInvalidValue;
     const int n_panels = (int)((a.N + NT - 1) / NT);
     long wgs = (long)a.n_rg * n_panels;
     wgs = (wgs + 7) / 8 * 8;
@@ -310,14 +368,8 @@ hipError_t launch_sweep(const SweepArgs &a, hipStream_t st)
     const size_t vals_bytes = a.nnzb * 512, traffic = vals_bytes + a.K * a.N * 2 + a.M * a.N * (a.c_f32 ? 4 : 2);
     const uint32_t touch_bytes = traffic >= ((size_t)128 << 20) && vals_bytes <= (size_t)launched * THREADS * 128 * 2 ? (uint32_t)vals_bytes : 0;
     dim3 grid((unsigned)launched), block(THREADS);
-    if (a.c_f32)
-        hipLaunchKernelGGL((spmm_sweep_kernel<true>), grid, block, lds_bytes, st, a.vals, a.B, a.C,
-                           a.rg_chunk_ptr, a.chunk_ids, a.op_ptr, a.ops, a.row_map, (int)a.N, (long)a.K,
-                           a.n_rg, n_panels, (uint32_t)(a.nnzb * 512), touch_bytes, (int)wgs);
-    else
-        hipLaunchKernelGGL((spmm_sweep_kernel<false>), grid, block, lds_bytes, st, a.vals, a.B, a.C,
-                           a.rg_chunk_ptr, a.chunk_ids, a.op_ptr, a.ops, a.row_map, (int)a.N, (long)a.K,
-                           a.n_rg, n_panels, (uint32_t)(a.nnzb * 512), touch_bytes, (int)wgs);
+    hipLaunchKernelGGL(kernel, grid, block, lds_bytes, st, a.vals, a.B, a.C, a.rg_chunk_ptr, a.chunk_ids, a.op_ptr, a.ops, a.row_map, (int)a.N,
+                       (long)a.K, a.n_rg, n_panels, (uint32_t)vals_bytes, touch_bytes, (int)wgs);
     return hipGetLastError();
 }
 

@@ -377,11 +377,12 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
 }
 
 void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::vector<int32_t> &op_ptr, const SweepOpHost *ops,
-                          std::vector<SweepOpHost> &dev)
+                          bool b_row_major, std::vector<SweepOpHost> &dev)
 {
+    const uint32_t block_bytes = sweep_block_bytes(b_row_major), tramp_base = sweep_tramp_base(b_row_major);
     constexpr int DEV_AHEAD = SWEEP_DEV_AHEAD, HEAD = SWEEP_DEV_HEAD;
     const size_t n_streams = op_ptr.size() - 1;
-    dev.assign((size_t)op_ptr.back() + HEAD * n_streams + SWEEP_OP_PAD, SweepOpHost{0, SWEEP_ZERO_OFF, 0, SWEEP_DEV_END_OFF});
+    dev.assign((size_t)op_ptr.back() + HEAD * n_streams + SWEEP_OP_PAD, SweepOpHost{0, SWEEP_ZERO_OFF, 0, sweep_end_off(b_row_major)});
     std::vector<long> a_issue;
     for (size_t s = 0; s < n_streams; s++) {
         const SweepOpHost *op = ops + op_ptr[s];
@@ -412,9 +413,10 @@ void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::v
             const uint32_t v = seq - a_issue[i] > DEV_AHEAD ? 1u : 0u;
             const uint32_t code = (block & ~1u) | v;
             out[i].w0 = a_offset(i + DEV_AHEAD - 1);
-            out[i].w1 = op[i].w1;
-            out[i].w2 = op[i].w2;
-            out[i].w3 = opens ? SWEEP_DEV_TRAMP_BASE + (m * SWEEP_N_BLOCKS + code) * SWEEP_TRAMP_BYTES : code * SWEEP_BLOCK_BYTES;
+            const uint32_t lo = op[i].w1, hi = op[i].w1 + op[i].w2;
+            out[i].w1 = b_row_major ? sweep_lds_offset_row_major(lo) : lo;
+            out[i].w2 = (b_row_major ? sweep_lds_offset_row_major(hi) : hi) - out[i].w1;
+            out[i].w3 = opens ? tramp_base + (m * SWEEP_N_BLOCKS + code) * SWEEP_TRAMP_BYTES : code * block_bytes;
         }
         // the end stays what dev was filled with
     }
@@ -424,12 +426,12 @@ void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::v
 
 // Test hook (not part of smat.h): the streams of a plan that smat_internal_sweep_plan handed out as the kernel runs them, in
 // out[0 .. op_ptr[8 n_rg] + 2 * 8 n_rg + 16).
-extern "C" int smat_internal_sweep_encode(const int32_t *rg_chunk_ptr, int64_t n_rg, const int32_t *op_ptr, const uint32_t *ops, uint32_t *out)
+extern "C" int smat_internal_sweep_encode(const int32_t *rg_chunk_ptr, int64_t n_rg, const int32_t *op_ptr, const uint32_t *ops, int b_row_major, uint32_t *out)
 {
     return smat::guarded("smat_internal_sweep_encode", [&] {
         const std::vector<int32_t> chunk_ptr(rg_chunk_ptr, rg_chunk_ptr + n_rg + 1), ptr(op_ptr, op_ptr + n_rg * smat::SWEEP_WAVES + 1);
         std::vector<smat::SweepOpHost> dev;
-        smat::encode_sweep_streams(chunk_ptr, ptr, reinterpret_cast<const smat::SweepOpHost *>(ops), dev);
+        smat::encode_sweep_streams(chunk_ptr, ptr, reinterpret_cast<const smat::SweepOpHost *>(ops), b_row_major != 0, dev);
         memcpy(out, dev.data(), dev.size() * sizeof(smat::SweepOpHost));
         return (int)SMAT_OK;
     });

@@ -34,6 +34,6 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
 // The plan's streams as the kernel runs them (second part of sweep_format.h): stream s from dev[op_ptr[s] + SWEEP_DEV_HEAD * s] on,
 // and SWEEP_OP_PAD entries after the last.
 void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::vector<int32_t> &op_ptr, const SweepOpHost *ops,
-                          std::vector<SweepOpHost> &dev);
+                          bool b_row_major, std::vector<SweepOpHost> &dev);
 
 } // namespace smat

@@ -11,22 +11,29 @@ from smat_amd._lib import lib
 from tests.test_sweep_plan import BLOCK_BYTES, COPIES, END_OFF, MARK_OFF, MIN_OPS, N_BLOCKS, PAD, TRAMP_BASE, TRAMP_BYTES, WAVES, ZERO_OFF, random_mask_matrix, sweep_plan
 
 AHEAD, HEAD, MARKS, TOUCHES = 7, 2, 4, 2
-DEV_MARK_OFF = TRAMP_BASE + MARKS * N_BLOCKS * TRAMP_BYTES
-DEV_END_OFF = DEV_MARK_OFF + 512
 
 
-def encode(plan):
+def encode(plan, row_major):
     fn = lib.smat_internal_sweep_encode
     fn.restype = C.c_int
-    fn.argtypes = [C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]
+    fn.argtypes = [C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]
     n_rg = plan["rg_chunk_ptr"].size - 1
     out = np.zeros((plan["n_entries"] + HEAD * WAVES * n_rg + PAD, 4), np.uint32)
-    assert fn(plan["rg_chunk_ptr"].ctypes.data, n_rg, plan["op_ptr"].ctypes.data, plan["ops"].ctypes.data, out.ctypes.data) == 0
+    assert fn(plan["rg_chunk_ptr"].ctypes.data, n_rg, plan["op_ptr"].ctypes.data, plan["ops"].ctypes.data, row_major, out.ctypes.data) == 0
     return out
 
 
-def check(plan):
-    dev = encode(plan)
+def lds_offset(off, row_major):
+    """of a block in a stage of [8-slab group][column][slot] -> in one of [slab][k][column]; the region of zeros stays"""
+    return np.where(off == ZERO_OFF, off, (off // 16384 * 8 + off % 16384 // 32) * 2048) if row_major else off
+
+
+def check(plan, row_major):
+    dev = encode(plan, row_major)
+    block_bytes = 192 if row_major else BLOCK_BYTES
+    tramp_base = N_BLOCKS * block_bytes
+    mark_off = tramp_base + MARKS * N_BLOCKS * TRAMP_BYTES
+    end_off = mark_off + 512
     seen = set()
     for s in range(plan["op_ptr"].size - 1):
         a, b = plan["op_ptr"][s], plan["op_ptr"][s + 1]
@@ -36,10 +43,13 @@ def check(plan):
         if a == b:
             continue
         n = ops.shape[0] - 1
-        assert ops[n, 3] == END_OFF and tuple(out[n]) == (0, ZERO_OFF, 0, DEV_END_OFF)
+        assert ops[n, 3] == END_OFF and tuple(out[n]) == (0, ZERO_OFF, 0, end_off)
         a_of = np.concatenate([ops[:n, 0], np.zeros(AHEAD, np.int64)])
         assert np.array_equal(head[:AHEAD], a_of[:AHEAD]) and not head[AHEAD:].any()
-        assert np.array_equal(out[:n, 0], a_of[AHEAD - 1:AHEAD - 1 + n]) and np.array_equal(out[:n, 1:3], ops[:n, 1:3])
+        assert np.array_equal(out[:n, 0], a_of[AHEAD - 1:AHEAD - 1 + n])
+        delta = ops[:n, 2].astype(np.uint32).view(np.int32), out[:n, 2].astype(np.uint32).view(np.int32)
+        assert np.array_equal(out[:n, 1], lds_offset(ops[:n, 1], row_major))
+        assert np.array_equal(out[:n, 1] + delta[1], lds_offset(ops[:n, 1] + delta[0], row_major))
         n_chunks = int(plan["rg_chunk_ptr"][s // WAVES + 1] - plan["rg_chunk_ptr"][s // WAVES])
         # issue order: copies of chunks 0..2, the first A operands, the touches, then per position [copies of a boundary], A
         issued = [("copy", c) for c in range(min(3, n_chunks)) for _ in range(COPIES)]
@@ -51,8 +61,8 @@ def check(plan):
         for i in range(n):
             w3, plan_w3 = int(out[i, 3]), int(ops[i, 3])
             if plan_w3 >= TRAMP_BASE:
-                m, k = divmod((w3 - TRAMP_BASE) // TRAMP_BYTES, N_BLOCKS)
-                assert TRAMP_BASE <= w3 < DEV_MARK_OFF and (w3 - TRAMP_BASE) % TRAMP_BYTES == 0
+                m, k = divmod((w3 - tramp_base) // TRAMP_BYTES, N_BLOCKS)
+                assert tramp_base <= w3 < mark_off and (w3 - tramp_base) % TRAMP_BYTES == 0
                 plan_k = (plan_w3 - TRAMP_BASE) // TRAMP_BYTES
                 assert landed(("copy", cur + 2), MIN_OPS + m) or cur + 2 >= n_chunks
                 cur += 1
@@ -60,26 +70,27 @@ def check(plan):
                     issued += [("copy", cur + 2)] * COPIES
                 seen.add(("mark", m))
             else:
-                assert w3 < TRAMP_BASE and w3 % BLOCK_BYTES == 0
-                k, plan_k = w3 // BLOCK_BYTES, plan_w3 // BLOCK_BYTES
+                assert w3 < tramp_base and w3 % block_bytes == 0
+                k, plan_k = w3 // block_bytes, plan_w3 // BLOCK_BYTES
             assert k // 2 == plan_k // 2  # stream position and block row
             issued.append(("a", i + AHEAD))
             assert landed(("a", i), AHEAD + COPIES * (k % 2))
             seen.add(("op", k % 2))
         assert cur == n_chunks - 1
     tail = dev[dev.shape[0] - PAD:]
-    assert np.all(tail == np.array([0, ZERO_OFF, 0, DEV_END_OFF], np.uint32))
+    assert np.all(tail == np.array([0, ZERO_OFF, 0, end_off], np.uint32))
     return seen
 
 
+@pytest.mark.parametrize("row_major", [0, 1])
 @pytest.mark.parametrize("mb,kb,density,seed,group_rows", [(64, 64, 0.10, 1, 64), (70, 40, 0.30, 2, 64), (16, 300, 0.03, 3, 16), (50, 20, 0.02, 4, 32),
                                                            (64, 16, 0.5, 5, 64), (3, 2, 1.0, 6, 16), (130, 33, 0.0005, 7, 64)])
-def test_waits_of_the_device_streams(mb, kb, density, seed, group_rows):
+def test_waits_of_the_device_streams(mb, kb, density, seed, group_rows, row_major):
     A = random_mask_matrix(mb, kb, density, seed)
-    check(sweep_plan(A["b_row_ptr"], A["b_col_idx"], A["M"], A["K"], group_rows=group_rows))
+    check(sweep_plan(A["b_row_ptr"], A["b_col_idx"], A["M"], A["K"], group_rows=group_rows), row_major)
 
 
 def test_device_streams_use_every_wait():
     A = gen.block_pruned(4096, 0.10, 0.02)
     plan = sweep_plan(A["b_row_ptr"], A["b_col_idx"], A["M"], A["K"])
-    assert check(plan) == {("op", 0), ("op", 1)} | {("mark", m) for m in range(MARKS)}
+    assert check(plan, 0) == {("op", 0), ("op", 1)} | {("mark", m) for m in range(MARKS)}
