@@ -129,6 +129,9 @@ extern "C" void smat_internal_fail_alloc(int64_t n) { g_dev_fail_in.store(n); }
 // Test hook (not part of smat.h): block rows that the compact kernel's list of this plan splits, -1 without a list.
 extern "C" int smat_internal_compact_split_rows(const smat_plan *p) { return p->compact ? p->compact->n_split_rows : -1; }
 
+// Test hook (not part of smat.h): rows of B that the compact kernel's copy holds, 0 where it holds all or there is no list.
+extern "C" int64_t smat_internal_compact_placed_rows(const smat_plan *p) { return p->compact ? p->compact->n_placed : 0; }
+
 extern "C" const char *smat_version(void) { return "smat-amd 0.1 gfx950"; }
 
 static int check_shapes(const void *vals, const void *row_ptr, const void *col_idx, const void *B,
@@ -780,7 +783,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     std::vector<uint8_t> skip; // the blocks that the sweep kernel takes
     if (block_split) { // the list without them
         e = compact_full_blocks(census, skip);
-        if (e == hipSuccess) e = compact_build(census, vals, row_ptr, col_idx, p->K, p->n_cap, nullptr, true, &c);
+        if (e == hipSuccess) e = compact_build(census, vals, row_ptr, col_idx, p->K, p->n_cap, p->d_bcol != nullptr, nullptr, true, &c);
         if (e != hipSuccess) return fail(e);
         if (c->n_split_rows > 0) { // partial tiles through the workspace cannot be added to C: one kernel for everything
             block_split = false;
@@ -803,7 +806,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
         if (want == SMAT_KERNEL_AUTO && dense_kernel == SMAT_KERNEL_ROWWISE) e = sweep_small_groups(*p);
         return e == hipSuccess ? SMAT_OK : fail(e);
     }
-    if (!c) e = compact_build(census, vals, row_ptr, col_idx, p->K, p->n_cap, mixed ? &dense : nullptr, false, &c);
+    if (!c) e = compact_build(census, vals, row_ptr, col_idx, p->K, p->n_cap, p->d_bcol != nullptr, mixed ? &dense : nullptr, false, &c);
     if (e != hipSuccess) return fail(e);
     if (!p->d_bt) e = dev_malloc(&p->d_bt, p->bt_bytes());
     std::vector<int32_t> dense_list;

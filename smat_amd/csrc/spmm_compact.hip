@@ -57,6 +57,7 @@ int g_force_tq = 0; // test hook: 1 or 2 = panels of 64 or 128 columns whatever 
 constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts as full (of 16)
 constexpr int TASK_STEPS = 12;     // short items are put together up to this many steps (8 to 24: level; one item each: 9 % slower on R-MAT)
 constexpr int LONG_ROW_STEPS = 56; // steps from which a block row is split where a launch has few wavefronts
+constexpr size_t PLACE_MIN_BYTES = (size_t)16 << 20; // of B, from which the rows that its copy does not need are looked for
 constexpr int LIST_PAD = 2304; // entries readable past the end of the list (the index loads of the 64-column panel run up to 16 steps ahead)
 
 // ---- census of nonzero block columns ----
@@ -248,6 +249,22 @@ __global__ void row_steps_kernel(const int32_t *__restrict__ starts, const int32
     if (i < n) out[i] = first_step[starts[i] / 32];
 }
 
+// used[row] = 1 for the rows of B that the list names; padding names row 0.
+__global__ __launch_bounds__(256) void mark_rows_kernel(const int32_t *__restrict__ cols, long n, int32_t *__restrict__ used)
+{
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) used[cols[i]] = 1;
+}
+// place of a used row among the used ones, -1 for the others
+__global__ __launch_bounds__(256) void place_rows_kernel(const int32_t *__restrict__ used, const int32_t *__restrict__ before, long K, int32_t *__restrict__ place)
+{
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < K) place[k] = used[k] ? before[k] : -1;
+}
+__global__ __launch_bounds__(256) void place_cols_kernel(const int32_t *__restrict__ cols, const int32_t *__restrict__ place, long n, int32_t *__restrict__ out)
+{
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) out[i] = max(place[cols[i]], 0);
+}
+
 // raw[br] = what the blocks before block row br hold: columns in the lower, nonzeros in the upper half; raw[mb] = total
 __global__ void row_offsets_kernel(const int32_t *__restrict__ row_ptr, const unsigned long long *__restrict__ offset,
                                    const unsigned long long *__restrict__ count, long mb, long nnzb, unsigned long long *__restrict__ raw)
@@ -282,8 +299,9 @@ __global__ __launch_bounds__(256) void copy_blocks_kernel(const uint16_t *__rest
 // reads 8 n of one k back (two 8-byte LDS reads) and stores 16 bytes.
 // The output is split into panels of `panel` columns, each a K x panel row-major matrix of leading
 // dimension ld, one panel after the other (panel >= N and ld = N: plain row-major K x N).
+// place != NULL: row k goes to row place[k] of a copy of `rows` rows, or nowhere (-1).
 __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__restrict__ B, uint16_t *__restrict__ Bt,
-                                                          int N, long K, int panel, long ld)
+                                                          int N, long K, int panel, long ld, long rows, const int32_t *__restrict__ place)
 {
     constexpr int LD = 68; // halfs per LDS row (k): 8-byte aligned rows, dword writes spread over the banks
     __shared__ __align__(16) uint16_t tile[64 * LD];
@@ -309,10 +327,12 @@ __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__rest
 #pragma unroll
     for (int half = 0; half < 2; half++) {
         const int k = a + 32 * half;
-        if (k0 + k < K && n0 + seg * 8 < N) {
+        long row = k0 + k;
+        if (place && k0 + k < K) row = place[k0 + k];
+        if (k0 + k < K && n0 + seg * 8 < N && row >= 0) {
             const uint2 lo = *reinterpret_cast<const uint2 *>(tile + k * LD + seg * 8);
             const uint2 hi = *reinterpret_cast<const uint2 *>(tile + k * LD + seg * 8 + 4);
-            uint16_t *out = Bt + (long)(n0 / panel) * K * panel + (k0 + k) * ld + n0 % panel + seg * 8;
+            uint16_t *out = Bt + (long)(n0 / panel) * rows * panel + row * ld + n0 % panel + seg * 8;
             *reinterpret_cast<u32x4 *>(out) = (u32x4){lo.x, lo.y, hi.x, hi.y};
         }
     }
@@ -595,12 +615,15 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
     constexpr int PANEL = 64 * TQ;
     const int n_panels = (int)((a.N + PANEL - 1) / PANEL);
     long panel_stride = PANEL, row_stride = (long)a.N;
+    const int32_t *cols = p.d_cols;
     if (!a.b_row_major) {
+        const long rows = p.d_place ? (long)p.n_placed : (long)a.K; // of the copy
+        if (p.d_place) cols = p.d_cols_placed;
         dim3 grid((unsigned)((a.K + 63) / 64), (unsigned)((a.N + 63) / 64));
-        hipLaunchKernelGGL(transpose_b_kernel, grid, dim3(256), 0, st, a.B, a.Bt, (int)a.N, (long)a.K, PANEL, (long)PANEL);
+        hipLaunchKernelGGL(transpose_b_kernel, grid, dim3(256), 0, st, a.B, a.Bt, (int)a.N, (long)a.K, PANEL, (long)PANEL, rows, (const int32_t *)p.d_place);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        panel_stride = (long)a.K * PANEL;
+        panel_stride = rows * PANEL;
         row_stride = PANEL;
     }
     const long total = (long)p.n_tasks * n_panels;
@@ -619,7 +642,7 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
     const bool big = a.K > ((size_t)1 << 24) || a.K * (size_t)row_stride * 2 >= ((size_t)1 << 32) || row_stride >= (1L << 23);
     auto launch = [&](auto af, auto f32, auto acc, auto wide) {
         hipLaunchKernelGGL((spmm_compact_kernel<TQ, decltype(f32)::value, decltype(acc)::value, decltype(af)::value, decltype(wide)::value>),
-                           dim3((unsigned)wgs), dim3(256), 0, st, p.d_acol, p.d_entries, p.d_step_range, p.d_cols, a.Bt, a.C, p.d_workspace,
+                           dim3((unsigned)wgs), dim3(256), 0, st, p.d_acol, p.d_entries, p.d_step_range, cols, a.Bt, a.C, p.d_workspace,
                            p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, (unsigned)xcd_run);
     };
     using std::false_type;
@@ -649,7 +672,8 @@ using Scratch = DevScratch;
 hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, size_t N, size_t K, hipStream_t st)
 {
     dim3 grid((unsigned)((N + 63) / 64), (unsigned)((K + 63) / 64));
-    hipLaunchKernelGGL(transpose_b_kernel, grid, dim3(256), 0, st, B_row_major, out, (int)K, (long)N, 0x7fffffff, (long)K);
+    hipLaunchKernelGGL(transpose_b_kernel, grid, dim3(256), 0, st, B_row_major, out, (int)K, (long)N, 0x7fffffff, (long)K, (long)N,
+                       (const int32_t *)nullptr);
     return hipGetLastError();
 }
 
@@ -768,6 +792,8 @@ void compact_destroy(CompactPlan *p)
 {
     if (!p) return;
     if (p->d_cols) (void)dev_free(p->d_cols);
+    if (p->d_place) (void)dev_free(p->d_place);
+    if (p->d_cols_placed) (void)dev_free(p->d_cols_placed);
     if (p->d_acol) (void)dev_free(p->d_acol);
     if (p->d_entries) (void)dev_free(p->d_entries);
     if (p->d_step_range) (void)dev_free(p->d_step_range);
@@ -875,8 +901,44 @@ static bool lists_nonzeros(int64_t nnz, int64_t n_cols, size_t n_rows, size_t N)
     return 2 * nnz <= 3 * n_cols || (n_cols >= 500000 && nnz <= 4 * n_cols);
 }
 
+// The copy of B without the rows that no listed column names, where those are an eighth or more.  R-MAT scale 20, 16 a row: 48 % of
+// the columns are empty, and the rows of B under the others fill 67 of 128 MiB a panel, which the memory-side cache holds for
+// the gathers: N = 128 transposition 101 -> 94 us, product 469 -> 401; scale 18, N = 256 226 -> 211, both together; scale 16 equal.
+// With the rows that most columns meet in front the gathers take as long.  Not looked for below 16 MiB, where the
+// transposition is little more than a launch, nor where the plan is made for row-major B, which is read in place.
+static hipError_t place_rows(CompactPlan &p, size_t K, long total)
+{
+    hipError_t e = hipSuccess;
+    Scratch used, before, tmp;
+    size_t bytes = 0;
+    SMAT_STEP(used.alloc((K + 1) * sizeof(int32_t)));
+    SMAT_STEP(before.alloc((K + 1) * sizeof(int32_t)));
+    SMAT_STEP(hipMemsetAsync(used.p, 0, (K + 1) * sizeof(int32_t), nullptr));
+    const unsigned blocks = (unsigned)std::min<long>((total + 255) / 256, 256L * 8);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(mark_rows_kernel, dim3(blocks), dim3(256), 0, 0, (const int32_t *)p.d_cols, total, (int32_t *)used.p);
+        e = hipGetLastError();
+    }
+    SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, (int32_t *)used.p, (int32_t *)before.p, (int)(K + 1)));
+    SMAT_STEP(tmp.alloc(bytes));
+    SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, (int32_t *)used.p, (int32_t *)before.p, (int)(K + 1)));
+    int32_t n = 0;
+    SMAT_STEP(hipMemcpy(&n, (int32_t *)before.p + K, sizeof n, hipMemcpyDeviceToHost));
+    if (e != hipSuccess || (size_t)n > K / 8 * 7) return e;
+    const long padded = total + LIST_PAD;
+    SMAT_STEP(dev_malloc(&p.d_place, K * sizeof(int32_t)));
+    SMAT_STEP(dev_malloc(&p.d_cols_placed, (size_t)padded * sizeof(int32_t)));
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(place_rows_kernel, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, 0, (const int32_t *)used.p, (const int32_t *)before.p, (long)K, p.d_place);
+        hipLaunchKernelGGL(place_cols_kernel, dim3(blocks), dim3(256), 0, 0, (const int32_t *)p.d_cols, (const int32_t *)p.d_place, padded, p.d_cols_placed);
+        e = hipGetLastError();
+    }
+    p.n_placed = n;
+    return e;
+}
+
 hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx, size_t K, size_t n_cap,
-                         const std::vector<uint8_t> *leave_rows, bool drop_full, CompactPlan **out)
+                         bool b_row_major, const std::vector<uint8_t> *leave_rows, bool drop_full, CompactPlan **out)
 {
     *out = nullptr;
     const size_t mb = s.mb, nnzb = s.nnzb;
@@ -990,6 +1052,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
             }
         }
     }
+    if (e == hipSuccess && total > 0 && !b_row_major && K * n_cap * sizeof(uint16_t) >= PLACE_MIN_BYTES) e = place_rows(*p, K, (long)total);
     // Work items: whole block rows; rows much longer than the average in chunks of 32-column steps, all of a row's about
     // as long.  Long rows that are all alike stay whole: their partial tiles are 2 * 16 * N floats to write and read again
     // for each (32768 x 65536, 131 a row, N = 256: 138 us whole, 191 in chunks of 1792 columns; 8192 x 65536, 140 a row,

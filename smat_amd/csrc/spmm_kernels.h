@@ -94,6 +94,10 @@ hipError_t launch_reduce(const float *workspace, const SplitRow *split_rows, int
 // row are listed once (from the zero pattern of the values) and multiplied 32 at a time.
 struct CompactPlan {
     int32_t *d_cols = nullptr;   // row of B (absolute column of A) of every listed column; block rows padded to 32
+    // Where many rows of B meet no nonzero, the copy of a column-major B holds the others only: their places in it, -1 for a row
+    // that has none (K int32), how many there are, and the list that names places instead of rows.
+    int32_t *d_place = nullptr, *d_cols_placed = nullptr;
+    int64_t n_placed = 0;
     uint16_t *d_acol = nullptr;  // the 16 values of every listed column, in MFMA operand order (32 bytes per column), or
     uint32_t *d_entries = nullptr;  // their nonzeros: value << 16 | byte in the step's operand
     int2 *d_step_range = nullptr;   // entries [x, y) of every step of 32 listed columns
@@ -134,7 +138,7 @@ hipError_t compact_full_blocks(const CompactCensus &s, std::vector<uint8_t> &ful
 // them).  drop_full: full blocks get no listed columns (another kernel multiplies them); from then on the census is
 // that of the other blocks.
 hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx, size_t K, size_t n_cap,
-                         const std::vector<uint8_t> *leave_rows, bool drop_full, CompactPlan **out);
+                         bool b_row_major, const std::vector<uint8_t> *leave_rows, bool drop_full, CompactPlan **out);
 // out[j * 256 ..] = block ids_host[j] of vals (device to device, synchronous).
 hipError_t copy_blocks(const uint16_t *vals, const int32_t *ids_host, size_t n, uint16_t *out);
 void compact_destroy(CompactPlan *p);
