@@ -104,44 +104,60 @@ __device__ __forceinline__ unsigned long long checksum_term(uint32_t v, long i)
 // blocks with at least FULL_BLOCK_COLS nonzero columns, nonzero columns of the others, nonzeros.
 enum { SUM_CHECK, SUM_FULL, SUM_COLS_REST, SUM_NNZ, N_SUMS };
 
+// combined over the 16 lanes of a DPP row, in all of them
+__device__ __forceinline__ uint32_t row_or(uint32_t v)
+{
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false); // row_ror:8
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, false);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false);
+    return v;
+}
+__device__ __forceinline__ uint32_t row_sum(uint32_t v)
+{
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false);
+    return v;
+}
+
 // Per block: mask of its nonzero columns; their number in the lower half of count, the number of nonzeros in the upper.
+// Bound by the read of the values.  A lane holds one row of one half of a block, a DPP row of 16 lanes that half: its eight bits
+// are or-ed and counted in the VALU, where exchanging the values through LDS was most of the time (237 k blocks, 121 MB:
+// 40 -> 24 us).
 __global__ __launch_bounds__(256) void colmask_kernel(const uint16_t *__restrict__ vals, long nnzb,
                                                       uint16_t *__restrict__ mask, unsigned long long *__restrict__ count,
                                                       unsigned long long *__restrict__ sums)
 {
     unsigned long long total[N_SUMS] = {0, 0, 0, 0};
     const int lane = threadIdx.x & 63;
+    const int at = (lane & 15) * 16 + ((lane >> 4) & 1) * 8; // row lane % 16, half lane / 16 % 2: 8 values
     const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const long n_waves = ((long)gridDim.x * blockDim.x) >> 6;
-    for (long pb = wave * 2; pb < nnzb; pb += n_waves * 2) {
+    auto load = [&](long pb) {
         const long blk = pb + (lane >> 5);
-        // lane % 32 = row * 2 + half: 8 values of one row
-        u32x4 w = {0u, 0u, 0u, 0u};
-        if (blk < nnzb) w = *reinterpret_cast<const u32x4 *>(vals + blk * 256 + (lane & 31) * 8);
-        int nz = 0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            total[SUM_CHECK] += checksum_term(w[q], blk * 128 + (lane & 31) * 4 + q);
-            w[q] &= 0x7fff7fffu; // -0.0 is a zero
-            nz += ((w[q] & 0xffffu) != 0) + ((w[q] >> 16) != 0);
-        }
-#pragma unroll
-        for (int d = 1; d <= 16; d <<= 1) {
-            if (d >= 2) { // OR over the 16 rows (lane bits 1..4)
-                w[0] |= __shfl_xor(w[0], d);
-                w[1] |= __shfl_xor(w[1], d);
-                w[2] |= __shfl_xor(w[2], d);
-                w[3] |= __shfl_xor(w[3], d);
-            }
-            nz += __shfl_xor(nz, d);
-        }
+        return blk < nnzb ? *reinterpret_cast<const u32x4 *>(vals + blk * 256 + at) : (u32x4){0u, 0u, 0u, 0u};
+    };
+    u32x4 next = load(wave * 2);
+    for (long pb = wave * 2; pb < nnzb; pb += n_waves * 2) {
+        const u32x4 w = next;
+        next = load(pb + n_waves * 2);
+        const long blk = pb + (lane >> 5);
+        // the checksum of four dwords from dword i on: (2 i + 1) sum of w[q] + 2 sum of q w[q]
+        const unsigned long long plain = ((unsigned long long)w[0] + w[1]) + ((unsigned long long)w[2] + w[3]);
+        const unsigned long long weighted = (unsigned long long)w[1] + 2ull * w[2] + 3ull * w[3];
+        total[SUM_CHECK] += checksum_term(1, blk * 128 + at / 2) * plain + 2ull * weighted;
         uint32_t bits = 0;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            if (w[q] & 0xffffu) bits |= 1u << (2 * q);
-            if (w[q] >> 16) bits |= 1u << (2 * q + 1);
+        for (int q = 0; q < 4; q++) { // -0.0 is a zero
+            if (w[q] & 0x7fffu) bits |= 1u << (2 * q);
+            if (w[q] & 0x7fff0000u) bits |= 2u << (2 * q);
         }
-        const uint32_t other = __shfl_xor(bits, 1); // the other half of the row
+        const uint32_t nz_half = row_sum(__popc(bits));
+        bits = row_or(bits);
+        // lanes 0 and 32 put the halves of their blocks together
+        const uint32_t other = __shfl(bits, (lane & 32) | 16), nz = nz_half + __shfl(nz_half, (lane & 32) | 16);
         if ((lane & 31) == 0 && blk < nnzb) {
             const uint32_t m = bits | (other << 8);
             const int cols = __popc(m);
@@ -167,55 +183,86 @@ __global__ __launch_bounds__(256) void values_checksum_kernel(const u32x4 *__res
     add_totals<1>(total, sums);
 }
 
-// One thread per block: its nonzero columns go to positions padded_start[br] + (columns of the block row in the blocks
-// before it) .. of the padded list, and
+// The block row that block p belongs to, the largest br with row_ptr[br] <= p, by all lanes of a wavefront together (p the
+// same in all): every step looks at 64 rows.
+__device__ __forceinline__ long row_of_block(const int32_t *__restrict__ row_ptr, long mb, long p, int lane)
+{
+    long lo = 0, n = mb; // br is one of lo .. lo + n - 1
+    while (n > 1) {
+        const long step = (n + 63) / 64;
+        const long probe = lo + lane * step;
+        const unsigned long long at_most = __ballot(lane * step < n && row_ptr[probe] <= p); // a run of low bits: row_ptr ascends
+        const int last = 63 - __clzll((long long)at_most); // row_ptr[lo] <= p always
+        n = n - last * step < step ? n - last * step : step;
+        lo += last * step;
+    }
+    return lo;
+}
+
+// The nonzero columns of a block go to positions padded_start[br] + (columns of the block row in the blocks before it) .. of
+// the padded list, and
 //   acol != NULL: their 16 values each to acol, in MFMA operand order;
 //   else: their nonzeros to entries from entry_start[br] + (nonzeros of the block row before) on, column by column,
 //         each with its place in the operand of its step, and the range of entries of every step to step_range.
-__global__ void gather_kernel(const uint16_t *__restrict__ vals, const uint16_t *__restrict__ mask,
+// A wavefront takes GATHER_BLOCKS consecutive blocks, four at a time: lane (g = lane / 16, r = lane % 16) holds row r of one.
+// Bound by the second read of the values.  (One thread per block read them 2 bytes at a time, 64 cache lines a load, behind a
+// search of ten loads one after the other: 237 k blocks 54 -> 35 us;
+// 4, 8, 32 blocks a wavefront 36, 35, 39.)
+constexpr int GATHER_BLOCKS = 16;
+__global__ __launch_bounds__(256) void gather_kernel(const uint16_t *__restrict__ vals, const uint16_t *__restrict__ mask,
                               const unsigned long long *__restrict__ offset, const int32_t *__restrict__ row_ptr,
                               const int32_t *__restrict__ col_idx, const unsigned long long *__restrict__ raw,
                               const int2 *__restrict__ start, long mb, long nnzb, bool drop_full, int32_t *__restrict__ cols,
                               uint16_t *__restrict__ acol, uint32_t *__restrict__ entries, int2 *__restrict__ step_range)
 {
-    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= nnzb) return;
-    uint32_t m = mask[p];
-    if (!m || (drop_full && __popc(m) >= FULL_BLOCK_COLS)) return;
-    long lo = 0, hi = mb; // block row of p: largest br with row_ptr[br] <= p
-    while (hi - lo > 1) {
-        const long mid = (lo + hi) >> 1;
-        if (row_ptr[mid] <= p) lo = mid; else hi = mid;
-    }
-    const int2 first = start[lo]; // of the columns and of the entries
-    if (first.x < 0) return; // a block row that another kernel multiplies
-    const unsigned long long before = offset[p] - raw[lo]; // no borrow: both halves of offset[p] are at least those of raw
-    const long row_end = (long)first.x + (long)(uint32_t)(raw[lo + 1] - raw[lo]);
-    long o = (long)first.x + (long)(uint32_t)before;
-    int32_t at = first.y + (int32_t)(before >> 32);
-    const int32_t c0 = col_idx[p];
-    const uint16_t *blk = vals + p * 256;
-    while (m) {
-        const int k = __ffs(m) - 1;
-        m &= m - 1;
-        // inside its group of 8 the even entries come first, then the odd ones: the lanes of the product kernel that
-        // gather the even (odd) entries of a group read their four indices with one 16-byte load
-        cols[(o & ~7L) + ((o & 1) << 2) + ((o & 7) >> 1)] = c0 + k;
-        if (acol) {
-            uint16_t *dst = acol + ((o >> 3) * 16) * 8 + (o & 7); // (step*4 + g) = o / 8
-#pragma unroll
-            for (int r = 0; r < 16; r++) dst[r * 8] = blk[r * 16 + k];
-        } else {
-            if ((o & 31) == 0) step_range[o >> 5].x = at;
-            const uint32_t place = (uint32_t)((o & 31) >> 3) * 128u + (uint32_t)(o & 7); // half of the step's operand, row 0; the entry holds it in bytes
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const uint32_t v = blk[r * 16 + k];
-                if (v & 0x7fffu) entries[at++] = v << 16 | (place + r * 8) * 2;
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const long p_first = (((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * GATHER_BLOCKS;
+    if (p_first >= nnzb) return;
+    long br = row_of_block(row_ptr, mb, p_first, lane);
+    for (int i = 0; i < GATHER_BLOCKS && p_first + i < nnzb; i += 4) {
+        const bool live = p_first + i + g < nnzb;
+        const long p = live ? p_first + i + g : nnzb - 1;
+        // p is in br or a little further on; past a run of empty rows the rest is halved
+        int ahead = 0;
+        while (ahead < 8 && row_ptr[br + 1] <= p) br++, ahead++;
+        if (ahead == 8) {
+            long lo = br, hi = mb;
+            while (hi - lo > 1) {
+                const long mid = (lo + hi) >> 1;
+                if (row_ptr[mid] <= p) lo = mid; else hi = mid;
             }
-            if ((o & 31) == 31 || o + 1 == row_end) step_range[o >> 5].y = at;
+            br = lo;
         }
-        o++;
+        uint32_t m = live ? mask[p] : 0;
+        const int2 first = start[br]; // of the columns and of the entries
+        if ((drop_full && __popc(m) >= FULL_BLOCK_COLS) || first.x < 0) m = 0; // another kernel multiplies the block or the row
+        const u32x4 w[2] = {reinterpret_cast<const u32x4 *>(vals + p * 256 + r * 16)[0], reinterpret_cast<const u32x4 *>(vals + p * 256 + r * 16)[1]};
+        const unsigned long long before = offset[p] - raw[br]; // no borrow: both halves of offset[p] are at least those of raw
+        const long row_end = (long)first.x + (long)(uint32_t)(raw[br + 1] - raw[br]);
+        long o = (long)first.x + (long)(uint32_t)before;
+        int32_t at = first.y + (int32_t)(before >> 32);
+        const int32_t c0 = col_idx[p];
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+            const bool has = (m >> k) & 1;
+            if (!__any(has)) continue;
+            const uint32_t v = k & 1 ? w[k / 8][k % 8 / 2] >> 16 : w[k / 8][k % 8 / 2] & 0xffffu;
+            const uint32_t nonzero = (uint32_t)(__ballot(has && (v & 0x7fffu)) >> (16 * g)) & 0xffffu; // rows of the lane's block
+            if (!has) continue;
+            // inside its group of 8 the even entries come first, then the odd ones: the lanes of the product kernel that
+            // gather the even (odd) entries of a group read their four indices with one 16-byte load
+            if (r == 0) cols[(o & ~7L) + ((o & 1) << 2) + ((o & 7) >> 1)] = c0 + k;
+            if (acol) {
+                acol[((o >> 3) * 16 + r) * 8 + (o & 7)] = (uint16_t)v; // (step*4 + g) = o / 8
+            } else {
+                if (r == 0 && (o & 31) == 0) step_range[o >> 5].x = at;
+                const uint32_t place = (uint32_t)((o & 31) >> 3) * 128u + (uint32_t)(o & 7); // half of the step's operand, row 0; the entry holds it in bytes
+                if ((nonzero >> r) & 1) entries[at + __popc(nonzero & ((1u << r) - 1u))] = v << 16 | (place + r * 8) * 2;
+                at += __popc(nonzero);
+                if (r == 0 && ((o & 31) == 31 || o + 1 == row_end)) step_range[o >> 5].y = at;
+            }
+            o++;
+        }
     }
 }
 
@@ -996,7 +1043,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     if (e == hipSuccess && nnzb) {
         SMAT_STEP(hipMemcpy(starts.p, start.data(), (mb + 1) * sizeof(int2), hipMemcpyHostToDevice));
         if (e == hipSuccess) {
-            hipLaunchKernelGGL(gather_kernel, dim3((unsigned)((nnzb + 255) / 256)), dim3(256), 0, 0, vals, (const uint16_t *)s.mask.p,
+            hipLaunchKernelGGL(gather_kernel, dim3((unsigned)((nnzb + 4 * GATHER_BLOCKS - 1) / (4 * GATHER_BLOCKS))), dim3(256), 0, 0, vals, (const uint16_t *)s.mask.p,
                                (const unsigned long long *)s.offset.p, row_ptr, col_idx, (const unsigned long long *)s.rows.p, (const int2 *)starts.p,
                                (long)mb, (long)nnzb, drop_full, p->d_cols, p->d_acol, p->d_entries, p->d_step_range);
             e = hipGetLastError();
