@@ -10,7 +10,7 @@ to the block of the next descriptor.  A block is specialised for
     r  the block row of the wavefront the op adds to (which accumulators),
     v  whether the copies of a chunk boundary were issued between the load of its A operand and now (which s_waitcnt vmcnt),
 
-and a chunk boundary for the ops of the chunk it ends (4, 5, 6, 7 or more: again an s_waitcnt),
+and a chunk boundary for the ops of the chunk it ends (2, 3, .., 7 or more: again an s_waitcnt),
 
 so the run-time choices cost no instruction besides the jump.  It is written by hand because a
 wavefront issues in order: every instruction next to its MFMAs adds to its run time.  Blocks have a
@@ -20,12 +20,12 @@ Run after changing:
     python3 gen_sweep_loop.py > spmm_sweep_loop.inc
 
 Stream position i, J = i % 8.  Block of op i (AHEAD = 7):
-    even position: LDS reads of the B operands of op i + 1 (into set (J + 1) % 2), then a wait until only those
+    J % 4 < 3: LDS reads of the B operands of op i + 1 (into set (J + 1) % 2), then a wait until only those
     four are left: LDS reads return in order, so the reads of op i are in registers.  Scalar loads share the
     counter and return in any order; with one of them under way the same wait holds for the reads of op i
     (it then also waits for the first read of op i + 1 or for the scalar load, whichever comes first)
-    odd position: wait for everything (the reads of op i, and the descriptors that the odd position before it
-    asked for), scalar load of the descriptors of ops i + 7 and i + 8 (32 bytes), LDS reads of op i + 1
+    J % 4 == 3: wait for everything (the reads of op i, and the descriptors that the position four before it
+    asked for), scalar load of the descriptors of ops i + 5 .. i + 8 (64 bytes), LDS reads of op i + 1
     load of the A operand of op i + AHEAD (into slot (J + AHEAD) % 8 = (J - 1) % 8); its address is in the entry of op i + 1,
     as that of op i may be overwritten already
     wait for the A operand of op i, 4 MFMAs, jump to op i + 1
@@ -39,8 +39,8 @@ no stream position: no operand load and no descriptor slot is spent on it.
 
 Row-major B: rows of 64 columns, 128 bytes, as they lie in B; the operands come out of LDS through transposing reads of
 8 bytes a lane (ds_read_b64_tr_b16: the four rows that 16 lanes read come back as four k of one column each), eight instead
-of four an op; tile t is at the address of tile 0 with 8 t xor-ed to it.  LDS operations under way are counted in four bits, so an even position waits for op i when half of the
-reads of op i + 1 are on their way.
+of four an op; tile t is at the address of tile 0 with 8 t xor-ed to it.  LDS operations under way are counted in four bits, so a position waits for op i when half of the reads of
+op i + 1 are on their way.
 
 Registers (fixed, all listed as clobbers):
     v40-v71    B operands, two sets of 4 tiles x 4 registers
@@ -65,13 +65,13 @@ BSETS, ARING = 2, 8                      # B operands are read from LDS one posi
 RING = 8
 N_BLOCKS = 8 * 8 * 2                     # SWEEP_N_BLOCKS: stream position % 8 x block row x v
 TRAMP_BYTES = 8                          # SWEEP_TRAMP_BYTES
-MIN_OPS, MARKS = 4, 4                    # SWEEP_MIN_OPS, SWEEP_DEV_MARKS: boundaries after chunks of 4, 5, 6, 7 and more ops
+MIN_OPS, MARKS = 2, 6                    # SWEEP_DEV_MIN_OPS, SWEEP_DEV_MARKS: boundaries after chunks of 2, 3, .., 7 and more ops
 MARK_BYTES = 512                         # SWEEP_MARK_BYTES
 COPIES = 4
 TOUCHES = 2                              # loads of the entry code that bring A into the caches
 
 S_RING0 = 40
-DESC_AHEAD = 7   # an odd position loads the descriptors of ops i + DESC_AHEAD and the one after
+DESC_AHEAD = 5   # a position with J % 4 == 3 loads the descriptors of ops i + DESC_AHEAD and the three after
 S_DP, S_BASE, S_CUR, S_NEXTK, S_CP, S_T0, S_T1, S_JMP = 72, 74, 76, 77, 78, 80, 81, 84
 S_RET = 86
 S_HEAD = 88
@@ -152,16 +152,16 @@ def a_load(slot, offset):
 
 
 def top_wait(J):
-    """B operands of op i are in registers.  An even position asks for the reads of op i + 1 first and waits until
-    only they are left; an odd position waits for everything (reads of op i, descriptors asked for two positions
-    ago), asks for two descriptors and then for the reads of op i + 1."""
-    if J % 2 == 0:
+    """B operands of op i are in registers.  Three of four positions ask for the reads of op i + 1 first and wait until only
+    they are left; the fourth waits for everything (reads of op i, descriptors asked for four positions ago), asks for four
+    descriptors and then for the reads of op i + 1."""
+    if J % 4 != 3:
         b_reads(J + 1, J + 1, wait=4)
         return
     emit("s_waitcnt lgkmcnt(0)")
     s0 = S_RING0 + 4 * ((J + DESC_AHEAD) % RING)
-    emit(f"s_load_dwordx8 s[{s0}:{s0 + 7}], s[{S_DP}:{S_DP + 1}], 0x0")
-    emit(f"s_add_u32 s{S_DP}, s{S_DP}, 32")
+    emit(f"s_load_dwordx16 s[{s0}:{s0 + 15}], s[{S_DP}:{S_DP + 1}], 0x0")
+    emit(f"s_add_u32 s{S_DP}, s{S_DP}, 64")
     emit(f"s_addc_u32 s{S_DP + 1}, s{S_DP + 1}, 0")
     b_reads(J + 1, J + 1)
 
@@ -205,6 +205,7 @@ def boundary_code():
     emit(f"s_add_u32 s{S_T0}, s{S_CUR}, 2")
     emit(f"s_cmp_ge_u32 s{S_T0}, %[n_chunks]")
     emit("s_cbranch_scc1 Lmn_%=")
+    emit("s_waitcnt lgkmcnt(0)")                      # the id that the boundary before asked for
     # copies of chunk cur + 2 into stage (cur + 2) % 4: rows of B from k = 256 * id (the id was loaded by the previous boundary)
     if ROW_MAJOR:
         emit(f"s_mul_i32 s{S_T1}, s{S_NEXTK}, %[chunk_bytes]")
@@ -282,7 +283,7 @@ def loop():
 clob = ([f'"v{i}"' for i in range(V_B0, V_TOUCH + 1)] + [f'"s{i}"' for i in range(S_RING0, S_LAST + 1)] +
         [f'"a{i}"' for i in range(128)] + ['"vcc"', '"scc"', '"memory"'])
 print("// generated by gen_sweep_loop.py; do not edit")
-print(f"static_assert(SWEEP_DEV_AHEAD == {AHEAD} && SWEEP_MIN_OPS == {MIN_OPS} && SWEEP_DEV_MARKS == {MARKS} && SWEEP_N_BLOCKS == {N_BLOCKS} && "
+print(f"static_assert(SWEEP_DEV_AHEAD == {AHEAD} && SWEEP_DEV_MIN_OPS == {MIN_OPS} && SWEEP_DEV_MARKS == {MARKS} && SWEEP_N_BLOCKS == {N_BLOCKS} && "
       f"SWEEP_TRAMP_BYTES == {TRAMP_BYTES} && SWEEP_MARK_BYTES == {MARK_BYTES}, \"regenerate spmm_sweep_loop.inc\");")
 for ROW_MAJOR in (True, False):
     out.clear()

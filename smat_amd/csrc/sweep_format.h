@@ -53,24 +53,26 @@ constexpr uint32_t SWEEP_MARK_BYTES = 512;
 constexpr uint32_t SWEEP_END_OFF = SWEEP_MARK_OFF + SWEEP_MARK_BYTES;               // 17920
 
 // The streams as the kernel runs them.  Each starts with SWEEP_DEV_HEAD entries that hold, one uint32 after the other, the A
-// offsets of its first AHEAD ops (0 behind the last op), where AHEAD = SWEEP_DEV_AHEAD; then come the entries of the plan with
+// offsets of its first AHEAD ops (0 behind the last op), where AHEAD = SWEEP_DEV_AHEAD; then come the entries of the plan,
+// without the fillers that do not open a chunk as far as SWEEP_DEV_MIN_OPS ops of the chunk are left, with
 //   w0  the A offset of op i + AHEAD - 1 (0 behind the last op): the position in front asks for it
 //   w1, w2 as in the plan; in streams for row-major B the LDS offsets are those of stages of [16 slabs][16 k][64 columns]
 //   w3  op      its block, v = 1 when the copies of a chunk boundary were issued after the load of this op's A operand; the
 //               block waits until AHEAD + 4 v vector memory operations are under way, with the copies of two boundaries in
 //               between (chunks of less than AHEAD ops) for a little more than it has to
 //       first op of every chunk but the first:  sweep_tramp_base + (m * SWEEP_N_BLOCKS + the op's block index) *
-//               SWEEP_TRAMP_BYTES, m = min(ops of the chunk before, AHEAD) - SWEEP_MIN_OPS: so many more A loads than
-//               SWEEP_MIN_OPS may be under way when the boundary's own copies have landed
+//               SWEEP_TRAMP_BYTES, m = min(ops of the chunk before, AHEAD) - SWEEP_DEV_MIN_OPS: so many more A loads than
+//               SWEEP_DEV_MIN_OPS may be under way when the boundary's own copies have landed
 //       end     sweep_end_off
 // The two loops (column-major and row-major B) have blocks of different sizes.
 constexpr int SWEEP_DEV_AHEAD = 7; // with a ring of eight operands the most there is room for
 constexpr int SWEEP_DEV_HEAD = 2;
-constexpr int SWEEP_DEV_MARKS = SWEEP_DEV_AHEAD - SWEEP_MIN_OPS + 1;
+constexpr int SWEEP_DEV_MIN_OPS = 2; // ops per wavefront and chunk
+constexpr int SWEEP_DEV_MARKS = SWEEP_DEV_AHEAD - SWEEP_DEV_MIN_OPS + 1;
 constexpr uint32_t sweep_block_bytes(bool row_major) { return row_major ? 192 : SWEEP_BLOCK_BYTES; }
 constexpr uint32_t sweep_tramp_base(bool row_major) { return SWEEP_N_BLOCKS * sweep_block_bytes(row_major); }
 constexpr uint32_t sweep_end_off(bool row_major) { return sweep_tramp_base(row_major) + SWEEP_DEV_MARKS * SWEEP_N_BLOCKS * SWEEP_TRAMP_BYTES + SWEEP_MARK_BYTES; }
-static_assert(SWEEP_DEV_AHEAD <= 4 * SWEEP_DEV_HEAD && SWEEP_DEV_AHEAD > SWEEP_MIN_OPS, "the head holds the offsets of the first ops");
+static_assert(SWEEP_DEV_AHEAD <= 4 * SWEEP_DEV_HEAD && SWEEP_DEV_AHEAD > SWEEP_DEV_MIN_OPS, "the head holds the offsets of the first ops");
 
 inline uint32_t sweep_lds_offset(int32_t chunk_pos, int32_t slab)
 {

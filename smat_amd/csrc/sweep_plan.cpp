@@ -380,45 +380,65 @@ void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::v
                           bool b_row_major, std::vector<SweepOpHost> &dev)
 {
     const uint32_t block_bytes = sweep_block_bytes(b_row_major), tramp_base = sweep_tramp_base(b_row_major);
-    constexpr int DEV_AHEAD = SWEEP_DEV_AHEAD, HEAD = SWEEP_DEV_HEAD;
+    constexpr int DEV_AHEAD = SWEEP_DEV_AHEAD, DEV_MIN = SWEEP_DEV_MIN_OPS, HEAD = SWEEP_DEV_HEAD;
     const size_t n_streams = op_ptr.size() - 1;
     dev.assign((size_t)op_ptr.back() + HEAD * n_streams + SWEEP_OP_PAD, SweepOpHost{0, SWEEP_ZERO_OFF, 0, sweep_end_off(b_row_major)});
+    struct Op { SweepOpHost op; uint32_t row; bool opens; };
+    std::vector<Op> kept;
     std::vector<long> a_issue;
     for (size_t s = 0; s < n_streams; s++) {
         const SweepOpHost *op = ops + op_ptr[s];
         SweepOpHost *out = dev.data() + op_ptr[s] + HEAD * s;
-        const size_t len = (size_t)(op_ptr[s + 1] - op_ptr[s]), n_ops = len ? len - 1 : 0; // the end is no op
+        const size_t len = (size_t)(op_ptr[s + 1] - op_ptr[s]), n_plan = len ? len - 1 : 0; // the end is no op
         const long n_chunks = rg_chunk_ptr[s / WAVES + 1] - rg_chunk_ptr[s / WAVES];
-        auto a_offset = [&](size_t i) { return i < n_ops ? op[i].w0 : 0u; };
+        // the fillers of the plan keep chunks at MIN_OPS ops: those past DEV_MIN go, but not the one that opens a chunk, which
+        // stands there because no other op may
+        kept.clear();
+        for (size_t i = 0; i < n_plan;) {
+            size_t end = i + 1;
+            while (end < n_plan && op[end].w3 < SWEEP_TRAMP_BASE) end++;
+            long work = 0, taken = 0;
+            auto filler = [&](size_t k) { return op[k].w1 == SWEEP_ZERO_OFF && op[k].w2 == 0; };
+            for (size_t k = i; k < end; k++) work += k == i || !filler(k);
+            long fill = DEV_MIN - work;
+            for (size_t k = i; k < end; k++) {
+                if (k > i && filler(k) && fill-- <= 0) continue;
+                const bool opens = op[k].w3 >= SWEEP_TRAMP_BASE;
+                const uint32_t block = opens ? (op[k].w3 - SWEEP_TRAMP_BASE) / SWEEP_TRAMP_BYTES : op[k].w3 / SWEEP_BLOCK_BYTES;
+                kept.push_back(Op{op[k], block / 2 % 8, opens});
+                taken++;
+            }
+            if (taken < DEV_MIN) throw std::logic_error("sweep plan: chunk boundaries closer than the copies' wait allows");
+            i = end;
+        }
+        const size_t n_ops = kept.size();
+        auto a_offset = [&](size_t i) { return i < n_ops ? kept[i].op.w0 : 0u; };
         uint32_t head[4 * HEAD] = {0};
         for (int k = 0; k < DEV_AHEAD; k++) head[k] = a_offset((size_t)k);
         memcpy(out, head, sizeof head);
         out += HEAD;
         // vector memory operations in issue order: what is younger than the load of an op's A operand when the op needs it
-        a_issue.assign(len + DEV_AHEAD + 1, 0);
+        a_issue.assign(n_ops + DEV_AHEAD + 1, 0);
         long seq = 0, cur = 0, in_chunk = 0;
         for (int k = 0; k < DEV_AHEAD; k++) a_issue[(size_t)k] = ++seq;
         for (size_t i = 0; i < n_ops; i++) {
-            const bool opens = op[i].w3 >= SWEEP_TRAMP_BASE;
-            const uint32_t block = opens ? (op[i].w3 - SWEEP_TRAMP_BASE) / SWEEP_TRAMP_BYTES : op[i].w3 / SWEEP_BLOCK_BYTES;
+            const bool opens = kept[i].opens;
             uint32_t m = 0;
             if (opens) {
-                if (in_chunk < MIN_OPS) throw std::logic_error("sweep plan: chunk boundaries closer than the copies' wait allows");
-                m = (uint32_t)(std::min<long>(in_chunk, DEV_AHEAD) - MIN_OPS);
+                m = (uint32_t)(std::min<long>(in_chunk, DEV_AHEAD) - DEV_MIN);
                 in_chunk = 0;
                 if (++cur + 2 < n_chunks) seq += COPIES;
             }
             in_chunk++;
             a_issue[i + DEV_AHEAD] = ++seq;
-            const uint32_t v = seq - a_issue[i] > DEV_AHEAD ? 1u : 0u;
-            const uint32_t code = (block & ~1u) | v;
+            const uint32_t code = (uint32_t)((i % 8 * 8 + kept[i].row) * 2) + (seq - a_issue[i] > DEV_AHEAD ? 1u : 0u);
+            const uint32_t lo = kept[i].op.w1, hi = lo + kept[i].op.w2;
             out[i].w0 = a_offset(i + DEV_AHEAD - 1);
-            const uint32_t lo = op[i].w1, hi = op[i].w1 + op[i].w2;
             out[i].w1 = b_row_major ? sweep_lds_offset_row_major(lo) : lo;
             out[i].w2 = (b_row_major ? sweep_lds_offset_row_major(hi) : hi) - out[i].w1;
             out[i].w3 = opens ? tramp_base + (m * SWEEP_N_BLOCKS + code) * SWEEP_TRAMP_BYTES : code * block_bytes;
         }
-        // the end stays what dev was filled with
+        // the end, and what the dropped fillers leave behind it, stay what dev was filled with
     }
 }
 

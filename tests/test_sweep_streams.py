@@ -8,9 +8,9 @@ import pytest
 
 from smat_amd import generators as gen
 from smat_amd._lib import lib
-from tests.test_sweep_plan import BLOCK_BYTES, COPIES, END_OFF, MARK_OFF, MIN_OPS, N_BLOCKS, PAD, TRAMP_BASE, TRAMP_BYTES, WAVES, ZERO_OFF, random_mask_matrix, sweep_plan
+from tests.test_sweep_plan import BLOCK_BYTES, COPIES, END_OFF, N_BLOCKS, PAD, TRAMP_BASE, TRAMP_BYTES, WAVES, ZERO_OFF, random_mask_matrix, sweep_plan
 
-AHEAD, HEAD, MARKS, TOUCHES = 7, 2, 4, 2
+AHEAD, HEAD, DEV_MIN_OPS, MARKS, TOUCHES = 7, 2, 2, 6, 2
 
 
 def encode(plan, row_major):
@@ -42,14 +42,27 @@ def check(plan, row_major):
         out = dev[a + HEAD * (s + 1):b + HEAD * (s + 1)].astype(np.int64)
         if a == b:
             continue
-        n = ops.shape[0] - 1
-        assert ops[n, 3] == END_OFF and tuple(out[n]) == (0, ZERO_OFF, 0, end_off)
-        a_of = np.concatenate([ops[:n, 0], np.zeros(AHEAD, np.int64)])
+        assert ops[-1, 3] == END_OFF
+        # what is left of the plan's entries: all but fillers that do not open a chunk, two of a chunk at least
+        opens = ops[:-1, 3] >= TRAMP_BASE
+        chunk = np.cumsum(opens)
+        first = opens | (np.arange(opens.size) == 0)
+        filler = (ops[:-1, 1] == ZERO_OFF) & (ops[:-1, 2] == 0)
+        keep = first | ~filler
+        for c in range(chunk[-1] + 1):
+            spare = np.flatnonzero((chunk == c) & ~keep)
+            keep[spare[:max(0, DEV_MIN_OPS - int(keep[chunk == c].sum()))]] = True
+        assert np.all(np.bincount(chunk[keep]) >= DEV_MIN_OPS)
+        seen.add(("dropped", bool((~keep).any())))
+        ops = ops[:-1][keep]
+        n = ops.shape[0]
+        assert np.all(out[n:] == (0, ZERO_OFF, 0, end_off))
+        a_of = np.concatenate([ops[:, 0], np.zeros(AHEAD, np.int64)])
         assert np.array_equal(head[:AHEAD], a_of[:AHEAD]) and not head[AHEAD:].any()
         assert np.array_equal(out[:n, 0], a_of[AHEAD - 1:AHEAD - 1 + n])
-        delta = ops[:n, 2].astype(np.uint32).view(np.int32), out[:n, 2].astype(np.uint32).view(np.int32)
-        assert np.array_equal(out[:n, 1], lds_offset(ops[:n, 1], row_major))
-        assert np.array_equal(out[:n, 1] + delta[1], lds_offset(ops[:n, 1] + delta[0], row_major))
+        delta = ops[:, 2].astype(np.uint32).view(np.int32), out[:n, 2].astype(np.uint32).view(np.int32)
+        assert np.array_equal(out[:n, 1], lds_offset(ops[:, 1], row_major))
+        assert np.array_equal(out[:n, 1] + delta[1], lds_offset(ops[:, 1] + delta[0], row_major))
         n_chunks = int(plan["rg_chunk_ptr"][s // WAVES + 1] - plan["rg_chunk_ptr"][s // WAVES])
         # issue order: copies of chunks 0..2, the first A operands, the touches, then per position [copies of a boundary], A
         issued = [("copy", c) for c in range(min(3, n_chunks)) for _ in range(COPIES)]
@@ -64,7 +77,7 @@ def check(plan, row_major):
                 m, k = divmod((w3 - tramp_base) // TRAMP_BYTES, N_BLOCKS)
                 assert tramp_base <= w3 < mark_off and (w3 - tramp_base) % TRAMP_BYTES == 0
                 plan_k = (plan_w3 - TRAMP_BASE) // TRAMP_BYTES
-                assert landed(("copy", cur + 2), MIN_OPS + m) or cur + 2 >= n_chunks
+                assert landed(("copy", cur + 2), DEV_MIN_OPS + m) or cur + 2 >= n_chunks
                 cur += 1
                 if cur + 2 < n_chunks:
                     issued += [("copy", cur + 2)] * COPIES
@@ -72,7 +85,7 @@ def check(plan, row_major):
             else:
                 assert w3 < tramp_base and w3 % block_bytes == 0
                 k, plan_k = w3 // block_bytes, plan_w3 // BLOCK_BYTES
-            assert k // 2 == plan_k // 2  # stream position and block row
+            assert k // 16 == i % 8 and k // 2 % 8 == plan_k // 2 % 8  # stream position and block row
             issued.append(("a", i + AHEAD))
             assert landed(("a", i), AHEAD + COPIES * (k % 2))
             seen.add(("op", k % 2))
@@ -93,4 +106,7 @@ def test_waits_of_the_device_streams(mb, kb, density, seed, group_rows, row_majo
 def test_device_streams_use_every_wait():
     A = gen.block_pruned(4096, 0.10, 0.02)
     plan = sweep_plan(A["b_row_ptr"], A["b_col_idx"], A["M"], A["K"])
-    assert check(plan, 0) == {("op", 0), ("op", 1)} | {("mark", m) for m in range(MARKS)}
+    seen = check(plan, 0)
+    A = random_mask_matrix(64, 200, 0.03, 1)
+    seen |= check(sweep_plan(A["b_row_ptr"], A["b_col_idx"], A["M"], A["K"], group_rows=32), 0)
+    assert seen == {("op", 0), ("op", 1), ("dropped", False), ("dropped", True)} | {("mark", m) for m in range(MARKS)}
