@@ -1105,13 +1105,30 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     // for each (32768 x 65536, 131 a row, N = 256: 138 us whole, 191 in chunks of 1792 columns; 8192 x 65536, 140 a row,
     // N = 1024: 175 against 241) - except where whole rows would be fewer than four wavefronts a CU (2048 x 65536, 140 a row,
     // N = 256, 512 wavefronts: 43 us whole, 34 in halves; 512 x 65536, 300 a row, N = 1024, 512 of them: 96 against 75).
+    // How long a chunk: what a wavefront's place on the device does in a launch (steps and panels over 16 places a CU) bounds the
+    // time that one chunk may take, and the partial tiles ask for long ones.  Steps of a chunk, us (R-MAT, 16 a row, avg 7 steps):
+    //   scale 20, N = 128, 240 steps a place: 14 605, 28 519, 56 488, 112 483
+    //   scale 18, N = 256, 120:               14 242, 28 211, 56 203, 84 211, 112 216
+    //   scale 17, N = 256, 60:                14 130, 21 107, 28 104, 56 110
+    //   scale 16, N = 128, 15:                14 34.7, 21 32.4, 28 32.9, 56 41.5
+    //   scale 14, N = 128, 4:                 7 17.1, 14 17.6, 21 18.5, 28 20.0, 56 28.8
+    // The rule, 16 steps and 0.38 of those of a place, against four times the average in every launch, as before: scale 20 520 -> 488,
+    // scale 13, N = 256 19.1 -> 16.1; of 24 R-MAT products two are slower, by 2 %.  Whether a list is split at all, which costs a launch, is decided by four
+    // times the average and 16 steps, or the chunk where that is longer.
     const std::vector<int32_t> &cc_host = padded;
     size_t nonempty = 0;
-    for (size_t i = 0; i < mb; i++) nonempty += cc_host[i + 1] > cc_host[i];
+    long longest = 0;
+    for (size_t i = 0; i < mb; i++) {
+        const long len = cc_host[i + 1] - cc_host[i];
+        nonempty += len > 0;
+        if (!dense[i]) longest = std::max(longest, len);
+    }
     const double avg = nonempty ? (double)total / (double)nonempty : 0.0;
-    long chunk = (long)(4.0 * avg + 0.5);
-    chunk = std::max(chunk, 512L);
-    chunk = (chunk + 31) / 32 * 32;
+    const double steps_a_place = (double)(total / 32) * (double)((n_cap + 63) / 64) / (16.0 * 256.0);
+    const double share = n_cap < 64 ? 0.8 : 0.38; // narrow: a step brings less, and a partial tile takes a store all the same
+    long chunk = 32 * (long)(std::max(16.0 + share * steps_a_place, 2.5 * avg / 32.0) + 0.5);
+    const long from = std::max((long)(4.0 * avg + 0.5), 512L);
+    if (longest <= from) chunk = std::max(chunk, from);
     if (nonempty * ((n_cap + 63) / 64) < 1024) chunk = std::min(chunk, 32L * LONG_ROW_STEPS);
     std::vector<WorkItem> items;
     std::vector<SplitRow> split;
