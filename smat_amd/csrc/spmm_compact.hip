@@ -347,6 +347,8 @@ __global__ __launch_bounds__(256) void copy_blocks_kernel(const uint16_t *__rest
 // The output is split into panels of `panel` columns, each a K x panel row-major matrix of leading
 // dimension ld, one panel after the other (panel >= N and ld = N: plain row-major K x N).
 // place != NULL: row k goes to row place[k] of a copy of `rows` rows, or nowhere (-1).
+// STREAM: B does not stay in the caches behind the loads, which leaves them to the copy (launch_transpose).
+template <bool STREAM>
 __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__restrict__ B, uint16_t *__restrict__ Bt,
                                                           int N, long K, int panel, long ld, long rows, const int32_t *__restrict__ place)
 {
@@ -355,34 +357,50 @@ __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__rest
     const int t = threadIdx.x;
     const long k0 = (long)blockIdx.x * 64;
     const int n0 = blockIdx.y * 64;
-    {
-        const int np = t >> 3, seg = t & 7; // columns 2np, 2np+1; k = 8seg .. 8seg+7
-        u32x4 v0 = {0u, 0u, 0u, 0u}, v1 = {0u, 0u, 0u, 0u};
-        if (k0 + seg * 8 < K) {
-            if (n0 + 2 * np < N) v0 = *reinterpret_cast<const u32x4 *>(B + (long)(n0 + 2 * np) * K + k0 + seg * 8);
-            if (n0 + 2 * np + 1 < N) v1 = *reinterpret_cast<const u32x4 *>(B + (long)(n0 + 2 * np + 1) * K + k0 + seg * 8);
-        }
+    const int a = t >> 3, seg = t & 7;
+    u32x4 v0 = {0u, 0u, 0u, 0u}, v1 = {0u, 0u, 0u, 0u}; // columns 2a, 2a+1; k = 8seg .. 8seg+7
+    if (k0 + seg * 8 < K) {
+        const u32x4 *p0 = reinterpret_cast<const u32x4 *>(B + (long)(n0 + 2 * a) * K + k0 + seg * 8);
+        const u32x4 *p1 = reinterpret_cast<const u32x4 *>(B + (long)(n0 + 2 * a + 1) * K + k0 + seg * 8);
+        if (n0 + 2 * a < N) v0 = STREAM ? __builtin_nontemporal_load(p0) : *p0;
+        if (n0 + 2 * a + 1 < N) v1 = STREAM ? __builtin_nontemporal_load(p1) : *p1;
+    }
+    long to[2]; // the rows that this thread stores, asked for beside the values (behind the barrier: 94 instead of 87 us for 256 MiB)
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
-            uint32_t *row = reinterpret_cast<uint32_t *>(tile + (seg * 8 + 2 * w) * LD + 2 * np);
-            row[0] = __builtin_amdgcn_perm(v1[w], v0[w], 0x05040100u);      // k = 8seg + 2w
-            row[LD / 2] = __builtin_amdgcn_perm(v1[w], v0[w], 0x07060302u); // k = 8seg + 2w + 1
-        }
+    for (int half = 0; half < 2; half++) {
+        const long k = k0 + a + 32 * half;
+        to[half] = k >= K ? -1 : place ? (long)place[k] : k;
+    }
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        uint32_t *row = reinterpret_cast<uint32_t *>(tile + (seg * 8 + 2 * w) * LD + 2 * a);
+        row[0] = __builtin_amdgcn_perm(v1[w], v0[w], 0x05040100u);      // k = 8seg + 2w
+        row[LD / 2] = __builtin_amdgcn_perm(v1[w], v0[w], 0x07060302u); // k = 8seg + 2w + 1
     }
     __syncthreads();
-    const int a = t >> 3, seg = t & 7;
 #pragma unroll
     for (int half = 0; half < 2; half++) {
         const int k = a + 32 * half;
-        long row = k0 + k;
-        if (place && k0 + k < K) row = place[k0 + k];
-        if (k0 + k < K && n0 + seg * 8 < N && row >= 0) {
+        if (to[half] >= 0 && n0 + seg * 8 < N) {
             const uint2 lo = *reinterpret_cast<const uint2 *>(tile + k * LD + seg * 8);
             const uint2 hi = *reinterpret_cast<const uint2 *>(tile + k * LD + seg * 8 + 4);
-            uint16_t *out = Bt + (long)(n0 / panel) * rows * panel + row * ld + n0 % panel + seg * 8;
+            uint16_t *out = Bt + (long)(n0 / panel) * rows * panel + to[half] * ld + n0 % panel + seg * 8;
             *reinterpret_cast<u32x4 *>(out) = (u32x4){lo.x, lo.y, hi.x, hi.y};
         }
     }
+}
+
+// A B of half of the memory-side cache and more is not there any more when the next launch reads it, so it need not displace
+// the copy and the lists on its way through (R-MAT scale 20, N = 128, 256 MiB: 485 -> 472 us).  A smaller one may be
+// (27-point stencil 64^3, N = 64, 33 MB, the same B again: 41.0 us, past the caches 44.3).
+static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, size_t K, int panel, long ld, long rows, const int32_t *place, hipStream_t st)
+{
+    const dim3 grid((unsigned)((K + 63) / 64), (unsigned)((N + 63) / 64));
+    if (N * K * sizeof(uint16_t) >= (size_t)128 << 20)
+        hipLaunchKernelGGL(transpose_b_kernel<true>, grid, dim3(256), 0, st, B, Bt, (int)N, (long)K, panel, ld, rows, place);
+    else
+        hipLaunchKernelGGL(transpose_b_kernel<false>, grid, dim3(256), 0, st, B, Bt, (int)N, (long)K, panel, ld, rows, place);
+    return hipGetLastError();
 }
 
 // ---- the product ----
@@ -666,9 +684,7 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
     if (!a.b_row_major) {
         const long rows = p.d_place ? (long)p.n_placed : (long)a.K; // of the copy
         if (p.d_place) cols = p.d_cols_placed;
-        dim3 grid((unsigned)((a.K + 63) / 64), (unsigned)((a.N + 63) / 64));
-        hipLaunchKernelGGL(transpose_b_kernel, grid, dim3(256), 0, st, a.B, a.Bt, (int)a.N, (long)a.K, PANEL, (long)PANEL, rows, (const int32_t *)p.d_place);
-        hipError_t e = hipGetLastError();
+        const hipError_t e = launch_transpose(a.B, a.Bt, a.N, a.K, PANEL, PANEL, rows, p.d_place, st);
         if (e != hipSuccess) return e;
         panel_stride = rows * PANEL;
         row_stride = PANEL;
@@ -718,10 +734,7 @@ using Scratch = DevScratch;
 // two dimensions swapped (N % 8 == 0 and K % 16 == 0 keep every 16-byte access aligned).
 hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, size_t N, size_t K, hipStream_t st)
 {
-    dim3 grid((unsigned)((N + 63) / 64), (unsigned)((K + 63) / 64));
-    hipLaunchKernelGGL(transpose_b_kernel, grid, dim3(256), 0, st, B_row_major, out, (int)K, (long)N, 0x7fffffff, (long)K, (long)N,
-                       (const int32_t *)nullptr);
-    return hipGetLastError();
+    return launch_transpose(B_row_major, out, K, N, 0x7fffffff, (long)K, (long)N, nullptr, st);
 }
 
 // The panel width of a launch, in units of 64 columns.
