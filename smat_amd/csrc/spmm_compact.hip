@@ -52,12 +52,15 @@ int g_force_run = 0;
 int g_tune = 1; // test hook: 0 = attaching values measures nothing, the estimate decides the deal
 int g_last_run = 0; // test hook: the run length of the latest launch
 int g_force_list = 0; // test hook: 1 = lists of whole columns, 2 = of nonzeros, 0 = compact_build decides
+int g_force_staged = 0; // test hook: 1 = entries go through LDS in blocks wherever they may, 2 = nowhere, 0 = the launcher decides
 int g_force_tq = 0; // test hook: 1 or 2 = panels of 64 or 128 columns whatever the sizes say, 0 = the launcher decides
 
 constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts as full (of 16)
 constexpr int TASK_STEPS = 12;     // short items are put together up to this many steps (8 to 24: level; one item each: 9 % slower on R-MAT)
 constexpr int LONG_ROW_STEPS = 56; // steps from which a block row is split where a launch has few wavefronts
 constexpr size_t PLACE_MIN_BYTES = (size_t)16 << 20; // of B, from which the rows that its copy does not need are looked for
+constexpr double STAGED_STEPS = 20.0; // a place's steps from which entries are staged: of 10 products with 20 and more one was slower, by 0.6 %, of 14 with fewer one faster, by 6 %
+constexpr int ENTRY_PAD = 1024; // entries readable past the last one (blocks of 256, one ahead, another for the steps past the end of a task)
 constexpr int LIST_PAD = 2304; // entries readable past the end of the list (the index loads of the 64-column panel run up to 16 steps ahead)
 
 // ---- census of nonzero block columns ----
@@ -424,7 +427,7 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 //   * The A operand (AF): 0: acol, 1 KiB a step.  1, 2: entries, 4 bytes per nonzero; the at most 64 * AF of a step are put
 //     to their places in 1 KiB of LDS that is zero otherwise, read back as the operand and cleared again (LDS operations
 //     of a wavefront complete in order: nothing is waited for in between).
-//   * Every load of a step is unconditional and nothing in the loop uses scalar loads, so that what is in flight can be
+//   * Every load of a step (but a new block of indices or entries) is unconditional and nothing in the loop uses scalar loads, so that what is in flight can be
 //     counted; the gathers asked for past the end of the task read row 0.
 // Whole products with all of it (before: operands merged in the VALU, A in whole columns, an item per wavefront): R-MAT
 // scale 20, N = 128, 703 -> 590 us; Erdos-Renyi 16384^2, 0.1 %, N = 256, 17.3 -> 16.0 us.  A third copy of the step's code
@@ -441,15 +444,21 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 //     before it asked for the next ones.  A task that ends with the first step ends there with s_endpgm.
 //   * LDS for four workgroups a CU (TQ = 1): with five, which the registers now allow, the gathers of R-MAT scale 20 lose 0.6 %
 //     and 16384^2 2 % (three: 16384^2 11 %).
-template <int TQ, bool C_F32, bool C_ACC, int AF, bool BIG>
+//
+// Entries (AF > 0) come from memory in the step before they are needed, 256 bytes a load, or, STAGED, 256 at a time ahead of
+// that, one load of 1 KiB to LDS: a load of 256 bytes takes the vector memory path as long as one of 1 KiB, and a list that
+// no cache holds arrives early enough.  That pays where a wavefront's place on the device has many steps to do, before the
+// longer way of the first entries of a task counts (STAGED_STEPS): stencil 64^3, N = 64 57.5 -> 53.3 us, N = 256 186 -> 177; R-MAT
+// scale 18, N = 64 74.7 -> 69.4, scale 20, N = 128 474 -> 463; but stencil 40^3, N = 64 13.8 -> 15.2; 16384^2, 16 a row, N = 128 10.8 -> 11.6.
+template <int TQ, bool C_F32, bool C_ACC, int AF, bool STAGED, bool BIG>
 __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const uint16_t *__restrict__ acol, const uint32_t *__restrict__ entries, const int2 *__restrict__ step_range, const int32_t *__restrict__ cols,
     const uint16_t *__restrict__ Bt, void *__restrict__ Cout, float *__restrict__ workspace, const WorkItem *__restrict__ items,
     const int4 *__restrict__ tasks, int n_tasks, int N, int n_panels, long panel_stride, long row_stride, unsigned xcd_run)
 {
-    constexpr int A_BYTES = 1024, B_BYTES = 4096 * TQ, I_BYTES = 2048, UNUSED_BYTES = TQ == 1 ? 2048 : 0;
-    static_assert((A_BYTES + B_BYTES + I_BYTES + UNUSED_BYTES) % 1024 == 0, "entries hold offsets that are or-ed to the address of the A tile");
-    __shared__ __align__(1024) unsigned char lds[4][A_BYTES + B_BYTES + I_BYTES + UNUSED_BYTES];
+    constexpr int A_BYTES = 1024, B_BYTES = 4096 * TQ, I_BYTES = 2048, E_BYTES = STAGED ? 2048 : 0, UNUSED_BYTES = TQ == 1 ? 2048 - E_BYTES : 0;
+    static_assert((A_BYTES + B_BYTES + I_BYTES + E_BYTES + UNUSED_BYTES) % 1024 == 0, "entries hold offsets that are or-ed to the address of the A tile");
+    __shared__ __align__(1024) unsigned char lds[4][A_BYTES + B_BYTES + I_BYTES + E_BYTES + UNUSED_BYTES];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // Panel-major order of the (panel, task) space.  An XCD gets the workgroup ids that are equal modulo 8, whatever
@@ -524,10 +533,22 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     auto load_block = [&](int s) { return reinterpret_cast<const u32x4 *>(cols + s)[lane]; };
     auto put_block = [&](int s, u32x4 x) { *reinterpret_cast<u32x4 *>(i_tile + (((s >> 5) - first_step) & 8) * 128 + lane * 16) = x; };
     auto indices = [&](int s) { return *reinterpret_cast<const u32x4 *>(i_tile + (((s >> 5) - first_step) & 15) * 128 + oct * 16); };
+    // Entries the same way: 256 of them, 1 KiB, a load, to one half of 2 KiB of LDS; the next 256 are on their way meanwhile.
+    unsigned char *const e_tile = lds[wave] + A_BYTES + B_BYTES + I_BYTES;
+    u32x4 e_next = {0u, 0u, 0u, 0u}, e_after = {0u, 0u, 0u, 0u};
+    int e_block = 0, e_end = 0; // of 256 entries: the one in e_next, and the last of the task as far as its ranges are here
+    auto load_entries = [&](int b) { return reinterpret_cast<const u32x4 *>(entries)[(long)b * 64 + lane]; };
+    if constexpr (STAGED) {
+        e_block = __builtin_amdgcn_readlane(ranges.x, 0) >> 8;
+        const int steps = (e_last >> 5) - first_step;
+        e_end = steps > 64 ? 0x7fffffff : (__builtin_amdgcn_readlane(ranges.y, steps > 0 ? steps - 1 : 0) - 1) >> 8;
+        e_next = load_entries(e_block);
+        e_after = load_entries(e_block + 1);
+    }
     auto request = [&](int s, const u32x4 x, Operands &o) {
         if constexpr (AF == 0) {
             o.aw = *reinterpret_cast<const u32x4 *>(acol + ((long)(s >> 3) + g) * 128 + i16 * 8);
-        } else {
+        } else if constexpr (!STAGED) {
             const int first = __builtin_amdgcn_readlane(ranges.x, (s >> 5) - range_from);
             o.n = __builtin_amdgcn_readlane(ranges.y, (s >> 5) - range_from) - first;
 #pragma unroll
@@ -547,6 +568,19 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
                 for (int j = 0; j < 4; j++)
                     o.L[q][j] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const unsigned char *>(Bp) +
                                                                  (size_t)(uint32_t)(__umul24(x[j], stride) + (uint32_t)boff[q] * 2u));
+        }
+        if constexpr (STAGED) {
+            const int first = __builtin_amdgcn_readlane(ranges.x, (s >> 5) - range_from);
+            o.n = __builtin_amdgcn_readlane(ranges.y, (s >> 5) - range_from) - first;
+            // a step has at most 128 entries: one more block, two for the first step of a task
+            for (int k = 0; k < 2 && (first + o.n - 1) >> 8 >= e_block; k++) {
+                *reinterpret_cast<u32x4 *>(e_tile + (e_block & 1) * 1024 + lane * 16) = e_next;
+                e_next = e_after;
+                if (++e_block < e_end) e_after = load_entries(e_block + 1);
+            }
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int u = 0; u < AF; u++) o.ent[u] = *reinterpret_cast<const uint32_t *>(e_tile + ((first + lane + 64 * u) & 511) * 4); // past the step's end: unused
         }
     };
     auto a_operand = [&](const Operands &o) {
@@ -703,24 +737,25 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
     if (a.accumulate && p.n_split_rows > 0) return hipErrorInvalidValue; // partial tiles through the workspace overwrite C
     // 32-bit byte offsets from indices of 24 bits
     const bool big = a.K > ((size_t)1 << 24) || a.K * (size_t)row_stride * 2 >= ((size_t)1 << 32) || row_stride >= (1L << 23);
-    auto launch = [&](auto af, auto f32, auto acc, auto wide) {
-        hipLaunchKernelGGL((spmm_compact_kernel<TQ, decltype(f32)::value, decltype(acc)::value, decltype(af)::value, decltype(wide)::value>),
+    auto launch = [&](auto af, auto staged, auto f32, auto acc, auto wide) {
+        hipLaunchKernelGGL((spmm_compact_kernel<TQ, decltype(f32)::value, decltype(acc)::value, decltype(af)::value, decltype(staged)::value, decltype(wide)::value>),
                            dim3((unsigned)wgs), dim3(256), 0, st, p.d_acol, p.d_entries, p.d_step_range, cols, a.Bt, a.C, p.d_workspace,
                            p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, (unsigned)xcd_run);
     };
     using std::false_type;
     using std::true_type;
-    auto by_output = [&](auto af, auto wide) {
-        if (a.c_f32) {
-            if (a.accumulate) launch(af, true_type{}, true_type{}, wide); else launch(af, true_type{}, false_type{}, wide);
+    auto by_output = [&](auto af, auto staged, auto wide) {
+        if (a.accumulate) { // never staged
+            if (a.c_f32) launch(af, false_type{}, true_type{}, true_type{}, wide); else launch(af, false_type{}, false_type{}, true_type{}, wide);
         } else {
-            if (a.accumulate) launch(af, false_type{}, true_type{}, wide); else launch(af, false_type{}, false_type{}, wide);
+            if (a.c_f32) launch(af, staged, true_type{}, false_type{}, wide); else launch(af, staged, false_type{}, false_type{}, wide);
         }
     };
+    const bool staged = g_force_staged ? g_force_staged == 1 : (double)p.n_steps * n_panels >= STAGED_STEPS * 16.0 * 256.0;
     auto by_entries = [&](auto wide) {
-        if (p.d_acol) by_output(std::integral_constant<int, 0>{}, wide);
-        else if (p.entries_ahead == 1) by_output(std::integral_constant<int, 1>{}, wide);
-        else by_output(std::integral_constant<int, 2>{}, wide);
+        if (p.d_acol) by_output(std::integral_constant<int, 0>{}, false_type{}, wide);
+        else if (p.entries_ahead == 1) staged ? by_output(std::integral_constant<int, 1>{}, true_type{}, wide) : by_output(std::integral_constant<int, 1>{}, false_type{}, wide);
+        else staged ? by_output(std::integral_constant<int, 2>{}, true_type{}, wide) : by_output(std::integral_constant<int, 2>{}, false_type{}, wide);
     };
     if (big) by_entries(true_type{}); else by_entries(false_type{});
     return hipGetLastError();
@@ -1044,7 +1079,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     if (by_entry) {
         const size_t steps = cap / 32;
         p->entries_ahead = nnz <= 48 * (total / 32) ? 1 : 2; // most steps have no more than 64 a load
-        SMAT_STEP(dev_malloc(&p->d_entries, ((size_t)nnz + 128) * sizeof(uint32_t)));
+        SMAT_STEP(dev_malloc(&p->d_entries, ((size_t)nnz + ENTRY_PAD) * sizeof(uint32_t)));
         SMAT_STEP(dev_malloc(&p->d_step_range, steps * sizeof(int2)));
         SMAT_STEP(hipMemsetAsync(p->d_step_range, 0, steps * sizeof(int2), nullptr)); // the steps read ahead of the last one have no entries
     } else {
@@ -1212,6 +1247,8 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
 extern "C" void smat_internal_compact_panel(int tq) { smat::g_force_tq = tq; }
 // Test hook: 1 = lists of whole columns, 2 = of nonzeros (where their number allows it), 0 = as the sizes say (the default).
 extern "C" void smat_internal_compact_list(int what) { smat::g_force_list = what; }
+// Test hook: 1 = entries go through LDS in blocks of 256 wherever they may, 2 = nowhere, 0 = as the sizes say (the default).
+extern "C" void smat_internal_compact_staged(int what) { smat::g_force_staged = what; }
 // Test hooks for the deal of the compact kernel's workgroups to the XCDs: a run length that every launch uses
 // (0 = chosen per plan and number of panels), the run length of the latest launch, and the choice itself for a list
 // of item costs (host only).
