@@ -59,7 +59,10 @@ constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts
 constexpr int TASK_STEPS = 12;     // short items are put together up to this many steps (8 to 24: level; one item each: 9 % slower on R-MAT)
 constexpr int LONG_ROW_STEPS = 56; // steps from which a block row is split where a launch has few wavefronts
 constexpr size_t PLACE_MIN_BYTES = (size_t)16 << 20; // of B, from which the rows that its copy does not need are looked for
-constexpr double STAGED_STEPS = 20.0; // a place's steps from which entries are staged: of 10 products with 20 and more one was slower, by 0.6 %, of 14 with fewer one faster, by 6 %
+// A place's steps and bytes of the lists from which entries are staged.  Of 9 products with both none was slower; of 14 with fewer
+// steps one would be faster, by 6 %; lists that the L2s hold from panel to panel lose (8192^2, 30 a row, N = 2048 63.7 -> 65.0 us).
+constexpr double STAGED_STEPS = 20.0;
+constexpr int64_t STAGED_BYTES = 4 << 20;
 constexpr int ENTRY_PAD = 1024; // entries readable past the last one (blocks of 256, one ahead, another for the steps past the end of a task)
 constexpr int LIST_PAD = 2304; // entries readable past the end of the list (the index loads of the 64-column panel run up to 16 steps ahead)
 
@@ -448,7 +451,7 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 // Entries (AF > 0) come from memory in the step before they are needed, 256 bytes a load, or, STAGED, 256 at a time ahead of
 // that, one load of 1 KiB to LDS: a load of 256 bytes takes the vector memory path as long as one of 1 KiB, and a list that
 // no cache holds arrives early enough.  That pays where a wavefront's place on the device has many steps to do, before the
-// longer way of the first entries of a task counts (STAGED_STEPS): stencil 64^3, N = 64 57.5 -> 53.3 us, N = 256 186 -> 177; R-MAT
+// longer way of the first entries of a task counts, and where the lists are long (STAGED_STEPS, STAGED_BYTES): stencil 64^3, N = 64 57.5 -> 53.3 us, N = 256 186 -> 177; R-MAT
 // scale 18, N = 64 74.7 -> 69.4, scale 20, N = 128 474 -> 463; but stencil 40^3, N = 64 13.8 -> 15.2; 16384^2, 16 a row, N = 128 10.8 -> 11.6.
 template <int TQ, bool C_F32, bool C_ACC, int AF, bool STAGED, bool BIG>
 __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
@@ -751,7 +754,8 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
             if (a.c_f32) launch(af, staged, true_type{}, false_type{}, wide); else launch(af, staged, false_type{}, false_type{}, wide);
         }
     };
-    const bool staged = g_force_staged ? g_force_staged == 1 : (double)p.n_steps * n_panels >= STAGED_STEPS * 16.0 * 256.0;
+    const bool staged = g_force_staged ? g_force_staged == 1 : (double)p.n_steps * n_panels >= STAGED_STEPS * 16.0 * 256.0 &&
+                                                                p.n_steps * 128 + p.n_entries * 4 >= STAGED_BYTES;
     auto by_entries = [&](auto wide) {
         if (p.d_acol) by_output(std::integral_constant<int, 0>{}, false_type{}, wide);
         else if (p.entries_ahead == 1) staged ? by_output(std::integral_constant<int, 1>{}, true_type{}, wide) : by_output(std::integral_constant<int, 1>{}, false_type{}, wide);
@@ -1078,6 +1082,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     SMAT_STEP(hipMemsetAsync(p->d_cols, 0, cap * sizeof(int32_t), nullptr)); // padding: row 0 of B
     if (by_entry) {
         const size_t steps = cap / 32;
+        p->n_entries = nnz;
         p->entries_ahead = nnz <= 48 * (total / 32) ? 1 : 2; // most steps have no more than 64 a load
         SMAT_STEP(dev_malloc(&p->d_entries, ((size_t)nnz + ENTRY_PAD) * sizeof(uint32_t)));
         SMAT_STEP(dev_malloc(&p->d_step_range, steps * sizeof(int2)));

@@ -109,6 +109,7 @@ struct CompactPlan {
     int n_items = 0, n_tasks = 0, n_split_rows = 0, n_slots = 0;
     int64_t n_steps = 0;          // of 32 columns, of all block rows listed
     int64_t n_cols = 0;           // nonzero block columns listed (without padding)
+    int64_t n_entries = 0;        // nonzeros listed one by one
     int64_t n_cols_all = 0;       // nonzero block columns of the whole matrix
     uint64_t values_checksum = 0; // of the block values the lists were made from
     XcdDeal deal;                 // of the tasks
