@@ -128,18 +128,19 @@ __global__ __launch_bounds__(THREADS) void spmm_sweep_kernel(
     // A workgroup takes the tiles vb = blockIdx.x, blockIdx.x + gridDim.x, ... of the virtual grid n_vb.
     const int total = n_rg * n_panels;
     const int per_xcd = n_vb >> 3;
-    constexpr int RGB = 4;
-    const int n_blk = (n_rg + RGB - 1) / RGB;
+    // (Blocks of 4 and, where 4 does not divide the row groups, of 3: one row group left over would have its panels of B to itself.)
+    const int n_blk = (n_rg + 3) / 4, size = n_rg / n_blk, big = n_rg - n_blk * size; // `big` blocks of size + 1, then those of size
     bool zeros_written = false;
   for (int vb = blockIdx.x; vb < n_vb; vb += gridDim.x) {
     const int tile = (vb & 7) * per_xcd + (vb >> 3);
     if (tile >= total) continue;
-    int gb = tile / (RGB * n_panels);
-    gb = gb < n_blk - 1 ? gb : n_blk - 1;
-    const int rem = tile - gb * RGB * n_panels;
-    const int rgs_here = n_rg - gb * RGB < RGB ? n_rg - gb * RGB : RGB;
+    const bool in_big = tile < big * (size + 1) * n_panels;
+    const int in_part = in_big ? tile : tile - big * (size + 1) * n_panels;
+    const int rgs_here = in_big ? size + 1 : size;
+    const int blk = in_part / (rgs_here * n_panels);
+    const int rem = in_part - blk * rgs_here * n_panels;
     const int pos = rem / rgs_here;
-    const int rg = gb * RGB + rem - pos * rgs_here;
+    const int rg = (in_big ? 0 : big * (size + 1)) + blk * rgs_here + rem - pos * rgs_here;
     // Row-major B: the panels that an XCD has at a time are every other one of 16.  What the device reads at a time is then 128
     // of every 256 bytes of the rows and comes from all memory channels; neighbouring panels would leave out a half of them
     // where the rows are a power of two apart (8192^2, 10 %, N = 4096: 113 -> 103 us, with N = 4032 102 either way).

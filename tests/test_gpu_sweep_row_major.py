@@ -1,4 +1,6 @@
 """Sweep kernel on row-major B read in place: the bits that it writes for the column-major copy of the same B."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -63,3 +65,27 @@ def test_infinities_in_row_major_b_stay_in_their_column(smat, cuda):
     smat.spmm(vals, rpd, cid, Bd, C, mb * 16, N, kb * 16, ci.size, plan=plan, kernel=smat.KERNEL_SWEEP, b_row_major=True)
     torch.cuda.synchronize()
     assert bool(torch.isfinite(C).all())
+
+
+# row groups of fewer than 64 block rows chosen for the rounds (29 to 43): blocks of three and four row groups in the
+# order of the tiles, a last group that is not full
+@pytest.mark.parametrize("mb,N", [(128, 8960), (200, 4136), (321, 2728), (450, 2408)])
+@pytest.mark.parametrize("row_major", [False, True])
+def test_groups_chosen_for_the_rounds_match_the_oracle(smat, cuda, oracle, mb, N, row_major):
+    import torch
+    A = gen.random_bcsr(mb, 40, 0.3, seed=mb)
+    M, K, nnzb = A["M"], A["K"], A["nnzb"]
+    rows = smat.lib.smat_internal_sweep_even_rounds
+    rows.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int]
+    g = rows(A["b_row_ptr"].ctypes.data, A["b_col_idx"].ctypes.data, M, K, N, int(row_major))
+    assert g < 64
+    B = gen.dense_b(K, N, seed=N)
+    vals, rp, ci = (to_dev(torch, x, cuda) for x in (A["b_val"], A["b_row_ptr"].astype(np.int32), A["b_col_idx"].astype(np.int32)))
+    Bd = to_dev(torch, np.ascontiguousarray(B.reshape(N, K).T) if row_major else B, cuda)
+    plan = smat.Plan(A["b_row_ptr"], M, K, nnzb, N, col_idx_host=A["b_col_idx"], b_row_major=row_major)
+    assert plan.info()["kernel"] == smat.KERNEL_SWEEP
+    C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+    smat.spmm(vals, rp, ci, Bd, C, M, N, K, nnzb, plan=plan, b_row_major=row_major)
+    torch.cuda.synchronize()
+    want = oracle.spmm_bcsr(M, N, K, A["b_row_ptr"], A["b_col_idx"], A["b_val"], B, threads=4)
+    assert oracle.compare(C.cpu().numpy().view(np.uint16), want)[0] <= 1e-3
