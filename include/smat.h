@@ -80,18 +80,19 @@ int smat_plan_cache_clear(void);
 #define SMAT_B_COL_MAJOR 0 /* B[n*K + k]: the reference layout               */
 #define SMAT_B_ROW_MAJOR 1 /* B[k*N + n].  The compact kernel reads rows of B and takes this layout in place
                             * (column-major B is first copied row-major into plan scratch on every launch).
-                            * The row-wise and sweep kernels feed the MFMA 8 consecutive k of one column
-                            * per lane: for them a row-major B is first transposed into the reference
-                            * layout in plan scratch (one read and one write of B per launch), which needs
-                            * a plan created with b_layout = SMAT_B_ROW_MAJOR and n_hint >= N; C has the
-                            * same bits as for column-major B */
+                            * So does the sweep kernel, unless many row groups share a large B.  The
+                            * row-wise kernel feeds the MFMA 8 consecutive k of one column per lane: for it
+                            * a row-major B is first transposed into the reference layout in plan scratch
+                            * (one read and one write of B per launch).  Both need a plan created with
+                            * b_layout = SMAT_B_ROW_MAJOR and n_hint >= N; C has the same bits as for
+                            * column-major B through that plan */
 #define SMAT_C_F16 0       /* the reference output type                      */
 #define SMAT_C_F32 1       /* keep the fp32 accumulators                     */
 
 #define SMAT_KERNEL_AUTO 0
 #define SMAT_KERNEL_ROWWISE 1 /* one wavefront per (block-row chunk, N panel), operands straight from L2;
                                * the plan decides whether B is first repacked slab-major into scratch   */
-#define SMAT_KERNEL_SWEEP 2   /* workgroup sweeps K for a group of 64 block rows x 64 columns, B staged in LDS
+#define SMAT_KERNEL_SWEEP 2   /* workgroup sweeps K for a group of up to 64 block rows x 64 columns, B staged in LDS
                                * in chunks of 16 block columns; needs a plan made with col_idx_host, between 2
                                * and 2^23 - 1 blocks and K below 2^28.  SMAT_KERNEL_AUTO takes it when at least
                                * 5% of the blocks exist and (M/1024) x (N/64) workgroups fill the 256 CUs, or

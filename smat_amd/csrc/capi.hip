@@ -284,7 +284,8 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
     }
     // a plan made for a wide N, used with a narrow one: too few workgroups for the sweep kernel
     if (kernel == SMAT_KERNEL_SWEEP && o.kernel == SMAT_KERNEL_AUTO) {
-        const bool in_place = o.b_layout == SMAT_B_ROW_MAJOR && plan->sweep.d_ops_row_major && sweep_takes_row_major(N, K, plan->sweep.n_rg);
+        // whatever the layout of this launch: both give the same bits through one plan
+        const bool in_place = plan->sweep.d_ops_row_major && sweep_takes_row_major(N, K, plan->sweep.n_rg);
         const double row_wise = rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, plan->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN,
                                                     a.b_packed != nullptr) + (in_place ? to_col_major_us(K, N) : 0.0);
         const double factor = in_place ? sweep_in_place_factor(N) : 1.0;

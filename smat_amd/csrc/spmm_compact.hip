@@ -452,7 +452,10 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 // that, one load of 1 KiB to LDS: a load of 256 bytes takes the vector memory path as long as one of 1 KiB, and a list that
 // no cache holds arrives early enough.  That pays where a wavefront's place on the device has many steps to do, before the
 // longer way of the first entries of a task counts, and where the lists are long (STAGED_STEPS, STAGED_BYTES): stencil 64^3, N = 64 57.5 -> 53.3 us, N = 256 186 -> 177; R-MAT
-// scale 18, N = 64 74.7 -> 69.4, scale 20, N = 128 474 -> 463; but stencil 40^3, N = 64 13.8 -> 15.2; 16384^2, 16 a row, N = 128 10.8 -> 11.6.
+// scale 18, N = 64 74.7 -> 69.4, scale 20, N = 128 474 -> 463; but stencil 40^3, N = 64 13.8 -> 15.2; 16384^2, 16 a row, N = 128 10.8 -> 11.6.  The figures are
+// with other inputs in every launch; with the same ones again, the lists still in the memory-side cache, the stencil loses (64^3, N = 64
+// 37.5..40.7 -> 39.8..42.1 us, N = 256 140..144 -> 145) and R-MAT gains as much.  A block asked for on every second step, which makes the
+// waits exact, is slower than one asked for when it is needed (R-MAT scale 20 461 -> 477).
 template <int TQ, bool C_F32, bool C_ACC, int AF, bool STAGED, bool BIG>
 __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const uint16_t *__restrict__ acol, const uint32_t *__restrict__ entries, const int2 *__restrict__ step_range, const int32_t *__restrict__ cols,
