@@ -330,6 +330,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
             SweepArgs w{};
             w.vals = vals; w.B = B; w.C = C; w.M = M; w.N = N; w.K = K; w.nnzb = nnzb; w.c_f32 = a.c_f32;
             plan->sweep_dense.fill(w, sweep_row_major);
+            w.whole = false;
             e = launch_sweep(w, static_cast<hipStream_t>(o.stream));
         } else {
             SpmmArgs d = a;

@@ -77,6 +77,7 @@ struct SweepArgs {
     size_t M, N, K, nnzb;
     bool c_f32;
     bool b_row_major;            // B[k*N + n]; ops are the streams for it
+    bool whole = true;           // every block of vals is multiplied (not so in a plan of some of the block rows)
     const int32_t *rg_chunk_ptr; // device, n_rg + 1: range of the row group in chunk_ids
     const int32_t *chunk_ids;    // device: the K chunks in which the row group has blocks, ascending (+ SWEEP_CHUNK_PAD entries)
     const int32_t *op_ptr;       // device, n_rg * SWEEP_WAVES + 1: range of (row group, wavefront) in ops

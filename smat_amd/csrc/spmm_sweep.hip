@@ -365,9 +365,9 @@ hipError_t launch_sweep(const SweepArgs &a, hipStream_t st)
     // A is touched ahead where the launch before has displaced it: where A, B and C are more than half of the 256 MiB of the
     // memory-side cache.  8192^2, 10 %, N = 4096, inputs changing: 101.5 -> 97.2 us.  With A still in that cache the touches only
     // cost (the same with N = 2048: 42.1 -> 43.2 us; 3088 x 4112, 15 %, N = 1000: 22.7 -> 23.0), and so they do where two per
-    // lane do not reach the end of A (8192^2, 30 %, N = 4096: 202.5 -> 204.6).
+    // lane do not reach the end of A (8192^2, 30 %, N = 4096: 202.5 -> 204.6), and where some rows of A are another kernel's.
     const size_t vals_bytes = a.nnzb * 512, traffic = vals_bytes + a.K * a.N * 2 + a.M * a.N * (a.c_f32 ? 4 : 2);
-    const uint32_t touch_bytes = traffic >= ((size_t)128 << 20) && vals_bytes <= (size_t)launched * THREADS * 128 * 2 ? (uint32_t)vals_bytes : 0;
+    const uint32_t touch_bytes = a.whole && traffic >= ((size_t)128 << 20) && vals_bytes <= (size_t)launched * THREADS * 128 * 2 ? (uint32_t)vals_bytes : 0;
     dim3 grid((unsigned)launched), block(THREADS);
     hipLaunchKernelGGL(kernel, grid, block, lds_bytes, st, a.vals, a.B, a.C, a.rg_chunk_ptr, a.chunk_ids, a.op_ptr, a.ops, a.row_map, (int)a.N,
                        (long)a.K, a.n_rg, n_panels, (uint32_t)vals_bytes, touch_bytes, (int)wgs);
