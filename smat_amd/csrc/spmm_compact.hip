@@ -59,10 +59,14 @@ constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts
 constexpr int TASK_STEPS = 12;     // short items are put together up to this many steps (8 to 24: level; one item each: 9 % slower on R-MAT)
 constexpr int LONG_ROW_STEPS = 56; // steps from which a block row is split where a launch has few wavefronts
 constexpr size_t PLACE_MIN_BYTES = (size_t)16 << 20; // of B, from which the rows that its copy does not need are looked for
-// A place's steps and bytes of the lists from which entries are staged.  Of 9 products with both none was slower; of 14 with fewer
-// steps one would be faster, by 6 %; lists that the L2s hold from panel to panel lose (8192^2, 30 a row, N = 2048 63.7 -> 65.0 us).
+// Entries are staged from so many steps of a place, so many bytes of lists and so many bytes that the product reads and writes. A
+// product that touches less leaves its lists in the memory-side cache (256 MiB) for the next one even where a few matrices take
+// turns, and loads step by step are early enough.  Of 44 products, direct -> staged, three matrices in turn: R-MAT and stencils above the
+// lines gain 2 to 7 % (row-major B 48^3, N = 256 loses 2), uniform rows 0 to 14 %; below the third line: 54336 x 5408, 31 a row, N = 192 46.2 -> 47.8 us, N = 768
+// 119.9 -> 122.1; 8192 x 65536, 60 a row, N = 256 28.9 -> 30.7; stencil 56^3, N = 96, row-major 44.2 -> 46.7 (but 65536^2, 16 a row, N = 192 53.6 -> 51.5).
 constexpr double STAGED_STEPS = 20.0;
 constexpr int64_t STAGED_BYTES = 4 << 20;
+constexpr int64_t STAGED_TOUCHED = 112 << 20, STAGED_TOUCHED_IN_PLACE = 100 << 20; // with a copy of B, which is touched too, and without
 constexpr int ENTRY_PAD = 1024; // entries readable past the last one (blocks of 256, one ahead, another for the steps past the end of a task)
 constexpr int LIST_PAD = 2304; // entries readable past the end of the list (the index loads of the 64-column panel run up to 16 steps ahead)
 
@@ -451,7 +455,7 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 // Entries (AF > 0) come from memory in the step before they are needed, 256 bytes a load, or, STAGED, 256 at a time ahead of
 // that, one load of 1 KiB to LDS: a load of 256 bytes takes the vector memory path as long as one of 1 KiB, and a list that
 // no cache holds arrives early enough.  That pays where a wavefront's place on the device has many steps to do, before the
-// longer way of the first entries of a task counts, and where the lists are long (STAGED_STEPS, STAGED_BYTES): stencil 64^3, N = 64 57.5 -> 53.3 us, N = 256 186 -> 177; R-MAT
+// longer way of the first entries of a task counts, and where the lists are long and come from far (STAGED_STEPS, STAGED_BYTES, STAGED_TOUCHED): stencil 64^3, N = 64 57.5 -> 53.3 us, N = 256 186 -> 177; R-MAT
 // scale 18, N = 64 74.7 -> 69.4, scale 20, N = 128 474 -> 463; but stencil 40^3, N = 64 13.8 -> 15.2; 16384^2, 16 a row, N = 128 10.8 -> 11.6.  The figures are
 // with other inputs in every launch; with the same ones again, the lists still in the memory-side cache, the stencil loses (64^3, N = 64
 // 37.5..40.7 -> 39.8..42.1 us, N = 256 140..144 -> 145) and R-MAT gains as much.  A block asked for on every second step, which makes the
@@ -757,8 +761,10 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
             if (a.c_f32) launch(af, staged, true_type{}, false_type{}, wide); else launch(af, staged, false_type{}, false_type{}, wide);
         }
     };
-    const bool staged = g_force_staged ? g_force_staged == 1 : (double)p.n_steps * n_panels >= STAGED_STEPS * 16.0 * 256.0 &&
-                                                                p.n_steps * 128 + p.n_entries * 4 >= STAGED_BYTES;
+    const int64_t list_bytes = p.n_steps * 128 + p.n_entries * 4, b_bytes = (int64_t)a.K * a.N * 2, c_bytes = (int64_t)a.M * a.N * (a.c_f32 ? 4 : 2);
+    const bool staged = g_force_staged ? g_force_staged == 1
+                                       : (double)p.n_steps * n_panels >= STAGED_STEPS * 16.0 * 256.0 && list_bytes >= STAGED_BYTES &&
+                                             list_bytes + c_bytes + (a.b_row_major ? b_bytes : 2 * b_bytes) >= (a.b_row_major ? STAGED_TOUCHED_IN_PLACE : STAGED_TOUCHED);
     auto by_entries = [&](auto wide) {
         if (p.d_acol) by_output(std::integral_constant<int, 0>{}, false_type{}, wide);
         else if (p.entries_ahead == 1) staged ? by_output(std::integral_constant<int, 1>{}, true_type{}, wide) : by_output(std::integral_constant<int, 1>{}, false_type{}, wide);
