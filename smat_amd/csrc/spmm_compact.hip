@@ -58,7 +58,10 @@ int g_force_tq = 0; // test hook: 1 or 2 = panels of 64 or 128 columns whatever 
 constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts as full (of 16)
 constexpr int TASK_STEPS = 12;     // short items are put together up to this many steps (8 to 24: level; one item each: 9 % slower on R-MAT)
 constexpr int LONG_ROW_STEPS = 56; // steps from which a block row is split where a launch has few wavefronts
-constexpr size_t PLACE_MIN_BYTES = (size_t)16 << 20; // of B, from which the rows that its copy does not need are looked for
+// Bytes of B that its copy has to leave out, and an eighth of B: less does not pay for the place of every row, which the transposition
+// has to know (copy of all rows -> of those that are used, N = 256: 2000 x 40000, 40 a row, 2.8 MB left out 17.0 -> 17.9 us; 14 a row, 10 MB 13.2 -> 13.4;
+// 6 a row, 15 MB 11.9 -> 11.4; N = 512, 32768 x 65536, 3.5 a row, 11.6 MB 52.4 -> 49.9; N = 1000, 4096 x 65536, 10 a row, 60 MB 72.5 -> 55.2).
+constexpr size_t PLACE_MIN_BYTES = (size_t)21 << 19;
 // Entries are staged from so many steps of a place, so many bytes of lists and so many bytes that the product reads and writes. A
 // product that touches less leaves its lists in the memory-side cache (256 MiB) for the next one even where a few matrices take
 // turns, and loads step by step are early enough.  Of 44 products, direct -> staged, three matrices in turn: R-MAT and stencils above the
@@ -1014,7 +1017,7 @@ static bool lists_nonzeros(int64_t nnz, int64_t n_cols, size_t n_rows, size_t N)
 // the gathers: N = 128 transposition 101 -> 94 us, product 469 -> 401; scale 18, N = 256 226 -> 211, both together; scale 16 equal.
 // With the rows that most columns meet in front the gathers take as long.  Not looked for below 16 MiB, where the
 // transposition is little more than a launch, nor where the plan is made for row-major B, which is read in place.
-static hipError_t place_rows(CompactPlan &p, size_t K, long total)
+static hipError_t place_rows(CompactPlan &p, size_t K, size_t n_cap, long total)
 {
     hipError_t e = hipSuccess;
     Scratch used, before, tmp;
@@ -1032,7 +1035,7 @@ static hipError_t place_rows(CompactPlan &p, size_t K, long total)
     SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, (int32_t *)used.p, (int32_t *)before.p, (int)(K + 1)));
     int32_t n = 0;
     SMAT_STEP(hipMemcpy(&n, (int32_t *)before.p + K, sizeof n, hipMemcpyDeviceToHost));
-    if (e != hipSuccess || (size_t)n > K / 8 * 7) return e;
+    if (e != hipSuccess || (size_t)n > K / 8 * 7 || (K - (size_t)n) * n_cap * sizeof(uint16_t) < PLACE_MIN_BYTES) return e;
     const long padded = total + LIST_PAD;
     SMAT_STEP(dev_malloc(&p.d_place, K * sizeof(int32_t)));
     SMAT_STEP(dev_malloc(&p.d_cols_placed, (size_t)padded * sizeof(int32_t)));
@@ -1161,7 +1164,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
             }
         }
     }
-    if (e == hipSuccess && total > 0 && !b_row_major && K * n_cap * sizeof(uint16_t) >= PLACE_MIN_BYTES) e = place_rows(*p, K, (long)total);
+    if (e == hipSuccess && total > 0 && !b_row_major && K * n_cap * sizeof(uint16_t) >= PLACE_MIN_BYTES) e = place_rows(*p, K, n_cap, (long)total);
     // Work items: whole block rows; rows much longer than the average in chunks of 32-column steps, all of a row's about
     // as long.  Long rows that are all alike stay whole: their partial tiles are 2 * 16 * N floats to write and read again
     // for each (32768 x 65536, 131 a row, N = 256: 138 us whole, 191 in chunks of 1792 columns; 8192 x 65536, 140 a row,
