@@ -1178,7 +1178,9 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     //   scale 16, N = 128, 15:                14 34.7, 21 32.4, 28 32.9, 56 41.5
     //   scale 14, N = 128, 4:                 7 17.1, 14 17.6, 21 18.5, 28 20.0, 56 28.8
     // The rule, 16 steps and 0.38 of those of a place, against four times the average in every launch, as before: scale 20 520 -> 488,
-    // scale 13, N = 256 19.1 -> 16.1; of 24 R-MAT products two are slower, by 2 %.  Whether a list is split at all, which costs a launch, is decided by four
+    // scale 13, N = 256 19.1 -> 16.1.  With one panel, as many steps as a
+    // place has: N = 64, four times the average / 0.38 / 1.0: scale 15 19.4 / 17.1 / 17.9, 17 34.5 / 36.4 / 34.3, 18 76.2 / 69.6 / 67.1; N = 16, scale 19
+    // 98.0 / - / 93.3.  Whether a list is split at all, which costs a launch, is decided by four
     // times the average and 16 steps, or the chunk where that is longer.
     const std::vector<int32_t> &cc_host = padded;
     size_t nonempty = 0;
@@ -1190,7 +1192,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     }
     const double avg = nonempty ? (double)total / (double)nonempty : 0.0;
     const double steps_a_place = (double)(total / 32) * (double)((n_cap + 63) / 64) / (16.0 * 256.0);
-    const double share = n_cap < 64 ? 0.8 : 0.38; // narrow: a step brings less, and a partial tile takes a store all the same
+    const double share = n_cap <= 64 ? 1.0 : 0.38; // one panel: see above
     long chunk = 32 * (long)(std::max(16.0 + share * steps_a_place, 2.5 * avg / 32.0) + 0.5);
     const long from = std::max((long)(4.0 * avg + 0.5), 512L);
     if (longest <= from) chunk = std::max(chunk, from);
