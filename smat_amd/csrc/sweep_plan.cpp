@@ -7,11 +7,8 @@
 #include <cstring>
 #include <functional>
 #include <queue>
-#include <utility>
-
-#include <emmintrin.h>
-
 #include <stdexcept>
+#include <utility>
 
 #include "../../include/smat.h"
 #include "errors.h"
@@ -23,6 +20,11 @@ namespace {
 constexpr int G = SWEEP_G, RW = SWEEP_RW, WAVES = SWEEP_WAVES, S = SWEEP_S, MIN_OPS = SWEEP_MIN_OPS;
 constexpr int AHEAD = SWEEP_AHEAD, COPIES = SWEEP_COPIES;
 constexpr int VM_MARK = MIN_OPS; // a chunk boundary waits until at most this many vector memory operations are under way
+// Eight counters of 16 bits, by the compiler's vector types: a register wherever the host has one of 128 bits.
+typedef int16_t Counters __attribute__((vector_size(16)));
+inline Counters smaller(Counters a, Counters b) { return a < b ? a : b; }
+inline Counters larger(Counters a, Counters b) { return a > b ? a : b; }
+
 // Sum of the cheapest caps of the periods (see build_sweep_plan) for the assignment win, n periods, with rows ri of wavefront wi
 // and rj of wavefront wj changed over (ri NULL: none); LONG_MAX as soon as it cannot be below `below`.  The eight wavefronts are the
 // eight 16-bit lanes of a register: a plan tries thousands of such changes a row group and this is nearly all of its time
@@ -30,39 +32,38 @@ constexpr int VM_MARK = MIN_OPS; // a chunk boundary waits until at most this ma
 long sum_of_caps(const int16_t *win, size_t n, const int16_t *ri, const int16_t *rj, int wi, int wj, long below, int32_t *caps_out)
 {
     static_assert(WAVES == 8 && RW * 3 * S < 32768, "a wavefront's ops of three chunks, in a lane of 16 bits");
-    alignas(16) int16_t sign_of[WAVES] = {0};
-    if (ri) sign_of[wi] = -1, sign_of[wj] = 1;
-    const __m128i sign = _mm_load_si128((const __m128i *)sign_of), zero = _mm_setzero_si128();
-    __m128i due = zero, next = zero; // pending ops with deadline p - at the start of period p - and p + 1
+    const Counters zero = {0, 0, 0, 0, 0, 0, 0, 0}, halves = {4, 5, 6, 7, 0, 1, 2, 3}, pairs = {2, 3, 0, 1, 6, 7, 4, 5}, ones = {1, 0, 3, 2, 5, 4, 7, 6};
+    Counters sign = zero;
+    if (ri) sign[wi] = -1, sign[wj] = 1;
+    Counters due = zero, next = zero; // pending ops with deadline p - at the start of period p - and p + 1
     long sum = 0, rest = (long)n * MIN_OPS; // what the periods to come cost at least
     for (size_t p = 0; p < n; p++) {
-        __m128i c[3];
+        Counters c[3];
         for (size_t len = 0; len < 3; len++) {
             const size_t x = p * 3 + len;
-            c[len] = _mm_loadu_si128((const __m128i *)(win + x * WAVES));
-            if (ri) c[len] = _mm_add_epi16(c[len], _mm_mullo_epi16(sign, _mm_set1_epi16((int16_t)(ri[x] - rj[x]))));
+            memcpy(&c[len], win + x * WAVES, sizeof(Counters));
+            if (ri) c[len] += sign * (int16_t)(ri[x] - rj[x]);
         }
-        const __m128i p0 = _mm_add_epi16(due, c[0]), p1 = _mm_add_epi16(next, c[1]), p2 = c[2];
-        __m128i cap = _mm_max_epi16(p0, _mm_shuffle_epi32(p0, _MM_SHUFFLE(1, 0, 3, 2)));
-        cap = _mm_max_epi16(cap, _mm_shuffle_epi32(cap, _MM_SHUFFLE(2, 3, 0, 1)));
-        cap = _mm_max_epi16(cap, _mm_shufflehi_epi16(_mm_shufflelo_epi16(cap, _MM_SHUFFLE(2, 3, 0, 1)), _MM_SHUFFLE(2, 3, 0, 1)));
-        cap = _mm_max_epi16(cap, _mm_set1_epi16((int16_t)MIN_OPS));
-        const int32_t cap_p = (int16_t)_mm_extract_epi16(cap, 0);
+        const Counters p0 = due + c[0], p1 = next + c[1], p2 = c[2];
+        Counters cap = larger(p0, __builtin_shuffle(p0, halves)); // the largest of the eight, in all of them
+        cap = larger(cap, __builtin_shuffle(cap, pairs));
+        cap = larger(cap, __builtin_shuffle(cap, ones));
+        cap = larger(cap, zero + (int16_t)MIN_OPS);
+        const int32_t cap_p = cap[0];
         sum += cap_p;
         rest -= MIN_OPS;
         if (sum + rest >= below) return LONG_MAX;
         if (caps_out) caps_out[p] = cap_p;
         // the ops due now run; what is left of the cap goes to the next deadlines, but the last pending op stays for the next
         // period when it may (see the schedule in build_sweep_plan)
-        __m128i room = _mm_sub_epi16(cap, p0);
+        Counters room = cap - p0;
         if (p + 1 < n) {
-            const __m128i pending = _mm_add_epi16(p1, p2);
-            const __m128i keep_one = _mm_andnot_si128(_mm_cmpgt_epi16(pending, room), _mm_cmpgt_epi16(pending, zero));
-            room = _mm_or_si128(_mm_andnot_si128(keep_one, room), _mm_and_si128(keep_one, _mm_sub_epi16(pending, _mm_set1_epi16(1))));
+            const Counters pending = p1 + p2;
+            room = (pending > zero) & (pending <= room) ? pending - (int16_t)1 : room;
         }
-        const __m128i r1 = _mm_min_epi16(room, p1);
-        due = _mm_sub_epi16(p1, r1);
-        next = _mm_sub_epi16(p2, _mm_min_epi16(_mm_sub_epi16(room, r1), p2));
+        const Counters r1 = smaller(room, p1);
+        due = p1 - r1;
+        next = p2 - smaller(room - r1, p2);
     }
     return sum;
 }
