@@ -62,11 +62,13 @@ constexpr int LONG_ROW_STEPS = 56; // steps from which a block row is split wher
 // has to know (copy of all rows -> of those that are used, N = 256: 2000 x 40000, 40 a row, 2.8 MB left out 17.0 -> 17.9 us; 14 a row, 10 MB 13.2 -> 13.4;
 // 6 a row, 15 MB 11.9 -> 11.4; N = 512, 32768 x 65536, 3.5 a row, 11.6 MB 52.4 -> 49.9; N = 1000, 4096 x 65536, 10 a row, 60 MB 72.5 -> 55.2).
 constexpr size_t PLACE_MIN_BYTES = (size_t)21 << 19;
-// Entries are staged from so many steps of a place, so many bytes of lists and so many bytes that the product reads and writes. A
-// product that touches less leaves its lists in the memory-side cache (256 MiB) for the next one even where a few matrices take
-// turns, and loads step by step are early enough.  Of 44 products, direct -> staged, three matrices in turn: R-MAT and stencils above the
-// lines gain 2 to 7 % (row-major B 48^3, N = 256 loses 2), uniform rows 0 to 14 %; below the third line: 54336 x 5408, 31 a row, N = 192 46.2 -> 47.8 us, N = 768
-// 119.9 -> 122.1; 8192 x 65536, 60 a row, N = 256 28.9 -> 30.7; stencil 56^3, N = 96, row-major 44.2 -> 46.7 (but 65536^2, 16 a row, N = 192 53.6 -> 51.5).
+// Entries are staged where a wavefront's place on the device has many steps to do (before the longer way of the first entries of a task
+// counts: 16384^2, 16 a row, N = 128 10.9 -> 11.5 us), where the lists are longer than the L2s hold, and where the product touches
+// nearly half of the memory-side cache of 256 MiB or more.  Whether A is still in that cache when it is multiplied again follows
+// from what the program does in between, which nothing here can know.  What is taken: products below the third line, two of which
+// fit side by side, find their lists there again as a rule, larger ones do not.  In the figures beside the kernel a
+// larger product gains 7 to 10 % where its lists do come from HBM and loses 0 to 4 % where they do not (row-major B 6 and 6 %); a smaller one would gain 2 to 7 and
+// lose 0 to 7.
 constexpr double STAGED_STEPS = 20.0;
 constexpr int64_t STAGED_BYTES = 4 << 20;
 constexpr int64_t STAGED_TOUCHED = 112 << 20, STAGED_TOUCHED_IN_PLACE = 100 << 20; // with a copy of B, which is touched too, and without
@@ -457,12 +459,19 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 //
 // Entries (AF > 0) come from memory in the step before they are needed, 256 bytes a load, or, STAGED, 256 at a time ahead of
 // that, one load of 1 KiB to LDS: a load of 256 bytes takes the vector memory path as long as one of 1 KiB, and a list that
-// no cache holds arrives early enough.  That pays where a wavefront's place on the device has many steps to do, before the
-// longer way of the first entries of a task counts, and where the lists are long and come from far (STAGED_STEPS, STAGED_BYTES, STAGED_TOUCHED): stencil 64^3, N = 64 57.5 -> 53.3 us, N = 256 186 -> 177; R-MAT
-// scale 18, N = 64 74.7 -> 69.4, scale 20, N = 128 474 -> 463; but stencil 40^3, N = 64 13.8 -> 15.2; 16384^2, 16 a row, N = 128 10.8 -> 11.6.  The figures are
-// with other inputs in every launch; with the same ones again, the lists still in the memory-side cache, the stencil loses (64^3, N = 64
-// 37.5..40.7 -> 39.8..42.1 us, N = 256 140..144 -> 145) and R-MAT gains as much.  A block asked for on every second step, which makes the
-// waits exact, is slower than one asked for when it is needed (R-MAT scale 20 461 -> 477).
+// comes from HBM arrives early enough.  A list that the memory-side cache still holds comes early enough either way, and
+// then the trip through LDS costs a few percent where columns hold several nonzeros.  Direct / staged, us: with everything
+// flushed before every launch; three matrices in turn; the same A with another B and C; the same everything:
+//   stencil 64^3, N = 64           74.7/68.4   57.5/52.8   40.6/42.3   37.8/39.5
+//   64^3, N = 64, row-major B                  38.1/35.7   26.5/28.2   26.8/28.0
+//   64^3, N = 128                              103.5/94.3  77.5/79.5   68.9/71.7
+//   R-MAT scale 18, N = 64                     72.3/67.5   57.5/57.0   57.3/56.8
+//   scale 20, N = 128                          474/458     474/457     474/457
+//   65536^2, 16 a row, N = 192     64.4/61.3   53.6/52.4   55.4/55.1   55.5/55.0
+//   stencil 48^3, N = 128          55.9/52.4   40.1/39.9   34.6/37.1   34.7/37.1
+//   8192 x 32768, 60 a row, N = 512 56.5/54.8  40.3/41.0   41.5/43.1   41.6/43.1
+// The launcher's rule is at STAGED_STEPS.  A block asked for on every second step, which makes all waits exact, is slower than one
+// asked for when it is needed (R-MAT scale 20 461 -> 477).
 template <int TQ, bool C_F32, bool C_ACC, int AF, bool STAGED, bool BIG>
 __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const uint16_t *__restrict__ acol, const uint32_t *__restrict__ entries, const int2 *__restrict__ step_range, const int32_t *__restrict__ cols,
@@ -546,17 +555,26 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     auto load_block = [&](int s) { return reinterpret_cast<const u32x4 *>(cols + s)[lane]; };
     auto put_block = [&](int s, u32x4 x) { *reinterpret_cast<u32x4 *>(i_tile + (((s >> 5) - first_step) & 8) * 128 + lane * 16) = x; };
     auto indices = [&](int s) { return *reinterpret_cast<const u32x4 *>(i_tile + (((s >> 5) - first_step) & 15) * 128 + oct * 16); };
-    // Entries the same way: 256 of them, 1 KiB, a load, to one half of 2 KiB of LDS; the next 256 are on their way meanwhile.
+    // Entries the same way: 256 of them, 1 KiB, a load, to one half of 2 KiB of LDS.  A block goes there when the first step that
+    // needs it is asked for, and the one after it is loaded into the same registers then.  (Two blocks in registers, the further one moved
+    // down, was every load in flight waited for at each move: the compiler's count of what is younger than a load that only some
+    // steps make is zero where its registers are copied.  Waited for so -> as here: stencil 64^3, N = 64 53.3 -> 52.8 us with inputs from
+    // HBM, 40.6 -> 39.5 with the same ones again; N = 128 97 -> 94; 48^3, N = 256 78 -> 74; R-MAT scale 20, N = 128 461.7 -> 458.4;
+    // 65536^2, 40 a row, N = 192 101.7 -> 102.9.)
     unsigned char *const e_tile = lds[wave] + A_BYTES + B_BYTES + I_BYTES;
-    u32x4 e_next = {0u, 0u, 0u, 0u}, e_after = {0u, 0u, 0u, 0u};
+    u32x4 e_next = {0u, 0u, 0u, 0u};
     int e_block = 0, e_end = 0; // of 256 entries: the one in e_next, and the last of the task as far as its ranges are here
     auto load_entries = [&](int b) { return reinterpret_cast<const u32x4 *>(entries)[(long)b * 64 + lane]; };
+    auto put_entries = [&](int b, u32x4 x) { *reinterpret_cast<u32x4 *>(e_tile + (b & 1) * 1024 + lane * 16) = x; };
+    u32x4 e_first = {0u, 0u, 0u, 0u}, e_second = {0u, 0u, 0u, 0u};
     if constexpr (STAGED) {
-        e_block = __builtin_amdgcn_readlane(ranges.x, 0) >> 8;
+        const int b = __builtin_amdgcn_readlane(ranges.x, 0) >> 8;
         const int steps = (e_last >> 5) - first_step;
         e_end = steps > 64 ? 0x7fffffff : (__builtin_amdgcn_readlane(ranges.y, steps > 0 ? steps - 1 : 0) - 1) >> 8;
-        e_next = load_entries(e_block);
-        e_after = load_entries(e_block + 1);
+        e_first = load_entries(b);
+        e_second = load_entries(b + 1);
+        e_block = b + 2;
+        if (e_block <= e_end) e_next = load_entries(e_block);
     }
     auto request = [&](int s, const u32x4 x, Operands &o) {
         if constexpr (AF == 0) {
@@ -585,11 +603,11 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
         if constexpr (STAGED) {
             const int first = __builtin_amdgcn_readlane(ranges.x, (s >> 5) - range_from);
             o.n = __builtin_amdgcn_readlane(ranges.y, (s >> 5) - range_from) - first;
-            // a step has at most 128 entries: one more block, two for the first step of a task
-            for (int k = 0; k < 2 && (first + o.n - 1) >> 8 >= e_block; k++) {
-                *reinterpret_cast<u32x4 *>(e_tile + (e_block & 1) * 1024 + lane * 16) = e_next;
-                e_next = e_after;
-                if (++e_block < e_end) e_after = load_entries(e_block + 1);
+            // a step has at most 128 entries, which lie in the last block that is in LDS or reach into the one in e_next
+            if ((first + o.n - 1) >> 8 >= e_block) {
+                put_entries(e_block, e_next);
+                e_block++;
+                if (e_block <= e_end) e_next = load_entries(e_block);
             }
             asm volatile("" ::: "memory");
 #pragma unroll
@@ -682,6 +700,10 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     u32x4 block = load_block(e); // of the 8 steps after those in LDS
     put_block(e, block);
     block = load_block(e + 256);
+    if constexpr (STAGED) {
+        put_entries(e_block, e_first); // blocks e_block - 2
+        put_entries(e_block + 1, e_second); // and e_block - 1
+    }
     asm volatile("" ::: "memory");
     request(e, indices(e), op_a);
     int next = e + 32; // the step whose operands are asked for
