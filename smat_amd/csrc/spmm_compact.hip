@@ -1070,6 +1070,34 @@ static hipError_t place_rows(CompactPlan &p, size_t K, size_t n_cap, long total)
     return e;
 }
 
+// Steps of the chunks that long block rows are cut into, for a list of `steps` steps in `rows` block rows, the longest of `longest`
+// steps, and products of n_cap columns.
+//
+// What a wavefront's place on the device does in a launch (steps and panels over 16 places a CU) bounds the time that one chunk may
+// take, and the partial tiles ask for long ones.  Chunks are the first items of a panel, so one that takes as long as its panel
+// ends with it, and where several panels follow each other it may take longer.  Steps of a chunk, us (R-MAT, 16 a row, avg 7 steps):
+//   scale 20, N = 128, 240 steps a place:  14 607, 28 512, 56 486, 112 458, 224 480
+//   scale 19, N = 128, 120:                14 268, 28 236, 56 221, 112 225, 224 234
+//   scale 18, N = 256, 120:                14 248, 28 207, 56 196, 112 211
+//   scale 18, N = 64, 30:                  14 79.0, 28 68.7, 56 65.3, 112 80.0
+//   scale 17, N = 1024, 240:               14 477, 28 385, 56 359, 112 378
+//   scale 16, N = 128, 15:                 14 35.5, 28 33.0, 56 42.2
+//   scale 14, N = 128, 4:                  14 17.8, 28 20.5, 56 32.0
+// Taken: 16 steps and those that a place has in one panel, or 0.38 of what it has in all, whichever is more; with 0.38 alone two panels take longer
+// (scale 20, N = 128 461 against 457, scale 19 217 against 213), with those of one panel alone many do (scale 17, N = 1024 377 against 359).
+// Whether a list is split at all, which costs a launch: where its longest row has more than four times the average, and more than 16
+// steps, and more than a chunk.
+static long split_chunk_steps(long steps, size_t rows, long longest, size_t n_cap)
+{
+    const size_t panels = (n_cap + 63) / 64;
+    const double avg = rows ? (double)steps / (double)rows : 0.0, one_panel = (double)steps / (16.0 * 256.0);
+    long chunk = (long)(std::max(16.0 + std::max(one_panel, 0.38 * one_panel * (double)panels), 2.5 * avg) + 0.5);
+    const long from = std::max((long)(4.0 * avg), 16L);
+    if (longest <= from) chunk = std::max(chunk, from);
+    if (rows * panels < 1024) chunk = std::min(chunk, (long)LONG_ROW_STEPS);
+    return chunk;
+}
+
 hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx, size_t K, size_t n_cap,
                          bool b_row_major, const std::vector<uint8_t> *leave_rows, bool drop_full, CompactPlan **out)
 {
@@ -1192,18 +1220,6 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     // for each (32768 x 65536, 131 a row, N = 256: 138 us whole, 191 in chunks of 1792 columns; 8192 x 65536, 140 a row,
     // N = 1024: 175 against 241) - except where whole rows would be fewer than four wavefronts a CU (2048 x 65536, 140 a row,
     // N = 256, 512 wavefronts: 43 us whole, 34 in halves; 512 x 65536, 300 a row, N = 1024, 512 of them: 96 against 75).
-    // How long a chunk: what a wavefront's place on the device does in a launch (steps and panels over 16 places a CU) bounds the
-    // time that one chunk may take, and the partial tiles ask for long ones.  Steps of a chunk, us (R-MAT, 16 a row, avg 7 steps):
-    //   scale 20, N = 128, 240 steps a place: 14 605, 28 519, 56 488, 112 483
-    //   scale 18, N = 256, 120:               14 242, 28 211, 56 203, 84 211, 112 216
-    //   scale 17, N = 256, 60:                14 130, 21 107, 28 104, 56 110
-    //   scale 16, N = 128, 15:                14 34.7, 21 32.4, 28 32.9, 56 41.5
-    //   scale 14, N = 128, 4:                 7 17.1, 14 17.6, 21 18.5, 28 20.0, 56 28.8
-    // The rule, 16 steps and 0.38 of those of a place, against four times the average in every launch, as before: scale 20 520 -> 488,
-    // scale 13, N = 256 19.1 -> 16.1.  With one panel, as many steps as a
-    // place has: N = 64, four times the average / 0.38 / 1.0: scale 15 19.4 / 17.1 / 17.9, 17 34.5 / 36.4 / 34.3, 18 76.2 / 69.6 / 67.1; N = 16, scale 19
-    // 98.0 / - / 93.3.  Whether a list is split at all, which costs a launch, is decided by four
-    // times the average and 16 steps, or the chunk where that is longer.
     const std::vector<int32_t> &cc_host = padded;
     size_t nonempty = 0;
     long longest = 0;
@@ -1212,13 +1228,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         nonempty += len > 0;
         if (!dense[i]) longest = std::max(longest, len);
     }
-    const double avg = nonempty ? (double)total / (double)nonempty : 0.0;
-    const double steps_a_place = (double)(total / 32) * (double)((n_cap + 63) / 64) / (16.0 * 256.0);
-    const double share = n_cap <= 64 ? 1.0 : 0.38; // one panel: see above
-    long chunk = 32 * (long)(std::max(16.0 + share * steps_a_place, 2.5 * avg / 32.0) + 0.5);
-    const long from = std::max((long)(4.0 * avg + 0.5), 512L);
-    if (longest <= from) chunk = std::max(chunk, from);
-    if (nonempty * ((n_cap + 63) / 64) < 1024) chunk = std::min(chunk, 32L * LONG_ROW_STEPS);
+    const long chunk = 32 * split_chunk_steps((long)(total / 32), nonempty, longest / 32, n_cap);
     std::vector<WorkItem> items;
     std::vector<SplitRow> split;
     int slot = 0;
@@ -1290,6 +1300,8 @@ extern "C" void smat_internal_compact_panel(int tq) { smat::g_force_tq = tq; }
 extern "C" void smat_internal_compact_list(int what) { smat::g_force_list = what; }
 // Test hook: 1 = entries go through LDS in blocks of 256 wherever they may, 2 = nowhere, 0 = as the sizes say (the default).
 extern "C" void smat_internal_compact_staged(int what) { smat::g_force_staged = what; }
+// Test hook (host only): steps of the chunks of split rows.
+extern "C" long smat_internal_compact_chunk(long steps, size_t rows, long longest, size_t n_cap) { return smat::split_chunk_steps(steps, rows, longest, n_cap); }
 // Test hooks for the deal of the compact kernel's workgroups to the XCDs: a run length that every launch uses
 // (0 = chosen per plan and number of panels), the run length of the latest launch, and the choice itself for a list
 // of item costs (host only).
