@@ -58,9 +58,12 @@ int g_force_tq = 0; // test hook: 1 or 2 = panels of 64 or 128 columns whatever 
 constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts as full (of 16)
 constexpr int TASK_STEPS = 12;     // short items are put together up to this many steps (8 to 24: level; one item each: 9 % slower on R-MAT)
 constexpr int LONG_ROW_STEPS = 56; // steps from which a block row is split where a launch has few wavefronts
-// Bytes of B that its copy has to leave out, and an eighth of B: less does not pay for the place of every row, which the transposition
-// has to know (copy of all rows -> of those that are used, N = 256: 2000 x 40000, 40 a row, 2.8 MB left out 17.0 -> 17.9 us; 14 a row, 10 MB 13.2 -> 13.4;
-// 6 a row, 15 MB 11.9 -> 11.4; N = 512, 32768 x 65536, 3.5 a row, 11.6 MB 52.4 -> 49.9; N = 1000, 4096 x 65536, 10 a row, 60 MB 72.5 -> 55.2).
+// Bytes of B that its copy has to leave out, and an eighth of B.  The place of every row, which the transposition has to read, costs 0.2 to 0.9 us
+// where nothing else changes; what is left out is not written (1 us for about 6 MB where B comes from HBM) and not between the gathered
+// rows, which counts from some 20 MB on.  70 products (uniform rows and R-MAT, K 8,192 to 1,048,576, N 16 to 1,008), copy of all rows -> of the used ones: from
+// 11 MB on none is slower in any mode, with inputs taking turns from equal (3792 x 46784, 8 a row, N = 280, 14 MB 16.7 -> 16.7 us) over 20.8 -> 17.9
+// (1264 x 35568, 10 a row, N = 480, 24 MB) to 213 -> 163 (17392 x 150672, 5 a row, N = 912, 148 MB).  Between 5 and 11 MB 14.6 -> 15.4 (13680 x 110544, 5 a
+// row, N = 72, 9 MB) to 55.2 -> 51.1 (R-MAT scale 17, N = 72, 8 MB); below 5 MB 17.5 -> 18.4 (5888 x 76192, 27 a row, N = 112, 2 MB) to 35.8 -> 35.2.
 constexpr size_t PLACE_MIN_BYTES = (size_t)21 << 19;
 // Entries are staged where a wavefront's place on the device has many steps to do (before the longer way of the first entries of a task
 // counts: 16384^2, 16 a row, N = 128 10.9 -> 11.5 us), where the lists are longer than the L2s hold, and where the product touches
