@@ -221,7 +221,8 @@ __device__ __forceinline__ long row_of_block(const int32_t *__restrict__ row_ptr
 // the padded list, and
 //   acol != NULL: their 16 values each to acol, in MFMA operand order;
 //   else: their nonzeros to entries from entry_start[br] + (nonzeros of the block row before) on, column by column,
-//         each with its place in the operand of its step, and the range of entries of every step to step_range.
+//         each with its place in the operand of its step, and the range of entries of every step to step_range;
+//   used != NULL: used[row] = 1 for the rows of B that the list names.
 // A wavefront takes GATHER_BLOCKS consecutive blocks, four at a time: lane (g = lane / 16, r = lane % 16) holds row r of one.
 // Bound by the second read of the values.  (One thread per block read them 2 bytes at a time, 64 cache lines a load, behind a
 // search of ten loads one after the other: 237 k blocks 54 -> 35 us;
@@ -231,7 +232,7 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint16_t *__restrict_
                               const unsigned long long *__restrict__ offset, const int32_t *__restrict__ row_ptr,
                               const int32_t *__restrict__ col_idx, const unsigned long long *__restrict__ raw,
                               const int2 *__restrict__ start, long mb, long nnzb, bool drop_full, int32_t *__restrict__ cols,
-                              uint16_t *__restrict__ acol, uint32_t *__restrict__ entries, int2 *__restrict__ step_range)
+                              uint16_t *__restrict__ acol, uint32_t *__restrict__ entries, int2 *__restrict__ step_range, uint8_t *__restrict__ used)
 {
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const long p_first = (((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * GATHER_BLOCKS;
@@ -269,7 +270,10 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint16_t *__restrict_
             if (!has) continue;
             // inside its group of 8 the even entries come first, then the odd ones: the lanes of the product kernel that
             // gather the even (odd) entries of a group read their four indices with one 16-byte load
-            if (r == 0) cols[(o & ~7L) + ((o & 1) << 2) + ((o & 7) >> 1)] = c0 + k;
+            if (r == 0) {
+                cols[(o & ~7L) + ((o & 1) << 2) + ((o & 7) >> 1)] = c0 + k;
+                if (used) used[c0 + k] = 1;
+            }
             if (acol) {
                 acol[((o >> 3) * 16 + r) * 8 + (o & 7)] = (uint16_t)v; // (step*4 + g) = o / 8
             } else {
@@ -314,13 +318,30 @@ __global__ void row_steps_kernel(const int32_t *__restrict__ starts, const int32
     if (i < n) out[i] = first_step[starts[i] / 32];
 }
 
-// used[row] = 1 for the rows of B that the list names; padding names row 0.
-__global__ __launch_bounds__(256) void mark_rows_kernel(const int32_t *__restrict__ cols, long n, int32_t *__restrict__ used)
+// *count = how many of the K rows of B are used, row 0, which padding names, among them.  used: K bytes and zeros up to a multiple of 16.  One workgroup:
+// a few loads a lane up to 10^5 rows, and nothing to clear or to add up behind it.
+__global__ __launch_bounds__(1024) void count_rows_kernel(uint8_t *__restrict__ used, long K, int32_t *__restrict__ count)
 {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) used[cols[i]] = 1;
+    __shared__ int32_t part[16];
+    int32_t n = 0;
+    for (long i = threadIdx.x; i < (K + 15) / 16; i += 1024) {
+        u32x4 v = reinterpret_cast<const u32x4 *>(used)[i];
+        if (i == 0) v[0] |= 1u;
+#pragma unroll
+        for (int q = 0; q < 4; q++) n += __popc(v[q]); // every byte is 0 or 1
+    }
+    if (threadIdx.x == 0) used[0] = 1;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) n += __shfl_xor(n, d);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; w++) n += part[w];
+        *count = n;
+    }
 }
 // place of a used row among the used ones, -1 for the others
-__global__ __launch_bounds__(256) void place_rows_kernel(const int32_t *__restrict__ used, const int32_t *__restrict__ before, long K, int32_t *__restrict__ place)
+__global__ __launch_bounds__(256) void place_rows_kernel(const uint8_t *__restrict__ used, const int32_t *__restrict__ before, long K, int32_t *__restrict__ place)
 {
     const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (k < K) place[k] = used[k] ? before[k] : -1;
@@ -1037,39 +1058,36 @@ static bool lists_nonzeros(int64_t nnz, int64_t n_cols, size_t n_rows, size_t N)
     return 2 * nnz <= 3 * n_cols || (n_cols >= 500000 && nnz <= 4 * n_cols);
 }
 
+struct ByteToInt {
+    __host__ __device__ int32_t operator()(uint8_t v) const { return v; }
+};
 // The copy of B without the rows that no listed column names, where those are an eighth or more.  R-MAT scale 20, 16 a row: 48 % of
 // the columns are empty, and the rows of B under the others fill 67 of 128 MiB a panel, which the memory-side cache holds for
 // the gathers: N = 128 transposition 101 -> 94 us, product 469 -> 401; scale 18, N = 256 226 -> 211, both together; scale 16 equal.
-// With the rows that most columns meet in front the gathers take as long.  Not looked for below 16 MiB, where the
-// transposition is little more than a launch, nor where the plan is made for row-major B, which is read in place.
-static hipError_t place_rows(CompactPlan &p, size_t K, size_t n_cap, long total)
+// With the rows that most columns meet in front the gathers take as long.  The list is marked and counted on the way (gather_kernel,
+// count_rows_kernel), and the number comes to the host where it waits anyway, since most matrices use all rows of B: with a pass over
+// the list, a scan and a copy of their own attaching took 35 to 50 us longer for nothing (stencil 64^3 942 us, so 916; 54336^2, 16 a row, N = 256
+// 1053 and 1032; 16384^2, N = 512 631 and 604).
+static hipError_t place_rows(CompactPlan &p, const uint8_t *used, int32_t n_used, size_t K, long total)
 {
     hipError_t e = hipSuccess;
-    Scratch used, before, tmp;
+    Scratch before, tmp;
     size_t bytes = 0;
-    SMAT_STEP(used.alloc((K + 1) * sizeof(int32_t)));
-    SMAT_STEP(before.alloc((K + 1) * sizeof(int32_t)));
-    SMAT_STEP(hipMemsetAsync(used.p, 0, (K + 1) * sizeof(int32_t), nullptr));
-    const unsigned blocks = (unsigned)std::min<long>((total + 255) / 256, 256L * 8);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(mark_rows_kernel, dim3(blocks), dim3(256), 0, 0, (const int32_t *)p.d_cols, total, (int32_t *)used.p);
-        e = hipGetLastError();
-    }
-    SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, (int32_t *)used.p, (int32_t *)before.p, (int)(K + 1)));
-    SMAT_STEP(tmp.alloc(bytes));
-    SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, (int32_t *)used.p, (int32_t *)before.p, (int)(K + 1)));
-    int32_t n = 0;
-    SMAT_STEP(hipMemcpy(&n, (int32_t *)before.p + K, sizeof n, hipMemcpyDeviceToHost));
-    if (e != hipSuccess || (size_t)n > K / 8 * 7 || (K - (size_t)n) * n_cap * sizeof(uint16_t) < PLACE_MIN_BYTES) return e;
     const long padded = total + LIST_PAD;
+    const hipcub::TransformInputIterator<int32_t, ByteToInt, const uint8_t *> flags(used, ByteToInt{});
+    SMAT_STEP(before.alloc(K * sizeof(int32_t)));
+    SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, flags, (int32_t *)before.p, (int)K));
+    SMAT_STEP(tmp.alloc(bytes));
+    SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, flags, (int32_t *)before.p, (int)K));
     SMAT_STEP(dev_malloc(&p.d_place, K * sizeof(int32_t)));
     SMAT_STEP(dev_malloc(&p.d_cols_placed, (size_t)padded * sizeof(int32_t)));
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(place_rows_kernel, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, 0, (const int32_t *)used.p, (const int32_t *)before.p, (long)K, p.d_place);
-        hipLaunchKernelGGL(place_cols_kernel, dim3(blocks), dim3(256), 0, 0, (const int32_t *)p.d_cols, (const int32_t *)p.d_place, padded, p.d_cols_placed);
+        hipLaunchKernelGGL(place_rows_kernel, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, 0, used, (const int32_t *)before.p, (long)K, p.d_place);
+        hipLaunchKernelGGL(place_cols_kernel, dim3((unsigned)std::min<long>((padded + 255) / 256, 256L * 8)), dim3(256), 0, 0, (const int32_t *)p.d_cols,
+                           (const int32_t *)p.d_place, padded, p.d_cols_placed);
         e = hipGetLastError();
     }
-    p.n_placed = n;
+    p.n_placed = n_used;
     return e;
 }
 
@@ -1156,6 +1174,20 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         SMAT_STEP(dev_malloc(&p->d_acol, cap * 16 * sizeof(uint16_t)));
         SMAT_STEP(hipMemsetAsync(p->d_acol, 0, cap * 16 * sizeof(uint16_t), nullptr));
     }
+    // Rows of B that the list names, looked for where the copy might do without others: not below PLACE_MIN_BYTES of B, nor where the
+    // plan is made for row-major B, which is read in place.
+    const bool look = total > 0 && !b_row_major && K * n_cap * sizeof(uint16_t) >= PLACE_MIN_BYTES;
+    const size_t used_bytes = (K + 15) / 16 * 16;
+    Scratch used; // a byte a row, and their number
+    int32_t n_used = 0;
+    if (look) {
+        SMAT_STEP(used.alloc(used_bytes + sizeof(int32_t)));
+        SMAT_STEP(hipMemsetAsync(used.p, 0, used_bytes, nullptr));
+    }
+    auto count_used = [&](int32_t *to) {
+        hipLaunchKernelGGL(count_rows_kernel, dim3(1), dim3(1024), 0, 0, (uint8_t *)used.p, (long)K, to);
+        return hipGetLastError();
+    };
     Scratch starts;
     SMAT_STEP(starts.alloc((mb + 1) * sizeof(int2)));
     if (e == hipSuccess && nnzb) {
@@ -1163,7 +1195,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         if (e == hipSuccess) {
             hipLaunchKernelGGL(gather_kernel, dim3((unsigned)((nnzb + 4 * GATHER_BLOCKS - 1) / (4 * GATHER_BLOCKS))), dim3(256), 0, 0, vals, (const uint16_t *)s.mask.p,
                                (const unsigned long long *)s.offset.p, row_ptr, col_idx, (const unsigned long long *)s.rows.p, (const int2 *)starts.p,
-                               (long)mb, (long)nnzb, drop_full, p->d_cols, p->d_acol, p->d_entries, p->d_step_range);
+                               (long)mb, (long)nnzb, drop_full, p->d_cols, p->d_acol, p->d_entries, p->d_step_range, (uint8_t *)used.p);
             e = hipGetLastError();
         }
     }
@@ -1173,7 +1205,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         Scratch steps, first, tmp, starts_dev, row_first;
         size_t bytes = 0;
         SMAT_STEP(steps.alloc(((size_t)n_groups + 1) * sizeof(int32_t)));
-        SMAT_STEP(first.alloc(((size_t)n_groups + 1) * sizeof(int32_t)));
+        SMAT_STEP(first.alloc(((size_t)n_groups + 2) * sizeof(int32_t))); // one more for the rows that are used
         SMAT_STEP(hipMemsetAsync(steps.p, 0, ((size_t)n_groups + 1) * sizeof(int32_t), nullptr));
         if (e == hipSuccess) {
             hipLaunchKernelGGL(count_steps_kernel, dim3((unsigned)((n_groups + 255) / 256)), dim3(256), 0, 0, p->d_step_range, n_groups, most, (int32_t *)steps.p);
@@ -1182,8 +1214,11 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, (int32_t *)steps.p, (int32_t *)first.p, n_groups + 1));
         SMAT_STEP(tmp.alloc(bytes));
         SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, (int32_t *)steps.p, (int32_t *)first.p, n_groups + 1));
-        int32_t n_steps = 0;
-        SMAT_STEP(hipMemcpy(&n_steps, (int32_t *)first.p + n_groups, sizeof n_steps, hipMemcpyDeviceToHost));
+        if (look) SMAT_STEP(count_used((int32_t *)first.p + n_groups + 1));
+        int32_t numbers[2] = {0, 0};
+        SMAT_STEP(hipMemcpy(numbers, (int32_t *)first.p + n_groups, (look ? 2 : 1) * sizeof(int32_t), hipMemcpyDeviceToHost));
+        const int32_t n_steps = numbers[0];
+        n_used = numbers[1];
         if (e == hipSuccess && n_steps > n_groups) {
             if ((int64_t)n_steps * 32 > 0x7fffff00) e = hipErrorInvalidValue;
             const size_t step_cap = (size_t)n_steps + (padded_groups - (size_t)n_groups);
@@ -1217,7 +1252,13 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
             }
         }
     }
-    if (e == hipSuccess && total > 0 && !b_row_major && K * n_cap * sizeof(uint16_t) >= PLACE_MIN_BYTES) e = place_rows(*p, K, n_cap, (long)total);
+    auto place_if_it_pays = [&] {
+        if (e == hipSuccess && (size_t)n_used <= K / 8 * 7 && (K - (size_t)n_used) * n_cap * sizeof(uint16_t) >= PLACE_MIN_BYTES)
+            e = place_rows(*p, (const uint8_t *)used.p, n_used, K, (long)total);
+    };
+    int32_t *const count = reinterpret_cast<int32_t *>(static_cast<uint8_t *>(used.p) + used_bytes);
+    if (look && by_entry) place_if_it_pays();
+    else if (look) SMAT_STEP(count_used(count));
     // Work items: whole block rows; rows much longer than the average in chunks of 32-column steps, all of a row's about
     // as long.  Long rows that are all alike stay whole: their partial tiles are 2 * 16 * N floats to write and read again
     // for each (32768 x 65536, 131 a row, N = 256: 138 us whole, 191 in chunks of 1792 columns; 8192 x 65536, 140 a row,
@@ -1283,6 +1324,10 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         SMAT_STEP(dev_malloc(&p->d_split, split.size() * sizeof(SplitRow)));
         SMAT_STEP(hipMemcpy(p->d_split, split.data(), split.size() * sizeof(SplitRow), hipMemcpyHostToDevice));
         SMAT_STEP(dev_malloc(&p->d_workspace, (size_t)slot * 16 * n_cap * sizeof(float)));
+    }
+    if (look && !by_entry) { // the number is there when everything else is
+        SMAT_STEP(hipMemcpy(&n_used, count, sizeof n_used, hipMemcpyDeviceToHost));
+        place_if_it_pays();
     }
     SMAT_STEP(hipDeviceSynchronize());
 #undef SMAT_STEP

@@ -84,3 +84,46 @@ def test_products_on_the_placed_rows(smat, cuda, oracle, used, placed, N, c_f32,
     # the same lists on B in place, through either plan, and narrower than the plan: the same bits
     assert np.array_equal(got, product(in_place, N, True)) and np.array_equal(got, product(plan, N, True))
     assert np.array_equal(got[:, :72], product(plan, 72, False))
+
+
+@pytest.mark.parametrize("whole_columns", [False, True])
+@pytest.mark.parametrize("K,used", [(65536, "odd"), (65552, "odd"), (262160, "last"), (65536, "all")])
+def test_used_rows_are_counted_on_the_way(smat, cuda, whole_columns, K, used):
+    """The copy holds the rows that the list names and row 0, which padding names; to find that none can be left out takes one
+    allocation and no list, scan or copy of its own."""
+    import torch
+    columns = {"odd": np.arange(1, K, 2), "last": np.arange(K - 700, K), "all": np.arange(K)}[used]
+    A = matrix(60 if used != "all" else 1, K, columns, 5)
+    if used == "all":
+        v = np.zeros((K // 16, 16, 16), np.float16)
+        v[:, 0, :] = 0.5
+        A["b_row_ptr"] = np.append(A["b_row_ptr"], A["b_row_ptr"][-1] + K // 16).astype(np.int32)
+        A["b_col_idx"] = np.append(A["b_col_idx"], np.arange(0, K, 16)).astype(np.int32)
+        A["b_val"] = np.append(A["b_val"], v.reshape(-1).view(np.uint16))
+        A["M"], A["nnzb"] = A["M"] + 16, A["nnzb"] + K // 16
+    M, nnzb = A["M"], A["nnzb"]
+    vals, rp, ci = (to_dev(torch, x, cuda) for x in (A["b_val"], A["b_row_ptr"], A["b_col_idx"]))
+    nonzero = (A["b_val"].reshape(-1, 16, 16) & 0x7fff != 0).any(axis=1)
+    named = np.zeros(K, bool)
+    np.logical_or.at(named, (A["b_col_idx"][:, None] + np.arange(16)).reshape(-1), nonzero.reshape(-1))
+    named[0] = True
+    counts, allocated = (ctypes.c_int64 * 2)(), []
+    fn = smat.lib.smat_internal_compact_placed_rows
+    fn.restype, fn.argtypes = ctypes.c_int64, [ctypes.c_void_p]
+    smat.lib.smat_internal_compact_list(1 if whole_columns else 2)
+    smat.lib.smat_internal_compact_tune(0)
+    try:
+        for N in (8, 256):  # a B that is too small to look, and one that is not
+            plan = smat.Plan(A["b_row_ptr"], M, K, nnzb, N, col_idx_host=A["b_col_idx"], kernel=smat.KERNEL_COMPACT)
+            plan.attach_values(vals, rp, ci)
+            smat.lib.smat_internal_alloc_counts(counts)
+            before = counts[0]
+            plan.attach_values(vals, rp, ci)
+            smat.lib.smat_internal_alloc_counts(counts)
+            allocated.append(counts[0] - before)
+            assert fn(plan.handle) == (named.sum() if N == 256 and used != "all" else 0)
+    finally:
+        smat.lib.smat_internal_compact_list(0)
+        smat.lib.smat_internal_compact_tune(1)
+    if used == "all":
+        assert allocated[1] <= allocated[0] + 1
