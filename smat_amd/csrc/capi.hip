@@ -161,19 +161,21 @@ static bool sweep_fills_device(size_t mb, size_t n)
 }
 
 // Time of a product with fp16 results through the sweep kernel, from the tiles (row groups x panels of 64 columns, one
-// workgroup of a compute unit each), the chunks that the row groups list together and the ops of a wavefront per chunk: a
-// tile costs 0.65 us, a chunk 0.32 us and 0.111 us per op (the plan fills up to four), C 0.66 us per 10^6 elements.  Fitted
-// to 153 matrices (random blocks 768^2 to 16384^2 at 3 to 36 %, bands; N = 64 to 4096) on row groups of 16, 32 and 64, three
-// products on their own inputs in turn: 8 % standard deviation, all but a few within 25 %.  Estimate (measured), us:
-//   3088 x 4112, 15 %, N = 1000:  18.1 (19.9) / 19.3 (19.9) / 25.0 (27.3)
-//   8192 x 8192, 10 %, N = 640:   55.2 (50.7) / 30.8 (28.9) / 42.3 (37.6); N = 1536: 84.5 (78.7) / 60.1 (56.3) / 47.1 (41.9)
-//   768 x 3072, 10 %, N = 4096:   14.6 (14.0) / 14.6 (15.0) / 16.7 (17.0)
+// workgroup of a compute unit each), the chunks that the row groups list together and the blocks of a wavefront per chunk: a
+// tile costs 0.65 us, a chunk 0.74 us, which it takes however few blocks it has, or 0.35 us and 0.058 per block where a
+// wavefront has more than six, C 0.66 us per 10^6 elements.  Against 1166 products (400 matrices, random blocks 768^2 to 16384^2 at 3 to 36 % and
+// bands, N = 64 to 4096, on row groups of 16, 32 and 64, three on their own inputs in turn): 10 % standard deviation, none in the mean, 57 of them
+// more than 25 % off.  The same terms fitted to these products anew: 9.5 %, and a choice between the kernels that is no better (1.2 % from the best
+// in the mean, 1.1 with these).  Estimate (measured) on row groups of 16 / 32 / 64, us:
+//   3088 x 4112, 15 %, N = 1000:  18.1 (19.1) / 19.3 (19.5) / 25.1 (25.7)
+//   8192 x 8192, 10 %, N = 640:   55.2 (49.6) / 30.8 (28.7) / 42.3 (36.2); N = 1536: 84.5 (77.7) / 60.1 (55.8) / 47.1 (43.2)
+//   768 x 3072, 10 %, N = 4096:   14.6 (13.7) / 14.6 (14.9) / 16.7 (16.7)
 static double sweep_estimate_us(size_t n_rg, size_t listed_chunks, size_t nnzb, size_t M, size_t N)
 {
     if (n_rg == 0 || listed_chunks == 0) return 1e30;
     const size_t tiles = n_rg * ((N + 16 * SWEEP_TN - 1) / (16 * SWEEP_TN)), rounds = (tiles + 255) / 256;
-    const double ops = 0.525 * (double)nnzb / ((double)listed_chunks * SWEEP_WAVES) + 0.3;
-    const double chunk = 0.32 + 0.111 * std::max(3.8, ops);
+    const double blocks = (double)nnzb / ((double)listed_chunks * SWEEP_WAVES);
+    const double chunk = std::max(0.7418, 0.3533 + 0.058275 * blocks);
     return 3.0 + (double)rounds * (0.65 + (double)listed_chunks / (double)n_rg * chunk) + 0.66e-6 * (double)M * (double)N;
 }
 // The same through the row-wise kernel, fitted to those of 239 products that it can lose: the rounds of 1024 wavefronts that
@@ -212,9 +214,10 @@ static size_t sweep_listed_chunks(const int32_t *row_ptr, const int32_t *col_idx
 
 // Block rows of a row group for a product of N columns whose tiles fill the device: 64, or fewer where the tiles of 64 would
 // leave the last round of 256 workgroups nearly empty and the estimate gains 10 %.  (An emptier round is also a faster one, which
-// the estimate does not know: of 14 products it promised 17 % in the mean and gave 11; where it promised less than 10 %, 8 % to be
-// lost was among it.)  Rows of a group, us: 8192^2, 10 %, N = 2304: 64 74.7, 37 61.8; N = 3072: 64 89.4, 52 82.3; 30 %, N = 2296: 64 169,
-// 37 126; 16384 x 4096, 10 %, N = 1200: 64 42.6, 40 37.3; 12000 x 6000, 7 %, N = 2000: 64 52.2, 47 (estimate 9 % less) 53 to 56.
+// the estimate does not know: of 28 products it promised 20 % in the mean and gave 12; where it promised less than 10 %, 8 % to be
+// lost was among it, and one that it takes loses 7: 11456 x 7904, 9 %, N = 2912 122.6 -> 131.3 us.)  Rows of a group, us: 8192^2, 10 %, N = 2304: 64 80.5, 37 69.5; N = 3072:
+// 64 93.9, 52 88.5; 30 %, N = 2296: 64 168, 37 135; 16384 x 4096, 10 %, N = 1200: 64 45.3, 40 43.6; 12304 x 7936, 21 %, N = 1360: 64 119, 34 96; 12000 x 6000, 7 %, N = 2000:
+// 64 57.0, 47 (estimate 9 % less) 53 to 56 against 52.2.
 static size_t sweep_even_rounds(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t N, bool b_row_major)
 {
     const size_t nnzb = (size_t)row_ptr[mb], n64 = (mb + SWEEP_G - 1) / SWEEP_G;
