@@ -147,7 +147,9 @@ typedef struct smat_plan smat_plan;
  *               otherwise SMAT_KERNEL_SWEEP / SMAT_KERNEL_MIXED are refused with
  *               SMAT_ERR_INVALID and SMAT_KERNEL_AUTO stays with the row-wise kernel, which
  *               takes the blocks of a row in any order (as mmaCBT.cu:44-66 does).
- * n_hint: the N the plan will mostly be used with (panel width choice). */
+ * n_hint: the N the plan will mostly be used with.  The choice of the kernel, the panel width and how long block rows are cut
+ * follow from it: plans of one matrix made with different n_hint may sum the products of a row in different orders, so their
+ * results agree up to fp32 rounding and not bit by bit.  Two plans made alike give the same bits. */
 int smat_plan_create(smat_plan **plan, const int32_t *row_ptr_host, const int32_t *col_idx_host,
                      size_t M, size_t K, size_t nnzb, size_t n_hint, const smat_spmm_opts *opts);
 /* Optional: lets the plan look at the block values (DEVICE arrays of the matrix the plan was
@@ -183,7 +185,8 @@ int smat_plan_check(const smat_plan *plan, const int32_t *row_ptr_host, const in
                     size_t M, size_t K, size_t nnzb);
 /* Fills info[0..11]: kernel id, row-wise work items, split block rows, chunk size,
  * workspace bytes, panel width, sweep stream entries, sweep (row group, K chunk) records,
- * bytes of the scratch copies of B (0 = B is read in place), nonzero block columns listed by
+ * bytes of the scratch for copies of B (0 = B is read in place by every launch; a plan for row-major B keeps scratch for
+ * the launches that need B column-major, also where its own kernel reads B in place), nonzero block columns listed by
  * smat_plan_attach_values (0 = not attached), and for mixed dispatch the row-wise work items (-1: the
  * split is per block, not per block row) and the blocks that the dense kernel takes. */
 int smat_plan_info(const smat_plan *plan, int64_t *info);

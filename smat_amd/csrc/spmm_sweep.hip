@@ -362,10 +362,15 @@ hipError_t launch_sweep(const SweepArgs &a, hipStream_t st)
             if (launched > resident) launched = resident;
         }
     }
-    // A is touched ahead where the launch before has displaced it: where A, B and C are more than half of the 256 MiB of the
-    // memory-side cache.  8192^2, 10 %, N = 4096, inputs changing: 101.5 -> 97.2 us.  With A still in that cache the touches only
-    // cost (the same with N = 2048: 42.1 -> 43.2 us; 3088 x 4112, 15 %, N = 1000: 22.7 -> 23.0), and so they do where two per
-    // lane do not reach the end of A (8192^2, 30 %, N = 4096: 202.5 -> 204.6), and where some rows of A are another kernel's.
+    // A is touched ahead where A, B and C are more than half of the 256 MiB of the memory-side cache: a product of that size finds A
+    // there again only if nothing like it ran in between.  Without / with, us, three matrices in turn; the same A with another B and C; the same everything:
+    //   8192^2, 10 %, N = 4096            99.8/94.7    92.1/92.1    81.9/81.4
+    //   the same, row-major B             103.6/100.3  97.5/98.4    86.4/84.7
+    //   8192^2, 20 %, N = 4096            147.5/141.2  136.3/136.8  127.9/130.7
+    //   8192 x 16384, 10 %, N = 4096      173.3/165.2  161.2/163.1  148.1/149.8
+    //   16384^2, 5 %, N = 4096            272.5/269.9  266.1/268.2  210.0/213.9
+    // With less the touches only cost (8192^2, 10 %, N = 2048: 41.1/42.2; 3088 x 4112, 15 %, N = 1000: 22.7/23.0), and so they do where two per
+    // lane do not reach the end of A (8192^2, 30 %, N = 4096: 202.5/204.6), and where some rows of A are another kernel's.
     const size_t vals_bytes = a.nnzb * 512, traffic = vals_bytes + a.K * a.N * 2 + a.M * a.N * (a.c_f32 ? 4 : 2);
     const uint32_t touch_bytes = a.whole && traffic >= ((size_t)128 << 20) && vals_bytes <= (size_t)launched * THREADS * 128 * 2 ? (uint32_t)vals_bytes : 0;
     dim3 grid((unsigned)launched), block(THREADS);
