@@ -448,8 +448,8 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 // steps, so that the loads of the next step are under way across the end of an item.
 //
 // What a step of 32 columns x 64 columns of C waits for is the vector memory path: 4 KiB of rows of B and 0.15 to 1 KiB of A.
-// Counted on R-MAT scale 20 (stencil 64^3): its data unit is busy 92 (65) % of the time, the vector L1 waits for the L2 62
-// (23) %, LDS is active 30 (37) %, and a step has 21 (30) VALU instructions, 16 (19) of LDS and 6 (7) loads.  Operands merged in
+// Counted on R-MAT scale 20 (stencil 64^3), entries by blocks: its data unit is busy 91 (65) % of the time, the vector L1 waits for the L2 54
+// (26) %, LDS is active 40 (39) %, and a step has 22 (36) VALU instructions, 18 (21) of LDS and 4.7 (5.3) loads.  Operands merged in
 // the VALU took 130 VALU instructions a step, of which 56 exchanged and merged halves between lanes.  Hence:
 //   * Rows of B go from the registers they were gathered into through 4 KiB of LDS, [entry][64 columns], and come back as
 //     MFMA operands through transposing reads (ds_read_b64_tr_b16): no VALU work.  Lane (octet o = lane / 8, c = lane & 7)
