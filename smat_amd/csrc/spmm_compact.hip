@@ -1113,7 +1113,7 @@ static long split_chunk_steps(long steps, size_t rows, long longest, size_t n_ca
     const size_t panels = (n_cap + 63) / 64;
     const double avg = rows ? (double)steps / (double)rows : 0.0, one_panel = (double)steps / (16.0 * 256.0);
     long chunk = (long)(std::max(16.0 + std::max(one_panel, 0.38 * one_panel * (double)panels), 2.5 * avg) + 0.5);
-    const long from = std::max((long)(4.0 * avg), 16L);
+    const long from = std::max((long)(128.0 * avg + 0.5), 512L) / 32; // four times the average, rounded to a column
     if (longest <= from) chunk = std::max(chunk, from);
     if (rows * panels < 1024) chunk = std::min(chunk, (long)LONG_ROW_STEPS);
     return chunk;

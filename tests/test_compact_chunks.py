@@ -30,6 +30,7 @@ def test_which_lists_are_split():
     # not longer than four times the average (or 16 steps): whole
     assert _fn(80000, 10000, 32, 64) >= 32
     assert _fn(10000, 10000, 16, 64) >= 16
+    assert _fn(9426, 967, 39, 1000) >= 39  # 4 x 9426 / 967 steps are 38.99, to the column 39
     # longer, but no longer than a chunk: whole
     assert _fn(240 * PLACES, 65536, 100, 1024) >= 100
     # longer than a chunk: split
