@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -78,6 +79,7 @@ struct smat_plan {
     float *d_workspace_dense = nullptr;
     int n_items_dense = 0, n_split_dense = 0;
     int64_t n_blocks_dense = 0;
+    WindowPlan *window = nullptr; // the row-wise kernel's place is taken by the one that multiplies from windows of B
     uint16_t *d_bcol = nullptr; // column-major copy of a row-major B, K * n_cap halves (plans made for SMAT_B_ROW_MAJOR)
 };
 
@@ -128,6 +130,9 @@ extern "C" void smat_internal_fail_alloc(int64_t n) { g_dev_fail_in.store(n); }
 
 // Test hook (not part of smat.h): block rows that the compact kernel's list of this plan splits, -1 without a list.
 extern "C" int smat_internal_compact_split_rows(const smat_plan *p) { return p->compact ? p->compact->n_split_rows : -1; }
+
+// Test hook (not part of smat.h): block rows of a group whose window the plan's products multiply from, 0 without windows.
+extern "C" int smat_internal_plan_window_rows(const smat_plan *p) { return p->window ? p->window->rows : 0; }
 
 // Test hook (not part of smat.h): rows of B that the compact kernel's copy holds, 0 where it holds all or there is no list.
 extern "C" int64_t smat_internal_compact_placed_rows(const smat_plan *p) { return p->compact ? p->compact->n_placed : 0; }
@@ -368,7 +373,11 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         plan->sweep.fill(w, sweep_row_major);
         e = launch_sweep(w, static_cast<hipStream_t>(o.stream));
     } else {
-        e = launch_rowwise(a, static_cast<hipStream_t>(o.stream));
+        bool window = plan && plan->window && o.kernel == SMAT_KERNEL_AUTO;
+        if (window && N != plan->n_cap && !window_forced()) // made for another width
+            window = !rowwise_shares_items(N, (size_t)plan->n_items, nnzb / (size_t)plan->n_items) && window_launch_us(*plan->window, M, K, N, nnzb, a.c_f32) <
+                     rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, RowLengths::EVEN, a.b_packed != nullptr);
+        e = window ? launch_window(a, *plan->window, static_cast<hipStream_t>(o.stream)) : launch_rowwise(a, static_cast<hipStream_t>(o.stream));
     }
     if (e != hipSuccess)
         return set_error(SMAT_ERR_HIP, "SpMM launch failed: %s", hipGetErrorString(e));
@@ -686,14 +695,10 @@ extern "C" int smat_internal_sweep_group_rows(const int32_t *row_ptr, const int3
 // The streams are built once the values are known to be dense.  The search for a better deal of the rows to the wavefronts
 // takes a tenth of the time (16 counter updates a block: 3088 x 4112, 15 % 0.84 ms for all, without the search 0.75, with a
 // million updates, 0.5 % fewer ops in the busiest wavefronts, 1.8; same kernel times).
-static hipError_t sweep_small_groups(smat_plan &p)
+static hipError_t sweep_small_groups(smat_plan &p, size_t group_rows)
 {
     const size_t mb = p.M / 16, kb = p.K / 16, nnzb = p.nnzb;
-    if (p.col_idx_host.size() != nnzb) return hipSuccess;
     const int32_t *row_ptr = p.row_ptr_host.data(), *col_idx = p.col_idx_host.data();
-    const size_t group_rows = sweep_group_rows(row_ptr, col_idx, p.M, p.K, nnzb, p.n_cap, (size_t)p.n_items,
-                                               p.n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, p.d_bpack != nullptr, p.d_bcol != nullptr);
-    if (!group_rows) return hipSuccess;
     SweepPlanHost h;
     build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 16.0 * (double)nnzb);
     const hipError_t e = p.sweep.upload(h, p.d_bcol != nullptr);
@@ -706,6 +711,41 @@ static hipError_t sweep_small_groups(smat_plan &p)
     p.kernel = SMAT_KERNEL_SWEEP;
     return hipSuccess;
 }
+
+// A plan that plan creation left with the row-wise kernel: windows instead, where the block rows are short enough, none is split
+// and none shared by wavefronts (which sums in another order: plans with and without windows give the same bits), and the
+// estimate is below 0.9 of the row-wise kernel's and of other_us, the time of what else there is; both are off by 10 %.  Row-wise
+// -> windows, us: 27-point stencil 64^3, N = 64 90 -> 56, 48^3, N = 256 111 -> 59, 48 x 25 x 48, N = 56 20.4 -> 12.7; bands of
+// 14224 rows and 182, N = 544 33 -> 17, of 65536 and 20, N = 256 30 -> 15, of 8960 and 120, N = 48 7.4 -> 5.
+static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us)
+{
+    const size_t mb = p.M / 16, kb = p.K / 16;
+    if (p.kernel != SMAT_KERNEL_ROWWISE || p.kernel_requested != SMAT_KERNEL_AUTO || p.n_split_rows || !window_takes_rows(p.max_item_blocks)) return hipSuccess;
+    if (rowwise_shares_items(p.n_cap, (size_t)p.n_items, p.nnzb / std::max<size_t>((size_t)p.n_items, 1)) && !window_forced()) return hipSuccess;
+    if (p.n_cap <= 16 && !window_forced()) return hipSuccess; // 18 -> 17, 10.4 -> 9.2, but 8.2 -> 9, 6.6 -> 7
+    // its estimate knows nothing of the bytes that come from memory, A above all and three times B where that is repacked: 64^3 64 us and
+    // 64 us of bytes, measured 90; 73 x 61 x 62, N = 88 104 and 72, 125; 44 x 47 x 66, N = 40 31 and 26, 38
+    const double once = ((double)p.nnzb * 512.0 + 2.0 * (double)(p.K + p.M) * (double)p.n_cap) / 5e6;
+    const double row_wise = std::hypot(rowwise_estimate_us(p.M, p.K, p.n_cap, p.nnzb, (size_t)p.n_items, RowLengths::EVEN, p.d_bpack != nullptr),
+                                       once + (p.d_bpack ? 4.0 * (double)p.K * (double)p.n_cap / 5e6 : 0.0));
+    const double copy = p.d_bcol ? to_col_major_us(p.K, p.n_cap) : 0.0; // before either
+    const double bar = 0.9 * std::min(row_wise, other_us - copy);
+    // a launch, or the bytes that windows do not save
+    if (!window_forced() && bar < std::max(4.7, 2.0 + once)) return hipSuccess;
+    WindowWidths widths;
+    void *slots = nullptr;
+    if (p.nnzb <= 16384 && p.col_idx_host.size() == p.nnzb) // sooner done than a kernel is waited for
+        window_widths_host(p.row_ptr_host.data(), p.col_idx_host.data(), mb, kb, widths);
+    else {
+        const hipError_t e = window_widths(row_ptr, col_idx, mb, kb, p.nnzb, widths, &slots);
+        if (e != hipSuccess) return e;
+    }
+    int size;
+    const double us = window_choose(widths, p.M, p.K, p.n_cap, p.nnzb, p.max_item_blocks, &size);
+    if (size < 0 || (!window_forced() && us >= bar)) return slots ? dev_free(slots) : hipSuccess;
+    return window_build(widths, size, slots, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, &p.window);
+}
+hipError_t smat::plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx) { return take_window(*p, row_ptr, col_idx, 1e30); }
 
 static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, const int32_t *row_ptr,
                                         const int32_t *col_idx, const int32_t *row_ptr_host)
@@ -733,6 +773,8 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
         if (p->d_workspace_dense) { (void)dev_free(p->d_workspace_dense); p->d_workspace_dense = nullptr; }
         p->n_items_dense = p->n_split_dense = 0;
         p->n_blocks_dense = 0;
+        window_destroy(p->window);
+        p->window = nullptr;
     };
     auto fail = [&](hipError_t err) {
         if (p->compact) { compact_destroy(p->compact); p->compact = nullptr; }
@@ -832,14 +874,24 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     drop_mixed();
     // the compact kernel for everything: few nonzero columns per block - unless the plan has the sweep kernel's work
     // list and the same estimate says that one is faster (blocks of both kinds in a matrix that is dense enough)
-    const bool take = mixed || block_split || want == SMAT_KERNEL_COMPACT ||
-                      (want == SMAT_KERNEL_AUTO && (double)census.n_cols_all < 0.6 * 16.0 * (double)p->nnzb &&
-                       !(dense_kernel == SMAT_KERNEL_SWEEP && t_sweep_all < t_compact_all));
-    if (!take) { // nothing would use the list: the plan keeps (or goes back to) a dense kernel
-        if (p->kernel == SMAT_KERNEL_COMPACT || p->kernel == SMAT_KERNEL_MIXED) p->kernel = dense_kernel;
-        if (want == SMAT_KERNEL_AUTO && dense_kernel == SMAT_KERNEL_ROWWISE) e = sweep_small_groups(*p);
-        return e == hipSuccess ? SMAT_OK : fail(e);
+    bool take = mixed || block_split || want == SMAT_KERNEL_COMPACT ||
+                (want == SMAT_KERNEL_AUTO && (double)census.n_cols_all < 0.6 * 16.0 * (double)p->nnzb &&
+                 !(dense_kernel == SMAT_KERNEL_SWEEP && t_sweep_all < t_compact_all));
+    if (p->kernel == SMAT_KERNEL_COMPACT || p->kernel == SMAT_KERNEL_MIXED) p->kernel = dense_kernel;
+    if (want == SMAT_KERNEL_AUTO && dense_kernel == SMAT_KERNEL_ROWWISE && !mixed && !block_split) {
+        // Windows against the compact kernel (whole panels of 64 columns; row-major B in place), or against the row-wise one where the
+        // sweep kernel's rule leaves a matrix to it.
+        size_t group_rows = 0;
+        if (!take && p->col_idx_host.size() == p->nnzb)
+            group_rows = sweep_group_rows(row_ptr_host, p->col_idx_host.data(), p->M, p->K, p->nnzb, p->n_cap, (size_t)p->n_items,
+                                          p->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, p->d_bpack != nullptr, p->d_bcol != nullptr);
+        if (group_rows) e = sweep_small_groups(*p, group_rows);
+        else e = take_window(*p, row_ptr, col_idx,
+                             take ? (double)census.n_cols_all * (double)((p->n_cap + 63) / 64 * 64) * 2.0 / 10e6 + (p->d_bcol ? 3.0 : t_pass) : 1e30);
+        if (e != hipSuccess) return fail(e);
+        if (p->window) take = false;
     }
+    if (!take) return SMAT_OK; // nothing would use the list: the plan keeps (or goes back to) a dense kernel
     if (!c) e = compact_build(census, vals, row_ptr, col_idx, p->K, p->n_cap, p->d_bcol != nullptr, mixed ? &dense : nullptr, false, &c);
     if (e != hipSuccess) return fail(e);
     if (!p->d_bt) e = dev_malloc(&p->d_bt, p->bt_bytes());
@@ -929,6 +981,7 @@ extern "C" int smat_plan_destroy(smat_plan *p)
     if (!p) return SMAT_OK;
     if (p->compact) compact_destroy(p->compact);
     if (p->d_bt) (void)dev_free(p->d_bt);
+    window_destroy(p->window);
     if (p->d_bcol) (void)dev_free(p->d_bcol);
     if (p->d_items_dense) (void)dev_free(p->d_items_dense);
     if (p->d_split_dense) (void)dev_free(p->d_split_dense);

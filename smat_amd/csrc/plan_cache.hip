@@ -23,6 +23,7 @@
 #include "../../include/smat.h"
 #include "devmem.h"
 #include "errors.h"
+#include "spmm_kernels.h"
 
 using namespace smat;
 
@@ -124,6 +125,8 @@ void build_entry(Entry &en, const uint16_t *vals, Mode mode)
         smat_plan_destroy(p);
         return;
     }
+    if (mode == MODE_PATTERN && en.nnzb) // without it (no memory for its lists) the plan is as good as before
+        (void)plan_take_window(p, static_cast<const int32_t *>(en.row_ptr), static_cast<const int32_t *>(en.col_idx));
     en.plan = p;
     g_cache.built++;
 }

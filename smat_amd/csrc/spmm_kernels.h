@@ -171,6 +171,34 @@ hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, siz
 enum class RowLengths { EVEN, SPLIT, UNKNOWN };
 int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, RowLengths lengths, bool packed);
 bool rowwise_shares_items(size_t N, size_t n_items, size_t avg_blocks);
+// ---- whole blocks from windows of B in LDS (spmm_window.hip) ----
+// For matrices whose neighbouring block rows use the same block columns.
+constexpr int WINDOW_SIZES = 3;
+struct WindowWidths { // over the groups of 4, 8 and 16 consecutive block rows: the most block columns that one uses, and all together
+    uint32_t most[WINDOW_SIZES] = {}, pad = 0;
+    unsigned long long sum[WINDOW_SIZES] = {};
+};
+struct WindowPlan {
+    int rows = 0, cap = 0, n_groups = 0; // block rows of a group, block columns of the widest window (a multiple of 4)
+    unsigned long long sum = 0;
+    int most_blocks = 0;                 // of a block row
+    int32_t *d_window = nullptr, *d_count = nullptr; // window of group i: d_count[i] first columns from d_window[i * cap] on
+    uint32_t *d_slot = nullptr;          // of every block: its place in the window, and its block column
+};
+// row_ptr / col_idx: device arrays.  All but the launch and the estimates are synchronous, on the default stream.
+// *slots: memory for the entries of the blocks, which window_build takes over (or NULL).
+hipError_t window_widths(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, WindowWidths &out, void **slots);
+void window_widths_host(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, WindowWidths &out); // the same from host arrays
+// The size of group (index into the widths, -1 = none fits) that is fastest for a product of N columns, and its time in us.
+double window_choose(const WindowWidths &w, size_t M, size_t K, size_t N, size_t nnzb, int most_blocks, int *size);
+hipError_t window_build(const WindowWidths &w, int size, void *slots, const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, int most_blocks,
+                        WindowPlan **out);
+void window_destroy(WindowPlan *p);
+bool window_forced(); // by the test hook
+bool window_takes_rows(int most_blocks); // block rows of so many blocks
+double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, size_t M, size_t K, size_t N, size_t nnzb, int most_blocks, bool c_f32);
+double window_launch_us(const WindowPlan &p, size_t M, size_t K, size_t N, size_t nnzb, bool c_f32); // 1e30: not at this N
+hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st); // column-major B
 hipError_t launch_sweep(const SweepArgs &a, hipStream_t st);
 // Whether the sweep kernel reads a row-major B of this size in place; otherwise B is brought into column-major order first, one
 // read and one write of it.  In place a row group reads 128 bytes of every row of B where it reads 512 of every column of the
@@ -181,4 +209,10 @@ hipError_t launch_sweep(const SweepArgs &a, hipStream_t st);
 bool sweep_takes_row_major(size_t N, size_t K, int n_rg);
 hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st);
 
+} // namespace smat
+
+struct smat_plan;
+namespace smat {
+// A plan that has no better kernel than the row-wise one gets windows where they are faster (row_ptr / col_idx: device arrays).
+hipError_t plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx);
 } // namespace smat

@@ -1,0 +1,158 @@
+"""Products from windows of B in LDS: matrices whose neighbouring block rows use the same block columns."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from smat_amd import generators as gen
+
+pytestmark = pytest.mark.gpu
+
+
+def to_dev(torch, a, cuda):
+    return torch.from_numpy(np.ascontiguousarray(a).view(np.int16) if a.dtype == np.uint16 else np.ascontiguousarray(a)).to(cuda)
+
+
+@pytest.fixture
+def force(smat):
+    smat.lib.smat_internal_window_force.argtypes = [ctypes.c_int, ctypes.c_int]
+    yield smat.lib.smat_internal_window_force
+    smat.lib.smat_internal_window_force(0, 0)
+    smat.lib.smat_plan_cache_clear()
+
+
+def local_matrix(mb, kb, width, seed, empty=()):
+    """Block row i has up to `width` blocks around column i * kb / mb, an odd and an even number of them, `empty` rows none.
+    Values are small whole numbers: every order of the sums gives the same bits."""
+    rng = np.random.default_rng(seed)
+    rp, ci = [0], []
+    for i in range(mb):
+        if i not in empty:
+            lo = max(0, min(i * kb // mb - width // 2, kb - width))
+            n = rng.integers(1, width + 1)
+            ci += sorted((lo + rng.choice(min(width, kb), n, replace=False)).tolist())
+        rp.append(len(ci))
+    vals = rng.integers(-3, 4, len(ci) * 256).astype(np.float16).view(np.uint16)
+    return np.array(rp, np.int32), np.array(ci, np.int32) * 16, vals
+
+
+def whole_b(K, N, seed):
+    return np.random.default_rng(seed).integers(-4, 5, K * N).astype(np.float16).view(np.uint16)
+
+
+# block rows around whole groups of 4, 8 and 16; rows of one block to the most that a wavefront holds (24 blocks on 4 tiles, 34 on 1
+# and 2); N below, at and past a panel and half a panel
+@pytest.mark.parametrize("mb,kb,width", [(1, 3, 2), (15, 20, 5), (33, 33, 12), (70, 64, 24), (130, 200, 34)])
+@pytest.mark.parametrize("N", [8, 24, 32, 72, 136, 320])
+@pytest.mark.parametrize("rows,tiles", [(4, 1), (4, 2), (8, 2), (8, 4), (16, 1), (16, 2), (16, 4)])
+def test_windows_match_the_oracle(smat, cuda, oracle, force, mb, kb, width, N, rows, tiles):
+    import torch
+    if tiles == 4 and width > 24:
+        pytest.skip("rows of more than 24 blocks")
+    if width > 24 and rows == 4 and tiles == 2 or width > 20 and rows == 8 and tiles == 4:
+        pytest.skip("windows wider than fit")
+    rp, ci, vals = local_matrix(mb, kb, width, seed=mb + rows, empty=(0, 2) if mb > 8 else ())
+    M, K, nnzb = mb * 16, kb * 16, len(ci)
+    B = whole_b(K, N, seed=N)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci, B)]
+    want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B, threads=4)
+    force(rows, tiles)
+    for c_f32 in (False, True):
+        plan = smat.Plan(rp, M, K, nnzb, N, col_idx_host=ci)
+        plan.attach_values(d[0], d[1], d[2])
+        assert smat.lib.smat_internal_plan_window_rows(plan.handle) == rows
+        C = torch.full((M, N), float("nan"), dtype=torch.float32 if c_f32 else torch.float16, device=cuda)
+        smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, nnzb, plan=plan, c_f32=c_f32)
+        assert np.array_equal(C.cpu().numpy().astype(np.float32), want.astype(np.float16 if not c_f32 else np.float32).astype(np.float32))
+        plan.close()
+
+
+def test_many_panels_and_units(smat, cuda, oracle, force):
+    """More units than workgroups, panels split among several: every group of a 40,000-row band at a width of several panels."""
+    import torch
+    rp, ci, vals = local_matrix(2500, 2500, 9, seed=5)
+    M = K = 40000
+    N = 200
+    B = whole_b(K, N, seed=1)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci, B)]
+    want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B, threads=8).astype(np.float16)
+    for rows, tiles in ((4, 1), (8, 2), (16, 4)):
+        force(rows, tiles)
+        plan = smat.Plan(rp, M, K, len(ci), N, col_idx_host=ci)
+        plan.attach_values(d[0], d[1], d[2])
+        C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+        smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, len(ci), plan=plan)
+        assert np.array_equal(C.cpu().numpy(), want)
+        plan.close()
+
+
+def test_infinities_stay_with_the_blocks_that_meet_them(smat, cuda, oracle, force):
+    """An odd number of blocks in a row: the second half of its last pair multiplies zeros by zeros, also where the row before had infinities there."""
+    import torch
+    mb, kb, N = 48, 48, 64
+    rp, ci = np.arange(mb + 1, dtype=np.int32) * 3, np.empty(mb * 3, np.int32)
+    for i in range(mb):
+        ci[3 * i:3 * i + 3] = np.array([max(0, min(i - 1, kb - 3)) + j for j in range(3)]) * 16
+    vals = np.ones(mb * 3 * 256, np.float16)
+    vals[3 * 20 * 256:(3 * 20 + 3) * 256] = np.inf
+    vals = vals.view(np.uint16)
+    M, K = mb * 16, kb * 16
+    B = np.ones((N, K), np.float16)
+    B[:, 30 * 16] = np.inf
+    B = B.reshape(-1).view(np.uint16)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci, B)]
+    want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B, threads=4).astype(np.float16)
+    for rows in (4, 8, 16):
+        force(rows, 2)
+        plan = smat.Plan(rp, M, K, len(ci), N, col_idx_host=ci)
+        plan.attach_values(d[0], d[1], d[2])
+        C = torch.zeros((M, N), dtype=torch.float16, device=cuda)
+        smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, len(ci), plan=plan)
+        assert np.array_equal(C.cpu().numpy(), want, equal_nan=True)
+        plan.close()
+
+
+def test_a_pattern_rewritten_in_place_is_multiplied_as_it_is(smat, cuda, oracle, force):
+    """The drop-in call keeps the windows of the pattern it saw first; blocks that moved since are multiplied where they are now."""
+    import torch
+    force(8, 2)
+    rp, ci, vals = local_matrix(100, 100, 7, seed=2)
+    M = K = 1600
+    N = 96
+    B = whole_b(K, N, seed=3)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci, B)]
+    smat.lib.smat_plan_cache_clear()
+    C = torch.empty((M, N), dtype=torch.float16, device=cuda)
+    for seed in (None, 11, 12):
+        if seed is not None:
+            rng = np.random.default_rng(seed)
+            for i in range(0, 100, 3):
+                ci[rp[i]:rp[i + 1]] = np.sort(rng.choice(100, rp[i + 1] - rp[i], replace=False)).astype(np.int32) * 16
+            d[2].copy_(torch.from_numpy(ci))
+        smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, len(ci), drop_in=True)
+        want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B, threads=4).astype(np.float16)
+        assert np.array_equal(C.cpu().numpy(), want)
+
+
+def test_which_products_take_windows(smat, cuda):
+    """Local patterns do, as the drop-in call and with values; random ones, rows too long and products of a launch's length do not."""
+    import torch
+
+    def rows(A, N, row_major=False):
+        ci, rp = A["b_col_idx"].astype(np.int32), A["b_row_ptr"].astype(np.int32)
+        d = [to_dev(torch, x, cuda) for x in (A["b_val"], rp, ci)]
+        plan = smat.Plan(rp, A["M"], A["K"], len(ci), N, col_idx_host=ci, b_row_major=row_major)
+        plan.attach_values(*d)
+        r = smat.lib.smat_internal_plan_window_rows(plan.handle)
+        plan.close()
+        return r
+
+    def blocked(d):
+        A = smat.csr_to_bcsr(d["M"], d["K"], d["row_ptr"], d["col_idx"], d["val"])
+        return {"M": A.M, "K": A.K, "b_row_ptr": A.row_ptr, "b_col_idx": A.col_idx, "b_val": A.val}
+
+    assert rows(blocked(gen.stencil27(32)), 512) > 0
+    assert rows(blocked(gen.band(8960, 120)), 48) > 0
+    assert rows(blocked(gen.band(512, 16)), 32) == 0
+    assert rows(blocked(gen.band(8192, 400)), 256) == 0
+    assert rows(gen.random_bcsr(128, 128, 0.2, seed=1), 512) == 0
