@@ -879,7 +879,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
                  !(dense_kernel == SMAT_KERNEL_SWEEP && t_sweep_all < t_compact_all));
     if (p->kernel == SMAT_KERNEL_COMPACT || p->kernel == SMAT_KERNEL_MIXED) p->kernel = dense_kernel;
     if (want == SMAT_KERNEL_AUTO && dense_kernel == SMAT_KERNEL_ROWWISE && !mixed && !block_split) {
-        // Windows against the compact kernel (whole panels of 64 columns; row-major B in place), or against the row-wise one where the
+        // Windows against the compact kernel (whole panels of 16, 32 or 64 columns; row-major B in place), or against the row-wise one where the
         // sweep kernel's rule leaves a matrix to it.
         size_t group_rows = 0;
         if (!take && p->col_idx_host.size() == p->nnzb)
@@ -887,7 +887,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
                                           p->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, p->d_bpack != nullptr, p->d_bcol != nullptr);
         if (group_rows) e = sweep_small_groups(*p, group_rows);
         else e = take_window(*p, row_ptr, col_idx,
-                             take ? (double)census.n_cols_all * (double)((p->n_cap + 63) / 64 * 64) * 2.0 / 10e6 + (p->d_bcol ? 3.0 : t_pass) : 1e30);
+                             take ? (double)census.n_cols_all * (double)(p->n_cap <= 16 ? 16 : p->n_cap <= 32 ? 32 : (p->n_cap + 63) / 64 * 64) * 2.0 / 10e6 + (p->d_bcol ? 3.0 : t_pass) : 1e30);
         if (e != hipSuccess) return fail(e);
         if (p->window) take = false;
     }

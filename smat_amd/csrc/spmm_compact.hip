@@ -21,10 +21,10 @@
 //    The SpMM then does not read the block values any more: they must be attached again when
 //    they change.
 //  * transpose_b_kernel: column-major B (B[n*K + k]) -> Bt at the start of every launch, so that
-//    the row of B under a nonzero column is contiguous.  Bt holds the panels of 64*TQ columns one
-//    after the other, each a row-major K x 64*TQ matrix: the pass over a panel gathers from one
-//    contiguous K * 128*TQ bytes.
-//  * spmm_compact_kernel<TQ>: one wavefront per (run of work items, panel of 64*TQ columns).  A step takes
+//    the row of B under a nonzero column is contiguous.  Bt holds the panels of W columns one
+//    after the other, each a row-major K x W matrix: the pass over a panel gathers from one
+//    contiguous K * 2*W bytes.
+//  * spmm_compact_kernel<W>: one wavefront per (run of work items, panel of W columns).  A step takes
 //    32 columns = K of one v_mfma_f32_16x16x32_f16.  The product is formed as C^T = B^T * A^T like in the other
 //    kernels; every gather is 16 bytes per lane (a CU keeps a limited number of vector memory instructions and of
 //    cache lines in flight, so an instruction should bring as much as it can).  The index list keeps, inside every
@@ -43,6 +43,7 @@
 namespace smat {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -380,23 +381,24 @@ __global__ __launch_bounds__(256) void copy_blocks_kernel(const uint16_t *__rest
 }
 
 // ---- B: column-major -> row-major ----
-// 64 n x 64 k tile through LDS.  A thread reads 16 bytes (8 k) of two neighbouring columns, pairs
+// Tile of COLS n x 4096 / COLS k through LDS.  A thread reads 16 bytes (8 k) of two neighbouring columns, pairs
 // the values of equal k into dwords and writes them to the transposed tile; then every thread
-// reads 8 n of one k back (two 8-byte LDS reads) and stores 16 bytes.
+// reads 8 n of one k back (two 8-byte LDS reads) and stores 16 bytes.  COLS = 64; 16 and 32 for a B of no more columns.
 // The output is split into panels of `panel` columns, each a K x panel row-major matrix of leading
 // dimension ld, one panel after the other (panel >= N and ld = N: plain row-major K x N).
 // place != NULL: row k goes to row place[k] of a copy of `rows` rows, or nowhere (-1).
 // STREAM: B does not stay in the caches behind the loads, which leaves them to the copy (launch_transpose).
-template <bool STREAM>
+template <int COLS, bool STREAM>
 __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__restrict__ B, uint16_t *__restrict__ Bt,
                                                           int N, long K, int panel, long ld, long rows, const int32_t *__restrict__ place)
 {
-    constexpr int LD = 68; // halfs per LDS row (k): 8-byte aligned rows, dword writes spread over the banks
-    __shared__ __align__(16) uint16_t tile[64 * LD];
+    constexpr int KT = 4096 / COLS; // k of a tile
+    constexpr int LD = COLS + 4; // halfs per LDS row (k): 8-byte aligned rows, dword writes spread over the banks
+    __shared__ __align__(16) uint16_t tile[KT * LD];
     const int t = threadIdx.x;
-    const long k0 = (long)blockIdx.x * 64;
-    const int n0 = blockIdx.y * 64;
-    const int a = t >> 3, seg = t & 7;
+    const long k0 = (long)blockIdx.x * KT;
+    const int n0 = blockIdx.y * COLS;
+    const int a = t / (KT / 8), seg = t % (KT / 8);
     u32x4 v0 = {0u, 0u, 0u, 0u}, v1 = {0u, 0u, 0u, 0u}; // columns 2a, 2a+1; k = 8seg .. 8seg+7
     if (k0 + seg * 8 < K) {
         const u32x4 *p0 = reinterpret_cast<const u32x4 *>(B + (long)(n0 + 2 * a) * K + k0 + seg * 8);
@@ -404,26 +406,27 @@ __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__rest
         if (n0 + 2 * a < N) v0 = STREAM ? __builtin_nontemporal_load(p0) : *p0;
         if (n0 + 2 * a + 1 < N) v1 = STREAM ? __builtin_nontemporal_load(p1) : *p1;
     }
-    long to[2]; // the rows that this thread stores, asked for beside the values (behind the barrier: 94 instead of 87 us for 256 MiB)
+    const int row = t / (COLS / 8), piece = t % (COLS / 8); // stored by this thread: rows row, row + KT / 2
+    long to[2]; // where they go, asked for beside the values (behind the barrier: 94 instead of 87 us for 256 MiB)
 #pragma unroll
     for (int half = 0; half < 2; half++) {
-        const long k = k0 + a + 32 * half;
+        const long k = k0 + row + KT / 2 * half;
         to[half] = k >= K ? -1 : place ? (long)place[k] : k;
     }
 #pragma unroll
     for (int w = 0; w < 4; w++) {
-        uint32_t *row = reinterpret_cast<uint32_t *>(tile + (seg * 8 + 2 * w) * LD + 2 * a);
-        row[0] = __builtin_amdgcn_perm(v1[w], v0[w], 0x05040100u);      // k = 8seg + 2w
-        row[LD / 2] = __builtin_amdgcn_perm(v1[w], v0[w], 0x07060302u); // k = 8seg + 2w + 1
+        uint32_t *at = reinterpret_cast<uint32_t *>(tile + (seg * 8 + 2 * w) * LD + 2 * a);
+        at[0] = __builtin_amdgcn_perm(v1[w], v0[w], 0x05040100u);      // k = 8seg + 2w
+        at[LD / 2] = __builtin_amdgcn_perm(v1[w], v0[w], 0x07060302u); // k = 8seg + 2w + 1
     }
     __syncthreads();
 #pragma unroll
     for (int half = 0; half < 2; half++) {
-        const int k = a + 32 * half;
-        if (to[half] >= 0 && n0 + seg * 8 < N) {
-            const uint2 lo = *reinterpret_cast<const uint2 *>(tile + k * LD + seg * 8);
-            const uint2 hi = *reinterpret_cast<const uint2 *>(tile + k * LD + seg * 8 + 4);
-            uint16_t *out = Bt + (long)(n0 / panel) * rows * panel + to[half] * ld + n0 % panel + seg * 8;
+        const int k = row + KT / 2 * half;
+        if (to[half] >= 0 && n0 + piece * 8 < N) {
+            const uint2 lo = *reinterpret_cast<const uint2 *>(tile + k * LD + piece * 8);
+            const uint2 hi = *reinterpret_cast<const uint2 *>(tile + k * LD + piece * 8 + 4);
+            uint16_t *out = Bt + (long)(n0 / panel) * rows * panel + to[half] * ld + n0 % panel + piece * 8;
             *reinterpret_cast<u32x4 *>(out) = (u32x4){lo.x, lo.y, hi.x, hi.y};
         }
     }
@@ -434,17 +437,23 @@ __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__rest
 // (27-point stencil 64^3, N = 64, 33 MB, the same B again: 41.0 us, past the caches 44.3).
 static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, size_t K, int panel, long ld, long rows, const int32_t *place, hipStream_t st)
 {
-    const dim3 grid((unsigned)((K + 63) / 64), (unsigned)((N + 63) / 64));
-    if (N * K * sizeof(uint16_t) >= (size_t)128 << 20)
-        hipLaunchKernelGGL(transpose_b_kernel<true>, grid, dim3(256), 0, st, B, Bt, (int)N, (long)K, panel, ld, rows, place);
-    else
-        hipLaunchKernelGGL(transpose_b_kernel<false>, grid, dim3(256), 0, st, B, Bt, (int)N, (long)K, panel, ld, rows, place);
+    auto launch = [&](auto cols, auto stream) {
+        constexpr int COLS = decltype(cols)::value;
+        const dim3 grid((unsigned)((K + 4096 / COLS - 1) / (4096 / COLS)), (unsigned)((N + COLS - 1) / COLS));
+        hipLaunchKernelGGL((transpose_b_kernel<COLS, decltype(stream)::value>), grid, dim3(256), 0, st, B, Bt, (int)N, (long)K, panel, ld, rows, place);
+    };
+    using std::false_type;
+    using std::integral_constant;
+    if (N * K * sizeof(uint16_t) >= (size_t)128 << 20) launch(integral_constant<int, 64>{}, std::true_type{});
+    else if (N <= 16) launch(integral_constant<int, 16>{}, false_type{});
+    else if (N <= 32) launch(integral_constant<int, 32>{}, false_type{});
+    else launch(integral_constant<int, 64>{}, false_type{});
     return hipGetLastError();
 }
 
 // ---- the product ----
 
-// A wavefront takes a task x a panel of 64 TQ columns.  A task is a run of items of the list, worked off as one stream of
+// A wavefront takes a task x a panel of W = 16, 32, 64 or 128 columns.  A task is a run of items of the list, worked off as one stream of
 // steps, so that the loads of the next step are under way across the end of an item.
 //
 // What a step of 32 columns x 64 columns of C waits for is the vector memory path: 4 KiB of rows of B and 0.15 to 1 KiB of A.
@@ -452,7 +461,7 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 // (26) %, LDS is active 40 (39) %, and a step has 22 (36) VALU instructions, 18 (21) of LDS and 4.7 (5.3) loads.  Operands merged in
 // the VALU took 130 VALU instructions a step, of which 56 exchanged and merged halves between lanes.  Hence:
 //   * Rows of B go from the registers they were gathered into through 4 KiB of LDS, [entry][64 columns], and come back as
-//     MFMA operands through transposing reads (ds_read_b64_tr_b16): no VALU work.  Lane (octet o = lane / 8, c = lane & 7)
+//     MFMA operands through transposing reads (ds_read_b64_tr_b16): no VALU work.  With W >= 64 lane (octet o = lane / 8, c = lane & 7)
 //     gathers columns 8c .. 8c + 7 of the entries k = 8 (o / 2) + 2j + (o & 1), j = 0 .. 3; the 16-byte pieces of the rows k
 //     with k & 2 are swapped in pairs, which leaves 16 of the 71 clocks that a step keeps LDS active to bank conflicts (AF = 0,
 //     counted).  In lane (i = lane % 16, g = lane / 16) n-tile t of the
@@ -473,12 +482,12 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 // part of the blocks it multiplies); work items that go through the workspace are not made for such plans.
 //
 // What the compiler has to be told (over 110 drawn random matrices 2.8 % in the mean, 4096 x 512, 64 a row, N = 1024: 19.5 -> 17.9 us):
-//   * __launch_bounds__(256, 2): with one wavefront per SIMD allowed, the accumulators go to accumulation registers and 16 TQ of
+//   * __launch_bounds__(256, 2): with one wavefront per SIMD allowed, the accumulators go to accumulation registers and W / 4 of
 //     them are moved there and back every two steps.
 //   * The loop ends at its bottom only.  A way out of its middle is turned into one that seems to lead from the first step
 //     back to the first, where the registers of the second still seem to be waited for: every other step waited for operands
 //     before it asked for the next ones.  A task that ends with the first step ends there with s_endpgm.
-//   * LDS for four workgroups a CU (TQ = 1): with five, which the registers now allow, the gathers of R-MAT scale 20 lose 0.6 %
+//   * LDS for four workgroups a CU (W = 64): with five, which the registers now allow, the gathers of R-MAT scale 20 lose 0.6 %
 //     and 16384^2 2 % (three: 16384^2 11 %).
 //
 // Entries (AF > 0) come from memory in the step before they are needed, 256 bytes a load, or, STAGED, 256 at a time ahead of
@@ -496,13 +505,14 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 //   8192 x 32768, 60 a row, N = 512 56.5/54.8  40.3/41.0   41.5/43.1   41.6/43.1
 // The launcher's rule is at STAGED_STEPS.  A block asked for on every second step, which makes all waits exact, is slower than one
 // asked for when it is needed (R-MAT scale 20 461 -> 477).
-template <int TQ, bool C_F32, bool C_ACC, int AF, bool STAGED, bool BIG>
+template <int W, bool C_F32, bool C_ACC, int AF, bool STAGED, bool BIG>
 __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const uint16_t *__restrict__ acol, const uint32_t *__restrict__ entries, const int2 *__restrict__ step_range, const int32_t *__restrict__ cols,
     const uint16_t *__restrict__ Bt, void *__restrict__ Cout, float *__restrict__ workspace, const WorkItem *__restrict__ items,
     const int4 *__restrict__ tasks, int n_tasks, int N, int n_panels, long panel_stride, long row_stride, unsigned xcd_run)
 {
-    constexpr int A_BYTES = 1024, B_BYTES = 4096 * TQ, I_BYTES = 2048, E_BYTES = STAGED ? 2048 : 0, UNUSED_BYTES = TQ == 1 ? 2048 - E_BYTES : 0;
+    constexpr int TQ = W > 64 ? 2 : 1, PW = W / TQ, T = PW / 16; // a row of PW columns is gathered by PW / 8 lanes, 32 rows by T instructions
+    constexpr int A_BYTES = 1024, B_BYTES = 64 * W, I_BYTES = 2048, E_BYTES = STAGED ? 2048 : 0, UNUSED_BYTES = W == 64 ? 2048 - E_BYTES : 0;
     static_assert((A_BYTES + B_BYTES + I_BYTES + E_BYTES + UNUSED_BYTES) % 1024 == 0, "entries hold offsets that are or-ed to the address of the A tile");
     __shared__ __align__(1024) unsigned char lds[4][A_BYTES + B_BYTES + I_BYTES + E_BYTES + UNUSED_BYTES];
     const int lane = threadIdx.x & 63;
@@ -535,28 +545,30 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     enter();
 
     const int i16 = lane & 15, g = lane >> 4;
-    const int n0 = panel * 64 * TQ;
-    // Row `col` of this panel of B starts at Bp + col * row_stride (B in place: panel_stride = 64 TQ, row_stride = N; the
-    // transposed copy: panels one after the other, row_stride = 64 TQ).
+    const int n0 = panel * W;
+    // Row `col` of this panel of B starts at Bp + col * row_stride (B in place: panel_stride = W, row_stride = N; the
+    // transposed copy: panels one after the other, row_stride = W).
     const uint16_t *Bp = Bt + (long)panel * panel_stride;
     int boff[TQ]; // N % 8 == 0: all of the lane's columns or none (then its column 0)
 #pragma unroll
-    for (int q = 0; q < TQ; q++) boff[q] = n0 + 64 * q + 8 * (lane & 7) < N ? 64 * q + 8 * (lane & 7) : 0;
+    for (int q = 0; q < TQ; q++) boff[q] = n0 + 64 * q + 8 * (lane % (PW / 8)) < N ? 64 * q + 8 * (lane % (PW / 8)) : 0;
 
     unsigned char *const a_tile = lds[wave], *const b_tile = lds[wave] + A_BYTES;
     const uint32_t a_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)a_tile; // a multiple of 1024
-    const int oct = lane >> 3, c8 = lane & 7, row0 = (8 * (oct >> 1) + (oct & 1)) * 128;
-    unsigned char *const put_even = b_tile + row0 + c8 * 16, *const put_odd = b_tile + row0 + (c8 ^ 1) * 16; // entry j: + j * 256
-    const int swap = (i16 >> 3) & 1;
-    const unsigned char *const get = b_tile + (8 * g + (i16 >> 2)) * 128 + (i16 & 3) * 32;
+    // lane -> places first_place + j, j < T, of the step's 32 in the list, which are entries 8 (place / 8) + 2 (place % 4) + (place / 4) % 2
+    const int c8 = lane % (PW / 8), first_place = T * (lane / (PW / 8));
+    const int row0 = (8 * (first_place >> 3) + 2 * (first_place & 3) + ((first_place >> 2) & 1)) * (2 * PW);
+    unsigned char *const put_even = b_tile + row0 + c8 * 16, *const put_odd = b_tile + row0 + (PW == 64 ? c8 ^ 1 : c8) * 16; // entry j: + j * 4 * PW
+    const int swap = PW == 64 ? (i16 >> 3) & 1 : 0;
+    const unsigned char *const get = b_tile + (8 * g + (i16 >> 2)) * (2 * PW) + (i16 & 3) * (PW / 2);
     const unsigned char *const get01 = get + 16 * swap, *const get23 = get - 16 * swap; // tiles 0, 1 and 2, 3: + t * 8
 
-    f32x4 acc[TQ][4];
+    f32x4 acc[TQ][T];
     auto clear_acc = [&] {
 #pragma unroll
         for (int q = 0; q < TQ; q++)
 #pragma unroll
-            for (int t = 0; t < 4; t++) acc[q][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < T; t++) acc[q][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
     };
     clear_acc();
 
@@ -564,7 +576,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
         u32x4 aw;                  // AF = 0
         uint32_t ent[AF ? AF : 1]; // AF > 0
         int n;                     // the step's entries
-        u32x4 L[TQ][4];
+        u32x4 L[TQ][T];
     };
     int2 ranges = {0, 0}; // entries of the step range_from + lane
     const int first_step = e >> 5;
@@ -578,7 +590,8 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     unsigned char *const i_tile = lds[wave] + A_BYTES + B_BYTES;
     auto load_block = [&](int s) { return reinterpret_cast<const u32x4 *>(cols + s)[lane]; };
     auto put_block = [&](int s, u32x4 x) { *reinterpret_cast<u32x4 *>(i_tile + (((s >> 5) - first_step) & 8) * 128 + lane * 16) = x; };
-    auto indices = [&](int s) { return *reinterpret_cast<const u32x4 *>(i_tile + (((s >> 5) - first_step) & 15) * 128 + oct * 16); };
+    typedef uint32_t Indices __attribute__((ext_vector_type(T)));
+    auto indices = [&](int s) { return *reinterpret_cast<const Indices *>(i_tile + (((s >> 5) - first_step) & 15) * 128 + first_place * 4); };
     // Entries the same way: 256 of them, 1 KiB, a load, to one half of 2 KiB of LDS.  A block goes there when the first step that
     // needs it is asked for, and the one after it is loaded into the same registers then.  (Two blocks in registers, the further one moved
     // down, was every load in flight waited for at each move: the compiler's count of what is younger than a load that only some
@@ -600,7 +613,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
         e_block = b + 2;
         if (e_block <= e_end) e_next = load_entries(e_block);
     }
-    auto request = [&](int s, const u32x4 x, Operands &o) {
+    auto request = [&](int s, const Indices x, Operands &o) {
         if constexpr (AF == 0) {
             o.aw = *reinterpret_cast<const u32x4 *>(acol + ((long)(s >> 3) + g) * 128 + i16 * 8);
         } else if constexpr (!STAGED) {
@@ -614,13 +627,13 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
 #pragma unroll
             for (int q = 0; q < TQ; q++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) o.L[q][j] = *reinterpret_cast<const u32x4 *>(Bp + (long)x[j] * stride + boff[q]);
+                for (int j = 0; j < T; j++) o.L[q][j] = *reinterpret_cast<const u32x4 *>(Bp + (long)x[j] * stride + boff[q]);
         } else {
             const uint32_t stride = s < e_last ? (uint32_t)row_stride * 2u : 0u;
 #pragma unroll
             for (int q = 0; q < TQ; q++)
 #pragma unroll
-                for (int j = 0; j < 4; j++)
+                for (int j = 0; j < T; j++)
                     o.L[q][j] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const unsigned char *>(Bp) +
                                                                  (size_t)(uint32_t)(__umul24(x[j], stride) + (uint32_t)boff[q] * 2u));
         }
@@ -659,23 +672,23 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
 #pragma unroll
         for (int q = 0; q < TQ; q++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) *reinterpret_cast<u32x4 *>((j & 1 ? put_odd : put_even) + q * 4096 + j * 256) = o.L[q][j];
+            for (int j = 0; j < T; j++) *reinterpret_cast<u32x4 *>((j & 1 ? put_odd : put_even) + q * 4096 + j * 4 * PW) = o.L[q][j];
         asm volatile("" ::: "memory");
-        f16x8 b[TQ][4];
+        f16x8 b[TQ][T];
 #pragma unroll
         for (int q = 0; q < TQ; q++)
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
+            for (int t = 0; t < T; t++) {
                 const unsigned char *p = (t < 2 ? get01 : get23) + q * 4096 + t * 8;
                 const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p);
-                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(p + 512));
+                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(p + 8 * PW));
                 b[q][t] = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
             }
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int q = 0; q < TQ; q++)
 #pragma unroll
-            for (int t = 0; t < 4; t++) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[q][t], av, acc[q][t], 0, 0, 0);
+            for (int t = 0; t < T; t++) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[q][t], av, acc[q][t], 0, 0, 0);
     };
     // The tile of item `it` goes out (acc[q][t][r] = C[16 br + i16][n0 + 64 q + 16 g + 4 t + r]); the next item that has
     // steps is the current one afterwards.
@@ -684,12 +697,12 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
             const long m = (long)br * 16 + i16;
 #pragma unroll
             for (int q = 0; q < TQ; q++) {
-                const int c0 = n0 + 64 * q + 16 * g;
+                const int c0 = n0 + 64 * q + PW / 4 * g;
                 if (dst >= 0 || C_F32) {
                     float *row = dst >= 0 ? workspace + ((long)dst * 16 + i16) * (long)N
                                           : reinterpret_cast<float *>(Cout) + m * (long)N;
 #pragma unroll
-                    for (int t = 0; t < 4; t++)
+                    for (int t = 0; t < T; t++)
                         if (c0 + 4 * t < N) {
                             f32x4 v = acc[q][t];
                             if (C_ACC && dst < 0) v += *reinterpret_cast<const f32x4 *>(row + c0 + 4 * t);
@@ -697,19 +710,24 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
                         }
                 } else {
                     uint16_t *row = reinterpret_cast<uint16_t *>(Cout) + m * (long)N;
+                    if constexpr (T == 1) {
+                        static_assert(!C_ACC, "narrow panels are not accumulated");
+                        if (c0 < N) *reinterpret_cast<f16x4 *>(row + c0) = __builtin_convertvector(acc[q][0], f16x4);
+                    } else {
 #pragma unroll
-                    for (int h = 0; h < 2; h++) {
-                        if (c0 + 8 * h >= N) continue;
-                        f16x8 v;
-                        if (C_ACC) {
-                            const f16x8 old = *reinterpret_cast<const f16x8 *>(row + c0 + 8 * h);
+                        for (int h = 0; h < T / 2; h++) {
+                            if (c0 + 8 * h >= N) continue;
+                            f16x8 v;
+                            if (C_ACC) {
+                                const f16x8 old = *reinterpret_cast<const f16x8 *>(row + c0 + 8 * h);
 #pragma unroll
-                            for (int j = 0; j < 8; j++) v[j] = (_Float16)(acc[q][2 * h + j / 4][j % 4] + (float)old[j]);
-                        } else {
+                                for (int j = 0; j < 8; j++) v[j] = (_Float16)(acc[q][2 * h + j / 4][j % 4] + (float)old[j]);
+                            } else {
 #pragma unroll
-                            for (int j = 0; j < 8; j++) v[j] = (_Float16)acc[q][2 * h + j / 4][j % 4];
+                                for (int j = 0; j < 8; j++) v[j] = (_Float16)acc[q][2 * h + j / 4][j % 4];
+                            }
+                            *reinterpret_cast<f16x8 *>(row + c0 + 8 * h) = v;
                         }
-                        *reinterpret_cast<f16x8 *>(row + c0 + 8 * h) = v;
                     }
                 }
             }
@@ -731,7 +749,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     asm volatile("" ::: "memory");
     request(e, indices(e), op_a);
     int next = e + 32; // the step whose operands are asked for
-    u32x4 x = indices(next); // read from LDS a step before they are used
+    Indices x = indices(next); // read from LDS a step before they are used
     // Before the first step that `ranges` does not reach (every 64 steps): the ranges of 64 steps from there on.  The wait for
     // them is inside, so that no other step has one; a task of up to 62 steps never gets here.
     auto more_ranges = [&] {
@@ -766,11 +784,11 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     } while (it < tk.y);
 }
 
-template <int TQ>
-hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
+template <int W>
+hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
 {
     const CompactPlan &p = *a.plan;
-    constexpr int PANEL = 64 * TQ;
+    constexpr int PANEL = W;
     const int n_panels = (int)((a.N + PANEL - 1) / PANEL);
     long panel_stride = PANEL, row_stride = (long)a.N;
     const int32_t *cols = p.d_cols;
@@ -797,16 +815,18 @@ hipError_t launch_compact_tq(const CompactArgs &a, hipStream_t st)
     // 32-bit byte offsets from indices of 24 bits
     const bool big = a.K > ((size_t)1 << 24) || a.K * (size_t)row_stride * 2 >= ((size_t)1 << 32) || row_stride >= (1L << 23);
     auto launch = [&](auto af, auto staged, auto f32, auto acc, auto wide) {
-        hipLaunchKernelGGL((spmm_compact_kernel<TQ, decltype(f32)::value, decltype(acc)::value, decltype(af)::value, decltype(staged)::value, decltype(wide)::value>),
+        hipLaunchKernelGGL((spmm_compact_kernel<W, decltype(f32)::value, decltype(acc)::value, decltype(af)::value, decltype(staged)::value, decltype(wide)::value>),
                            dim3((unsigned)wgs), dim3(256), 0, st, p.d_acol, p.d_entries, p.d_step_range, cols, a.Bt, a.C, p.d_workspace,
                            p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, (unsigned)xcd_run);
     };
     using std::false_type;
     using std::true_type;
     auto by_output = [&](auto af, auto staged, auto wide) {
-        if (a.accumulate) { // never staged
+        if constexpr (W >= 64) if (a.accumulate) { // never staged
             if (a.c_f32) launch(af, false_type{}, true_type{}, true_type{}, wide); else launch(af, false_type{}, false_type{}, true_type{}, wide);
-        } else {
+            return;
+        }
+        {
             if (a.c_f32) launch(af, staged, true_type{}, false_type{}, wide); else launch(af, staged, false_type{}, false_type{}, wide);
         }
     };
@@ -834,15 +854,19 @@ hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, siz
     return launch_transpose(B_row_major, out, K, N, 0x7fffffff, (long)K, (long)N, nullptr, st);
 }
 
-// The panel width of a launch, in units of 64 columns.
-static int compact_panel_width(const CompactPlan &p, size_t N, size_t K)
+// The columns of a panel of a launch.  A product of up to 16 or 32 columns takes panels of that many: a row of B is then 32 or 64 bytes, a step
+// gathers its 32 rows in one or two instructions instead of four, and brings as many lines less (same order of sums, same bits).  Panels of
+// 64 columns -> 16 or 32, us: R-MAT scale 18, 22 a row, N = 8 61 -> 45, N = 16 in fp32 68 -> 47, N = 32 72 -> 61; 27-point stencil 64^3, N = 16 37.4 -> 19.8, N = 32
+// 43.4 -> 30.0; 61648 x 25136, 13 a row, N = 16 13.6 -> 10.9; 16384^2, 16 a row, N = 32, row-major B 6.1 -> 5.8.
+static int compact_panel_width(const CompactPlan &p, size_t N, size_t K, bool accumulate)
 {
     const long items = p.n_items;
+    if (g_force_tq == 0 && N <= 32 && !accumulate) return N <= 16 ? 16 : 32;
     int tq = 1;
     if (N >= 128 && items * (long)(N / 128) >= 2048 && p.n_cols >= (int64_t)items * 384) tq = 2;
     if (g_force_tq == 1 || g_force_tq == 2) tq = g_force_tq;
     while (tq > 1 && K * (size_t)(64 * tq) * sizeof(uint16_t) > ((size_t)128 << 20)) tq >>= 1;
-    return tq;
+    return 64 * tq;
 }
 
 hipError_t launch_compact(const CompactArgs &a_in, hipStream_t st)
@@ -857,9 +881,12 @@ hipError_t launch_compact(const CompactArgs &a_in, hipStream_t st)
     // rows of B that the gathers hit at random come from one panel at a time: a panel is kept under half of the
     // 256 MiB memory-side cache (the lists of A and the rows of C stream through it too).  On a 2^20-row B at
     // N = 128 the panel of 64 columns (128 MiB) takes 0.74 x the time of the panel of 128.
-    const int tq = compact_panel_width(*a.plan, a.N, a.K);
-    if (tq == 2) e = launch_compact_tq<2>(a, st);
-    else e = launch_compact_tq<1>(a, st);
+    switch (compact_panel_width(*a.plan, a.N, a.K, a.accumulate)) {
+    case 128: e = launch_compact_as<128>(a, st); break;
+    case 32: e = launch_compact_as<32>(a, st); break;
+    case 16: e = launch_compact_as<16>(a, st); break;
+    default: e = launch_compact_as<64>(a, st);
+    }
     if (e != hipSuccess) return e;
     if (a.plan->n_split_rows > 0)
         e = launch_reduce(a.plan->d_workspace, a.plan->d_split, a.plan->n_split_rows, a.C, a.N, a.c_f32, st);
@@ -875,11 +902,11 @@ hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t
     // launch before left in the L2s, and how many of them hold a line of it follows from the deal (16384^2, 0.1 %, N = 256: the
     // product kernel alone is fastest in runs of 128, 10.9 against 11.9 us; launch after launch it is 64, 19.8 against 21.4.
     // 8192 x 16384, 24 a row, N = 512: 24.2 against 27.1 in runs of 32 and 128).
-    const int tq = compact_panel_width(p, N, K);
-    const int n_panels = (int)((N + 64 * tq - 1) / (64 * tq));
+    const int width = compact_panel_width(p, N, K, accumulate);
+    const int n_panels = (int)((N + width - 1) / width);
     const long wgs = ((long)p.n_tasks * n_panels + 3) / 4;
     const unsigned eighth = (unsigned)std::max<long>((wgs + 7) / 8, 1);
-    // the run length of an untuned launch, as launch_compact_tq computes it for this N
+    // the run length of an untuned launch, as launch_compact_as computes it for this N
     const unsigned base = std::min(eighth, p.deal.run((size_t)p.n_tasks, n_panels));
     constexpr int MAX_RUNS = 4;
     unsigned runs[MAX_RUNS] = {base};
