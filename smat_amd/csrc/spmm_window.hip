@@ -571,7 +571,10 @@ double window_choose(const WindowWidths &w, size_t M, size_t K, size_t N, size_t
     for (int i = 0; i < WINDOW_SIZES; i++) {
         if (w.most[i] == 0 || (g_force_rows && SIZES[i] != g_force_rows)) continue;
         for (int t : {1, 2, 4}) {
-            const double e = window_estimate_us(SIZES[i], (int)((w.most[i] + 3) / 4 * 4), w.sum[i], t, M, K, N, nnzb, most_blocks, false);
+            double e = window_estimate_us(SIZES[i], (int)((w.most[i] + 3) / 4 * 4), w.sum[i], t, M, K, N, nnzb, most_blocks, false);
+            // Nothing shared: the pieces that the copies bring are single blocks, 32 bytes of a column (1376 x 5344, 4 %, N = 896: estimate 9.8,
+            // 13.6 us, row-wise 11.4; 12656 x 832, 6 %, N = 352 11.4 -> 8.4 all the same).
+            if ((double)w.sum[i] > 0.8 * (double)nnzb) e *= 1.25;
             if (e < best) best = e, *size = i;
         }
     }
