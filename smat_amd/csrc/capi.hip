@@ -205,6 +205,12 @@ static double rowwise_estimate_us(size_t M, size_t K, size_t N, size_t nnzb, siz
 // with N = 2040, rows that straddle cache lines, 50 against 43).
 static double to_col_major_us(size_t K, size_t N) { return 2.0 + 0.6e-6 * (double)K * (double)N; }
 static double sweep_in_place_factor(size_t N) { return N % 64 == 0 ? 1.05 : 1.13; }
+// The compact kernel and the pass over a column-major B before it: gathers of whole panels of 16, 32 or 64 columns.  27 stencils, N = 8 to
+// 256: 11 % standard deviation.
+static double compact_estimate_us(int64_t cols, size_t K, size_t N)
+{
+    return 6.0 + (double)cols * (double)(N <= 16 ? 16 : N <= 32 ? 32 : (N + 63) / 64 * 64) * 2.0 / 10e6 + (double)K * (double)N / 1e6;
+}
 static size_t sweep_listed_chunks(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t group_rows)
 {
     std::vector<size_t> seen((kb + SWEEP_S - 1) / SWEEP_S, 0); // the last row group that listed the chunk, from 1
@@ -357,6 +363,9 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
             c.accumulate = plan->sweep_blocks.d_ops != nullptr;
             e = launch_compact(c, static_cast<hipStream_t>(o.stream));
         }
+    } else if (kernel == SMAT_KERNEL_COMPACT && o.kernel == SMAT_KERNEL_AUTO && plan->window && o.b_layout == SMAT_B_COL_MAJOR && N <= plan->n_cap &&
+               (N == plan->n_cap || window_forced() || window_launch_us(a, *plan->window) < 0.9 * compact_estimate_us(plan->compact->n_cols, K, N))) {
+        e = launch_window(a, *plan->window, static_cast<hipStream_t>(o.stream));
     } else if (kernel == SMAT_KERNEL_COMPACT) {
         if (!plan || !plan->compact || !plan->d_bt || N > plan->n_cap)
             return set_error(SMAT_ERR_INVALID,
@@ -375,7 +384,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
     } else {
         bool window = plan && plan->window && o.kernel == SMAT_KERNEL_AUTO;
         if (window && N != plan->n_cap && !window_forced()) // made for another width
-            window = !rowwise_shares_items(N, (size_t)plan->n_items, nnzb / (size_t)plan->n_items) && window_launch_us(*plan->window, M, K, N, nnzb, a.c_f32) <
+            window = !rowwise_shares_items(N, (size_t)plan->n_items, nnzb / (size_t)plan->n_items) && window_launch_us(a, *plan->window) <
                      rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, RowLengths::EVEN, a.b_packed != nullptr);
         e = window ? launch_window(a, *plan->window, static_cast<hipStream_t>(o.stream)) : launch_rowwise(a, static_cast<hipStream_t>(o.stream));
     }
@@ -717,19 +726,20 @@ static hipError_t sweep_small_groups(smat_plan &p, size_t group_rows)
 // estimate is below 0.9 of the row-wise kernel's and of other_us, the time of what else there is; both are off by 10 %.  Row-wise
 // -> windows, us: 27-point stencil 64^3, N = 64 90 -> 56, 48^3, N = 256 111 -> 59, 48 x 25 x 48, N = 56 20.4 -> 12.7; bands of
 // 14224 rows and 182, N = 544 33 -> 17, of 65536 and 20, N = 256 30 -> 15, of 8960 and 120, N = 48 7.4 -> 5.
-static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us)
+// census: of the values, where the compact kernel would multiply: the window kernel then multiplies what it would, the values as attached.
+static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us, const uint16_t *vals, const CompactCensus *census)
 {
     const size_t mb = p.M / 16, kb = p.K / 16;
     if (p.kernel != SMAT_KERNEL_ROWWISE || p.kernel_requested != SMAT_KERNEL_AUTO || p.n_split_rows || !window_takes_rows(p.max_item_blocks)) return hipSuccess;
-    if (rowwise_shares_items(p.n_cap, (size_t)p.n_items, p.nnzb / std::max<size_t>((size_t)p.n_items, 1)) && !window_forced()) return hipSuccess;
-    if (p.n_cap <= 16 && !window_forced()) return hipSuccess; // 18 -> 17, 10.4 -> 9.2, but 8.2 -> 9, 6.6 -> 7
+    if (!census && rowwise_shares_items(p.n_cap, (size_t)p.n_items, p.nnzb / std::max<size_t>((size_t)p.n_items, 1)) && !window_forced()) return hipSuccess;
+    if (!census && p.n_cap <= 16 && !window_forced()) return hipSuccess; // 18 -> 17, 10.4 -> 9.2, but 8.2 -> 9, 6.6 -> 7
     // its estimate knows nothing of the bytes that come from memory, A above all and three times B where that is repacked: 64^3 64 us and
     // 64 us of bytes, measured 90; 73 x 61 x 62, N = 88 104 and 72, 125; 44 x 47 x 66, N = 40 31 and 26, 38
-    const double once = ((double)p.nnzb * 512.0 + 2.0 * (double)(p.K + p.M) * (double)p.n_cap) / 5e6;
+    const double once = ((census ? 4.0 * (double)census->nnz + 12.0 * (double)p.nnzb : 512.0 * (double)p.nnzb) + 2.0 * (double)(p.K + p.M) * (double)p.n_cap) / 5e6;
     const double row_wise = std::hypot(rowwise_estimate_us(p.M, p.K, p.n_cap, p.nnzb, (size_t)p.n_items, RowLengths::EVEN, p.d_bpack != nullptr),
                                        once + (p.d_bpack ? 4.0 * (double)p.K * (double)p.n_cap / 5e6 : 0.0));
     const double copy = p.d_bcol ? to_col_major_us(p.K, p.n_cap) : 0.0; // before either
-    const double bar = 0.9 * std::min(row_wise, other_us - copy);
+    const double bar = 0.9 * (census ? other_us - copy : row_wise);
     // a launch, or the bytes that windows do not save
     if (!window_forced() && bar < std::max(4.7, 2.0 + once)) return hipSuccess;
     WindowWidths widths;
@@ -741,11 +751,19 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
         if (e != hipSuccess) return e;
     }
     int size;
-    const double us = window_choose(widths, p.M, p.K, p.n_cap, p.nnzb, p.max_item_blocks, &size);
+    const double us = window_choose(widths, WindowProduct{p.M, p.K, p.n_cap, p.nnzb, census ? census->nnz : -1, p.max_item_blocks, false}, &size);
     if (size < 0 || (!window_forced() && us >= bar)) return slots ? dev_free(slots) : hipSuccess;
-    return window_build(widths, size, slots, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, &p.window);
+    hipError_t e = window_build(widths, size, slots, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, &p.window);
+    if (e != hipSuccess || !census) return e;
+    bool taken;
+    e = window_attach_entries(*p.window, vals, row_ptr, (const unsigned long long *)census->offset.p, mb, p.nnzb, census->nnz, &taken);
+    if (e != hipSuccess || !taken) {
+        window_destroy(p.window);
+        p.window = nullptr;
+    }
+    return e;
 }
-hipError_t smat::plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx) { return take_window(*p, row_ptr, col_idx, 1e30); }
+hipError_t smat::plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx) { return take_window(*p, row_ptr, col_idx, 1e30, nullptr, nullptr); }
 
 static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, const int32_t *row_ptr,
                                         const int32_t *col_idx, const int32_t *row_ptr_host)
@@ -886,10 +904,9 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
             group_rows = sweep_group_rows(row_ptr_host, p->col_idx_host.data(), p->M, p->K, p->nnzb, p->n_cap, (size_t)p->n_items,
                                           p->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, p->d_bpack != nullptr, p->d_bcol != nullptr);
         if (group_rows) e = sweep_small_groups(*p, group_rows);
-        else e = take_window(*p, row_ptr, col_idx,
-                             take ? (double)census.n_cols_all * (double)(p->n_cap <= 16 ? 16 : p->n_cap <= 32 ? 32 : (p->n_cap + 63) / 64 * 64) * 2.0 / 10e6 + (p->d_bcol ? 3.0 : t_pass) : 1e30);
+        else if (!take || !p->d_bcol)
+            e = take_window(*p, row_ptr, col_idx, compact_estimate_us(census.n_cols_all, p->K, p->n_cap), vals, take ? &census : nullptr);
         if (e != hipSuccess) return fail(e);
-        if (p->window) take = false;
     }
     if (!take) return SMAT_OK; // nothing would use the list: the plan keeps (or goes back to) a dense kernel
     if (!c) e = compact_build(census, vals, row_ptr, col_idx, p->K, p->n_cap, p->d_bcol != nullptr, mixed ? &dense : nullptr, false, &c);
@@ -961,7 +978,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     p->kernel = mixed || block_split ? SMAT_KERNEL_MIXED : SMAT_KERNEL_COMPACT;
     // the deal of the compact kernel's work items to the XCDs, measured on this list at the plan's width (B in the
     // layout the plan was made for: d_bcol is the scratch of a plan for row-major B)
-    e = compact_tune(*c, p->d_bt, p->M, p->n_cap, p->K, p->d_bcol != nullptr, block_split);
+    if (!p->window) e = compact_tune(*c, p->d_bt, p->M, p->n_cap, p->K, p->d_bcol != nullptr, block_split); // else its launches are not what the plan is for
     if (e != hipSuccess) return set_error(SMAT_ERR_HIP, "timing the compact kernel failed: %s", hipGetErrorString(e));
     if (p->d_bpack && want == SMAT_KERNEL_AUTO && !mixed) { // the row-wise kernel's scratch is not needed any more
         (void)dev_free(p->d_bpack);

@@ -184,20 +184,33 @@ struct WindowPlan {
     int most_blocks = 0;                 // of a block row
     int32_t *d_window = nullptr, *d_count = nullptr; // window of group i: d_count[i] first columns from d_window[i * cap] on
     uint32_t *d_slot = nullptr;          // of every block: its place in the window, and its block column
+    // With attached values: the nonzeros instead of the blocks, and the pattern as it was then (window_entries_kernel).
+    int64_t nnz = -1;
+    uint32_t *d_entries = nullptr, *d_table = nullptr;
+    int32_t *d_blocks = nullptr;
+};
+struct WindowProduct {
+    size_t M, K, N, nnzb;
+    int64_t nnz; // -1: whole blocks
+    int most_blocks; // of a block row
+    bool c_f32;
 };
 // row_ptr / col_idx: device arrays.  All but the launch and the estimates are synchronous, on the default stream.
 // *slots: memory for the entries of the blocks, which window_build takes over (or NULL).
 hipError_t window_widths(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, WindowWidths &out, void **slots);
 void window_widths_host(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, WindowWidths &out); // the same from host arrays
 // The size of group (index into the widths, -1 = none fits) that is fastest for a product of N columns, and its time in us.
-double window_choose(const WindowWidths &w, size_t M, size_t K, size_t N, size_t nnzb, int most_blocks, int *size);
+double window_choose(const WindowWidths &widths, const WindowProduct &w, int *size);
 hipError_t window_build(const WindowWidths &w, int size, void *slots, const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, int most_blocks,
                         WindowPlan **out);
 void window_destroy(WindowPlan *p);
 bool window_forced(); // by the test hook
 bool window_takes_rows(int most_blocks); // block rows of so many blocks
-double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, size_t M, size_t K, size_t N, size_t nnzb, int most_blocks, bool c_f32);
-double window_launch_us(const WindowPlan &p, size_t M, size_t K, size_t N, size_t nnzb, bool c_f32); // 1e30: not at this N
+// offset: of every block, the nonzeros before it in the upper half.  *taken: false where a pair of blocks has too many.
+hipError_t window_attach_entries(WindowPlan &p, const uint16_t *vals, const int32_t *row_ptr, const unsigned long long *offset, size_t mb, size_t nnzb, int64_t nnz,
+                                 bool *taken);
+double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, const WindowProduct &w);
+double window_launch_us(const SpmmArgs &a, const WindowPlan &p); // 1e30: not at this N
 hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st); // column-major B
 hipError_t launch_sweep(const SweepArgs &a, hipStream_t st);
 // Whether the sweep kernel reads a row-major B of this size in place; otherwise B is brought into column-major order first, one

@@ -27,6 +27,7 @@ namespace smat {
 namespace {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int COPIES = 7;               // KiB of a window that a wavefront copies at a time
 constexpr int SLOT_BITS = 10;           // of a block's entry: its place in the window; above them its block column
@@ -34,6 +35,10 @@ constexpr int BITMAP_WORDS = 8192;      // block columns of the matrix / 32
 constexpr size_t MAX_LDS = 160 * 1024;  // of a compute unit
 constexpr int CU_WAVES = 16;            // wavefronts of 128 registers on a compute unit
 constexpr int SIZES[WINDOW_SIZES] = {4, 8, 16}; // block rows of a group
+// block pairs of a row that a wavefront holds
+constexpr int MAX_PAIRS = 17;
+template <int TN> constexpr int pairs_held = TN == 4 ? 12 : MAX_PAIRS;
+constexpr int LIST_BITS = 26; // of a pair's list: the fours of entries before it; above them its own fours
 
 // ---- which block columns a group uses ----
 
@@ -120,44 +125,82 @@ __global__ __launch_bounds__(256) void window_list_kernel(const int32_t *__restr
     }
 }
 
-// ---- the product ----
-
-// Waits until at most n of the wavefront's vector memory operations are under way (they end in order).
-__device__ __forceinline__ void wait_vector_memory(int n)
+// The nonzeros of the blocks, pair by pair of a block row: value << 16 | byte in the pair's MFMA operand, filled up to a multiple of
+// four with the last one.  table: MAX_PAIRS pairs a block row, the places of the two blocks in the window (16 bits each) and the list, the fours of
+// entries before it and its own << LIST_BITS; behind the table the blocks of every row.  A wavefront takes a block row; offset[p]: nonzeros before
+// block p in the upper half.  Bound by the read of the values.
+__global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr,
+                                                             const uint32_t *__restrict__ slot, const unsigned long long *__restrict__ offset, int mb,
+                                                             uint32_t *__restrict__ entries, uint32_t *__restrict__ table, uint32_t *__restrict__ most)
 {
-#define SMAT_WAIT(I) case I: asm volatile("s_waitcnt vmcnt(" #I ")" ::: "memory"); break;
-    switch (n) {
-        SMAT_WAIT(1) SMAT_WAIT(2) SMAT_WAIT(3) SMAT_WAIT(4) SMAT_WAIT(5) SMAT_WAIT(6) SMAT_WAIT(7) SMAT_WAIT(8) SMAT_WAIT(9) SMAT_WAIT(10)
-        SMAT_WAIT(11) SMAT_WAIT(12) SMAT_WAIT(13) SMAT_WAIT(14) SMAT_WAIT(15) SMAT_WAIT(16) SMAT_WAIT(17) SMAT_WAIT(18) SMAT_WAIT(19)
-        SMAT_WAIT(20) SMAT_WAIT(21) SMAT_WAIT(22)
-    default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int lane = threadIdx.x & 63, br = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (br >= mb) return;
+    const int p0 = row_ptr[br], blocks = row_ptr[br + 1] - p0;
+    const int sel = lane >> 5, at = (lane & 15) * 16 + ((lane >> 4) & 1) * 8;
+    if (lane == 0) table[(long)mb * (2 * MAX_PAIRS) + br] = (uint32_t)blocks;
+    uint32_t longest = 0;
+    auto load = [&](int d) {
+        const int b = 2 * d + sel;
+        return b < blocks ? *reinterpret_cast<const u32x4 *>(vals + (long)(p0 + b) * 256 + at) : (u32x4){0u, 0u, 0u, 0u};
+    };
+    u32x4 w = load(0);
+    for (int d = 0; d < MAX_PAIRS; d++) {
+        const u32x4 now = w;
+        w = load(d + 1);
+        uint32_t *const to = table + (long)br * (2 * MAX_PAIRS) + 2 * d;
+        if (2 * d >= blocks) {
+            if (lane < 2) to[lane] = 0;
+            continue;
+        }
+        uint32_t n = 0, before = 0; // nonzeros of the pair, and of the lanes before this one
+        uint32_t bits = 0;
+#pragma unroll
+        for (int k = 0; k < 8; k++) { // -0.0 is a zero
+            const bool has = (now[k / 2] >> (k & 1 ? 16 : 0) & 0x7fffu) != 0;
+            bits |= (uint32_t)has << k;
+            const unsigned long long all = __ballot(has);
+            n += __popcll(all);
+            before += __popcll(all & ((1ull << lane) - 1ull));
+        }
+        const uint32_t first = ((uint32_t)(offset[p0 + 2 * d] >> 32) + 8u * (uint32_t)((p0 + br + 1) / 2 + d)) & ~3u, end = (n + 3u) & ~3u;
+        uint32_t i = before;
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            if (bits >> k & 1) {
+                const uint32_t e = (now[k / 2] >> (k & 1 ? 16 : 0)) << 16 | (uint32_t)(lane * 16 + k * 2);
+                entries[first + i] = e;
+                if (++i == n)
+                    for (; i < end; i++) entries[first + i] = e;
+            }
+        if (lane == 0) {
+            const int b = p0 + 2 * d;
+            const uint32_t s0 = slot[b] & ((1u << SLOT_BITS) - 1u), s1 = 2 * d + 1 < blocks ? slot[b + 1] & ((1u << SLOT_BITS) - 1u) : s0;
+            to[0] = s0 | s1 << 16;
+            to[1] = first / 4 | min(end / 4, (1u << (32 - LIST_BITS)) - 1u) << LIST_BITS;
+        }
+        longest = max(longest, end);
     }
-#undef SMAT_WAIT
+    if (lane == 0 && longest > 4 * ((1u << (32 - LIST_BITS)) - 1)) atomicMax(most, longest); // too many for a pair
 }
 
-// A workgroup goes through steps: a part of a panel (16 TN columns) of a group.  While it multiplies one from one half of its
-// LDS, the window of the next is copied to the other half; the A operands of a wavefront's block row stay in its registers for all
-// panels of a unit and are replaced, pair by pair, by those of the next unit's row as the last part is done with them.
-//
-// Bound by what a step costs beside its work: with 16 wavefronts on a compute unit (128 registers each) a step of the 27-point
-// stencil on 48^3, N = 256 takes 3 us, of which copies alone would be 1.9 and LDS reads and MFMAs alone 1.9 (timed with the rest
-// taken out), and the two overlap by half; on 64^3 at N = 64 the read of A, 185 MB, from HBM is as long (49 us for all its bytes at
-// the rate of a copy).  Us, row-wise kernel -> windows, step by step: 48^3, N = 256 111 -> one workgroup a group and panel, window and A asked
-// for and waited for in turn 88 -> steps, two halves of LDS, A kept for all panels 68 -> parts unrolled, loads counted instead of all
-// waited for, 128 bytes of a row of C at a time 59; 64^3, N = 64 90 -> 62 -> 66 -> 56; band of 65536 and 20, N = 256 30 -> 21 -> 16 -> 15.
-// What the panel width costs: 16 columns instead of 32 on 48^3 66, on 64^3 63; groups of 8 instead of 16 66 and 58.
-//
-// The row-wise kernel reads the pattern where it lies, so this one does: it compares the block columns with those its windows were
-// made of and takes a row that has other ones from memory.
-//
-// block pairs of a row that a wavefront holds
-template <int TN> constexpr int pairs_held = TN == 4 ? 12 : 17;
+// ---- the product ----
 
-template <int TN, int PARTS, bool C_F32>
+// Waits until at most n of the wavefront's vector memory operations are under way (they end in order), or a few less.
+__device__ __forceinline__ void wait_vector_memory(int n)
+{
+    if (n < 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (n < 4) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    else if (n < 6) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    else if (n < 10) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    else if (n < 14) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(14)" ::: "memory");
+}
+
+template <int TN, int PARTS, bool C_F32, bool ENTRIES>
 __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr,
                                                            const int32_t *__restrict__ col_idx, const uint16_t *__restrict__ B, void *__restrict__ Cout,
                                                            const int32_t *__restrict__ window, const int32_t *__restrict__ count,
-                                                           const uint32_t *__restrict__ slot, int mb, int rows, int cap, int n_groups, int n_panels,
+                                                           const uint32_t *__restrict__ slot, const uint32_t *__restrict__ entries, int mb, int rows, int cap, int n_groups, int n_panels,
                                                            int panels_per_unit, int N, long K)
 {
     constexpr int NP = pairs_held<TN>, U = TN == 4 ? 1 : 2, TILES = TN * PARTS;
@@ -187,7 +230,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
     const int i16 = lane & 15, g = lane >> 4, sel = g >> 1, kh = g & 1;
 
     const uint32_t lbase = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)lds;
-    const uint32_t buffer = (uint32_t)cap * (P * 32);
+    const uint32_t buffer = ENTRIES ? (uint32_t)max(cap * (P * 32), rows * 1024) : (uint32_t)cap * (P * 32);
     // Piece o of column c of a quad lies at place o ^ swizzle(c) of its 128 bytes: the 16 columns that an operand takes lie in different banks.
     auto swizzle = [](uint32_t c) { return ((c >> 1) & 1u) | ((c / (P / 4)) & 3u) << 1; };
     // the lane, for addresses that are made anew where they are used instead of being kept in registers
@@ -202,15 +245,24 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
     // The block row of a wavefront in a group: what is asked for, and what is made of it.
     struct Asked {
         int p0, blocks;
-        uint32_t q0, q1, c0, c1; // lane j: blocks 2 j and 2 j + 1
+        uint32_t q0, q1, c0, c1; // lane j: blocks 2 j and 2 j + 1; ENTRIES: their places in q0, their entries in q1
     };
     struct Row {
         int p0, blocks;  // blocks: 0 where the wavefront has none
         uint32_t packed; // lane j: places of blocks 2 j and 2 j + 1 in the window, in 32 bytes
         bool known;
     };
+    uint32_t list = 0; // ENTRIES: of the row taken last, lane j: the entries of blocks 2 j and 2 j + 1
     auto ask_row = [&](int gr, Asked &r) {
         const int br = gr * rows + wave, b = br < mb ? br : mb - 1;
+        if constexpr (ENTRIES) { // a table of MAX_PAIRS pairs a block row, and the blocks of every row behind it
+            r.p0 = 0;
+            r.blocks = br < mb ? __builtin_amdgcn_readfirstlane(row_ptr[b]) : 0;
+            const uint32_t at = (uint32_t)min(lane_here(), MAX_PAIRS - 1) * 8u;
+            load_dword(r.q0, slot + (long)b * (2 * MAX_PAIRS), at);
+            load_dword(r.q1, slot + (long)b * (2 * MAX_PAIRS), at + 4u);
+            return;
+        }
         r.p0 = __builtin_amdgcn_readfirstlane(row_ptr[b]);
         r.blocks = br < mb ? __builtin_amdgcn_readfirstlane(row_ptr[b + 1]) - r.p0 : 0;
         if (r.blocks <= 0) r.blocks = 0, r.p0 = 0;
@@ -223,6 +275,11 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
     };
     auto place = [&](uint32_t q) { return (q & ((1u << SLOT_BITS) - 1u)) / 4 * (QUAD_BYTES / 32) + (q & 3u); };
     auto take_row = [&](Asked &r) {
+        if constexpr (ENTRIES) {
+            asm volatile("" : "+v"(r.q0), "+v"(r.q1));
+            list = r.q1;
+            return Row{0, r.blocks, place(r.q0 & 0xffffu) | place(r.q0 >> 16) << 16, true};
+        }
         asm volatile("" : "+v"(r.q0), "+v"(r.q1), "+v"(r.c0), "+v"(r.c1));
         const bool same = (r.q0 >> SLOT_BITS) * 16u == r.c0 && (r.q1 >> SLOT_BITS) * 16u == r.c1;
         return Row{r.p0, r.blocks, place(r.q0) | place(r.q1) << 16, r.blocks <= 2 * NP && (r.blocks == 0 || __all(same))};
@@ -231,8 +288,25 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
 #pragma unroll
     for (int d = 0; d < NP; d++) a[d] = (f16x8){0, 0, 0, 0, 0, 0, 0, 0};
     // Pair d of a row to a[d] where d < n: through a buffer that ends with the row, so that what is past its end is zero.
+    // ENTRIES: the pair's entries, four a lane, until build_a makes the operand of them.
     const uint32_t a_off = (uint32_t)(sel * 512 + i16 * 32 + kh * 16);
     auto load_a = [&](int d, const Row &r, int n) {
+        if constexpr (ENTRIES) {
+            // lanes past the list read past the end of the buffer: zeros, and no traffic
+            const uint32_t part_of = (uint32_t)__builtin_amdgcn_readlane((int)list, d);
+            const uint32_t l = (uint32_t)lane_here();
+            const uint32_t at = l < part_of >> LIST_BITS ? (part_of + l) << (32 - LIST_BITS) >> (32 - LIST_BITS - 4) : ~0u;
+            i32x4 all;
+            all[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)entries);
+            all[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)((uintptr_t)entries >> 32) & 0xffff);
+            all[2] = (int)(16u << LIST_BITS);
+            all[3] = 0x00020000;
+            asm volatile("s_cmp_le_i32 %3, %4\n\ts_cbranch_scc1 .Lskip%=\n\tbuffer_load_dwordx4 %0, %1, %2, 0 offen\n.Lskip%=:"
+                         : "+v"(a[d])
+                         : "v"(at), "s"(all), "s"(n), "n"(d)
+                         : "scc");
+            return;
+        }
         i32x4 row;
         const uint64_t base = (uint64_t)(uintptr_t)(vals + (long)r.p0 * 256);
         row[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)base);
@@ -245,6 +319,30 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
                      : "+v"(a[d]), "=&v"(tmp)
                      : "v"(a_off), "s"(row), "s"(n), "n"(d), "s"(d * 1024)
                      : "scc");
+    };
+    // ENTRIES: the operands of the row from its entries, through 1 KiB of LDS that this wavefront's next copies will overwrite.
+    auto build_a = [&](const Row &r, uint32_t tile) {
+        typedef __attribute__((address_space(3))) uint16_t lds_half;
+        typedef __attribute__((address_space(3))) u32x4 lds_quad;
+        const uint32_t mine = tile + (uint32_t)lane * 16u;
+        auto clear = [&] { *(lds_quad *)(uintptr_t)mine = (u32x4){0u, 0u, 0u, 0u}; };
+        clear();
+#pragma unroll
+        for (int d = 0; d < NP; d++) {
+            if (2 * d < r.blocks) {
+                const uint32_t fours = (uint32_t)__builtin_amdgcn_readlane((int)list, d) >> LIST_BITS;
+                const u32x4 e = __builtin_bit_cast(u32x4, a[d]);
+                asm volatile("" ::: "memory");
+                if ((uint32_t)lane < fours)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) *(lds_half *)(uintptr_t)(tile + (e[i] & 0x3ffu)) = (uint16_t)(e[i] >> 16);
+                asm volatile("" ::: "memory");
+                a[d] = __builtin_bit_cast(f16x8, *(lds_quad *)(uintptr_t)mine);
+                asm volatile("" ::: "memory");
+                clear();
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
     // pairs to load: a multiple of U, the last ones zeros
     auto loads_of = [&](const Row &r) { return min(((r.blocks + 1) / 2 + U - 1) / U * U, NP); };
@@ -273,7 +371,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
         for (int t = 0; t < COPIES; t++) asm volatile("" : "+v"(from_k[t]));
     };
     // a part's columns of the window to LDS; returns the instructions
-    auto stage = [&](int pan, int part, uint32_t dst) {
+    auto stage = [&](int pan, int part, uint32_t dst, int t0 = 0, int t1 = COPIES) { // the t0-th to t1-th of the wavefront
         const int n0 = pan * PANEL + part * (P / 4);
         const uint64_t base = (uint64_t)(uintptr_t)(B + (long)n0 * K);
         const int lane = lane_here();
@@ -284,7 +382,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
 #pragma unroll
         for (int t = 0; t < COPIES; t++) {
             const int q = copy_quad + t * quads_apart;
-            if (q < quads) {
+            if (t >= t0 && t < t1 && q < quads) {
                 asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(from + 2u * from_k[t]), "s"(base),
                              "s"(dst + (uint32_t)(q * QUAD_BYTES) + (uint32_t)copy_part * 1024u)
                              : "memory");
@@ -339,7 +437,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
                     for (int t = 0; t < TN; t++) bv[u][t] = *(const __attribute__((address_space(3))) f16x8 *)(uintptr_t)(b + t * 512);
                 }
                 if (2 * (d0 + U) > blocks) { // what is past the end of the row: zeros times zeros
-                    asm volatile("");
+                    const int sel = lane_here() >> 5;
 #pragma unroll
                     for (int u = 0; u < U; u++)
 #pragma unroll
@@ -373,8 +471,13 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
     stage(panel, 0, lbase);
 #pragma unroll
     for (int d = 0; d < NP; d++) load_a(d, row, loads_of(row));
+    const uint32_t tile = lbase + (uint32_t)(copy_quad * QUAD_BYTES + copy_part * 1024); // of build_a, in either half
+    if constexpr (ENTRIES) {
+        wait_a(0);
+        build_a(row, tile + buffer);
+    }
     Unit soon = unit_after(here_unit);
-    bool loaded = true, ahead = false; // a[] is under way; the row of the unit after next is
+    bool loaded = !ENTRIES, ahead = false; // a[] is under way; the row of the unit after next is
     if (PARTS == 1 && is_last(here_unit, panel) && soon.unit < my_units) {
         ask_window(soon.group);
         ask_row(soon.group, asked);
@@ -387,11 +490,25 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
         ahead = false;
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // A part's copies, and on the way the operands of the row, where they are new: ENTRIES makes them in the place of its first copy.
+    auto stage_and_take_a = [&](int pan, int part, bool copy) {
+        const uint32_t to = buf ^ buffer;
+        if constexpr (ENTRIES) {
+            if (loaded) {
+                const int copies = copy ? stage(pan, part, lbase + to, 1) : 0;
+                wait_a(copies);
+                build_a(row, tile + to);
+                if (copy) stage(pan, part, lbase + to, 0, 1);
+                return;
+            }
+        }
+        const int copies = copy ? stage(pan, part, lbase + to) : 0;
+        if (loaded) wait_a(copies);
+    };
     for (;;) { // a panel
         const bool last = is_last(here_unit, panel), more = !last || soon.unit < my_units;
         if constexpr (PARTS == 2) {
-            const int copies = stage(panel, 1, lbase + (buf ^ buffer));
-            if (loaded) wait_a(copies);
+            stage_and_take_a(panel, 1, true);
             if (last && more) { // the unit's last copies are on their way: the window and the row of the next
                 ask_window(soon.group);
                 ask_row(soon.group, asked);
@@ -405,8 +522,11 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
             }
         }
         const int staged = last ? soon.end - panels_per_unit : panel + 1;
-        const int copies = more ? stage(staged, 0, lbase + (buf ^ buffer)) : 0;
-        if (loaded) wait_a(copies);
+        stage_and_take_a(staged, 0, more);
+        if (PARTS == 1 && ahead) {
+            next = take_row(asked);
+            ahead = false;
+        }
         loaded = last && more;
         if (PARTS == 1 && more && is_last(last ? soon : here_unit, staged)) {
             const Unit later = last ? unit_after(soon) : soon;
@@ -421,7 +541,10 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
         else multiply(std::integral_constant<int, PARTS - 1>(), std::false_type(), 0);
         asm volatile("" ::: "memory");
         const int br = here_unit.group * rows + wave, n0 = panel * PANEL;
-        if (br < mb) store_tile<TILES, C_F32>(acc, br, -1, n0, i16, g, Cout, nullptr, N);
+        if (br < mb) {
+            const int l = lane_here();
+            store_tile<TILES, C_F32>(acc, br, -1, n0, l & 15, l >> 4, Cout, nullptr, N);
+        }
         asm volatile("" ::: "memory");
         if (!more) break;
         // store instructions: at least so many where no column is past N
@@ -433,21 +556,18 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
             soon = unit_after(soon);
             panel = staged;
         } else panel++;
-        if (ahead) {
-            take_window();
-            next = take_row(asked);
-            ahead = false;
-        }
+        if (ahead) take_window();
     }
 }
 
 int g_force_rows = 0, g_force_tiles = 0; // test hook
 
+size_t lds_of(int rows, int cap, int tiles, bool entries) { return 2 * std::max((size_t)cap * tiles * 512, entries ? (size_t)rows * 1024 : 0); }
 // Whether windows of `cap` block columns fit: twice in LDS, and COPIES KiB a wavefront.
-bool fits(int rows, int cap, int tiles)
+bool fits(int rows, int cap, int tiles, bool entries)
 {
-    const size_t part = (size_t)cap * tiles * 512;
-    return cap < 1 << SLOT_BITS && rows % (2 * tiles) == 0 && part <= (size_t)COPIES * 1024 * rows && 2 * part <= MAX_LDS;
+    return cap < 1 << SLOT_BITS && rows % (2 * tiles) == 0 && (size_t)cap * tiles * 512 <= (size_t)COPIES * 1024 * rows &&
+           lds_of(rows, cap, tiles, entries) <= MAX_LDS;
 }
 // Parts of a panel: two where N is wider than one.
 int parts_of(int tiles, size_t N) { return tiles < 4 && N > (size_t)16 * tiles ? 2 : 1; }
@@ -457,11 +577,11 @@ struct Launch {
 };
 // The panels of a group are split into the units that leave the last round of workgroups fullest; half a panel more for every unit,
 // whose A is read again.
-Launch launch_of(int rows, int cap, int tiles, int n_groups, size_t N)
+Launch launch_of(int rows, int cap, int tiles, int n_groups, size_t N, bool entries)
 {
     const size_t panel = (size_t)16 * tiles * parts_of(tiles, N);
     Launch l{(int)((N + panel - 1) / panel), 0, 0, 0};
-    const int slots = 32 * std::max(1, std::min(CU_WAVES / rows, (int)(MAX_LDS / ((size_t)cap * tiles * 1024)))); // workgroups of an XCD at a time
+    const int slots = 32 * std::max(1, std::min(CU_WAVES / rows, (int)(MAX_LDS / lds_of(rows, cap, tiles, entries)))); // workgroups of an XCD at a time
     const int my_groups = (n_groups + 7) / 8;
     double best = 1e30;
     for (int split = 1; split <= std::min(l.n_panels, 64); split++) {
@@ -473,30 +593,30 @@ Launch launch_of(int rows, int cap, int tiles, int n_groups, size_t N)
     return l;
 }
 
-template <int TN, int PARTS, bool C_F32>
+template <int TN, int PARTS, bool C_F32, bool ENTRIES>
 hipError_t launch_as(const SpmmArgs &a, const WindowPlan &p, const Launch &l, hipStream_t st)
 {
     static std::atomic<uint64_t> prepared{0}; // devices on which the kernel may have that much LDS
-    const size_t lds = (size_t)p.cap * TN * 1024;
+    const size_t lds = lds_of(p.rows, p.cap, TN, ENTRIES);
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev >= 64 || !(prepared.load(std::memory_order_relaxed) >> dev & 1)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(spmm_window_kernel<TN, PARTS, C_F32>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MAX_LDS);
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(spmm_window_kernel<TN, PARTS, C_F32, ENTRIES>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MAX_LDS);
         if (e != hipSuccess) return e;
         if (dev < 64) prepared.fetch_or(1ull << dev, std::memory_order_relaxed);
     }
-    hipLaunchKernelGGL((spmm_window_kernel<TN, PARTS, C_F32>), dim3((unsigned)l.workgroups), dim3((unsigned)(p.rows * 64)), lds, st, a.vals, a.row_ptr, a.col_idx, a.B,
-                       a.C, p.d_window, p.d_count, p.d_slot, (int)(a.M / 16), p.rows, p.cap, p.n_groups, l.n_panels, l.panels_per_unit, (int)a.N, (long)a.K);
+    hipLaunchKernelGGL((spmm_window_kernel<TN, PARTS, C_F32, ENTRIES>), dim3((unsigned)l.workgroups), dim3((unsigned)(p.rows * 64)), lds, st, a.vals, ENTRIES ? p.d_blocks : a.row_ptr, a.col_idx, a.B,
+                       a.C, p.d_window, p.d_count, ENTRIES ? p.d_table : p.d_slot, p.d_entries, (int)(a.M / 16), p.rows, p.cap, p.n_groups, l.n_panels, l.panels_per_unit, (int)a.N, (long)a.K);
     return hipGetLastError();
 }
 
-int best_tiles(const WindowPlan &p, size_t M, size_t K, size_t N, size_t nnzb, bool c_f32, double *us)
+int best_tiles(const WindowPlan &p, const WindowProduct &w, double *us)
 {
     int tiles = 0;
     *us = 1e30;
     for (int t : {1, 2, 4}) {
-        const double e = window_estimate_us(p.rows, p.cap, p.sum, t, M, K, N, nnzb, p.most_blocks, c_f32);
+        const double e = window_estimate_us(p.rows, p.cap, p.sum, t, w);
         if (e < *us) *us = e, tiles = t;
     }
     return g_force_tiles && tiles ? g_force_tiles : tiles;
@@ -510,17 +630,27 @@ int best_tiles(const WindowPlan &p, size_t M, size_t K, size_t N, size_t nnzb, b
 // and pruned matrices, N = 8 to 1,000, three on their own inputs in turn: 10 % standard deviation, and the group and panel it picks are
 // 4 % from the best in the mean.  Estimate (measured), us: stencil 73 x 61 x 62, N = 88, groups of 8 80 (85); band of 52960 and 64, N = 472,
 // groups of 16 34 (34.5); band of 2144 and 47, N = 808, groups of 4 5.5 (5.6).
-double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, size_t M, size_t K, size_t N, size_t nnzb, int most_blocks, bool c_f32)
+// ENTRIES: the building of the operands besides, for every unit; fitted to 130 products of 27 stencils, N = 8 to 256: 9 %.  71 x 55 x 67,
+// N = 40 36 (35.5); 41 x 35 x 30, N = 208 22 (22.4); 72 x 51 x 40, N = 144 51 (62).
+double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, const WindowProduct &w)
 {
-    if (!fits(rows, cap, tiles) || most_blocks > 2 * (tiles == 4 ? pairs_held<4> : pairs_held<1>)) return 1e30;
-    const size_t mb = M / 16;
-    const Launch l = launch_of(rows, cap, tiles, (int)((mb + rows - 1) / rows), N);
-    const double parts = parts_of(tiles, N), units = (l.n_panels + l.panels_per_unit - 1) / l.panels_per_unit;
-    const double c_bytes = (double)M * (double)N * (c_f32 ? 4.0 : 2.0), a_bytes = (double)nnzb * 512.0;
-    const double steps = l.rounds * l.panels_per_unit * parts * (1.07 + 0.0155 * (double)nnzb / (double)mb * tiles);
-    const double path = ((double)sum * 512.0 * tiles * parts * l.n_panels + a_bytes * units + c_bytes) / 8.7e6;
-    const double memory = (a_bytes + 2.0 * (double)K * (double)N + c_bytes) / 5.0e6;
-    return std::max(4.7, 1.6 + 2.2 * rows / 16.0 + std::pow(std::pow(steps, 4.0) + std::pow(path, 4.0) + std::pow(memory, 4.0), 0.25));
+    const bool entries = w.nnz >= 0;
+    if (!fits(rows, cap, tiles, entries) || w.most_blocks > 2 * (tiles == 4 ? pairs_held<4> : pairs_held<1>)) return 1e30;
+    const size_t mb = w.M / 16;
+    const Launch l = launch_of(rows, cap, tiles, (int)((mb + rows - 1) / rows), w.N, entries);
+    const double parts = parts_of(tiles, w.N), units = (l.n_panels + l.panels_per_unit - 1) / l.panels_per_unit;
+    const double c_bytes = (double)w.M * (double)w.N * (w.c_f32 ? 4.0 : 2.0), a_bytes = entries ? 4.0 * (double)w.nnz + 12.0 * (double)w.nnzb : 512.0 * (double)w.nnzb;
+    const double blocks = (double)w.nnzb / (double)mb * tiles, groups16 = rows / 16.0, copies = (double)sum * 512.0 * tiles * parts * l.n_panels + a_bytes * units + c_bytes;
+    const double once = a_bytes + 2.0 * (double)w.K * (double)w.N + c_bytes;
+    double steps, path, memory, start;
+    if (entries) {
+        steps = l.rounds * (l.panels_per_unit * parts * (1.13 + 0.008 * blocks) + 1.3 + 2.5 * groups16);
+        path = copies / 11.9e6, memory = once / 2.4e6, start = 2.4;
+    } else {
+        steps = l.rounds * l.panels_per_unit * parts * (1.07 + 0.0155 * blocks);
+        path = copies / 8.7e6, memory = once / 5.0e6, start = 1.6 + 2.2 * groups16;
+    }
+    return std::max(4.7, start + std::pow(std::pow(steps, 4.0) + std::pow(path, 4.0) + std::pow(memory, 4.0), 0.25));
 }
 
 hipError_t window_widths(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, WindowWidths &out, void **slots)
@@ -564,17 +694,21 @@ void window_widths_host(const int32_t *row_ptr, const int32_t *col_idx, size_t m
         }
 }
 
-double window_choose(const WindowWidths &w, size_t M, size_t K, size_t N, size_t nnzb, int most_blocks, int *size)
+double window_choose(const WindowWidths &widths, const WindowProduct &w, int *size)
 {
     double best = 1e30;
     *size = -1;
     for (int i = 0; i < WINDOW_SIZES; i++) {
-        if (w.most[i] == 0 || (g_force_rows && SIZES[i] != g_force_rows)) continue;
+        if (widths.most[i] == 0 || (g_force_rows && SIZES[i] != g_force_rows)) continue;
         for (int t : {1, 2, 4}) {
-            double e = window_estimate_us(SIZES[i], (int)((w.most[i] + 3) / 4 * 4), w.sum[i], t, M, K, N, nnzb, most_blocks, false);
-            // Nothing shared: the pieces that the copies bring are single blocks, 32 bytes of a column (1376 x 5344, 4 %, N = 896: estimate 9.8,
-            // 13.6 us, row-wise 11.4; 12656 x 832, 6 %, N = 352 11.4 -> 8.4 all the same).
-            if ((double)w.sum[i] > 0.8 * (double)nnzb) e *= 1.25;
+            double e = window_estimate_us(SIZES[i], (int)((widths.most[i] + 3) / 4 * 4), widths.sum[i], t, w);
+            // Nothing shared: the pieces that the copies bring are single blocks, 32 bytes of a column, and from a B beyond an XCD's 4 MiB of L2 each
+            // costs a cache line (928 x 4160, 3 %, N = 3472: estimate 12, 27 us, row-wise 15; 1376 x 5344, 4 %, N = 896 9.8, 13.6 and 11.4;
+            // 12656 x 832, 6 %, N = 352 11.4 -> 8.4 all the same).
+            if ((double)widths.sum[i] > 0.8 * (double)w.nnzb) {
+                if (2 * w.K * w.N > (size_t)4 << 20) continue;
+                e *= 1.25;
+            }
             if (e < best) best = e, *size = i;
         }
     }
@@ -614,10 +748,36 @@ hipError_t window_build(const WindowWidths &w, int size, void *slots, const int3
     return hipSuccess;
 }
 
+hipError_t window_attach_entries(WindowPlan &p, const uint16_t *vals, const int32_t *row_ptr, const unsigned long long *offset, size_t mb, size_t nnzb, int64_t nnz,
+                                 bool *taken)
+{
+    *taken = false;
+    const size_t room = (size_t)nnz + 8 * ((nnzb + mb + 1) / 2 + MAX_PAIRS) + 16;
+    if (room / 4 >= (size_t)1 << LIST_BITS) return hipSuccess;
+    const size_t table = mb * (2 * MAX_PAIRS + 1);
+    hipError_t e = dev_malloc(&p.d_entries, (room + table + 1) * sizeof(uint32_t));
+    if (e != hipSuccess) return e;
+    p.d_table = p.d_entries + (room + 1) / 2 * 2; // pairs of words
+    p.d_blocks = reinterpret_cast<int32_t *>(p.d_table + mb * (2 * MAX_PAIRS));
+    p.nnz = nnz;
+    DevScratch most;
+    uint32_t too_many = 0;
+    e = most.alloc(sizeof too_many);
+    if (e == hipSuccess) e = hipMemsetAsync(most.p, 0, sizeof too_many, nullptr);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(window_entries_kernel, dim3((unsigned)((mb + 3) / 4)), dim3(256), 0, nullptr, vals, row_ptr, p.d_slot, offset, (int)mb, p.d_entries, p.d_table,
+                           (uint32_t *)most.p);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpy(&too_many, most.p, sizeof too_many, hipMemcpyDeviceToHost);
+    *taken = e == hipSuccess && too_many == 0;
+    return e;
+}
+
 void window_destroy(WindowPlan *p)
 {
     if (!p) return;
-    for (void *q : {(void *)p->d_window, (void *)p->d_slot})
+    for (void *q : {(void *)p->d_window, (void *)p->d_slot, (void *)p->d_entries})
         if (q) (void)dev_free(q);
     delete p;
 }
@@ -625,25 +785,36 @@ void window_destroy(WindowPlan *p)
 bool window_forced() { return g_force_rows > 0; }
 bool window_takes_rows(int most_blocks) { return most_blocks > 0 && most_blocks <= 2 * pairs_held<1>; }
 
-double window_launch_us(const WindowPlan &p, size_t M, size_t K, size_t N, size_t nnzb, bool c_f32)
+static WindowProduct product_of(const SpmmArgs &a, const WindowPlan &p)
+{
+    return WindowProduct{a.M, a.K, a.N, a.nnzb, p.nnz, p.most_blocks, a.c_f32};
+}
+double window_launch_us(const SpmmArgs &a, const WindowPlan &p)
 {
     double us;
-    (void)best_tiles(p, M, K, N, nnzb, c_f32, &us);
+    (void)best_tiles(p, product_of(a, p), &us);
     return us;
 }
 
 hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st)
 {
     double us;
-    const int tiles = best_tiles(p, a.M, a.K, a.N, a.nnzb, a.c_f32, &us);
-    if (tiles == 0 || !fits(p.rows, p.cap, tiles)) return hipErrorInvalidValue;
-    const Launch l = launch_of(p.rows, p.cap, tiles, p.n_groups, a.N);
-    const bool two = parts_of(tiles, a.N) == 2;
-    if (tiles == 4) return a.c_f32 ? launch_as<4, 1, true>(a, p, l, st) : launch_as<4, 1, false>(a, p, l, st);
-    if (tiles == 2 && two) return a.c_f32 ? launch_as<2, 2, true>(a, p, l, st) : launch_as<2, 2, false>(a, p, l, st);
-    if (tiles == 2) return a.c_f32 ? launch_as<2, 1, true>(a, p, l, st) : launch_as<2, 1, false>(a, p, l, st);
-    if (two) return a.c_f32 ? launch_as<1, 2, true>(a, p, l, st) : launch_as<1, 2, false>(a, p, l, st);
-    return a.c_f32 ? launch_as<1, 1, true>(a, p, l, st) : launch_as<1, 1, false>(a, p, l, st);
+    const int tiles = best_tiles(p, product_of(a, p), &us);
+    const bool entries = p.d_entries != nullptr;
+    if (tiles == 0 || !fits(p.rows, p.cap, tiles, entries)) return hipErrorInvalidValue;
+    const Launch l = launch_of(p.rows, p.cap, tiles, p.n_groups, a.N, entries);
+    auto as = [&](auto tn, auto parts) {
+        constexpr int TN = decltype(tn)::value, PARTS = decltype(parts)::value;
+        if (entries) return a.c_f32 ? launch_as<TN, PARTS, true, true>(a, p, l, st) : launch_as<TN, PARTS, false, true>(a, p, l, st);
+        return a.c_f32 ? launch_as<TN, PARTS, true, false>(a, p, l, st) : launch_as<TN, PARTS, false, false>(a, p, l, st);
+    };
+    using std::integral_constant;
+    const integral_constant<int, 1> one;
+    const integral_constant<int, 2> two;
+    const bool halves = parts_of(tiles, a.N) == 2;
+    if (tiles == 4) return as(integral_constant<int, 4>(), one);
+    if (tiles == 2) return halves ? as(two, two) : as(two, one);
+    return halves ? as(one, two) : as(one, one);
 }
 
 } // namespace smat

@@ -156,3 +156,65 @@ def test_which_products_take_windows(smat, cuda):
     assert rows(blocked(gen.band(512, 16)), 32) == 0
     assert rows(blocked(gen.band(8192, 400)), 256) == 0
     assert rows(gen.random_bcsr(128, 128, 0.2, seed=1), 512) == 0
+
+
+def sparse_values(nnzb, seed, most):
+    """Blocks of up to `most` nonzeros, some of none, small whole numbers."""
+    rng = np.random.default_rng(seed)
+    vals = np.zeros((nnzb, 256), np.float16)
+    for b in vals:
+        at = rng.choice(256, rng.integers(0, most + 1), replace=False)
+        b[at] = rng.choice([-3, -2, -1, 1, 2, 3], len(at))
+    return vals.reshape(-1).view(np.uint16)
+
+
+# lists of a pair around 0, a lane's four and what a wavefront holds (256); the last block of odd rows alone
+@pytest.mark.parametrize("mb,kb,width", [(1, 3, 2), (33, 33, 12), (130, 200, 34)])
+@pytest.mark.parametrize("most", [1, 40, 127])
+@pytest.mark.parametrize("rows,tiles,N", [(4, 1, 8), (8, 2, 24), (16, 1, 72), (16, 2, 136), (16, 4, 320)])
+def test_windows_of_listed_nonzeros_match_the_oracle(smat, cuda, oracle, force, mb, kb, width, most, rows, tiles, N):
+    import torch
+    if tiles == 4 and width > 24:
+        pytest.skip("rows of more than 24 blocks")
+    rp, ci, _ = local_matrix(mb, kb, width, seed=mb + rows, empty=(0, 2) if mb > 8 else ())
+    M, K, nnzb = mb * 16, kb * 16, len(ci)
+    vals, B = sparse_values(nnzb, most, most), whole_b(K, N, seed=N)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci, B)]
+    want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B, threads=4)
+    force(rows, tiles)
+    plan = smat.Plan(rp, M, K, nnzb, N, col_idx_host=ci)
+    plan.attach_values(d[0], d[1], d[2])
+    assert smat.lib.smat_internal_plan_window_rows(plan.handle) == rows
+    listed = plan.info()["kernel"] == smat.KERNEL_COMPACT
+    assert listed or most > 1  # a tenth of a block's columns or most of them
+    if listed:
+        d[0].zero_()  # the values are the ones attached
+    for n in {N, max(8, N * 3 // 4 // 8 * 8)}:
+        for c_f32 in (False, True):
+            for kernel in (smat.KERNEL_AUTO, smat.KERNEL_COMPACT) if listed else (smat.KERNEL_AUTO,):
+                C = torch.full((M, n), float("nan"), dtype=torch.float32 if c_f32 else torch.float16, device=cuda)
+                smat.spmm(d[0], d[1], d[2], d[3][:K * n], C, M, n, K, nnzb, plan=plan, c_f32=c_f32, kernel=kernel)
+                assert np.array_equal(C.cpu().numpy().astype(np.float32), want[:, :n].astype(np.float16 if not c_f32 else np.float32).astype(np.float32))
+    plan.close()
+
+
+def test_values_attached_again_replace_the_listed_ones(smat, cuda, oracle, force):
+    """Between lists, from a list to full blocks and back, and to columns too full for a list; a launch wider than the plan is refused as before."""
+    import torch
+    rp, ci, full = local_matrix(60, 60, 9, seed=4)
+    M = K = 960
+    N = 64
+    B = whole_b(K, N + 8, seed=6)
+    force(8, 2)
+    d = [to_dev(torch, x, cuda) for x in (full, rp, ci, B)]
+    plan = smat.Plan(rp, M, K, len(ci), N, col_idx_host=ci)
+    C = torch.empty((M, N), dtype=torch.float16, device=cuda)
+    columns = np.where(np.arange(256) % 16 < 9, np.float16(2), np.float16(0))  # 288 nonzeros in a pair
+    for vals in (sparse_values(len(ci), 6, 1), full, sparse_values(len(ci), 9, 2), np.tile(columns, len(ci)).view(np.uint16), sparse_values(len(ci), 3, 3)):
+        d[0].copy_(to_dev(torch, vals, cuda))
+        plan.attach_values(d[0], d[1], d[2])
+        smat.spmm(d[0], d[1], d[2], d[3][:K * N], C, M, N, K, len(ci), plan=plan)
+        assert np.array_equal(C.cpu().numpy(), oracle.spmm_bcsr(M, N, K, rp, ci, vals, B[:K * N], threads=4).astype(np.float16))
+    with pytest.raises(smat.SmatError):
+        smat.spmm(d[0], d[1], d[2], d[3], torch.empty((M, N + 8), dtype=torch.float16, device=cuda), M, N + 8, K, len(ci), plan=plan)
+    plan.close()
