@@ -628,7 +628,7 @@ int best_tiles(const WindowPlan &p, const WindowProduct &w, double *us)
 // 16 columns), the bytes that a compute unit's memory path moves (copies of windows, A once a unit, C: 8.7 TB/s on all), those
 // that come from memory (5 TB/s), whichever is longest, and the start (1.6 us, and up to 2.2 for groups of 16).  Fitted to 311 products of 41 bands, stencils
 // and pruned matrices, N = 8 to 1,000, three on their own inputs in turn: 10 % standard deviation, and the group and panel it picks are
-// 4 % from the best in the mean.  Estimate (measured), us: stencil 73 x 61 x 62, N = 88, groups of 8 80 (85); band of 52960 and 64, N = 472,
+// 4 % from the best in the mean; never below 5.5 us (4.6 to 5.5 measured), for the row-wise kernel is as fast there.  Estimate (measured), us: stencil 73 x 61 x 62, N = 88, groups of 8 80 (85); band of 52960 and 64, N = 472,
 // groups of 16 34 (34.5); band of 2144 and 47, N = 808, groups of 4 5.5 (5.6).
 // ENTRIES: the building of the operands besides, for every unit; fitted to 130 products of 27 stencils, N = 8 to 256: 9 %.  71 x 55 x 67,
 // N = 40 36 (35.5); 41 x 35 x 30, N = 208 22 (22.4); 72 x 51 x 40, N = 144 51 (62).
@@ -650,7 +650,7 @@ double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, 
         steps = l.rounds * l.panels_per_unit * parts * (1.07 + 0.0155 * blocks);
         path = copies / 8.7e6, memory = once / 5.0e6, start = 1.6 + 2.2 * groups16;
     }
-    return std::max(4.7, start + std::pow(std::pow(steps, 4.0) + std::pow(path, 4.0) + std::pow(memory, 4.0), 0.25));
+    return std::max(entries ? 4.7 : 5.5, start + std::pow(std::pow(steps, 4.0) + std::pow(path, 4.0) + std::pow(memory, 4.0), 0.25));
 }
 
 hipError_t window_widths(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, WindowWidths &out, void **slots)
@@ -705,7 +705,7 @@ double window_choose(const WindowWidths &widths, const WindowProduct &w, int *si
             // Nothing shared: the pieces that the copies bring are single blocks, 32 bytes of a column, and from a B beyond an XCD's 4 MiB of L2 each
             // costs a cache line (928 x 4160, 3 %, N = 3472: estimate 12, 27 us, row-wise 15; 1376 x 5344, 4 %, N = 896 9.8, 13.6 and 11.4;
             // 12656 x 832, 6 %, N = 352 11.4 -> 8.4 all the same).
-            if ((double)widths.sum[i] > 0.8 * (double)w.nnzb) {
+            if ((double)widths.sum[i] > 0.75 * (double)w.nnzb) {
                 if (2 * w.K * w.N > (size_t)4 << 20) continue;
                 e *= 1.25;
             }
