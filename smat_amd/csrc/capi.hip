@@ -80,6 +80,7 @@ struct smat_plan {
     int n_items_dense = 0, n_split_dense = 0;
     int64_t n_blocks_dense = 0;
     WindowPlan *window = nullptr; // the row-wise kernel's place is taken by the one that multiplies from windows of B
+    ResidentPlan *resident = nullptr; // or these, of the values as they were attached
     uint16_t *d_bcol = nullptr; // column-major copy of a row-major B, K * n_cap halves (plans made for SMAT_B_ROW_MAJOR)
 };
 
@@ -132,6 +133,7 @@ extern "C" void smat_internal_fail_alloc(int64_t n) { g_dev_fail_in.store(n); }
 extern "C" int smat_internal_compact_split_rows(const smat_plan *p) { return p->compact ? p->compact->n_split_rows : -1; }
 
 // Test hook (not part of smat.h): block rows of a group whose window the plan's products multiply from, 0 without windows.
+extern "C" int smat_internal_plan_resident(const smat_plan *p) { return p->resident != nullptr; }
 extern "C" int smat_internal_plan_window_rows(const smat_plan *p) { return p->window ? p->window->rows : 0; }
 
 // Test hook (not part of smat.h): rows of B that the compact kernel's copy holds, 0 where it holds all or there is no list.
@@ -205,11 +207,16 @@ static double rowwise_estimate_us(size_t M, size_t K, size_t N, size_t nnzb, siz
 // with N = 2040, rows that straddle cache lines, 50 against 43).
 static double to_col_major_us(size_t K, size_t N) { return 2.0 + 0.6e-6 * (double)K * (double)N; }
 static double sweep_in_place_factor(size_t N) { return N % 64 == 0 ? 1.05 : 1.13; }
-// The compact kernel and the pass over a column-major B before it: gathers of whole panels of 16, 32 or 64 columns.  27 stencils, N = 8 to
-// 256: 11 % standard deviation.
-static double compact_estimate_us(int64_t cols, size_t K, size_t N)
+// The compact kernel and the pass over a column-major B before it: gathers of whole panels of 16, 32 or 64 columns, B, and the bytes of
+// all (B three times) beyond what is found in the caches.  80 stencils and uniform random matrices, N = 8 to 816: 9.5 % standard deviation.
+static double compact_estimate_us(double cols, double list_bytes, size_t M, size_t K, size_t N)
 {
-    return 6.0 + (double)cols * (double)(N <= 16 ? 16 : N <= 32 ? 32 : (N + 63) / 64 * 64) * 2.0 / 10e6 + (double)K * (double)N / 1e6;
+    const double b = 2.0 * (double)K * (double)N, gathered = cols * (double)(N <= 16 ? 16 : N <= 32 ? 32 : (N + 63) / 64 * 64) * 2.0;
+    return 7.8 + gathered / 16.1e6 + b / 4.5e6 + std::max(0.0, 3.0 * b + 2.0 * (double)M * (double)N + list_bytes - 28e6) / 8.25e6;
+}
+static double compact_estimate_us(const CompactPlan &c, size_t M, size_t K, size_t N)
+{
+    return compact_estimate_us((double)c.n_cols, c.d_acol ? 36.0 * (double)c.n_cols : 4.25 * (double)c.n_cols + 4.0 * (double)c.n_entries, M, K, N);
 }
 static size_t sweep_listed_chunks(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t group_rows)
 {
@@ -364,8 +371,11 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
             e = launch_compact(c, static_cast<hipStream_t>(o.stream));
         }
     } else if (kernel == SMAT_KERNEL_COMPACT && o.kernel == SMAT_KERNEL_AUTO && plan->window && o.b_layout == SMAT_B_COL_MAJOR && N <= plan->n_cap &&
-               (N == plan->n_cap || window_forced() || window_launch_us(a, *plan->window) < 0.9 * compact_estimate_us(plan->compact->n_cols, K, N))) {
+               (N == plan->n_cap || window_forced() || window_launch_us(a, *plan->window) < 0.9 * compact_estimate_us(*plan->compact, M, K, N))) {
         e = launch_window(a, *plan->window, static_cast<hipStream_t>(o.stream));
+    } else if (kernel == SMAT_KERNEL_COMPACT && o.kernel == SMAT_KERNEL_AUTO && plan->resident && o.b_layout == SMAT_B_COL_MAJOR && N <= plan->n_cap &&
+               (N == plan->n_cap || resident_forced() || resident_launch_us(*plan->resident, K, N) < 0.9 * compact_estimate_us(*plan->compact, M, K, N))) {
+        e = launch_resident(a, *plan->resident, static_cast<hipStream_t>(o.stream));
     } else if (kernel == SMAT_KERNEL_COMPACT) {
         if (!plan || !plan->compact || !plan->d_bt || N > plan->n_cap)
             return set_error(SMAT_ERR_INVALID,
@@ -763,7 +773,15 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     }
     return e;
 }
-hipError_t smat::plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx) { return take_window(*p, row_ptr, col_idx, 1e30, nullptr, nullptr); }
+// No memory for the windows is not an error of the plan.
+static hipError_t take_window_if_room(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us, const uint16_t *vals, const CompactCensus *census)
+{
+    const hipError_t e = take_window(p, row_ptr, col_idx, other_us, vals, census);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    return hipSuccess;
+}
+hipError_t smat::plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx) { return take_window_if_room(*p, row_ptr, col_idx, 1e30, nullptr, nullptr); }
 
 static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, const int32_t *row_ptr,
                                         const int32_t *col_idx, const int32_t *row_ptr_host)
@@ -793,6 +811,8 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
         p->n_blocks_dense = 0;
         window_destroy(p->window);
         p->window = nullptr;
+        resident_destroy(p->resident);
+        p->resident = nullptr;
     };
     auto fail = [&](hipError_t err) {
         if (p->compact) { compact_destroy(p->compact); p->compact = nullptr; }
@@ -905,7 +925,8 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
                                           p->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, p->d_bpack != nullptr, p->d_bcol != nullptr);
         if (group_rows) e = sweep_small_groups(*p, group_rows);
         else if (!take || !p->d_bcol)
-            e = take_window(*p, row_ptr, col_idx, compact_estimate_us(census.n_cols_all, p->K, p->n_cap), vals, take ? &census : nullptr);
+            e = take_window_if_room(*p, row_ptr, col_idx, compact_estimate_us((double)census.n_cols_all, std::min(36.0 * (double)census.n_cols_all, 4.25 * (double)census.n_cols_all + 4.0 * (double)census.nnz), p->M, p->K,
+                                                p->n_cap), vals, take ? &census : nullptr);
         if (e != hipSuccess) return fail(e);
     }
     if (!take) return SMAT_OK; // nothing would use the list: the plan keeps (or goes back to) a dense kernel
@@ -978,7 +999,20 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     p->kernel = mixed || block_split ? SMAT_KERNEL_MIXED : SMAT_KERNEL_COMPACT;
     // the deal of the compact kernel's work items to the XCDs, measured on this list at the plan's width (B in the
     // layout the plan was made for: d_bcol is the scratch of a plan for row-major B)
-    if (!p->window) e = compact_tune(*c, p->d_bt, p->M, p->n_cap, p->K, p->d_bcol != nullptr, block_split); // else its launches are not what the plan is for
+    // Columns of B in LDS against the compact kernel; no memory for their lists is not an error of the plan.
+    if (want == SMAT_KERNEL_AUTO && !mixed && !block_split && !p->window && !p->d_bcol) {
+        const double bar = 0.9 * compact_estimate_us(*c, p->M, p->K, p->n_cap);
+        if (resident_forced() || resident_estimate_us(p->M, p->K, p->n_cap, census.nnz) < bar) {
+            e = resident_build(*c, p->M, p->K, census.nnz, &p->resident);
+            if (e == hipErrorOutOfMemory) e = hipSuccess, (void)hipGetLastError();
+            if (e != hipSuccess) return fail(e);
+        }
+        if (p->resident && !resident_forced() && resident_launch_us(*p->resident, p->K, p->n_cap) >= bar) {
+            resident_destroy(p->resident);
+            p->resident = nullptr;
+        }
+    }
+    if (!p->window && !p->resident) e = compact_tune(*c, p->d_bt, p->M, p->n_cap, p->K, p->d_bcol != nullptr, block_split); // else its launches are not what the plan is for
     if (e != hipSuccess) return set_error(SMAT_ERR_HIP, "timing the compact kernel failed: %s", hipGetErrorString(e));
     if (p->d_bpack && want == SMAT_KERNEL_AUTO && !mixed) { // the row-wise kernel's scratch is not needed any more
         (void)dev_free(p->d_bpack);
@@ -999,6 +1033,7 @@ extern "C" int smat_plan_destroy(smat_plan *p)
     if (p->compact) compact_destroy(p->compact);
     if (p->d_bt) (void)dev_free(p->d_bt);
     window_destroy(p->window);
+    resident_destroy(p->resident);
     if (p->d_bcol) (void)dev_free(p->d_bcol);
     if (p->d_items_dense) (void)dev_free(p->d_items_dense);
     if (p->d_split_dense) (void)dev_free(p->d_split_dense);

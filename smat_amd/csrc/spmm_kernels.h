@@ -212,6 +212,22 @@ hipError_t window_attach_entries(WindowPlan &p, const uint16_t *vals, const int3
 double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, const WindowProduct &w);
 double window_launch_us(const SpmmArgs &a, const WindowPlan &p); // 1e30: not at this N
 hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st); // column-major B
+
+// ---- columns of B in LDS (spmm_resident.hip) ----
+struct ResidentPlan {
+    int n_slices = 0, longest = 0; // of 64 rows each; nonzeros of the longest row
+    int64_t fours = 0;             // fours of nonzeros a lane, of all slices
+    uint32_t *d_list = nullptr;    // of every lane its row, then value << 16 | row of B; 256 * d_first[s] before slice s
+    uint32_t *d_first = nullptr;
+};
+// From the lists of the compact kernel, which must be all of the matrix; synchronous, on the default stream.  *out: NULL where they do not fit.
+hipError_t resident_build(const CompactPlan &c, size_t M, size_t K, int64_t nnz, ResidentPlan **out);
+void resident_destroy(ResidentPlan *p);
+bool resident_forced(); // by the test hook
+double resident_estimate_us(size_t M, size_t K, size_t N, int64_t nnz); // for rows of about the same length; 1e30: K too long
+double resident_launch_us(const ResidentPlan &p, size_t K, size_t N);
+hipError_t launch_resident(const SpmmArgs &a, const ResidentPlan &p, hipStream_t st); // column-major B
+
 hipError_t launch_sweep(const SweepArgs &a, hipStream_t st);
 // Whether the sweep kernel reads a row-major B of this size in place; otherwise B is brought into column-major order first, one
 // read and one write of it.  In place a row group reads 128 bytes of every row of B where it reads 512 of every column of the
