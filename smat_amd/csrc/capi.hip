@@ -461,20 +461,37 @@ static uint64_t mix_word(uint64_t h, uint64_t v)
     h = (h ^ v) * 0x9e3779b97f4a7c15ull;
     return h ^ (h >> 29);
 }
+struct Hash { // of bytes that come in pieces, all but the last of whole 32 bytes
+    uint64_t lane[4], bytes = 0;
+    explicit Hash(uint64_t h) : lane{h, h ^ 0xbf58476d1ce4e5b9ull, h ^ 0x94d049bb133111ebull, h ^ 0xd6e8feb86659fd93ull} {}
+    void add(const void *data, size_t n)
+    {
+        const unsigned char *p = static_cast<const unsigned char *>(data);
+        bytes += n;
+        size_t i = 0;
+        for (; i + 32 <= n; i += 32) {
+            uint64_t v[4];
+            memcpy(v, p + i, 32);
+            for (int l = 0; l < 4; l++) lane[l] = mix_word(lane[l], v[l]);
+        }
+        rest_bytes = n - i;
+        memcpy(rest, p + i, rest_bytes);
+    }
+    uint64_t end()
+    {
+        uint64_t v[4] = {0, 0, 0, 0};
+        memcpy(v, rest, rest_bytes);
+        for (int l = 0; l < 4; l++) lane[l] = mix_word(lane[l], v[l]);
+        return mix_word(mix_word(mix_word(mix_word(bytes, lane[0]), lane[1]), lane[2]), lane[3]);
+    }
+    unsigned char rest[32];
+    size_t rest_bytes = 0;
+};
 static uint64_t hash_bytes(uint64_t h, const void *data, size_t bytes)
 {
-    const unsigned char *p = static_cast<const unsigned char *>(data);
-    uint64_t lane[4] = {h, h ^ 0xbf58476d1ce4e5b9ull, h ^ 0x94d049bb133111ebull, h ^ 0xd6e8feb86659fd93ull};
-    size_t i = 0;
-    for (; i + 32 <= bytes; i += 32) {
-        uint64_t v[4];
-        memcpy(v, p + i, 32);
-        for (int l = 0; l < 4; l++) lane[l] = mix_word(lane[l], v[l]);
-    }
-    uint64_t rest[4] = {0, 0, 0, 0};
-    memcpy(rest, p + i, bytes - i);
-    for (int l = 0; l < 4; l++) lane[l] = mix_word(lane[l], rest[l]);
-    return mix_word(mix_word(mix_word(mix_word(bytes, lane[0]), lane[1]), lane[2]), lane[3]);
+    Hash s(h);
+    s.add(data, bytes);
+    return s.end();
 }
 static uint64_t pattern_fingerprint(const int32_t *row_ptr_host, const int32_t *col_idx_host, size_t mb, size_t nnzb)
 {
@@ -547,20 +564,32 @@ static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
     // it needs the columns of a block row strictly ascending, as csrToBcsr emits them (matrix.h:441-463).  The
     // row-wise kernel does not care about the order (like mmaCBT.cu:44-66).
     bool cols_ascending = true;
+    uint64_t fingerprint = pattern_fingerprint(row_ptr_host, nullptr, mb, nnzb);
     if (col_idx_host) {
-        // without a branch per block, so that the compiler can take several at a time; what is wrong is looked up after
-        uint32_t largest = 0, low_bits = 0; // a negative index is a huge one
-        for (size_t p = 0; p < nnzb; p++) {
-            largest = std::max(largest, (uint32_t)col_idx_host[p]);
-            low_bits |= (uint32_t)col_idx_host[p] & 15u;
+        // One pass over the columns, 16 KiB at a time while they are in the first level cache, without a branch per block; what is wrong is looked
+        // up after.  Bits of either word that matter: a column is negative, above limit or no multiple of 16.
+        const int32_t limit = (int32_t)std::min<size_t>(K - 1, 0x7fffffff);
+        int32_t low_bits = 0, signs = 0;
+        size_t descents = 0, allowed = 0; // where a column does not exceed the one before: only between block rows
+        Hash columns(fingerprint);
+        for (size_t from = 0; from < nnzb; from += 4096) {
+            const size_t n = std::min<size_t>(4096, nnzb - from);
+            const int32_t *const c = col_idx_host + from;
+            uint32_t here = from > 0 && c[0] <= c[-1];
+            for (size_t i = 0; i < n; i++) {
+                low_bits |= c[i];
+                signs |= c[i] | (int32_t)((uint32_t)limit - (uint32_t)c[i]);
+            }
+            for (size_t i = 1; i < n; i++) here += c[i] <= c[i - 1];
+            descents += here;
+            columns.add(c, n * sizeof(int32_t));
         }
-        if (nnzb && (low_bits || (size_t)largest >= K || largest > 0x7fffffffu))
+        fingerprint = columns.end();
+        if (nnzb && ((low_bits & 15) || signs < 0 || K == 0))
             for (size_t p = 0; p < nnzb; p++)
                 if (col_idx_host[p] < 0 || col_idx_host[p] % 16 || (size_t)col_idx_host[p] >= K)
                     return set_error(SMAT_ERR_INVALID, "col_idx_host[%zu] = %d is not a block column of K = %zu",
                                      p, col_idx_host[p], K);
-        size_t descents = 0, allowed = 0; // where a column does not exceed the one before: only between block rows
-        for (size_t p = 1; p < nnzb; p++) descents += col_idx_host[p] <= col_idx_host[p - 1];
         for (size_t i = 1; i < mb; i++) {
             const int32_t p = row_ptr_host[i];
             if (p > 0 && (size_t)p < nnzb && p != row_ptr_host[i - 1]) allowed += col_idx_host[p] <= col_idx_host[p - 1];
@@ -576,7 +605,7 @@ static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
     PlanHolder holder{p};
     p->M = M; p->K = K; p->nnzb = nnzb; p->n_cap = n_hint;
     p->kernel_requested = want;
-    p->fingerprint = pattern_fingerprint(row_ptr_host, col_idx_host, mb, nnzb);
+    p->fingerprint = fingerprint;
     p->fingerprint_has_cols = col_idx_host != nullptr;
     p->row_ptr_host.assign(row_ptr_host, row_ptr_host + mb + 1);
     if (col_idx_host && cols_ascending && (want == SMAT_KERNEL_AUTO || want == SMAT_KERNEL_MIXED)) p->col_idx_host.assign(col_idx_host, col_idx_host + nnzb);
@@ -995,6 +1024,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
         compact_destroy(c);
         return fail(e);
     }
+    census.waited();
     p->compact = c;
     p->kernel = mixed || block_split ? SMAT_KERNEL_MIXED : SMAT_KERNEL_COMPACT;
     // the deal of the compact kernel's work items to the XCDs, measured on this list at the plan's width (B in the

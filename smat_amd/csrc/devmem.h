@@ -29,18 +29,24 @@ hipError_t dev_free_idle(void *p);
 // Gives the kept blocks, of the current device or of all, back to the driver.
 void dev_trim(bool all_devices);
 
-// Scratch memory of one call; the call has waited for its kernels when it goes out of scope.
+// Scratch memory of one call.  Its release waits for the device (some 18 us behind a copy to the host) unless the call says that it has
+// waited since the last use.
 struct DevScratch {
     void *p = nullptr;
+    bool idle = false;
     DevScratch() = default;
     DevScratch(const DevScratch &) = delete;
     DevScratch &operator=(const DevScratch &) = delete;
     ~DevScratch() { release(); }
     void release()
     {
-        if (p) (void)dev_free(p);
+        if (p) (void)(idle ? dev_free_idle(p) : dev_free(p));
         p = nullptr;
     }
-    hipError_t alloc(size_t bytes) { return dev_malloc(&p, bytes ? bytes : 16); }
+    hipError_t alloc(size_t bytes)
+    {
+        idle = false;
+        return dev_malloc(&p, bytes ? bytes : 16);
+    }
 };
 } // namespace smat

@@ -34,6 +34,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cstring>
 #include <type_traits>
 #include <vector>
 
@@ -144,10 +145,10 @@ __device__ __forceinline__ uint32_t row_sum(uint32_t v)
 // Per block: mask of its nonzero columns; their number in the lower half of count, the number of nonzeros in the upper.
 // Bound by the read of the values.  A lane holds one row of one half of a block, a DPP row of 16 lanes that half: its eight bits
 // are or-ed and counted in the VALU, where exchanging the values through LDS was most of the time (237 k blocks, 121 MB:
-// 40 -> 24 us).
+// 40 -> 24 us).  The only nonzero of a block is put beside the mask, 4 bytes that spare the lists a second look at the 512 of the block.
 __global__ __launch_bounds__(256) void colmask_kernel(const uint16_t *__restrict__ vals, long nnzb,
-                                                      uint16_t *__restrict__ mask, unsigned long long *__restrict__ count,
-                                                      unsigned long long *__restrict__ sums)
+                                                      uint16_t *__restrict__ mask, uint32_t *__restrict__ single,
+                                                      unsigned long long *__restrict__ count, unsigned long long *__restrict__ sums)
 {
     unsigned long long total[N_SUMS] = {0, 0, 0, 0};
     const int lane = threadIdx.x & 63;
@@ -173,14 +174,19 @@ __global__ __launch_bounds__(256) void colmask_kernel(const uint16_t *__restrict
             if (w[q] & 0x7fffu) bits |= 1u << (2 * q);
             if (w[q] & 0x7fff0000u) bits |= 2u << (2 * q);
         }
-        const uint32_t nz_half = row_sum(__popc(bits));
+        const uint32_t mine = bits, nz_half = row_sum(__popc(bits));
         bits = row_or(bits);
         // lanes 0 and 32 put the halves of their blocks together
-        const uint32_t other = __shfl(bits, (lane & 32) | 16), nz = nz_half + __shfl(nz_half, (lane & 32) | 16);
+        const uint32_t other = __shfl(bits, (lane & 32) | 16), nz = nz_half + __shfl_xor(nz_half, 16);
+        if (nz == 1 && mine && blk < nnzb) {
+            const uint32_t i = (uint32_t)__ffs((int)mine) - 1, pair = i & 4 ? (i & 2 ? w[3] : w[2]) : (i & 2 ? w[1] : w[0]);
+            single[blk] = (i & 1 ? pair & 0xffff0000u : pair << 16) | (uint32_t)(lane & 15);
+        }
         if ((lane & 31) == 0 && blk < nnzb) {
             const uint32_t m = bits | (other << 8);
             const int cols = __popc(m);
             mask[blk] = (uint16_t)m;
+            if (nz != 1) single[blk] = 0;
             count[blk] = (unsigned long long)nz << 32 | (unsigned)cols;
             total[SUM_NNZ] += nz;
             if (cols >= FULL_BLOCK_COLS) total[SUM_FULL]++;
@@ -225,11 +231,11 @@ __device__ __forceinline__ long row_of_block(const int32_t *__restrict__ row_ptr
 //         each with its place in the operand of its step, and the range of entries of every step to step_range;
 //   used != NULL: used[row] = 1 for the rows of B that the list names.
 // A wavefront takes GATHER_BLOCKS consecutive blocks, four at a time: lane (g = lane / 16, r = lane % 16) holds row r of one.
-// Bound by the second read of the values.  (One thread per block read them 2 bytes at a time, 64 cache lines a load, behind a
+// Bound by the second read of the values, where blocks hold more than one nonzero, and by what it writes.  (One thread per block read them 2 bytes at a time, 64 cache lines a load, behind a
 // search of ten loads one after the other: 237 k blocks 54 -> 35 us;
 // 4, 8, 32 blocks a wavefront 36, 35, 39.)
 constexpr int GATHER_BLOCKS = 16;
-__global__ __launch_bounds__(256) void gather_kernel(const uint16_t *__restrict__ vals, const uint16_t *__restrict__ mask,
+__global__ __launch_bounds__(256) void gather_kernel(const uint16_t *__restrict__ vals, const uint16_t *__restrict__ mask, const uint32_t *__restrict__ single,
                               const unsigned long long *__restrict__ offset, const int32_t *__restrict__ row_ptr,
                               const int32_t *__restrict__ col_idx, const unsigned long long *__restrict__ raw,
                               const int2 *__restrict__ start, long mb, long nnzb, bool drop_full, int32_t *__restrict__ cols,
@@ -256,7 +262,9 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint16_t *__restrict_
         uint32_t m = live ? mask[p] : 0;
         const int2 first = start[br]; // of the columns and of the entries
         if ((drop_full && __popc(m) >= FULL_BLOCK_COLS) || first.x < 0) m = 0; // another kernel multiplies the block or the row
-        const u32x4 w[2] = {reinterpret_cast<const u32x4 *>(vals + p * 256 + r * 16)[0], reinterpret_cast<const u32x4 *>(vals + p * 256 + r * 16)[1]};
+        const uint32_t only = single[p], mine = r == (int)(only & 15) ? only >> 16 : 0;
+        u32x4 w[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
+        if (m && !only) w[0] = reinterpret_cast<const u32x4 *>(vals + p * 256 + r * 16)[0], w[1] = reinterpret_cast<const u32x4 *>(vals + p * 256 + r * 16)[1];
         const unsigned long long before = offset[p] - raw[br]; // no borrow: both halves of offset[p] are at least those of raw
         const long row_end = (long)first.x + (long)(uint32_t)(raw[br + 1] - raw[br]);
         long o = (long)first.x + (long)(uint32_t)before;
@@ -266,7 +274,7 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint16_t *__restrict_
         for (int k = 0; k < 16; k++) {
             const bool has = (m >> k) & 1;
             if (!__any(has)) continue;
-            const uint32_t v = k & 1 ? w[k / 8][k % 8 / 2] >> 16 : w[k / 8][k % 8 / 2] & 0xffffu;
+            const uint32_t v = only ? mine : k & 1 ? w[k / 8][k % 8 / 2] >> 16 : w[k / 8][k % 8 / 2] & 0xffffu;
             const uint32_t nonzero = (uint32_t)(__ballot(has && (v & 0x7fffu)) >> (16 * g)) & 0xffffu; // rows of the lane's block
             if (!has) continue;
             // inside its group of 8 the even entries come first, then the odd ones: the lanes of the product kernel that
@@ -982,7 +990,6 @@ void compact_destroy(CompactPlan *p)
     if (p->d_entries) (void)dev_free(p->d_entries);
     if (p->d_step_range) (void)dev_free(p->d_step_range);
     if (p->d_items) (void)dev_free(p->d_items);
-    if (p->d_tasks) (void)dev_free(p->d_tasks);
     if (p->d_split) (void)dev_free(p->d_split);
     if (p->d_workspace) (void)dev_free(p->d_workspace);
     delete p;
@@ -1022,6 +1029,7 @@ static hipError_t census_offsets(CompactCensus &s, const int32_t *row_ptr)
         e = hipGetLastError();
     }
     SMAT_STEP(hipMemcpy(s.raw.data(), s.rows.p, (s.mb + 1) * 8, hipMemcpyDeviceToHost));
+    tmp.idle = e == hipSuccess;
     return e;
 }
 
@@ -1033,9 +1041,10 @@ hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t m
     s.raw.assign(mb + 1, 0);
     if (!nnzb) return e;
     Scratch sums;
-    for (Scratch *q : {&s.mask, &s.count, &s.offset, &s.rows}) q->release();
+    for (Scratch *q : {&s.mask, &s.single, &s.count, &s.offset, &s.rows}) q->release();
     s.dropped = false;
     SMAT_STEP(s.mask.alloc(nnzb * 2));
+    SMAT_STEP(s.single.alloc(nnzb * 4));
     SMAT_STEP(s.count.alloc(nnzb * 8));
     SMAT_STEP(s.offset.alloc(nnzb * 8));
     SMAT_STEP(s.rows.alloc((mb + 1) * 8));
@@ -1044,12 +1053,13 @@ hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t m
     if (e == hipSuccess) {
         const long waves = std::min<long>((long)(nnzb + 1) / 2, 256L * 32);
         hipLaunchKernelGGL(colmask_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, 0, vals, (long)nnzb,
-                           (uint16_t *)s.mask.p, (unsigned long long *)s.count.p, (unsigned long long *)sums.p);
+                           (uint16_t *)s.mask.p, (uint32_t *)s.single.p, (unsigned long long *)s.count.p, (unsigned long long *)sums.p);
         e = hipGetLastError();
     }
     SMAT_STEP(census_offsets(s, row_ptr));
     unsigned long long total[N_SUMS] = {0};
     SMAT_STEP(fetch_totals(sums.p, total, N_SUMS));
+    sums.idle = e == hipSuccess;
     s.values_checksum = total[SUM_CHECK];
     s.full_blocks = (int64_t)total[SUM_FULL];
     s.cols_rest = (int64_t)total[SUM_COLS_REST];
@@ -1220,7 +1230,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     if (e == hipSuccess && nnzb) {
         SMAT_STEP(hipMemcpy(starts.p, start.data(), (mb + 1) * sizeof(int2), hipMemcpyHostToDevice));
         if (e == hipSuccess) {
-            hipLaunchKernelGGL(gather_kernel, dim3((unsigned)((nnzb + 4 * GATHER_BLOCKS - 1) / (4 * GATHER_BLOCKS))), dim3(256), 0, 0, vals, (const uint16_t *)s.mask.p,
+            hipLaunchKernelGGL(gather_kernel, dim3((unsigned)((nnzb + 4 * GATHER_BLOCKS - 1) / (4 * GATHER_BLOCKS))), dim3(256), 0, 0, vals, (const uint16_t *)s.mask.p, (const uint32_t *)s.single.p,
                                (const unsigned long long *)s.offset.p, row_ptr, col_idx, (const unsigned long long *)s.rows.p, (const int2 *)starts.p,
                                (long)mb, (long)nnzb, drop_full, p->d_cols, p->d_acol, p->d_entries, p->d_step_range, (uint8_t *)used.p);
             e = hipGetLastError();
@@ -1278,6 +1288,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
                 if (range) (void)dev_free(range);
             }
         }
+        for (Scratch *q : {&steps, &first, &tmp, &starts_dev, &row_first}) q->idle = e == hipSuccess; // a copy to the host came last
     }
     auto place_if_it_pays = [&] {
         if (e == hipSuccess && (size_t)n_used <= K / 8 * 7 && (K - (size_t)n_used) * n_cap * sizeof(uint16_t) >= PLACE_MIN_BYTES)
@@ -1341,11 +1352,14 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     p->n_items = (int)items.size();
     p->n_tasks = (int)tasks.size();
     p->n_steps = total / 32;
-    SMAT_STEP(dev_malloc(&p->d_tasks, std::max<size_t>(tasks.size(), 1) * sizeof(int4)));
-    if (!tasks.empty()) SMAT_STEP(hipMemcpy(p->d_tasks, tasks.data(), tasks.size() * sizeof(int4), hipMemcpyHostToDevice));
     p->n_split_rows = (int)split.size();
     p->n_slots = slot;
-    SMAT_STEP(dev_malloc(&p->d_items, std::max<size_t>(items.size(), 1) * sizeof(WorkItem)));
+    static_assert(sizeof(WorkItem) == sizeof(int4), "the tasks lie behind the items");
+    SMAT_STEP(dev_malloc(&p->d_items, (items.size() + tasks.size() + 1) * sizeof(WorkItem)));
+    p->d_tasks = reinterpret_cast<int4 *>(p->d_items + items.size());
+    const size_t n_items = items.size();
+    items.resize(n_items + tasks.size());
+    if (!tasks.empty()) memcpy(static_cast<void *>(items.data() + n_items), tasks.data(), tasks.size() * sizeof(int4));
     if (!items.empty()) SMAT_STEP(hipMemcpy(p->d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
     if (!split.empty()) {
         SMAT_STEP(dev_malloc(&p->d_split, split.size() * sizeof(SplitRow)));
@@ -1358,6 +1372,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     }
     SMAT_STEP(hipDeviceSynchronize());
 #undef SMAT_STEP
+    starts.idle = used.idle = e == hipSuccess;
     if (e != hipSuccess) {
         compact_destroy(p);
         return e;

@@ -104,7 +104,7 @@ struct CompactPlan {
     int2 *d_step_range = nullptr;   // entries [x, y) of every step of 32 listed columns
     int entries_ahead = 0;          // loads of 64 entries that the product kernel asks for ahead: 1 or 2
     WorkItem *d_items = nullptr; // begin/end index the padded list
-    int4 *d_tasks = nullptr;     // runs of items: first item, items, first and last column of the list
+    int4 *d_tasks = nullptr;     // runs of items: first item, items, first and last column of the list (behind d_items, in their memory)
     SplitRow *d_split = nullptr;
     float *d_workspace = nullptr; // n_slots * 16 * n_cap floats
     int n_items = 0, n_tasks = 0, n_split_rows = 0, n_slots = 0;
@@ -124,6 +124,7 @@ struct CompactPlan {
 struct CompactCensus {
     size_t mb = 0, nnzb = 0;
     DevScratch mask;          // uint16 per block: its nonzero columns
+    DevScratch single;        // uint32 per block: value << 16 | row of its only nonzero, 0 where it has none or more
     DevScratch count, offset; // uint64 per block: nonzero columns | nonzeros << 32, and their exclusive sums
     DevScratch rows;          // the same sums at the block rows (mb + 1)
     std::vector<uint64_t> raw; // rows on the host
@@ -131,6 +132,7 @@ struct CompactCensus {
     uint64_t values_checksum = 0;
     int64_t n_cols_all = 0, nnz = 0;
     int64_t full_blocks = 0, cols_rest = 0; // blocks with at least 10 of their 16 columns nonzero, nonzero columns of the others
+    void waited() { mask.idle = single.idle = count.idle = offset.idle = rows.idle = true; } // for all that uses them
     int64_t cols_of_row(size_t br) const { return (int64_t)(uint32_t)(raw[br + 1] - raw[br]); }
 };
 // vals / row_ptr / col_idx here and below: device BCSR arrays.  Synchronous.

@@ -426,31 +426,31 @@ hipError_t resident_build(const CompactPlan &c, size_t M, size_t K, int64_t nnz,
     // fours: those of the nonzeros and the rows' numbers, up to one more a slice, and what the longest rows leave the shorter ones of their slice
     const size_t fours = ((size_t)nnz + 255) / 256 + (size_t)n_slices + (MAX_ROW + 3) / 4 + 1;
     DevScratch tmp;
-    uint32_t *lengths = nullptr, *places = nullptr, *rows_of = nullptr, *longest = nullptr;
-    hipError_t e = tmp.alloc((2 * M + MAX_ROW + 2) * sizeof(uint32_t));
+    uint32_t *lengths = nullptr, *places = nullptr, *rows_of = nullptr;
+    hipError_t e = tmp.alloc((2 * M + MAX_ROW + 1) * sizeof(uint32_t));
     if (e == hipSuccess) {
-        rows_of = static_cast<uint32_t *>(tmp.p), longest = rows_of + MAX_ROW + 1, lengths = longest + 1, places = lengths + M;
+        rows_of = static_cast<uint32_t *>(tmp.p), lengths = rows_of + MAX_ROW + 1, places = lengths + M;
         e = dev_malloc(&p->d_list, fours * 1024);
     }
     if (e == hipSuccess) e = dev_malloc(&p->d_first, ((size_t)n_slices + 2) * sizeof(uint32_t));
     if (e == hipSuccess) {
-        e = hipMemsetAsync(rows_of, 0, (MAX_ROW + 2) * sizeof(uint32_t), nullptr);
+        e = hipMemsetAsync(rows_of, 0, (MAX_ROW + 1) * sizeof(uint32_t), nullptr);
     }
     if (e == hipSuccess) e = hipMemsetD32Async((hipDeviceptr_t)p->d_list, (int)K, fours * 256, nullptr);
     const unsigned wgs = (unsigned)((c.n_items + WAVES - 1) / WAVES);
     if (e == hipSuccess) {
         hipLaunchKernelGGL(resident_lengths_kernel, dim3(wgs), dim3(1024), 0, nullptr, c.d_items, c.n_items, c.d_acol, c.d_entries, c.d_step_range, (int32_t *)lengths, rows_of);
-        hipLaunchKernelGGL(resident_slices_kernel, dim3(1), dim3(1024), 0, nullptr, rows_of, n_slices, p->d_first, longest);
+        hipLaunchKernelGGL(resident_slices_kernel, dim3(1), dim3(1024), 0, nullptr, rows_of, n_slices, p->d_first, p->d_first + n_slices + 1);
         hipLaunchKernelGGL(resident_places_kernel, dim3((unsigned)((M + 1023) / 1024)), dim3(1024), 0, nullptr, (const int32_t *)lengths, (int)M, rows_of, places);
         hipLaunchKernelGGL(resident_fill_kernel, dim3(wgs), dim3(1024), 0, nullptr, c.d_items, c.n_items, c.d_acol, c.d_entries, c.d_step_range, c.d_cols, places, p->d_first,
                            (int)M, p->d_list);
         e = hipGetLastError();
     }
     uint32_t n[2] = {0, 0};
-    if (e == hipSuccess) e = hipMemcpy(&n[0], longest, sizeof n[0], hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(&n[1], p->d_first + n_slices, sizeof n[1], hipMemcpyDeviceToHost);
-    p->longest = (int)n[0];
-    p->fours = n[1];
+    if (e == hipSuccess) e = hipMemcpy(n, p->d_first + n_slices, sizeof n, hipMemcpyDeviceToHost);
+    tmp.idle = e == hipSuccess;
+    p->fours = n[0];
+    p->longest = (int)n[1];
     if (e != hipSuccess || p->longest >= MAX_ROW) {
         (void)hipDeviceSynchronize();
         resident_destroy(p);
