@@ -38,7 +38,9 @@ constexpr int SIZES[WINDOW_SIZES] = {4, 8, 16}; // block rows of a group
 // block pairs of a row that a wavefront holds
 constexpr int MAX_PAIRS = 17;
 template <int TN> constexpr int pairs_held = TN == 4 ? 12 : MAX_PAIRS;
-constexpr int LIST_BITS = 26; // of a pair's list: the fours of entries before it; above them its own fours
+// Listed nonzeros become operands a round of so many pairs at a time.
+constexpr int ROUND = 4, MAX_ROUNDS = (MAX_PAIRS + ROUND - 1) / ROUND;
+constexpr int LIST_BITS = 26; // of a round's list: the fours of entries before it; above them its own fours
 
 // ---- which block columns a group uses ----
 
@@ -125,12 +127,12 @@ __global__ __launch_bounds__(256) void window_list_kernel(const int32_t *__restr
     }
 }
 
-// The nonzeros of the blocks, pair by pair of a block row: value << 16 | byte in the pair's MFMA operand, filled up to a multiple of
-// four with the last one.  table: MAX_PAIRS pairs a block row, the places of the two blocks in the window (16 bits each) and the list, the fours of
-// entries before it and its own << LIST_BITS; behind the table the blocks of every row.  A wavefront takes a block row; offset[p]: nonzeros before
-// block p in the upper half.  Bound by the read of the values.
+// The nonzeros of the blocks, ROUND pairs of a block row after the other: value << 16 | byte in the MFMA operands of the round, which lie
+// rows KiB apart, filled up to a multiple of four with the last one.  table: MAX_PAIRS words twice a block row, the places of the two blocks of
+// pair j in the window (16 bits each) and the list of round j, the fours of entries before it and its own << LIST_BITS; behind the table the blocks of
+// every row.  A wavefront takes a block row; offset[p]: nonzeros before block p in the upper half.  Bound by the read of the values.
 __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr,
-                                                             const uint32_t *__restrict__ slot, const unsigned long long *__restrict__ offset, int mb,
+                                                             const uint32_t *__restrict__ slot, const unsigned long long *__restrict__ offset, int mb, int rows,
                                                              uint32_t *__restrict__ entries, uint32_t *__restrict__ table, uint32_t *__restrict__ most)
 {
     const int lane = threadIdx.x & 63, br = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -138,49 +140,47 @@ __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__r
     const int p0 = row_ptr[br], blocks = row_ptr[br + 1] - p0;
     const int sel = lane >> 5, at = (lane & 15) * 16 + ((lane >> 4) & 1) * 8;
     if (lane == 0) table[(long)mb * (2 * MAX_PAIRS) + br] = (uint32_t)blocks;
-    uint32_t longest = 0;
     auto load = [&](int d) {
         const int b = 2 * d + sel;
         return b < blocks ? *reinterpret_cast<const u32x4 *>(vals + (long)(p0 + b) * 256 + at) : (u32x4){0u, 0u, 0u, 0u};
     };
     u32x4 w = load(0);
-    for (int d = 0; d < MAX_PAIRS; d++) {
+    uint32_t longest = 0, first = 0, n = 0, last = 0, places = 0, list = 0; // places, list: of pair and round `lane`
+    for (int d = 0; 2 * d < blocks; d++) {
         const u32x4 now = w;
         w = load(d + 1);
-        uint32_t *const to = table + (long)br * (2 * MAX_PAIRS) + 2 * d;
-        if (2 * d >= blocks) {
-            if (lane < 2) to[lane] = 0;
-            continue;
-        }
-        uint32_t n = 0, before = 0; // nonzeros of the pair, and of the lanes before this one
-        uint32_t bits = 0;
+        if (d % ROUND == 0) first = ((uint32_t)(offset[p0 + 2 * d] >> 32) + 8u * (uint32_t)((p0 + br + 1) / 2 + d)) & ~3u, n = 0;
+        uint32_t i = n, bits = 0; // nonzeros of the round before those of this lane
 #pragma unroll
         for (int k = 0; k < 8; k++) { // -0.0 is a zero
             const bool has = (now[k / 2] >> (k & 1 ? 16 : 0) & 0x7fffu) != 0;
             bits |= (uint32_t)has << k;
             const unsigned long long all = __ballot(has);
             n += __popcll(all);
-            before += __popcll(all & ((1ull << lane) - 1ull));
+            i += __popcll(all & ((1ull << lane) - 1ull));
         }
-        const uint32_t first = ((uint32_t)(offset[p0 + 2 * d] >> 32) + 8u * (uint32_t)((p0 + br + 1) / 2 + d)) & ~3u, end = (n + 3u) & ~3u;
-        uint32_t i = before;
+        uint32_t e = 0;
 #pragma unroll
         for (int k = 0; k < 8; k++)
             if (bits >> k & 1) {
-                const uint32_t e = (now[k / 2] >> (k & 1 ? 16 : 0)) << 16 | (uint32_t)(lane * 16 + k * 2);
-                entries[first + i] = e;
-                if (++i == n)
-                    for (; i < end; i++) entries[first + i] = e;
+                e = (now[k / 2] >> (k & 1 ? 16 : 0)) << 16 | (uint32_t)(d % ROUND * rows * 1024 + lane * 16 + k * 2);
+                entries[first + i++] = e;
             }
-        if (lane == 0) {
-            const int b = p0 + 2 * d;
-            const uint32_t s0 = slot[b] & ((1u << SLOT_BITS) - 1u), s1 = 2 * d + 1 < blocks ? slot[b + 1] & ((1u << SLOT_BITS) - 1u) : s0;
-            to[0] = s0 | s1 << 16;
-            to[1] = first / 4 | min(end / 4, (1u << (32 - LIST_BITS)) - 1u) << LIST_BITS;
+        const unsigned long long some = __ballot(bits != 0);
+        if (some) last = __shfl(e, 63 - __clzll((long long)some));
+        const uint32_t end = (n + 3u) & ~3u;
+        if (d % ROUND == ROUND - 1 || 2 * d + 2 >= blocks) {
+            if (n + lane < end) entries[first + n + lane] = last;
+            if (lane == d / ROUND) list = first / 4 | min(end / 4, (1u << (32 - LIST_BITS)) - 1u) << LIST_BITS;
+            longest = max(longest, end);
         }
-        longest = max(longest, end);
+        const int b = p0 + 2 * d;
+        const uint32_t s0 = slot[b] & ((1u << SLOT_BITS) - 1u), s1 = 2 * d + 1 < blocks ? slot[b + 1] & ((1u << SLOT_BITS) - 1u) : s0;
+        if (lane == d) places = s0 | s1 << 16;
     }
-    if (lane == 0 && longest > 4 * ((1u << (32 - LIST_BITS)) - 1)) atomicMax(most, longest); // too many for a pair
+    uint32_t *const to = table + (long)br * (2 * MAX_PAIRS);
+    if (lane < MAX_PAIRS) to[2 * lane] = places, to[2 * lane + 1] = list;
+    if (lane == 0 && longest > 4 * ((1u << (32 - LIST_BITS)) - 1)) atomicMax(most, longest); // too many for a round
 }
 
 // ---- the product ----
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
     const int i16 = lane & 15, g = lane >> 4, sel = g >> 1, kh = g & 1;
 
     const uint32_t lbase = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)lds;
-    const uint32_t buffer = ENTRIES ? (uint32_t)max(cap * (P * 32), rows * 1024) : (uint32_t)cap * (P * 32);
+    const uint32_t buffer = ENTRIES ? (uint32_t)max(cap * (P * 32), rows * (ROUND * 1024)) : (uint32_t)cap * (P * 32);
     // Piece o of column c of a quad lies at place o ^ swizzle(c) of its 128 bytes: the 16 columns that an operand takes lie in different banks.
     auto swizzle = [](uint32_t c) { return ((c >> 1) & 1u) | ((c / (P / 4)) & 3u) << 1; };
     // the lane, for addresses that are made anew where they are used instead of being kept in registers
@@ -245,14 +245,14 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
     // The block row of a wavefront in a group: what is asked for, and what is made of it.
     struct Asked {
         int p0, blocks;
-        uint32_t q0, q1, c0, c1; // lane j: blocks 2 j and 2 j + 1; ENTRIES: their places in q0, their entries in q1
+        uint32_t q0, q1, c0, c1; // lane j: blocks 2 j and 2 j + 1; ENTRIES: their places in q0, the list of round j in q1
     };
     struct Row {
         int p0, blocks;  // blocks: 0 where the wavefront has none
         uint32_t packed; // lane j: places of blocks 2 j and 2 j + 1 in the window, in 32 bytes
         bool known;
     };
-    uint32_t list = 0; // ENTRIES: of the row taken last, lane j: the entries of blocks 2 j and 2 j + 1
+    uint32_t list = 0; // ENTRIES: of the row taken last, lane j: the list of round j
     auto ask_row = [&](int gr, Asked &r) {
         const int br = gr * rows + wave, b = br < mb ? br : mb - 1;
         if constexpr (ENTRIES) { // a table of MAX_PAIRS pairs a block row, and the blocks of every row behind it
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
 #pragma unroll
     for (int d = 0; d < NP; d++) a[d] = (f16x8){0, 0, 0, 0, 0, 0, 0, 0};
     // Pair d of a row to a[d] where d < n: through a buffer that ends with the row, so that what is past its end is zero.
-    // ENTRIES: the pair's entries, four a lane, until build_a makes the operand of them.
+    // ENTRIES: the entries of round d, four a lane, until build_a makes operands of them.
     const uint32_t a_off = (uint32_t)(sel * 512 + i16 * 32 + kh * 16);
     auto load_a = [&](int d, const Row &r, int n) {
         if constexpr (ENTRIES) {
@@ -320,32 +320,42 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
                      : "v"(a_off), "s"(row), "s"(n), "n"(d), "s"(d * 1024)
                      : "scc");
     };
-    // ENTRIES: the operands of the row from its entries, through 1 KiB of LDS that this wavefront's next copies will overwrite.
+    // ENTRIES: the operands of the row from its entries, a round after the other, the last one first (the entries of the others lie in front of
+    // its operands), through ROUND KiB of LDS that this wavefront's next copies will overwrite.
     auto build_a = [&](const Row &r, uint32_t tile) {
         typedef __attribute__((address_space(3))) uint16_t lds_half;
         typedef __attribute__((address_space(3))) u32x4 lds_quad;
-        const uint32_t mine = tile + (uint32_t)lane * 16u;
-        auto clear = [&] { *(lds_quad *)(uintptr_t)mine = (u32x4){0u, 0u, 0u, 0u}; };
-        clear();
+        const uint32_t mine = tile + (uint32_t)lane_here() * 16u;
 #pragma unroll
-        for (int d = 0; d < NP; d++) {
-            if (2 * d < r.blocks) {
-                const uint32_t fours = (uint32_t)__builtin_amdgcn_readlane((int)list, d) >> LIST_BITS;
-                const u32x4 e = __builtin_bit_cast(u32x4, a[d]);
-                asm volatile("" ::: "memory");
-                if ((uint32_t)lane < fours)
+        for (int k = MAX_ROUNDS - 1; k >= 0; k--) {
+            if (k * ROUND < NP && 2 * k * ROUND < r.blocks) {
+                const uint32_t fours = (uint32_t)__builtin_amdgcn_readlane((int)list, k) >> LIST_BITS;
+                const u32x4 e = __builtin_bit_cast(u32x4, a[k]);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) *(lds_half *)(uintptr_t)(tile + (e[i] & 0x3ffu)) = (uint16_t)(e[i] >> 16);
+                for (int j = 0; j < ROUND; j++)
+                    if (k * ROUND + j < NP) *(lds_quad *)(uintptr_t)(mine + (uint32_t)(j * rows * 1024)) = (u32x4){0u, 0u, 0u, 0u};
                 asm volatile("" ::: "memory");
-                a[d] = __builtin_bit_cast(f16x8, *(lds_quad *)(uintptr_t)mine);
+                if ((uint32_t)lane_here() < fours) {
+                    uint32_t x[4] = {e[0], e[1], e[2], e[3]};
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        uint32_t to;
+                        asm("v_mad_u32_u16 %0, %1, 1, %2" : "=v"(to) : "v"(x[i]), "s"(tile)); // its low half
+                        *(lds_half *)(uintptr_t)to = (uint16_t)(x[i] >> 16);
+                    }
+                }
                 asm volatile("" ::: "memory");
-                clear();
+#pragma unroll
+                for (int j = 0; j < ROUND; j++)
+                    if (k * ROUND + j < NP) a[k * ROUND + j < NP ? k * ROUND + j : 0] = __builtin_bit_cast(f16x8, *(lds_quad *)(uintptr_t)(mine + (uint32_t)(j * rows * 1024)));
+                asm volatile("" ::: "memory");
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
-    // pairs to load: a multiple of U, the last ones zeros
-    auto loads_of = [&](const Row &r) { return min(((r.blocks + 1) / 2 + U - 1) / U * U, NP); };
+    // what is loaded: pairs, a multiple of U, the last ones zeros, or rounds
+    auto loads_of = [&](const Row &r) { return ENTRIES ? (r.blocks + 2 * ROUND - 1) / (2 * ROUND) : min(((r.blocks + 1) / 2 + U - 1) / U * U, NP); };
+    constexpr int LOADS = ENTRIES ? (NP + ROUND - 1) / ROUND : NP;
     auto wait_a = [&](int younger) {
         wait_vector_memory(younger);
 #pragma unroll
@@ -371,7 +381,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
         for (int t = 0; t < COPIES; t++) asm volatile("" : "+v"(from_k[t]));
     };
     // a part's columns of the window to LDS; returns the instructions
-    auto stage = [&](int pan, int part, uint32_t dst, int t0 = 0, int t1 = COPIES) { // the t0-th to t1-th of the wavefront
+    auto stage = [&](int pan, int part, uint32_t dst) {
         const int n0 = pan * PANEL + part * (P / 4);
         const uint64_t base = (uint64_t)(uintptr_t)(B + (long)n0 * K);
         const int lane = lane_here();
@@ -382,7 +392,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
 #pragma unroll
         for (int t = 0; t < COPIES; t++) {
             const int q = copy_quad + t * quads_apart;
-            if (t >= t0 && t < t1 && q < quads) {
+            if (q < quads) {
                 asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(from + 2u * from_k[t]), "s"(base),
                              "s"(dst + (uint32_t)(q * QUAD_BYTES) + (uint32_t)copy_part * 1024u)
                              : "memory");
@@ -452,7 +462,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
             if constexpr (RELOAD)
 #pragma unroll
                 for (int u = 0; u < U; u++)
-                    if (d0 + u < NP) load_a(d0 + u < NP ? d0 + u : 0, next, n_reload);
+                    if (d0 + u < LOADS) load_a(d0 + u < LOADS ? d0 + u : 0, next, n_reload);
         }
     };
     // Everybody has left the part's buffer, and the next part's copies, which all but `younger` operations are older than, have landed.
@@ -470,7 +480,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
     row = next = take_row(asked);
     stage(panel, 0, lbase);
 #pragma unroll
-    for (int d = 0; d < NP; d++) load_a(d, row, loads_of(row));
+    for (int d = 0; d < LOADS; d++) load_a(d, row, loads_of(row));
     const uint32_t tile = lbase + (uint32_t)(copy_quad * QUAD_BYTES + copy_part * 1024); // of build_a, in either half
     if constexpr (ENTRIES) {
         wait_a(0);
@@ -490,20 +500,16 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
         ahead = false;
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    // A part's copies, and on the way the operands of the row, where they are new: ENTRIES makes them in the place of its first copy.
+    // A part's copies, and the operands of the row, where they are new: ENTRIES makes them in the place of its first copies.
+    int stored = 0; // stores that are younger than the loads of the row
     auto stage_and_take_a = [&](int pan, int part, bool copy) {
         const uint32_t to = buf ^ buffer;
-        if constexpr (ENTRIES) {
-            if (loaded) {
-                const int copies = copy ? stage(pan, part, lbase + to, 1) : 0;
-                wait_a(copies);
-                build_a(row, tile + to);
-                if (copy) stage(pan, part, lbase + to, 0, 1);
-                return;
-            }
+        if (ENTRIES && loaded) {
+            wait_a(stored);
+            build_a(row, tile + to);
         }
         const int copies = copy ? stage(pan, part, lbase + to) : 0;
-        if (loaded) wait_a(copies);
+        if (!ENTRIES && loaded) wait_a(copies);
     };
     for (;;) { // a panel
         const bool last = is_last(here_unit, panel), more = !last || soon.unit < my_units;
@@ -549,7 +555,8 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
         if (!more) break;
         // store instructions: at least so many where no column is past N
         constexpr int STORES = C_F32 ? TILES : (TILES + 1) / 2;
-        meet(reload + (br < mb && n0 + PANEL <= N ? STORES : 0));
+        stored = br < mb && n0 + PANEL <= N ? STORES : 0;
+        meet(reload + stored);
         if (last) {
             row = next;
             here_unit = soon;
@@ -562,7 +569,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
 
 int g_force_rows = 0, g_force_tiles = 0; // test hook
 
-size_t lds_of(int rows, int cap, int tiles, bool entries) { return 2 * std::max((size_t)cap * tiles * 512, entries ? (size_t)rows * 1024 : 0); }
+size_t lds_of(int rows, int cap, int tiles, bool entries) { return 2 * std::max((size_t)cap * tiles * 512, entries ? (size_t)rows * (ROUND * 1024) : 0); }
 // Whether windows of `cap` block columns fit: twice in LDS, and COPIES KiB a wavefront.
 bool fits(int rows, int cap, int tiles, bool entries)
 {
@@ -630,8 +637,8 @@ int best_tiles(const WindowPlan &p, const WindowProduct &w, double *us)
 // and pruned matrices, N = 8 to 1,000, three on their own inputs in turn: 10 % standard deviation, and the group and panel it picks are
 // 4 % from the best in the mean; never below 5.5 us (4.6 to 5.5 measured), for the row-wise kernel is as fast there.  Estimate (measured), us: stencil 73 x 61 x 62, N = 88, groups of 8 80 (85); band of 52960 and 64, N = 472,
 // groups of 16 34 (34.5); band of 2144 and 47, N = 808, groups of 4 5.5 (5.6).
-// ENTRIES: the building of the operands besides, for every unit; fitted to 130 products of 27 stencils, N = 8 to 256: 9 %.  71 x 55 x 67,
-// N = 40 36 (35.5); 41 x 35 x 30, N = 208 22 (22.4); 72 x 51 x 40, N = 144 51 (62).
+// ENTRIES: the building of the operands besides, for every unit; fitted to 186 products of 39 stencils, N = 8 to 256: 8 %.  66 x 31 x 43,
+// N = 120 25 (26); 41 x 35 x 30, N = 208 20.6 (21.1); 72 x 51 x 40, N = 144 48 (56).
 double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, const WindowProduct &w)
 {
     const bool entries = w.nnz >= 0;
@@ -644,8 +651,8 @@ double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, 
     const double once = a_bytes + 2.0 * (double)w.K * (double)w.N + c_bytes;
     double steps, path, memory, start;
     if (entries) {
-        steps = l.rounds * (l.panels_per_unit * parts * (1.13 + 0.008 * blocks) + 1.3 + 2.5 * groups16);
-        path = copies / 11.9e6, memory = once / 2.4e6, start = 2.4;
+        steps = l.rounds * (l.panels_per_unit * parts * (0.96 + 0.014 * blocks) + 2.3 * groups16);
+        path = copies / 11.9e6, memory = once / 2.7e6, start = 2.75;
     } else {
         steps = l.rounds * l.panels_per_unit * parts * (1.07 + 0.0155 * blocks);
         path = copies / 8.7e6, memory = once / 5.0e6, start = 1.6 + 2.2 * groups16;
@@ -765,7 +772,7 @@ hipError_t window_attach_entries(WindowPlan &p, const uint16_t *vals, const int3
     e = most.alloc(sizeof too_many);
     if (e == hipSuccess) e = hipMemsetAsync(most.p, 0, sizeof too_many, nullptr);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(window_entries_kernel, dim3((unsigned)((mb + 3) / 4)), dim3(256), 0, nullptr, vals, row_ptr, p.d_slot, offset, (int)mb, p.d_entries, p.d_table,
+        hipLaunchKernelGGL(window_entries_kernel, dim3((unsigned)((mb + 3) / 4)), dim3(256), 0, nullptr, vals, row_ptr, p.d_slot, offset, (int)mb, p.rows, p.d_entries, p.d_table,
                            (uint32_t *)most.p);
         e = hipGetLastError();
     }
