@@ -384,6 +384,10 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         c.B = B; c.Bt = plan->d_bt; c.b_row_major = o.b_layout == SMAT_B_ROW_MAJOR; c.C = C; c.M = M; c.N = N; c.K = K; c.c_f32 = a.c_f32;
         c.plan = plan->compact;
         e = launch_compact(c, static_cast<hipStream_t>(o.stream));
+    } else if (kernel == SMAT_KERNEL_SWEEP && o.kernel == SMAT_KERNEL_AUTO && plan->window && o.b_layout == SMAT_B_COL_MAJOR &&
+               (N == plan->n_cap || window_forced() ||
+                window_launch_us(a, *plan->window) < 0.9 * sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N))) {
+        e = launch_window(a, *plan->window, static_cast<hipStream_t>(o.stream));
     } else if (kernel == SMAT_KERNEL_SWEEP) {
         if (!plan || !plan->sweep.d_ops)
             return set_error(SMAT_ERR_INVALID, "SMAT_KERNEL_SWEEP needs a plan built for it (with col_idx_host)");
@@ -709,7 +713,7 @@ extern "C" int smat_plan_create(smat_plan **out, const int32_t *row_ptr_host,
 // with the row-wise kernel.  Returns the block rows of a group, 0 = row-wise.
 static int g_force_group_rows = 0; // test hook: 64, 32 or 16 whatever the estimates say
 static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, size_t n_items,
-                               RowLengths lengths, bool packed, bool b_row_major)
+                               RowLengths lengths, bool packed, bool b_row_major, double *us = nullptr)
 {
     const size_t mb = M / 16, kb = K / 16;
     if (nnzb < 2 || nnzb >= (size_t)1 << 23 || K >= (size_t)1 << 28 || kb <= 2 * SWEEP_S) return 0;
@@ -725,6 +729,7 @@ static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, s
         const double t = in_place ? sweep_in_place_factor(N) * sweep : sweep + to_col_major;
         if (t < best) best = t, group_rows = rows;
     }
+    if (us) *us = best;
     return group_rows;
 }
 // Test hook (not part of smat.h): sweep_even_rounds.
@@ -769,7 +774,7 @@ static hipError_t sweep_small_groups(smat_plan &p, size_t group_rows)
 static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us, const uint16_t *vals, const CompactCensus *census)
 {
     const size_t mb = p.M / 16, kb = p.K / 16;
-    if (p.kernel != SMAT_KERNEL_ROWWISE || p.kernel_requested != SMAT_KERNEL_AUTO || p.n_split_rows || !window_takes_rows(p.max_item_blocks)) return hipSuccess;
+    if ((p.kernel != SMAT_KERNEL_ROWWISE && !(p.kernel == SMAT_KERNEL_SWEEP && p.sweep_few_tiles)) || p.kernel_requested != SMAT_KERNEL_AUTO || p.n_split_rows || !window_takes_rows(p.max_item_blocks)) return hipSuccess;
     if (!census && rowwise_shares_items(p.n_cap, (size_t)p.n_items, p.nnzb / std::max<size_t>((size_t)p.n_items, 1)) && !window_forced()) return hipSuccess;
     if (!census && p.n_cap <= 16 && !window_forced()) return hipSuccess; // 18 -> 17, 10.4 -> 9.2, but 8.2 -> 9, 6.6 -> 7
     // its estimate knows nothing of the bytes that come from memory, A above all and three times B where that is repacked: 64^3 64 us and
@@ -778,7 +783,7 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     const double row_wise = std::hypot(rowwise_estimate_us(p.M, p.K, p.n_cap, p.nnzb, (size_t)p.n_items, RowLengths::EVEN, p.d_bpack != nullptr),
                                        once + (p.d_bpack ? 4.0 * (double)p.K * (double)p.n_cap / 5e6 : 0.0));
     const double copy = p.d_bcol ? to_col_major_us(p.K, p.n_cap) : 0.0; // before either
-    const double bar = 0.9 * (census ? other_us - copy : row_wise);
+    const double bar = 0.9 * (census ? other_us - copy : std::min(row_wise, other_us));
     // a launch, or the bytes that windows do not save
     if (!window_forced() && bar < std::max(4.7, 2.0 + once)) return hipSuccess;
     WindowWidths widths;
@@ -791,7 +796,10 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     }
     int size;
     const double us = window_choose(widths, WindowProduct{p.M, p.K, p.n_cap, p.nnzb, census ? census->nnz : -1, p.max_item_blocks, false}, &size);
-    if (size < 0 || (!window_forced() && us >= bar)) return slots ? dev_free(slots) : hipSuccess;
+    // The sweep kernel brings all block columns in turn, and multiplies faster: not where the windows are most of them too (2448 x 1280, 16 %,
+    // N = 552 7.9 -> 8.7 us).
+    const bool most_of_b = size >= 0 && !census && other_us < 1e30 && (double)widths.sum[size] > 0.5 * (double)kb * (double)mb / (4 << size);
+    if (size < 0 || (!window_forced() && (us >= bar || most_of_b))) return slots ? dev_free(slots) : hipSuccess;
     hipError_t e = window_build(widths, size, slots, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, &p.window);
     if (e != hipSuccess || !census) return e;
     bool taken;
@@ -949,13 +957,23 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
         // Windows against the compact kernel (whole panels of 16, 32 or 64 columns; row-major B in place), or against the row-wise one where the
         // sweep kernel's rule leaves a matrix to it.
         size_t group_rows = 0;
+        double sweep_us = 1e30;
         if (!take && p->col_idx_host.size() == p->nnzb)
             group_rows = sweep_group_rows(row_ptr_host, p->col_idx_host.data(), p->M, p->K, p->nnzb, p->n_cap, (size_t)p->n_items,
-                                          p->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, p->d_bpack != nullptr, p->d_bcol != nullptr);
-        if (group_rows) e = sweep_small_groups(*p, group_rows);
-        else if (!take || !p->d_bcol)
+                                          p->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, p->d_bpack != nullptr, p->d_bcol != nullptr, &sweep_us);
+        if (group_rows) {
+            // Windows against the sweep kernel, whose streams are made all the same: the plan says that kernel, and launches that ask for it
+            // get it.  us: bands of 13296 rows and 30, N = 304 9.6 -> 7.5, 8320 and 25, N = 576 10.4 -> 8.7, 39584 and 18, N = 904 55 -> 48; 21 x 14 x 52,
+            // N = 88 8.4 -> 6.2, 21 x 76 x 25, N = 224 22.6 -> 20.1.
+            if (!p->d_bcol && !g_force_group_rows) e = take_window_if_room(*p, row_ptr, col_idx, sweep_us, nullptr, nullptr);
+            if (e == hipSuccess) e = sweep_small_groups(*p, group_rows);
+        } else if (!take || !p->d_bcol)
             e = take_window_if_room(*p, row_ptr, col_idx, compact_estimate_us((double)census.n_cols_all, std::min(36.0 * (double)census.n_cols_all, 4.25 * (double)census.n_cols_all + 4.0 * (double)census.nnz), p->M, p->K,
                                                 p->n_cap), vals, take ? &census : nullptr);
+        if (e != hipSuccess) return fail(e);
+    }
+    if (want == SMAT_KERNEL_AUTO && dense_kernel == SMAT_KERNEL_SWEEP && p->sweep_few_tiles && !take && !p->d_bcol) { // attached before
+        e = take_window_if_room(*p, row_ptr, col_idx, sweep_estimate_us((size_t)p->sweep.n_rg, p->sweep_chunks, p->nnzb, p->M, p->n_cap), nullptr, nullptr);
         if (e != hipSuccess) return fail(e);
     }
     if (!take) return SMAT_OK; // nothing would use the list: the plan keeps (or goes back to) a dense kernel

@@ -218,3 +218,25 @@ def test_values_attached_again_replace_the_listed_ones(smat, cuda, oracle, force
     with pytest.raises(smat.SmatError):
         smat.spmm(d[0], d[1], d[2], d[3], torch.empty((M, N + 8), dtype=torch.float16, device=cuda), M, N + 8, K, len(ci), plan=plan)
     plan.close()
+
+
+def test_plans_for_the_sweep_kernel_may_multiply_from_windows(smat, cuda, oracle, force):
+    """A narrow band: the plan says the sweep kernel and takes launches for it, launches that leave the choice take windows, attached twice or not."""
+    import torch
+    d = gen.band(13296, 30)
+    A = smat.csr_to_bcsr(d["M"], d["K"], d["row_ptr"], d["col_idx"], d["val"])
+    N, nnzb = 304, len(A.col_idx)
+    vals = np.random.default_rng(1).integers(-3, 4, nnzb * 256).astype(np.float16).view(np.uint16)
+    B = whole_b(A.K, N, seed=2)
+    t = [to_dev(torch, x, cuda) for x in (vals, A.row_ptr, A.col_idx, B)]
+    want = oracle.spmm_bcsr(A.M, N, A.K, A.row_ptr, A.col_idx, vals, B, threads=8).astype(np.float16)
+    plan = smat.Plan(A.row_ptr, A.M, A.K, nnzb, N, col_idx_host=A.col_idx)
+    for _ in range(2):
+        plan.attach_values(*t[:3])
+        assert plan.info()["kernel"] == smat.KERNEL_SWEEP and smat.lib.smat_internal_plan_window_rows(plan.handle) > 0
+        for n in (N, 128):
+            for kernel in (smat.KERNEL_AUTO, smat.KERNEL_SWEEP):
+                C = torch.full((A.M, n), float("nan"), dtype=torch.float16, device=cuda)
+                smat.spmm(t[0], t[1], t[2], t[3][:A.K * n], C, A.M, n, A.K, nnzb, plan=plan, kernel=kernel)
+                assert np.array_equal(C.cpu().numpy(), want[:, :n])
+    plan.close()
