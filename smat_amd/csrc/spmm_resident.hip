@@ -363,18 +363,24 @@ int best_columns(const ResidentPlan &p, size_t K, size_t N, Launch *l)
     return best;
 }
 
+// The kernel may have as much LDS as there is: said once on a device, when a plan is made, so that a captured launch says nothing.
+template <int T, bool C_F32>
+hipError_t prepare()
+{
+    static std::atomic<uint64_t> prepared{0};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess || (dev < 64 && prepared.load(std::memory_order_relaxed) >> dev & 1)) return e;
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(spmm_resident_kernel<T, C_F32>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MAX_LDS);
+    if (e == hipSuccess && dev < 64) prepared.fetch_or(1ull << dev, std::memory_order_relaxed);
+    return e;
+}
+
 template <int T, bool C_F32>
 hipError_t launch_as(const SpmmArgs &a, const ResidentPlan &p, const Launch &l, hipStream_t st)
 {
-    static std::atomic<uint64_t> prepared{0}; // devices on which the kernel may have that much LDS
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+    const hipError_t e = prepare<T, C_F32>();
     if (e != hipSuccess) return e;
-    if (dev >= 64 || !(prepared.load(std::memory_order_relaxed) >> dev & 1)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(spmm_resident_kernel<T, C_F32>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MAX_LDS);
-        if (e != hipSuccess) return e;
-        if (dev < 64) prepared.fetch_or(1ull << dev, std::memory_order_relaxed);
-    }
     const int units = l.groups * l.shares;
     hipLaunchKernelGGL((spmm_resident_kernel<T, C_F32>), dim3((unsigned)((units + 7) / 8 * 8)), dim3(1024), lds_of(a.K, T), st, (const u32x4 *)p.d_list, p.d_first, p.n_slices,
                        a.B, a.C, (int)a.N, (int)a.K, l.groups, l.shares, (int)columns_together(a.K, a.N));
@@ -446,6 +452,8 @@ hipError_t resident_build(const CompactPlan &c, size_t M, size_t K, int64_t nnz,
                            (int)M, p->d_list);
         e = hipGetLastError();
     }
+    for (auto f : {prepare<2, false>, prepare<2, true>, prepare<4, false>, prepare<4, true>, prepare<8, false>, prepare<8, true>})
+        if (e == hipSuccess) e = f();
     uint32_t n[2] = {0, 0};
     if (e == hipSuccess) e = hipMemcpy(n, p->d_first + n_slices, sizeof n, hipMemcpyDeviceToHost);
     tmp.idle = e == hipSuccess;

@@ -600,19 +600,35 @@ Launch launch_of(int rows, int cap, int tiles, int n_groups, size_t N, bool entr
     return l;
 }
 
+// The kernel may have as much LDS as there is: said once on a device, when a plan is made, so that a captured launch says nothing.
+template <int TN, int PARTS, bool C_F32, bool ENTRIES>
+hipError_t prepare()
+{
+    static std::atomic<uint64_t> prepared{0};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess || (dev < 64 && prepared.load(std::memory_order_relaxed) >> dev & 1)) return e;
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(spmm_window_kernel<TN, PARTS, C_F32, ENTRIES>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MAX_LDS);
+    if (e == hipSuccess && dev < 64) prepared.fetch_or(1ull << dev, std::memory_order_relaxed);
+    return e;
+}
+template <bool ENTRIES>
+hipError_t prepare_all()
+{
+    for (auto f : {prepare<1, 1, false, ENTRIES>, prepare<1, 1, true, ENTRIES>, prepare<1, 2, false, ENTRIES>, prepare<1, 2, true, ENTRIES>, prepare<2, 1, false, ENTRIES>,
+                   prepare<2, 1, true, ENTRIES>, prepare<2, 2, false, ENTRIES>, prepare<2, 2, true, ENTRIES>, prepare<4, 1, false, ENTRIES>, prepare<4, 1, true, ENTRIES>}) {
+        const hipError_t e = f();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 template <int TN, int PARTS, bool C_F32, bool ENTRIES>
 hipError_t launch_as(const SpmmArgs &a, const WindowPlan &p, const Launch &l, hipStream_t st)
 {
-    static std::atomic<uint64_t> prepared{0}; // devices on which the kernel may have that much LDS
     const size_t lds = lds_of(p.rows, p.cap, TN, ENTRIES);
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+    const hipError_t e = prepare<TN, PARTS, C_F32, ENTRIES>();
     if (e != hipSuccess) return e;
-    if (dev >= 64 || !(prepared.load(std::memory_order_relaxed) >> dev & 1)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(spmm_window_kernel<TN, PARTS, C_F32, ENTRIES>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MAX_LDS);
-        if (e != hipSuccess) return e;
-        if (dev < 64) prepared.fetch_or(1ull << dev, std::memory_order_relaxed);
-    }
     hipLaunchKernelGGL((spmm_window_kernel<TN, PARTS, C_F32, ENTRIES>), dim3((unsigned)l.workgroups), dim3((unsigned)(p.rows * 64)), lds, st, a.vals, ENTRIES ? p.d_blocks : a.row_ptr, a.col_idx, a.B,
                        a.C, p.d_window, p.d_count, ENTRIES ? p.d_table : p.d_slot, p.d_entries, (int)(a.M / 16), p.rows, p.cap, p.n_groups, l.n_panels, l.panels_per_unit, (int)a.N, (long)a.K);
     return hipGetLastError();
@@ -746,6 +762,7 @@ hipError_t window_build(const WindowWidths &w, int size, void *slots, const int3
                            p->d_window, p->d_count, p->d_slot);
         e = hipGetLastError();
     }
+    if (e == hipSuccess) e = prepare_all<false>();
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr); // launches on other streams read the lists
     if (e != hipSuccess) {
         window_destroy(p);
@@ -776,6 +793,7 @@ hipError_t window_attach_entries(WindowPlan &p, const uint16_t *vals, const int3
                            (uint32_t *)most.p);
         e = hipGetLastError();
     }
+    if (e == hipSuccess) e = prepare_all<true>();
     if (e == hipSuccess) e = hipMemcpy(&too_many, most.p, sizeof too_many, hipMemcpyDeviceToHost);
     *taken = e == hipSuccess && too_many == 0;
     return e;

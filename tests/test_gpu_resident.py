@@ -134,3 +134,39 @@ def test_which_products_hold_columns(smat, cuda, force):
     assert takes(2048, 2048, 8, 64) == 1
     assert takes(4096, 16384, 16, 256) == 1
     assert takes(1024, 65536, 8, 64) == 0
+
+
+@pytest.mark.parametrize("windows", [False, True])
+def test_captured_launches_replay(smat, cuda, oracle, force, windows):
+    """Columns in LDS and windows of listed nonzeros in a graph, replayed between launches outside of it, B changing from replay to replay."""
+    import torch
+    force(4 if not windows else -1, 0)
+    smat.lib.smat_internal_window_force(8 if windows else -1, 2 if windows else 0)
+    M, K, N = 2048, 2048, 64
+    rng = np.random.default_rng(3)
+    if windows:  # every row two nonzeros near the diagonal
+        rp = np.arange(M + 1, dtype=np.int32) * 2
+        lo = np.clip(np.arange(M) - 20, 0, K - 41)
+        ci = np.sort(lo[:, None] + np.stack([rng.integers(0, 20, M), rng.integers(20, 41, M)], 1), 1).astype(np.int32).reshape(-1)
+        A = smat.csr_to_bcsr(M, K, rp, ci, np.ones(2 * M, np.float16).view(np.uint16))
+    else:
+        A = scattered(smat, np.full(M, 5), K, seed=8)
+    Bs = [rng.integers(-4, 5, K * N).astype(np.float16).view(np.uint16) for _ in range(4)]
+    d = [to_dev(torch, x, cuda) for x in (A.val, A.row_ptr, A.col_idx, Bs[0])]
+    plan = plan_of(smat, A, d, N)
+    assert plan.info()["kernel"] == smat.KERNEL_COMPACT
+    assert smat.lib.smat_internal_plan_resident(plan.handle) == (not windows) and (smat.lib.smat_internal_plan_window_rows(plan.handle) == 8) == windows
+    C = torch.zeros((M, N), dtype=torch.float16, device=cuda)
+    other = torch.zeros_like(C)
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, len(A.col_idx), plan=plan, stream=torch.cuda.current_stream().cuda_stream)
+    for B in Bs:
+        d[3].copy_(to_dev(torch, B, cuda))
+        C.fill_(float("nan"))
+        graph.replay()
+        smat.spmm(d[0], d[1], d[2], d[3], other, M, N, K, len(A.col_idx), plan=plan)
+        torch.cuda.synchronize()
+        want = oracle.spmm_bcsr(M, N, K, A.row_ptr, A.col_idx, A.val, B, threads=4).astype(np.float16)
+        assert np.array_equal(C.cpu().numpy(), want) and torch.equal(C, other)
+    plan.close()
