@@ -230,10 +230,10 @@ __device__ __forceinline__ long row_of_block(const int32_t *__restrict__ row_ptr
 //   else: their nonzeros to entries from entry_start[br] + (nonzeros of the block row before) on, column by column,
 //         each with its place in the operand of its step, and the range of entries of every step to step_range;
 //   used != NULL: used[row] = 1 for the rows of B that the list names.
-// A wavefront takes GATHER_BLOCKS consecutive blocks, four at a time: lane (g = lane / 16, r = lane % 16) holds row r of one.
-// Bound by the second read of the values, where blocks hold more than one nonzero, and by what it writes.  (One thread per block read them 2 bytes at a time, 64 cache lines a load, behind a
-// search of ten loads one after the other: 237 k blocks 54 -> 35 us;
-// 4, 8, 32 blocks a wavefront 36, 35, 39.)
+// A wavefront takes GATHER_BLOCKS consecutive blocks.  A lane looks one up and, where it holds one nonzero, writes that; the others follow four at a
+// time: lane (g = lane / 16, r = lane % 16) holds row r of one.  Bound by loads that need each other (row, its start, values) and by the
+// second read of the values of those others.  (Looking the blocks up four at a time, all 16 lanes alike, took 36 us for 16384^2, 16 a row, 98 % of the
+// blocks of one nonzero; now 16.  64 blocks a wavefront 17.)
 constexpr int GATHER_BLOCKS = 16;
 __global__ __launch_bounds__(256) void gather_kernel(const uint16_t *__restrict__ vals, const uint16_t *__restrict__ mask, const uint32_t *__restrict__ single,
                               const unsigned long long *__restrict__ offset, const int32_t *__restrict__ row_ptr,
@@ -244,37 +244,59 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint16_t *__restrict_
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const long p_first = (((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * GATHER_BLOCKS;
     if (p_first >= nnzb) return;
+    // A lane looks its block up: the row, which is that of the first block or a little further on (past a run of empty rows the rest is halved).
+    const bool live = lane < GATHER_BLOCKS && p_first + lane < nnzb;
+    const long p_mine = live ? p_first + lane : p_first;
     long br = row_of_block(row_ptr, mb, p_first, lane);
-    for (int i = 0; i < GATHER_BLOCKS && p_first + i < nnzb; i += 4) {
-        const bool live = p_first + i + g < nnzb;
-        const long p = live ? p_first + i + g : nnzb - 1;
-        // p is in br or a little further on; past a run of empty rows the rest is halved
-        int ahead = 0;
-        while (ahead < 8 && row_ptr[br + 1] <= p) br++, ahead++;
-        if (ahead == 8) {
-            long lo = br, hi = mb;
-            while (hi - lo > 1) {
-                const long mid = (lo + hi) >> 1;
-                if (row_ptr[mid] <= p) lo = mid; else hi = mid;
-            }
-            br = lo;
+    int ahead = 0;
+    while (ahead < 8 && row_ptr[br + 1] <= p_mine) br++, ahead++;
+    if (ahead == 8) {
+        long lo = br, hi = mb;
+        while (hi - lo > 1) {
+            const long mid = (lo + hi) >> 1;
+            if (row_ptr[mid] <= p_mine) lo = mid; else hi = mid;
         }
-        uint32_t m = live ? mask[p] : 0;
-        const int2 first = start[br]; // of the columns and of the entries
-        if ((drop_full && __popc(m) >= FULL_BLOCK_COLS) || first.x < 0) m = 0; // another kernel multiplies the block or the row
-        const uint32_t only = single[p], mine = r == (int)(only & 15) ? only >> 16 : 0;
+        br = lo;
+    }
+    uint32_t m_mine = live ? mask[p_mine] : 0;
+    const uint32_t only = single[p_mine];
+    const int2 first = start[br]; // of the columns and of the entries
+    if (first.x < 0 || (drop_full && __popc(m_mine) >= FULL_BLOCK_COLS)) m_mine = 0; // another kernel multiplies the row or the block
+    const unsigned long long before = offset[p_mine] - raw[br]; // no borrow: both halves of offset[p] are at least those of raw
+    const int o_mine = first.x + (int)(uint32_t)before, end_mine = first.x + (int)(uint32_t)(raw[br + 1] - raw[br]);
+    const int at_mine = first.y + (int)(before >> 32), c_mine = col_idx[p_mine];
+    if (m_mine && only) { // acol holds zeros
+        const int o = o_mine, c = c_mine + __ffs((int)m_mine) - 1;
+        cols[(o & ~7) + ((o & 1) << 2) + ((o & 7) >> 1)] = c; // their order: below
+        if (used) used[c] = 1;
+        if (acol) {
+            acol[((long)(o >> 3) * 16 + (only & 15)) * 8 + (o & 7)] = (uint16_t)(only >> 16);
+        } else {
+            entries[at_mine] = (only & 0xffff0000u) | (((uint32_t)((o & 31) >> 3) * 128u + (uint32_t)(o & 7) + (only & 15) * 8u) * 2u);
+            if ((o & 31) == 0) step_range[o >> 5].x = at_mine;
+            if ((o & 31) == 31 || o + 1 == end_mine) step_range[o >> 5].y = at_mine + 1;
+        }
+    }
+    // The others four at a time, 16 lanes a block.
+    for (unsigned long long left = __ballot(m_mine != 0 && !only); left;) {
+        unsigned long long l = left;
+        for (int i = 0; i < 4; i++) {
+            if (i < g) l &= l - 1;
+            left &= left - 1;
+        }
+        const int of = l ? __ffsll((long long)l) - 1 : 0;
+        const uint32_t m_of = __shfl(m_mine, of), m = l ? m_of : 0; // all lanes take part
+        const long p = p_first + of, row_end = __shfl(end_mine, of);
         u32x4 w[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
-        if (m && !only) w[0] = reinterpret_cast<const u32x4 *>(vals + p * 256 + r * 16)[0], w[1] = reinterpret_cast<const u32x4 *>(vals + p * 256 + r * 16)[1];
-        const unsigned long long before = offset[p] - raw[br]; // no borrow: both halves of offset[p] are at least those of raw
-        const long row_end = (long)first.x + (long)(uint32_t)(raw[br + 1] - raw[br]);
-        long o = (long)first.x + (long)(uint32_t)before;
-        int32_t at = first.y + (int32_t)(before >> 32);
-        const int32_t c0 = col_idx[p];
+        if (m) w[0] = reinterpret_cast<const u32x4 *>(vals + p * 256 + r * 16)[0], w[1] = reinterpret_cast<const u32x4 *>(vals + p * 256 + r * 16)[1];
+        long o = __shfl(o_mine, of);
+        int32_t at = __shfl(at_mine, of);
+        const int32_t c0 = __shfl(c_mine, of);
 #pragma unroll
         for (int k = 0; k < 16; k++) {
             const bool has = (m >> k) & 1;
             if (!__any(has)) continue;
-            const uint32_t v = only ? mine : k & 1 ? w[k / 8][k % 8 / 2] >> 16 : w[k / 8][k % 8 / 2] & 0xffffu;
+            const uint32_t v = k & 1 ? w[k / 8][k % 8 / 2] >> 16 : w[k / 8][k % 8 / 2] & 0xffffu;
             const uint32_t nonzero = (uint32_t)(__ballot(has && (v & 0x7fffu)) >> (16 * g)) & 0xffffu; // rows of the lane's block
             if (!has) continue;
             // inside its group of 8 the even entries come first, then the odd ones: the lanes of the product kernel that

@@ -44,22 +44,57 @@ size_t lds_of(size_t K, int T) { return ((K + 1) * 2 * T + 15) / 16 * 16; }
 
 // ---- the lists, from the compact kernel's ----
 
-// The 8 values of row `lane % 16` in columns 8 * (lane / 16) .. of a step of 32 listed columns.  tile: 1 KiB of the wavefront's own.
-__device__ __forceinline__ u32x4 step_values(const uint16_t *__restrict__ acol, const uint32_t *__restrict__ entries, const int2 *__restrict__ range, long step,
-                                             u32x4 *tile, int lane)
-{
-    if (acol) return reinterpret_cast<const u32x4 *>(acol)[step * 64 + lane];
-    asm volatile("" ::: "memory");
-    tile[lane] = (u32x4){0, 0, 0, 0};
-    asm volatile("" ::: "memory");
-    const int2 r = range[step];
-    for (int i = r.x + lane; i < r.y; i += 64) {
-        const uint32_t e = entries[i];
-        reinterpret_cast<uint16_t *>(tile)[(e & 0xffffu) / 2] = (uint16_t)(e >> 16);
+// The steps of 32 listed columns of an item one after the other: of each the 8 values of row `lane % 16` in columns 8 * (lane / 16) .., asked
+// for a step ahead (a wavefront that asked when it needed them waited for three loads in turn every step: 16384 rows of 16 25 -> 15 us).
+constexpr int BUILD_WAVES = 4; // of a workgroup: as many as there are block rows would be too few workgroups
+struct Steps {
+    const uint16_t *acol;
+    const uint32_t *entries;
+    const int2 *range;
+    uint16_t *tile; // 1 KiB of the wavefront's own
+    int lane;
+    long first, end, next;
+    u32x4 values;
+    uint32_t e[2];
+    int n;
+    int2 ranges; // of step next / 64 * 64 + lane from the first
+    __device__ __forceinline__ Steps(const WorkItem &it, const uint16_t *acol, const uint32_t *entries, const int2 *range, u32x4 *tile, int lane)
+        : acol(acol), entries(entries), range(range), tile(reinterpret_cast<uint16_t *>(tile)), lane(lane), first(it.begin / 32), end(it.end / 32), next(first)
+    {
+        ask();
     }
-    asm volatile("" ::: "memory");
-    return tile[lane];
-}
+    __device__ __forceinline__ void ask()
+    {
+        if (next >= end) return;
+        if (acol) {
+            values = reinterpret_cast<const u32x4 *>(acol)[next * 64 + lane];
+        } else {
+            const int i = (int)(next - first) & 63;
+            if (i == 0) ranges = next + lane < end ? range[next + lane] : int2{0, 0};
+            const int from = __builtin_amdgcn_readlane(ranges.x, i);
+            n = __builtin_amdgcn_readlane(ranges.y, i) - from; // 128 at most
+            e[0] = lane < n ? entries[from + lane] : 0;
+            e[1] = lane + 64 < n ? entries[from + lane + 64] : 0;
+        }
+        next++;
+    }
+    __device__ __forceinline__ u32x4 take()
+    {
+        if (acol) {
+            const u32x4 v = values;
+            ask();
+            return v;
+        }
+        asm volatile("" ::: "memory");
+        reinterpret_cast<u32x4 *>(tile)[lane] = (u32x4){0, 0, 0, 0};
+        asm volatile("" ::: "memory");
+        if (lane < n) tile[(e[0] & 0xffffu) / 2] = (uint16_t)(e[0] >> 16);
+        if (lane + 64 < n) tile[(e[1] & 0xffffu) / 2] = (uint16_t)(e[1] >> 16);
+        asm volatile("" ::: "memory");
+        ask();
+        return reinterpret_cast<const u32x4 *>(tile)[lane];
+    }
+};
 __device__ __forceinline__ uint32_t half_of(const u32x4 &v, int j) { return j & 1 ? v[j / 2] >> 16 : v[j / 2] & 0xffffu; }
 // Nonzeros of the lane's 8 values
 __device__ __forceinline__ int nonzeros(const u32x4 &v)
@@ -71,19 +106,20 @@ __device__ __forceinline__ int nonzeros(const u32x4 &v)
 }
 
 // length[row] of every row, and how many rows are of every length.  A wavefront takes a block row.
-__global__ __launch_bounds__(1024) void resident_lengths_kernel(const WorkItem *__restrict__ items, int n_items, const uint16_t *__restrict__ acol,
+__global__ __launch_bounds__(64 * BUILD_WAVES) void resident_lengths_kernel(const WorkItem *__restrict__ items, int n_items, const uint16_t *__restrict__ acol,
                                                                 const uint32_t *__restrict__ entries, const int2 *__restrict__ range, int32_t *__restrict__ length,
                                                                 uint32_t *__restrict__ rows_of)
 {
-    __shared__ u32x4 tiles[WAVES][64];
+    __shared__ u32x4 tiles[BUILD_WAVES][64];
     __shared__ uint32_t mine[MAX_ROW + 1];
-    for (int i = threadIdx.x; i <= MAX_ROW; i += 1024) mine[i] = 0;
+    for (int i = threadIdx.x; i <= MAX_ROW; i += 64 * BUILD_WAVES) mine[i] = 0;
     __syncthreads();
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * WAVES + w;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * BUILD_WAVES + w;
     if (i < n_items) {
         const WorkItem it = items[i];
         int n = 0;
-        for (long s = it.begin / 32; s < it.end / 32; s++) n += nonzeros(step_values(acol, entries, range, s, tiles[w], lane));
+        Steps steps(it, acol, entries, range, tiles[w], lane);
+        for (long s = steps.first; s < steps.end; s++) n += nonzeros(steps.take());
         n += __shfl_xor(n, 16);
         n += __shfl_xor(n, 32);
         if (lane < 16) {
@@ -92,7 +128,7 @@ __global__ __launch_bounds__(1024) void resident_lengths_kernel(const WorkItem *
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i <= MAX_ROW; i += 1024)
+    for (int i = threadIdx.x; i <= MAX_ROW; i += 64 * BUILD_WAVES)
         if (mine[i]) atomicAdd(&rows_of[i], mine[i]);
 }
 
@@ -162,12 +198,12 @@ __global__ __launch_bounds__(1024) void resident_places_kernel(const int32_t *__
 }
 
 // The number of every row and its nonzeros in the order of their columns.  list: of slice s from 256 * first[s] on, four words after the other for each lane.
-__global__ __launch_bounds__(1024) void resident_fill_kernel(const WorkItem *__restrict__ items, int n_items, const uint16_t *__restrict__ acol,
+__global__ __launch_bounds__(64 * BUILD_WAVES) void resident_fill_kernel(const WorkItem *__restrict__ items, int n_items, const uint16_t *__restrict__ acol,
                                                              const uint32_t *__restrict__ entries, const int2 *__restrict__ range, const int32_t *__restrict__ cols,
                                                              const uint32_t *__restrict__ place, const uint32_t *__restrict__ first, int M, uint32_t *__restrict__ list)
 {
-    __shared__ u32x4 tiles[WAVES][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * WAVES + w, g = lane >> 4;
+    __shared__ u32x4 tiles[BUILD_WAVES][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * BUILD_WAVES + w, g = lane >> 4;
     if (i == 0 && M + lane < (M + 63) / 64 * 64) list[(size_t)first[M / 64] * 256 + ((M + lane) & 63) * 4] = PADDED; // places without a row
     if (i >= n_items) return;
     const WorkItem it = items[i];
@@ -176,8 +212,14 @@ __global__ __launch_bounds__(1024) void resident_fill_kernel(const WorkItem *__r
     const int room = (int)(first[slice + 1] - first[slice]) * 4;
     if (lane < 16) to[0] = (uint32_t)(it.block_row * 16 + lane);
     int done = 1;
-    for (long s = it.begin / 32; s < it.end / 32; s++) {
-        const u32x4 v = step_values(acol, entries, range, s, tiles[w], lane);
+    Steps steps(it, acol, entries, range, tiles[w], lane);
+    auto columns = [&](long s, int i) { return reinterpret_cast<const u32x4 *>(cols)[s * 8 + g * 2 + i]; };
+    u32x4 here[2], soon[2];
+    if (steps.first < steps.end) soon[0] = columns(steps.first, 0), soon[1] = columns(steps.first, 1);
+    for (long s = steps.first; s < steps.end; s++) {
+        here[0] = soon[0], here[1] = soon[1];
+        if (s + 1 < steps.end) soon[0] = columns(s + 1, 0), soon[1] = columns(s + 1, 1);
+        const u32x4 v = steps.take();
         const int n = nonzeros(v);
         int before = 0, all = 0;
 #pragma unroll
@@ -187,12 +229,11 @@ __global__ __launch_bounds__(1024) void resident_fill_kernel(const WorkItem *__r
             all += of;
         }
         int o = done + before;
-        const long c = s * 32 + g * 8;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
+        for (int j = 0; j < 8; j++) { // the even columns come first
             const uint32_t h = half_of(v, j);
             if (h & 0x7fffu) {
-                if (o < room) to[(size_t)(o / 4) * 256 + (o & 3)] = h << 16 | (uint32_t)cols[c + ((j & 1) << 2) + (j >> 1)];
+                if (o < room) to[(size_t)(o / 4) * 256 + (o & 3)] = h << 16 | here[j & 1][j >> 1];
                 o++;
             }
         }
@@ -443,12 +484,12 @@ hipError_t resident_build(const CompactPlan &c, size_t M, size_t K, int64_t nnz,
         e = hipMemsetAsync(rows_of, 0, (MAX_ROW + 1) * sizeof(uint32_t), nullptr);
     }
     if (e == hipSuccess) e = hipMemsetD32Async((hipDeviceptr_t)p->d_list, (int)K, fours * 256, nullptr);
-    const unsigned wgs = (unsigned)((c.n_items + WAVES - 1) / WAVES);
+    const unsigned wgs = (unsigned)((c.n_items + BUILD_WAVES - 1) / BUILD_WAVES);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(resident_lengths_kernel, dim3(wgs), dim3(1024), 0, nullptr, c.d_items, c.n_items, c.d_acol, c.d_entries, c.d_step_range, (int32_t *)lengths, rows_of);
+        hipLaunchKernelGGL(resident_lengths_kernel, dim3(wgs), dim3(64 * BUILD_WAVES), 0, nullptr, c.d_items, c.n_items, c.d_acol, c.d_entries, c.d_step_range, (int32_t *)lengths, rows_of);
         hipLaunchKernelGGL(resident_slices_kernel, dim3(1), dim3(1024), 0, nullptr, rows_of, n_slices, p->d_first, p->d_first + n_slices + 1);
         hipLaunchKernelGGL(resident_places_kernel, dim3((unsigned)((M + 1023) / 1024)), dim3(1024), 0, nullptr, (const int32_t *)lengths, (int)M, rows_of, places);
-        hipLaunchKernelGGL(resident_fill_kernel, dim3(wgs), dim3(1024), 0, nullptr, c.d_items, c.n_items, c.d_acol, c.d_entries, c.d_step_range, c.d_cols, places, p->d_first,
+        hipLaunchKernelGGL(resident_fill_kernel, dim3(wgs), dim3(64 * BUILD_WAVES), 0, nullptr, c.d_items, c.n_items, c.d_acol, c.d_entries, c.d_step_range, c.d_cols, places, p->d_first,
                            (int)M, p->d_list);
         e = hipGetLastError();
     }
