@@ -158,8 +158,11 @@ int smat_plan_create(smat_plan **plan, const int32_t *row_ptr_host, const int32_
  * SMAT_KERNEL_COMPACT multiplies only those and touches only the rows of B under them; with
  * SMAT_KERNEL_AUTO the plan switches to that kernel when fewer than 60% of the block columns
  * are nonzero.  The compact kernel works from the copy: attach again after the values change.
+ * Where it is estimated to be faster, launches of such a plan on a column-major B that leave the kernel to the plan multiply the listed nonzeros
+ * from windows of B in LDS, shared by neighbouring block rows that use the same block columns, or with whole columns of B in LDS; launches that ask
+ * for SMAT_KERNEL_COMPACT get that kernel.  Plans for the row-wise or sweep kernel may multiply whole blocks from such windows in the same way.
  * The new list is built before the old one is dropped; if the call fails the plan has no list and
- * SMAT_KERNEL_AUTO goes back to the sweep or row-wise kernel.  When the plan takes the compact kernel, the call also
+ * SMAT_KERNEL_AUTO goes back to the sweep or row-wise kernel.  When the plan takes the compact kernel and neither windows nor columns, the call also
  * times ten or so launches of it on zeros (temporary device buffers of K x n_hint and M x n_hint halves, freed before it
  * returns; skipped if they do not fit) to choose how the work is dealt to the GPU's eight XCDs: a choice that moves
  * no bit of any result.  Synchronous.  No counterpart in the reference, which multiplies every block as a dense
@@ -197,7 +200,8 @@ int smat_plan_info(const smat_plan *plan, int64_t *info);
  * Non-finite inputs: one MFMA covers two blocks.  The row-wise kernel multiplies an unpaired
  * block together with a block of zeros and no others (a complete pair under an Inf in B gives what a
  * block-by-block product gives), the compact kernel pads a block row with zero columns and may list a column with many
- * nonzeros several times, each time with a part of them and zeros (0 x Inf = NaN where B holds Inf or NaN).  The sweep kernel multiplies an unpaired block together with
+ * nonzeros several times, each time with a part of them and zeros (0 x Inf = NaN where B holds Inf or NaN); windows of listed nonzeros multiply the
+ * blocks whole, columns in LDS the nonzeros alone.  The sweep kernel multiplies an unpaired block together with
  * a neighbouring block of the SAME block row and 16 rows of zeros in place of B, and its filler ops multiply two
  * blocks of the block row they add to by zeros: an Inf or NaN in vals stays in its own block row of C (where a
  * block-by-block product, mmaCBT.cu:44-66, has an Inf or NaN as well).  Only a block that is alone in its block
