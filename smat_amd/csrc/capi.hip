@@ -800,7 +800,7 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     // N = 552 7.9 -> 8.7 us).
     const bool most_of_b = size >= 0 && !census && other_us < 1e30 && (double)widths.sum[size] > 0.5 * (double)kb * (double)mb / (4 << size);
     if (size < 0 || (!window_forced() && (us >= bar || most_of_b))) return slots ? dev_free(slots) : hipSuccess;
-    hipError_t e = window_build(widths, size, slots, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, &p.window);
+    hipError_t e = window_build(widths, size, slots, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, !census, &p.window);
     if (e != hipSuccess || !census) return e;
     bool taken;
     e = window_attach_entries(*p.window, vals, row_ptr, (const unsigned long long *)census->offset.p, mb, p.nnzb, census->nnz, &taken);
@@ -1050,7 +1050,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     // Columns of B in LDS against the compact kernel; no memory for their lists is not an error of the plan.
     if (want == SMAT_KERNEL_AUTO && !mixed && !block_split && !p->window && !p->d_bcol) {
         const double bar = 0.9 * compact_estimate_us(*c, p->M, p->K, p->n_cap);
-        if (resident_forced() || resident_estimate_us(p->M, p->K, p->n_cap, census.nnz) < bar) {
+        if (resident_forced() || resident_estimate_us(p->M, p->K, p->n_cap, census.nnz, c->n_split_rows > 0) < bar) {
             e = resident_build(*c, p->M, p->K, census.nnz, &p->resident);
             if (e == hipErrorOutOfMemory) e = hipSuccess, (void)hipGetLastError();
             if (e != hipSuccess) return fail(e);

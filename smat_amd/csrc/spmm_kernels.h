@@ -203,8 +203,9 @@ hipError_t window_widths(const int32_t *row_ptr, const int32_t *col_idx, size_t 
 void window_widths_host(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, WindowWidths &out); // the same from host arrays
 // The size of group (index into the widths, -1 = none fits) that is fastest for a product of N columns, and its time in us.
 double window_choose(const WindowWidths &widths, const WindowProduct &w, int *size);
+// wait = false: the caller waits for the default stream before the plan is used.
 hipError_t window_build(const WindowWidths &w, int size, void *slots, const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, int most_blocks,
-                        WindowPlan **out);
+                        bool wait, WindowPlan **out);
 void window_destroy(WindowPlan *p);
 bool window_forced(); // by the test hook
 bool window_takes_rows(int most_blocks); // block rows of so many blocks
@@ -217,16 +218,16 @@ hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st)
 
 // ---- columns of B in LDS (spmm_resident.hip) ----
 struct ResidentPlan {
-    int n_slices = 0, longest = 0; // of 64 rows each; nonzeros of the longest row
+    int n_slices = 0, longest = 0; // of 64 lanes each; nonzeros of the longest lane
     int64_t fours = 0;             // fours of nonzeros a lane, of all slices
-    uint32_t *d_list = nullptr;    // of every lane its row, then value << 16 | row of B; 256 * d_first[s] before slice s
+    uint32_t *d_list = nullptr;    // of every lane its row and the lanes that share it, then value << 16 | row of B; 256 * d_first[s] before slice s
     uint32_t *d_first = nullptr;
 };
 // From the lists of the compact kernel, which must be all of the matrix; synchronous, on the default stream.  *out: NULL where they do not fit.
 hipError_t resident_build(const CompactPlan &c, size_t M, size_t K, int64_t nnz, ResidentPlan **out);
 void resident_destroy(ResidentPlan *p);
 bool resident_forced(); // by the test hook
-double resident_estimate_us(size_t M, size_t K, size_t N, int64_t nnz); // for rows of about the same length; 1e30: K too long
+double resident_estimate_us(size_t M, size_t K, size_t N, int64_t nnz, bool long_rows); // before the lists are there; 1e30: K too long
 double resident_launch_us(const ResidentPlan &p, size_t K, size_t N);
 hipError_t launch_resident(const SpmmArgs &a, const ResidentPlan &p, hipStream_t st); // column-major B
 

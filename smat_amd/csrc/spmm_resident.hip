@@ -13,7 +13,8 @@
 // allows and the launch is still wide enough for.  Loads of the list four ahead, since 16 wavefronts wait for them together.
 //
 // Rows are put in order of their lengths and dealt 64 at a time, back and forth over the wavefronts, so that the lanes of one
-// end together and the wavefronts have equally much.  Lists are padded to fours of nonzeros by zeros that meet a row of zeros behind B.
+// end together and the wavefronts have equally much.  A row of more than PART nonzeros is shared by 2 to 64 neighbouring lanes, whose sums
+// are added in the end.  Lists are padded to fours of nonzeros by zeros that meet a row of zeros behind B.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -36,17 +37,37 @@ template <int T> using floats = float __attribute__((ext_vector_type(T)));
 
 constexpr int WAVES = 16;              // wavefronts of a workgroup
 constexpr size_t MAX_LDS = 160 * 1024;
-constexpr int PADDED = 0x7fffffff;     // the row of a lane that has none
 constexpr int AHEAD = 4;               // fours that a wavefront asks for ahead
-constexpr int MAX_ROW = 2047;          // nonzeros of a row
+constexpr int PART = 64;               // nonzeros of a lane
+constexpr int SHARED = 6;              // a row is shared by 1 << SHARED lanes at most
+constexpr int MAX_ROW = PART << SHARED;
+constexpr uint32_t ROW_BITS = 28;      // of a lane's first word: its row; above them the logarithm of the lanes that share it
+constexpr uint32_t PADDED = (1u << ROW_BITS) - 1; // the row of a lane that has none
+// Kinds of rows, the longest first: those shared by 64, 32, .. 2 lanes, then those of PART, PART - 1, .. 0 nonzeros.
+constexpr int KINDS = SHARED + PART + 1;
+__host__ __device__ constexpr int lanes_log(int kind) { return kind < SHARED ? SHARED - kind : 0; }
+__device__ __forceinline__ int kind_of(int n)
+{
+    if (n <= PART) return SHARED + PART - n;
+    const int log = 32 - __clz((n + PART - 1) / PART - 1);
+    return log < SHARED ? SHARED - log : 0; // longer ones than MAX_ROW: the lists are not taken
+}
+// Numbers of rows of every kind and the longest row, COUNTS times: additions to one word queue up at 12 ns each.
+constexpr int COUNTS = 16;
+struct ResidentTotals { // in front of ResidentPlan::d_first
+    uint32_t n_slices, fours, longest, places;
+    uint32_t rows_of[COUNTS][KINDS], longest_of[COUNTS];
+};
+constexpr size_t IN_FRONT = sizeof(ResidentTotals) / sizeof(uint32_t);
 
 size_t lds_of(size_t K, int T) { return ((K + 1) * 2 * T + 15) / 16 * 16; }
 
 // ---- the lists, from the compact kernel's ----
 
 // The steps of 32 listed columns of an item one after the other: of each the 8 values of row `lane % 16` in columns 8 * (lane / 16) .., asked
-// for a step ahead (a wavefront that asked when it needed them waited for three loads in turn every step: 16384 rows of 16 25 -> 15 us).
-constexpr int BUILD_WAVES = 4; // of a workgroup: as many as there are block rows would be too few workgroups
+// for a step ahead (a wavefront that asked when it needed them waited for three loads in turn every step: 16384 rows of 16 25 -> 15 us).  The
+// wavefronts of a workgroup take an eighth of an item each.
+constexpr int BUILD_WAVES = 8;
 struct Steps {
     const uint16_t *acol;
     const uint32_t *entries;
@@ -58,9 +79,12 @@ struct Steps {
     uint32_t e[2];
     int n;
     int2 ranges; // of step next / 64 * 64 + lane from the first
-    __device__ __forceinline__ Steps(const WorkItem &it, const uint16_t *acol, const uint32_t *entries, const int2 *range, u32x4 *tile, int lane)
-        : acol(acol), entries(entries), range(range), tile(reinterpret_cast<uint16_t *>(tile)), lane(lane), first(it.begin / 32), end(it.end / 32), next(first)
+    __device__ __forceinline__ Steps(const WorkItem &it, int eighth, const uint16_t *acol, const uint32_t *entries, const int2 *range, u32x4 *tile, int lane)
+        : acol(acol), entries(entries), range(range), tile(reinterpret_cast<uint16_t *>(tile)), lane(lane)
     {
+        const long each = (it.end - it.begin) / 32 / BUILD_WAVES + ((it.end - it.begin) / 32 % BUILD_WAVES != 0);
+        end = min((long)it.begin / 32 + (eighth + 1) * each, (long)it.end / 32);
+        next = first = min((long)it.begin / 32 + eighth * each, end);
         ask();
     }
     __device__ __forceinline__ void ask()
@@ -105,38 +129,78 @@ __device__ __forceinline__ int nonzeros(const u32x4 &v)
     return n;
 }
 
-// length[row] of every row, and how many rows are of every length.  A wavefront takes a block row.
-__global__ __launch_bounds__(64 * BUILD_WAVES) void resident_lengths_kernel(const WorkItem *__restrict__ items, int n_items, const uint16_t *__restrict__ acol,
-                                                                const uint32_t *__restrict__ entries, const int2 *__restrict__ range, int32_t *__restrict__ length,
-                                                                uint32_t *__restrict__ rows_of)
+// Nonzeros of the rows of an item: of a block row that is one item to length, and to the numbers of rows of every kind; of a part of a block row to
+// its own 16 in parts.  before: nonzeros of the eighths before every eighth of the item.  A workgroup takes an item.
+__global__ __launch_bounds__(64 * BUILD_WAVES) void resident_lengths_kernel(const WorkItem *__restrict__ items, const uint16_t *__restrict__ acol,
+                                                                            const uint32_t *__restrict__ entries, const int2 *__restrict__ range,
+                                                                            int32_t *__restrict__ length, int32_t *__restrict__ parts, int32_t *__restrict__ before,
+                                                                            ResidentTotals *__restrict__ totals)
 {
     __shared__ u32x4 tiles[BUILD_WAVES][64];
-    __shared__ uint32_t mine[MAX_ROW + 1];
-    for (int i = threadIdx.x; i <= MAX_ROW; i += 64 * BUILD_WAVES) mine[i] = 0;
+    __shared__ int32_t of[BUILD_WAVES][16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const WorkItem it = items[blockIdx.x];
+    int n = 0;
+    Steps steps(it, w, acol, entries, range, tiles[w], lane);
+    for (long s = steps.first; s < steps.end; s++) n += nonzeros(steps.take());
+    n += __shfl_xor(n, 16);
+    n += __shfl_xor(n, 32);
+    if (lane < 16) of[w][lane] = n;
     __syncthreads();
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * BUILD_WAVES + w;
-    if (i < n_items) {
-        const WorkItem it = items[i];
-        int n = 0;
-        Steps steps(it, acol, entries, range, tiles[w], lane);
-        for (long s = steps.first; s < steps.end; s++) n += nonzeros(steps.take());
-        n += __shfl_xor(n, 16);
-        n += __shfl_xor(n, 32);
-        if (lane < 16) {
-            length[it.block_row * 16 + lane] = n;
-            atomicAdd(&mine[min(n, MAX_ROW)], 1u);
-        }
+    if (w) return;
+    if (lane >= 16) return;
+    const int m = lane; // row
+    int all = 0;
+#pragma unroll
+    for (int k = 0; k < BUILD_WAVES; k++) {
+        before[((size_t)blockIdx.x * BUILD_WAVES + k) * 16 + m] = all;
+        all += of[k][m];
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i <= MAX_ROW; i += 64 * BUILD_WAVES)
-        if (mine[i]) atomicAdd(&rows_of[i], mine[i]);
+    (it.dst < 0 ? length + it.block_row * 16 : parts + it.dst * 16)[m] = all;
+    if (it.dst >= 0) return;
+    // one addition for the rows of a kind
+    const int copy = (int)blockIdx.x % COUNTS;
+    const int kind = kind_of(all);
+    int same = 0, first = 16, most = all;
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        const int other = __shfl(kind, k);
+        if (other == kind) same++, first = min(first, k);
+        most = max(most, __shfl(all, k));
+    }
+    if (first == m) atomicAdd(&totals->rows_of[copy][kind], (uint32_t)same);
+    if (m == 0) atomicMax(&totals->longest_of[copy], (uint32_t)most);
 }
 
-// Longest rows first: rows_of[length] becomes the place of the first row of that length; first[s] the fours before slice s
-// (64 rows), first[n_slices] those of all; *longest the longest row.  One workgroup.
-__global__ __launch_bounds__(1024) void resident_slices_kernel(uint32_t *__restrict__ rows_of, int n_slices, uint32_t *__restrict__ first, uint32_t *__restrict__ longest)
+// parts of a split block row: from nonzeros of every part to those of the parts before it.  A wavefront takes a block row, four parts at a time.
+__global__ __launch_bounds__(64) void resident_parts_kernel(const SplitRow *__restrict__ split, int32_t *__restrict__ length, int32_t *__restrict__ parts,
+                                                            ResidentTotals *__restrict__ totals)
 {
-    __shared__ uint32_t place[MAX_ROW + 2], part[1024], carry;
+    const SplitRow row = split[blockIdx.x];
+    const int lane = threadIdx.x, g = lane >> 4;
+    int before = 0;
+    for (int p = row.slot_begin; p < row.slot_end; p += 4) {
+        const int n = p + g < row.slot_end ? parts[(p + g) * 16 + (lane & 15)] : 0;
+        int mine = before;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int of = __shfl(n, (lane & 15) + 16 * k);
+            mine += k < g ? of : 0;
+            before += of;
+        }
+        if (p + g < row.slot_end) parts[(p + g) * 16 + (lane & 15)] = mine;
+    }
+    if (lane < 16) {
+        length[row.block_row * 16 + lane] = before;
+        atomicAdd(&totals->rows_of[blockIdx.x % COUNTS][kind_of(before)], 1u);
+        atomicMax(&totals->longest_of[blockIdx.x % COUNTS], (uint32_t)before);
+    }
+}
+
+// rows_of[0][kind] becomes the place of the first row of that kind; first[s] the fours before slice s (64 places), first[n_slices] those of all.  One workgroup.
+__global__ __launch_bounds__(1024) void resident_slices_kernel(uint32_t *__restrict__ first, ResidentTotals *__restrict__ totals)
+{
+    __shared__ uint32_t place[KINDS + 1], part[1024], carry;
     const int t = (int)threadIdx.x;
     auto scan = [&](uint32_t v) { // exclusive sum over the workgroup; part[1023] holds the inclusive one of all
         part[t] = v;
@@ -149,24 +213,32 @@ __global__ __launch_bounds__(1024) void resident_slices_kernel(uint32_t *__restr
         }
         return part[t] - v;
     };
-    const uint32_t a = rows_of[MAX_ROW - 2 * t], b = rows_of[MAX_ROW - 2 * t - 1];
-    const uint32_t before = scan(a + b);
-    place[2 * t] = before, place[2 * t + 1] = before + a; // of length MAX_ROW - index
-    if (t == 0) place[MAX_ROW + 1] = 0xffffffffu, carry = 0;
-    rows_of[MAX_ROW - 2 * t] = before, rows_of[MAX_ROW - 2 * t - 1] = before + a;
+    uint32_t rows = 0;
+    if (t < KINDS)
+#pragma unroll
+        for (int k = 0; k < COUNTS; k++) rows += totals->rows_of[k][t];
+    const uint32_t before = scan(rows << lanes_log(t));
+    const uint32_t places = part[1023];
+    if (t < KINDS) place[t] = before, totals->rows_of[0][t] = before;
+    if (t == 0) {
+        place[KINDS] = 0xffffffffu, carry = 0;
+        uint32_t longest = 0;
+        for (int k = 0; k < COUNTS; k++) longest = max(longest, totals->longest_of[k]);
+        totals->longest = longest;
+    }
     __syncthreads();
+    const int n_slices = (int)((places + 63) / 64);
     for (int s0 = 0; s0 < n_slices; s0 += 1024) {
         const int s = s0 + t;
         uint32_t fours = 0;
-        if (s < n_slices) { // the last index whose place is not behind the slice's first row
-            int lo = 0, hi = MAX_ROW + 1;
+        if (s < n_slices) { // the last kind whose place is not behind the slice's first row
+            int lo = 0, hi = KINDS;
             while (hi - lo > 1) {
                 const int mid = (lo + hi) / 2;
                 if (place[mid] <= (uint32_t)s * 64u) lo = mid; else hi = mid;
             }
-            const uint32_t len = (uint32_t)(MAX_ROW - lo);
+            const uint32_t len = lo < SHARED ? PART : (uint32_t)(SHARED + PART - lo);
             fours = (len + 4) / 4; // the row's number first
-            if (s == 0) *longest = len;
         }
         const uint32_t at = scan(fours);
         if (s < n_slices) first[s] = carry + at;
@@ -174,45 +246,67 @@ __global__ __launch_bounds__(1024) void resident_slices_kernel(uint32_t *__restr
         if (t == 0) carry += part[1023];
         __syncthreads();
     }
-    if (t == 0) first[n_slices] = carry;
+    if (t == 0) first[n_slices] = carry, totals->n_slices = (uint32_t)n_slices, totals->fours = carry, totals->places = places;
 }
 
-// The place of every row among the sorted ones.
-__global__ __launch_bounds__(1024) void resident_places_kernel(const int32_t *__restrict__ length, int M, uint32_t *__restrict__ next, uint32_t *__restrict__ place)
+// The place of every row among the sorted ones, and the first words of its lanes; the lists of lanes without a row, and a four of zeros behind all.
+__global__ __launch_bounds__(1024) void resident_places_kernel(const int32_t *__restrict__ length, int M, uint32_t *__restrict__ place,
+                                                               const uint32_t *__restrict__ first, ResidentTotals *__restrict__ totals, uint32_t K, uint32_t *__restrict__ list)
 {
-    __shared__ uint32_t mine[MAX_ROW + 1];
-    for (int i = threadIdx.x; i <= MAX_ROW; i += 1024) mine[i] = 0;
+    __shared__ uint32_t mine[KINDS];
+    for (int i = threadIdx.x; i < KINDS; i += 1024) mine[i] = 0;
     __syncthreads();
     const int row = (int)(blockIdx.x * 1024 + threadIdx.x);
-    const int n = row < M ? min(length[row], MAX_ROW) : 0;
+    const int kind = row < M ? kind_of(length[row]) : 0, log = lanes_log(kind);
     uint32_t at = 0;
-    if (row < M) at = atomicAdd(&mine[n], 1u);
-    __syncthreads();
-    for (int i = threadIdx.x; i <= MAX_ROW; i += 1024)
-        if (mine[i]) mine[i] = atomicAdd(&next[i], mine[i]);
-    __syncthreads();
-    if (row < M) {
-        at += mine[n];
-        place[row] = at;
+    // empty rows, of which there may be many, a wavefront at a time
+    const bool none = row < M && kind == KINDS - 1;
+    const unsigned long long nones = __ballot(none);
+    if (none) {
+        const int lead = __ffsll((long long)nones) - 1, lane = threadIdx.x & 63;
+        if (lane == lead) at = atomicAdd(&mine[kind], (uint32_t)__popcll(nones));
+        at = __shfl(at, lead) + __popcll(nones & ((1ull << lane) - 1));
+    } else if (row < M) {
+        at = atomicAdd(&mine[kind], 1u << log);
     }
+    __syncthreads();
+    for (int i = threadIdx.x; i < KINDS; i += 1024)
+        if (mine[i]) mine[i] = atomicAdd(&totals->rows_of[0][i], mine[i]);
+    __syncthreads();
+    auto word = [&](uint32_t at) -> uint32_t & { return list[(size_t)first[at / 64] * 256 + (at & 63) * 4]; };
+    if (row < M) {
+        at += mine[kind];
+        place[row] = at;
+        uint32_t *const to = &word(at);
+        for (uint32_t k = 0; k < 1u << log; k++) to[k * 4] = (uint32_t)log << ROW_BITS | (uint32_t)row;
+    }
+    if (blockIdx.x == 0 && totals->places + threadIdx.x < totals->n_slices * 64) {
+        uint32_t *const to = &word(totals->places + threadIdx.x);
+        to[0] = PADDED;
+        for (uint32_t w = 1; w < (totals->fours - first[totals->n_slices - 1]) * 4; w++) to[w / 4 * 256 + (w & 3)] = K;
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 256) list[(size_t)totals->fours * 256 + threadIdx.x] = K;
 }
 
-// The number of every row and its nonzeros in the order of their columns.  list: of slice s from 256 * first[s] on, four words after the other for each lane.
-__global__ __launch_bounds__(64 * BUILD_WAVES) void resident_fill_kernel(const WorkItem *__restrict__ items, int n_items, const uint16_t *__restrict__ acol,
-                                                             const uint32_t *__restrict__ entries, const int2 *__restrict__ range, const int32_t *__restrict__ cols,
-                                                             const uint32_t *__restrict__ place, const uint32_t *__restrict__ first, int M, uint32_t *__restrict__ list)
+// The nonzeros of every row in the order of their columns behind the first words, and zeros that meet the row of zeros behind B.  list: of slice s from 256 * first[s] on, four words after the other
+// for each lane.
+__global__ __launch_bounds__(64 * BUILD_WAVES) void resident_fill_kernel(const WorkItem *__restrict__ items, const uint16_t *__restrict__ acol,
+                                                                         const uint32_t *__restrict__ entries, const int2 *__restrict__ range,
+                                                                         const int32_t *__restrict__ cols, const int32_t *__restrict__ length,
+                                                                         const int32_t *__restrict__ parts, const int32_t *__restrict__ before_eighth,
+                                                                         const uint32_t *__restrict__ place,
+                                                                         const uint32_t *__restrict__ first, uint32_t K, bool zeros_there, uint32_t *__restrict__ list)
 {
     __shared__ u32x4 tiles[BUILD_WAVES][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * BUILD_WAVES + w, g = lane >> 4;
-    if (i == 0 && M + lane < (M + 63) / 64 * 64) list[(size_t)first[M / 64] * 256 + ((M + lane) & 63) * 4] = PADDED; // places without a row
-    if (i >= n_items) return;
-    const WorkItem it = items[i];
-    const uint32_t at = place[it.block_row * 16 + (lane & 15)], slice = at / 64;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4;
+    const WorkItem it = items[blockIdx.x];
+    const int row = it.block_row * 16 + (lane & 15), all_of_row = length[row], log = lanes_log(kind_of(all_of_row));
+    const uint32_t at = place[row], slice = at / 64; // the lanes that share a row are in one slice
     uint32_t *const to = list + (size_t)first[slice] * 256 + (at & 63) * 4;
-    const int room = (int)(first[slice + 1] - first[slice]) * 4;
-    if (lane < 16) to[0] = (uint32_t)(it.block_row * 16 + lane);
-    int done = 1;
-    Steps steps(it, acol, entries, range, tiles[w], lane);
+    const int room = (int)(first[slice + 1] - first[slice]) * 4, each = max((all_of_row + (1 << log) - 1) >> log, 1);
+    const float per_each = 1.0f / (float)each; // for numbers below MAX_ROW: a product has the quotient's whole part
+    int done = (it.dst < 0 ? 0 : parts[it.dst * 16 + (lane & 15)]) + before_eighth[((size_t)blockIdx.x * BUILD_WAVES + w) * 16 + (lane & 15)];
+    Steps steps(it, w, acol, entries, range, tiles[w], lane);
     auto columns = [&](long s, int i) { return reinterpret_cast<const u32x4 *>(cols)[s * 8 + g * 2 + i]; };
     u32x4 here[2], soon[2];
     if (steps.first < steps.end) soon[0] = columns(steps.first, 0), soon[1] = columns(steps.first, 1);
@@ -233,12 +327,16 @@ __global__ __launch_bounds__(64 * BUILD_WAVES) void resident_fill_kernel(const W
         for (int j = 0; j < 8; j++) { // the even columns come first
             const uint32_t h = half_of(v, j);
             if (h & 0x7fffu) {
-                if (o < room) to[(size_t)(o / 4) * 256 + (o & 3)] = h << 16 | here[j & 1][j >> 1];
+                const int share = log ? (int)(((float)o + 0.5f) * per_each) : 0, word = o - share * each + 1;
+                if (word < room && share < 1 << log) to[(size_t)(word / 4) * 256 + (word & 3) + share * 4] = h << 16 | here[j & 1][j >> 1];
                 o++;
             }
         }
         done += all;
     }
+    if (!zeros_there && done == all_of_row) // behind the last of them
+        for (int share = 0; share < 1 << log; share++)
+            for (int word = min(max(all_of_row - share * each, 0), each) + 1 + g; word < room; word += 4) to[(size_t)(word / 4) * 256 + (word & 3) + share * 4] = K;
 }
 
 // ---- the product ----
@@ -299,7 +397,8 @@ __global__ __launch_bounds__(1024) void spmm_resident_kernel(const u32x4 *__rest
     }
     __syncthreads();
 
-    int j = 0, s = slice_of(0), row = -1;
+    int j = 0, s = slice_of(0);
+    uint32_t row = PADDED; // and the lanes that share it
     uint32_t left = 0;
     bool fresh;
     floats<T> acc;
@@ -309,10 +408,18 @@ __global__ __launch_bounds__(1024) void spmm_resident_kernel(const u32x4 *__rest
         fresh = true;
     };
     auto store = [&] {
-        if (row == PADDED) return;
+        const uint32_t log = row >> ROW_BITS, m = row & PADDED;
+        if (__any(log != 0))
+            for (uint32_t d = 1; d < 1u << SHARED; d *= 2)
+#pragma unroll
+                for (int t = 0; t < T; t++) {
+                    const float other = __shfl_xor(acc[t], d);
+                    if (d < 1u << log) acc[t] += other;
+                }
+        if (m == PADDED || (lane & ((1u << log) - 1))) return;
         if constexpr (C_F32) {
             constexpr int V = T < 4 ? T : 4;
-            float *const c = static_cast<float *>(C) + (size_t)row * N + n0;
+            float *const c = static_cast<float *>(C) + (size_t)m * N + n0;
 #pragma unroll
             for (int t = 0; t < T; t += V) {
                 floats<V> v;
@@ -321,7 +428,7 @@ __global__ __launch_bounds__(1024) void spmm_resident_kernel(const u32x4 *__rest
                 *reinterpret_cast<floats<V> *>(c + t) = v;
             }
         } else {
-            *reinterpret_cast<halves<T> *>(static_cast<uint16_t *>(C) + (size_t)row * N + n0) = __builtin_convertvector(acc, halves<T>);
+            *reinterpret_cast<halves<T> *>(static_cast<uint16_t *>(C) + (size_t)m * N + n0) = __builtin_convertvector(acc, halves<T>);
         }
     };
     if (s >= n_slices) return;
@@ -334,7 +441,7 @@ __global__ __launch_bounds__(1024) void spmm_resident_kernel(const u32x4 *__rest
             halves<T> b[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) e[i] = q[k][i];
-            if (fresh) row = (int)e[0], e[0] = (uint32_t)K, fresh = false;
+            if (fresh) row = e[0], e[0] = (uint32_t)K, fresh = false;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 uint32_t at;
@@ -430,11 +537,12 @@ hipError_t launch_as(const SpmmArgs &a, const ResidentPlan &p, const Launch &l, 
 
 } // namespace
 
-double resident_estimate_us(size_t M, size_t K, size_t N, int64_t nnz)
+double resident_estimate_us(size_t M, size_t K, size_t N, int64_t nnz, bool long_rows)
 {
     ResidentPlan p;
     p.n_slices = (int)((M + 63) / 64);
     p.fours = nnz / 256 + (int64_t)p.n_slices * 3 / 4;
+    if (long_rows) p.fours += nnz / 768, p.longest = PART; // R-MAT scales 12 to 14: a third more
     Launch l;
     return best_columns(p, K, N, &l) ? l.us : 1e30;
 }
@@ -459,48 +567,58 @@ void resident_destroy(ResidentPlan *p)
 {
     if (!p) return;
     if (p->d_list) (void)dev_free(p->d_list);
-    if (p->d_first) (void)dev_free(p->d_first);
+    if (p->d_first) (void)dev_free(p->d_first - IN_FRONT);
     delete p;
 }
 
 hipError_t resident_build(const CompactPlan &c, size_t M, size_t K, int64_t nnz, ResidentPlan **out)
 {
     *out = nullptr;
-    if (c.n_split_rows || c.n_items == 0 || nnz <= 0 || nnz > 0x3fffffff || M > 0x3fffffff || lds_of(K, 2) > MAX_LDS) return hipSuccess;
+    if (c.n_items == 0 || nnz <= 0 || nnz > 0x3fffffff || M + (size_t)nnz / 32 >= PADDED || lds_of(K, 2) > MAX_LDS) return hipSuccess;
     ResidentPlan *p = new (std::nothrow) ResidentPlan();
     if (!p) return hipErrorOutOfMemory;
-    const int n_slices = p->n_slices = (int)((M + 63) / 64);
-    // fours: those of the nonzeros and the rows' numbers, up to one more a slice, and what the longest rows leave the shorter ones of their slice
-    const size_t fours = ((size_t)nnz + 255) / 256 + (size_t)n_slices + (MAX_ROW + 3) / 4 + 1;
+    // A shared row takes a place for every 32 of its nonzeros or fewer.  Fours: those of the nonzeros, one more a slice for the first words, PART / 4 + 1 a
+    // slice of shared rows, and what the longest rows leave the shorter ones of their slice.
+    const size_t most_slices = (M + (size_t)nnz / 32) / 64 + 1;
+    const size_t fours = ((size_t)nnz + 255) / 256 + most_slices + (PART / 4 + 1) * ((size_t)nnz / 2048 + 2) + 1;
     DevScratch tmp;
-    uint32_t *lengths = nullptr, *places = nullptr, *rows_of = nullptr;
-    hipError_t e = tmp.alloc((2 * M + MAX_ROW + 1) * sizeof(uint32_t));
+    uint32_t *places = nullptr;
+    int32_t *lengths = nullptr, *parts = nullptr, *before = nullptr;
+    ResidentTotals *totals = nullptr;
+    hipError_t e = tmp.alloc((2 * M + 16 * (size_t)c.n_slots + 16 * BUILD_WAVES * (size_t)c.n_items) * sizeof(uint32_t));
     if (e == hipSuccess) {
-        rows_of = static_cast<uint32_t *>(tmp.p), lengths = rows_of + MAX_ROW + 1, places = lengths + M;
+        places = static_cast<uint32_t *>(tmp.p), lengths = reinterpret_cast<int32_t *>(places + M), parts = lengths + M, before = parts + 16 * (size_t)c.n_slots;
         e = dev_malloc(&p->d_list, fours * 1024);
     }
-    if (e == hipSuccess) e = dev_malloc(&p->d_first, ((size_t)n_slices + 2) * sizeof(uint32_t));
+    if (e == hipSuccess) e = dev_malloc(&totals, (IN_FRONT + most_slices + 1) * sizeof(uint32_t));
     if (e == hipSuccess) {
-        e = hipMemsetAsync(rows_of, 0, (MAX_ROW + 1) * sizeof(uint32_t), nullptr);
+        p->d_first = reinterpret_cast<uint32_t *>(totals) + IN_FRONT;
+        e = hipMemsetAsync(totals, 0, IN_FRONT * sizeof(uint32_t), nullptr);
     }
-    if (e == hipSuccess) e = hipMemsetD32Async((hipDeviceptr_t)p->d_list, (int)K, fours * 256, nullptr);
-    const unsigned wgs = (unsigned)((c.n_items + BUILD_WAVES - 1) / BUILD_WAVES);
+    // the zeros of lanes that share rows are many: written beforehand
+    const bool long_rows = c.n_split_rows > 0 || nnz > (int64_t)M * (PART / 2);
+    if (e == hipSuccess && long_rows) e = hipMemsetD32Async((hipDeviceptr_t)p->d_list, (int)K, fours * 256, nullptr);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(resident_lengths_kernel, dim3(wgs), dim3(64 * BUILD_WAVES), 0, nullptr, c.d_items, c.n_items, c.d_acol, c.d_entries, c.d_step_range, (int32_t *)lengths, rows_of);
-        hipLaunchKernelGGL(resident_slices_kernel, dim3(1), dim3(1024), 0, nullptr, rows_of, n_slices, p->d_first, p->d_first + n_slices + 1);
-        hipLaunchKernelGGL(resident_places_kernel, dim3((unsigned)((M + 1023) / 1024)), dim3(1024), 0, nullptr, (const int32_t *)lengths, (int)M, rows_of, places);
-        hipLaunchKernelGGL(resident_fill_kernel, dim3(wgs), dim3(64 * BUILD_WAVES), 0, nullptr, c.d_items, c.n_items, c.d_acol, c.d_entries, c.d_step_range, c.d_cols, places, p->d_first,
-                           (int)M, p->d_list);
+        const dim3 items((unsigned)c.n_items), rows((unsigned)((M + 1023) / 1024));
+        hipLaunchKernelGGL(resident_lengths_kernel, items, dim3(64 * BUILD_WAVES), 0, nullptr, c.d_items, c.d_acol, c.d_entries, c.d_step_range, lengths, parts, before, totals);
+        if (c.n_split_rows) hipLaunchKernelGGL(resident_parts_kernel, dim3((unsigned)c.n_split_rows), dim3(64), 0, nullptr, c.d_split, lengths, parts, totals);
+        hipLaunchKernelGGL(resident_slices_kernel, dim3(1), dim3(1024), 0, nullptr, p->d_first, totals);
+        hipLaunchKernelGGL(resident_places_kernel, rows, dim3(1024), 0, nullptr, lengths, (int)M, places, p->d_first, totals, (uint32_t)K, p->d_list);
+        hipLaunchKernelGGL(resident_fill_kernel, items, dim3(64 * BUILD_WAVES), 0, nullptr, c.d_items, c.d_acol, c.d_entries, c.d_step_range, c.d_cols, lengths, parts, before,
+                           places, p->d_first, (uint32_t)K, long_rows, p->d_list);
         e = hipGetLastError();
     }
     for (auto f : {prepare<2, false>, prepare<2, true>, prepare<4, false>, prepare<4, true>, prepare<8, false>, prepare<8, true>})
         if (e == hipSuccess) e = f();
-    uint32_t n[2] = {0, 0};
-    if (e == hipSuccess) e = hipMemcpy(n, p->d_first + n_slices, sizeof n, hipMemcpyDeviceToHost);
+    struct {
+        uint32_t n_slices, fours, longest; // as ResidentTotals begins
+    } n{};
+    if (e == hipSuccess) e = hipMemcpy(&n, totals, sizeof n, hipMemcpyDeviceToHost);
     tmp.idle = e == hipSuccess;
-    p->fours = n[0];
-    p->longest = (int)n[1];
-    if (e != hipSuccess || p->longest >= MAX_ROW) {
+    p->n_slices = (int)n.n_slices;
+    p->fours = n.fours;
+    p->longest = (int)std::min<uint32_t>(n.longest, PART);
+    if (e != hipSuccess || n.longest > MAX_ROW) {
         (void)hipDeviceSynchronize();
         resident_destroy(p);
         return e;

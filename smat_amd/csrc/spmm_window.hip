@@ -686,7 +686,7 @@ hipError_t window_widths(const int32_t *row_ptr, const int32_t *col_idx, size_t 
     if (e != hipSuccess) return e;
     e = hipMemsetAsync(*slots, 0, sizeof out, nullptr);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(window_count_kernel, dim3((unsigned)std::min<size_t>((mb + SIZES[0] - 1) / SIZES[0], 512), WINDOW_SIZES), dim3(256), (size_t)words * 4, nullptr, row_ptr, col_idx,
+        hipLaunchKernelGGL(window_count_kernel, dim3((unsigned)std::min<size_t>((mb + SIZES[0] - 1) / SIZES[0], 256), WINDOW_SIZES), dim3(256), (size_t)words * 4, nullptr, row_ptr, col_idx,
                            (int)mb, words, (WindowWidths *)*slots);
         e = hipGetLastError();
     }
@@ -739,7 +739,7 @@ double window_choose(const WindowWidths &widths, const WindowProduct &w, int *si
 }
 
 hipError_t window_build(const WindowWidths &w, int size, void *slots, const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, int most_blocks,
-                        WindowPlan **out)
+                        bool wait, WindowPlan **out)
 {
     *out = nullptr;
     WindowPlan *p = new (std::nothrow) WindowPlan();
@@ -763,7 +763,7 @@ hipError_t window_build(const WindowWidths &w, int size, void *slots, const int3
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = prepare_all<false>();
-    if (e == hipSuccess) e = hipStreamSynchronize(nullptr); // launches on other streams read the lists
+    if (e == hipSuccess && wait) e = hipStreamSynchronize(nullptr); // launches on other streams read the lists
     if (e != hipSuccess) {
         window_destroy(p);
         return e;
@@ -795,6 +795,7 @@ hipError_t window_attach_entries(WindowPlan &p, const uint16_t *vals, const int3
     }
     if (e == hipSuccess) e = prepare_all<true>();
     if (e == hipSuccess) e = hipMemcpy(&too_many, most.p, sizeof too_many, hipMemcpyDeviceToHost);
+    most.idle = e == hipSuccess;
     *taken = e == hipSuccess && too_many == 0;
     return e;
 }

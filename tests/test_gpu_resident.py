@@ -68,7 +68,7 @@ def test_resident_columns_match_the_oracle(smat, cuda, oracle, force, M, K, colu
     plan.close()
 
 
-@pytest.mark.parametrize("longest,taken", [(2046, 1), (2047, 0)])
+@pytest.mark.parametrize("longest,taken", [(4096, 1), (4097, 0)])
 def test_rows_longer_than_a_list_stay_with_the_compact_kernel(smat, cuda, force, longest, taken):
     import torch
     M, K, N = 1040, 32768, 1000
@@ -90,6 +90,28 @@ def test_rows_longer_than_a_list_stay_with_the_compact_kernel(smat, cuda, force,
             full[16 * i:16 * i + 16, A.col_idx[q]:A.col_idx[q] + 16] = blocks[q]
     want = torch.from_numpy(full).to(cuda) @ torch.from_numpy(B.astype(np.float32).reshape(N, K)).to(cuda).T.contiguous()  # whole numbers: exact
     assert torch.equal(C, want)
+    plan.close()
+
+
+# rows shared by 2, 4, 8 and 64 lanes, at the borders between them, in block rows that the compact kernel's list splits and in ones that it leaves whole
+@pytest.mark.parametrize("heavy", [[65], [64, 65, 128, 129, 255, 257], [2049, 4000, 66, 1024]])
+@pytest.mark.parametrize("columns,shares,N", [(2, 1, 24), (4, 3, 40), (8, 1, 8)])
+def test_long_rows_are_shared_by_lanes(smat, cuda, oracle, force, heavy, columns, shares, N):
+    import torch
+    M, K = 1616, 10224
+    lengths = np.random.default_rng(len(heavy)).choice([0, 1, 3, 9], M)
+    lengths[20:20 + 17 * len(heavy):17] = heavy  # one in a block row
+    A = scattered(smat, lengths, K, seed=heavy[0])
+    B = np.random.default_rng(N).integers(-2, 3, K * N).astype(np.float16).view(np.uint16)
+    d = [to_dev(torch, x, cuda) for x in (A.val, A.row_ptr, A.col_idx, B)]
+    want = oracle.spmm_bcsr(M, N, K, A.row_ptr, A.col_idx, A.val, B, threads=8)
+    force(columns, shares)
+    plan = plan_of(smat, A, d, N)
+    assert plan.info()["kernel"] == smat.KERNEL_COMPACT and smat.lib.smat_internal_plan_resident(plan.handle) == 1
+    for c_f32 in (False, True):
+        C = torch.full((M, N), float("nan"), dtype=torch.float32 if c_f32 else torch.float16, device=cuda)
+        smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, len(A.col_idx), plan=plan, c_f32=c_f32)
+        assert np.array_equal(C.cpu().numpy().astype(np.float32), want.astype(np.float32 if c_f32 else np.float16).astype(np.float32))
     plan.close()
 
 
