@@ -240,3 +240,40 @@ def test_plans_for_the_sweep_kernel_may_multiply_from_windows(smat, cuda, oracle
                 smat.spmm(t[0], t[1], t[2], t[3][:A.K * n], C, A.M, n, A.K, nnzb, plan=plan, kernel=kernel)
                 assert np.array_equal(C.cpu().numpy(), want[:, :n])
     plan.close()
+
+
+@pytest.mark.parametrize("kind", ["blocks", "nonzeros", "columns"])
+def test_block_columns_in_any_order_and_twice(smat, cuda, oracle, force, kind):
+    """A block row whose columns do not ascend, some of them listed twice: windows of whole blocks, of listed nonzeros, and columns of B in LDS."""
+    import torch
+    rp, ci, vals = local_matrix(45, 50, 10, seed=31)
+    rng = np.random.default_rng(5)
+    for i in range(45):
+        row = ci[rp[i]:rp[i + 1]]
+        rng.shuffle(row)
+        if len(row) > 2:
+            row[1] = row[0]
+    M, K, N, nnzb = 720, 800, 72, len(ci)
+    if kind != "blocks":
+        vals = sparse_values(nnzb, 3, 4)
+    B = whole_b(K, N, seed=3)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci, B)]
+    want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B, threads=4).astype(np.float16)
+    smat.lib.smat_internal_resident_force.argtypes = [ctypes.c_int, ctypes.c_int]
+    try:
+        force(*((-1, 0) if kind == "columns" else (8, 2)))
+        smat.lib.smat_internal_resident_force(4 if kind == "columns" else -1, 0)
+        plan = smat.Plan(rp, M, K, nnzb, N, col_idx_host=ci)
+        plan.attach_values(*d[:3])
+        assert (smat.lib.smat_internal_plan_window_rows(plan.handle), smat.lib.smat_internal_plan_resident(plan.handle)) == ((0, 1) if kind == "columns" else (8, 0))
+        C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+        smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, nnzb, plan=plan)
+        assert np.array_equal(C.cpu().numpy(), want)
+        plan.close()
+        if kind == "blocks":
+            smat.lib.smat_plan_cache_clear()
+            C.fill_(float("nan"))
+            smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, nnzb, drop_in=True)
+            assert np.array_equal(C.cpu().numpy(), want)
+    finally:
+        smat.lib.smat_internal_resident_force(0, 0)
