@@ -801,12 +801,15 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     const bool most_of_b = size >= 0 && !census && other_us < 1e30 && (double)widths.sum[size] > 0.5 * (double)kb * (double)mb / (4 << size);
     if (size < 0 || (!window_forced() && (us >= bar || most_of_b))) return slots ? dev_free(slots) : hipSuccess;
     hipError_t e = window_build(widths, size, slots, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, !census, &p.window);
+    if (e == hipSuccess && !census) window_settle(*p.window, p.M, p.K, p.n_cap, p.nnzb);
     if (e != hipSuccess || !census) return e;
     bool taken;
     e = window_attach_entries(*p.window, vals, row_ptr, (const unsigned long long *)census->offset.p, mb, p.nnzb, census->nnz, &taken);
     if (e != hipSuccess || !taken) {
         window_destroy(p.window);
         p.window = nullptr;
+    } else {
+        window_settle(*p.window, p.M, p.K, p.n_cap, p.nnzb);
     }
     return e;
 }

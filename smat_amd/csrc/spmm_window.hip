@@ -815,6 +815,17 @@ static WindowProduct product_of(const SpmmArgs &a, const WindowPlan &p)
 {
     return WindowProduct{a.M, a.K, a.N, a.nnzb, p.nnz, p.most_blocks, a.c_f32};
 }
+void window_settle(WindowPlan &p, size_t M, size_t K, size_t N, size_t nnzb)
+{
+    p.n = N;
+    for (bool c_f32 : {false, true}) {
+        double us;
+        const int tiles = best_tiles(p, WindowProduct{M, K, N, nnzb, p.nnz, p.most_blocks, c_f32}, &us);
+        if (!tiles || !fits(p.rows, p.cap, tiles, p.d_entries != nullptr)) continue;
+        const Launch l = launch_of(p.rows, p.cap, tiles, p.n_groups, N, p.d_entries != nullptr);
+        p.own[c_f32] = {tiles, l.n_panels, l.panels_per_unit, l.workgroups};
+    }
+}
 double window_launch_us(const SpmmArgs &a, const WindowPlan &p)
 {
     double us;
@@ -824,11 +835,16 @@ double window_launch_us(const SpmmArgs &a, const WindowPlan &p)
 
 hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st)
 {
-    double us;
-    const int tiles = best_tiles(p, product_of(a, p), &us);
     const bool entries = p.d_entries != nullptr;
-    if (tiles == 0 || !fits(p.rows, p.cap, tiles, entries)) return hipErrorInvalidValue;
-    const Launch l = launch_of(p.rows, p.cap, tiles, p.n_groups, a.N, entries);
+    const auto &own = p.own[a.c_f32];
+    int tiles = own.tiles;
+    Launch l{own.n_panels, own.panels_per_unit, own.workgroups, 0};
+    if (a.N != p.n || !tiles || g_force_tiles) {
+        double us;
+        tiles = best_tiles(p, product_of(a, p), &us);
+        if (tiles == 0 || !fits(p.rows, p.cap, tiles, entries)) return hipErrorInvalidValue;
+        l = launch_of(p.rows, p.cap, tiles, p.n_groups, a.N, entries);
+    }
     auto as = [&](auto tn, auto parts) {
         constexpr int TN = decltype(tn)::value, PARTS = decltype(parts)::value;
         if (entries) return a.c_f32 ? launch_as<TN, PARTS, true, true>(a, p, l, st) : launch_as<TN, PARTS, false, true>(a, p, l, st);
