@@ -216,7 +216,8 @@ static double compact_estimate_us(double cols, double list_bytes, size_t M, size
 }
 static double compact_estimate_us(const CompactPlan &c, size_t M, size_t K, size_t N)
 {
-    return compact_estimate_us((double)c.n_cols, c.d_acol ? 36.0 * (double)c.n_cols : 4.25 * (double)c.n_cols + 4.0 * (double)c.n_entries, M, K, N);
+    // 3 us where the parts of split rows are added up (R-MAT scales 12 to 15)
+    return compact_estimate_us((double)c.n_cols, c.d_acol ? 36.0 * (double)c.n_cols : 4.25 * (double)c.n_cols + 4.0 * (double)c.n_entries, M, K, N) + (c.n_split_rows ? 3.0 : 0.0);
 }
 static size_t sweep_listed_chunks(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t group_rows)
 {
