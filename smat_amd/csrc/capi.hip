@@ -772,7 +772,9 @@ static hipError_t sweep_small_groups(smat_plan &p, size_t group_rows)
 // -> windows, us: 27-point stencil 64^3, N = 64 90 -> 56, 48^3, N = 256 111 -> 59, 48 x 25 x 48, N = 56 20.4 -> 12.7; bands of
 // 14224 rows and 182, N = 544 33 -> 17, of 65536 and 20, N = 256 30 -> 15, of 8960 and 120, N = 48 7.4 -> 5.
 // census: of the values, where the compact kernel would multiply: the window kernel then multiplies what it would, the values as attached.
-static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us, const uint16_t *vals, const CompactCensus *census)
+// wait: for the lists, which launches on other streams than the default one may read.
+static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us, const uint16_t *vals, const CompactCensus *census,
+                              bool wait = true)
 {
     const size_t mb = p.M / 16, kb = p.K / 16;
     if ((p.kernel != SMAT_KERNEL_ROWWISE && !(p.kernel == SMAT_KERNEL_SWEEP && p.sweep_few_tiles)) || p.kernel_requested != SMAT_KERNEL_AUTO || p.n_split_rows || !window_takes_rows(p.max_item_blocks)) return hipSuccess;
@@ -801,7 +803,7 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     // N = 552 7.9 -> 8.7 us).
     const bool most_of_b = size >= 0 && !census && other_us < 1e30 && (double)widths.sum[size] > 0.5 * (double)kb * (double)mb / (4 << size);
     if (size < 0 || (!window_forced() && (us >= bar || most_of_b))) return slots ? dev_free(slots) : hipSuccess;
-    hipError_t e = window_build(widths, size, slots, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, !census, &p.window);
+    hipError_t e = window_build(widths, size, slots, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, wait && !census, &p.window);
     if (e == hipSuccess && !census) window_settle(*p.window, p.M, p.K, p.n_cap, p.nnzb);
     if (e != hipSuccess || !census) return e;
     bool taken;
@@ -815,14 +817,17 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     return e;
 }
 // No memory for the windows is not an error of the plan.
-static hipError_t take_window_if_room(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us, const uint16_t *vals, const CompactCensus *census)
+static hipError_t take_window_if_room(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us, const uint16_t *vals, const CompactCensus *census,
+                                      bool wait = true)
 {
-    const hipError_t e = take_window(p, row_ptr, col_idx, other_us, vals, census);
+    const hipError_t e = take_window(p, row_ptr, col_idx, other_us, vals, census, wait);
     if (e != hipErrorOutOfMemory) return e;
     (void)hipGetLastError();
     return hipSuccess;
 }
-hipError_t smat::plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx) { return take_window_if_room(*p, row_ptr, col_idx, 1e30, nullptr, nullptr); }
+hipError_t smat::plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx) {
+    return take_window_if_room(*p, row_ptr, col_idx, 1e30, nullptr, nullptr, false); // a plan of the cache, which launches on the default stream alone
+}
 
 static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, const int32_t *row_ptr,
                                         const int32_t *col_idx, const int32_t *row_ptr_host)
