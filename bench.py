@@ -408,6 +408,11 @@ def main():
     kernel_id = (plan.info()["kernel"] if plan is not None else 1) if args.kernel == 0 else args.kernel
     if kernel_id == 4:
         kernel_id = 1
+    if plan is not None and args.kernel == 0 and not args.b_row_major:  # what such launches take in place of the plan's kernel
+        if smat_amd.lib.smat_internal_plan_window_rows(plan.handle):
+            kernel_id = "window"
+        elif smat_amd.lib.smat_internal_plan_resident(plan.handle):
+            kernel_id = "resident"
     prof = profiled(args.workload, kernel_id)
     roof["traffic"] = prof.get("traffic_bytes_per_launch")
     if prof:
