@@ -201,7 +201,7 @@ int smat_plan_info(const smat_plan *plan, int64_t *info);
  * block together with a block of zeros and no others (a complete pair under an Inf in B gives what a
  * block-by-block product gives), the compact kernel pads a block row with zero columns and may list a column with many
  * nonzeros several times, each time with a part of them and zeros (0 x Inf = NaN where B holds Inf or NaN); windows of listed nonzeros multiply the
- * blocks whole, columns in LDS the nonzeros alone.  The sweep kernel multiplies an unpaired block together with
+ * halves of blocks (8 columns) that hold any, columns in LDS the nonzeros alone.  The sweep kernel multiplies an unpaired block together with
  * a neighbouring block of the SAME block row and 16 rows of zeros in place of B, and its filler ops multiply two
  * blocks of the block row they add to by zeros: an Inf or NaN in vals stays in its own block row of C (where a
  * block-by-block product, mmaCBT.cu:44-66, has an Inf or NaN as well).  Only a block that is alone in its block

@@ -8,7 +8,8 @@
 //    are; the columns of every window in ascending order, and for every block its place in its window.
 //  * spmm_window_kernel: below.
 //
-// The order of the sums is that of the row-wise kernel (blocks of a row two by two from its first), the results have the same bits.
+// The order of the sums is that of the row-wise kernel (blocks of a row two by two from its first), the results have the same bits; with listed
+// nonzeros the halves of blocks without one are left out (window_entries_kernel).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -32,15 +33,18 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int COPIES = 7;               // KiB of a window that a wavefront copies at a time
 constexpr int SLOT_BITS = 10;           // of a block's entry: its place in the window; above them its block column
 constexpr int BITMAP_WORDS = 8192;      // block columns of the matrix / 32
+constexpr int MAX_LISTED = 128;         // block columns of a window with listed nonzeros: octets are named in 8 bits
 constexpr size_t MAX_LDS = 160 * 1024;  // of a compute unit
 constexpr int CU_WAVES = 16;            // wavefronts of 128 registers on a compute unit
 constexpr int SIZES[WINDOW_SIZES] = {4, 8, 16}; // block rows of a group
 // block pairs of a row that a wavefront holds
 constexpr int MAX_PAIRS = 17;
 template <int TN> constexpr int pairs_held = TN == 4 ? 12 : MAX_PAIRS;
-// Listed nonzeros become operands a round of so many pairs at a time.
+// Listed nonzeros become operands a round of so many steps at a time (three: 3 to 7 % slower where every octet holds some).
 constexpr int ROUND = 4, MAX_ROUNDS = (MAX_PAIRS + ROUND - 1) / ROUND;
+static_assert(ROUND % 2 == 0, "the product takes two steps at a time: behind an odd number the next one of its round, zeros");
 constexpr int LIST_BITS = 26; // of a round's list: the fours of entries before it; above them its own fours
+constexpr uint32_t MAX_LIST = 4 * ((1u << (32 - LIST_BITS)) - 1); // entries of a round: four a lane
 
 // ---- which block columns a group uses ----
 
@@ -127,60 +131,110 @@ __global__ __launch_bounds__(256) void window_list_kernel(const int32_t *__restr
     }
 }
 
-// The nonzeros of the blocks, ROUND pairs of a block row after the other: value << 16 | byte in the MFMA operands of the round, which lie
-// rows KiB apart, filled up to a multiple of four with the last one.  table: MAX_PAIRS words twice a block row, the places of the two blocks of
-// pair j in the window (16 bits each) and the list of round j, the fours of entries before it and its own << LIST_BITS; behind the table the blocks of
-// every row.  A wavefront takes a block row; offset[p]: nonzeros before block p in the upper half.  Bound by the read of the values.
+// The nonzeros of the blocks.  Unit: an octet, 8 neighbouring columns of a block; the product multiplies four of them a step, and those without a
+// nonzero are left out, a third of a 27-point stencil's (64^3, N = 64 36.0 -> 32.2 us).  ROUND steps of a block row after the other:
+// value << 16 | byte in the MFMA operands of the round, which lie rows KiB apart, filled up to a multiple of four with the last one.  A round
+// ends early where the next pair of blocks does not fit its list.  table: MAX_PAIRS pairs of words a block row, the places of the four octets of step j
+// in the window (8 bits each, in octets; of those that are none that of the row's first, which meets zeros) and the list of round j, the fours of
+// entries before it and its own << LIST_BITS; behind the table twice the steps of every row.  A wavefront takes a block
+// row; offset[p]: nonzeros before block p in the upper half.  Bound by the read of the values.
 __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr,
-                                                             const uint32_t *__restrict__ slot, const unsigned long long *__restrict__ offset, int mb, int rows,
+                                                             const uint32_t *__restrict__ slot, const unsigned long long *__restrict__ offset, int mb, int rows, int held,
                                                              uint32_t *__restrict__ entries, uint32_t *__restrict__ table, uint32_t *__restrict__ most)
 {
     const int lane = threadIdx.x & 63, br = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (br >= mb) return;
     const int p0 = row_ptr[br], blocks = row_ptr[br + 1] - p0;
-    const int sel = lane >> 5, at = (lane & 15) * 16 + ((lane >> 4) & 1) * 8;
-    if (lane == 0) table[(long)mb * (2 * MAX_PAIRS) + br] = (uint32_t)blocks;
+    const int g = lane >> 4, sel = g >> 1, at = (lane & 15) * 16 + (g & 1) * 8; // octet g of two blocks
     auto load = [&](int d) {
         const int b = 2 * d + sel;
         return b < blocks ? *reinterpret_cast<const u32x4 *>(vals + (long)(p0 + b) * 256 + at) : (u32x4){0u, 0u, 0u, 0u};
     };
     u32x4 w = load(0);
-    uint32_t longest = 0, first = 0, n = 0, last = 0, places = 0, list = 0; // places, list: of pair and round `lane`
+    uint32_t first = blocks > 0 ? ((uint32_t)(offset[p0] >> 32) + 8u * (uint32_t)((p0 + br + 1) / 2)) & ~3u : 0; // of the round
+    uint32_t octets = 0, n = 0, last = 0, longest = 0;   // of the row; entries of the round, the last one; of the longest round
+    uint32_t places = 0, list = 0, first_place = 0;       // places, list: of step and round `lane`
+    auto close = [&](uint32_t round) {                    // fills the round up; the next one begins behind it
+        const uint32_t end = (n + 3u) & ~3u;
+        if (n + lane < end) entries[first + n + lane] = last;
+        if (lane == (int)round) list = first / 4 | min(end, MAX_LIST) / 4 << LIST_BITS;
+        longest = max(longest, end);
+        first += end;
+    };
+    auto fill = [&](uint32_t from, uint32_t to) { // octets that are none
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if ((uint32_t)(lane * 4 + i) >= from && (uint32_t)(lane * 4 + i) < to) places |= first_place << (8 * i);
+    };
     for (int d = 0; 2 * d < blocks; d++) {
         const u32x4 now = w;
         w = load(d + 1);
-        if (d % ROUND == 0) first = ((uint32_t)(offset[p0 + 2 * d] >> 32) + 8u * (uint32_t)((p0 + br + 1) / 2 + d)) & ~3u, n = 0;
-        uint32_t i = n, bits = 0; // nonzeros of the round before those of this lane
+        const int b = min(2 * d + sel, blocks - 1);
+        const uint32_t place = (slot[p0 + b] & ((1u << SLOT_BITS) - 1u)) * 2u + (uint32_t)(g & 1);
+        uint32_t bits = 0, before = 0, all = 0; // entries of the lanes before this one, and of all
+        unsigned long long has_k[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) { // -0.0 is a zero
             const bool has = (now[k / 2] >> (k & 1 ? 16 : 0) & 0x7fffu) != 0;
             bits |= (uint32_t)has << k;
-            const unsigned long long all = __ballot(has);
-            n += __popcll(all);
-            i += __popcll(all & ((1ull << lane) - 1ull));
+            has_k[k] = __ballot(has);
+            all += __popcll(has_k[k]);
+            before += __popcll(has_k[k] & ((1ull << lane) - 1ull));
         }
-        uint32_t e = 0;
+        const unsigned long long some = __ballot(bits != 0);
+        uint32_t used = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) used |= (uint32_t)((some >> (16 * i) & 0xffffu) != 0) << i;
+        uint32_t round = octets / (4 * ROUND), o = octets + __popc(used & ((1u << g) - 1u)), n_in = 0;
+        bool now_in = o / (4 * ROUND) == round; // else in the next one
+        unsigned long long in = __ballot(bits != 0 && now_in);
+#pragma unroll
+        for (int k = 0; k < 8; k++) n_in += __popcll(has_k[k] & in);
+        if (n > 0 && n + n_in > MAX_LIST) { // all in the next one
+            close(round);
+            round++;
+            fill(octets, round * (4 * ROUND));
+            o += round * (4 * ROUND) - octets;
+            octets = round * (4 * ROUND);
+            now_in = true;
+            in = some;
+            n = 0;
+            n_in = all;
+        }
+        const uint32_t next = (first + n + n_in + 3u) & ~3u;
+        uint32_t i = now_in ? first + n + before : next + before - n_in, e = 0;
 #pragma unroll
         for (int k = 0; k < 8; k++)
             if (bits >> k & 1) {
-                e = (now[k / 2] >> (k & 1 ? 16 : 0)) << 16 | (uint32_t)(d % ROUND * rows * 1024 + lane * 16 + k * 2);
-                entries[first + i++] = e;
+                e = (now[k / 2] >> (k & 1 ? 16 : 0)) << 16 | (o / 4 % ROUND * (uint32_t)rows * 1024u + (o & 3u) * 256u + (uint32_t)(lane & 15) * 16u + (uint32_t)k * 2u);
+                entries[i++] = e;
             }
-        const unsigned long long some = __ballot(bits != 0);
-        if (some) last = __shfl(e, 63 - __clzll((long long)some));
-        const uint32_t end = (n + 3u) & ~3u;
-        if (d % ROUND == ROUND - 1 || 2 * d + 2 >= blocks) {
-            if (n + lane < end) entries[first + n + lane] = last;
-            if (lane == d / ROUND) list = first / 4 | min(end / 4, (1u << (32 - LIST_BITS)) - 1u) << LIST_BITS;
-            longest = max(longest, end);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t of = __shfl(place, 16 * i), at = octets + __popc(used & ((1u << i) - 1u));
+            if (used >> i & 1) {
+                if (at == 0) first_place = of;
+                if (lane == (int)(at / 4)) places |= of << (8 * (at & 3));
+            }
         }
-        const int b = p0 + 2 * d;
-        const uint32_t s0 = slot[b] & ((1u << SLOT_BITS) - 1u), s1 = 2 * d + 1 < blocks ? slot[b + 1] & ((1u << SLOT_BITS) - 1u) : s0;
-        if (lane == d) places = s0 | s1 << 16;
+        octets += __popc(used);
+        n += n_in;
+        if (in) last = __shfl(e, 63 - __clzll((long long)in));
+        if (octets / (4 * ROUND) != round) {
+            close(round);
+            n = all - n_in;
+            if (n) last = __shfl(e, 63 - __clzll((long long)some));
+        }
     }
+    if (octets % (4 * ROUND)) close(octets / (4 * ROUND));
     uint32_t *const to = table + (long)br * (2 * MAX_PAIRS);
+    fill(octets, ~0u);
     if (lane < MAX_PAIRS) to[2 * lane] = places, to[2 * lane + 1] = list;
-    if (lane == 0 && longest > 4 * ((1u << (32 - LIST_BITS)) - 1)) atomicMax(most, longest); // too many for a round
+    if (lane == 0) {
+        const uint32_t steps = min((octets + 3) / 4, (uint32_t)MAX_PAIRS);
+        table[(long)mb * (2 * MAX_PAIRS) + br] = 2 * steps;
+        if (longest > MAX_LIST || steps > (uint32_t)held || octets > 4 * MAX_PAIRS) atomicMax(most, max(longest, 1u)); // not for the windows
+    }
 }
 
 // ---- the product ----
@@ -245,17 +299,17 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
     // The block row of a wavefront in a group: what is asked for, and what is made of it.
     struct Asked {
         int p0, blocks;
-        uint32_t q0, q1, c0, c1; // lane j: blocks 2 j and 2 j + 1; ENTRIES: their places in q0, the list of round j in q1
+        uint32_t q0, q1, c0, c1; // lane j: blocks 2 j and 2 j + 1; ENTRIES: the places of step j in q0, the list of round j in q1
     };
     struct Row {
-        int p0, blocks;  // blocks: 0 where the wavefront has none
-        uint32_t packed; // lane j: places of blocks 2 j and 2 j + 1 in the window, in 32 bytes
+        int p0, blocks;  // blocks: 0 where the wavefront has none; ENTRIES: twice the steps
+        uint32_t packed; // lane j: places of blocks 2 j and 2 j + 1 in the window, in 32 bytes; ENTRIES: of the octets of step j, 8 bits each
         bool known;
     };
     uint32_t list = 0; // ENTRIES: of the row taken last, lane j: the list of round j
     auto ask_row = [&](int gr, Asked &r) {
         const int br = gr * rows + wave, b = br < mb ? br : mb - 1;
-        if constexpr (ENTRIES) { // a table of MAX_PAIRS pairs a block row, and the blocks of every row behind it
+        if constexpr (ENTRIES) { // a table of MAX_PAIRS pairs a block row, and twice the steps of every row behind it
             r.p0 = 0;
             r.blocks = br < mb ? __builtin_amdgcn_readfirstlane(row_ptr[b]) : 0;
             const uint32_t at = (uint32_t)min(lane_here(), MAX_PAIRS - 1) * 8u;
@@ -278,7 +332,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
         if constexpr (ENTRIES) {
             asm volatile("" : "+v"(r.q0), "+v"(r.q1));
             list = r.q1;
-            return Row{0, r.blocks, place(r.q0 & 0xffffu) | place(r.q0 >> 16) << 16, true};
+            return Row{0, r.blocks, r.q0, true};
         }
         asm volatile("" : "+v"(r.q0), "+v"(r.q1), "+v"(r.c0), "+v"(r.c1));
         const bool same = (r.q0 >> SLOT_BITS) * 16u == r.c0 && (r.q1 >> SLOT_BITS) * 16u == r.c1;
@@ -403,8 +457,8 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
     };
 
     const uint32_t c0 = (uint32_t)ncol_of<TN>(0, i16); // tile t: 4 t columns on
-    const uint32_t at = c0 * 128u + (((uint32_t)kh ^ swizzle(c0)) * 16u);
-    const uint32_t half = (uint32_t)sel * 16;
+    const uint32_t at = ENTRIES ? swizzle(c0) * 16u : c0 * 128u + (((uint32_t)kh ^ swizzle(c0)) * 16u);
+    const uint32_t half = ENTRIES ? (uint32_t)g * 8 : (uint32_t)sel * 16; // of what readlane brings, the lane's first bit
     const f16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
     f32x4 acc[TILES];
     Row row, next;
@@ -433,7 +487,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
             }
         }
         const int blocks = row.known ? row.blocks : 0;
-        const uint32_t b_at = lbase + buf;
+        const uint32_t b_at = lbase + buf + (ENTRIES ? c0 * 128u : 0u);
 #pragma unroll
         for (int d0 = 0; d0 < NP; d0 += U) { // the operands of U pairs at a time
             if (2 * d0 < blocks) {
@@ -441,12 +495,18 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
 #pragma unroll
                 for (int u = 0; u < U; u++) {
                     if (d0 + u >= NP) continue;
-                    const uint32_t v = __builtin_amdgcn_ubfe((uint32_t)__builtin_amdgcn_readlane((int)row.packed, d0 + u), half, 16);
-                    const uint32_t b = ((v << 5) ^ at) + b_at;
+                    const uint32_t four = (uint32_t)__builtin_amdgcn_readlane((int)row.packed, d0 + u);
+                    uint32_t b;
+                    if constexpr (ENTRIES) { // octets lie in 16 bytes, 8 to a quad
+                        b = ((__builtin_amdgcn_ubfe(four, half, 8) << 4) ^ at) + b_at;
+                        b += __umul24(__builtin_amdgcn_ubfe(four, half + 3, 5), (uint32_t)QUAD_BYTES - 128u);
+                    } else {
+                        b = ((__builtin_amdgcn_ubfe(four, half, 16) << 5) ^ at) + b_at;
+                    }
 #pragma unroll
                     for (int t = 0; t < TN; t++) bv[u][t] = *(const __attribute__((address_space(3))) f16x8 *)(uintptr_t)(b + t * 512);
                 }
-                if (2 * (d0 + U) > blocks) { // what is past the end of the row: zeros times zeros
+                if (!ENTRIES && 2 * (d0 + U) > blocks) { // what is past the end of the row: zeros times zeros
                     const int sel = lane_here() >> 5;
 #pragma unroll
                     for (int u = 0; u < U; u++)
@@ -573,7 +633,7 @@ size_t lds_of(int rows, int cap, int tiles, bool entries) { return 2 * std::max(
 // Whether windows of `cap` block columns fit: twice in LDS, and COPIES KiB a wavefront.
 bool fits(int rows, int cap, int tiles, bool entries)
 {
-    return cap < 1 << SLOT_BITS && rows % (2 * tiles) == 0 && (size_t)cap * tiles * 512 <= (size_t)COPIES * 1024 * rows &&
+    return (entries ? cap <= MAX_LISTED : cap < 1 << SLOT_BITS) && rows % (2 * tiles) == 0 && (size_t)cap * tiles * 512 <= (size_t)COPIES * 1024 * rows &&
            lds_of(rows, cap, tiles, entries) <= MAX_LDS;
 }
 // Parts of a panel: two where N is wider than one.
@@ -776,6 +836,7 @@ hipError_t window_attach_entries(WindowPlan &p, const uint16_t *vals, const int3
                                  bool *taken)
 {
     *taken = false;
+    if (p.cap > MAX_LISTED) return hipSuccess;
     const size_t room = (size_t)nnz + 8 * ((nnzb + mb + 1) / 2 + MAX_PAIRS) + 16;
     if (room / 4 >= (size_t)1 << LIST_BITS) return hipSuccess;
     const size_t table = mb * (2 * MAX_PAIRS + 1);
@@ -789,7 +850,8 @@ hipError_t window_attach_entries(WindowPlan &p, const uint16_t *vals, const int3
     e = most.alloc(sizeof too_many);
     if (e == hipSuccess) e = hipMemsetAsync(most.p, 0, sizeof too_many, nullptr);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(window_entries_kernel, dim3((unsigned)((mb + 3) / 4)), dim3(256), 0, nullptr, vals, row_ptr, p.d_slot, offset, (int)mb, p.rows, p.d_entries, p.d_table,
+        hipLaunchKernelGGL(window_entries_kernel, dim3((unsigned)((mb + 3) / 4)), dim3(256), 0, nullptr, vals, row_ptr, p.d_slot, offset, (int)mb, p.rows,
+                           p.most_blocks <= 2 * pairs_held<4> ? pairs_held<4> : MAX_PAIRS, p.d_entries, p.d_table,
                            (uint32_t *)most.p);
         e = hipGetLastError();
     }

@@ -277,3 +277,41 @@ def test_block_columns_in_any_order_and_twice(smat, cuda, oracle, force, kind):
             assert np.array_equal(C.cpu().numpy(), want)
     finally:
         smat.lib.smat_internal_resident_force(0, 0)
+
+
+# (nonzeros per octet of 8 columns, those of even and of odd ones): 16 octets a round and 252 nonzeros in its list are the edges
+@pytest.mark.parametrize("width", [1, 3, 7, 12, 15, 16, 17, 24])
+@pytest.mark.parametrize("octets", [(5, 0), (0, 3), (15, 0), (16, 0), (21, 0), (60, 0), (23, 20), (1, 1)])
+def test_octets_without_a_nonzero_are_left_out(smat, cuda, oracle, force, width, octets):
+    """Rounds that are full to the last place, end early and hold one octet; B is infinite where no octet holds a nonzero, places of none included."""
+    import torch
+    rng = np.random.default_rng(width)
+    mb, kb, N = 40, 40, 40
+    rp, ci, _ = local_matrix(mb, kb, width, seed=width, empty=(5,))
+    M, K, nnzb = mb * 16, kb * 16, len(ci)
+    vals = np.zeros((nnzb, 16, 2, 8), np.float16)  # row, octet, column
+    for b in vals:
+        for h, n in enumerate(octets):
+            for at in rng.choice(64, n, replace=False):
+                b[at // 4, h, at % 4 * 2 + h] = rng.choice([-2, -1, 1, 2])
+    vals = vals.reshape(-1).view(np.uint16)
+    B = whole_b(K, N, seed=3).view(np.float16).reshape(N, kb, 2, 8).copy()
+    for h, n in enumerate(octets):
+        if n == 0:
+            B[:, :, h] = 0
+    want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B.reshape(-1).view(np.uint16), threads=4).astype(np.float16)
+    for h, n in enumerate(octets):
+        if n == 0:
+            B[:, :, h] = np.inf
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci, B.reshape(-1).view(np.uint16))]
+    for rows, tiles in ((4, 1), (8, 2), (16, 4)):
+        force(rows, tiles)
+        plan = smat.Plan(rp, M, K, nnzb, N, col_idx_host=ci)
+        plan.attach_values(d[0], d[1], d[2])
+        if plan.info()["kernel"] == smat.KERNEL_COMPACT and smat.lib.smat_internal_plan_window_rows(plan.handle) == rows:
+            C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+            smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, nnzb, plan=plan)
+            assert np.array_equal(C.cpu().numpy(), want)
+        else:
+            assert max(octets) > 22  # more rounds than a wavefront holds
+        plan.close()
