@@ -239,6 +239,16 @@ __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__r
 
 // ---- the product ----
 
+// Column c < 16 TN of a part's copy lies so many columns behind the panel's first, n0 < N.  Past N, where nothing is stored, the panel's first stands
+// in: a whole part may lie past N (panels of two tiles and two parts, N % 64 = 8), so its own first column need not be one of B.
+template <int TN, int PARTS>
+__host__ __device__ __forceinline__ int copied_column(int n0, int part, int c, int N)
+{
+    constexpr int P = 16 * TN, PANEL = P * PARTS;
+    const int col = part * (P / 4) + c / (P / 4) * (PANEL / 4) + c % (P / 4);
+    return n0 + col < N ? col : 0;
+}
+
 // Waits until at most n of the wavefront's vector memory operations are under way (they end in order), or a few less.
 __device__ __forceinline__ void wait_vector_memory(int n)
 {
@@ -436,12 +446,11 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
     };
     // a part's columns of the window to LDS; returns the instructions
     auto stage = [&](int pan, int part, uint32_t dst) {
-        const int n0 = pan * PANEL + part * (P / 4);
+        const int n0 = pan * PANEL;
         const uint64_t base = (uint64_t)(uintptr_t)(B + (long)n0 * K);
         const int lane = lane_here();
-        const uint32_t c = copy_col(lane), col = c / (P / 4) * (PANEL / 4) + c % (P / 4);
-        const uint32_t from = (n0 + (int)col < N ? col : 0u) * (uint32_t)K * 2u // past N: not stored
-                              + 16u * (((uint32_t)lane ^ swizzle(c)) & 1u);
+        const uint32_t c = copy_col(lane);
+        const uint32_t from = (uint32_t)copied_column<TN, PARTS>(n0, part, (int)c, N) * (uint32_t)K * 2u + 16u * (((uint32_t)lane ^ swizzle(c)) & 1u);
         int n = 0;
 #pragma unroll
         for (int t = 0; t < COPIES; t++) {
@@ -926,3 +935,14 @@ hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st)
 // Test hook (not part of smat.h): groups of 4, 8 or 16 block rows and panels of 1, 2 or 4 tiles wherever they fit, whatever the
 // estimates say (0 = the choice); rows = -1: no windows.
 extern "C" void smat_internal_window_force(int rows, int tiles) { smat::g_force_rows = rows; smat::g_force_tiles = tiles; }
+
+// Test hook (not part of smat.h): the column of B that column c of a part's copy brings, of panel `panel` with `tiles` tiles a part; -1: no such panel.
+extern "C" int64_t smat_internal_window_copied_column(int tiles, int64_t N, int panel, int part, int c)
+{
+    using namespace smat;
+    const int parts = parts_of(tiles, (size_t)N), n0 = panel * 16 * tiles * parts;
+    if (n0 >= N || part >= parts || c >= 16 * tiles) return -1;
+    if (tiles == 4) return n0 + copied_column<4, 1>(n0, part, c, (int)N);
+    if (tiles == 2) return n0 + (parts == 2 ? copied_column<2, 2>(n0, part, c, (int)N) : copied_column<2, 1>(n0, part, c, (int)N));
+    return n0 + (parts == 2 ? copied_column<1, 2>(n0, part, c, (int)N) : copied_column<1, 1>(n0, part, c, (int)N));
+}
