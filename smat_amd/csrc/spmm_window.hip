@@ -436,7 +436,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
         const uint32_t piece = (uint32_t)(lane & 7) ^ swizzle(copy_col(lane));
 #pragma unroll
         for (int t = 0; t < COPIES; t++) {
-            const int q = min(copy_quad + t * quads_apart, quads - 1);
+            const int q = max(min(copy_quad + t * quads_apart, quads - 1), 0); // a group without blocks has none: what is there is not used
             load_dword(from_k[t], window + (long)gr * cap + q * 4, (piece >> 1) * 4u);
         }
     };

@@ -242,6 +242,28 @@ def test_plans_for_the_sweep_kernel_may_multiply_from_windows(smat, cuda, oracle
     plan.close()
 
 
+@pytest.mark.parametrize("rows,tiles,N", [(4, 1, 24), (8, 2, 136), (16, 2, 72), (16, 4, 64)])
+@pytest.mark.parametrize("listed", [False, True])
+def test_groups_without_blocks(smat, cuda, oracle, force, rows, tiles, N, listed):
+    """The first groups, some in the middle and the last one have no blocks: their rows of C are zeros."""
+    import torch
+    rp, ci, vals = local_matrix(200, 90, 7, seed=rows, empty=(*range(32), *range(64, 97), *range(160, 200)))
+    if listed:
+        vals = sparse_values(len(ci), 2, 1)
+    M, K, nnzb = 3200, 1440, len(ci)
+    B = whole_b(K, N, seed=N)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci, B)]
+    want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B, threads=4).astype(np.float16)
+    force(rows, tiles)
+    plan = smat.Plan(rp, M, K, nnzb, N, col_idx_host=ci)
+    plan.attach_values(*d[:3])
+    assert smat.lib.smat_internal_plan_window_rows(plan.handle) == rows and (plan.info()["kernel"] == smat.KERNEL_COMPACT) == listed
+    C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+    smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, nnzb, plan=plan)
+    assert np.array_equal(C.cpu().numpy(), want)
+    plan.close()
+
+
 @pytest.mark.parametrize("kind", ["blocks", "nonzeros", "columns"])
 def test_block_columns_in_any_order_and_twice(smat, cuda, oracle, force, kind):
     """A block row whose columns do not ascend, some of them listed twice: windows of whole blocks, of listed nonzeros, and columns of B in LDS."""
