@@ -44,6 +44,8 @@ template <int TN> constexpr int pairs_held = TN == 4 ? 12 : MAX_PAIRS;
 constexpr int ROUND = 4, MAX_ROUNDS = (MAX_PAIRS + ROUND - 1) / ROUND;
 static_assert(ROUND % 2 == 0, "the product takes two steps at a time: behind an odd number the next one of its round, zeros");
 constexpr int LIST_BITS = 26; // of a round's list: the fours of entries before it; above them its own fours
+constexpr int FILL_BITS = 4; // a round's places that are none: one at least is an octet
+static_assert(4 * ROUND <= 1 << FILL_BITS && 8 + FILL_BITS * MAX_ROUNDS <= 32, "");
 constexpr uint32_t MAX_LIST = 4 * ((1u << (32 - LIST_BITS)) - 1); // entries of a round: four a lane
 
 // ---- which block columns a group uses ----
@@ -132,11 +134,12 @@ __global__ __launch_bounds__(256) void window_list_kernel(const int32_t *__restr
 }
 
 // The nonzeros of the blocks.  Unit: an octet, 8 neighbouring columns of a block; the product multiplies four of them a step, and those without a
-// nonzero are left out, a third of a 27-point stencil's (64^3, N = 64 36.0 -> 32.2 us).  ROUND steps of a block row after the other:
+// nonzero are left out, a third of a 27-point stencil's (64^3, N = 64 36.0 -> 32.6 us).  ROUND steps of a block row after the other:
 // value << 16 | byte in the MFMA operands of the round, which lie rows KiB apart, filled up to a multiple of four with the last one.  A round
 // ends early where the next pair of blocks does not fit its list.  table: MAX_PAIRS pairs of words a block row, the places of the four octets of step j
-// in the window (8 bits each, in octets; of those that are none that of the row's first, which meets zeros) and the list of round j, the fours of
-// entries before it and its own << LIST_BITS; behind the table twice the steps of every row.  A wavefront takes a block
+// in the window (8 bits each, in octets; of those that are none that of the row's first) and the list of round j, the fours of
+// entries before it and its own << LIST_BITS; behind the table of every row twice its steps and, FILL_BITS each from bit 8 on, the places of every round
+// that are none, its last ones.  A wavefront takes a block
 // row; offset[p]: nonzeros before block p in the upper half.  Bound by the read of the values.
 __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr,
                                                              const uint32_t *__restrict__ slot, const unsigned long long *__restrict__ offset, int mb, int rows, int held,
@@ -153,6 +156,7 @@ __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__r
     u32x4 w = load(0);
     uint32_t first = blocks > 0 ? ((uint32_t)(offset[p0] >> 32) + 8u * (uint32_t)((p0 + br + 1) / 2)) & ~3u : 0; // of the round
     uint32_t octets = 0, n = 0, last = 0, longest = 0;   // of the row; entries of the round, the last one; of the longest round
+    uint32_t none = 0; // places of the rounds that are no octets
     uint32_t places = 0, list = 0, first_place = 0;       // places, list: of step and round `lane`
     auto close = [&](uint32_t round) {                    // fills the round up; the next one begins behind it
         const uint32_t end = (n + 3u) & ~3u;
@@ -194,6 +198,7 @@ __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__r
             close(round);
             round++;
             fill(octets, round * (4 * ROUND));
+            if (round <= MAX_ROUNDS) none |= (round * (4 * ROUND) - octets) << (FILL_BITS * (round - 1));
             o += round * (4 * ROUND) - octets;
             octets = round * (4 * ROUND);
             now_in = true;
@@ -226,13 +231,17 @@ __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__r
             if (n) last = __shfl(e, 63 - __clzll((long long)some));
         }
     }
-    if (octets % (4 * ROUND)) close(octets / (4 * ROUND));
+    if (octets % (4 * ROUND)) {
+        const uint32_t round = octets / (4 * ROUND);
+        close(round);
+        if (round < MAX_ROUNDS) none |= (4 * ROUND - octets % (4 * ROUND)) << (FILL_BITS * round);
+    }
     uint32_t *const to = table + (long)br * (2 * MAX_PAIRS);
     fill(octets, ~0u);
     if (lane < MAX_PAIRS) to[2 * lane] = places, to[2 * lane + 1] = list;
     if (lane == 0) {
         const uint32_t steps = min((octets + 3) / 4, (uint32_t)MAX_PAIRS);
-        table[(long)mb * (2 * MAX_PAIRS) + br] = 2 * steps;
+        table[(long)mb * (2 * MAX_PAIRS) + br] = 2 * steps | none << 8;
         if (longest > MAX_LIST || steps > (uint32_t)held || octets > 4 * MAX_PAIRS) atomicMax(most, max(longest, 1u)); // not for the windows
     }
 }
@@ -315,6 +324,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
         int p0, blocks;  // blocks: 0 where the wavefront has none; ENTRIES: twice the steps
         uint32_t packed; // lane j: places of blocks 2 j and 2 j + 1 in the window, in 32 bytes; ENTRIES: of the octets of step j, 8 bits each
         bool known;
+        uint32_t none;   // ENTRIES: places of round k that are no octets, FILL_BITS each
     };
     uint32_t list = 0; // ENTRIES: of the row taken last, lane j: the list of round j
     auto ask_row = [&](int gr, Asked &r) {
@@ -342,11 +352,11 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
         if constexpr (ENTRIES) {
             asm volatile("" : "+v"(r.q0), "+v"(r.q1));
             list = r.q1;
-            return Row{0, r.blocks, r.q0, true};
+            return Row{0, r.blocks & 0xff, r.q0, true, (uint32_t)r.blocks >> 8};
         }
         asm volatile("" : "+v"(r.q0), "+v"(r.q1), "+v"(r.c0), "+v"(r.c1));
         const bool same = (r.q0 >> SLOT_BITS) * 16u == r.c0 && (r.q1 >> SLOT_BITS) * 16u == r.c1;
-        return Row{r.p0, r.blocks, place(r.q0) | place(r.q1) << 16, r.blocks <= 2 * NP && (r.blocks == 0 || __all(same))};
+        return Row{r.p0, r.blocks, place(r.q0) | place(r.q1) << 16, r.blocks <= 2 * NP && (r.blocks == 0 || __all(same)), 0};
     };
     f16x8 a[NP];
 #pragma unroll
@@ -515,6 +525,17 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
 #pragma unroll
                     for (int t = 0; t < TN; t++) bv[u][t] = *(const __attribute__((address_space(3))) f16x8 *)(uintptr_t)(b + t * 512);
                 }
+                if constexpr (ENTRIES) // places that are no octets: zeros times zeros, whatever B holds under the octet that they name (64^3, N = 64 32.3 -> 32.6 us)
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        constexpr int LAST = 4 * (ROUND - 1);
+                        const int j = (d0 + u) % ROUND, none = (int)(row.none >> (FILL_BITS * ((d0 + u) / ROUND)) & ((1u << FILL_BITS) - 1u));
+                        if (d0 + u < NP && none > LAST - 4 * j) {
+                            const bool octet = (lane_here() >> 4) + 4 * j < 4 * ROUND - none;
+#pragma unroll
+                            for (int t = 0; t < TN; t++) bv[u][t] = octet ? bv[u][t] : zero8;
+                        }
+                    }
                 if (!ENTRIES && 2 * (d0 + U) > blocks) { // what is past the end of the row: zeros times zeros
                     const int sel = lane_here() >> 5;
 #pragma unroll

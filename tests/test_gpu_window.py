@@ -337,3 +337,37 @@ def test_octets_without_a_nonzero_are_left_out(smat, cuda, oracle, force, width,
         else:
             assert max(octets) > 22  # more rounds than a wavefront holds
         plan.close()
+
+
+@pytest.mark.parametrize("rows,tiles", [(4, 1), (8, 2), (16, 4)])
+@pytest.mark.parametrize("most", [1, 40, 62])  # rounds of 16 octets; ended early by the entries of 6 and of 4
+def test_infinities_under_the_first_octet_of_a_row(smat, cuda, oracle, force, rows, tiles, most):
+    """Octets, one a block, that do not fill a step or a round: the places left over do not multiply the row's first octet again.  A row whose own
+    nonzeros alone meet an infinity has that infinity, as block by block."""
+    import torch
+    rng = np.random.default_rng(most)
+    mb, kb, N = 41, 60, 24
+    rp = np.concatenate([[0], np.cumsum(np.arange(mb) % (18 if most == 1 else 8) + 1)]).astype(np.int32)
+    ci = np.concatenate([min(i, kb - rp[i + 1] + rp[i]) + np.arange(rp[i + 1] - rp[i]) for i in range(mb)]).astype(np.int32) * 16
+    M, K, nnzb = mb * 16, kb * 16, len(ci)
+    vals = np.zeros((nnzb, 16, 16), np.float16)
+    vals[:, 3, 0] = 2  # every block meets the infinities of its first column in this row
+    for b in vals:
+        at = rng.choice(np.delete(np.arange(1, 128), 3 * 8 - 1), most - 1, replace=False)
+        b[at // 8, at % 8] = 1
+    vals = vals.reshape(-1).view(np.uint16)
+    B = whole_b(K, N, seed=3).view(np.float16).reshape(N, K).copy()
+    first = ci[rp[:-1]]
+    B[:, first[rng.permutation(mb)[:5]]] = np.inf
+    B = B.reshape(-1).view(np.uint16)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci, B)]
+    want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B, threads=4).astype(np.float16)
+    assert np.isinf(want).any() and np.isfinite(want).any()
+    force(rows, tiles)
+    plan = smat.Plan(rp, M, K, nnzb, N, col_idx_host=ci)
+    plan.attach_values(d[0], d[1], d[2])
+    assert plan.info()["kernel"] == smat.KERNEL_COMPACT and smat.lib.smat_internal_plan_window_rows(plan.handle) == rows
+    C = torch.zeros((M, N), dtype=torch.float16, device=cuda)
+    smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, nnzb, plan=plan)
+    assert np.array_equal(C.cpu().numpy(), want, equal_nan=True)
+    plan.close()
