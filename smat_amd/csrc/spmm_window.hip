@@ -33,6 +33,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int COPIES = 7;               // KiB of a window that a wavefront copies at a time
 constexpr int SLOT_BITS = 10;           // of a block's entry: its place in the window; above them its block column
 constexpr int BITMAP_WORDS = 8192;      // block columns of the matrix / 32
+constexpr uint32_t NO_SLOT = 0xffffffffu; // a block that has none, which no column matches
 constexpr int MAX_LISTED = 128;         // block columns of a window with listed nonzeros: octets are named in 8 bits
 constexpr size_t MAX_LDS = 160 * 1024;  // of a compute unit
 constexpr int CU_WAVES = 16;            // wavefronts of 128 registers on a compute unit
@@ -127,9 +128,12 @@ __global__ __launch_bounds__(256) void window_list_kernel(const int32_t *__restr
     for (long p = row_ptr[first] + (long)threadIdx.x; p < row_ptr[last]; p += 256) {
         const int32_t col = col_idx[p];
         const uint32_t c = (uint32_t)col >> 4;
-        slot[p] = 0xffffffffu;
-        if (c < (uint32_t)words * 32u && !(col & 15))
-            slot[p] = c << SLOT_BITS | min((uint32_t)rank[c >> 5] + __popc(bitmap[c >> 5] & ((1u << (c & 31)) - 1u)), (uint32_t)cap - 1u);
+        uint32_t of = NO_SLOT; // not a column, or, where the widths were counted in another pattern, one without a place
+        if (c < (uint32_t)words * 32u && !(col & 15)) {
+            const uint32_t at = (uint32_t)rank[c >> 5] + __popc(bitmap[c >> 5] & ((1u << (c & 31)) - 1u));
+            if (at < (uint32_t)cap) of = c << SLOT_BITS | at;
+        }
+        slot[p] = of;
     }
 }
 
@@ -157,6 +161,7 @@ __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__r
     uint32_t first = blocks > 0 ? ((uint32_t)(offset[p0] >> 32) + 8u * (uint32_t)((p0 + br + 1) / 2)) & ~3u : 0; // of the round
     uint32_t octets = 0, n = 0, last = 0, longest = 0;   // of the row; entries of the round, the last one; of the longest round
     uint32_t none = 0; // places of the rounds that are no octets
+    bool no_slot = false;
     uint32_t places = 0, list = 0, first_place = 0;       // places, list: of step and round `lane`
     auto close = [&](uint32_t round) {                    // fills the round up; the next one begins behind it
         const uint32_t end = (n + 3u) & ~3u;
@@ -174,7 +179,8 @@ __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__r
         const u32x4 now = w;
         w = load(d + 1);
         const int b = min(2 * d + sel, blocks - 1);
-        const uint32_t place = (slot[p0 + b] & ((1u << SLOT_BITS) - 1u)) * 2u + (uint32_t)(g & 1);
+        const uint32_t of_block = slot[p0 + b], place = (of_block & ((1u << SLOT_BITS) - 1u)) * 2u + (uint32_t)(g & 1);
+        no_slot |= of_block == NO_SLOT;
         uint32_t bits = 0, before = 0, all = 0; // entries of the lanes before this one, and of all
         unsigned long long has_k[8];
 #pragma unroll
@@ -236,13 +242,14 @@ __global__ __launch_bounds__(256) void window_entries_kernel(const uint16_t *__r
         close(round);
         if (round < MAX_ROUNDS) none |= (4 * ROUND - octets % (4 * ROUND)) << (FILL_BITS * round);
     }
+    no_slot = __any(no_slot);
     uint32_t *const to = table + (long)br * (2 * MAX_PAIRS);
     fill(octets, ~0u);
     if (lane < MAX_PAIRS) to[2 * lane] = places, to[2 * lane + 1] = list;
     if (lane == 0) {
         const uint32_t steps = min((octets + 3) / 4, (uint32_t)MAX_PAIRS);
         table[(long)mb * (2 * MAX_PAIRS) + br] = 2 * steps | none << 8;
-        if (longest > MAX_LIST || steps > (uint32_t)held || octets > 4 * MAX_PAIRS) atomicMax(most, max(longest, 1u)); // not for the windows
+        if (no_slot || longest > MAX_LIST || steps > (uint32_t)held || octets > 4 * MAX_PAIRS) atomicMax(most, max(longest, 1u)); // not for the windows
     }
 }
 

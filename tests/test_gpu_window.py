@@ -134,6 +134,29 @@ def test_a_pattern_rewritten_in_place_is_multiplied_as_it_is(smat, cuda, oracle,
         assert np.array_equal(C.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("listed", [False, True])
+def test_columns_other_than_the_plan_s_are_multiplied_as_they_are(smat, cuda, oracle, force, listed):
+    """The columns on the device are not those that the widths of the windows were counted in: blocks without a place in a window are multiplied from
+    memory, lists of nonzeros are left to the compact kernel."""
+    import torch
+    force(8, 2)
+    rp, ci, vals = local_matrix(96, 100, 7, seed=2)
+    M, K, N, nnzb = 1536, 1600, 64, len(ci)
+    if listed:
+        vals = sparse_values(nnzb, 2, 1)
+    rng = np.random.default_rng(3)
+    moved = np.concatenate([np.sort(rng.choice(100, n, replace=False)) for n in np.diff(rp)]).astype(np.int32) * 16
+    B = whole_b(K, N, seed=3)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, moved, B)]
+    plan = smat.Plan(rp, M, K, nnzb, N, col_idx_host=ci)
+    plan.attach_values(*d[:3])
+    assert smat.lib.smat_internal_plan_window_rows(plan.handle) == (0 if listed else 8)
+    C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+    smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, nnzb, plan=plan)
+    assert np.array_equal(C.cpu().numpy(), oracle.spmm_bcsr(M, N, K, rp, moved, vals, B, threads=4).astype(np.float16))
+    plan.close()
+
+
 def test_which_products_take_windows(smat, cuda):
     """Local patterns do, as the drop-in call and with values; random ones, rows too long and products of a launch's length do not."""
     import torch
