@@ -255,6 +255,18 @@ static size_t sweep_even_rounds(const int32_t *row_ptr, const int32_t *col_idx, 
     return rows;
 }
 
+// The launch from windows of a plan that has them, or none: for another width than the plan's where the estimate is not below 0.9 of the other
+// kernel's, which an estimate below 0.9 of the least that windows are ever estimated to take settles without a look at them (bands and stencils of 4 to 5.5 us
+// at another width, 141 launches without this rule: 3 % slower in the mean than before there were windows, 13 % at most).
+template <class Other> static WindowLaunch window_or_not(const SpmmArgs &a, const smat_plan &p, Other &&other_us)
+{
+    if (a.N == p.n_cap || window_forced()) return window_launch(a, *p.window);
+    const double bar = 0.9 * other_us();
+    if (bar <= window_least_us(*p.window)) return WindowLaunch();
+    const WindowLaunch l = window_launch(a, *p.window);
+    return l.us < bar ? l : WindowLaunch();
+}
+
 extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_ptr,
                                       const int32_t *col_idx, const uint16_t *B, void *C, size_t M,
                                       size_t N, size_t K, size_t nnzb, const smat_spmm_opts *opts,
@@ -338,6 +350,25 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
             a.B = B = plan->d_bcol;
         }
     }
+    // Launches that leave the choice to the plan: windows of B or columns of B in LDS, which were weighed when the plan was made, or, for another width than
+    // its own, where they are estimated to be faster.
+    WindowLaunch windows;
+    bool columns = false;
+    if (plan && o.kernel == SMAT_KERNEL_AUTO && (plan->window || plan->resident)) {
+        const bool column_major = o.b_layout == SMAT_B_COL_MAJOR;
+        if (kernel == SMAT_KERNEL_ROWWISE && plan->window) { // a row-major B lies in column-major order by now
+            windows = window_or_not(a, *plan, [&] {
+                return rowwise_shares_items(N, (size_t)plan->n_items, nnzb / (size_t)plan->n_items) ? 0.0 :
+                       rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, RowLengths::EVEN, a.b_packed != nullptr);
+            });
+        } else if (kernel == SMAT_KERNEL_SWEEP && plan->window && column_major) {
+            windows = window_or_not(a, *plan, [&] { return sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N); });
+        } else if (kernel == SMAT_KERNEL_COMPACT && plan->window && column_major && N <= plan->n_cap) {
+            windows = window_or_not(a, *plan, [&] { return compact_estimate_us(*plan->compact, M, K, N); });
+        } else if (kernel == SMAT_KERNEL_COMPACT && plan->resident && column_major && N <= plan->n_cap) {
+            columns = N == plan->n_cap || resident_forced() || resident_launch_us(*plan->resident, K, N) < 0.9 * compact_estimate_us(*plan->compact, M, K, N);
+        }
+    }
     if (kernel == SMAT_KERNEL_MIXED) {
         // the block rows with mostly full blocks through the row-wise kernel, the others (and the empty ones) through
         // the compact kernel: disjoint rows of C, one after the other on the stream
@@ -371,11 +402,9 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
             c.accumulate = plan->sweep_blocks.d_ops != nullptr;
             e = launch_compact(c, static_cast<hipStream_t>(o.stream));
         }
-    } else if (kernel == SMAT_KERNEL_COMPACT && o.kernel == SMAT_KERNEL_AUTO && plan->window && o.b_layout == SMAT_B_COL_MAJOR && N <= plan->n_cap &&
-               (N == plan->n_cap || window_forced() || window_launch_us(a, *plan->window) < 0.9 * compact_estimate_us(*plan->compact, M, K, N))) {
-        e = launch_window(a, *plan->window, static_cast<hipStream_t>(o.stream));
-    } else if (kernel == SMAT_KERNEL_COMPACT && o.kernel == SMAT_KERNEL_AUTO && plan->resident && o.b_layout == SMAT_B_COL_MAJOR && N <= plan->n_cap &&
-               (N == plan->n_cap || resident_forced() || resident_launch_us(*plan->resident, K, N) < 0.9 * compact_estimate_us(*plan->compact, M, K, N))) {
+    } else if (windows.tiles) {
+        e = launch_window(a, *plan->window, windows, static_cast<hipStream_t>(o.stream));
+    } else if (columns) {
         e = launch_resident(a, *plan->resident, static_cast<hipStream_t>(o.stream));
     } else if (kernel == SMAT_KERNEL_COMPACT) {
         if (!plan || !plan->compact || !plan->d_bt || N > plan->n_cap)
@@ -385,10 +414,6 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         c.B = B; c.Bt = plan->d_bt; c.b_row_major = o.b_layout == SMAT_B_ROW_MAJOR; c.C = C; c.M = M; c.N = N; c.K = K; c.c_f32 = a.c_f32;
         c.plan = plan->compact;
         e = launch_compact(c, static_cast<hipStream_t>(o.stream));
-    } else if (kernel == SMAT_KERNEL_SWEEP && o.kernel == SMAT_KERNEL_AUTO && plan->window && o.b_layout == SMAT_B_COL_MAJOR &&
-               (N == plan->n_cap || window_forced() ||
-                window_launch_us(a, *plan->window) < 0.9 * sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N))) {
-        e = launch_window(a, *plan->window, static_cast<hipStream_t>(o.stream));
     } else if (kernel == SMAT_KERNEL_SWEEP) {
         if (!plan || !plan->sweep.d_ops)
             return set_error(SMAT_ERR_INVALID, "SMAT_KERNEL_SWEEP needs a plan built for it (with col_idx_host)");
@@ -397,11 +422,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         plan->sweep.fill(w, sweep_row_major);
         e = launch_sweep(w, static_cast<hipStream_t>(o.stream));
     } else {
-        bool window = plan && plan->window && o.kernel == SMAT_KERNEL_AUTO;
-        if (window && N != plan->n_cap && !window_forced()) // made for another width
-            window = !rowwise_shares_items(N, (size_t)plan->n_items, nnzb / (size_t)plan->n_items) && window_launch_us(a, *plan->window) <
-                     rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, RowLengths::EVEN, a.b_packed != nullptr);
-        e = window ? launch_window(a, *plan->window, static_cast<hipStream_t>(o.stream)) : launch_rowwise(a, static_cast<hipStream_t>(o.stream));
+        e = launch_rowwise(a, static_cast<hipStream_t>(o.stream));
     }
     if (e != hipSuccess)
         return set_error(SMAT_ERR_HIP, "SpMM launch failed: %s", hipGetErrorString(e));

@@ -180,6 +180,11 @@ struct WindowWidths { // over the groups of 4, 8 and 16 consecutive block rows: 
     uint32_t most[WINDOW_SIZES] = {}, pad = 0;
     unsigned long long sum[WINDOW_SIZES] = {};
 };
+struct WindowLaunch {
+    int tiles = 0; // 0: none
+    int n_panels = 0, panels_per_unit = 0, workgroups = 0;
+    double us = 1e30; // estimate
+};
 struct WindowPlan {
     int rows = 0, cap = 0, n_groups = 0; // block rows of a group, block columns of the widest window (a multiple of 4)
     unsigned long long sum = 0;
@@ -192,9 +197,7 @@ struct WindowPlan {
     int32_t *d_blocks = nullptr;
     // The launch of the plan's own width, for C in fp16 and fp32: 0.9 us of estimates that a call does without.
     size_t n = 0;
-    struct {
-        int tiles, n_panels, panels_per_unit, workgroups;
-    } own[2] = {};
+    WindowLaunch own[2];
 };
 struct WindowProduct {
     size_t M, K, N, nnzb;
@@ -219,8 +222,9 @@ bool window_takes_rows(int most_blocks); // block rows of so many blocks
 hipError_t window_attach_entries(WindowPlan &p, const uint16_t *vals, const int32_t *row_ptr, const unsigned long long *offset, size_t mb, size_t nnzb, int64_t nnz,
                                  bool *taken);
 double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, const WindowProduct &w);
-double window_launch_us(const SpmmArgs &a, const WindowPlan &p); // 1e30: not at this N
-hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st); // column-major B
+double window_least_us(const WindowPlan &p); // no estimate is lower
+WindowLaunch window_launch(const SpmmArgs &a, const WindowPlan &p); // of these sizes: the plan's own, or worked out
+hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, const WindowLaunch &l, hipStream_t st); // column-major B
 
 // ---- columns of B in LDS (spmm_resident.hip) ----
 struct ResidentPlan {

@@ -665,6 +665,7 @@ __global__ __launch_bounds__(1024) void spmm_window_kernel(const uint16_t *__res
 }
 
 int g_force_rows = 0, g_force_tiles = 0; // test hook
+std::atomic<int64_t> g_launches{0};      // test hook
 
 size_t lds_of(int rows, int cap, int tiles, bool entries) { return 2 * std::max((size_t)cap * tiles * 512, entries ? (size_t)rows * (ROUND * 1024) : 0); }
 // Whether windows of `cap` block columns fit: twice in LDS, and COPIES KiB a wavefront.
@@ -721,7 +722,7 @@ hipError_t prepare_all()
 }
 
 template <int TN, int PARTS, bool C_F32, bool ENTRIES>
-hipError_t launch_as(const SpmmArgs &a, const WindowPlan &p, const Launch &l, hipStream_t st)
+hipError_t launch_as(const SpmmArgs &a, const WindowPlan &p, const WindowLaunch &l, hipStream_t st)
 {
     const size_t lds = lds_of(p.rows, p.cap, TN, ENTRIES);
     const hipError_t e = prepare<TN, PARTS, C_F32, ENTRIES>();
@@ -730,6 +731,8 @@ hipError_t launch_as(const SpmmArgs &a, const WindowPlan &p, const Launch &l, hi
                        a.C, p.d_window, p.d_count, ENTRIES ? p.d_table : p.d_slot, p.d_entries, (int)(a.M / 16), p.rows, p.cap, p.n_groups, l.n_panels, l.panels_per_unit, (int)a.N, (long)a.K);
     return hipGetLastError();
 }
+
+double least_us(bool entries) { return entries ? 4.7 : 5.5; } // of a product, as estimated
 
 int best_tiles(const WindowPlan &p, const WindowProduct &w, double *us)
 {
@@ -770,7 +773,7 @@ double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, 
         steps = l.rounds * l.panels_per_unit * parts * (1.07 + 0.0155 * blocks);
         path = copies / 8.7e6, memory = once / 5.0e6, start = 1.6 + 2.2 * groups16;
     }
-    return std::max(entries ? 4.7 : 5.5, start + std::pow(std::pow(steps, 4.0) + std::pow(path, 4.0) + std::pow(memory, 4.0), 0.25));
+    return std::max(least_us(entries), start + std::pow(std::pow(steps, 4.0) + std::pow(path, 4.0) + std::pow(memory, 4.0), 0.25));
 }
 
 hipError_t window_widths(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, WindowWidths &out, void **slots)
@@ -910,40 +913,31 @@ void window_destroy(WindowPlan *p)
 bool window_forced() { return g_force_rows > 0; }
 bool window_takes_rows(int most_blocks) { return most_blocks > 0 && most_blocks <= 2 * pairs_held<1>; }
 
-static WindowProduct product_of(const SpmmArgs &a, const WindowPlan &p)
+double window_least_us(const WindowPlan &p) { return least_us(p.d_entries != nullptr); }
+
+static WindowLaunch work_out(const WindowPlan &p, const WindowProduct &w)
 {
-    return WindowProduct{a.M, a.K, a.N, a.nnzb, p.nnz, p.most_blocks, a.c_f32};
+    WindowLaunch r;
+    r.tiles = best_tiles(p, w, &r.us);
+    if (!r.tiles || !fits(p.rows, p.cap, r.tiles, p.d_entries != nullptr)) return WindowLaunch();
+    const Launch l = launch_of(p.rows, p.cap, r.tiles, p.n_groups, w.N, p.d_entries != nullptr);
+    r.n_panels = l.n_panels; r.panels_per_unit = l.panels_per_unit; r.workgroups = l.workgroups;
+    return r;
 }
 void window_settle(WindowPlan &p, size_t M, size_t K, size_t N, size_t nnzb)
 {
     p.n = N;
-    for (bool c_f32 : {false, true}) {
-        double us;
-        const int tiles = best_tiles(p, WindowProduct{M, K, N, nnzb, p.nnz, p.most_blocks, c_f32}, &us);
-        if (!tiles || !fits(p.rows, p.cap, tiles, p.d_entries != nullptr)) continue;
-        const Launch l = launch_of(p.rows, p.cap, tiles, p.n_groups, N, p.d_entries != nullptr);
-        p.own[c_f32] = {tiles, l.n_panels, l.panels_per_unit, l.workgroups};
-    }
+    for (bool c_f32 : {false, true}) p.own[c_f32] = work_out(p, WindowProduct{M, K, N, nnzb, p.nnz, p.most_blocks, c_f32});
 }
-double window_launch_us(const SpmmArgs &a, const WindowPlan &p)
+WindowLaunch window_launch(const SpmmArgs &a, const WindowPlan &p)
 {
-    double us;
-    (void)best_tiles(p, product_of(a, p), &us);
-    return us;
+    if (a.N == p.n && !g_force_tiles) return p.own[a.c_f32];
+    return work_out(p, WindowProduct{a.M, a.K, a.N, a.nnzb, p.nnz, p.most_blocks, a.c_f32});
 }
 
-hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st)
+hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, const WindowLaunch &l, hipStream_t st)
 {
     const bool entries = p.d_entries != nullptr;
-    const auto &own = p.own[a.c_f32];
-    int tiles = own.tiles;
-    Launch l{own.n_panels, own.panels_per_unit, own.workgroups, 0};
-    if (a.N != p.n || !tiles || g_force_tiles) {
-        double us;
-        tiles = best_tiles(p, product_of(a, p), &us);
-        if (tiles == 0 || !fits(p.rows, p.cap, tiles, entries)) return hipErrorInvalidValue;
-        l = launch_of(p.rows, p.cap, tiles, p.n_groups, a.N, entries);
-    }
     auto as = [&](auto tn, auto parts) {
         constexpr int TN = decltype(tn)::value, PARTS = decltype(parts)::value;
         if (entries) return a.c_f32 ? launch_as<TN, PARTS, true, true>(a, p, l, st) : launch_as<TN, PARTS, false, true>(a, p, l, st);
@@ -952,9 +946,11 @@ hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st)
     using std::integral_constant;
     const integral_constant<int, 1> one;
     const integral_constant<int, 2> two;
-    const bool halves = parts_of(tiles, a.N) == 2;
-    if (tiles == 4) return as(integral_constant<int, 4>(), one);
-    if (tiles == 2) return halves ? as(two, two) : as(two, one);
+    if (l.tiles == 0) return hipErrorInvalidValue;
+    g_launches.fetch_add(1, std::memory_order_relaxed);
+    const bool halves = parts_of(l.tiles, a.N) == 2;
+    if (l.tiles == 4) return as(integral_constant<int, 4>(), one);
+    if (l.tiles == 2) return halves ? as(two, two) : as(two, one);
     return halves ? as(one, two) : as(one, one);
 }
 
@@ -963,6 +959,8 @@ hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, hipStream_t st)
 // Test hook (not part of smat.h): groups of 4, 8 or 16 block rows and panels of 1, 2 or 4 tiles wherever they fit, whatever the
 // estimates say (0 = the choice); rows = -1: no windows.
 extern "C" void smat_internal_window_force(int rows, int tiles) { smat::g_force_rows = rows; smat::g_force_tiles = tiles; }
+// Test hook (not part of smat.h): products that were multiplied from windows so far.
+extern "C" int64_t smat_internal_window_launches(void) { return smat::g_launches.load(); }
 
 // Test hook (not part of smat.h): the column of B that column c of a part's copy brings, of panel `panel` with `tiles` tiles a part; -1: no such panel.
 extern "C" int64_t smat_internal_window_copied_column(int tiles, int64_t N, int panel, int part, int c)

@@ -181,6 +181,28 @@ def test_which_products_take_windows(smat, cuda):
     assert rows(gen.random_bcsr(128, 128, 0.2, seed=1), 512) == 0
 
 
+@pytest.mark.parametrize("m,bandwidth,n_hint,taken,left", [(4144, 51, 656, (656, 488), (128, 64)), (2192, 51, 584, (584,), (288, 112)),
+                                                           (20064, 150, 32, (32,), (8,)), (7056, 37, 320, (320,), (64,))])
+def test_launches_of_another_width_that_another_kernel_is_as_fast_for(smat, cuda, m, bandwidth, n_hint, taken, left):
+    """A launch's length: not from windows, which take 5 us at least, whatever the plan's own width takes."""
+    import torch
+    d = gen.band(m, bandwidth)
+    A = smat.csr_to_bcsr(d["M"], d["K"], d["row_ptr"], d["col_idx"], d["val"])
+    smat.lib.smat_internal_window_launches.restype = ctypes.c_int64
+    t = [to_dev(torch, x, cuda) for x in (A.val, A.row_ptr, A.col_idx, whole_b(A.K, n_hint, seed=1))]
+    plan = smat.Plan(A.row_ptr, A.M, A.K, A.nnzb, n_hint, col_idx_host=A.col_idx)
+    plan.attach_values(*t[:3])
+    assert smat.lib.smat_internal_plan_window_rows(plan.handle) > 0
+    C = torch.empty((A.M, n_hint), dtype=torch.float32, device=cuda)
+    for n in (*taken, *left):
+        for c_f32 in (False, True):
+            before = smat.lib.smat_internal_window_launches()
+            smat.spmm(*t, C, A.M, n, A.K, A.nnzb, plan=plan, c_f32=c_f32)
+            assert (smat.lib.smat_internal_window_launches() > before) == (n in taken), (n, c_f32)
+    torch.cuda.synchronize()
+    plan.close()
+
+
 def sparse_values(nnzb, seed, most):
     """Blocks of up to `most` nonzeros, some of none, small whole numbers."""
     rng = np.random.default_rng(seed)
