@@ -353,7 +353,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
     // Launches that leave the choice to the plan: windows of B or columns of B in LDS, which were weighed when the plan was made, or, for another width than
     // its own, where they are estimated to be faster.
     WindowLaunch windows;
-    bool columns = false;
+    ResidentLaunch columns;
     if (plan && o.kernel == SMAT_KERNEL_AUTO && (plan->window || plan->resident)) {
         const bool column_major = o.b_layout == SMAT_B_COL_MAJOR;
         if (kernel == SMAT_KERNEL_ROWWISE && plan->window) { // a row-major B lies in column-major order by now
@@ -366,7 +366,8 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         } else if (kernel == SMAT_KERNEL_COMPACT && plan->window && column_major && N <= plan->n_cap) {
             windows = window_or_not(a, *plan, [&] { return compact_estimate_us(*plan->compact, M, K, N); });
         } else if (kernel == SMAT_KERNEL_COMPACT && plan->resident && column_major && N <= plan->n_cap) {
-            columns = N == plan->n_cap || resident_forced() || resident_launch_us(*plan->resident, K, N) < 0.9 * compact_estimate_us(*plan->compact, M, K, N);
+            columns = resident_launch(*plan->resident, K, N);
+            if (N != plan->n_cap && !resident_forced() && columns.us >= 0.9 * compact_estimate_us(*plan->compact, M, K, N)) columns = ResidentLaunch();
         }
     }
     if (kernel == SMAT_KERNEL_MIXED) {
@@ -404,8 +405,8 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         }
     } else if (windows.tiles) {
         e = launch_window(a, *plan->window, windows, static_cast<hipStream_t>(o.stream));
-    } else if (columns) {
-        e = launch_resident(a, *plan->resident, static_cast<hipStream_t>(o.stream));
+    } else if (columns.columns) {
+        e = launch_resident(a, *plan->resident, columns, static_cast<hipStream_t>(o.stream));
     } else if (kernel == SMAT_KERNEL_COMPACT) {
         if (!plan || !plan->compact || !plan->d_bt || N > plan->n_cap)
             return set_error(SMAT_ERR_INVALID,
@@ -1085,7 +1086,8 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
             if (e == hipErrorOutOfMemory) e = hipSuccess, (void)hipGetLastError();
             if (e != hipSuccess) return fail(e);
         }
-        if (p->resident && !resident_forced() && resident_launch_us(*p->resident, p->K, p->n_cap) >= bar) {
+        if (p->resident) resident_settle(*p->resident, p->K, p->n_cap);
+        if (p->resident && !resident_forced() && p->resident->own.us >= bar) {
             resident_destroy(p->resident);
             p->resident = nullptr;
         }

@@ -227,19 +227,27 @@ WindowLaunch window_launch(const SpmmArgs &a, const WindowPlan &p); // of these 
 hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, const WindowLaunch &l, hipStream_t st); // column-major B
 
 // ---- columns of B in LDS (spmm_resident.hip) ----
+struct ResidentLaunch {
+    int columns = 0; // that a workgroup holds, 0: none
+    int groups = 0, shares = 0;
+    double us = 1e30; // estimate
+};
 struct ResidentPlan {
     int n_slices = 0, longest = 0; // of 64 lanes each; nonzeros of the longest lane
     int64_t fours = 0;             // fours of nonzeros a lane, of all slices
     uint32_t *d_list = nullptr;    // of every lane its row and the lanes that share it, then value << 16 | row of B; 256 * d_first[s] before slice s
     uint32_t *d_first = nullptr;
+    size_t n = 0; // the plan's own width, whose launch a call does not work out
+    ResidentLaunch own;
 };
 // From the lists of the compact kernel, which must be all of the matrix; synchronous, on the default stream.  *out: NULL where they do not fit.
 hipError_t resident_build(const CompactPlan &c, size_t M, size_t K, int64_t nnz, ResidentPlan **out);
 void resident_destroy(ResidentPlan *p);
 bool resident_forced(); // by the test hook
 double resident_estimate_us(size_t M, size_t K, size_t N, int64_t nnz, bool long_rows); // before the lists are there; 1e30: K too long
-double resident_launch_us(const ResidentPlan &p, size_t K, size_t N);
-hipError_t launch_resident(const SpmmArgs &a, const ResidentPlan &p, hipStream_t st); // column-major B
+void resident_settle(ResidentPlan &p, size_t K, size_t N); // the launch of width N
+ResidentLaunch resident_launch(const ResidentPlan &p, size_t K, size_t N);
+hipError_t launch_resident(const SpmmArgs &a, const ResidentPlan &p, const ResidentLaunch &l, hipStream_t st); // column-major B
 
 hipError_t launch_sweep(const SweepArgs &a, hipStream_t st);
 // Whether the sweep kernel reads a row-major B of this size in place; otherwise B is brought into column-major order first, one

@@ -469,10 +469,6 @@ __global__ __launch_bounds__(1024) void spmm_resident_kernel(const u32x4 *__rest
 
 int g_force_columns = 0, g_force_shares = 0; // test hook
 
-struct Launch {
-    int groups, shares;
-    double us;
-};
 // Workgroups of the same columns on one XCD, whose L2 then reads those columns of B alone, or workgroups of the same rows, whose
 // parts of a row of C meet in one L2.  16384 rows, 16 a row, rows together -> columns together, us: N = 64, K = 8192 6.4 -> 8.0; N = 128, K = 1040
 // 6.9 -> 8.2, K = 8192 10.1 -> 9.5; N = 256, K = 8192 13.7 -> 10.9, K = 16384 16.8 -> 14.0.
@@ -483,9 +479,9 @@ bool columns_together(size_t K, size_t N) { return N >= 128 && N * K >= (size_t)
 // the L2s take one by one, and bytes.  Fitted to 259 products of 40 uniform random matrices and 7 stencils, M and K 1,040 to 63,760, N = 8 to 816: 11 %
 // standard deviation, and what it picks is 0.6 % from the best tried in the mean.  Estimate (measured), us: 18736 x 18704, 38 a row, N = 88, 4 columns,
 // 11 shares 12.7 (13.4); 2000 x 6448, 40 a row, N = 816, 8 and 2 10.6 (10.6); 32400 x 2096, 17 a row, N = 680, fp32, 8 and 3 38 (51).
-Launch launch_of(const ResidentPlan &p, size_t K, size_t N, int T)
+ResidentLaunch launch_of(const ResidentPlan &p, size_t K, size_t N, int T)
 {
-    Launch best{(int)(N / T), 1, 1e30};
+    ResidentLaunch best{T, (int)(N / T), 1, 1e30};
     if (lds_of(K, T) > MAX_LDS || N % T) return best;
     const double four = T == 2 ? 0.0124 : T == 4 ? 0.014 : 0.0232, fill = 2.2 + 1.41e-5 * (double)K * 2.0 * T;
     const int most = std::max(1, std::min((p.n_slices + WAVES - 1) / WAVES, 512 / best.groups + 1));
@@ -499,14 +495,15 @@ Launch launch_of(const ResidentPlan &p, size_t K, size_t N, int T)
     return best;
 }
 
-int best_columns(const ResidentPlan &p, size_t K, size_t N, Launch *l)
+std::atomic<int64_t> g_searches{0}; // test hook
+ResidentLaunch best_launch(const ResidentPlan &p, size_t K, size_t N)
 {
-    int best = 0;
-    l->us = 1e30;
+    g_searches.fetch_add(1, std::memory_order_relaxed);
+    ResidentLaunch best;
     for (int T : {8, 4, 2}) {
         if (g_force_columns && T != g_force_columns) continue;
-        const Launch x = launch_of(p, K, N, T);
-        if (x.us < l->us) *l = x, best = T;
+        const ResidentLaunch x = launch_of(p, K, N, T);
+        if (x.us < best.us) best = x;
     }
     return best;
 }
@@ -525,7 +522,7 @@ hipError_t prepare()
 }
 
 template <int T, bool C_F32>
-hipError_t launch_as(const SpmmArgs &a, const ResidentPlan &p, const Launch &l, hipStream_t st)
+hipError_t launch_as(const SpmmArgs &a, const ResidentPlan &p, const ResidentLaunch &l, hipStream_t st)
 {
     const hipError_t e = prepare<T, C_F32>();
     if (e != hipSuccess) return e;
@@ -543,23 +540,25 @@ double resident_estimate_us(size_t M, size_t K, size_t N, int64_t nnz, bool long
     p.n_slices = (int)((M + 63) / 64);
     p.fours = nnz / 256 + (int64_t)p.n_slices * 3 / 4;
     if (long_rows) p.fours += nnz / 768, p.longest = PART; // R-MAT scales 12 to 14: a third more
-    Launch l;
-    return best_columns(p, K, N, &l) ? l.us : 1e30;
+    return best_launch(p, K, N).us;
 }
-double resident_launch_us(const ResidentPlan &p, size_t K, size_t N)
+// Worked out once for the plan's own width: 0.2 us of a call with 1,024 slices (65536 rows, N = 8 5.1 -> 4.9 of host time), nothing with 64 or fewer.
+void resident_settle(ResidentPlan &p, size_t K, size_t N)
 {
-    Launch l;
-    return best_columns(p, K, N, &l) ? l.us : 1e30;
+    p.n = N;
+    p.own = best_launch(p, K, N);
+}
+ResidentLaunch resident_launch(const ResidentPlan &p, size_t K, size_t N)
+{
+    return N == p.n && !g_force_columns ? p.own : best_launch(p, K, N);
 }
 bool resident_forced() { return g_force_columns > 0; }
 
-hipError_t launch_resident(const SpmmArgs &a, const ResidentPlan &p, hipStream_t st)
+hipError_t launch_resident(const SpmmArgs &a, const ResidentPlan &p, const ResidentLaunch &l, hipStream_t st)
 {
-    Launch l;
-    const int T = best_columns(p, a.K, a.N, &l);
-    if (T == 8) return a.c_f32 ? launch_as<8, true>(a, p, l, st) : launch_as<8, false>(a, p, l, st);
-    if (T == 4) return a.c_f32 ? launch_as<4, true>(a, p, l, st) : launch_as<4, false>(a, p, l, st);
-    if (T == 2) return a.c_f32 ? launch_as<2, true>(a, p, l, st) : launch_as<2, false>(a, p, l, st);
+    if (l.columns == 8) return a.c_f32 ? launch_as<8, true>(a, p, l, st) : launch_as<8, false>(a, p, l, st);
+    if (l.columns == 4) return a.c_f32 ? launch_as<4, true>(a, p, l, st) : launch_as<4, false>(a, p, l, st);
+    if (l.columns == 2) return a.c_f32 ? launch_as<2, true>(a, p, l, st) : launch_as<2, false>(a, p, l, st);
     return hipErrorInvalidValue;
 }
 
@@ -631,3 +630,5 @@ hipError_t resident_build(const CompactPlan &c, size_t M, size_t K, int64_t nnz,
 
 // Test hook: the columns of B that a workgroup holds (2, 4 or 8; 0 = chosen, -1 = no plan takes the kernel) and the shares of the rows (0 = chosen).
 extern "C" void smat_internal_resident_force(int columns, int shares) { smat::g_force_columns = columns; smat::g_force_shares = shares; }
+// Test hook: launches that were worked out so far.
+extern "C" int64_t smat_internal_resident_searches(void) { return smat::g_searches.load(); }

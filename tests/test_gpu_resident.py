@@ -158,6 +158,26 @@ def test_which_products_hold_columns(smat, cuda, force):
     assert takes(1024, 65536, 8, 64) == 0
 
 
+def test_calls_of_the_plan_s_width_do_not_work_out_their_launch(smat, cuda):
+    import torch
+    smat.lib.smat_internal_resident_searches.restype = ctypes.c_int64
+    M, K, N = 2048, 2048, 64
+    A = scattered(smat, np.full(M, 8), K, seed=M)
+    d = [to_dev(torch, x, cuda) for x in (A.val, A.row_ptr, A.col_idx, np.zeros(K * N, np.uint16))]
+    plan = plan_of(smat, A, d, N)
+    assert smat.lib.smat_internal_plan_resident(plan.handle) == 1
+    C = torch.empty((M, N), dtype=torch.float32, device=cuda)
+    searches = []
+    for n in (N, 40):
+        before = smat.lib.smat_internal_resident_searches()
+        for c_f32 in (False, True):
+            smat.spmm(*d, C, M, n, K, len(A.col_idx), plan=plan, c_f32=c_f32)
+        searches.append(smat.lib.smat_internal_resident_searches() - before)
+    assert searches == [0, 2]
+    torch.cuda.synchronize()
+    plan.close()
+
+
 @pytest.mark.parametrize("windows", [False, True])
 def test_captured_launches_replay(smat, cuda, oracle, force, windows):
     """Columns in LDS and windows of listed nonzeros in a graph, replayed between launches outside of it, B changing from replay to replay."""
