@@ -984,6 +984,18 @@ hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t
     return e;
 }
 
+// Of 36 such launches of two panels and more (stencils, N = 72 to 256, column- and row-major B) in one run an XCD 4.3 % slower in the mean than the best of the
+// runs that are tried, 21 % at most (45 x 15 x 54, N = 72, row-major 11.3 against 9.4 us); in halves 0.9 and 10, in quarters 2.6 and 12.  One panel, 66
+// launches: 0.7, 1.8, 3.6 %.  (Beside columns in LDS, uniform random matrices: 1.3, 2.0 and 4.9 %, left as they are.)
+void compact_deal_in_halves(CompactPlan &p, size_t N, size_t K)
+{
+    const int width = compact_panel_width(p, N, K, false), n_panels = (int)((N + width - 1) / width);
+    const unsigned eighth = (unsigned)((((long)p.n_tasks * n_panels + 3) / 4 + 7) / 8);
+    if (n_panels < 2 || eighth < 8 || p.deal.run((size_t)p.n_tasks, n_panels) < eighth) return;
+    p.tuned_n = N;
+    p.tuned_run = eighth / 2;
+}
+
 hipError_t values_checksum(const uint16_t *vals, size_t nnzb, uint64_t *out)
 {
     *out = 0;

@@ -243,6 +243,34 @@ def test_windows_of_listed_nonzeros_match_the_oracle(smat, cuda, oracle, force, 
     plan.close()
 
 
+@pytest.mark.parametrize("N", [64, 72])
+def test_launches_of_the_compact_kernel_beside_windows_run_in_halves(smat, cuda, N):
+    """Of two panels and more; one panel in one run an XCD."""
+    import torch
+    d = gen.stencil27(40)
+    A = smat.csr_to_bcsr(d["M"], d["K"], d["row_ptr"], d["col_idx"], d["val"])
+    t = [to_dev(torch, x, cuda) for x in (A.val, A.row_ptr, A.col_idx, whole_b(A.K, N, seed=1))]
+    plan = smat.Plan(A.row_ptr, A.M, A.K, A.nnzb, N, col_idx_host=A.col_idx)
+    plan.attach_values(*t[:3])
+    assert smat.lib.smat_internal_plan_window_rows(plan.handle) > 0 and plan.info()["kernel"] == smat.KERNEL_COMPACT
+    smat.lib.smat_internal_compact_run.argtypes = [ctypes.c_int]
+    C = torch.empty((A.M, N), dtype=torch.float16, device=cuda)
+    runs = {}
+    try:
+        for force_run in (0, 1 << 24):
+            smat.lib.smat_internal_compact_run(force_run)
+            for row_major in (False, True):
+                smat.spmm(*t, C, A.M, N, A.K, A.nnzb, plan=plan, b_row_major=row_major, kernel=smat.KERNEL_COMPACT)
+                runs[force_run, row_major] = smat.lib.smat_internal_compact_last_run()
+    finally:
+        smat.lib.smat_internal_compact_run(0)
+    torch.cuda.synchronize()
+    for row_major in (False, True):
+        eighth = runs[1 << 24, row_major]
+        assert eighth >= 8 and runs[0, row_major] == (eighth if N == 64 else eighth // 2)
+    plan.close()
+
+
 def test_values_attached_again_replace_the_listed_ones(smat, cuda, oracle, force):
     """Between lists, from a list to full blocks and back, and to columns too full for a list; a launch wider than the plan is refused as before."""
     import torch
