@@ -794,12 +794,12 @@ static hipError_t sweep_small_groups(smat_plan &p, size_t group_rows)
 // -> windows, us: 27-point stencil 64^3, N = 64 90 -> 56, 48^3, N = 256 111 -> 59, 48 x 25 x 48, N = 56 20.4 -> 12.7; bands of
 // 14224 rows and 182, N = 544 33 -> 17, of 65536 and 20, N = 256 30 -> 15, of 8960 and 120, N = 48 7.4 -> 5.
 // census: of the values, where the compact kernel would multiply: the window kernel then multiplies what it would, the values as attached.
-// wait: for the lists, which launches on other streams than the default one may read.
-static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us, const uint16_t *vals, const CompactCensus *census,
-                              bool wait = true)
+// Whole blocks: does not wait for the lists, which launches on other streams than the default one may read.
+static bool may_take_window(const smat_plan &p) { return p.kernel_requested == SMAT_KERNEL_AUTO && !p.n_split_rows && window_takes_rows(p.max_item_blocks); }
+static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, WindowCount &count, double other_us, const uint16_t *vals, const CompactCensus *census)
 {
     const size_t mb = p.M / 16, kb = p.K / 16;
-    if ((p.kernel != SMAT_KERNEL_ROWWISE && !(p.kernel == SMAT_KERNEL_SWEEP && p.sweep_few_tiles)) || p.kernel_requested != SMAT_KERNEL_AUTO || p.n_split_rows || !window_takes_rows(p.max_item_blocks)) return hipSuccess;
+    if ((p.kernel != SMAT_KERNEL_ROWWISE && !(p.kernel == SMAT_KERNEL_SWEEP && p.sweep_few_tiles)) || !may_take_window(p)) return hipSuccess;
     if (!census && rowwise_shares_items(p.n_cap, (size_t)p.n_items, p.nnzb / std::max<size_t>((size_t)p.n_items, 1)) && !window_forced()) return hipSuccess;
     if (!census && p.n_cap <= 16 && !window_forced()) return hipSuccess; // 18 -> 17, 10.4 -> 9.2, but 8.2 -> 9, 6.6 -> 7
     // its estimate knows nothing of the bytes that come from memory, A above all and three times B where that is repacked: 64^3 64 us and
@@ -811,21 +811,18 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     const double bar = 0.9 * (census ? other_us - copy : std::min(row_wise, other_us));
     // a launch, or the bytes that windows do not save
     if (!window_forced() && bar < std::max(4.7, 2.0 + once)) return hipSuccess;
-    WindowWidths widths;
-    void *slots = nullptr;
-    if (p.nnzb <= 16384 && p.col_idx_host.size() == p.nnzb) // sooner done than a kernel is waited for
-        window_widths_host(p.row_ptr_host.data(), p.col_idx_host.data(), mb, kb, widths);
-    else {
-        const hipError_t e = window_widths(row_ptr, col_idx, mb, kb, p.nnzb, widths, &slots);
-        if (e != hipSuccess) return e;
-    }
+    hipError_t e = hipSuccess;
+    if (!count.there && !count.begun && p.nnzb <= WindowCount::FEW && p.col_idx_host.size() == p.nnzb) count.on_host(p.row_ptr_host.data(), p.col_idx_host.data(), mb, kb);
+    else e = count.end(row_ptr, col_idx, mb, kb, p.nnzb);
+    if (e != hipSuccess) return e;
+    const WindowWidths &widths = count.widths;
     int size;
     const double us = window_choose(widths, WindowProduct{p.M, p.K, p.n_cap, p.nnzb, census ? census->nnz : -1, p.max_item_blocks, false}, &size);
     // The sweep kernel brings all block columns in turn, and multiplies faster: not where the windows are most of them too (2448 x 1280, 16 %,
     // N = 552 7.9 -> 8.7 us).
     const bool most_of_b = size >= 0 && !census && other_us < 1e30 && (double)widths.sum[size] > 0.5 * (double)kb * (double)mb / (4 << size);
-    if (size < 0 || (!window_forced() && (us >= bar || most_of_b))) return slots ? dev_free(slots) : hipSuccess;
-    hipError_t e = window_build(widths, size, slots, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, wait && !census, &p.window);
+    if (size < 0 || (!window_forced() && (us >= bar || most_of_b))) return hipSuccess;
+    e = window_build(widths, size, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, &p.window);
     if (e == hipSuccess && !census) window_settle(*p.window, p.M, p.K, p.n_cap, p.nnzb);
     if (e != hipSuccess || !census) return e;
     bool taken;
@@ -839,16 +836,15 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     return e;
 }
 // No memory for the windows is not an error of the plan.
-static hipError_t take_window_if_room(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, double other_us, const uint16_t *vals, const CompactCensus *census,
-                                      bool wait = true)
+static hipError_t take_window_if_room(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, WindowCount &count, double other_us, const uint16_t *vals, const CompactCensus *census)
 {
-    const hipError_t e = take_window(p, row_ptr, col_idx, other_us, vals, census, wait);
+    const hipError_t e = take_window(p, row_ptr, col_idx, count, other_us, vals, census);
     if (e != hipErrorOutOfMemory) return e;
     (void)hipGetLastError();
     return hipSuccess;
 }
-hipError_t smat::plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx) {
-    return take_window_if_room(*p, row_ptr, col_idx, 1e30, nullptr, nullptr, false); // a plan of the cache, which launches on the default stream alone
+hipError_t smat::plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx, WindowCount &count) {
+    return take_window_if_room(*p, row_ptr, col_idx, count, 1e30, nullptr, nullptr); // a plan of the cache, which launches on the default stream alone
 }
 
 static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, const int32_t *row_ptr,
@@ -895,7 +891,10 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     // without / with 2:4 / with dense rows) put to use per block row.
     CompactCensus census;
     CompactPlan *c = nullptr;
-    hipError_t e = compact_census(vals, row_ptr, mb, p->nnzb, census);
+    // The widths of windows beside it, where the host would not count them sooner once they are asked for.
+    WindowCount count;
+    hipError_t e = compact_census(vals, row_ptr, mb, p->nnzb, census, col_idx, p->K / 16,
+                                  may_take_window(*p) && (p->nnzb > WindowCount::FEW || p->col_idx_host.size() != p->nnzb) ? &count : nullptr);
     if (e != hipSuccess) return fail(e);
     std::vector<uint8_t> dense(mb, 0);
     int64_t dense_cols_all = 0;
@@ -996,18 +995,21 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
             // Windows against the sweep kernel, whose streams are made all the same: the plan says that kernel, and launches that ask for it
             // get it.  us: bands of 13296 rows and 30, N = 304 9.6 -> 7.5, 8320 and 25, N = 576 10.4 -> 8.7, 39584 and 18, N = 904 55 -> 48; 21 x 14 x 52,
             // N = 88 8.4 -> 6.2, 21 x 76 x 25, N = 224 22.6 -> 20.1.
-            if (!p->d_bcol && !g_force_group_rows) e = take_window_if_room(*p, row_ptr, col_idx, sweep_us, nullptr, nullptr);
+            if (!p->d_bcol && !g_force_group_rows) e = take_window_if_room(*p, row_ptr, col_idx, count, sweep_us, nullptr, nullptr);
             if (e == hipSuccess) e = sweep_small_groups(*p, group_rows);
         } else if (!take || !p->d_bcol)
-            e = take_window_if_room(*p, row_ptr, col_idx, compact_estimate_us((double)census.n_cols_all, std::min(36.0 * (double)census.n_cols_all, 4.25 * (double)census.n_cols_all + 4.0 * (double)census.nnz), p->M, p->K,
+            e = take_window_if_room(*p, row_ptr, col_idx, count, compact_estimate_us((double)census.n_cols_all, std::min(36.0 * (double)census.n_cols_all, 4.25 * (double)census.n_cols_all + 4.0 * (double)census.nnz), p->M, p->K,
                                                 p->n_cap), vals, take ? &census : nullptr);
         if (e != hipSuccess) return fail(e);
     }
     if (want == SMAT_KERNEL_AUTO && dense_kernel == SMAT_KERNEL_SWEEP && p->sweep_few_tiles && !take && !p->d_bcol) { // attached before
-        e = take_window_if_room(*p, row_ptr, col_idx, sweep_estimate_us((size_t)p->sweep.n_rg, p->sweep_chunks, p->nnzb, p->M, p->n_cap), nullptr, nullptr);
+        e = take_window_if_room(*p, row_ptr, col_idx, count, sweep_estimate_us((size_t)p->sweep.n_rg, p->sweep_chunks, p->nnzb, p->M, p->n_cap), nullptr, nullptr);
         if (e != hipSuccess) return fail(e);
     }
-    if (!take) return SMAT_OK; // nothing would use the list: the plan keeps (or goes back to) a dense kernel
+    if (!take) { // nothing would use the list: the plan keeps (or goes back to) a dense kernel
+        if (p->window) e = hipStreamSynchronize(nullptr); // launches on other streams read its lists
+        return e == hipSuccess ? SMAT_OK : fail(e);
+    }
     if (!c) e = compact_build(census, vals, row_ptr, col_idx, p->K, p->n_cap, p->d_bcol != nullptr, mixed ? &dense : nullptr, false, &c);
     if (e != hipSuccess) return fail(e);
     if (!p->d_bt) e = dev_malloc(&p->d_bt, p->bt_bytes());

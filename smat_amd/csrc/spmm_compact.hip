@@ -104,10 +104,11 @@ __device__ __forceinline__ void add_totals(const unsigned long long (&mine)[N], 
     }
 }
 // sums[i] of the pass, from the words that add_totals added to (synchronous)
-hipError_t fetch_totals(const void *d_sums, unsigned long long *out, int n)
+hipError_t fetch_totals(const void *d_sums, unsigned long long *out, int n, WindowCount *widths = nullptr) // widths: what WindowCount::launch put behind them
 {
-    std::vector<unsigned long long> all(SUM_BYTES / sizeof(unsigned long long));
-    const hipError_t e = hipMemcpy(all.data(), d_sums, SUM_BYTES, hipMemcpyDeviceToHost);
+    std::vector<unsigned long long> all((SUM_BYTES + (widths ? WindowCount::BYTES : 0)) / sizeof(unsigned long long));
+    const hipError_t e = hipMemcpy(all.data(), d_sums, all.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost);
+    if (e == hipSuccess && widths) widths->take(all.data() + SUM_BYTES / sizeof(unsigned long long));
     for (int i = 0; i < n; i++) {
         out[i] = 0;
         for (int s = 0; s < SUM_SLOTS; s++) out[i] += all[(size_t)(s * SUM_STRIDE + i)];
@@ -1067,7 +1068,7 @@ static hipError_t census_offsets(CompactCensus &s, const int32_t *row_ptr)
     return e;
 }
 
-hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t mb, size_t nnzb, CompactCensus &s)
+hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t mb, size_t nnzb, CompactCensus &s, const int32_t *col_idx, size_t kb, WindowCount *widths)
 {
     hipError_t e = hipSuccess;
     s.mb = mb;
@@ -1082,8 +1083,9 @@ hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t m
     SMAT_STEP(s.count.alloc(nnzb * 8));
     SMAT_STEP(s.offset.alloc(nnzb * 8));
     SMAT_STEP(s.rows.alloc((mb + 1) * 8));
-    SMAT_STEP(sums.alloc(SUM_BYTES));
+    SMAT_STEP(sums.alloc(SUM_BYTES + WindowCount::BYTES));
     SMAT_STEP(hipMemsetAsync(sums.p, 0, SUM_BYTES, nullptr));
+    if (e == hipSuccess && widths && !widths->launch(row_ptr, col_idx, mb, kb, nnzb, static_cast<unsigned char *>(sums.p) + SUM_BYTES)) widths = nullptr;
     if (e == hipSuccess) {
         const long waves = std::min<long>((long)(nnzb + 1) / 2, 256L * 32);
         hipLaunchKernelGGL(colmask_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, 0, vals, (long)nnzb,
@@ -1092,7 +1094,7 @@ hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t m
     }
     SMAT_STEP(census_offsets(s, row_ptr));
     unsigned long long total[N_SUMS] = {0};
-    SMAT_STEP(fetch_totals(sums.p, total, N_SUMS));
+    SMAT_STEP(fetch_totals(sums.p, total, N_SUMS, widths));
     sums.idle = e == hipSuccess;
     s.values_checksum = total[SUM_CHECK];
     s.full_blocks = (int64_t)total[SUM_FULL];

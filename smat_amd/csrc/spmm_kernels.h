@@ -135,8 +135,10 @@ struct CompactCensus {
     void waited() { mask.idle = single.idle = count.idle = offset.idle = rows.idle = true; } // for all that uses them
     int64_t cols_of_row(size_t br) const { return (int64_t)(uint32_t)(raw[br + 1] - raw[br]); }
 };
-// vals / row_ptr / col_idx here and below: device BCSR arrays.  Synchronous.
-hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t mb, size_t nnzb, CompactCensus &s);
+// vals / row_ptr / col_idx here and below: device BCSR arrays.  Synchronous.  widths != NULL: those of the windows of the pattern, kb block columns, too.
+struct WindowCount;
+hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t mb, size_t nnzb, CompactCensus &s, const int32_t *col_idx = nullptr, size_t kb = 0,
+                          WindowCount *widths = nullptr);
 hipError_t compact_full_blocks(const CompactCensus &s, std::vector<uint8_t> &full); // one flag per block
 // The lists of a plan.  leave_rows != NULL: flagged block rows get no list and no work item (a dense kernel multiplies
 // them).  drop_full: full blocks get no listed columns (another kernel multiplies them); from then on the census is
@@ -179,7 +181,7 @@ bool rowwise_shares_items(size_t N, size_t n_items, size_t avg_blocks);
 // For matrices whose neighbouring block rows use the same block columns.
 constexpr int WINDOW_SIZES = 3;
 struct WindowWidths { // over the groups of 4, 8 and 16 consecutive block rows: the most block columns that one uses, and all together
-    uint32_t most[WINDOW_SIZES] = {}, pad = 0;
+    uint32_t most[WINDOW_SIZES] = {};
     unsigned long long sum[WINDOW_SIZES] = {};
 };
 struct WindowLaunch {
@@ -207,20 +209,31 @@ struct WindowProduct {
     int most_blocks; // of a block row
     bool c_f32;
 };
-// row_ptr / col_idx: device arrays.  All but the launch and the estimates are synchronous, on the default stream.
-// *slots: memory for the entries of the blocks, which window_build takes over (or NULL).
-hipError_t window_widths(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, WindowWidths &out, void **slots);
-void window_widths_host(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, WindowWidths &out); // the same from host arrays
+// The widths of a pattern's windows, counted on the host or by a kernel, which runs while its caller does other work, or with another kernel's results
+// on their way to the host.  row_ptr / col_idx: device arrays; on the default stream.
+struct WindowCount {
+    static constexpr size_t FEW = 8192;      // blocks that the host counts sooner than it launches a kernel and fetches what that found
+    static constexpr int PARTS = 256;        // workgroups a size, at most
+    static constexpr size_t BYTES = WINDOW_SIZES * PARTS * 8;
+    WindowWidths widths;
+    bool there = false, begun = false;
+    bool launch(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, void *to); // BYTES there; false: none to come
+    void take(const void *parts); // what launch left, from host memory
+    void begin(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb); // does not wait
+    hipError_t end(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb); // of what has begun, or from the beginning
+    void on_host(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb); // host arrays, columns checked
+private:
+    DevScratch parts;
+};
 // The size of group (index into the widths, -1 = none fits) that is fastest for a product of N columns, and its time in us.
 double window_choose(const WindowWidths &widths, const WindowProduct &w, int *size);
-// wait = false: the caller waits for the default stream before the plan is used.
-hipError_t window_build(const WindowWidths &w, int size, void *slots, const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, int most_blocks,
-                        bool wait, WindowPlan **out);
+// row_ptr / col_idx: device arrays.  Does not wait: the caller does, for the default stream, before a launch on another one.
+hipError_t window_build(const WindowWidths &w, int size, const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, int most_blocks, WindowPlan **out);
 void window_settle(WindowPlan &p, size_t M, size_t K, size_t N, size_t nnzb); // the launch of width N
 void window_destroy(WindowPlan *p);
 bool window_forced(); // by the test hook
 bool window_takes_rows(int most_blocks); // block rows of so many blocks
-// offset: of every block, the nonzeros before it in the upper half.  *taken: false where a pair of blocks has too many.
+// offset: of every block, the nonzeros before it in the upper half.  *taken: false where a pair of blocks has too many.  Synchronous.
 hipError_t window_attach_entries(WindowPlan &p, const uint16_t *vals, const int32_t *row_ptr, const unsigned long long *offset, size_t mb, size_t nnzb, int64_t nnz,
                                  bool *taken);
 double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, const WindowProduct &w);
@@ -265,6 +278,6 @@ hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st);
 
 struct smat_plan;
 namespace smat {
-// A plan that has no better kernel than the row-wise one gets windows where they are faster (row_ptr / col_idx: device arrays).
-hipError_t plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx);
+// A plan that has no better kernel than the row-wise one gets windows where they are faster (row_ptr / col_idx: device arrays).  Does not wait, as window_build.
+hipError_t plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx, WindowCount &count);
 } // namespace smat

@@ -63,16 +63,15 @@ __device__ __forceinline__ void mark_columns(uint32_t *bitmap, int words, const 
     __syncthreads();
 }
 
-// A workgroup takes every gridDim.x-th group of one size: additions to one word queue up at 12 ns each (with a workgroup a group
-// 170 us for 16384 block rows).
+// A workgroup takes every gridDim.x-th group of one size; parts[size * WindowCount::PARTS + blockIdx.x]: the most block columns of one of its groups, and
+// those of all its groups.  (Additions to one word queue up at 12 ns each, and need zeros first.)
 __global__ __launch_bounds__(256) void window_count_kernel(const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_idx, int mb, int words,
-                                                           WindowWidths *__restrict__ stat)
+                                                           uint2 *__restrict__ parts)
 {
     extern __shared__ uint32_t bitmap[];
     __shared__ uint32_t part[4];
     const int rows = blockIdx.y == 0 ? SIZES[0] : blockIdx.y == 1 ? SIZES[1] : SIZES[2];
-    uint32_t most = 0;
-    unsigned long long sum = 0;
+    uint32_t most = 0, sum = 0; // of blocks, which are fewer than 2^31
     for (long first = (long)blockIdx.x * rows; first < mb; first += (long)gridDim.x * rows) {
         mark_columns(bitmap, words, row_ptr, col_idx, (int)first, (int)min(first + rows, (long)mb));
         uint32_t n = 0;
@@ -86,10 +85,7 @@ __global__ __launch_bounds__(256) void window_count_kernel(const int32_t *__rest
         sum += n;
         __syncthreads();
     }
-    if (threadIdx.x == 0 && most) {
-        atomicMax(&stat->most[blockIdx.y], most);
-        atomicAdd(&stat->sum[blockIdx.y], sum);
-    }
+    if (threadIdx.x == 0) parts[blockIdx.y * WindowCount::PARTS + blockIdx.x] = uint2{most, sum};
 }
 
 // window[group * cap ..]: the first columns of the group's blocks, ascending, filled up to a multiple of 4; slot[p]: the place
@@ -100,18 +96,26 @@ __global__ __launch_bounds__(256) void window_list_kernel(const int32_t *__restr
 {
     extern __shared__ uint32_t bitmap[]; // words, and as many half words of ranks behind them
     uint16_t *const rank = reinterpret_cast<uint16_t *>(bitmap + words);
-    __shared__ uint32_t part[256];
+    __shared__ uint32_t part[4];
     const int first = (int)blockIdx.x * rows, last = min(first + rows, mb);
     mark_columns(bitmap, words, row_ptr, col_idx, first, last);
     const int per = (words + 255) / 256, w0 = min((int)threadIdx.x * per, words), w1 = min(w0 + per, words);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint32_t n = 0;
     for (int w = w0; w < w1; w++) n += __popc(bitmap[w]);
-    part[threadIdx.x] = n;
+    uint32_t before = n; // to the sum of the threads before this one
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t of = __shfl_up(before, d);
+        before += lane >= d ? of : 0;
+    }
+    if (lane == 63) part[wave] = before;
+    before -= n;
     __syncthreads();
-    uint32_t before = 0, all = 0;
-    for (int t = 0; t < 256; t++) {
-        if (t < (int)threadIdx.x) before += part[t];
-        all += part[t];
+    uint32_t all = 0;
+    for (int w = 0; w < 4; w++) {
+        before += w < wave ? part[w] : 0;
+        all += part[w];
     }
     int32_t *const out = window + (long)blockIdx.x * cap;
     for (int w = w0; w < w1; w++) {
@@ -776,45 +780,68 @@ double window_estimate_us(int rows, int cap, unsigned long long sum, int tiles, 
     return std::max(least_us(entries), start + std::pow(std::pow(steps, 4.0) + std::pow(path, 4.0) + std::pow(memory, 4.0), 0.25));
 }
 
-hipError_t window_widths(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, WindowWidths &out, void **slots)
+bool WindowCount::launch(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, void *to)
 {
-    out = WindowWidths{};
-    *slots = nullptr;
     const int words = (int)((kb + 31) / 32);
-    if (nnzb == 0 || kb > (size_t)BITMAP_WORDS * 32) return hipSuccess; // none known
-    hipError_t e = dev_malloc(slots, std::max(nnzb * sizeof(uint32_t), sizeof out));
-    if (e != hipSuccess) return e;
-    e = hipMemsetAsync(*slots, 0, sizeof out, nullptr);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(window_count_kernel, dim3((unsigned)std::min<size_t>((mb + SIZES[0] - 1) / SIZES[0], 256), WINDOW_SIZES), dim3(256), (size_t)words * 4, nullptr, row_ptr, col_idx,
-                           (int)mb, words, (WindowWidths *)*slots);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpy(&out, *slots, sizeof out, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) {
-        (void)dev_free(*slots);
-        *slots = nullptr;
-    }
+    if (nnzb == 0 || kb > (size_t)BITMAP_WORDS * 32) return false;
+    static_assert(PARTS * WINDOW_SIZES * sizeof(uint2) == BYTES, "");
+    hipLaunchKernelGGL(window_count_kernel, dim3(PARTS, WINDOW_SIZES), dim3(256), (size_t)words * 4, nullptr, row_ptr, col_idx, (int)mb, words, (uint2 *)to);
+    return hipGetLastError() == hipSuccess;
+}
+
+void WindowCount::take(const void *from)
+{
+    const uint2 *of = static_cast<const uint2 *>(from);
+    widths = WindowWidths{};
+    for (int s = 0; s < WINDOW_SIZES; s++)
+        for (int i = 0; i < PARTS; i++) {
+            widths.most[s] = std::max(widths.most[s], of[s * PARTS + i].x);
+            widths.sum[s] += of[s * PARTS + i].y;
+        }
+    there = true;
+}
+
+void WindowCount::begin(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb)
+{
+    parts.release();
+    begun = parts.alloc(BYTES) == hipSuccess && launch(row_ptr, col_idx, mb, kb, nnzb, parts.p);
+}
+
+hipError_t WindowCount::end(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb)
+{
+    if (there) return hipSuccess;
+    widths = WindowWidths{}; // none known
+    if (!begun) begin(row_ptr, col_idx, mb, kb, nnzb);
+    there = true;
+    if (!begun) return parts.p ? hipSuccess : hipErrorOutOfMemory;
+    uint2 of[WINDOW_SIZES * PARTS];
+    const hipError_t e = hipMemcpy(of, parts.p, sizeof of, hipMemcpyDeviceToHost);
+    parts.idle = e == hipSuccess;
+    if (e == hipSuccess) take(of);
     return e;
 }
 
-void window_widths_host(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, WindowWidths &out)
+void WindowCount::on_host(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb)
 {
-    out = WindowWidths{};
-    std::vector<uint32_t> seen(kb, 0); // the last group that used the column, counted over all sizes from 1
-    uint32_t group = 0;
-    for (int s = 0; s < WINDOW_SIZES; s++)
-        for (size_t first = 0; first < mb; first += (size_t)SIZES[s]) {
-            group++;
-            uint32_t n = 0;
-            for (int32_t q = row_ptr[first], end = row_ptr[std::min(first + (size_t)SIZES[s], mb)]; q < end; q++) {
-                uint32_t &last = seen[(size_t)col_idx[q] / 16];
-                n += last != group;
-                last = group;
-            }
-            out.most[s] = std::max(out.most[s], n);
-            out.sum[s] += n;
+    static_assert(SIZES[0] == 4 && SIZES[1] == 8 && SIZES[2] == 16, "groups of one size are halves of those of the next");
+    widths = WindowWidths{};
+    there = true;
+    std::vector<uint32_t> seen(kb, 0); // the last block row that used the column, from 1
+    uint32_t n[WINDOW_SIZES] = {};
+    for (size_t r = 0; r < mb; r++) {
+        for (int32_t q = row_ptr[r]; q < row_ptr[r + 1]; q++) {
+            uint32_t &last = seen[(size_t)col_idx[q] / 16];
+            const uint32_t apart = (last - 1) ^ (uint32_t)r; // below the size of a group where both rows are in one
+            last = (uint32_t)r + 1;
+            for (int s = 0; s < WINDOW_SIZES; s++) n[s] += apart >= (uint32_t)SIZES[s];
         }
+        for (int s = 0; s < WINDOW_SIZES; s++)
+            if ((r + 1) % SIZES[s] == 0 || r + 1 == mb) {
+                widths.most[s] = std::max(widths.most[s], n[s]);
+                widths.sum[s] += n[s];
+                n[s] = 0;
+            }
+    }
 }
 
 double window_choose(const WindowWidths &widths, const WindowProduct &w, int *size)
@@ -838,23 +865,18 @@ double window_choose(const WindowWidths &widths, const WindowProduct &w, int *si
     return best;
 }
 
-hipError_t window_build(const WindowWidths &w, int size, void *slots, const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, int most_blocks,
-                        bool wait, WindowPlan **out)
+hipError_t window_build(const WindowWidths &w, int size, const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, int most_blocks, WindowPlan **out)
 {
     *out = nullptr;
     WindowPlan *p = new (std::nothrow) WindowPlan();
-    if (!p) {
-        if (slots) (void)dev_free(slots);
-        return hipErrorOutOfMemory;
-    }
-    p->d_slot = static_cast<uint32_t *>(slots);
+    if (!p) return hipErrorOutOfMemory;
     const int words = (int)((kb + 31) / 32);
     p->rows = SIZES[size];
     p->cap = (int)((w.most[size] + 3) / 4 * 4);
     p->sum = w.sum[size];
     p->most_blocks = most_blocks;
     p->n_groups = (int)((mb + p->rows - 1) / p->rows);
-    hipError_t e = slots ? hipSuccess : dev_malloc(&p->d_slot, nnzb * sizeof(uint32_t));
+    hipError_t e = dev_malloc(&p->d_slot, nnzb * sizeof(uint32_t));
     if (e == hipSuccess) e = dev_malloc(&p->d_window, (size_t)p->n_groups * (p->cap + 1) * sizeof(int32_t));
     p->d_count = p->d_window + (size_t)p->n_groups * p->cap;
     if (e == hipSuccess) {
@@ -863,7 +885,6 @@ hipError_t window_build(const WindowWidths &w, int size, void *slots, const int3
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = prepare_all<false>();
-    if (e == hipSuccess && wait) e = hipStreamSynchronize(nullptr); // launches on other streams read the lists
     if (e != hipSuccess) {
         window_destroy(p);
         return e;
@@ -961,6 +982,20 @@ hipError_t launch_window(const SpmmArgs &a, const WindowPlan &p, const WindowLau
 extern "C" void smat_internal_window_force(int rows, int tiles) { smat::g_force_rows = rows; smat::g_force_tiles = tiles; }
 // Test hook (not part of smat.h): products that were multiplied from windows so far.
 extern "C" int64_t smat_internal_window_launches(void) { return smat::g_launches.load(); }
+
+// Test hook (not part of smat.h): the widths of windows, most and sum of each size, from device arrays and from host arrays.
+extern "C" int smat_internal_window_widths(const int32_t *row_ptr, const int32_t *col_idx, const int32_t *row_ptr_host, const int32_t *col_idx_host, size_t mb, size_t kb,
+                                           size_t nnzb, int64_t *out)
+{
+    smat::WindowCount device, host;
+    const hipError_t e = device.end(row_ptr, col_idx, mb, kb, nnzb);
+    host.on_host(row_ptr_host, col_idx_host, mb, kb);
+    for (int i = 0; i < smat::WINDOW_SIZES; i++) {
+        *out++ = device.widths.most[i], *out++ = (int64_t)device.widths.sum[i];
+        *out++ = host.widths.most[i], *out++ = (int64_t)host.widths.sum[i];
+    }
+    return (int)e;
+}
 
 // Test hook (not part of smat.h): the column of B that column c of a part's copy brings, of panel `panel` with `tiles` tiles a part; -1: no such panel.
 extern "C" int64_t smat_internal_window_copied_column(int tiles, int64_t N, int panel, int part, int c)

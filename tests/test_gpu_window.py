@@ -16,6 +16,7 @@ def to_dev(torch, a, cuda):
 @pytest.fixture
 def force(smat):
     smat.lib.smat_internal_window_force.argtypes = [ctypes.c_int, ctypes.c_int]
+    smat.lib.smat_internal_window_launches.restype = ctypes.c_int64
     yield smat.lib.smat_internal_window_force
     smat.lib.smat_internal_window_force(0, 0)
     smat.lib.smat_plan_cache_clear()
@@ -154,6 +155,36 @@ def test_columns_other_than_the_plan_s_are_multiplied_as_they_are(smat, cuda, or
     C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
     smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, nnzb, plan=plan)
     assert np.array_equal(C.cpu().numpy(), oracle.spmm_bcsr(M, N, K, rp, moved, vals, B, threads=4).astype(np.float16))
+    plan.close()
+
+
+# words of the bitmap of a window: one, as many as threads, more; block rows that do and do not fill the groups, and more groups than workgroups
+@pytest.mark.parametrize("mb,kb,width", [(1, 3, 2), (37, 31, 9), (1500, 8192, 12), (7133, 20011, 12)])
+def test_widths_and_lists_of_windows(smat, cuda, oracle, force, mb, kb, width):
+    """The widths as the device and the host count them, and products from lists that the device makes of wide bitmaps."""
+    import torch
+    rp, ci, vals = local_matrix(mb, kb, width, seed=mb, empty=range(20, 90) if mb > 90 else ())
+    M, K, N, nnzb = mb * 16, kb * 16, 24, len(ci)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci)]
+    got = (ctypes.c_int64 * 12)()
+    ptr = lambda a: ctypes.c_void_p(a.data_ptr() if torch.is_tensor(a) else a.ctypes.data)
+    assert smat.lib.smat_internal_window_widths(ptr(d[1]), ptr(d[2]), ptr(rp), ptr(ci), ctypes.c_size_t(mb), ctypes.c_size_t(kb), ctypes.c_size_t(nnzb), got) == 0
+    for i, rows in enumerate((4, 8, 16)):
+        widths = [len(np.unique(ci[rp[g]:rp[min(g + rows, mb)]])) for g in range(0, mb, rows)]
+        assert list(got)[4 * i:4 * i + 4] == [max(widths), sum(widths)] * 2
+    B = whole_b(K, N, seed=N)
+    d.append(to_dev(torch, B, cuda))
+    want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B, threads=8).astype(np.float16)
+    force(8, 1)
+    plan = smat.Plan(rp, M, K, nnzb, N, col_idx_host=ci)
+    plan.attach_values(*d[:3])
+    smat.lib.smat_plan_cache_clear()
+    for p in (plan, None):
+        C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+        before = smat.lib.smat_internal_window_launches()
+        smat.spmm(*d, C, M, N, K, nnzb, plan=p, drop_in=p is None)
+        assert smat.lib.smat_internal_window_launches() == before + 1
+        assert np.array_equal(C.cpu().numpy(), want)
     plan.close()
 
 
