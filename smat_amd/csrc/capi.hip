@@ -1094,7 +1094,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
             p->resident = nullptr;
         }
     }
-    if (p->window) compact_deal_in_halves(*c, p->n_cap, p->K);
+    if (p->window) compact_deal_beside_windows(*c, p->n_cap, p->K);
     if (!p->window && !p->resident) e = compact_tune(*c, p->d_bt, p->M, p->n_cap, p->K, p->d_bcol != nullptr, block_split); // else its launches are not what the plan is for
     if (e != hipSuccess) return set_error(SMAT_ERR_HIP, "timing the compact kernel failed: %s", hipGetErrorString(e));
     if (p->d_bpack && want == SMAT_KERNEL_AUTO && !mixed) { // the row-wise kernel's scratch is not needed any more

@@ -987,14 +987,16 @@ hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t
 
 // Of 36 such launches of two panels and more (stencils, N = 72 to 256, column- and row-major B) in one run an XCD 4.3 % slower in the mean than the best of the
 // runs that are tried, 21 % at most (45 x 15 x 54, N = 72, row-major 11.3 against 9.4 us); in halves 0.9 and 10, in quarters 2.6 and 12.  One panel, 66
-// launches: 0.7, 1.8, 3.6 %.  (Beside columns in LDS, uniform random matrices: 1.3, 2.0 and 4.9 %, left as they are.)
-void compact_deal_in_halves(CompactPlan &p, size_t N, size_t K)
+// launches: 0.7, 1.8, 3.6 %.  Where the panels are a multiple of four, a quarter of an eighth is whole panels again: 41 stencils, N = 200 to 256 and
+// 456 to 512, against the runs that were timed, halves 1 % slower column-major and 2.4 row-major, 25 at most (56 x 14 x 25, N = 240, row-major
+// 10.9 us, 12.9 in halves), quarters 0 and 2.5 % faster, 9 slower at most; of five to seven panels quarters are 1 to 3 % slower than halves.  (Beside columns in LDS, uniform random matrices: 1.3, 2.0 and 4.9 %, left as they are.)
+void compact_deal_beside_windows(CompactPlan &p, size_t N, size_t K)
 {
     const int width = compact_panel_width(p, N, K, false), n_panels = (int)((N + width - 1) / width);
     const unsigned eighth = (unsigned)((((long)p.n_tasks * n_panels + 3) / 4 + 7) / 8);
     if (n_panels < 2 || eighth < 8 || p.deal.run((size_t)p.n_tasks, n_panels) < eighth) return;
     p.tuned_n = N;
-    p.tuned_run = eighth / 2;
+    p.tuned_run = eighth / (n_panels % 4 ? 2 : 4);
 }
 
 hipError_t values_checksum(const uint16_t *vals, size_t nnzb, uint64_t *out)

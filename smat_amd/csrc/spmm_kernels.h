@@ -168,8 +168,8 @@ hipError_t launch_compact(const CompactArgs &a, hipStream_t st);
 // Synchronous, default stream; a plan too large for the temporary buffers, or whose single launch would take longer than
 // 20 ms, keeps the estimate's choice.
 hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t K, bool b_row_major, bool accumulate);
-// Without trials, for plans that multiply from windows where they may: an even list of neighbouring block rows in runs of half an eighth of the launch.
-void compact_deal_in_halves(CompactPlan &p, size_t N, size_t K);
+// Without trials, for plans that multiply from windows where they may: an even list of neighbouring block rows in runs of half or a quarter of an eighth of the launch.
+void compact_deal_beside_windows(CompactPlan &p, size_t N, size_t K);
 hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, size_t N, size_t K, hipStream_t st);
 
 // What a launch of the row-wise kernel knows about the lengths of its items: no block row is much longer than the average

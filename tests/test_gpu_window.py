@@ -274,9 +274,9 @@ def test_windows_of_listed_nonzeros_match_the_oracle(smat, cuda, oracle, force, 
     plan.close()
 
 
-@pytest.mark.parametrize("N", [64, 72])
-def test_launches_of_the_compact_kernel_beside_windows_run_in_halves(smat, cuda, N):
-    """Of two panels and more; one panel in one run an XCD."""
+@pytest.mark.parametrize("N,parts", [(64, 1), (72, 2), (192, 2), (200, 4), (264, 2)])
+def test_launches_of_the_compact_kernel_beside_windows_run_in_parts(smat, cuda, N, parts):
+    """Halves where there are two panels and more, quarters of four; one panel in one run an XCD."""
     import torch
     d = gen.stencil27(40)
     A = smat.csr_to_bcsr(d["M"], d["K"], d["row_ptr"], d["col_idx"], d["val"])
@@ -298,7 +298,7 @@ def test_launches_of_the_compact_kernel_beside_windows_run_in_halves(smat, cuda,
     torch.cuda.synchronize()
     for row_major in (False, True):
         eighth = runs[1 << 24, row_major]
-        assert eighth >= 8 and runs[0, row_major] == (eighth if N == 64 else eighth // 2)
+        assert eighth >= 8 and runs[0, row_major] == eighth // parts
     plan.close()
 
 
