@@ -202,6 +202,19 @@ static double rowwise_estimate_us(size_t M, size_t K, size_t N, size_t nnzb, siz
     const double column = !packed || tiles <= 4 ? 1.0 : tiles == 8 ? 0.83 : 0.8;
     return start + (double)rounds * (double)tiles * (double)nnzb / (double)n_items * (packed ? 0.0274 * column : 0.074);
 }
+// The same on B in place up to 14 us, with what neighbouring block rows find of each other's rows of B in the caches: share4, block columns of a group of four
+// rows per block.  Fitted to 1,600 products (bands, stencils and random patterns, N = 24 to 4,096): 7 to 8 % standard deviation, where the estimate above is 20 % too high
+// in the mean for longer rows, 30 to 40 for bands, and 21 % off either way for shorter ones.  Columns of B a multiple of a cache line apart (K % 64 == 0) are slower to
+// gather: bands of 11 blocks a row, 1 to 5 panels 4.5 us, 5.4 with such a K.
+static double rowwise_in_place_us(size_t M, size_t K, size_t N, size_t nnzb, size_t n_items, int most_blocks, double share4)
+{
+    const double mn = 1e-6 * (double)M * (double)N, aligned = K % 64 == 0 ? 1.0 : 0.0;
+    if (rowwise_takes_short_rows(N, n_items, most_blocks))
+        return 2.62 + 1.56 * mn + 0.49e-6 * (double)K * (double)N + 4.26e-6 * share4 * (double)nnzb * (double)N + 0.435 * aligned;
+    const double avg = (double)nnzb / (double)n_items;
+    const size_t tiles = (size_t)rowwise_panel_tiles(N, n_items, (size_t)avg, RowLengths::EVEN, false), wavefronts = n_items * ((N + 16 * tiles - 1) / (16 * tiles));
+    return 2.48 + 0.56 * mn + (double)tiles * avg * ((double)((wavefronts + 1023) / 1024) * (0.038 + 0.0189 * aligned) + (double)wavefronts / 1024.0 * 0.0338 * share4);
+}
 // A row-major B into column-major order, for the kernels that do not read it in place (8192 x 4096 23 us, 4112 x 504 3 us beside
 // the launch that follows); and what the sweep kernel takes longer on a row-major B in place (8192^2, 10 %, N = 4096 103 against 97 us,
 // with N = 2040, rows that straddle cache lines, 50 against 43).
@@ -265,6 +278,21 @@ template <class Other> static WindowLaunch window_or_not(const SpmmArgs &a, cons
     if (bar <= window_least_us(*p.window)) return WindowLaunch();
     const WindowLaunch l = window_launch(a, *p.window);
     return l.us < bar ? l : WindowLaunch();
+}
+
+// Windows of whole blocks in the place of the row-wise kernel on B in place, for products of less than 14 us: not where what is fitted to such products says that they
+// are slower, or, of patterns that share little, less than 5 % faster.  The estimates behind the choice so far know little of these, nor of narrow bands of few block rows: 31 of 60
+// random patterns that windows were chosen for were up to 52 % slower for it, 45 of 260 bands up to 25 % (random 1664 x 2064, 4 %, N = 1560 8.2 -> 12.5 us; band of 1248 rows and 75,
+// N = 832 4.48 -> 5.58).
+constexpr double SHORT_US = 14.0;
+static double rowwise_in_place_us(const smat_plan &p, size_t N, double share4)
+{
+    if (N < 24) return SHORT_US; // not fitted to these
+    return rowwise_in_place_us(p.M, p.K, N, p.nnzb, (size_t)p.n_items, p.max_item_blocks, share4);
+}
+static bool windows_beat(const smat_plan &p, const WindowPlan &shape, const WindowLaunch &l, size_t N, double in_place)
+{
+    return l.tiles && window_short_us(shape, l, p.M, p.K, N, p.nnzb) < (shape.share > 0.6 ? 0.95 : 1.0) * in_place;
 }
 
 extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_ptr,
@@ -357,10 +385,16 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
     if (plan && o.kernel == SMAT_KERNEL_AUTO && (plan->window || plan->resident)) {
         const bool column_major = o.b_layout == SMAT_B_COL_MAJOR;
         if (kernel == SMAT_KERNEL_ROWWISE && plan->window) { // a row-major B lies in column-major order by now
-            windows = window_or_not(a, *plan, [&] {
-                return rowwise_shares_items(N, (size_t)plan->n_items, nnzb / (size_t)plan->n_items) ? 0.0 :
-                       rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, RowLengths::EVEN, a.b_packed != nullptr);
-            });
+            const bool shares = rowwise_shares_items(N, (size_t)plan->n_items, nnzb / (size_t)plan->n_items);
+            const double in_place = N == plan->n_cap || window_forced() || shares || a.b_packed ? SHORT_US : rowwise_in_place_us(*plan, N, plan->window->share4);
+            if (in_place < SHORT_US) {
+                windows = window_launch(a, *plan->window);
+                if (!windows_beat(*plan, *plan->window, windows, N, in_place)) windows = WindowLaunch();
+            } else {
+                windows = window_or_not(a, *plan, [&] {
+                    return shares ? 0.0 : rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, RowLengths::EVEN, a.b_packed != nullptr);
+                });
+            }
         } else if (kernel == SMAT_KERNEL_SWEEP && plan->window && column_major) {
             windows = window_or_not(a, *plan, [&] { return sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N); });
         } else if (kernel == SMAT_KERNEL_COMPACT && plan->window && column_major && N <= plan->n_cap) {
@@ -822,6 +856,12 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     // N = 552 7.9 -> 8.7 us).
     const bool most_of_b = size >= 0 && !census && other_us < 1e30 && (double)widths.sum[size] > 0.5 * (double)kb * (double)mb / (4 << size);
     if (size < 0 || (!window_forced() && (us >= bar || most_of_b))) return hipSuccess;
+    if (!census && !p.d_bpack && (vals || other_us > 1e29) && !window_forced()) { // beside the row-wise kernel, not the sweep kernel
+        WindowPlan shape;
+        const WindowLaunch l = window_launch_of(widths, size, WindowProduct{p.M, p.K, p.n_cap, p.nnzb, -1, p.max_item_blocks, false}, shape);
+        const double in_place = rowwise_in_place_us(p, p.n_cap, shape.share4);
+        if (in_place < SHORT_US && !windows_beat(p, shape, l, p.n_cap, in_place)) return hipSuccess;
+    }
     e = window_build(widths, size, row_ptr, col_idx, mb, kb, p.nnzb, p.max_item_blocks, &p.window);
     if (e == hipSuccess && !census) window_settle(*p.window, p.M, p.K, p.n_cap, p.nnzb);
     if (e != hipSuccess || !census) return e;

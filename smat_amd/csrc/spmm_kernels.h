@@ -177,6 +177,7 @@ hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, siz
 enum class RowLengths { EVEN, SPLIT, UNKNOWN };
 int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, RowLengths lengths, bool packed);
 bool rowwise_shares_items(size_t N, size_t n_items, size_t avg_blocks);
+bool rowwise_takes_short_rows(size_t N, size_t n_items, int most_blocks); // by the short-row kernel: B in place, no split rows
 // ---- whole blocks from windows of B in LDS (spmm_window.hip) ----
 // For matrices whose neighbouring block rows use the same block columns.
 constexpr int WINDOW_SIZES = 3;
@@ -186,12 +187,13 @@ struct WindowWidths { // over the groups of 4, 8 and 16 consecutive block rows: 
 };
 struct WindowLaunch {
     int tiles = 0; // 0: none
-    int n_panels = 0, panels_per_unit = 0, workgroups = 0;
+    int n_panels = 0, panels_per_unit = 0, workgroups = 0, rounds = 0;
     double us = 1e30; // estimate
 };
 struct WindowPlan {
     int rows = 0, cap = 0, n_groups = 0; // block rows of a group, block columns of the widest window (a multiple of 4)
     unsigned long long sum = 0;
+    double share = 1.0, share4 = 1.0;    // window columns per block, in groups of this size and of 4
     int most_blocks = 0;                 // of a block row
     int32_t *d_window = nullptr, *d_count = nullptr; // window of group i: d_count[i] first columns from d_window[i * cap] on
     uint32_t *d_slot = nullptr;          // of every block: its place in the window, and its block column
@@ -227,6 +229,9 @@ private:
 };
 // The size of group (index into the widths, -1 = none fits) that is fastest for a product of N columns, and its time in us.
 double window_choose(const WindowWidths &widths, const WindowProduct &w, int *size);
+// The launch of a product from windows of that size, of whole blocks, and their shares, before anything is built.
+WindowLaunch window_launch_of(const WindowWidths &widths, int size, const WindowProduct &w, WindowPlan &shape);
+double window_short_us(const WindowPlan &p, const WindowLaunch &l, size_t M, size_t K, size_t N, size_t nnzb); // of whole blocks, up to 14 us
 // row_ptr / col_idx: device arrays.  Does not wait: the caller does, for the default stream, before a launch on another one.
 hipError_t window_build(const WindowWidths &w, int size, const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, int most_blocks, WindowPlan **out);
 void window_settle(WindowPlan &p, size_t M, size_t K, size_t N, size_t nnzb); // the launch of width N

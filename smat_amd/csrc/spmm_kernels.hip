@@ -547,7 +547,11 @@ bool rowwise_shares_items(size_t N, size_t n_items, size_t avg_blocks)
 
 // The short-row kernel: rows of at most 2 * SHORT_NP blocks, no split rows, B in place, few wavefronts.
 constexpr int SHORT_NP = 5;
-constexpr long SHORT_MAX_WAVES = 8192;
+constexpr size_t SHORT_MAX_WAVES = 8192;
+bool rowwise_takes_short_rows(size_t N, size_t n_items, int most_blocks)
+{
+    return most_blocks > 0 && most_blocks <= 2 * SHORT_NP && N >= 32 && n_items * ((N + 31) / 32) <= SHORT_MAX_WAVES;
+}
 
 template <int TN>
 static hipError_t launch_rowwise_short(const SpmmArgs &a, hipStream_t st)
@@ -589,8 +593,7 @@ static hipError_t launch_rowwise_split(const SpmmArgs &a, hipStream_t st)
 hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st)
 {
     hipError_t e;
-    if (!a.b_packed && a.n_split_rows == 0 && a.max_item_blocks > 0 && a.max_item_blocks <= 2 * SHORT_NP && a.N >= 32 &&
-        (long)a.n_items * (long)((a.N + 31) / 32) <= SHORT_MAX_WAVES) {
+    if (!a.b_packed && a.n_split_rows == 0 && rowwise_takes_short_rows(a.N, (size_t)a.n_items, a.max_item_blocks)) {
         // 32-column panels while that still leaves the chip short of wavefronts, else 64
         const bool narrow = (long)a.n_items * (long)((a.N + 63) / 64) < 2048;
         return narrow ? launch_rowwise_short<2>(a, st) : launch_rowwise_short<4>(a, st);

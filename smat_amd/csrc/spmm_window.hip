@@ -865,17 +865,24 @@ double window_choose(const WindowWidths &widths, const WindowProduct &w, int *si
     return best;
 }
 
+static void shape_of(WindowPlan &p, const WindowWidths &w, int size, size_t mb, size_t nnzb, int most_blocks)
+{
+    p.rows = SIZES[size];
+    p.cap = (int)((w.most[size] + 3) / 4 * 4);
+    p.sum = w.sum[size];
+    p.share = (double)w.sum[size] / (double)nnzb;
+    p.share4 = (double)w.sum[0] / (double)nnzb;
+    p.most_blocks = most_blocks;
+    p.n_groups = (int)((mb + p.rows - 1) / p.rows);
+}
+
 hipError_t window_build(const WindowWidths &w, int size, const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, int most_blocks, WindowPlan **out)
 {
     *out = nullptr;
     WindowPlan *p = new (std::nothrow) WindowPlan();
     if (!p) return hipErrorOutOfMemory;
     const int words = (int)((kb + 31) / 32);
-    p->rows = SIZES[size];
-    p->cap = (int)((w.most[size] + 3) / 4 * 4);
-    p->sum = w.sum[size];
-    p->most_blocks = most_blocks;
-    p->n_groups = (int)((mb + p->rows - 1) / p->rows);
+    shape_of(*p, w, size, mb, nnzb, most_blocks);
     hipError_t e = dev_malloc(&p->d_slot, nnzb * sizeof(uint32_t));
     if (e == hipSuccess) e = dev_malloc(&p->d_window, (size_t)p->n_groups * (p->cap + 1) * sizeof(int32_t));
     p->d_count = p->d_window + (size_t)p->n_groups * p->cap;
@@ -942,8 +949,23 @@ static WindowLaunch work_out(const WindowPlan &p, const WindowProduct &w)
     r.tiles = best_tiles(p, w, &r.us);
     if (!r.tiles || !fits(p.rows, p.cap, r.tiles, p.d_entries != nullptr)) return WindowLaunch();
     const Launch l = launch_of(p.rows, p.cap, r.tiles, p.n_groups, w.N, p.d_entries != nullptr);
-    r.n_panels = l.n_panels; r.panels_per_unit = l.panels_per_unit; r.workgroups = l.workgroups;
+    r.n_panels = l.n_panels; r.panels_per_unit = l.panels_per_unit; r.workgroups = l.workgroups; r.rounds = l.rounds;
     return r;
+}
+WindowLaunch window_launch_of(const WindowWidths &widths, int size, const WindowProduct &w, WindowPlan &shape)
+{
+    shape_of(shape, widths, size, w.M / 16, w.nnzb, w.most_blocks);
+    return work_out(shape, w);
+}
+// Below 5.5 us, and where little is shared, the estimate above says little: here the start, the steps one after the other, their blocks, the copies, B and C, and the parts of the
+// panels; copies of single blocks of a B beyond half an XCD's L2, a cache line for 32 bytes of it, cost twice.  Fitted to 3,474 launches of less than 16 us of every size of group and
+// panel (240 bands, 200 stencils, 200 random patterns, N = 24 to 2,048): 6 % standard deviation, 15 for the estimate above.
+double window_short_us(const WindowPlan &p, const WindowLaunch &l, size_t M, size_t K, size_t N, size_t nnzb)
+{
+    const double parts = parts_of(l.tiles, N), steps = (double)l.rounds * l.panels_per_unit * parts, b = 2e-6 * (double)K * (double)N, c = 2e-6 * (double)M * (double)N;
+    const double copies = 512e-6 * (double)p.sum * l.tiles * parts * l.n_panels;
+    return 2.28 + 2.1 * p.rows / 16.0 + steps * (0.356 + 0.0102 * (double)nnzb * 16.0 / (double)M * l.tiles) + 0.143 * (b + c) +
+           copies * (p.share > 0.6 && b > 2.0 ? 0.133 : 0.0666) + 0.0153 * parts * l.n_panels;
 }
 void window_settle(WindowPlan &p, size_t M, size_t K, size_t N, size_t nnzb)
 {

@@ -234,6 +234,47 @@ def test_launches_of_another_width_that_another_kernel_is_as_fast_for(smat, cuda
     plan.close()
 
 
+def blocked_band(smat, m, bandwidth):
+    d = gen.band(m, bandwidth)
+    A = smat.csr_to_bcsr(d["M"], d["K"], d["row_ptr"], d["col_idx"], d["val"])
+    return A.M, A.K, A.row_ptr, A.col_idx, A.val
+
+
+def blocked_random(mb, kb, density):
+    A = gen.random_bcsr(mb, kb, density, seed=1)
+    return A["M"], A["K"], A["b_row_ptr"].astype(np.int32), A["b_col_idx"].astype(np.int32), A["b_val"]
+
+
+@pytest.mark.parametrize("matrix,n_hint,own,others", [
+    # 12.5, 15.3 and 11.4 us from windows, 8.2, 10.8 and 8.1 from memory; little is shared
+    ((104, 129, 0.04), 1560, False, {}), ((84, 193, 0.0399), 1848, False, {}), ((148, 55, 0.0398), 2024, False, {}),
+    # 5.6 and 5.0, one round of wavefronts of the row-wise kernel 4.5 and 4.1
+    ((1248, 75), 832, False, {}), ((688, 77), 968, False, {}),
+    # 4.5 and 5.8, before 5.7 and 9.0
+    ((2112, 82), 216, True, {}), ((2464, 15), 912, True, {}),
+    # of other widths 4.1 and 4.0, before 5.4 and 5.4; columns of B that are whole cache lines apart
+    ((1536, 73), 304, True, {224: True, 120: True}), ((1472, 68), 280, True, {208: True}),
+])
+def test_short_products_take_windows_where_they_are_faster(smat, cuda, oracle, matrix, n_hint, own, others):
+    import torch
+    M, K, rp, ci, _ = blocked_band(smat, *matrix) if len(matrix) == 2 else blocked_random(*matrix)
+    vals = np.random.default_rng(1).integers(-3, 4, len(ci) * 256).astype(np.float16).view(np.uint16)
+    B = whole_b(K, n_hint, seed=2)
+    t = [to_dev(torch, x, cuda) for x in (vals, rp, ci, B)]
+    want = oracle.spmm_bcsr(M, n_hint, K, rp, ci, vals, B, threads=8).astype(np.float16)
+    plan = smat.Plan(rp, M, K, len(ci), n_hint, col_idx_host=ci)
+    plan.attach_values(*t[:3])
+    assert (smat.lib.smat_internal_plan_window_rows(plan.handle) > 0) == own
+    smat.lib.smat_internal_window_launches.restype = ctypes.c_int64
+    for n, taken in {n_hint: own, **others}.items():
+        C = torch.full((M, n), float("nan"), dtype=torch.float16, device=cuda)
+        before = smat.lib.smat_internal_window_launches()
+        smat.spmm(*t, C, M, n, K, len(ci), plan=plan)
+        assert (smat.lib.smat_internal_window_launches() > before) == taken, n
+        assert np.array_equal(C.cpu().numpy(), want[:, :n])
+    plan.close()
+
+
 def sparse_values(nnzb, seed, most):
     """Blocks of up to `most` nonzeros, some of none, small whole numbers."""
     rng = np.random.default_rng(seed)
