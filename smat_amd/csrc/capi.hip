@@ -132,8 +132,9 @@ extern "C" void smat_internal_fail_alloc(int64_t n) { g_dev_fail_in.store(n); }
 // Test hook (not part of smat.h): block rows that the compact kernel's list of this plan splits, -1 without a list.
 extern "C" int smat_internal_compact_split_rows(const smat_plan *p) { return p->compact ? p->compact->n_split_rows : -1; }
 
-// Test hook (not part of smat.h): block rows of a group whose window the plan's products multiply from, 0 without windows.
+// Test hook (not part of smat.h): whether the plan's products hold columns of B in LDS.
 extern "C" int smat_internal_plan_resident(const smat_plan *p) { return p->resident != nullptr; }
+// Test hook (not part of smat.h): block rows of a group whose window the plan's products multiply from, 0 without windows.
 extern "C" int smat_internal_plan_window_rows(const smat_plan *p) { return p->window ? p->window->rows : 0; }
 
 // Test hook (not part of smat.h): rows of B that the compact kernel's copy holds, 0 where it holds all or there is no list.
