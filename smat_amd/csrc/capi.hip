@@ -605,6 +605,20 @@ struct PlanHolder { // frees a half-built plan on every way out but the good one
 };
 } // namespace
 
+// Row-wise kernel: repacking B slab-major costs a launch plus one read and one write of B
+// per SpMM (about 3 us + 4*K*N bytes at 4 TB/s) and lets the operand gather, nnzb*16*N*2
+// bytes, run at about 20 TB/s instead of 7.6 TB/s (measured on the row-wise kernel).
+static bool repack_pays(size_t K, size_t N, size_t nnzb)
+{
+    const double gather_bytes = (double)nnzb * 16.0 * (double)N * 2.0;
+    return gather_bytes * (1.0 / 7.6e6 - 1.0 / 20e6) > 1.5 * (3.0 + 4.0 * (double)K * (double)N / 4e6);
+}
+// The sweep kernel's work list is made with the plan, for M = 16 mb and N = n_hint.
+static bool sweep_from_the_start(size_t mb, size_t kb, size_t N, size_t nnzb)
+{
+    return sweep_fills_device(mb, N) && (double)nnzb >= 0.05 * (double)mb * (double)kb && nnzb < (size_t)1 << 23 && nnzb >= 2;
+}
+
 static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
                                  const int32_t *col_idx_host, size_t M, size_t K, size_t nnzb,
                                  size_t n_hint, const smat_spmm_opts *opts)
@@ -701,17 +715,8 @@ static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
         p->workspace_bytes = (size_t)slot * 16 * n_hint * sizeof(float);
         if (e == hipSuccess) e = dev_malloc(&p->d_workspace, p->workspace_bytes);
     }
-    // Row-wise kernel: repacking B slab-major costs a launch plus one read and one write of B
-    // per SpMM (about 3 us + 4*K*N bytes at 4 TB/s) and lets the operand gather, nnzb*16*N*2
-    // bytes, run at about 20 TB/s instead of 7.6 TB/s (measured on the row-wise kernel).
-    {
-        const double gather_bytes = (double)nnzb * 16.0 * (double)n_hint * 2.0;
-        const double gain_us = gather_bytes * (1.0 / 7.6e6 - 1.0 / 20e6);
-        const double cost_us = 3.0 + 4.0 * (double)K * (double)n_hint / 4e6;
-        if (e == hipSuccess && want != SMAT_KERNEL_ROWWISE_DIRECT &&
-            (gain_us > 1.5 * cost_us || want == SMAT_KERNEL_ROWWISE_PACKED))
-            e = dev_malloc(&p->d_bpack, K * n_hint * sizeof(uint16_t));
-    }
+    if (e == hipSuccess && want != SMAT_KERNEL_ROWWISE_DIRECT && (repack_pays(K, n_hint, nnzb) || want == SMAT_KERNEL_ROWWISE_PACKED))
+        e = dev_malloc(&p->d_bpack, K * n_hint * sizeof(uint16_t));
     p->panel_tiles = rowwise_panel_tiles(n_hint, items.size(), items.empty() ? 0 : nnzb / items.size(),
                                          split.empty() ? RowLengths::EVEN : RowLengths::SPLIT, p->d_bpack != nullptr);
     // The sweep kernel pays one pass over the B panel per group of 32 block rows,
@@ -722,9 +727,7 @@ static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
     // rows x panels of 128 columns) fill the 256 CUs, and loses (0.3x .. 0.9x) when they do not.
     if (e == hipSuccess && opts && opts->b_layout == SMAT_B_ROW_MAJOR) e = dev_malloc(&p->d_bcol, K * n_hint * sizeof(uint16_t));
     bool sweep = want == SMAT_KERNEL_SWEEP;
-    if (want == SMAT_KERNEL_AUTO && col_idx_host && cols_ascending && sweep_fills_device(mb, n_hint) &&
-        (double)nnzb >= 0.05 * (double)mb * (double)kb)
-        sweep = true;
+    if (want == SMAT_KERNEL_AUTO && col_idx_host && cols_ascending && sweep_from_the_start(mb, kb, n_hint, nnzb)) sweep = true;
     if (sweep && (nnzb >= (size_t)1 << 23 || nnzb < 2)) { // blocks are addressed in pairs, with 32-bit byte offsets
         if (want == SMAT_KERNEL_SWEEP)
             return set_error(SMAT_ERR_UNSUPPORTED, "SMAT_KERNEL_SWEEP takes between 2 and 2^23 - 1 nonzero blocks");
@@ -830,22 +833,40 @@ static hipError_t sweep_small_groups(smat_plan &p, size_t group_rows)
 // 14224 rows and 182, N = 544 33 -> 17, of 65536 and 20, N = 256 30 -> 15, of 8960 and 120, N = 48 7.4 -> 5.
 // census: of the values, where the compact kernel would multiply: the window kernel then multiplies what it would, the values as attached.
 // Whole blocks: does not wait for the lists, which launches on other streams than the default one may read.
+// Not where wavefronts share items, nor for narrow products: 18 -> 17, 10.4 -> 9.2, but 8.2 -> 9, 6.6 -> 7.
+static bool beside_rowwise(size_t N, size_t n_items, size_t nnzb)
+{
+    return window_forced() || (N > 16 && !rowwise_shares_items(N, n_items, nnzb / std::max<size_t>(n_items, 1)));
+}
+static double bytes_once_us(size_t M, size_t K, size_t N, double a_bytes) { return (a_bytes + 2.0 * (double)(K + M) * (double)N) / 5e6; }
+// The estimate of the row-wise kernel knows nothing of the bytes that come from memory, A above all and three times B where that is repacked: 64^3 64 us and
+// 64 us of bytes, measured 90; 73 x 61 x 62, N = 88 104 and 72, 125; 44 x 47 x 66, N = 40 31 and 26, 38.
+static double rowwise_from_memory_us(size_t M, size_t K, size_t N, size_t nnzb, size_t n_items, bool packed)
+{
+    return std::hypot(rowwise_estimate_us(M, K, N, nnzb, n_items, RowLengths::EVEN, packed),
+                      bytes_once_us(M, K, N, 512.0 * (double)nnzb) + (packed ? 4.0 * (double)K * (double)N / 5e6 : 0.0));
+}
+// Windows take a launch, or the bytes that they do not save.
+static double least_bar_us(double once) { return std::max(4.7, 2.0 + once); }
+// What take_window asks before it looks at the widths, of a drop-in call, before there is a plan.  (Counted all the same, first calls with random patterns, few of which get that
+// far, took 3 % longer in the mean.)
+bool smat::drop_in_may_take_window(size_t M, size_t K, size_t N, size_t nnzb, int most_blocks)
+{
+    const size_t mb = M / 16;
+    if (!window_takes_rows(most_blocks) || !beside_rowwise(N, mb, nnzb)) return false;
+    return window_forced() || (!sweep_from_the_start(mb, K / 16, N, nnzb) && 0.9 * rowwise_from_memory_us(M, K, N, nnzb, mb, repack_pays(K, N, nnzb)) >=
+                                                                                 least_bar_us(bytes_once_us(M, K, N, 512.0 * (double)nnzb)));
+}
 static bool may_take_window(const smat_plan &p) { return p.kernel_requested == SMAT_KERNEL_AUTO && !p.n_split_rows && window_takes_rows(p.max_item_blocks); }
 static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, WindowCount &count, double other_us, const uint16_t *vals, const CompactCensus *census)
 {
     const size_t mb = p.M / 16, kb = p.K / 16;
     if ((p.kernel != SMAT_KERNEL_ROWWISE && !(p.kernel == SMAT_KERNEL_SWEEP && p.sweep_few_tiles)) || !may_take_window(p)) return hipSuccess;
-    if (!census && rowwise_shares_items(p.n_cap, (size_t)p.n_items, p.nnzb / std::max<size_t>((size_t)p.n_items, 1)) && !window_forced()) return hipSuccess;
-    if (!census && p.n_cap <= 16 && !window_forced()) return hipSuccess; // 18 -> 17, 10.4 -> 9.2, but 8.2 -> 9, 6.6 -> 7
-    // its estimate knows nothing of the bytes that come from memory, A above all and three times B where that is repacked: 64^3 64 us and
-    // 64 us of bytes, measured 90; 73 x 61 x 62, N = 88 104 and 72, 125; 44 x 47 x 66, N = 40 31 and 26, 38
-    const double once = ((census ? 4.0 * (double)census->nnz + 12.0 * (double)p.nnzb : 512.0 * (double)p.nnzb) + 2.0 * (double)(p.K + p.M) * (double)p.n_cap) / 5e6;
-    const double row_wise = std::hypot(rowwise_estimate_us(p.M, p.K, p.n_cap, p.nnzb, (size_t)p.n_items, RowLengths::EVEN, p.d_bpack != nullptr),
-                                       once + (p.d_bpack ? 4.0 * (double)p.K * (double)p.n_cap / 5e6 : 0.0));
+    if (!census && !beside_rowwise(p.n_cap, (size_t)p.n_items, p.nnzb)) return hipSuccess;
+    const double once = bytes_once_us(p.M, p.K, p.n_cap, census ? 4.0 * (double)census->nnz + 12.0 * (double)p.nnzb : 512.0 * (double)p.nnzb);
     const double copy = p.d_bcol ? to_col_major_us(p.K, p.n_cap) : 0.0; // before either
-    const double bar = 0.9 * (census ? other_us - copy : std::min(row_wise, other_us));
-    // a launch, or the bytes that windows do not save
-    if (!window_forced() && bar < std::max(4.7, 2.0 + once)) return hipSuccess;
+    const double bar = 0.9 * (census ? other_us - copy : std::min(rowwise_from_memory_us(p.M, p.K, p.n_cap, p.nnzb, (size_t)p.n_items, p.d_bpack != nullptr), other_us));
+    if (!window_forced() && bar < least_bar_us(once)) return hipSuccess;
     hipError_t e = hipSuccess;
     if (!count.there && !count.begun && p.nnzb <= WindowCount::FEW && p.col_idx_host.size() == p.nnzb) count.on_host(p.row_ptr_host.data(), p.col_idx_host.data(), mb, kb);
     else e = count.end(row_ptr, col_idx, mb, kb, p.nnzb);

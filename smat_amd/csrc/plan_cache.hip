@@ -117,10 +117,11 @@ void build_entry(Entry &en, const uint16_t *vals, Mode mode)
     if (hipMemcpy(rp.data(), en.row_ptr, rp.size() * sizeof(int32_t), hipMemcpyDeviceToHost) != hipSuccess) return;
     if (en.nnzb && hipMemcpy(ci.data(), en.col_idx, ci.size() * sizeof(int32_t), hipMemcpyDeviceToHost) != hipSuccess) return;
     WindowCount count; // windows are weighed when the plan is there; until then the host has the checksum and the plan to do
-    if (mode == MODE_PATTERN && en.N > 16 && en.nnzb > WindowCount::FEW) {
+    if (mode == MODE_PATTERN && en.nnzb > WindowCount::FEW) {
         int32_t longest = 0;
         for (size_t i = 0; i < mb; i++) longest = std::max(longest, rp[i + 1] - rp[i]);
-        if (window_takes_rows(longest)) count.begin(static_cast<const int32_t *>(en.row_ptr), static_cast<const int32_t *>(en.col_idx), mb, en.K / 16, en.nnzb);
+        if (drop_in_may_take_window(en.M, en.K, en.N, en.nnzb, longest))
+            count.begin(static_cast<const int32_t *>(en.row_ptr), static_cast<const int32_t *>(en.col_idx), mb, en.K / 16, en.nnzb);
     }
     en.checksum = host_checksum(rp.data(), (long)rp.size(), ci.data(), (long)ci.size());
     smat_spmm_opts o = {SMAT_B_COL_MAJOR, SMAT_C_F16, SMAT_KERNEL_AUTO, 0, nullptr};

@@ -285,4 +285,5 @@ struct smat_plan;
 namespace smat {
 // A plan that has no better kernel than the row-wise one gets windows where they are faster (row_ptr / col_idx: device arrays).  Does not wait, as window_build.
 hipError_t plan_take_window(smat_plan *p, const int32_t *row_ptr, const int32_t *col_idx, WindowCount &count);
+bool drop_in_may_take_window(size_t M, size_t K, size_t N, size_t nnzb, int most_blocks); // whether it may, as far as sizes tell
 } // namespace smat
