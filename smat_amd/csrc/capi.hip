@@ -857,6 +857,11 @@ bool smat::drop_in_may_take_window(size_t M, size_t K, size_t N, size_t nnzb, in
     return window_forced() || (!sweep_from_the_start(mb, K / 16, N, nnzb) && 0.9 * rowwise_from_memory_us(M, K, N, nnzb, mb, repack_pays(K, N, nnzb)) >=
                                                                                  least_bar_us(bytes_once_us(M, K, N, 512.0 * (double)nnzb)));
 }
+// Test hook (not part of smat.h): the same.
+extern "C" int smat_internal_drop_in_may_take_window(size_t M, size_t K, size_t N, size_t nnzb, int most_blocks)
+{
+    return drop_in_may_take_window(M, K, N, nnzb, most_blocks);
+}
 static bool may_take_window(const smat_plan &p) { return p.kernel_requested == SMAT_KERNEL_AUTO && !p.n_split_rows && window_takes_rows(p.max_item_blocks); }
 static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_t *col_idx, WindowCount &count, double other_us, const uint16_t *vals, const CompactCensus *census)
 {
