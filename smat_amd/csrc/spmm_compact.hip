@@ -34,6 +34,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 #include <vector>
@@ -55,6 +56,7 @@ int g_tune = 1; // test hook: 0 = attaching values measures nothing, the estimat
 int g_last_run = 0; // test hook: the run length of the latest launch
 int g_force_list = 0; // test hook: 1 = lists of whole columns, 2 = of nonzeros, 0 = compact_build decides
 int g_force_staged = 0; // test hook: 1 = entries go through LDS in blocks wherever they may, 2 = nowhere, 0 = the launcher decides
+int g_force_order = 0; // test hook: 1 = tasks of lists with split rows in the order of their items, 0 = order_tasks
 int g_force_tq = 0; // test hook: 1 or 2 = panels of 64 or 128 columns whatever the sizes say, 0 = the launcher decides
 
 constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts as full (of 16)
@@ -562,6 +564,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const int panel = __builtin_amdgcn_readfirstlane((int)(w / n_tasks));
     const int task = __builtin_amdgcn_readfirstlane((int)(w - (long)panel * n_tasks));
     const int4 tk = tasks[task]; // first item, items (at most 64), first and last column of the stream
+    if (tk.y == 0) return;       // a place that order_tasks left empty
     int e = tk.z;
     const int e_last = tk.w;
     // Scalar loads share a counter with the LDS operations below, which would wait for them at every step: the items of
@@ -836,6 +839,7 @@ hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
     if (wgs == 0) return hipSuccess;
     long xcd_run = p.deal.run((size_t)p.n_tasks, n_panels);
     if (p.tuned_run > 0 && p.tuned_n == a.N) xcd_run = p.tuned_run;
+    if (p.ordered) xcd_run = 1;
     if (a.xcd_run > 0) xcd_run = a.xcd_run;
     if (g_force_run > 0) xcd_run = g_force_run;
     xcd_run = std::min<long>((wgs + 7) / 8, xcd_run);
@@ -928,7 +932,7 @@ hipError_t compact_tune(CompactPlan &p, uint16_t *Bt, size_t M, size_t N, size_t
 {
     p.tuned_n = 0;
     p.tuned_run = 0;
-    if (!g_tune || p.n_items == 0 || N == 0 || !Bt) return hipSuccess;
+    if (!g_tune || p.n_items == 0 || N == 0 || !Bt || p.ordered) return hipSuccess;
     // Timed as a program launches it, the transposition of a column-major B included: the copy is written over what the
     // launch before left in the L2s, and how many of them hold a line of it follows from the deal (16384^2, 0.1 %, N = 256: the
     // product kernel alone is fastest in runs of 128, 10.9 against 11.9 us; launch after launch it is 64, 19.8 against 21.4.
@@ -994,7 +998,7 @@ void compact_deal_beside_windows(CompactPlan &p, size_t N, size_t K)
 {
     const int width = compact_panel_width(p, N, K, false), n_panels = (int)((N + width - 1) / width);
     const unsigned eighth = (unsigned)((((long)p.n_tasks * n_panels + 3) / 4 + 7) / 8);
-    if (n_panels < 2 || eighth < 8 || p.deal.run((size_t)p.n_tasks, n_panels) < eighth) return;
+    if (p.ordered || n_panels < 2 || eighth < 8 || p.deal.run((size_t)p.n_tasks, n_panels) < eighth) return;
     p.tuned_n = N;
     p.tuned_run = eighth / (n_panels % 4 ? 2 : 4);
 }
@@ -1194,6 +1198,70 @@ static long split_chunk_steps(long steps, size_t rows, long longest, size_t n_ca
     return chunk;
 }
 
+// The order of the tasks of a list with split rows, which is skewed, and the XCD of each: workgroup i, tasks 4 i .. 4 i + 3, runs on XCD i % 8.
+//
+// Bound by the lines that the L2s miss: 128-byte rows at random out of 67 MiB come at 7.2 TB/s however many wavefronts ask (220 lines per us and CU, with
+// 2 MiB 750), and in the order of the block rows a product of R-MAT scale 20 moved 6.6 TB/s.  Long rows list their columns in ascending order, so
+//   * a chunk of a split row goes to the XCD of the eighth of its row that it begins in: an XCD gathers from an eighth of B for the chunks of all rows, and those
+//     that run at the same time from about the same part of it;
+//   * whole rows come by classes of length, the longest first: what runs at the same time advances through B at about the same pace.  256 tasks of a class,
+//     or what is a 256th of the launch, go to the XCD that has least to do so far, which makes the XCDs even where runs of the deal left up to 4 %.  Inside
+//     a class rows keep their order.
+// A model of the caches finds 67 % of what is asked for in them, 55 % in the order before, 61 with exact lengths in runs of 16 tasks, 73 with rows from 1000 columns on cut
+// in eighths too, whose partial tiles would be ten times as many.  In the order of the block rows -> so, us: R-MAT scale 20, 16 a row, N = 128 456 -> 428, row-major 449 -> 377, N =
+// 64 228 -> 190; 18, 22 a row, N = 64, row-major 63 -> 55; 18, 16, N = 128 111 -> 107; 15, 16, N = 256 33.6 -> 31.3; 15, N = 24, 14, 13 and 12 within 1 %.
+// Classes are octaves; two of them where a column-major B has more than two panels (18, 10 a row, N = 256 159.1, with octaves 161.9, with two 157.9; 19, 22 a row, N = 200 513, 513,
+// 517; with two panels or fewer two octaves are 1 to 5 % slower).
+static void order_tasks(std::vector<int4> &tasks, std::vector<uint32_t> &costs, const std::vector<WorkItem> &items, const std::vector<int32_t> &row_first, int octaves)
+{
+    struct Task {
+        int4 t;
+        uint32_t cost;
+        double key; // chunk: where it begins in its row; whole rows: class
+    };
+    std::vector<Task> chunks, whole;
+    uint64_t total = 0, total_chunks = 0;
+    for (size_t i = 0; i < tasks.size(); i++) {
+        const WorkItem &w = items[(size_t)tasks[i].x];
+        total += costs[i];
+        if (w.dst >= 0) {
+            const double from = row_first[(size_t)w.block_row], to = row_first[(size_t)w.block_row + 1];
+            chunks.push_back(Task{tasks[i], costs[i], ((double)w.begin - from) / (to - from)});
+            total_chunks += costs[i];
+        } else {
+            whole.push_back(Task{tasks[i], costs[i], (double)(std::ilogb((double)costs[i]) / octaves)});
+        }
+    }
+    std::stable_sort(chunks.begin(), chunks.end(), [](const Task &a, const Task &b) { return a.key < b.key; });
+    std::stable_sort(whole.begin(), whole.end(), [](const Task &a, const Task &b) { return a.key > b.key; });
+    std::vector<Task> queue[8];
+    uint64_t load[8] = {};
+    auto put = [&](int x, const Task &t) { queue[x].push_back(t); load[x] += t.cost; };
+    uint64_t before = 0;
+    for (const Task &t : chunks) {
+        put((int)std::min<uint64_t>(7, before * 8 / total_chunks), t);
+        before += t.cost;
+    }
+    for (size_t i = 0; i < whole.size();) {
+        const int x = (int)(std::min_element(load, load + 8) - load);
+        uint64_t piece = 0;
+        for (size_t n = 0; i < whole.size() && n < 256 && (n % 4 || n == 0 || piece * 256 < total); n++, i++) {
+            piece += whole[i].cost;
+            put(x, whole[i]);
+        }
+    }
+    size_t rounds = 0; // of a workgroup an XCD; places past the end of a queue stay empty
+    for (const auto &q : queue) rounds = std::max(rounds, (q.size() + 3) / 4);
+    tasks.assign(rounds * 32, int4{0, 0, 0, 0});
+    costs.assign(rounds * 32, 0);
+    for (int x = 0; x < 8; x++)
+        for (size_t i = 0; i < queue[x].size(); i++) {
+            const size_t at = (i / 4 * 8 + (size_t)x) * 4 + i % 4;
+            tasks[at] = queue[x][i].t;
+            costs[at] = queue[x][i].cost;
+        }
+}
+
 hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx, size_t K, size_t n_cap,
                          bool b_row_major, const std::vector<uint8_t> *leave_rows, bool drop_full, CompactPlan **out)
 {
@@ -1373,7 +1441,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     // and one per item for the stores of its tile.
     const long task_steps = std::min<long>(TASK_STEPS, (long)(total / 32 * (int64_t)((n_cap + 63) / 64) / 7168));
     std::vector<int4> tasks;
-    std::vector<uint64_t> cost_prefix(1, 0);
+    std::vector<uint32_t> costs;
     for (size_t i = 0; i < items.size();) {
         size_t j = i + 1;
         long steps = (items[i].end - items[i].begin) / 32;
@@ -1383,9 +1451,13 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
             j++;
         }
         tasks.push_back(int4{(int)i, (int)(j - i), items[i].begin, items[j - 1].end});
-        cost_prefix.push_back(cost_prefix.back() + (uint64_t)steps + 2 + (uint64_t)(j - i));
+        costs.push_back((uint32_t)steps + 2 + (uint32_t)(j - i));
         i = j;
     }
+    p->ordered = !split.empty() && g_force_order != 1;
+    if (p->ordered) order_tasks(tasks, costs, items, cc_host, n_cap > 128 && !b_row_major ? 2 : 1);
+    std::vector<uint64_t> cost_prefix(costs.size() + 1, 0);
+    for (size_t i = 0; i < costs.size(); i++) cost_prefix[i + 1] = cost_prefix[i] + costs[i];
     p->deal.set_costs(std::move(cost_prefix));
     p->n_items = (int)items.size();
     p->n_tasks = (int)tasks.size();
@@ -1428,6 +1500,8 @@ extern "C" void smat_internal_compact_panel(int tq) { smat::g_force_tq = tq; }
 extern "C" void smat_internal_compact_list(int what) { smat::g_force_list = what; }
 // Test hook: 1 = entries go through LDS in blocks of 256 wherever they may, 2 = nowhere, 0 = as the sizes say (the default).
 extern "C" void smat_internal_compact_staged(int what) { smat::g_force_staged = what; }
+// Test hook: 1 = tasks of lists with split rows in the order of their items, 0 = as order_tasks says (the default).
+extern "C" void smat_internal_compact_order(int what) { smat::g_force_order = what; }
 // Test hook (host only): steps of the chunks of split rows.
 extern "C" long smat_internal_compact_chunk(long steps, size_t rows, long longest, size_t n_cap) { return smat::split_chunk_steps(steps, rows, longest, n_cap); }
 // Test hooks for the deal of the compact kernel's workgroups to the XCDs: a run length that every launch uses

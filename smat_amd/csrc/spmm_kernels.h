@@ -108,6 +108,7 @@ struct CompactPlan {
     SplitRow *d_split = nullptr;
     float *d_workspace = nullptr; // n_slots * 16 * n_cap floats
     int n_items = 0, n_tasks = 0, n_split_rows = 0, n_slots = 0;
+    bool ordered = false;         // the tasks lie as order_tasks deals them: workgroup i to XCD i % 8
     int64_t n_steps = 0;          // of 32 columns, of all block rows listed
     int64_t n_cols = 0;           // nonzero block columns listed (without padding)
     int64_t n_entries = 0;        // nonzeros listed one by one
