@@ -20,6 +20,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "row_tile.h"
 #include "spmm_kernels.h"
@@ -146,27 +147,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
         issue(0, a0, b0);
         SMAT_ORDER_FENCE();
         int j = 0;
-        for (; j + 2 <= npair; j += 2) {
+        for (; j + 2 < npair; j += 2) {
             issue(j + 1, a1, b1);
             SMAT_ORDER_FENCE();
             multiply(j, a0, b0);
             SMAT_ORDER_FENCE();
-            issue(j + 2, a0, b0); // past the end this reloads the last pair, unused
+            issue(j + 2, a0, b0);
             SMAT_ORDER_FENCE();
             multiply(j + 1, a1, b1);
             SMAT_ORDER_FENCE();
         }
-        if (j < npair) multiply(j, a0, b0); // odd number of pairs: the last one is already in set 0
+        if (j + 1 < npair) { // two are left: nothing is asked for beyond them
+            issue(j + 1, a1, b1);
+            SMAT_ORDER_FENCE();
+            multiply(j, a0, b0);
+            SMAT_ORDER_FENCE();
+            multiply(j + 1, a1, b1);
+        } else {
+            multiply(j, a0, b0);
+        }
     }
 
     store_tile<TN, C_F32>(acc, br, dst, n0, i16, g, Cout, workspace, N);
 }
 
 // Launches of few (item, panel) pairs with long items: the four wavefronts of a workgroup share one, each takes a run of
-// the item's block pairs with the operands of NP pairs in flight, and the partial tiles are added in LDS in the order of
-// the runs.  Bound by the chain item -> column indices -> operands of a wavefront and by too few of them: 8192^2 with 10 %
-// of the blocks and N = 16 (512 items) takes 6.6 us where one wavefront per item takes 9.1; 1024 x 8192 with 30 % and
-// N = 64 (64 items of 154 blocks) 13.8 against 39.8.  Eight wavefronts per item are no faster than four.
+// the item's block pairs, NP of them in flight, and the partial tiles are added in LDS in the order of the runs.
+// Bound by the loads of B in place, whose 64 lanes ask for 32 pieces of 32 bytes: 53 clocks of a CU each, whatever is in flight (8192^2 with
+// 10 % of the blocks, N = 16: 1.7 us a launch, 4.7 with the loads of A, 6.1 with those of B).  So no load is made for nothing: what is left of a run has code
+// of its own length, where the last pair was asked for again up to NP times (same bits, us): that matrix 6.66 -> 6.1, 1184 x 5264, 27 %, N = 80 10.2 -> 8.2, 976 x
+// 16096, 36 %, N = 32 17.8 -> 13.9, 2896 x 14064, 30 %, N = 32 15.2 -> 12.2.  Three to twelve pairs in flight are level, and so are eight wavefronts (5.9 to 6.1 us
+// on the first); sixteen lose 20 to 40 % at N = 64.
 template <int TN, bool C_F32, bool PACKED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void spmm_rowwise_split_kernel(
     const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_idx,
@@ -174,7 +185,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
     int n_items, int N, long K, int n_panels)
 {
     constexpr int SPLIT = 4, PANEL = 16 * TN;
-    constexpr int NP = TN <= 2 ? 4 : 3;
+    constexpr int NP = 4;
     __shared__ f32x4 part[SPLIT][TN][64];
     const int lane = threadIdx.x & 63;
     const int run = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -216,30 +227,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
             const int first = p0 + 2 * jw, last = p1 - 1;
             const int myc = col_idx[first + lane < last ? first + lane : last];
             const int jend = jw + 32 < j1 ? jw + 32 : j1;
-            auto blocks = [&](int j, int &q0, int &q1) {
-                const int jj = j < jend ? j : jend - 1; // past the end: the last pair again, not used
-                q0 = p0 + 2 * jj;
-                q1 = q0 < last ? q0 + 1 : q0; // a single block pairs with itself
-            };
-            auto multiply = [&](int j, f16x8 a, const f16x8 (&b)[TN]) {
-                const bool past = j >= jend; // zeros times zeros: an Inf or NaN in the B of the last pair must not meet a zero
-                a = past || (sel && p0 + 2 * j >= last) ? zero8 : a; // single block: the upper K half contributes nothing
+            // the operands of R pairs at once, as many as there are
+            auto pairs = [&](int j, auto count) {
+                constexpr int R = decltype(count)::value;
+                f16x8 a[R], b[R][TN];
 #pragma unroll
-                for (int t = 0; t < TN; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(past ? zero8 : b[t], a, acc[t], 0, 0, 0);
-            };
-            for (int j = jw; j < jend; j += NP) { // the operands of NP pairs at once; a run is seldom more than one batch
-                f16x8 a[NP], b[NP][TN];
-#pragma unroll
-                for (int u = 0; u < NP; u++) { // the values first: they do not wait for the column indices
-                    int q0, q1;
-                    blocks(j + u, q0, q1);
+                for (int u = 0; u < R; u++) { // the values first: they do not wait for the column indices
+                    const int q0 = p0 + 2 * (j + u), q1 = q0 < last ? q0 + 1 : q0; // a single block pairs with itself
                     a[u] = load_f16x8(abase + (long)(sel ? q1 : q0) * 256);
                 }
                 SMAT_ORDER_FENCE();
 #pragma unroll
-                for (int u = 0; u < NP; u++) {
-                    int q0, q1;
-                    blocks(j + u, q0, q1);
+                for (int u = 0; u < R; u++) {
+                    const int q0 = p0 + 2 * (j + u), q1 = q0 < last ? q0 + 1 : q0;
                     const int c0 = __builtin_amdgcn_readlane(myc, q0 - first), c1 = __builtin_amdgcn_readlane(myc, q1 - first);
                     const int bc = sel ? c1 : c0;
                     const long boffs = PACKED ? (long)bc * N : (long)bc;
@@ -248,8 +248,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
                 }
                 SMAT_ORDER_FENCE();
 #pragma unroll
-                for (int u = 0; u < NP; u++) multiply(j + u, a[u], b[u]);
-            }
+                for (int u = 0; u < R; u++) {
+                    const f16x8 au = sel && p0 + 2 * (j + u) >= last ? zero8 : a[u]; // single block: the upper K half contributes nothing
+#pragma unroll
+                    for (int t = 0; t < TN; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[u][t], au, acc[t], 0, 0, 0);
+                }
+            };
+            using std::integral_constant;
+            int j = jw;
+            for (; j + NP <= jend; j += NP) pairs(j, integral_constant<int, NP>{});
+            if (jend - j == 3) pairs(j, integral_constant<int, 3>{});
+            else if (jend - j == 2) pairs(j, integral_constant<int, 2>{});
+            else if (jend - j == 1) pairs(j, integral_constant<int, 1>{});
         }
     }
     if (run > 0)
@@ -267,8 +277,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
 // Small problems with short block rows (a band matrix: 9 blocks per row, 256 rows): the kernel above keeps the
 // operands of two block pairs in flight, so a row of five pairs costs four memory latencies one after the other
 // and the launch is over before the chip is busy.  Here a wavefront asks for the operands of all its pairs
-// (at most NP) at once: work item -> column indices -> operands, three latencies, then NP x TN MFMAs (pairs past
-// the end of the row are zeros times zeros).  Whole block rows only (dst < 0), B in place.
+// (at most NP) at once: work item -> column indices -> operands, three latencies, then the MFMAs.  As in the kernel above the loads of B are what a CU does
+// most of the time, so rows of fewer pairs have code of their own instead of loads for NP (band of 2208 rows and 12, N = 536: 6.13 -> 4.78 us, of 5328, N = 256
+// 6.24 -> 5.05).  Whole block rows only (dst < 0), B in place.
 template <int TN, bool C_F32, int NP>
 __global__ __launch_bounds__(256) void spmm_rowwise_short_kernel(
     const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_idx,
@@ -311,27 +322,39 @@ __global__ __launch_bounds__(256) void spmm_rowwise_short_kernel(
         const uint16_t *abase = vals + i16 * 16 + kh * 8;
         const f16x8 zero8 = zero_f16x8();
         const int myc = col_idx[p0 + (lane < cnt ? lane : cnt - 1)];
-        f16x8 a[NP], b[NP][TN];
+        auto pairs = [&](auto count) {
+            constexpr int R = decltype(count)::value;
+            f16x8 a[R], b[R][TN];
+            const int last = cnt - 1;
 #pragma unroll
-        for (int j = 0; j < NP; j++) {
-            const int jj = j < npair ? j : npair - 1; // past the end: the last pair again, not used
-            const int second = (2 * jj + 1 < cnt) ? 2 * jj + 1 : 2 * jj; // a single block pairs with itself
-            const int c0 = __builtin_amdgcn_readlane(myc, 2 * jj);
-            const int c1 = __builtin_amdgcn_readlane(myc, second);
-            const long pp = (long)p0 + (sel ? second : 2 * jj);
-            a[j] = load_f16x8(abase + pp * 256);
-            const long bc = sel ? c1 : c0;
+            for (int u = 0; u < R; u++) { // the values first: they do not wait for the column indices
+                const int second = u < R - 1 ? 2 * u + 1 : last; // a single block pairs with itself
+                a[u] = load_f16x8(abase + ((long)p0 + (sel ? second : 2 * u)) * 256);
+            }
+            SMAT_ORDER_FENCE();
 #pragma unroll
-            for (int t = 0; t < TN; t++) b[j][t] = load_f16x8(B + boff[t] + bc);
-        }
-        SMAT_ORDER_FENCE();
+            for (int u = 0; u < R; u++) {
+                const int c0 = __builtin_amdgcn_readlane(myc, 2 * u), c1 = __builtin_amdgcn_readlane(myc, u < R - 1 ? 2 * u + 1 : last);
+                const long bc = sel ? c1 : c0;
 #pragma unroll
-        for (int j = 0; j < NP; j++) {
-            f16x8 aj = a[j];
-            const bool past = j >= npair; // zeros times zeros: an Inf or NaN in the B of the last pair must not meet a zero
-            aj = past || (sel && 2 * j + 1 >= cnt) ? zero8 : aj; // single block: the upper K half contributes nothing
+                for (int t = 0; t < TN; t++) b[u][t] = load_f16x8(B + boff[t] + bc);
+            }
+            SMAT_ORDER_FENCE();
 #pragma unroll
-            for (int t = 0; t < TN; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(past ? zero8 : b[j][t], aj, acc[t], 0, 0, 0);
+            for (int u = 0; u < R; u++) {
+                const f16x8 au = u == R - 1 && sel && 2 * u == last ? zero8 : a[u]; // single block: the upper K half contributes nothing
+#pragma unroll
+                for (int t = 0; t < TN; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[u][t], au, acc[t], 0, 0, 0);
+            }
+        };
+        static_assert(NP == 5, "a case for each number of pairs");
+        using std::integral_constant;
+        switch (npair) { // uniform over the wavefront
+        case 1: pairs(integral_constant<int, 1>{}); break;
+        case 2: pairs(integral_constant<int, 2>{}); break;
+        case 3: pairs(integral_constant<int, 3>{}); break;
+        case 4: pairs(integral_constant<int, 4>{}); break;
+        default: pairs(integral_constant<int, 5>{}); break;
         }
     }
     // acc[t][r] = C[br*16 + i16][n0 + ncol_of(t, 4*g + r)]: 4*TN consecutive columns per lane, as in the kernel above
