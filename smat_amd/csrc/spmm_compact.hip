@@ -520,8 +520,6 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 //   * The loop ends at its bottom only.  A way out of its middle is turned into one that seems to lead from the first step
 //     back to the first, where the registers of the second still seem to be waited for: every other step waited for operands
 //     before it asked for the next ones.  A task that ends with the first step ends there with s_endpgm.
-//   * LDS for four workgroups a CU (W = 64): with five, which the registers now allow, the gathers of R-MAT scale 20 lose 0.6 %
-//     and 16384^2 2 % (three: 16384^2 11 %).
 //
 // Entries (AF > 0) come from memory in the step before they are needed, 256 bytes a load, or, STAGED, 256 at a time ahead of
 // that, one load of 1 KiB to LDS: a load of 256 bytes takes the vector memory path as long as one of 1 KiB, and a list that
@@ -538,6 +536,8 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 //   8192 x 32768, 60 a row, N = 512 56.5/54.8  40.3/41.0   41.5/43.1   41.6/43.1
 // The launcher's rule is at STAGED_STEPS.  A block asked for on every second step, which makes all waits exact, is slower than one
 // asked for when it is needed (R-MAT scale 20 461 -> 477).
+// LDS of a wavefront.  W = 64: for sixteen a CU; with more the gathers of R-MAT scale 20 lose 0.6 % and 16384^2 2 % (twelve: 16384^2 11 %).
+constexpr int compact_lds_bytes(int W, bool staged) { return W == 64 ? 10240 : 1024 + 64 * W + 2048 + (staged ? 2048 : 0); }
 template <int W, bool C_F32, bool C_ACC, int AF, bool STAGED, bool BIG>
 __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const uint16_t *__restrict__ acol, const uint32_t *__restrict__ entries, const int2 *__restrict__ step_range, const int32_t *__restrict__ cols,
@@ -545,11 +545,13 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const int4 *__restrict__ tasks, int n_tasks, int N, int n_panels, long panel_stride, long row_stride, unsigned xcd_run)
 {
     constexpr int TQ = W > 64 ? 2 : 1, PW = W / TQ, T = PW / 16; // a row of PW columns is gathered by PW / 8 lanes, 32 rows by T instructions
-    constexpr int A_BYTES = 1024, B_BYTES = 64 * W, I_BYTES = 2048, E_BYTES = STAGED ? 2048 : 0, UNUSED_BYTES = W == 64 ? 2048 - E_BYTES : 0;
-    static_assert((A_BYTES + B_BYTES + I_BYTES + E_BYTES + UNUSED_BYTES) % 1024 == 0, "entries hold offsets that are or-ed to the address of the A tile");
-    __shared__ __align__(1024) unsigned char lds[4][A_BYTES + B_BYTES + I_BYTES + E_BYTES + UNUSED_BYTES];
+    constexpr int A_BYTES = 1024, B_BYTES = 64 * W, I_BYTES = 2048;
+    static_assert(compact_lds_bytes(W, STAGED) >= A_BYTES + B_BYTES + I_BYTES + (STAGED ? 2048 : 0), "the tiles of a wavefront");
+    static_assert(compact_lds_bytes(W, STAGED) % 1024 == 0, "entries hold offsets that are or-ed to the address of the A tile");
+    extern __shared__ __align__(1024) unsigned char lds_of_workgroup[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned char *const lds = lds_of_workgroup + wave * compact_lds_bytes(W, STAGED);
     // Panel-major order of the (panel, task) space.  An XCD gets the workgroup ids that are equal modulo 8, whatever
     // their work costs; here the XCDs take runs of xcd_run consecutive workgroups of that order in turn (gridDim.x is a
     // multiple of 8 * xcd_run).  One run per XCD keeps neighbouring block rows, which share rows of B, on one L2;
@@ -559,7 +561,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const unsigned slot = blockIdx.x >> 3;
     const unsigned run = __builtin_amdgcn_readfirstlane(slot / xcd_run);
     const long wg = ((long)run * 8 + (blockIdx.x & 7)) * xcd_run + (slot - run * xcd_run);
-    const long w = wg * 4 + wave;
+    const long w = wg * (blockDim.x >> 6) + wave;
     if (w >= total) return;
     const int panel = __builtin_amdgcn_readfirstlane((int)(w / n_tasks));
     const int task = __builtin_amdgcn_readfirstlane((int)(w - (long)panel * n_tasks));
@@ -587,7 +589,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
 #pragma unroll
     for (int q = 0; q < TQ; q++) boff[q] = n0 + 64 * q + 8 * (lane % (PW / 8)) < N ? 64 * q + 8 * (lane % (PW / 8)) : 0;
 
-    unsigned char *const a_tile = lds[wave], *const b_tile = lds[wave] + A_BYTES;
+    unsigned char *const a_tile = lds, *const b_tile = lds + A_BYTES;
     const uint32_t a_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)a_tile; // a multiple of 1024
     // lane -> places first_place + j, j < T, of the step's 32 in the list, which are entries 8 (place / 8) + 2 (place % 4) + (place / 4) % 2
     const int c8 = lane % (PW / 8), first_place = T * (lane / (PW / 8));
@@ -621,7 +623,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     }
     // The indices of 8 steps are 1 KiB, one load, and go to one half of 2 KiB of LDS, from where each lane takes the four of
     // its octet (an instruction that brings 128 bytes costs the vector memory path as much as one that brings 1 KiB).
-    unsigned char *const i_tile = lds[wave] + A_BYTES + B_BYTES;
+    unsigned char *const i_tile = lds + A_BYTES + B_BYTES;
     auto load_block = [&](int s) { return reinterpret_cast<const u32x4 *>(cols + s)[lane]; };
     auto put_block = [&](int s, u32x4 x) { *reinterpret_cast<u32x4 *>(i_tile + (((s >> 5) - first_step) & 8) * 128 + lane * 16) = x; };
     typedef uint32_t Indices __attribute__((ext_vector_type(T)));
@@ -632,7 +634,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     // steps make is zero where its registers are copied.  Waited for so -> as here: stencil 64^3, N = 64 53.3 -> 52.8 us with inputs from
     // HBM, 40.6 -> 39.5 with the same ones again; N = 128 97 -> 94; 48^3, N = 256 78 -> 74; R-MAT scale 20, N = 128 461.7 -> 458.4;
     // 65536^2, 40 a row, N = 192 101.7 -> 102.9.)
-    unsigned char *const e_tile = lds[wave] + A_BYTES + B_BYTES + I_BYTES;
+    unsigned char *const e_tile = lds + A_BYTES + B_BYTES + I_BYTES;
     u32x4 e_next = {0u, 0u, 0u, 0u};
     int e_block = 0, e_end = 0; // of 256 entries: the one in e_next, and the last of the task as far as its ranges are here
     auto load_entries = [&](int b) { return reinterpret_cast<const u32x4 *>(entries)[(long)b * 64 + lane]; };
@@ -844,6 +846,12 @@ hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
     if (g_force_run > 0) xcd_run = g_force_run;
     xcd_run = std::min<long>((wgs + 7) / 8, xcd_run);
     g_last_run = (int)xcd_run;
+    // A workgroup of four tasks keeps its place until the longest is done; one task each is up to 12 % faster (4864 x 6496, 12 % of full blocks and 15 more a row, N =
+    // 400 30.5 -> 26.6 us, 40000 x 60000, 10 a row, N = 64, row-major 9.7 -> 9.3, R-MAT scale 18, N = 64 63.9 -> 62.7).  Where a place has many steps to do the end of a launch
+    // matters less than the lines that neighbouring tasks find of each other's in their L1: four (R-MAT scale 20, N = 128, row-major 366, one each 378; 19, N = 256 362 and 365, 40000 x 60000, 30 a row, N = 256 73.8 and 74.6).
+    const int waves = (double)p.n_steps * n_panels >= 32.0 * 16.0 * 256.0 ? 4 : 1;
+    xcd_run *= 4 / waves;
+    wgs = (total + waves - 1) / waves;
     wgs = (wgs + 8 * xcd_run - 1) / (8 * xcd_run) * (8 * xcd_run);
     if (wgs > 0x7fffffffL) return hipErrorInvalidValue;
     if (a.accumulate && p.n_split_rows > 0) return hipErrorInvalidValue; // partial tiles through the workspace overwrite C
@@ -851,7 +859,7 @@ hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
     const bool big = a.K > ((size_t)1 << 24) || a.K * (size_t)row_stride * 2 >= ((size_t)1 << 32) || row_stride >= (1L << 23);
     auto launch = [&](auto af, auto staged, auto f32, auto acc, auto wide) {
         hipLaunchKernelGGL((spmm_compact_kernel<W, decltype(f32)::value, decltype(acc)::value, decltype(af)::value, decltype(staged)::value, decltype(wide)::value>),
-                           dim3((unsigned)wgs), dim3(256), 0, st, p.d_acol, p.d_entries, p.d_step_range, cols, a.Bt, a.C, p.d_workspace,
+                           dim3((unsigned)wgs), dim3(64 * waves), (size_t)(waves * compact_lds_bytes(W, decltype(staged)::value)), st, p.d_acol, p.d_entries, p.d_step_range, cols, a.Bt, a.C, p.d_workspace,
                            p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, (unsigned)xcd_run);
     };
     using std::false_type;

@@ -31,7 +31,7 @@ struct SplitRow {
 
 // How a launch over a work list deals its workgroups to the eight XCDs.  The dispatcher gives an XCD the workgroup
 // ids that are equal modulo 8, whatever their work costs; the row-wise and the compact kernel lay the panel-major
-// (panel, item) space (4 items per workgroup) out in runs of consecutive workgroups that the XCDs take in turn.
+// (panel, item) space out in runs of consecutive workgroups, counted as if of 4 items each, that the XCDs take in turn.
 // One run per XCD keeps neighbouring block rows, which share rows of B, on one L2; short runs even out a list whose
 // cost per item changes along it.
 // choose_xcd_run: the longest run among {an eighth of the launch, 1024, 256, 64, 16, 4} that keeps the estimated load

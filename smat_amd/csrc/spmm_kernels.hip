@@ -39,13 +39,15 @@ __device__ __forceinline__ f16x8 zero_f16x8()
     return z;
 }
 
-// One wavefront per work item x N panel.  blockDim = 256 (4 wavefronts).
+// One wavefront per work item x N panel, a workgroup of its own: workgroups of four kept their places until the longest of four items was done, and the last
+// round of a launch had fewer of them than there are compute units.  Workgroups of four -> of one, us (120 products of random blocks, in place and repacked, are 10 and 4 % faster
+// in the mean and 6 % slower at most, those of 6 us): 8272 x 4176, 32 %, N = 72 39.9 -> 28.4, 5680 x 9936, 15 %, N = 136 48.9 -> 34.8, repacked 23.8 -> 20.5; 8368 x
+// 2736, 32 %, N = 48 15.8 -> 11.6; 27-point stencil of 78944 rows, N = 128 27.8 -> 23.8.  (The short-row kernel keeps workgroups of four: bands of few rows, N = 968 4.96, of one 6.20.)
 //   items == nullptr : item w is the whole block row w (no work list)
 //   items != nullptr : items[w] = {block row, first block, end block, dst}
 //                      dst < 0  -> write the finished tile to C
 //                      dst >= 0 -> write the fp32 partial tile to workspace slot dst
-// Item index runs fastest inside a panel, so the four wavefronts of a workgroup
-// and neighbouring workgroups share one B panel (K x 16*TN) in L2.  Workgroup
+// Item index runs fastest inside a panel, so neighbouring workgroups share one B panel (K x 16*TN) in L2.  Workgroup
 // ids are dealt round-robin to the 8 XCDs by the dispatcher; the remap below
 // gives the XCDs runs of xcd_run consecutive workgroups of the (panel-major) item
 // space in turn: an eighth of the launch each, so that an XCD's private L2 holds few
@@ -59,22 +61,18 @@ __device__ __forceinline__ f16x8 zero_f16x8()
 // the 16 x 16 operand of one (block column, n-tile) is 512 contiguous bytes and a
 // wavefront load touches 8 full cache lines instead of 32 quarter-used ones.
 template <int TN, bool C_F32, bool PACKED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void spmm_rowwise_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 4))) void spmm_rowwise_kernel(
     const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr,
     const int32_t *__restrict__ col_idx, const uint16_t *__restrict__ B, void *__restrict__ Cout,
     float *__restrict__ workspace, const WorkItem *__restrict__ items, int n_items, int N, long K,
     int n_panels, unsigned xcd_run)
 {
     constexpr int PANEL = 16 * TN;
-    const int lane = threadIdx.x & 63;
-    // wavefront-uniform values are forced into scalar registers
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-
+    const int lane = threadIdx.x;
     const long total = (long)n_items * n_panels;
     const unsigned slot = blockIdx.x >> 3;
-    const unsigned run = __builtin_amdgcn_readfirstlane(slot / xcd_run);
-    const long wg = ((long)run * 8 + (blockIdx.x & 7)) * xcd_run + (slot - run * xcd_run);
-    const long w = wg * 4 + wave;
+    const unsigned run = __builtin_amdgcn_readfirstlane(slot / xcd_run); // wavefront-uniform values are forced into scalar registers
+    const long w = ((long)run * 8 + (blockIdx.x & 7)) * xcd_run + (slot - run * xcd_run);
     if (w >= total) return;
     const int panel = (int)(w / n_items);
     const int it = (int)(w - (long)panel * n_items);
@@ -454,12 +452,11 @@ static hipError_t launch_rowwise_tn(const SpmmArgs &a, hipStream_t st)
     const int panel = 16 * TN;
     const int n_panels = (int)((a.N + panel - 1) / panel);
     const long total = (long)a.n_items * n_panels;
-    long wgs = (total + 3) / 4;
-    if (wgs == 0) return hipSuccess;
-    const long xcd_run = a.deal && a.items ? (long)a.deal->run((size_t)a.n_items, n_panels) : (wgs + 7) / 8;
-    wgs = (wgs + 8 * xcd_run - 1) / (8 * xcd_run) * (8 * xcd_run);
+    if (total == 0) return hipSuccess;
+    const long xcd_run = 4 * (a.deal && a.items ? (long)a.deal->run((size_t)a.n_items, n_panels) : ((total + 3) / 4 + 7) / 8);
+    const long wgs = (total + 8 * xcd_run - 1) / (8 * xcd_run) * (8 * xcd_run);
     if (wgs > 0x7fffffffL) return hipErrorInvalidValue;
-    dim3 grid((unsigned)wgs), block(256);
+    dim3 grid((unsigned)wgs), block(64);
 #define SMAT_LAUNCH_ROWWISE(F32, PK)                                                              \
     hipLaunchKernelGGL((spmm_rowwise_kernel<TN, F32, PK>), grid, block, 0, st, a.vals, a.row_ptr, \
                        a.col_idx, a.b_packed ? a.b_packed : a.B, a.C, a.workspace, a.items,       \
