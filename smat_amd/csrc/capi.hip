@@ -216,6 +216,13 @@ static double rowwise_in_place_us(size_t M, size_t K, size_t N, size_t nnzb, siz
     const size_t tiles = (size_t)rowwise_panel_tiles(N, n_items, (size_t)avg, RowLengths::EVEN, false), wavefronts = n_items * ((N + 16 * tiles - 1) / (16 * tiles));
     return 2.48 + 0.56 * mn + (double)tiles * avg * ((double)((wavefronts + 1023) / 1024) * (0.038 + 0.0189 * aligned) + (double)wavefronts / 1024.0 * 0.0338 * share4);
 }
+// The row-wise kernel on a row-major B in place: the rows of B under the blocks of every panel and the blocks, 17.5 TB/s, and C.  215 products (random blocks, bands, N = 8 to
+// 4096, 5 to 1,000 us): 11 % standard deviation, 1 % low in the mean.
+static double rowwise_row_major_us(size_t M, size_t N, size_t nnzb)
+{
+    const size_t width = N <= 16 ? 16 : N <= 32 ? 32 : 64, panels = (N + width - 1) / width;
+    return 4.8 + 0.33e-6 * (double)M * (double)N + 0.057e-6 * (double)nnzb * (double)panels * (double)(32 * width + 512);
+}
 // A row-major B into column-major order, for the kernels that do not read it in place (8192 x 4096 23 us, 4112 x 504 3 us beside
 // the launch that follows); and what the sweep kernel takes longer on a row-major B in place (8192^2, 10 %, N = 4096 103 against 97 us,
 // with N = 2040, rows that straddle cache lines, 50 against 43).
@@ -296,6 +303,17 @@ static bool windows_beat(const smat_plan &p, const WindowPlan &shape, const Wind
     return l.tiles && window_short_us(shape, l, p.M, p.K, N, p.nnzb) < (shape.share > 0.6 ? 0.95 : 1.0) * in_place;
 }
 
+// Whether a launch of the row-wise kernel reads a row-major B in place: always but for large products on a repacked B, which are 5 to 35 % slower for it (13696 x 6768, 19 %,
+// N = 2384 287 -> 391 us, 8160 x 9536, 24 %, N = 336 61 -> 72; 120 drawn products otherwise 0.44 to 0.93 of the time: a launch less, and loads of whole lines instead of 32
+// pieces), and but for windows that are estimated to be faster, the pass over B before them included.
+static bool rowwise_stays_row_major(const smat_plan &p, const SpmmArgs &a)
+{
+    const double in_place = rowwise_row_major_us(a.M, a.N, a.nnzb);
+    if (p.window && in_place > window_launch(a, *p.window).us + to_col_major_us(a.K, a.N)) return false;
+    return !a.b_packed || in_place <= rowwise_estimate_us(a.M, a.K, a.N, a.nnzb, (size_t)p.n_items, p.n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, true) +
+                                          to_col_major_us(a.K, a.N);
+}
+
 extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_ptr,
                                       const int32_t *col_idx, const uint16_t *B, void *C, size_t M,
                                       size_t N, size_t K, size_t nnzb, const smat_spmm_opts *opts,
@@ -349,8 +367,9 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
     if (kernel == SMAT_KERNEL_SWEEP && o.kernel == SMAT_KERNEL_AUTO) {
         // whatever the layout of this launch: both give the same bits through one plan
         const bool in_place = plan->sweep.d_ops_row_major && sweep_takes_row_major(N, K, plan->sweep.n_rg);
-        const double row_wise = rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, plan->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN,
-                                                    a.b_packed != nullptr) + (in_place ? to_col_major_us(K, N) : 0.0);
+        double row_wise = rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, plan->n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN,
+                                              a.b_packed != nullptr) + (in_place ? to_col_major_us(K, N) : 0.0);
+        if (plan->d_bcol) row_wise = std::min(row_wise, rowwise_row_major_us(M, N, nnzb));
         const double factor = in_place ? sweep_in_place_factor(N) : 1.0;
         if (plan->sweep_few_tiles ? factor * sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N) > row_wise
                                   : !sweep_fills_device(M / 16, N))
@@ -362,8 +381,8 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         return set_error(SMAT_ERR_INVALID, "SMAT_KERNEL_MIXED needs a plan that split the block rows when the values were "
                                            "attached (smat_plan_attach_values) and n_hint >= N");
     if (o.b_layout == SMAT_B_ROW_MAJOR && kernel != SMAT_KERNEL_COMPACT) {
-        // the row-wise kernel wants 8 consecutive k of one column in a lane: B is first brought into the reference layout in
-        // plan scratch, then it runs as for column-major B; the sweep kernel reads B in place (same bits in C either way)
+        // The row-wise and the sweep kernel read B in place, or it is first brought into the reference layout in plan scratch, and they run as for
+        // column-major B (same bits in C either way).
         if (!plan || !plan->d_bcol || N > plan->n_cap)
             return set_error(SMAT_ERR_UNSUPPORTED,
                              "row-major B (B[k*N+n]) with the row-wise or sweep kernel needs a plan created with "
@@ -371,9 +390,11 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
         const smat_plan::SweepDev *sweep = kernel == SMAT_KERNEL_SWEEP ? &plan->sweep
                                          : kernel != SMAT_KERNEL_MIXED ? nullptr
                                          : plan->sweep_blocks.d_ops    ? &plan->sweep_blocks
-                                                                       : &plan->sweep_dense;
+                                         : plan->sweep_dense.d_ops     ? &plan->sweep_dense
+                                                                       : nullptr;
         sweep_row_major = sweep && sweep->d_ops_row_major && sweep_takes_row_major(N, K, sweep->n_rg);
-        if (!sweep_row_major) {
+        a.b_row_major = !sweep && rowwise_stays_row_major(*plan, a);
+        if (!sweep_row_major && !a.b_row_major) {
             e = launch_b_to_col_major(B, plan->d_bcol, N, K, static_cast<hipStream_t>(o.stream));
             if (e != hipSuccess) return set_error(SMAT_ERR_HIP, "SpMM launch failed: %s", hipGetErrorString(e));
             a.B = B = plan->d_bcol;
@@ -385,7 +406,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
     ResidentLaunch columns;
     if (plan && o.kernel == SMAT_KERNEL_AUTO && (plan->window || plan->resident)) {
         const bool column_major = o.b_layout == SMAT_B_COL_MAJOR;
-        if (kernel == SMAT_KERNEL_ROWWISE && plan->window) { // a row-major B lies in column-major order by now
+        if (kernel == SMAT_KERNEL_ROWWISE && plan->window && !a.b_row_major) { // a row-major B lies in column-major order by now
             const bool shares = rowwise_shares_items(N, (size_t)plan->n_items, nnzb / (size_t)plan->n_items);
             const double in_place = N == plan->n_cap || window_forced() || shares || a.b_packed ? SHORT_US : rowwise_in_place_us(*plan, N, plan->window->share4);
             if (in_place < SHORT_US) {
@@ -422,7 +443,7 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
             w.whole = false;
             e = launch_sweep(w, static_cast<hipStream_t>(o.stream));
         } else {
-            SpmmArgs d = a;
+            SpmmArgs d = a; // a row-major B in place, or turned by now
             d.items = plan->d_items_dense; d.n_items = plan->n_items_dense;
             d.split_rows = plan->d_split_dense; d.n_split_rows = plan->n_split_dense;
             d.workspace = plan->d_workspace_dense;
@@ -780,8 +801,10 @@ static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, s
     if (nnzb < 2 || nnzb >= (size_t)1 << 23 || K >= (size_t)1 << 28 || kb <= 2 * SWEEP_S) return 0;
     if (g_force_group_rows) return (size_t)g_force_group_rows;
     const double to_col_major = b_row_major ? to_col_major_us(K, N) : 0.0;
-    const double row_wise = rowwise_estimate_us(M, K, N, nnzb, n_items, lengths, packed) + to_col_major;
-    double best = std::min(row_wise / (packed ? 1.1 : 1.2), row_wise - 0.11e-3 * (double)nnzb);
+    double row_wise = rowwise_estimate_us(M, K, N, nnzb, n_items, lengths, packed) + to_col_major;
+    if (b_row_major) row_wise = std::min(row_wise, rowwise_row_major_us(M, N, nnzb));
+    // (the estimate on a row-major B in place errs to either side)
+    double best = std::min(row_wise / (b_row_major ? 1.0 : packed ? 1.1 : 1.2), row_wise - 0.11e-3 * (double)nnzb);
     size_t group_rows = 0;
     for (size_t rows : {(size_t)SWEEP_G, (size_t)SWEEP_G / 2, (size_t)SWEEP_G / 4}) {
         const size_t n_rg = (mb + rows - 1) / rows;
@@ -870,7 +893,8 @@ static hipError_t take_window(smat_plan &p, const int32_t *row_ptr, const int32_
     if (!census && !beside_rowwise(p.n_cap, (size_t)p.n_items, p.nnzb)) return hipSuccess;
     const double once = bytes_once_us(p.M, p.K, p.n_cap, census ? 4.0 * (double)census->nnz + 12.0 * (double)p.nnzb : 512.0 * (double)p.nnzb);
     const double copy = p.d_bcol ? to_col_major_us(p.K, p.n_cap) : 0.0; // before either
-    const double bar = 0.9 * (census ? other_us - copy : std::min(rowwise_from_memory_us(p.M, p.K, p.n_cap, p.nnzb, (size_t)p.n_items, p.d_bpack != nullptr), other_us));
+    double bar = 0.9 * (census ? other_us - copy : std::min(rowwise_from_memory_us(p.M, p.K, p.n_cap, p.nnzb, (size_t)p.n_items, p.d_bpack != nullptr), other_us));
+    if (p.d_bcol) bar = std::min(bar, 0.9 * (rowwise_row_major_us(p.M, p.n_cap, p.nnzb) - copy)); // which does without it
     if (!window_forced() && bar < least_bar_us(once)) return hipSuccess;
     hipError_t e = hipSuccess;
     if (!count.there && !count.begun && p.nnzb <= WindowCount::FEW && p.col_idx_host.size() == p.nnzb) count.on_host(p.row_ptr_host.data(), p.col_idx_host.data(), mb, kb);

@@ -63,6 +63,7 @@ struct SpmmArgs {
     const SplitRow *split_rows; // device
     int n_split_rows;
     float *workspace; // device, n_slots * 16 * N floats
+    bool b_row_major;   // B[k * N + n], read in place (launch_rowwise); b_packed is not looked at
     uint16_t *b_packed; // device scratch of K * N halves, or nullptr: read the column-major B directly
     int max_item_blocks; // blocks of the longest work item, 0 = not known (no plan): lets short rows take the short-row kernel
     const XcdDeal *deal; // how to deal the items to the XCDs; nullptr = an eighth of the launch each

@@ -375,6 +375,145 @@ __global__ __launch_bounds__(256) void spmm_rowwise_short_kernel(
     }
 }
 
+// Row-major B (B[k * N + n]) in place: the 16 rows of B under a block are PW columns of it each, 2 * PW consecutive bytes, which go from the registers they
+// were loaded into through LDS and come back as MFMA operands through transposing reads (ds_read_b64_tr_b16; layout and the swap of pieces against bank
+// conflicts as in the compact kernel).  Pairs of blocks, their order and the shares of an item are those of the kernels above: same bits.
+// SHARES = 4: four wavefronts share an item as in spmm_rowwise_split_kernel; 1: one wavefront, a workgroup of its own.
+// Bound by the rows of B and the blocks that a wavefront brings over the L2, 17.5 TB/s of them in large launches: 64 lanes ask for 8 to 32 whole pieces of 128 to 32 bytes, 16
+// clocks, where they ask for 32 pieces of 32 bytes of a column-major B, 53.  Before, B was turned in a launch of its own, 1.7 us and its bytes three times, and read as
+// above.  That -> this, us: band of 5024 rows and 12, N = 240 8.0 -> 4.6; 2320 x 1328, 5 %, N = 632 9.2 -> 4.7; 960 x 11824, 6 %, N = 912, fp32 28 -> 12; band of 41472 and 64, N = 208
+// 43 -> 22; stencil 49648, N = 8 9.2 -> 6.1; 2304 x 5840, 6 %, N = 2072 48 -> 24.
+template <int PW, bool C_F32, int SHARES>
+__global__ __launch_bounds__(64 * SHARES) __attribute__((amdgpu_waves_per_eu(1, 4))) void spmm_rowwise_row_major_kernel(
+    const uint16_t *__restrict__ vals, const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_idx,
+    const uint16_t *__restrict__ B, void *__restrict__ Cout, float *__restrict__ workspace, const WorkItem *__restrict__ items,
+    int n_items, int N, int n_panels, unsigned xcd_run)
+{
+    constexpr int T = PW / 16, NP = 4; // tiles of 16 columns, and loads that bring the 32 rows of B under a pair; pairs in flight
+    constexpr int TILE = 64 * PW;      // bytes of 32 rows
+    __shared__ __align__(1024) unsigned char tiles[SHARES][TILE];
+    const int lane = threadIdx.x & 63;
+    const int share = SHARES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long total = (long)n_items * n_panels;
+    const unsigned slot = blockIdx.x >> 3, run = __builtin_amdgcn_readfirstlane(slot / xcd_run);
+    const long w = ((long)run * 8 + (blockIdx.x & 7)) * xcd_run + (slot - run * xcd_run);
+    if (w >= total) return; // the whole workgroup
+    const int panel = (int)(w / n_items);
+    const int it = (int)(w - (long)panel * n_items);
+    int br, p0, p1, dst;
+    if (items) {
+        const WorkItem wi = items[it];
+        br = wi.block_row; p0 = wi.begin; p1 = wi.end; dst = wi.dst;
+    } else {
+        br = it; p0 = row_ptr[it]; p1 = row_ptr[it + 1]; dst = -1;
+    }
+    br = __builtin_amdgcn_readfirstlane(br);
+    p0 = __builtin_amdgcn_readfirstlane(p0);
+    p1 = __builtin_amdgcn_readfirstlane(p1);
+    dst = __builtin_amdgcn_readfirstlane(dst);
+
+    const int i16 = lane & 15, g = lane >> 4, sel = g >> 1;
+    const int n0 = panel * PW;
+    // load j < T: 16 bytes of row k = row0 + 2 j of the pair's 32
+    const int c8 = lane % (PW / 8), place = T * (lane / (PW / 8));
+    const int row0 = 8 * (place >> 3) + 2 * (place & 3) + ((place >> 2) & 1);
+    const bool second_block = row0 >= 16;
+    const uint16_t *const from = B + (long)(row0 & 15) * N + (n0 + 8 * c8 < N ? n0 + 8 * c8 : 0); // N % 8 == 0: all of the lane's columns or none
+    unsigned char *const tile = tiles[share];
+    unsigned char *const put_even = tile + row0 * (2 * PW) + c8 * 16, *const put_odd = tile + row0 * (2 * PW) + (PW == 64 ? c8 ^ 1 : c8) * 16;
+    const int swap = PW == 64 ? (i16 >> 3) & 1 : 0;
+    const unsigned char *const get = tile + (8 * g + (i16 >> 2)) * (2 * PW) + (i16 & 3) * (PW / 2);
+    const unsigned char *const get01 = get + 16 * swap, *const get23 = get - 16 * swap;
+    const uint16_t *const abase = vals + i16 * 16 + (g & 1) * 8;
+    const f16x8 zero8 = zero_f16x8();
+
+    f32x4 acc[T];
+#pragma unroll
+    for (int t = 0; t < T; t++) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int last = p1 - 1, npair = (p1 - p0 + 1) >> 1, per = (npair + SHARES - 1) / SHARES;
+    const int j_first = share * per, j_last = SHARES == 1 ? npair : j_first + per < npair ? j_first + per : npair;
+    for (int jw = j_first; jw < j_last; jw += 32) { // a window of 64 column indices
+        const int first = p0 + 2 * jw;
+        const int myc = col_idx[first + lane < last ? first + lane : last];
+        const int j_end = jw + 32 < j_last ? jw + 32 : j_last;
+        auto pairs = [&](int j, auto count) {
+            constexpr int R = decltype(count)::value;
+            f16x8 a[R], b[R][T];
+#pragma unroll
+            for (int u = 0; u < R; u++) { // the values first: they do not wait for the column indices
+                const int q0 = p0 + 2 * (j + u), q1 = q0 < last ? q0 + 1 : q0; // a single block pairs with itself
+                a[u] = load_f16x8(abase + (long)(sel ? q1 : q0) * 256);
+            }
+            SMAT_ORDER_FENCE();
+#pragma unroll
+            for (int u = 0; u < R; u++) {
+                const int q0 = p0 + 2 * (j + u), q1 = q0 < last ? q0 + 1 : q0;
+                const long o0 = (long)__builtin_amdgcn_readlane(myc, q0 - first) * N, o1 = (long)__builtin_amdgcn_readlane(myc, q1 - first) * N;
+                const uint16_t *const p = from + (second_block ? o1 : o0);
+#pragma unroll
+                for (int l = 0; l < T; l++) b[u][l] = load_f16x8(p + (long)(2 * l) * N);
+            }
+            SMAT_ORDER_FENCE();
+#pragma unroll
+            for (int u = 0; u < R; u++) {
+                const f16x8 au = sel && p0 + 2 * (j + u) >= last ? zero8 : a[u]; // single block: the upper K half contributes nothing
+#pragma unroll
+                for (int l = 0; l < T; l++) *reinterpret_cast<f16x8 *>((l & 1 ? put_odd : put_even) + l * 4 * PW) = b[u][l];
+                asm volatile("" ::: "memory"); // LDS operations of a wavefront complete in order
+                f16x8 op[T];
+#pragma unroll
+                for (int t = 0; t < T; t++) {
+                    typedef short s16x4 __attribute__((ext_vector_type(4)));
+                    const unsigned char *const q = (t < 2 ? get01 : get23) + t * 8;
+                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)q);
+                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(q + 8 * PW));
+                    op[t] = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                }
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int t = 0; t < T; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[t], au, acc[t], 0, 0, 0);
+            }
+        };
+        using std::integral_constant;
+        int j = jw;
+        for (; j + NP <= j_end; j += NP) pairs(j, integral_constant<int, NP>{});
+        if (j_end - j == 3) pairs(j, integral_constant<int, 3>{});
+        else if (j_end - j == 2) pairs(j, integral_constant<int, 2>{});
+        else if (j_end - j == 1) pairs(j, integral_constant<int, 1>{});
+    }
+    if constexpr (SHARES > 1) {
+        f32x4 *const part = reinterpret_cast<f32x4 *>(tile); // T KiB, the size of the tile
+        asm volatile("" ::: "memory");
+        if (share > 0)
+#pragma unroll
+            for (int t = 0; t < T; t++) part[t * 64 + lane] = acc[t];
+        __syncthreads();
+        if (share > 0) return;
+#pragma unroll
+        for (int s = 1; s < SHARES; s++)
+#pragma unroll
+            for (int t = 0; t < T; t++) acc[t] += reinterpret_cast<const f32x4 *>(tiles[s])[t * 64 + lane];
+    }
+    // acc[t][r] = C[16 br + i16][n0 + PW / 4 * g + 4 t + r]
+    const int c0 = n0 + PW / 4 * g;
+    if (dst >= 0 || C_F32) {
+        float *const row = dst >= 0 ? workspace + ((long)dst * 16 + i16) * (long)N : reinterpret_cast<float *>(Cout) + ((long)br * 16 + i16) * (long)N;
+#pragma unroll
+        for (int t = 0; t < T; t++)
+            if (c0 + 4 * t < N) *reinterpret_cast<f32x4 *>(row + c0 + 4 * t) = acc[t];
+    } else {
+        uint16_t *const row = reinterpret_cast<uint16_t *>(Cout) + ((long)br * 16 + i16) * (long)N;
+        if constexpr (T == 1) {
+            if (c0 < N) *reinterpret_cast<f16x4 *>(row + c0) = __builtin_convertvector(acc[0], f16x4);
+        } else {
+#pragma unroll
+            for (int t = 0; t < T; t += 2)
+                if (c0 + 4 * t < N)
+                    *reinterpret_cast<f16x8 *>(row + c0 + 4 * t) = __builtin_shufflevector(__builtin_convertvector(acc[t], f16x4), __builtin_convertvector(acc[t + 1], f16x4), 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    }
+}
+
 // Sums the fp32 partial tiles of every split block row in slot order and writes
 // the finished rows to C.  One thread per 4 consecutive columns of one row.
 template <bool C_F32>
@@ -610,9 +749,42 @@ static hipError_t launch_rowwise_split(const SpmmArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
+template <int PW>
+static hipError_t launch_rowwise_row_major(const SpmmArgs &a, bool shared, hipStream_t st)
+{
+    const int n_panels = (int)((a.N + PW - 1) / PW);
+    const long total = (long)a.n_items * n_panels;
+    if (total == 0) return hipSuccess;
+    const long eighth = (total + 7) / 8;
+    const long xcd_run = shared ? eighth : 4 * (a.deal && a.items ? (long)a.deal->run((size_t)a.n_items, n_panels) : ((total + 3) / 4 + 7) / 8);
+    const long wgs = (total + 8 * xcd_run - 1) / (8 * xcd_run) * (8 * xcd_run);
+    if (wgs > 0x7fffffffL) return hipErrorInvalidValue;
+#define SMAT_LAUNCH_ROW_MAJOR(F32, SHARES)                                                                                                   \
+    hipLaunchKernelGGL((spmm_rowwise_row_major_kernel<PW, F32, SHARES>), dim3((unsigned)wgs), dim3(64 * SHARES), 0, st, a.vals, a.row_ptr,  \
+                       a.col_idx, a.B, a.C, a.workspace, a.items, a.n_items, (int)a.N, n_panels, (unsigned)xcd_run)
+    if (shared) {
+        if (a.c_f32) SMAT_LAUNCH_ROW_MAJOR(true, 4);
+        else SMAT_LAUNCH_ROW_MAJOR(false, 4);
+    } else {
+        if (a.c_f32) SMAT_LAUNCH_ROW_MAJOR(true, 1);
+        else SMAT_LAUNCH_ROW_MAJOR(false, 1);
+    }
+#undef SMAT_LAUNCH_ROW_MAJOR
+    return hipGetLastError();
+}
+
 hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st)
 {
     hipError_t e;
+    const size_t n_items = (size_t)a.rule_items, avg = n_items ? a.nnzb / n_items : 0;
+    const bool shares = rowwise_shares_items(a.N, n_items, avg);
+    if (a.b_row_major) {
+        if (a.N <= 16) e = launch_rowwise_row_major<16>(a, shares, st);
+        else if (a.N <= 32) e = launch_rowwise_row_major<32>(a, shares, st);
+        else e = launch_rowwise_row_major<64>(a, shares, st);
+        if (e == hipSuccess && a.n_split_rows > 0) e = launch_reduce(a.workspace, a.split_rows, a.n_split_rows, a.C, a.N, a.c_f32, st);
+        return e;
+    }
     if (!a.b_packed && a.n_split_rows == 0 && rowwise_takes_short_rows(a.N, (size_t)a.n_items, a.max_item_blocks)) {
         // 32-column panels while that still leaves the chip short of wavefronts, else 64
         const bool narrow = (long)a.n_items * (long)((a.N + 63) / 64) < 2048;
@@ -624,8 +796,7 @@ hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st)
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    const size_t n_items = (size_t)a.rule_items, avg = n_items ? a.nnzb / n_items : 0;
-    if (rowwise_shares_items(a.N, n_items, avg)) {
+    if (shares) {
         if (a.N < 32) e = launch_rowwise_split<1>(a, st);
         else if (a.N < 64) e = launch_rowwise_split<2>(a, st);
         else e = launch_rowwise_split<4>(a, st);

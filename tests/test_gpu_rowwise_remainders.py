@@ -1,5 +1,6 @@
 """The row-wise kernels at every number of block pairs that is left over: rows of 0 to 10 blocks (all pairs asked for at once), rows that four wavefronts
-share (runs of 1 to 9 pairs, some empty), and rows that one wavefront takes two pairs at a time, past the 64 blocks of one load of indices."""
+share (runs of 1 to 9 pairs, some empty), and rows that one wavefront takes two pairs at a time, past the 64 blocks of one load of indices; on either
+layout of B."""
 import numpy as np
 import pytest
 
@@ -26,6 +27,14 @@ def test_every_remainder(smat, cuda, oracle, rows, N, packed):
     C = torch.full((M, N), float("nan"), dtype=torch.float32, device=cuda)
     smat.spmm(vals, rp, ci, Bd, C, M, N, K, nnzb, plan=plan, kernel=kernel, c_f32=True)
     torch.cuda.synchronize()
+    if not packed:  # B as rows, read in place, gives the same bits
+        plan = smat.Plan(A["b_row_ptr"], M, K, nnzb, N, col_idx_host=A["b_col_idx"], kernel=kernel, b_row_major=True)
+        rows_of_b = Bd.view(N, K).t().contiguous()
+        for c_f32, same in ((True, C), (False, C.half())):
+            R = torch.full((M, N), float("nan"), dtype=same.dtype, device=cuda)
+            smat.spmm(vals, rp, ci, rows_of_b, R, M, N, K, nnzb, plan=plan, kernel=kernel, c_f32=c_f32, b_row_major=True)
+            torch.cuda.synchronize()
+            assert torch.equal(R, same)
     # fp32 sums of exact products in another order: n roundings of 2^-24 of what the terms add up to, n <= 70 * 16
     dense = np.zeros((M, K))
     v = A["b_val"].view(np.float16).astype(np.float64).reshape(-1, 16, 16)
