@@ -216,6 +216,7 @@ class Plan:
         ci = None if col_idx_host is None else np.ascontiguousarray(col_idx_host, dtype=np.int32)
         opts = SpmmOpts(1 if b_row_major else 0, 0, kernel, 0, None)
         check(lib.smat_plan_create(C.byref(self._h), _p(rp), _p(ci), M, K, nnzb, n_hint, C.byref(opts)))
+        self._address = self._h.value  # for the call from the extension module
         self._rp_host = rp
 
     def check(self, row_ptr_host, col_idx_host, M, K, nnzb):
@@ -250,6 +251,7 @@ class Plan:
         if self._h:
             lib.smat_plan_destroy(self._h)
             self._h = C.c_void_p()
+            self._address = 0
 
     def __del__(self):
         try:
@@ -277,7 +279,7 @@ def spmm(vals, row_ptr, col_idx, B, C_out, M, N, K, nnzb, plan=None, c_f32=False
 
     drop_in=True calls the positional drop-in entry point (smat_spmm_bcsr_f16) with
     NULL block_info / rel_map; otherwise the options entry point."""
-    # A small product is over sooner than the call that launches it: addresses go to ctypes as plain integers and the
+    # For arguments that the extension module leaves to Python, or all where there is none: addresses go to ctypes as plain integers and the
     # options are not made anew (1.1 us of Python per call when they were).
     v = vals.data_ptr() if vals is not None else None
     rp = row_ptr.data_ptr() if row_ptr is not None else None
@@ -294,3 +296,12 @@ def spmm(vals, row_ptr, col_idx, B, C_out, M, N, K, nnzb, plan=None, c_f32=False
         rc = _launch(v, rp, ci, b, c, M, N, K, nnzb, o, plan._h if plan is not None else None)
     if rc:
         check(rc)
+
+
+try:
+    from . import _call  # the same call at a quarter of what it costs in Python
+except ImportError:  # built without Python's headers, or by another Python
+    pass
+else:
+    _call.bind(C.cast(_launch, C.c_void_p).value, C.cast(_launch_drop_in, C.c_void_p).value, spmm, check, Plan)
+    spmm = _call.spmm
