@@ -9,7 +9,7 @@
 
 #include <cstdint>
 
-#include "../../include/smat.h"
+#include "../../../include/smat.h"
 
 namespace {
 
