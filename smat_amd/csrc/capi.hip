@@ -593,6 +593,38 @@ static void rowwise_costs(const std::vector<WorkItem> &items, XcdDeal &deal)
     deal.set_costs(std::move(prefix));
 }
 
+// Blocks of a chunk of a split block row.  Rows are split where one has more than four times the average and 64 blocks; a chunk is then no longer than 32 blocks and 0.4 of what
+// one of 4,096 wavefronts has to do in a launch of the plan's width, since the longest item is as long as a small launch.  Chunks of four times the average -> these, us (R-MAT,
+// row-wise): scale 12, 16 a row, N = 128 30.7 -> 18.6 (of 16, 32, 64, 128 blocks 18.3, 17.8, 18.5, 25.7); 13, 16, N = 24 32 -> 14; 14, 20, N = 104 56 -> 39 (64: 38, 32: 42); 15, 16, N = 200
+// 172 -> 148; 16, 16, N = 16 94 -> 68; 17, 16, N = 72 413 -> 386 (64: 417); 19, 9, N = 40 882 -> 864.
+static long rowwise_chunk(const int32_t *row_ptr_host, size_t mb, size_t nnzb, size_t n_hint, double avg)
+{
+    const auto even = [](double blocks) { return ((long)(blocks + 0.5) + 1) & ~1L; }; // pairs stay aligned with the MFMA's K = 32
+    const long longest = std::max(even(4.0 * avg), 64L);
+    for (size_t i = 0; i < mb; i++)
+        if (row_ptr_host[i + 1] - row_ptr_host[i] > longest)
+            return std::min(longest, even(32.0 + 0.4 * (double)nnzb * (double)((n_hint + 63) / 64) / 4096.0));
+    return longest;
+}
+// The items of a list with split rows in the order that the compact kernel's tasks have (spmm_compact.hip): chunks by where they begin in their rows, whole rows by octaves of
+// length.  Chunks of one row after the other -> this, us (R-MAT, row-wise): scale 14, 12 a row, N = 256 60.2 -> 56.6; 16, 16, N = 184 304 -> 287; 16, 20, N = 256 509 -> 482; 18, 12, N = 128
+// 1031 -> 852; 19, 16, N = 8 531 -> 485; scale 12 and 13 equal.
+static void order_split_items(const int32_t *row_ptr_host, std::vector<WorkItem> &items)
+{
+    std::vector<std::pair<double, WorkItem>> chunks;
+    std::vector<WorkItem> whole[32];
+    for (const WorkItem &w : items) {
+        const double from = row_ptr_host[w.block_row], to = row_ptr_host[w.block_row + 1];
+        if (w.dst >= 0) chunks.emplace_back(((double)w.begin - from) / (to - from), w);
+        else whole[31 - __builtin_clz((unsigned)(w.end - w.begin) | 1u)].push_back(w);
+    }
+    std::stable_sort(chunks.begin(), chunks.end(), [](const auto &a, const auto &b) { return a.first < b.first; });
+    size_t at = 0;
+    for (const auto &c : chunks) items[at++] = c.second;
+    for (int octave = 31; octave >= 0; octave--)
+        for (const WorkItem &w : whole[octave]) items[at++] = w;
+}
+
 static int rowwise_work_list(const int32_t *row_ptr_host, size_t mb, long chunk, const uint8_t *only,
                              std::vector<WorkItem> &items, std::vector<SplitRow> &split)
 {
@@ -707,19 +739,16 @@ static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
     p->row_ptr_host.assign(row_ptr_host, row_ptr_host + mb + 1);
     if (col_idx_host && cols_ascending && (want == SMAT_KERNEL_AUTO || want == SMAT_KERNEL_MIXED)) p->col_idx_host.assign(col_idx_host, col_idx_host + nnzb);
 
-    // A block row is split when it is much longer than the average: chunks of
-    // `chunk` blocks (even, so block pairs stay aligned with the MFMA K = 32).
     size_t nonempty = 0;
     for (size_t i = 0; i < mb; i++) nonempty += row_ptr_host[i + 1] > row_ptr_host[i];
     const double avg = nonempty ? (double)nnzb / (double)nonempty : 0.0;
-    long chunk = (long)(4.0 * avg + 0.5);
-    chunk = std::max(chunk, 64L);
-    chunk = (chunk + 1) & ~1L;
+    const long chunk = rowwise_chunk(row_ptr_host, mb, nnzb, n_hint, avg);
     p->chunk = (int)chunk;
 
     std::vector<WorkItem> items;
     std::vector<SplitRow> split;
     const int slot = rowwise_work_list(row_ptr_host, mb, chunk, nullptr, items, split);
+    if (!split.empty()) order_split_items(row_ptr_host, items);
     p->n_items = (int)items.size();
     rowwise_costs(items, p->deal);
     for (const WorkItem &wi : items) p->max_item_blocks = std::max(p->max_item_blocks, wi.end - wi.begin);

@@ -34,7 +34,6 @@
 #include <stdint.h>
 
 #include <algorithm>
-#include <cmath>
 #include <cstring>
 #include <type_traits>
 #include <vector>
@@ -1225,9 +1224,9 @@ static void order_tasks(std::vector<int4> &tasks, std::vector<uint32_t> &costs, 
     struct Task {
         int4 t;
         uint32_t cost;
-        double key; // chunk: where it begins in its row; whole rows: class
+        double begins; // chunk: where in its row
     };
-    std::vector<Task> chunks, whole;
+    std::vector<Task> chunks, of_class[32], whole;
     uint64_t total = 0, total_chunks = 0;
     for (size_t i = 0; i < tasks.size(); i++) {
         const WorkItem &w = items[(size_t)tasks[i].x];
@@ -1237,11 +1236,11 @@ static void order_tasks(std::vector<int4> &tasks, std::vector<uint32_t> &costs, 
             chunks.push_back(Task{tasks[i], costs[i], ((double)w.begin - from) / (to - from)});
             total_chunks += costs[i];
         } else {
-            whole.push_back(Task{tasks[i], costs[i], (double)(std::ilogb((double)costs[i]) / octaves)});
+            of_class[(31 - __builtin_clz(costs[i] | 1u)) / octaves].push_back(Task{tasks[i], costs[i], 0.0});
         }
     }
-    std::stable_sort(chunks.begin(), chunks.end(), [](const Task &a, const Task &b) { return a.key < b.key; });
-    std::stable_sort(whole.begin(), whole.end(), [](const Task &a, const Task &b) { return a.key > b.key; });
+    std::stable_sort(chunks.begin(), chunks.end(), [](const Task &a, const Task &b) { return a.begins < b.begins; });
+    for (int c = 31; c >= 0; c--) whole.insert(whole.end(), of_class[c].begin(), of_class[c].end());
     std::vector<Task> queue[8];
     uint64_t load[8] = {};
     auto put = [&](int x, const Task &t) { queue[x].push_back(t); load[x] += t.cost; };
