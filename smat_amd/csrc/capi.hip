@@ -611,18 +611,15 @@ static long rowwise_chunk(const int32_t *row_ptr_host, size_t mb, size_t nnzb, s
 // 1031 -> 852; 19, 16, N = 8 531 -> 485; scale 12 and 13 equal.
 static void order_split_items(const int32_t *row_ptr_host, std::vector<WorkItem> &items)
 {
-    std::vector<std::pair<double, WorkItem>> chunks;
-    std::vector<WorkItem> whole[32];
-    for (const WorkItem &w : items) {
-        const double from = row_ptr_host[w.block_row], to = row_ptr_host[w.block_row + 1];
-        if (w.dst >= 0) chunks.emplace_back(((double)w.begin - from) / (to - from), w);
-        else whole[31 - __builtin_clz((unsigned)(w.end - w.begin) | 1u)].push_back(w);
+    std::vector<uint16_t> keys(items.size());
+    for (size_t i = 0; i < items.size(); i++) {
+        const WorkItem &w = items[i];
+        keys[i] = w.dst >= 0 ? begin_key(w.begin, row_ptr_host[w.block_row], row_ptr_host[w.block_row + 1]) : (uint16_t)(BEGIN_KEYS + 31 - octave_of((uint32_t)(w.end - w.begin)));
     }
-    std::stable_sort(chunks.begin(), chunks.end(), [](const auto &a, const auto &b) { return a.first < b.first; });
-    size_t at = 0;
-    for (const auto &c : chunks) items[at++] = c.second;
-    for (int octave = 31; octave >= 0; octave--)
-        for (const WorkItem &w : whole[octave]) items[at++] = w;
+    const std::vector<uint32_t> order = ordered_by(keys, BEGIN_KEYS + 32);
+    std::vector<WorkItem> ordered(items.size());
+    for (size_t i = 0; i < items.size(); i++) ordered[i] = items[order[i]];
+    items.swap(ordered);
 }
 
 static int rowwise_work_list(const int32_t *row_ptr_host, size_t mb, long chunk, const uint8_t *only,

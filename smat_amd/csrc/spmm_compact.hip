@@ -1221,52 +1221,46 @@ static long split_chunk_steps(long steps, size_t rows, long longest, size_t n_ca
 // 517; with two panels or fewer two octaves are 1 to 5 % slower).
 static void order_tasks(std::vector<int4> &tasks, std::vector<uint32_t> &costs, const std::vector<WorkItem> &items, const std::vector<int32_t> &row_first, int octaves)
 {
-    struct Task {
-        int4 t;
-        uint32_t cost;
-        double begins; // chunk: where in its row
-    };
-    std::vector<Task> chunks, of_class[32], whole;
     uint64_t total = 0, total_chunks = 0;
+    std::vector<uint16_t> keys(tasks.size());
     for (size_t i = 0; i < tasks.size(); i++) {
         const WorkItem &w = items[(size_t)tasks[i].x];
         total += costs[i];
-        if (w.dst >= 0) {
-            const double from = row_first[(size_t)w.block_row], to = row_first[(size_t)w.block_row + 1];
-            chunks.push_back(Task{tasks[i], costs[i], ((double)w.begin - from) / (to - from)});
-            total_chunks += costs[i];
-        } else {
-            of_class[(31 - __builtin_clz(costs[i] | 1u)) / octaves].push_back(Task{tasks[i], costs[i], 0.0});
-        }
+        if (w.dst >= 0) total_chunks += costs[i];
+        keys[i] = w.dst >= 0 ? begin_key(w.begin, row_first[(size_t)w.block_row], row_first[(size_t)w.block_row + 1])
+                             : (uint16_t)(BEGIN_KEYS + 31 - octave_of(costs[i]) / octaves);
     }
-    std::stable_sort(chunks.begin(), chunks.end(), [](const Task &a, const Task &b) { return a.begins < b.begins; });
-    for (int c = 31; c >= 0; c--) whole.insert(whole.end(), of_class[c].begin(), of_class[c].end());
-    std::vector<Task> queue[8];
+    const std::vector<uint32_t> order = ordered_by(keys, BEGIN_KEYS + 32);
+    std::vector<uint32_t> queue[8];
+    for (auto &q : queue) q.reserve(tasks.size() / 4);
     uint64_t load[8] = {};
-    auto put = [&](int x, const Task &t) { queue[x].push_back(t); load[x] += t.cost; };
+    auto put = [&](int x, uint32_t i) { queue[x].push_back(i); load[x] += costs[i]; };
     uint64_t before = 0;
-    for (const Task &t : chunks) {
-        put((int)std::min<uint64_t>(7, before * 8 / total_chunks), t);
-        before += t.cost;
+    size_t at = 0;
+    for (; at < order.size() && keys[order[at]] < BEGIN_KEYS; at++) { // the chunks
+        put((int)std::min<uint64_t>(7, before * 8 / total_chunks), order[at]);
+        before += costs[order[at]];
     }
-    for (size_t i = 0; i < whole.size();) {
+    while (at < order.size()) {
         const int x = (int)(std::min_element(load, load + 8) - load);
         uint64_t piece = 0;
-        for (size_t n = 0; i < whole.size() && n < 256 && (n % 4 || n == 0 || piece * 256 < total); n++, i++) {
-            piece += whole[i].cost;
-            put(x, whole[i]);
+        for (size_t n = 0; at < order.size() && n < 256 && (n % 4 || n == 0 || piece * 256 < total); n++, at++) {
+            piece += costs[order[at]];
+            put(x, order[at]);
         }
     }
-    size_t rounds = 0; // of a workgroup an XCD; places past the end of a queue stay empty
+    size_t rounds = 0; // of four tasks an XCD; places past the end of a queue stay empty
     for (const auto &q : queue) rounds = std::max(rounds, (q.size() + 3) / 4);
-    tasks.assign(rounds * 32, int4{0, 0, 0, 0});
-    costs.assign(rounds * 32, 0);
+    std::vector<int4> placed(rounds * 32, int4{0, 0, 0, 0});
+    std::vector<uint32_t> placed_costs(rounds * 32, 0);
     for (int x = 0; x < 8; x++)
         for (size_t i = 0; i < queue[x].size(); i++) {
-            const size_t at = (i / 4 * 8 + (size_t)x) * 4 + i % 4;
-            tasks[at] = queue[x][i].t;
-            costs[at] = queue[x][i].cost;
+            const size_t to = (i / 4 * 8 + (size_t)x) * 4 + i % 4;
+            placed[to] = tasks[queue[x][i]];
+            placed_costs[to] = costs[queue[x][i]];
         }
+    tasks.swap(placed);
+    costs.swap(placed_costs);
 }
 
 hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *row_ptr, const int32_t *col_idx, size_t K, size_t n_cap,

@@ -69,6 +69,23 @@ struct SpmmArgs {
     const XcdDeal *deal; // how to deal the items to the XCDs; nullptr = an eighth of the launch each
 };
 
+// Where chunk [begin, ..) of a split row begins in it, and the octave of a cost, as keys that lists with split rows are ordered by; ordered_by: the places of the keys
+// from 0 to n_keys - 1, equal ones in the order they have (counted, not compared: ordering 10,000 items is 0.05 ms of a new plan, 0.2 when they were sorted).
+constexpr int BEGIN_KEYS = 32768;
+inline uint16_t begin_key(int32_t begin, int32_t row_begin, int32_t row_end)
+{
+    return (uint16_t)((int64_t)(begin - row_begin) * BEGIN_KEYS / (row_end - row_begin));
+}
+inline int octave_of(uint32_t cost) { return 31 - __builtin_clz(cost | 1u); }
+inline std::vector<uint32_t> ordered_by(const std::vector<uint16_t> &keys, int n_keys)
+{
+    std::vector<uint32_t> next((size_t)n_keys + 1, 0), order(keys.size());
+    for (uint16_t k : keys) next[(size_t)k + 1]++;
+    for (int k = 0; k < n_keys; k++) next[(size_t)k + 1] += next[(size_t)k];
+    for (size_t i = 0; i < keys.size(); i++) order[next[keys[i]]++] = (uint32_t)i;
+    return order;
+}
+
 // Stream format and geometry of the sweep kernel: sweep_format.h (shared with the host-side plan builder).
 
 struct SweepArgs {
