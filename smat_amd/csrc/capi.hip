@@ -1194,6 +1194,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     }
     census.waited();
     p->compact = c;
+    c->by_name = want != SMAT_KERNEL_AUTO;
     p->kernel = mixed || block_split ? SMAT_KERNEL_MIXED : SMAT_KERNEL_COMPACT;
     // the deal of the compact kernel's work items to the XCDs, measured on this list at the plan's width (B in the
     // layout the plan was made for: d_bcol is the scratch of a plan for row-major B)

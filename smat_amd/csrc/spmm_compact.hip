@@ -52,10 +52,12 @@ namespace {
 
 int g_force_run = 0;
 int g_tune = 1; // test hook: 0 = attaching values measures nothing, the estimate decides the deal
+int g_last_share = 1; // test hook: wavefronts a task of the latest launch
 int g_last_run = 0; // test hook: the run length of the latest launch
 int g_force_list = 0; // test hook: 1 = lists of whole columns, 2 = of nonzeros, 0 = compact_build decides
 int g_force_staged = 0; // test hook: 1 = entries go through LDS in blocks wherever they may, 2 = nowhere, 0 = the launcher decides
 int g_force_order = 0; // test hook: 1 = tasks of lists with split rows in the order of their items, 0 = order_tasks
+int g_force_share = 0; // test hook: 1, 2 or 4 = wavefronts that share a task where they may, 0 = the launcher decides
 int g_force_tq = 0; // test hook: 1 or 2 = panels of 64 or 128 columns whatever the sizes say, 0 = the launcher decides
 
 constexpr int FULL_BLOCK_COLS = 10; // nonzero columns from which a block counts as full (of 16)
@@ -486,7 +488,8 @@ static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, si
 // ---- the product ----
 
 // A wavefront takes a task x a panel of W = 16, 32, 64 or 128 columns.  A task is a run of items of the list, worked off as one stream of
-// steps, so that the loads of the next step are under way across the end of an item.
+// steps, so that the loads of the next step are under way across the end of an item.  In short launches the wavefronts of a workgroup share a task
+// of one item (`shared`, compact_share).
 //
 // What a step of 32 columns x 64 columns of C waits for is the vector memory path: 4 KiB of rows of B and 0.15 to 1 KiB of A.
 // Counted on R-MAT scale 20 (stencil 64^3), entries by blocks: its data unit is busy 91 (65) % of the time, the vector L1 waits for the L2 54
@@ -541,7 +544,7 @@ template <int W, bool C_F32, bool C_ACC, int AF, bool STAGED, bool BIG>
 __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const uint16_t *__restrict__ acol, const uint32_t *__restrict__ entries, const int2 *__restrict__ step_range, const int32_t *__restrict__ cols,
     const uint16_t *__restrict__ Bt, void *__restrict__ Cout, float *__restrict__ workspace, const WorkItem *__restrict__ items,
-    const int4 *__restrict__ tasks, int n_tasks, int N, int n_panels, long panel_stride, long row_stride, unsigned xcd_run)
+    const int4 *__restrict__ tasks, int n_tasks, int N, int n_panels, long panel_stride, long row_stride, unsigned xcd_run, bool shared)
 {
     constexpr int TQ = W > 64 ? 2 : 1, PW = W / TQ, T = PW / 16; // a row of PW columns is gathered by PW / 8 lanes, 32 rows by T instructions
     constexpr int A_BYTES = 1024, B_BYTES = 64 * W, I_BYTES = 2048;
@@ -560,21 +563,27 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const unsigned slot = blockIdx.x >> 3;
     const unsigned run = __builtin_amdgcn_readfirstlane(slot / xcd_run);
     const long wg = ((long)run * 8 + (blockIdx.x & 7)) * xcd_run + (slot - run * xcd_run);
-    const long w = wg * (blockDim.x >> 6) + wave;
+    const int wavefronts = blockDim.x >> 6;
+    const long w = shared ? wg : wg * wavefronts + wave;
     if (w >= total) return;
     const int panel = __builtin_amdgcn_readfirstlane((int)(w / n_tasks));
     const int task = __builtin_amdgcn_readfirstlane((int)(w - (long)panel * n_tasks));
     const int4 tk = tasks[task]; // first item, items (at most 64), first and last column of the stream
     if (tk.y == 0) return;       // a place that order_tasks left empty
-    int e = tk.z;
-    const int e_last = tk.w;
+    int e = tk.z, e_last = tk.w;
+    if (shared) { // tasks of one item: this wavefront's steps of it
+        const int steps = ((e_last - e) / 32 + wavefronts - 1) / wavefronts;
+        e = min(e + wave * steps * 32, e_last);
+        e_last = min(e + steps * 32, e_last);
+    }
+    const int begin = e;
     // Scalar loads share a counter with the LDS operations below, which would wait for them at every step: the items of
     // the task and the entry ranges of its steps come in through vector loads, one per lane, and are read from the lanes.
     const WorkItem mine = items[tk.x + (lane < tk.y ? lane : tk.y - 1)];
     int it = 0, item_end, br, dst;
     auto enter = [&] {
         br = __builtin_amdgcn_readlane(mine.block_row, it);
-        item_end = __builtin_amdgcn_readlane(mine.end, it);
+        item_end = shared ? e_last : __builtin_amdgcn_readlane(mine.end, it);
         dst = __builtin_amdgcn_readlane(mine.dst, it);
     };
     enter();
@@ -728,6 +737,23 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     // The tile of item `it` goes out (acc[q][t][r] = C[16 br + i16][n0 + 64 q + 16 g + 4 t + r]); the next item that has
     // steps is the current one afterwards.
     auto finish = [&] {
+        if (shared) { // the parts of the others are added in their order by the first wavefront
+            constexpr int OWN = compact_lds_bytes(W, STAGED);
+            static_assert(OWN >= TQ * T * 1024, "a tile of sums");
+            asm volatile("" ::: "memory");
+            if (wave > 0) {
+#pragma unroll
+                for (int t = 0; t < TQ * T; t++) *reinterpret_cast<f32x4 *>(lds + t * 1024 + lane * 16) = acc[t / T][t % T];
+            }
+            __syncthreads();
+            if (wave > 0) {
+                it = tk.y;
+                return;
+            }
+            for (int v = 1; v < wavefronts; v++)
+#pragma unroll
+                for (int t = 0; t < TQ * T; t++) acc[t / T][t % T] += *reinterpret_cast<const f32x4 *>(lds_of_workgroup + v * OWN + t * 1024 + lane * 16);
+        }
         do {
             const long m = (long)br * 16 + i16;
 #pragma unroll
@@ -798,7 +824,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     auto end_if_done = [&] { asm volatile("s_cmp_lt_i32 %0, %1\n\ts_cbranch_scc1 1f\n\ts_endpgm\n1:" ::"s"(it), "s"(tk.y) : "scc", "memory"); };
     do {
 #define SMAT_STEP_OF(CUR, NEW, DONE)                                                                        \
-        if (((next + 32 - tk.z) & 255) == 0) {                                                         \
+        if (((next + 32 - begin) & 255) == 0) {                                                         \
             put_block(next + 32, block);                                                               \
             block = load_block(next + 288);                                                            \
             more_ranges();                                                                             \
@@ -817,6 +843,17 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
         SMAT_STEP_OF(op_b, op_a, )
 #undef SMAT_STEP_OF
     } while (it < tk.y);
+}
+
+// Wavefronts that share a task.  A launch of less than a wavefront a SIMD takes as long as one of them goes from step to step, 0.3 us each; with the steps of a task between
+// two or four of a workgroup, whose sums meet in LDS (1 us), it is shorter as long as there is room for them, and longer (up to 10 %) where a task has few steps or the
+// wavefronts are enough.  Alone / two / four, us, the copy of B among them: 3584 x 4112, 8 % of full blocks and 10 more a row, N = 96 (448 tasks and panels of 15 steps) 10.5 / 8.7 / 8.6,
+// 4416 x 8160, 8 % and 3, N = 72 (552 of 22) 13.4 / 11.0 / 11.4, 2832 x 2144, 32 a row, N = 48 (177 of 14) 5.65 / 4.37 / 4.07, 6992 x 7616, 7 % and 4, N = 80 (874 of 18) 12.7 / 11.4 / 12.0;
+// 5776 x 6752, 5 % and 3, N = 192 (1083 of 12) 12.2 / 12.2 / 12.5, 4288 x 1088, 8 a row, N = 48 (268 of 4) 3.88 / 4.06 / 4.11.
+int compact_share(const CompactPlan &p, long total)
+{
+    if (p.by_name || total > 900 || p.n_steps < 6 * (int64_t)p.n_tasks) return 1;
+    return total > 400 || p.n_steps < 12 * (int64_t)p.n_tasks ? 2 : 4;
 }
 
 template <int W>
@@ -848,9 +885,10 @@ hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
     // A workgroup of four tasks keeps its place until the longest is done; one task each is up to 12 % faster (4864 x 6496, 12 % of full blocks and 15 more a row, N =
     // 400 30.5 -> 26.6 us, 40000 x 60000, 10 a row, N = 64, row-major 9.7 -> 9.3, R-MAT scale 18, N = 64 63.9 -> 62.7).  Where a place has many steps to do the end of a launch
     // matters less than the lines that neighbouring tasks find of each other's in their L1: four (R-MAT scale 20, N = 128, row-major 366, one each 378; 19, N = 256 362 and 365, 40000 x 60000, 30 a row, N = 256 73.8 and 74.6).
-    const int waves = (double)p.n_steps * n_panels >= 32.0 * 16.0 * 256.0 ? 4 : 1;
-    xcd_run *= 4 / waves;
-    wgs = (total + waves - 1) / waves;
+    const int share = g_last_share = !p.may_share ? 1 : g_force_share ? g_force_share : compact_share(p, total);
+    const int waves = share > 1 ? share : (double)p.n_steps * n_panels >= 32.0 * 16.0 * 256.0 ? 4 : 1;
+    xcd_run *= share > 1 ? 4 : 4 / waves;
+    wgs = share > 1 ? total : (total + waves - 1) / waves;
     wgs = (wgs + 8 * xcd_run - 1) / (8 * xcd_run) * (8 * xcd_run);
     if (wgs > 0x7fffffffL) return hipErrorInvalidValue;
     if (a.accumulate && p.n_split_rows > 0) return hipErrorInvalidValue; // partial tiles through the workspace overwrite C
@@ -859,7 +897,7 @@ hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
     auto launch = [&](auto af, auto staged, auto f32, auto acc, auto wide) {
         hipLaunchKernelGGL((spmm_compact_kernel<W, decltype(f32)::value, decltype(acc)::value, decltype(af)::value, decltype(staged)::value, decltype(wide)::value>),
                            dim3((unsigned)wgs), dim3(64 * waves), (size_t)(waves * compact_lds_bytes(W, decltype(staged)::value)), st, p.d_acol, p.d_entries, p.d_step_range, cols, a.Bt, a.C, p.d_workspace,
-                           p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, (unsigned)xcd_run);
+                           p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, (unsigned)xcd_run, share > 1);
     };
     using std::false_type;
     using std::true_type;
@@ -1460,6 +1498,9 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
     std::vector<uint64_t> cost_prefix(costs.size() + 1, 0);
     for (size_t i = 0; i < costs.size(); i++) cost_prefix[i + 1] = cost_prefix[i] + costs[i];
     p->deal.set_costs(std::move(cost_prefix));
+    // Not where columns of B may be held in LDS (few nonzeros a column, column-major), whose sums are to be as close to the exact ones as this kernel's: 60 a row 6.4e-7 root
+    // mean square error, this kernel's 9.0e-7 in one sum and 5.6e-7 in two.
+    p->may_share = (nnz >= 2 * n_cols || b_row_major || !resident_holds(K)) && std::all_of(tasks.begin(), tasks.end(), [](const int4 &t) { return t.y <= 1; });
     p->n_items = (int)items.size();
     p->n_tasks = (int)tasks.size();
     p->n_steps = total / 32;
@@ -1503,6 +1544,9 @@ extern "C" void smat_internal_compact_list(int what) { smat::g_force_list = what
 extern "C" void smat_internal_compact_staged(int what) { smat::g_force_staged = what; }
 // Test hook: 1 = tasks of lists with split rows in the order of their items, 0 = as order_tasks says (the default).
 extern "C" void smat_internal_compact_order(int what) { smat::g_force_order = what; }
+// Test hook: 1, 2 or 4 = wavefronts of a launch that share a task, where tasks are of one item, 0 = as the sizes say (the default).
+extern "C" void smat_internal_compact_share(int what) { smat::g_force_share = what; }
+extern "C" int smat_internal_compact_last_share(void) { return smat::g_last_share; }
 // Test hook (host only): steps of the chunks of split rows.
 extern "C" long smat_internal_compact_chunk(long steps, size_t rows, long longest, size_t n_cap) { return smat::split_chunk_steps(steps, rows, longest, n_cap); }
 // Test hooks for the deal of the compact kernel's workgroups to the XCDs: a run length that every launch uses

@@ -127,6 +127,8 @@ struct CompactPlan {
     float *d_workspace = nullptr; // n_slots * 16 * n_cap floats
     int n_items = 0, n_tasks = 0, n_split_rows = 0, n_slots = 0;
     bool ordered = false;         // the tasks lie as order_tasks deals them: workgroup i to XCD i % 8
+    bool by_name = false;         // the plan was asked for this kernel or for mixed dispatch, whose products have the same bits as it
+    bool may_share = false;       // the steps of a task between wavefronts: every task is one item
     int64_t n_steps = 0;          // of 32 columns, of all block rows listed
     int64_t n_cols = 0;           // nonzero block columns listed (without padding)
     int64_t n_entries = 0;        // nonzeros listed one by one
@@ -283,6 +285,7 @@ struct ResidentPlan {
 hipError_t resident_build(const CompactPlan &c, size_t M, size_t K, int64_t nnz, ResidentPlan **out);
 void resident_destroy(ResidentPlan *p);
 bool resident_forced(); // by the test hook
+bool resident_holds(size_t K); // two columns of B
 double resident_estimate_us(size_t M, size_t K, size_t N, int64_t nnz, bool long_rows); // before the lists are there; 1e30: K too long
 void resident_settle(ResidentPlan &p, size_t K, size_t N); // the launch of width N
 ResidentLaunch resident_launch(const ResidentPlan &p, size_t K, size_t N);

@@ -553,6 +553,7 @@ ResidentLaunch resident_launch(const ResidentPlan &p, size_t K, size_t N)
     return N == p.n && !g_force_columns ? p.own : best_launch(p, K, N);
 }
 bool resident_forced() { return g_force_columns > 0; }
+bool resident_holds(size_t K) { return lds_of(K, 2) <= MAX_LDS; }
 
 hipError_t launch_resident(const SpmmArgs &a, const ResidentPlan &p, const ResidentLaunch &l, hipStream_t st)
 {
@@ -573,7 +574,7 @@ void resident_destroy(ResidentPlan *p)
 hipError_t resident_build(const CompactPlan &c, size_t M, size_t K, int64_t nnz, ResidentPlan **out)
 {
     *out = nullptr;
-    if (c.n_items == 0 || nnz <= 0 || nnz > 0x3fffffff || M + (size_t)nnz / 32 >= PADDED || lds_of(K, 2) > MAX_LDS) return hipSuccess;
+    if (c.n_items == 0 || nnz <= 0 || nnz > 0x3fffffff || M + (size_t)nnz / 32 >= PADDED || !resident_holds(K)) return hipSuccess;
     ResidentPlan *p = new (std::nothrow) ResidentPlan();
     if (!p) return hipErrorOutOfMemory;
     // A shared row takes a place for every 32 of its nonzeros or fewer.  Fours: those of the nonzeros, one more a slice for the first words, PART / 4 + 1 a
