@@ -419,12 +419,12 @@ __global__ __launch_bounds__(256) void copy_blocks_kernel(const uint16_t *__rest
 // the values of equal k into dwords and writes them to the transposed tile; then every thread
 // reads 8 n of one k back (two 8-byte LDS reads) and stores 16 bytes.  COLS = 64; 16 and 32 for a B of no more columns.
 // The output is split into panels of `panel` columns, each a K x panel row-major matrix of leading
-// dimension ld, one panel after the other (panel >= N and ld = N: plain row-major K x N).
+// dimension ld, the last one last_ld, one panel after the other (panel >= N and ld = N: plain row-major K x N).
 // place != NULL: row k goes to row place[k] of a copy of `rows` rows, or nowhere (-1).
 // STREAM: B does not stay in the caches behind the loads, which leaves them to the copy (launch_transpose).
 template <int COLS, bool STREAM>
 __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__restrict__ B, uint16_t *__restrict__ Bt,
-                                                          int N, long K, int panel, long ld, long rows, const int32_t *__restrict__ place)
+                                                          int N, long K, int panel, long ld, long last_ld, long rows, const int32_t *__restrict__ place)
 {
     constexpr int KT = 4096 / COLS; // k of a tile
     constexpr int LD = COLS + 4; // halfs per LDS row (k): 8-byte aligned rows, dword writes spread over the banks
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__rest
         if (to[half] >= 0 && n0 + piece * 8 < N) {
             const uint2 lo = *reinterpret_cast<const uint2 *>(tile + k * LD + piece * 8);
             const uint2 hi = *reinterpret_cast<const uint2 *>(tile + k * LD + piece * 8 + 4);
-            uint16_t *out = Bt + (long)(n0 / panel) * rows * panel + to[half] * ld + n0 % panel + piece * 8;
+            uint16_t *out = Bt + (long)(n0 / panel) * rows * panel + to[half] * (n0 / panel == (N - 1) / panel ? last_ld : ld) + n0 % panel + piece * 8;
             *reinterpret_cast<u32x4 *>(out) = (u32x4){lo.x, lo.y, hi.x, hi.y};
         }
     }
@@ -469,12 +469,12 @@ __global__ __launch_bounds__(256) void transpose_b_kernel(const uint16_t *__rest
 // A B of half of the memory-side cache and more is not there any more when the next launch reads it, so it need not displace
 // the copy and the lists on its way through (R-MAT scale 20, N = 128, 256 MiB: 485 -> 472 us).  A smaller one may be
 // (27-point stencil 64^3, N = 64, 33 MB, the same B again: 41.0 us, past the caches 44.3).
-static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, size_t K, int panel, long ld, long rows, const int32_t *place, hipStream_t st)
+static hipError_t launch_transpose(const uint16_t *B, uint16_t *Bt, size_t N, size_t K, int panel, long ld, long last_ld, long rows, const int32_t *place, hipStream_t st)
 {
     auto launch = [&](auto cols, auto stream) {
         constexpr int COLS = decltype(cols)::value;
         const dim3 grid((unsigned)((K + 4096 / COLS - 1) / (4096 / COLS)), (unsigned)((N + COLS - 1) / COLS));
-        hipLaunchKernelGGL((transpose_b_kernel<COLS, decltype(stream)::value>), grid, dim3(256), 0, st, B, Bt, (int)N, (long)K, panel, ld, rows, place);
+        hipLaunchKernelGGL((transpose_b_kernel<COLS, decltype(stream)::value>), grid, dim3(256), 0, st, B, Bt, (int)N, (long)K, panel, ld, last_ld, rows, place);
     };
     using std::false_type;
     using std::integral_constant;
@@ -544,7 +544,7 @@ template <int W, bool C_F32, bool C_ACC, int AF, bool STAGED, bool BIG>
 __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const uint16_t *__restrict__ acol, const uint32_t *__restrict__ entries, const int2 *__restrict__ step_range, const int32_t *__restrict__ cols,
     const uint16_t *__restrict__ Bt, void *__restrict__ Cout, float *__restrict__ workspace, const WorkItem *__restrict__ items,
-    const int4 *__restrict__ tasks, int n_tasks, int N, int n_panels, long panel_stride, long row_stride, unsigned xcd_run, bool shared)
+    const int4 *__restrict__ tasks, int n_tasks, int N, int n_panels, long panel_stride, long row_stride_of_most, long last_row_stride, unsigned xcd_run, bool shared)
 {
     constexpr int TQ = W > 64 ? 2 : 1, PW = W / TQ, T = PW / 16; // a row of PW columns is gathered by PW / 8 lanes, 32 rows by T instructions
     constexpr int A_BYTES = 1024, B_BYTES = 64 * W, I_BYTES = 2048;
@@ -591,7 +591,8 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const int i16 = lane & 15, g = lane >> 4;
     const int n0 = panel * W;
     // Row `col` of this panel of B starts at Bp + col * row_stride (B in place: panel_stride = W, row_stride = N; the
-    // transposed copy: panels one after the other, row_stride = W).
+    // transposed copy: panels one after the other, row_stride = W, in the last one no more than it needs).
+    const long row_stride = panel == n_panels - 1 ? last_row_stride : row_stride_of_most;
     const uint16_t *Bp = Bt + (long)panel * panel_stride;
     int boff[TQ]; // N % 8 == 0: all of the lane's columns or none (then its column 0)
 #pragma unroll
@@ -856,18 +857,29 @@ int compact_share(const CompactPlan &p, long total)
     return total > 400 || p.n_steps < 12 * (int64_t)p.n_tasks ? 2 : 4;
 }
 
+// Halves from row to row of the copy's last panel: 8, 16, 32, .. as many as hold the columns that are left, so that what is gathered at random lies on as few lines as may be.
+// A panel of 8 columns on rows of 128 bytes fills eight times the lines of the L2s.  Rows of the panel's width -> these, us: R-MAT scale 17, 10 a row, N = 72 42.3 -> 39.9; 18, 13, N = 136
+// 140.6 -> 133.5; 19, 14, N = 200 425 -> 396; 19, 12, N = 8 51.6 -> 44.0; where the columns fill the panel equal.
+long last_panel_width(size_t N, int panel)
+{
+    long width = 8;
+    while (width < (long)((N - 1) % (size_t)panel) + 1) width *= 2;
+    return width;
+}
+
 template <int W>
 hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
 {
     const CompactPlan &p = *a.plan;
     constexpr int PANEL = W;
     const int n_panels = (int)((a.N + PANEL - 1) / PANEL);
-    long panel_stride = PANEL, row_stride = (long)a.N;
+    long panel_stride = PANEL, row_stride = (long)a.N, last_row_stride = row_stride;
     const int32_t *cols = p.d_cols;
     if (!a.b_row_major) {
         const long rows = p.d_place ? (long)p.n_placed : (long)a.K; // of the copy
         if (p.d_place) cols = p.d_cols_placed;
-        const hipError_t e = launch_transpose(a.B, a.Bt, a.N, a.K, PANEL, PANEL, rows, p.d_place, st);
+        last_row_stride = last_panel_width(a.N, PANEL);
+        const hipError_t e = launch_transpose(a.B, a.Bt, a.N, a.K, PANEL, PANEL, last_row_stride, rows, p.d_place, st);
         if (e != hipSuccess) return e;
         panel_stride = rows * PANEL;
         row_stride = PANEL;
@@ -897,7 +909,7 @@ hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
     auto launch = [&](auto af, auto staged, auto f32, auto acc, auto wide) {
         hipLaunchKernelGGL((spmm_compact_kernel<W, decltype(f32)::value, decltype(acc)::value, decltype(af)::value, decltype(staged)::value, decltype(wide)::value>),
                            dim3((unsigned)wgs), dim3(64 * waves), (size_t)(waves * compact_lds_bytes(W, decltype(staged)::value)), st, p.d_acol, p.d_entries, p.d_step_range, cols, a.Bt, a.C, p.d_workspace,
-                           p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, (unsigned)xcd_run, share > 1);
+                           p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, last_row_stride, (unsigned)xcd_run, share > 1);
     };
     using std::false_type;
     using std::true_type;
@@ -931,7 +943,7 @@ using Scratch = DevScratch;
 // two dimensions swapped (N % 8 == 0 and K % 16 == 0 keep every 16-byte access aligned).
 hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, size_t N, size_t K, hipStream_t st)
 {
-    return launch_transpose(B_row_major, out, K, N, 0x7fffffff, (long)K, (long)N, nullptr, st);
+    return launch_transpose(B_row_major, out, K, N, 0x7fffffff, (long)K, (long)K, (long)N, nullptr, st);
 }
 
 // The columns of a panel of a launch.  A product of up to 16 or 32 columns takes panels of that many: a row of B is then 32 or 64 bytes, a step
