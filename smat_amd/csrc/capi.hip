@@ -101,10 +101,10 @@ hipError_t smat_plan::SweepDev::upload(const SweepPlanHost &h, bool b_row_major)
     up((void **)&d_op_ptr, h.op_ptr.data(), h.op_ptr.size() * sizeof(int32_t));
     up((void **)&d_row_map, h.row_map.data(), h.row_map.size() * sizeof(int32_t));
     std::vector<SweepOp> streams;
-    encode_sweep_streams(h.rg_chunk_ptr, h.op_ptr, h.ops.data(), false, streams);
+    encode_sweep_streams(h.rg_chunk_ptr, h.op_ptr, h.ops.data(), false, streams, h.light);
     up((void **)&d_ops, streams.data(), streams.size() * sizeof(SweepOp));
     if (b_row_major) {
-        encode_sweep_streams(h.rg_chunk_ptr, h.op_ptr, h.ops.data(), true, streams);
+        encode_sweep_streams(h.rg_chunk_ptr, h.op_ptr, h.ops.data(), true, streams, h.light);
         up((void **)&d_ops_row_major, streams.data(), streams.size() * sizeof(SweepOp));
     }
     if (e != hipSuccess) release();
@@ -168,6 +168,17 @@ static bool sweep_fills_device(size_t mb, size_t n)
     return n_rg * n_panels >= 256;
 }
 
+// Light streams (sweep_format.h) where a wavefront has few blocks in a chunk: a chunk is then as long as the copies of the one after the next take to come, which
+// may be two chunks' time, at the price of pairs of blocks two chunks apart and of a choice between three chunks to run an op in.  All other streams -> light, us, by the blocks of
+// a wavefront in a chunk: 2.7 (1216 x 13840, 9 %, N = 1888) 47.1 -> 38.3, 3.5 (4544 x 9520, 3 %, N = 4088) 86.6 -> 75.4, 4.3 (3088 x 4112, 15 %, N = 1000, fp32) 22.6 -> 21.0, 4.8 (4544 x 15056, 15 %,
+// N = 768) 52.3 -> 44.3, 6.4 (8192^2, 10 %, N = 640) 27.5 -> 26.0; 6 to 8, 18 products, 0.99 to 1.06 of the time saved; 9 (9312 x 11360, 8 %, N = 1384) 47.3 -> 48.0, 13 (8192^2, 10 %, N = 4096) 94.8 -> 97.3.
+static int g_force_light = 0; // test hook: 1 = all streams are light, -1 = none
+static bool sweep_light(size_t listed_chunks, size_t nnzb)
+{
+    if (g_force_light) return g_force_light > 0;
+    return (double)nnzb <= 8.0 * (double)listed_chunks * SWEEP_WAVES;
+}
+
 // Time of a product with fp16 results through the sweep kernel, from the tiles (row groups x panels of 64 columns, one
 // workgroup of a compute unit each), the chunks that the row groups list together and the blocks of a wavefront per chunk: a
 // tile costs 0.65 us, a chunk 0.74 us, which it takes however few blocks it has, or 0.35 us and 0.058 per block where a
@@ -178,30 +189,34 @@ static bool sweep_fills_device(size_t mb, size_t n)
 //   3088 x 4112, 15 %, N = 1000:  18.1 (19.1) / 19.3 (19.5) / 25.1 (25.7)
 //   8192 x 8192, 10 %, N = 640:   55.2 (49.6) / 30.8 (28.7) / 42.3 (36.2); N = 1536: 84.5 (77.7) / 60.1 (55.8) / 47.1 (43.2)
 //   768 x 3072, 10 %, N = 4096:   14.6 (13.7) / 14.6 (14.9) / 16.7 (16.7)
-static double sweep_estimate_us(size_t n_rg, size_t listed_chunks, size_t nnzb, size_t M, size_t N)
+// Light streams, measured since: a chunk takes 0.61 to 0.65 us however few blocks it has.
+static double sweep_estimate_us(size_t n_rg, size_t listed_chunks, size_t nnzb, size_t M, size_t N, bool may_be_light = true)
 {
     if (n_rg == 0 || listed_chunks == 0) return 1e30;
     const size_t tiles = n_rg * ((N + 16 * SWEEP_TN - 1) / (16 * SWEEP_TN)), rounds = (tiles + 255) / 256;
     const double blocks = (double)nnzb / ((double)listed_chunks * SWEEP_WAVES);
-    const double chunk = std::max(0.7418, 0.3533 + 0.058275 * blocks);
+    const double chunk = std::max(may_be_light && sweep_light(listed_chunks, nnzb) ? 0.63 : 0.7418, 0.3533 + 0.058275 * blocks);
     return 3.0 + (double)rounds * (0.65 + (double)listed_chunks / (double)n_rg * chunk) + 0.66e-6 * (double)M * (double)N;
 }
 // The same through the row-wise kernel, fitted to those of 239 products that it can lose: the rounds of 1024 wavefronts that
 // rowwise_panel_tiles counts and the blocks of an item, or the blocks of all where four wavefronts share an item, behind the
 // repack of B.  Standard deviation 7 % on repacked B, 12 % in place, 20 % with shared items.  Estimate (measured), us: 8192^2, 10 %,
 // N = 640 40.1 (41.7); 5008 x 3008, 20 %, N = 800 25.9 (25.2); 1040 x 16384, 35 %, N = 1000 83.4 (78.4); 768 x 3072, 10 %,
-// N = 4096, in place 21.7 (20.7); too high for narrow bands, whose rows share B (16384, 64, N = 1024: 55, measured 44.6).
-static double rowwise_estimate_us(size_t M, size_t K, size_t N, size_t nnzb, size_t n_items, RowLengths lengths, bool packed)
+// N = 4096, in place 21.7 (20.7); shared items in place, since they load no operands twice, 1472 x 9888, 18 %, N = 328 28.7 (25.7), 768 x 10912, 15 %, N = 240 10.6 (10.2); too high for narrow bands, whose rows share B (16384, 64, N = 1024: 55, measured 44.6).
+// beside_sweep: in place, a last round of few wavefronts counts half (1472 x 9888, 18 %, N = 328 28.9, whole 36.6 (25.7); 3328 x 12192, 5 %, N = 352 20, 24 (17.6); 928 x 13648, 13 %, N = 1304 55, 68 (42.5)).
+static double rowwise_estimate_us(size_t M, size_t K, size_t N, size_t nnzb, size_t n_items, RowLengths lengths, bool packed, bool beside_sweep = false)
 {
     n_items = std::max<size_t>(n_items, 1);
     const size_t avg = nnzb / n_items;
     const double start = 0.6e-6 * (double)M * (double)N + (packed ? 5.6 + 0.6e-6 * (double)K * (double)N : 2.7);
     if (rowwise_shares_items(N, n_items, avg))
-        return start + (double)nnzb * (double)((N + 63) / 64) / 256.0 * (packed ? 0.047 : 0.14);
+        return start + (double)nnzb * (double)((N + 63) / 64) / 256.0 * (packed ? 0.047 : 0.105);
     const size_t tiles = (size_t)rowwise_panel_tiles(N, n_items, avg, lengths, packed);
-    const size_t rounds = (n_items * ((N + 16 * tiles - 1) / (16 * tiles)) + 1023) / 1024;
+    const size_t wavefronts = n_items * ((N + 16 * tiles - 1) / (16 * tiles));
+    double rounds = (double)((wavefronts + 1023) / 1024);
+    if (beside_sweep && !packed) rounds = 0.5 * rounds + 0.5 * (double)wavefronts / 1024.0;
     const double column = !packed || tiles <= 4 ? 1.0 : tiles == 8 ? 0.83 : 0.8;
-    return start + (double)rounds * (double)tiles * (double)nnzb / (double)n_items * (packed ? 0.0274 * column : 0.074);
+    return start + rounds * (double)tiles * (double)nnzb / (double)n_items * (packed ? 0.0274 * column : 0.074);
 }
 // The same on B in place up to 14 us, with what neighbouring block rows find of each other's rows of B in the caches: share4, block columns of a group of four
 // rows per block.  Fitted to 1,600 products (bands, stencils and random patterns, N = 24 to 4,096): 7 to 8 % standard deviation, where the estimate above is 20 % too high
@@ -263,14 +278,14 @@ static size_t sweep_even_rounds(const int32_t *row_ptr, const int32_t *col_idx, 
     const size_t nnzb = (size_t)row_ptr[mb], n64 = (mb + SWEEP_G - 1) / SWEEP_G;
     if (nnzb == 0 || n64 == 0) return SWEEP_G;
     const size_t listed = sweep_listed_chunks(row_ptr, col_idx, mb, kb, SWEEP_G);
-    const double whole = sweep_estimate_us(n64, listed, nnzb, 16 * mb, N);
+    const double whole = sweep_estimate_us(n64, listed, nnzb, 16 * mb, N, false); // light streams gain either way
     double best = 0.9 * whole;
     size_t rows = SWEEP_G;
     for (size_t n_rg = n64 + 1; n_rg <= 2 * n64; n_rg++) {
         const size_t g = (mb + n_rg - 1) / n_rg;
         if ((mb + g - 1) / g != n_rg) continue;
         if (b_row_major && sweep_takes_row_major(N, 16 * kb, (int)n64) && !sweep_takes_row_major(N, 16 * kb, (int)n_rg)) break; // stays in place
-        const double t = sweep_estimate_us(n_rg, (listed * n_rg + n64 - 1) / n64, nnzb, 16 * mb, N);
+        const double t = sweep_estimate_us(n_rg, (listed * n_rg + n64 - 1) / n64, nnzb, 16 * mb, N, false);
         if (t < best) best = t, rows = g;
     }
     return rows;
@@ -782,8 +797,8 @@ static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
     }
     if (e == hipSuccess && sweep) {
         SweepPlanHost h;
-        build_sweep_plan(row_ptr_host, col_idx_host, mb, kb, h, nullptr, 0,
-                         want == SMAT_KERNEL_AUTO ? sweep_even_rounds(row_ptr_host, col_idx_host, mb, kb, n_hint, p->d_bcol != nullptr) : SWEEP_G);
+        const size_t group_rows = want == SMAT_KERNEL_AUTO ? sweep_even_rounds(row_ptr_host, col_idx_host, mb, kb, n_hint, p->d_bcol != nullptr) : SWEEP_G;
+        build_sweep_plan(row_ptr_host, col_idx_host, mb, kb, h, nullptr, 0, group_rows, 2e8, sweep_light(sweep_listed_chunks(row_ptr_host, col_idx_host, mb, kb, group_rows), nnzb));
         p->kernel = SMAT_KERNEL_SWEEP;
         static_assert(sizeof(SweepOpHost) == sizeof(SweepOp), "host and device op layouts");
         e = p->sweep.upload(h, p->d_bcol != nullptr);
@@ -819,6 +834,12 @@ extern "C" int smat_plan_create(smat_plan **out, const int32_t *row_ptr_host,
 // 40.0 -> 22.1, N = 1000 24.5 -> 19.9; 768 x 3072, 30 %, N = 4096: 29.6 -> 15.4; bands, whose row groups list few chunks: 16384 rows,
 // bandwidth 64, N = 1024 44.6 -> 19.4; 65536, 256, N = 512 146 -> 78.  A K of one or two chunks, less than the entry fetches, stays
 // with the row-wise kernel.  Returns the block rows of a group, 0 = row-wise.
+// As many block rows in every group (1056 x 7856, 5 %, N = 2176, fp32, groups of 64 and 2 rows 35.5 us, of 33 28.5, row-wise 23.4).
+static size_t even_rows(size_t mb, size_t group_rows)
+{
+    const size_t n_rg = (mb + group_rows - 1) / group_rows;
+    return (mb + n_rg - 1) / n_rg;
+}
 static int g_force_group_rows = 0; // test hook: 64, 32 or 16 whatever the estimates say
 static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, size_t n_items,
                                RowLengths lengths, bool packed, bool b_row_major, double *us = nullptr)
@@ -827,14 +848,14 @@ static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, s
     if (nnzb < 2 || nnzb >= (size_t)1 << 23 || K >= (size_t)1 << 28 || kb <= 2 * SWEEP_S) return 0;
     if (g_force_group_rows) return (size_t)g_force_group_rows;
     const double to_col_major = b_row_major ? to_col_major_us(K, N) : 0.0;
-    double row_wise = rowwise_estimate_us(M, K, N, nnzb, n_items, lengths, packed) + to_col_major;
+    double row_wise = rowwise_estimate_us(M, K, N, nnzb, n_items, lengths, packed, true) + to_col_major;
     if (b_row_major) row_wise = std::min(row_wise, rowwise_row_major_us(M, N, nnzb));
     // (the estimate on a row-major B in place errs to either side)
-    double best = std::min(row_wise / (b_row_major ? 1.0 : packed ? 1.1 : 1.2), row_wise - 0.11e-3 * (double)nnzb);
+    double best = std::min(row_wise / (b_row_major ? 1.05 : packed ? 1.1 : 1.2), row_wise - 0.11e-3 * (double)nnzb);
     size_t group_rows = 0;
     for (size_t rows : {(size_t)SWEEP_G, (size_t)SWEEP_G / 2, (size_t)SWEEP_G / 4}) {
         const size_t n_rg = (mb + rows - 1) / rows;
-        const double sweep = sweep_estimate_us(n_rg, sweep_listed_chunks(row_ptr, col_idx, mb, kb, rows), nnzb, M, N);
+        const double sweep = sweep_estimate_us(n_rg, sweep_listed_chunks(row_ptr, col_idx, mb, kb, even_rows(mb, rows)), nnzb, M, N);
         const bool in_place = b_row_major && sweep_takes_row_major(N, K, (int)n_rg);
         const double t = in_place ? sweep_in_place_factor(N) * sweep : sweep + to_col_major;
         if (t < best) best = t, group_rows = rows;
@@ -850,6 +871,7 @@ extern "C" int smat_internal_sweep_even_rounds(const int32_t *row_ptr, const int
 // Test hooks (not part of smat.h): row groups of 64, 32 or 16 wherever the sweep kernel may be taken at all (0 = the
 // choice, the default), and the choice itself.
 extern "C" void smat_internal_sweep_force_groups(int rows) { g_force_group_rows = rows; }
+extern "C" void smat_internal_sweep_force_light(int what) { g_force_light = what; }
 extern "C" int smat_internal_sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, int packed)
 {
     return (int)sweep_group_rows(row_ptr, col_idx, M, K, nnzb, N, M / 16, RowLengths::EVEN, packed != 0, false);
@@ -863,7 +885,8 @@ static hipError_t sweep_small_groups(smat_plan &p, size_t group_rows)
     const size_t mb = p.M / 16, kb = p.K / 16, nnzb = p.nnzb;
     const int32_t *row_ptr = p.row_ptr_host.data(), *col_idx = p.col_idx_host.data();
     SweepPlanHost h;
-    build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 16.0 * (double)nnzb);
+    group_rows = even_rows(mb, group_rows);
+    build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 16.0 * (double)nnzb, sweep_light(sweep_listed_chunks(row_ptr, col_idx, mb, kb, group_rows), nnzb));
     const hipError_t e = p.sweep.upload(h, p.d_bcol != nullptr);
     if (e != hipSuccess) {
         p.sweep.release();

@@ -10,7 +10,8 @@ to the block of the next descriptor.  A block is specialised for
     r  the block row of the wavefront the op adds to (which accumulators),
     v  whether the copies of a chunk boundary were issued between the load of its A operand and now (which s_waitcnt vmcnt),
 
-and a chunk boundary for the ops of the chunk it ends (2, 3, .., 7 or more: again an s_waitcnt),
+and a chunk boundary for the ops of the chunk it ends (2, 3, .., 7 or more: again an s_waitcnt), or, in light streams, of
+the two chunks before it (4, 5, 6, 7 or more, and the copies between them),
 
 so the run-time choices cost no instruction besides the jump.  It is written by hand because a
 wavefront issues in order: every instruction next to its MFMAs adds to its run time.  Blocks have a
@@ -67,6 +68,7 @@ N_BLOCKS = 8 * 8 * 2                     # SWEEP_N_BLOCKS: stream position % 8 x
 TRAMP_BYTES = 8                          # SWEEP_TRAMP_BYTES
 MIN_OPS, MARKS = 2, 6                    # SWEEP_DEV_MIN_OPS, SWEEP_DEV_MARKS: boundaries after chunks of 2, 3, .., 7 and more ops
 MARK_BYTES = 512                         # SWEEP_MARK_BYTES
+LIGHT_MARKS, LIGHT_GAP = 4, 64           # SWEEP_LIGHT_MARKS, SWEEP_LIGHT_GAP: boundaries of light streams, behind the end
 COPIES = 4
 TOUCHES = 2                              # loads of the entry code that bring A into the caches
 
@@ -95,6 +97,10 @@ def tramp_base():
 
 def mark_off():
     return tramp_base() + MARKS * N_BLOCKS * TRAMP_BYTES
+
+
+def light_base():
+    return mark_off() + MARK_BYTES + LIGHT_GAP
 
 
 def ring(slot, word):
@@ -188,7 +194,10 @@ def op_block(J, r, v):
 def trampoline(m, k):
     emit(f"s_movk_i32 s{S_RET}, {k * block_bytes()}")
     emit(f"s_branch Lmark{m}_%=")
-    emit(f".org Lb0_%= + {tramp_base() + (m * N_BLOCKS + k + 1) * TRAMP_BYTES}")
+    if m < MARKS:
+        emit(f".org Lb0_%= + {tramp_base() + (m * N_BLOCKS + k + 1) * TRAMP_BYTES}")
+    else:
+        emit(f".org Lb0_%= + {light_base() + ((m - MARKS) * N_BLOCKS + k + 1) * TRAMP_BYTES}")
 
 
 def boundary_code():
@@ -278,19 +287,32 @@ def loop():
     boundary_code()
     label("Lend")                                         # offset END_OFF: the descriptor after the last op jumps here
     emit("s_waitcnt vmcnt(0) lgkmcnt(0)")
+    # Light streams: an op runs in the chunk of its later block or the one after it, so the copies of a boundary have two chunks' time.
+    # Those of the chunk being entered have landed: since then the chunks before it have issued the copies of the next one and
+    # 2 * MIN_OPS + l A loads or more.
+    emit("s_branch Lout_%=")
+    emit(f".org Lb0_%= + {light_base()}")
+    for l in range(LIGHT_MARKS):
+        for k in range(N_BLOCKS):
+            trampoline(MARKS + l, k)
+    for l in range(LIGHT_MARKS):
+        label(f"Lmark{MARKS + l}")
+        emit(f"s_waitcnt vmcnt({COPIES + 2 * MIN_OPS + l})")
+        emit("s_branch Lmark_%=")
+    label("Lout")
 
 
 clob = ([f'"v{i}"' for i in range(V_B0, V_TOUCH + 1)] + [f'"s{i}"' for i in range(S_RING0, S_LAST + 1)] +
         [f'"a{i}"' for i in range(128)] + ['"vcc"', '"scc"', '"memory"'])
 print("// generated by gen_sweep_loop.py; do not edit")
 print(f"static_assert(SWEEP_DEV_AHEAD == {AHEAD} && SWEEP_DEV_MIN_OPS == {MIN_OPS} && SWEEP_DEV_MARKS == {MARKS} && SWEEP_N_BLOCKS == {N_BLOCKS} && "
-      f"SWEEP_TRAMP_BYTES == {TRAMP_BYTES} && SWEEP_MARK_BYTES == {MARK_BYTES}, \"regenerate spmm_sweep_loop.inc\");")
+      f"SWEEP_TRAMP_BYTES == {TRAMP_BYTES} && SWEEP_MARK_BYTES == {MARK_BYTES} && SWEEP_LIGHT_MARKS == {LIGHT_MARKS} && SWEEP_COPIES == {COPIES}, \"regenerate spmm_sweep_loop.inc\");")
 for ROW_MAJOR in (True, False):
     out.clear()
     loop()
     b = "true" if ROW_MAJOR else "false"
     print("#ifdef SMAT_SWEEP_ROW_MAJOR" if ROW_MAJOR else "#else")
-    print(f"static_assert(sweep_block_bytes({b}) == {block_bytes()} && sweep_tramp_base({b}) == {tramp_base()} && sweep_end_off({b}) == {mark_off() + MARK_BYTES}, "
+    print(f"static_assert(sweep_block_bytes({b}) == {block_bytes()} && sweep_tramp_base({b}) == {tramp_base()} && sweep_end_off({b}) == {mark_off() + MARK_BYTES} && sweep_light_base({b}) == {light_base()}, "
           f"\"regenerate spmm_sweep_loop.inc\");")
     print("asm volatile(")
     for line in out:

@@ -64,6 +64,12 @@ constexpr uint32_t SWEEP_END_OFF = SWEEP_MARK_OFF + SWEEP_MARK_BYTES;           
 //               SWEEP_TRAMP_BYTES, m = min(ops of the chunk before, AHEAD) - SWEEP_DEV_MIN_OPS: so many more A loads than
 //               SWEEP_DEV_MIN_OPS may be under way when the boundary's own copies have landed
 //       end     sweep_end_off
+// Light streams, for row groups whose wavefronts have little to do in a chunk: an op runs in the chunk of its later block or the one after,
+// so that the copies of a boundary may take two chunks' time.
+//       first op of every chunk but the first:  where copies were issued by the boundary before, sweep_light_base + (l * SWEEP_N_BLOCKS +
+//               the op's block index) * SWEEP_TRAMP_BYTES, l = min(ops of the two chunks before, AHEAD) - 2 SWEEP_DEV_MIN_OPS: as many A
+//               loads and SWEEP_COPIES more may be under way when the copies of the chunk being entered have landed; where not, as above with the ops
+//               of both chunks; both blocks of that op are in the chunk before (its LDS reads are issued before the barrier)
 // The two loops (column-major and row-major B) have blocks of different sizes.
 constexpr int SWEEP_DEV_AHEAD = 7; // with a ring of eight operands the most there is room for
 constexpr int SWEEP_DEV_HEAD = 2;
@@ -72,6 +78,8 @@ constexpr int SWEEP_DEV_MARKS = SWEEP_DEV_AHEAD - SWEEP_DEV_MIN_OPS + 1;
 constexpr uint32_t sweep_block_bytes(bool row_major) { return row_major ? 192 : SWEEP_BLOCK_BYTES; }
 constexpr uint32_t sweep_tramp_base(bool row_major) { return SWEEP_N_BLOCKS * sweep_block_bytes(row_major); }
 constexpr uint32_t sweep_end_off(bool row_major) { return sweep_tramp_base(row_major) + SWEEP_DEV_MARKS * SWEEP_N_BLOCKS * SWEEP_TRAMP_BYTES + SWEEP_MARK_BYTES; }
+constexpr int SWEEP_LIGHT_MARKS = SWEEP_DEV_AHEAD - 2 * SWEEP_DEV_MIN_OPS + 1;
+constexpr uint32_t sweep_light_base(bool row_major) { return sweep_end_off(row_major) + 64; }
 static_assert(SWEEP_DEV_AHEAD <= 4 * SWEEP_DEV_HEAD && SWEEP_DEV_AHEAD > SWEEP_DEV_MIN_OPS, "the head holds the offsets of the first ops");
 
 inline uint32_t sweep_lds_offset(int32_t chunk_pos, int32_t slab)

@@ -70,8 +70,9 @@ long sum_of_caps(const int16_t *win, size_t n, const int16_t *ri, const int16_t 
 } // namespace
 
 void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, SweepPlanHost &out,
-                      const int32_t *rows, size_t n_rows, size_t group_rows, double search)
+                      const int32_t *rows, size_t n_rows, size_t group_rows, double search, bool light)
 {
+    const int32_t lead = light ? 0 : 1; // chunks past the one being swept that an op may use
     if (!rows) n_rows = mb;
     const size_t GR = std::min<size_t>(std::max<size_t>(group_rows, 1), G); // block rows that share a group's 64 places
     const size_t n_rg = (n_rows + GR - 1) / GR;
@@ -119,6 +120,7 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
     const size_t n_kchunks = (kb + S - 1) / S;
     const int32_t nnzb = row_ptr[mb];
     out = SweepPlanHost();
+    out.light = light;
     out.rg_chunk_ptr.assign(n_rg + 1, 0);
     out.op_ptr.reserve(n_rg * WAVES + 1);
     out.row_map.assign(n_rg * G, -1);
@@ -158,7 +160,7 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
                 if (q + 1 < q_end) {
                     const int32_t bc1 = col_idx[q + 1] / 16;
                     const int32_t cl1 = local[(size_t)bc1 / S];
-                    if (cl1 - cl0 <= 2) { // three consecutive listed chunks are resident while the middle one is swept
+                    if (cl1 - cl0 <= 1 + lead) { // three (light streams: two) consecutive listed chunks are resident while one is swept
                         op.w0 = (uint32_t)q * 512u;
                         op.w2 = sweep_lds_offset(cl1, bc1 % S) - off0;
                         cl_hi = cl1;
@@ -186,8 +188,8 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
                     }
                 }
                 // While chunk p is swept, chunks p - 1, p and p + 1 are in LDS: the op may run in any period p with
-                // p - 1 <= cl0 and cl_hi <= p + 1.
-                const int32_t first = std::max(cl_hi - 1, 0), last = std::min<int32_t>(cl0 + 1, (int32_t)n_chunks - 1);
+                // p - 1 <= cl0 and cl_hi <= p + 1 (light streams: p - 1 and p, cl_hi <= p).
+                const int32_t first = std::max(cl_hi - lead, 0), last = std::min<int32_t>(cl0 + 1, (int32_t)n_chunks - 1);
                 (pair ? out.n_pairs : out.n_singles)++;
                 row_ops[lr].push_back(RowOp{first, last, cl_hi, op});
                 q += pair ? 2 : 1;
@@ -341,9 +343,9 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
                 if (c > 0) {
                     // The LDS reads of the op that opens a chunk are issued by the op before it, before the barrier of
                     // the boundary, when the copies of chunk c + 1 may still be under way: it has to be an op whose
-                    // chunks are c or c - 1.
+                    // chunks are c or c - 1 (light streams: when those of chunk c may be, an op of chunk c - 1).
                     size_t ok = 0;
-                    while (ok < list.size() && list[ok].hi > (int32_t)c) ok++;
+                    while (ok < list.size() && list[ok].hi > (int32_t)c - 1 + lead) ok++;
                     if (ok == list.size()) {
                         items.push_back(filler);
                         out.n_fillers++;
@@ -401,9 +403,9 @@ void build_sweep_plan(const int32_t *row_ptr, const int32_t *col_idx, size_t mb,
 }
 
 void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::vector<int32_t> &op_ptr, const SweepOpHost *ops,
-                          bool b_row_major, std::vector<SweepOpHost> &dev)
+                          bool b_row_major, std::vector<SweepOpHost> &dev, bool light)
 {
-    const uint32_t block_bytes = sweep_block_bytes(b_row_major), tramp_base = sweep_tramp_base(b_row_major);
+    const uint32_t block_bytes = sweep_block_bytes(b_row_major), tramp_base = sweep_tramp_base(b_row_major), light_base = sweep_light_base(b_row_major);
     constexpr int DEV_AHEAD = SWEEP_DEV_AHEAD, DEV_MIN = SWEEP_DEV_MIN_OPS, HEAD = SWEEP_DEV_HEAD;
     const size_t n_streams = op_ptr.size() - 1;
     dev.assign((size_t)op_ptr.back() + HEAD * n_streams + SWEEP_OP_PAD, SweepOpHost{0, SWEEP_ZERO_OFF, 0, sweep_end_off(b_row_major)});
@@ -443,15 +445,21 @@ void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::v
         out += HEAD;
         // vector memory operations in issue order: what is younger than the load of an op's A operand when the op needs it
         a_issue.assign(n_ops + DEV_AHEAD + 1, 0);
-        long seq = 0, cur = 0, in_chunk = 0;
+        long seq = 0, cur = 0, in_chunk = 0, in_chunk_before = 0;
+        bool copies_before = false; // by the boundary before
         for (int k = 0; k < DEV_AHEAD; k++) a_issue[(size_t)k] = ++seq;
         for (size_t i = 0; i < n_ops; i++) {
             const bool opens = kept[i].opens;
-            uint32_t m = 0;
+            uint32_t tramp = tramp_base;
             if (opens) {
-                m = (uint32_t)(std::min<long>(in_chunk, DEV_AHEAD) - DEV_MIN);
+                const long loads = std::min<long>(in_chunk + (light ? in_chunk_before : 0), DEV_AHEAD);
+                // (cur = 0: no boundary before this one, and no two chunks)
+                tramp = light && copies_before ? light_base + (uint32_t)(loads - 2 * DEV_MIN) * SWEEP_N_BLOCKS * SWEEP_TRAMP_BYTES
+                                               : tramp_base + (uint32_t)(loads - DEV_MIN) * SWEEP_N_BLOCKS * SWEEP_TRAMP_BYTES;
+                in_chunk_before = in_chunk;
                 in_chunk = 0;
-                if (++cur + 2 < n_chunks) seq += COPIES;
+                copies_before = ++cur + 2 < n_chunks;
+                if (copies_before) seq += COPIES;
             }
             in_chunk++;
             a_issue[i + DEV_AHEAD] = ++seq;
@@ -460,7 +468,7 @@ void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::v
             out[i].w0 = a_offset(i + DEV_AHEAD - 1);
             out[i].w1 = b_row_major ? sweep_lds_offset_row_major(lo) : lo;
             out[i].w2 = (b_row_major ? sweep_lds_offset_row_major(hi) : hi) - out[i].w1;
-            out[i].w3 = opens ? tramp_base + (m * SWEEP_N_BLOCKS + code) * SWEEP_TRAMP_BYTES : code * block_bytes;
+            out[i].w3 = opens ? tramp + code * SWEEP_TRAMP_BYTES : code * block_bytes;
         }
         // the end, and what the dropped fillers leave behind it, stay what dev was filled with
     }
@@ -468,14 +476,14 @@ void encode_sweep_streams(const std::vector<int32_t> &rg_chunk_ptr, const std::v
 
 } // namespace smat
 
-// Test hook (not part of smat.h): the streams of a plan that smat_internal_sweep_plan handed out as the kernel runs them, in
+// Test hook (not part of smat.h): the streams of a plan that smat_internal_sweep_plan handed out as the kernel runs them (b_row_major + 2: of a light plan), in
 // out[0 .. op_ptr[8 n_rg] + 2 * 8 n_rg + 16).
 extern "C" int smat_internal_sweep_encode(const int32_t *rg_chunk_ptr, int64_t n_rg, const int32_t *op_ptr, const uint32_t *ops, int b_row_major, uint32_t *out)
 {
     return smat::guarded("smat_internal_sweep_encode", [&] {
         const std::vector<int32_t> chunk_ptr(rg_chunk_ptr, rg_chunk_ptr + n_rg + 1), ptr(op_ptr, op_ptr + n_rg * smat::SWEEP_WAVES + 1);
         std::vector<smat::SweepOpHost> dev;
-        smat::encode_sweep_streams(chunk_ptr, ptr, reinterpret_cast<const smat::SweepOpHost *>(ops), b_row_major != 0, dev);
+        smat::encode_sweep_streams(chunk_ptr, ptr, reinterpret_cast<const smat::SweepOpHost *>(ops), (b_row_major & 1) != 0, dev, (b_row_major & 2) != 0);
         memcpy(out, dev.data(), dev.size() * sizeof(smat::SweepOpHost));
         return (int)SMAT_OK;
     });
@@ -485,14 +493,14 @@ extern "C" int smat_internal_sweep_encode(const int32_t *rg_chunk_ptr, int64_t n
 // allocated with malloc; release each with smat_host_free.  row_map: n_rg * 64 block rows (-1 = none).  counts[0..5] = row groups, listed
 // chunks, stream entries (ops, fillers, ends; without padding), pairs, singles, fillers.
 static int smat_internal_sweep_plan_impl(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K,
-                                         const int32_t *rows, size_t n_rows, size_t group_rows, int32_t **rg_chunk_ptr, int32_t **chunk_ids, int32_t **op_ptr,
+                                         const int32_t *rows, size_t n_rows, size_t group_rows, bool light, int32_t **rg_chunk_ptr, int32_t **chunk_ids, int32_t **op_ptr,
                                          uint32_t **ops, int32_t **row_map, int64_t *counts)
 {
     if (!row_ptr || !col_idx || !rg_chunk_ptr || !chunk_ids || !op_ptr || !ops || !row_map || !counts) return SMAT_ERR_INVALID;
     if (M == 0 || M % 16 || K % 16 || row_ptr[M / 16] < 2) return SMAT_ERR_INVALID;
     smat::SweepPlanHost p;
     try {
-        smat::build_sweep_plan(row_ptr, col_idx, M / 16, K / 16, p, rows, n_rows, group_rows);
+        smat::build_sweep_plan(row_ptr, col_idx, M / 16, K / 16, p, rows, n_rows, group_rows, 2e8, light);
     } catch (...) {
         return SMAT_ERR_NOMEM;
     }
@@ -527,7 +535,7 @@ extern "C" int smat_internal_sweep_plan(const int32_t *row_ptr, const int32_t *c
                                          uint32_t **ops, int32_t **row_map, int64_t *counts)
 {
     return smat::guarded("smat_internal_sweep_plan", [&] {
-        return smat_internal_sweep_plan_impl(row_ptr, col_idx, M, K, rows, n_rows, smat::SWEEP_G, rg_chunk_ptr, chunk_ids, op_ptr, ops, row_map, counts);
+        return smat_internal_sweep_plan_impl(row_ptr, col_idx, M, K, rows, n_rows, smat::SWEEP_G, false, rg_chunk_ptr, chunk_ids, op_ptr, ops, row_map, counts);
     });
 }
 // The same on row groups of group_rows (at most 64) block rows.
@@ -536,6 +544,15 @@ extern "C" int smat_internal_sweep_plan_groups(const int32_t *row_ptr, const int
                                                int32_t **row_map, int64_t *counts)
 {
     return smat::guarded("smat_internal_sweep_plan_groups", [&] {
-        return smat_internal_sweep_plan_impl(row_ptr, col_idx, M, K, nullptr, 0, group_rows, rg_chunk_ptr, chunk_ids, op_ptr, ops, row_map, counts);
+        return smat_internal_sweep_plan_impl(row_ptr, col_idx, M, K, nullptr, 0, group_rows, false, rg_chunk_ptr, chunk_ids, op_ptr, ops, row_map, counts);
+    });
+}
+// The same for light streams.
+extern "C" int smat_internal_sweep_plan_light(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t group_rows,
+                                              int32_t **rg_chunk_ptr, int32_t **chunk_ids, int32_t **op_ptr, uint32_t **ops,
+                                              int32_t **row_map, int64_t *counts)
+{
+    return smat::guarded("smat_internal_sweep_plan_light", [&] {
+        return smat_internal_sweep_plan_impl(row_ptr, col_idx, M, K, nullptr, 0, group_rows, true, rg_chunk_ptr, chunk_ids, op_ptr, ops, row_map, counts);
     });
 }
