@@ -106,17 +106,13 @@ __device__ __forceinline__ void add_totals(const unsigned long long (&mine)[N], 
         if (v) atomicAdd(&sums[(blockIdx.x % SUM_SLOTS) * SUM_STRIDE + threadIdx.x], v);
     }
 }
-// sums[i] of the pass, from the words that add_totals added to (synchronous)
-hipError_t fetch_totals(const void *d_sums, unsigned long long *out, int n, WindowCount *widths = nullptr) // widths: what WindowCount::launch put behind them
+// sums[i] of the pass, from the words that add_totals added to
+void add_up_totals(const unsigned long long *all, unsigned long long *out, int n)
 {
-    std::vector<unsigned long long> all((SUM_BYTES + (widths ? WindowCount::BYTES : 0)) / sizeof(unsigned long long));
-    const hipError_t e = hipMemcpy(all.data(), d_sums, all.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && widths) widths->take(all.data() + SUM_BYTES / sizeof(unsigned long long));
     for (int i = 0; i < n; i++) {
         out[i] = 0;
-        for (int s = 0; s < SUM_SLOTS; s++) out[i] += all[(size_t)(s * SUM_STRIDE + i)];
+        for (int s = 0; s < SUM_SLOTS; s++) out[i] += all[s * SUM_STRIDE + i];
     }
-    return e;
 }
 // Order-independent 64-bit checksum of the block values: sum over all dwords of value * (2 * index + 1).
 __device__ __forceinline__ unsigned long long checksum_term(uint32_t v, long i)
@@ -323,13 +319,13 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint16_t *__restrict_
     }
 }
 
-// Steps of every group of 32 listed columns: one for each `most` of its entries, at least one.
+// Steps of every group of 32 listed columns: one for each `most` of its entries, at least one; none behind the last group.
 __global__ void count_steps_kernel(const int2 *__restrict__ group_range, int n_groups, int most, int32_t *__restrict__ steps)
 {
     const int g = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (g >= n_groups) return;
-    const int n = group_range[g].y - group_range[g].x;
-    steps[g] = n > most ? (n + most - 1) / most : 1;
+    if (g > n_groups) return;
+    const int n = g < n_groups ? group_range[g].y - group_range[g].x : 0;
+    steps[g] = g == n_groups ? 0 : n > most ? (n + most - 1) / most : 1;
 }
 // The groups that take several steps are listed once for each, with another part of their entries.  32 threads a group.
 __global__ __launch_bounds__(256) void expand_steps_kernel(const int2 *__restrict__ group_range, const int32_t *__restrict__ group_cols,
@@ -1072,8 +1068,9 @@ hipError_t values_checksum(const uint16_t *vals, size_t nnzb, uint64_t *out)
     const unsigned blocks = (unsigned)std::min<long>((n_quads + 255) / 256, 256L * 8);
     hipLaunchKernelGGL(values_checksum_kernel, dim3(blocks), dim3(256), 0, 0, reinterpret_cast<const u32x4 *>(vals), n_quads, (unsigned long long *)d.p);
     e = hipGetLastError();
-    unsigned long long sum = 0;
-    if (e == hipSuccess) e = fetch_totals(d.p, &sum, 1);
+    unsigned long long sum = 0, all[SUM_BYTES / 8] = {0};
+    if (e == hipSuccess) e = hipMemcpy(all, d.p, SUM_BYTES, hipMemcpyDeviceToHost);
+    add_up_totals(all, &sum, 1);
     if (e == hipSuccess) *out = sum;
     return e;
 }
@@ -1112,7 +1109,8 @@ hipError_t copy_blocks(const uint16_t *vals, const int32_t *ids_host, size_t n, 
     } while (0)
 
 // count -> offset (exclusive sums), rows (what the blocks before every block row hold) and raw, its copy on the host
-static hipError_t census_offsets(CompactCensus &s, const int32_t *row_ptr)
+// more: bytes behind the rows' sums that come along to `to`.
+static hipError_t census_offsets(CompactCensus &s, const int32_t *row_ptr, size_t more = 0, unsigned long long *to = nullptr)
 {
     hipError_t e = hipSuccess;
     Scratch tmp;
@@ -1126,7 +1124,10 @@ static hipError_t census_offsets(CompactCensus &s, const int32_t *row_ptr)
                            (long)s.nnzb, (unsigned long long *)s.rows.p);
         e = hipGetLastError();
     }
-    SMAT_STEP(hipMemcpy(s.raw.data(), s.rows.p, (s.mb + 1) * 8, hipMemcpyDeviceToHost));
+    s.raw.resize(s.mb + 1 + more / 8);
+    SMAT_STEP(hipMemcpy(s.raw.data(), s.rows.p, (s.mb + 1) * 8 + more, hipMemcpyDeviceToHost));
+    std::copy(s.raw.begin() + (long)s.mb + 1, s.raw.end(), to);
+    s.raw.resize(s.mb + 1);
     tmp.idle = e == hipSuccess;
     return e;
 }
@@ -1138,27 +1139,28 @@ hipError_t compact_census(const uint16_t *vals, const int32_t *row_ptr, size_t m
     s.nnzb = nnzb;
     s.raw.assign(mb + 1, 0);
     if (!nnzb) return e;
-    Scratch sums;
     for (Scratch *q : {&s.mask, &s.single, &s.count, &s.offset, &s.rows}) q->release();
     s.dropped = false;
     SMAT_STEP(s.mask.alloc(nnzb * 2));
     SMAT_STEP(s.single.alloc(nnzb * 4));
     SMAT_STEP(s.count.alloc(nnzb * 8));
     SMAT_STEP(s.offset.alloc(nnzb * 8));
-    SMAT_STEP(s.rows.alloc((mb + 1) * 8));
-    SMAT_STEP(sums.alloc(SUM_BYTES + WindowCount::BYTES));
-    SMAT_STEP(hipMemsetAsync(sums.p, 0, SUM_BYTES, nullptr));
-    if (e == hipSuccess && widths && !widths->launch(row_ptr, col_idx, mb, kb, nnzb, static_cast<unsigned char *>(sums.p) + SUM_BYTES)) widths = nullptr;
+    SMAT_STEP(s.rows.alloc((mb + 1) * 8 + SUM_BYTES + WindowCount::BYTES)); // the totals behind the rows' sums: one copy to the host, 13 us a copy
+    unsigned long long *const sums = static_cast<unsigned long long *>(s.rows.p) + mb + 1;
+    SMAT_STEP(hipMemsetAsync(sums, 0, SUM_BYTES, nullptr));
+    if (e == hipSuccess && widths && !widths->launch(row_ptr, col_idx, mb, kb, nnzb, sums + SUM_BYTES / 8)) widths = nullptr;
     if (e == hipSuccess) {
         const long waves = std::min<long>((long)(nnzb + 1) / 2, 256L * 32);
         hipLaunchKernelGGL(colmask_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, 0, vals, (long)nnzb,
-                           (uint16_t *)s.mask.p, (uint32_t *)s.single.p, (unsigned long long *)s.count.p, (unsigned long long *)sums.p);
+                           (uint16_t *)s.mask.p, (uint32_t *)s.single.p, (unsigned long long *)s.count.p, sums);
         e = hipGetLastError();
     }
-    SMAT_STEP(census_offsets(s, row_ptr));
-    unsigned long long total[N_SUMS] = {0};
-    SMAT_STEP(fetch_totals(sums.p, total, N_SUMS, widths));
-    sums.idle = e == hipSuccess;
+    std::vector<unsigned long long> all((SUM_BYTES + (widths ? WindowCount::BYTES : 0)) / 8);
+    SMAT_STEP(census_offsets(s, row_ptr, all.size() * 8, all.data()));
+    if (e != hipSuccess) return e;
+    unsigned long long total[N_SUMS];
+    add_up_totals(all.data(), total, N_SUMS);
+    if (widths) widths->take(all.data() + SUM_BYTES / 8);
     s.values_checksum = total[SUM_CHECK];
     s.full_blocks = (int64_t)total[SUM_FULL];
     s.cols_rest = (int64_t)total[SUM_COLS_REST];
@@ -1400,9 +1402,8 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         size_t bytes = 0;
         SMAT_STEP(steps.alloc(((size_t)n_groups + 1) * sizeof(int32_t)));
         SMAT_STEP(first.alloc(((size_t)n_groups + 2) * sizeof(int32_t))); // one more for the rows that are used
-        SMAT_STEP(hipMemsetAsync(steps.p, 0, ((size_t)n_groups + 1) * sizeof(int32_t), nullptr));
         if (e == hipSuccess) {
-            hipLaunchKernelGGL(count_steps_kernel, dim3((unsigned)((n_groups + 255) / 256)), dim3(256), 0, 0, p->d_step_range, n_groups, most, (int32_t *)steps.p);
+            hipLaunchKernelGGL(count_steps_kernel, dim3((unsigned)((n_groups + 256) / 256)), dim3(256), 0, 0, p->d_step_range, n_groups, most, (int32_t *)steps.p);
             e = hipGetLastError();
         }
         SMAT_STEP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, (int32_t *)steps.p, (int32_t *)first.p, n_groups + 1));
@@ -1534,7 +1535,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         SMAT_STEP(hipMemcpy(&n_used, count, sizeof n_used, hipMemcpyDeviceToHost));
         place_if_it_pays();
     }
-    SMAT_STEP(hipDeviceSynchronize());
+    SMAT_STEP(hipStreamSynchronize(nullptr)); // launches on other streams read the lists
 #undef SMAT_STEP
     starts.idle = used.idle = e == hipSuccess;
     if (e != hipSuccess) {
