@@ -323,6 +323,9 @@ static bool windows_beat(const smat_plan &p, const WindowPlan &shape, const Wind
 // pieces), and but for windows that are estimated to be faster, the pass over B before them included.
 static bool rowwise_stays_row_major(const smat_plan &p, const SpmmArgs &a)
 {
+    const size_t width = a.N <= 16 ? 16 : a.N <= 32 ? 32 : 64;
+    // A launch has fewer than 2^32 threads, 64 of them for a panel of an item; a repacked B takes panels of up to 256 columns.
+    if (a.b_packed && (size_t)a.n_items * ((a.N + width - 1) / width) >= ((size_t)1 << 26) - ((size_t)1 << 16)) return false;
     const double in_place = rowwise_row_major_us(a.M, a.N, a.nnzb);
     if (p.window && in_place > window_launch(a, *p.window).us + to_col_major_us(a.K, a.N)) return false;
     return !a.b_packed || in_place <= rowwise_estimate_us(a.M, a.K, a.N, a.nnzb, (size_t)p.n_items, p.n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, true) +
