@@ -235,7 +235,7 @@ static double rowwise_in_place_us(size_t M, size_t K, size_t N, size_t nnzb, siz
 // 4096, 5 to 1,000 us): 11 % standard deviation, 1 % low in the mean.
 static double rowwise_row_major_us(size_t M, size_t N, size_t nnzb)
 {
-    const size_t width = N <= 16 ? 16 : N <= 32 ? 32 : 64, panels = (N + width - 1) / width;
+    const size_t width = rowwise_row_major_width(N), panels = (N + width - 1) / width;
     return 4.8 + 0.33e-6 * (double)M * (double)N + 0.057e-6 * (double)nnzb * (double)panels * (double)(32 * width + 512);
 }
 // A row-major B into column-major order, for the kernels that do not read it in place (8192 x 4096 23 us, 4112 x 504 3 us beside
@@ -321,15 +321,21 @@ static bool windows_beat(const smat_plan &p, const WindowPlan &shape, const Wind
 // Whether a launch of the row-wise kernel reads a row-major B in place: always but for large products on a repacked B, which are 5 to 35 % slower for it (13696 x 6768, 19 %,
 // N = 2384 287 -> 391 us, 8160 x 9536, 24 %, N = 336 61 -> 72; 120 drawn products otherwise 0.44 to 0.93 of the time: a launch less, and loads of whole lines instead of 32
 // pieces), and but for windows that are estimated to be faster, the pass over B before them included.
+static bool rowwise_stays_row_major(size_t M, size_t K, size_t N, size_t nnzb, size_t n_items, RowLengths lengths, bool packed)
+{
+    // from 128 columns on a column-major launch takes wider panels, on B in place as well as repacked, and fits where this one does not
+    if (N >= 128 && !rowwise_row_major_fits(n_items, N)) return false;
+    return !packed || rowwise_row_major_us(M, N, nnzb) <= rowwise_estimate_us(M, K, N, nnzb, n_items, lengths, true) + to_col_major_us(K, N);
+}
 static bool rowwise_stays_row_major(const smat_plan &p, const SpmmArgs &a)
 {
-    const size_t width = a.N <= 16 ? 16 : a.N <= 32 ? 32 : 64;
-    // A launch has fewer than 2^32 threads, 64 of them for a panel of an item; a repacked B takes panels of up to 256 columns.
-    if (a.b_packed && (size_t)a.n_items * ((a.N + width - 1) / width) >= ((size_t)1 << 26) - ((size_t)1 << 16)) return false;
-    const double in_place = rowwise_row_major_us(a.M, a.N, a.nnzb);
-    if (p.window && in_place > window_launch(a, *p.window).us + to_col_major_us(a.K, a.N)) return false;
-    return !a.b_packed || in_place <= rowwise_estimate_us(a.M, a.K, a.N, a.nnzb, (size_t)p.n_items, p.n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, true) +
-                                          to_col_major_us(a.K, a.N);
+    if (p.window && rowwise_row_major_us(a.M, a.N, a.nnzb) > window_launch(a, *p.window).us + to_col_major_us(a.K, a.N)) return false;
+    return rowwise_stays_row_major(a.M, a.K, a.N, a.nnzb, (size_t)p.n_items, p.n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, a.b_packed != nullptr);
+}
+// Test hook (not part of smat.h): whether a launch over whole block rows reads a row-major B in place, windows aside.
+extern "C" int smat_internal_rowwise_stays_row_major(size_t M, size_t K, size_t N, size_t nnzb, size_t n_items, int packed)
+{
+    return rowwise_stays_row_major(M, K, N, nnzb, n_items, RowLengths::EVEN, packed != 0);
 }
 
 extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_ptr,

@@ -198,6 +198,8 @@ hipError_t launch_b_to_col_major(const uint16_t *B_row_major, uint16_t *out, siz
 enum class RowLengths { EVEN, SPLIT, UNKNOWN };
 int rowwise_panel_tiles(size_t N, size_t n_items, size_t avg_blocks, RowLengths lengths, bool packed);
 bool rowwise_shares_items(size_t N, size_t n_items, size_t avg_blocks);
+size_t rowwise_row_major_width(size_t N); // columns of a panel on a row-major B in place
+bool rowwise_row_major_fits(size_t n_items, size_t N); // whether such a launch has less than 2^32 threads
 bool rowwise_takes_short_rows(size_t N, size_t n_items, int most_blocks); // by the short-row kernel: B in place, no split rows
 // ---- whole blocks from windows of B in LDS (spmm_window.hip) ----
 // For matrices whose neighbouring block rows use the same block columns.

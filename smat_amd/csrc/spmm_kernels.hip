@@ -749,6 +749,14 @@ static hipError_t launch_rowwise_split(const SpmmArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
+size_t rowwise_row_major_width(size_t N) { return N <= 16 ? 16 : N <= 32 ? 32 : 64; }
+// A launch has fewer than 2^32 threads, 64 of them for a panel of an item, and is rounded up to eight runs of at most 4096 items (deal) or of an eighth of it.
+bool rowwise_row_major_fits(size_t n_items, size_t N)
+{
+    const size_t width = rowwise_row_major_width(N);
+    return n_items * ((N + width - 1) / width) < ((size_t)1 << 26) - ((size_t)1 << 16);
+}
+
 template <int PW>
 static hipError_t launch_rowwise_row_major(const SpmmArgs &a, bool shared, hipStream_t st)
 {
@@ -758,7 +766,7 @@ static hipError_t launch_rowwise_row_major(const SpmmArgs &a, bool shared, hipSt
     const long eighth = (total + 7) / 8;
     const long xcd_run = shared ? eighth : 4 * (a.deal && a.items ? (long)a.deal->run((size_t)a.n_items, n_panels) : ((total + 3) / 4 + 7) / 8);
     const long wgs = (total + 8 * xcd_run - 1) / (8 * xcd_run) * (8 * xcd_run);
-    if (wgs > 0x7fffffffL) return hipErrorInvalidValue;
+    if (wgs * 64 * (shared ? 4 : 1) >= 1L << 32) return hipErrorInvalidValue;
 #define SMAT_LAUNCH_ROW_MAJOR(F32, SHARES)                                                                                                   \
     hipLaunchKernelGGL((spmm_rowwise_row_major_kernel<PW, F32, SHARES>), dim3((unsigned)wgs), dim3(64 * SHARES), 0, st, a.vals, a.row_ptr,  \
                        a.col_idx, a.B, a.C, a.workspace, a.items, a.n_items, (int)a.N, n_panels, (unsigned)xcd_run)
@@ -779,9 +787,11 @@ hipError_t launch_rowwise(const SpmmArgs &a, hipStream_t st)
     const size_t n_items = (size_t)a.rule_items, avg = n_items ? a.nnzb / n_items : 0;
     const bool shares = rowwise_shares_items(a.N, n_items, avg);
     if (a.b_row_major) {
-        if (a.N <= 16) e = launch_rowwise_row_major<16>(a, shares, st);
-        else if (a.N <= 32) e = launch_rowwise_row_major<32>(a, shares, st);
-        else e = launch_rowwise_row_major<64>(a, shares, st);
+        switch (rowwise_row_major_width(a.N)) {
+        case 16: e = launch_rowwise_row_major<16>(a, shares, st); break;
+        case 32: e = launch_rowwise_row_major<32>(a, shares, st); break;
+        default: e = launch_rowwise_row_major<64>(a, shares, st); break;
+        }
         if (e == hipSuccess && a.n_split_rows > 0) e = launch_reduce(a.workspace, a.split_rows, a.n_split_rows, a.C, a.N, a.c_f32, st);
         return e;
     }
