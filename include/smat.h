@@ -186,7 +186,7 @@ int smat_plan_destroy(smat_plan *plan);
  * the host arrays; SMAT_ERR_INVALID when they differ.  No counterpart in the reference. */
 int smat_plan_check(const smat_plan *plan, const int32_t *row_ptr_host, const int32_t *col_idx_host,
                     size_t M, size_t K, size_t nnzb);
-/* Fills info[0..11]: kernel id, row-wise work items, split block rows, chunk size,
+/* Fills info[0..11]: kernel id, row-wise work items, split block rows, blocks of a piece of one at most,
  * workspace bytes, panel width, sweep stream entries, sweep (row group, K chunk) records,
  * bytes of the scratch for copies of B (0 = B is read in place by every launch; a plan for row-major B keeps scratch for
  * the launches that need B column-major, also where its own kernel reads B in place), nonzero block columns listed by

@@ -27,11 +27,15 @@ using namespace smat;
                              hipGetErrorString(e_), __FILE__, __LINE__);                   \
     } while (0)
 
+struct RowCuts { // of the row-wise kernel's list (rowwise_cuts)
+    long above; // rows of more blocks are cut
+    long piece; // blocks of a piece, at most
+};
 struct smat_plan {
     int kernel = SMAT_KERNEL_ROWWISE;
     int kernel_requested = SMAT_KERNEL_AUTO;
     size_t M = 0, K = 0, nnzb = 0, n_cap = 0;
-    int chunk = 0;
+    RowCuts cuts = {0, 0};
     int panel_tiles = 0;
     int n_items = 0, n_split_rows = 0, n_slots = 0;
     int max_item_blocks = 0; // blocks of the longest row-wise work item
@@ -607,8 +611,6 @@ static uint64_t pattern_fingerprint(const int32_t *row_ptr_host, const int32_t *
     return h;
 }
 
-// Row-wise work list: whole block rows, rows longer than `chunk` blocks in chunks with a partial-sum slot each
-// (split rows first: they are the longest items).  only != NULL: just the block rows it flags.  Returns the slots.
 static void rowwise_costs(const std::vector<WorkItem> &items, XcdDeal &deal)
 {
     std::vector<uint64_t> prefix(items.size() + 1, 0);
@@ -617,36 +619,59 @@ static void rowwise_costs(const std::vector<WorkItem> &items, XcdDeal &deal)
     deal.set_costs(std::move(prefix));
 }
 
-// Blocks of a chunk of a split block row.  Rows are split where one has more than four times the average and 64 blocks; a chunk is then no longer than 32 blocks and 0.4 of what
-// one of 4,096 wavefronts has to do in a launch of the plan's width, since the longest item is as long as a small launch.  Chunks of four times the average -> these, us (R-MAT,
-// row-wise): scale 12, 16 a row, N = 128 30.7 -> 18.6 (of 16, 32, 64, 128 blocks 18.3, 17.8, 18.5, 25.7); 13, 16, N = 24 32 -> 14; 14, 20, N = 104 56 -> 39 (64: 38, 32: 42); 15, 16, N = 200
-// 172 -> 148; 16, 16, N = 16 94 -> 68; 17, 16, N = 72 413 -> 386 (64: 417); 19, 9, N = 40 882 -> 864.
-static long rowwise_chunk(const int32_t *row_ptr_host, size_t mb, size_t nnzb, size_t n_hint, double avg)
+// Which block rows are cut, and into what: where one has more than four times the average and 64 blocks, pieces of at most 32 blocks and 0.4 of what one of 4,096 wavefronts has to
+// do in a launch of the plan's width, since the longest item is as long as a small launch.  Pieces of four times the average -> these, us (R-MAT, row-wise): scale 12, 16 a row,
+// N = 128 27.1 -> 16.2; 13, 16, N = 24 29.7 -> 12.7; 14, 20, N = 104 54 -> 38; 15, 16, N = 200 146 -> 119; 16, 16, N = 16 75 -> 52; 17, 16, N = 72 396 -> 367.
+// Rows of more than twice the average are cut, and all rows longer than a piece where the launch has no more than a wavefront a SIMD (512 rows of 100 blocks and one of 570, N = 64
+// 43.7 -> 18.6 us).  Of the others those from the length on from which their partial tiles, 4 blocks' time each, take up to 5 % of the time of all blocks: the few long rows of a power law, not
+// the ordinary ones of a list with an outlier.  Whole / cut, us: R-MAT 14, 20 a row, N = 104 40.7 / 38.0, 16, 16, N = 16 58.4 / 51.5, 13, 24, N = 200 38.8 / 34.0; 1024 rows of 60 and one of 400, N = 128
+// 25.2 / 30.6, 128 of 200 and one of 1070, N = 1024 (6 %) 74 / 83, 3000 of 50, N = 32 19.4 / 23.9; 1024 rows each of 10 and 80, N = 256 56 / 64.
+static RowCuts rowwise_cuts(const int32_t *row_ptr_host, size_t mb, size_t n_hint)
 {
     const auto even = [](double blocks) { return ((long)(blocks + 0.5) + 1) & ~1L; }; // pairs stay aligned with the MFMA's K = 32
+    const double nnzb = (double)row_ptr_host[mb], panels = (double)((n_hint + 63) / 64);
+    size_t nonempty = 0;
+    long most = 0;
+    for (size_t i = 0; i < mb; i++) {
+        const long len = row_ptr_host[i + 1] - row_ptr_host[i];
+        nonempty += len > 0;
+        most = std::max(most, len);
+    }
+    const double avg = nonempty ? nnzb / (double)nonempty : 0.0;
     const long longest = std::max(even(4.0 * avg), 64L);
-    for (size_t i = 0; i < mb; i++)
-        if (row_ptr_host[i + 1] - row_ptr_host[i] > longest)
-            return std::min(longest, even(32.0 + 0.4 * (double)nnzb * (double)((n_hint + 63) / 64) / 4096.0));
-    return longest;
+    if (most <= longest) return {longest, longest};
+    const long piece = std::min(longest, even(32.0 + 0.4 * nnzb * panels / 4096.0));
+    if ((double)nonempty * panels <= 1024.0) return {piece, piece};
+    long above = std::max(piece, (long)(2.0 * avg));
+    std::vector<int64_t> tiles((size_t)(above - piece), 0); // partial ones, of the rows of piece + 1, piece + 2, .. blocks
+    for (size_t i = 0; i < mb; i++) {
+        const long len = row_ptr_host[i + 1] - row_ptr_host[i];
+        if (len > piece && len <= above) tiles[(size_t)(len - piece - 1)] += (len + piece - 1) / piece;
+    }
+    for (double left = 0.05 * nnzb / 4.0; above > piece && (left -= (double)tiles[(size_t)(above - piece - 1)]) >= 0.0;) above--;
+    return {above, piece};
 }
-// The items of a list with split rows in the order that the compact kernel's tasks have (spmm_compact.hip): chunks by where they begin in their rows, whole rows by octaves of
-// length.  Chunks of one row after the other -> this, us (R-MAT, row-wise): scale 14, 12 a row, N = 256 60.2 -> 56.6; 16, 16, N = 184 304 -> 287; 16, 20, N = 256 509 -> 482; 18, 12, N = 128
-// 1031 -> 852; 19, 16, N = 8 531 -> 485; scale 12 and 13 equal.
-static void order_split_items(const int32_t *row_ptr_host, std::vector<WorkItem> &items)
+// The items of a list with cut rows in the order that the compact kernel's tasks have (spmm_compact.hip): pieces by where they begin in their rows, whole rows by octaves of
+// length; whole rows that are longer than the pieces before them.  Pieces of one row after the other -> this, us
+// (R-MAT, row-wise): scale 14, 12 a row, N = 256 60.2 -> 56.6; 16, 16, N = 184 304 -> 287; 16, 20, N = 256 509 -> 482; 18, 12, N = 128 1031 -> 852; 19, 16, N = 8 531 -> 485; scale 12 and 13 equal.
+static void order_split_items(const int32_t *row_ptr_host, long piece, std::vector<WorkItem> &items)
 {
     std::vector<uint16_t> keys(items.size());
     for (size_t i = 0; i < items.size(); i++) {
         const WorkItem &w = items[i];
-        keys[i] = w.dst >= 0 ? begin_key(w.begin, row_ptr_host[w.block_row], row_ptr_host[w.block_row + 1]) : (uint16_t)(BEGIN_KEYS + 31 - octave_of((uint32_t)(w.end - w.begin)));
+        const int octave = 31 - octave_of((uint32_t)(w.end - w.begin));
+        keys[i] = (uint16_t)(w.dst >= 0                ? 32 + begin_key(w.begin, row_ptr_host[w.block_row], row_ptr_host[w.block_row + 1])
+                             : w.end - w.begin > piece ? octave
+                                                       : 32 + BEGIN_KEYS + octave);
     }
-    const std::vector<uint32_t> order = ordered_by(keys, BEGIN_KEYS + 32);
+    const std::vector<uint32_t> order = ordered_by(keys, BEGIN_KEYS + 64);
     std::vector<WorkItem> ordered(items.size());
     for (size_t i = 0; i < items.size(); i++) ordered[i] = items[order[i]];
     items.swap(ordered);
 }
 
-static int rowwise_work_list(const int32_t *row_ptr_host, size_t mb, long chunk, const uint8_t *only,
+// Row-wise work list: whole block rows, cut ones in pieces with a partial-sum slot each, before the others.  only != NULL: just the block rows it flags.  Returns the slots.
+static int rowwise_work_list(const int32_t *row_ptr_host, size_t mb, RowCuts cuts, const uint8_t *only,
                              std::vector<WorkItem> &items, std::vector<SplitRow> &split)
 {
     items.clear();
@@ -655,10 +680,10 @@ static int rowwise_work_list(const int32_t *row_ptr_host, size_t mb, long chunk,
     int slot = 0;
     for (size_t i = 0; i < mb; i++) {
         const long len = row_ptr_host[i + 1] - row_ptr_host[i];
-        if (len <= chunk || (only && !only[i])) continue;
+        if (len <= cuts.above || (only && !only[i])) continue;
         SplitRow sr{(int32_t)i, slot, slot, 0};
-        for (long b = row_ptr_host[i]; b < row_ptr_host[i + 1]; b += chunk) {
-            const long e = std::min<long>(b + chunk, row_ptr_host[i + 1]);
+        for (long b = row_ptr_host[i]; b < row_ptr_host[i + 1]; b += cuts.piece) {
+            const long e = std::min<long>(b + cuts.piece, row_ptr_host[i + 1]);
             items.push_back(WorkItem{(int32_t)i, (int32_t)b, (int32_t)e, slot++});
         }
         sr.slot_end = slot;
@@ -666,10 +691,30 @@ static int rowwise_work_list(const int32_t *row_ptr_host, size_t mb, long chunk,
     }
     for (size_t i = 0; i < mb; i++) {
         const long len = row_ptr_host[i + 1] - row_ptr_host[i];
-        if (len > chunk || (only && !only[i])) continue;
+        if (len > cuts.above || (only && !only[i])) continue;
         items.push_back(WorkItem{(int32_t)i, row_ptr_host[i], row_ptr_host[i + 1], -1});
     }
     return slot;
+}
+// The list of a plan of n_hint columns.
+static int rowwise_plan_list(const int32_t *row_ptr_host, size_t mb, RowCuts cuts, std::vector<WorkItem> &items, std::vector<SplitRow> &split)
+{
+    const int slots = rowwise_work_list(row_ptr_host, mb, cuts, nullptr, items, split);
+    if (!split.empty()) order_split_items(row_ptr_host, cuts.piece, items);
+    return slots;
+}
+// Test hook (not part of smat.h, host only): that list, items[4 i ..] = {block row, first block, end, slot or -1} of up to `room` items; counts[0..2] = items, cut rows, slots.
+extern "C" int smat_internal_rowwise_list(const int32_t *row_ptr_host, size_t mb, size_t n_hint, int32_t *out, size_t room, int64_t *counts)
+{
+    return smat::guarded("smat_internal_rowwise_list", [&] {
+        std::vector<WorkItem> items;
+        std::vector<SplitRow> split;
+        counts[2] = rowwise_plan_list(row_ptr_host, mb, rowwise_cuts(row_ptr_host, mb, n_hint), items, split);
+        counts[0] = (int64_t)items.size();
+        counts[1] = (int64_t)split.size();
+        memcpy(out, items.data(), std::min(room, items.size()) * sizeof(WorkItem));
+        return (int)SMAT_OK;
+    });
 }
 
 namespace {
@@ -760,16 +805,11 @@ static int smat_plan_create_impl(smat_plan **out, const int32_t *row_ptr_host,
     p->row_ptr_host.assign(row_ptr_host, row_ptr_host + mb + 1);
     if (col_idx_host && cols_ascending && (want == SMAT_KERNEL_AUTO || want == SMAT_KERNEL_MIXED)) p->col_idx_host.assign(col_idx_host, col_idx_host + nnzb);
 
-    size_t nonempty = 0;
-    for (size_t i = 0; i < mb; i++) nonempty += row_ptr_host[i + 1] > row_ptr_host[i];
-    const double avg = nonempty ? (double)nnzb / (double)nonempty : 0.0;
-    const long chunk = rowwise_chunk(row_ptr_host, mb, nnzb, n_hint, avg);
-    p->chunk = (int)chunk;
+    p->cuts = rowwise_cuts(row_ptr_host, mb, n_hint);
 
     std::vector<WorkItem> items;
     std::vector<SplitRow> split;
-    const int slot = rowwise_work_list(row_ptr_host, mb, chunk, nullptr, items, split);
-    if (!split.empty()) order_split_items(row_ptr_host, items);
+    const int slot = rowwise_plan_list(row_ptr_host, mb, p->cuts, items, split);
     p->n_items = (int)items.size();
     rowwise_costs(items, p->deal);
     for (const WorkItem &wi : items) p->max_item_blocks = std::max(p->max_item_blocks, wi.end - wi.begin);
@@ -1208,7 +1248,7 @@ static int smat_plan_attach_values_impl(smat_plan *p, const uint16_t *vals, cons
     } else if (e == hipSuccess && mixed) {
         std::vector<WorkItem> items;
         std::vector<SplitRow> split;
-        const int slots = rowwise_work_list(row_ptr_host, mb, p->chunk, dense.data(), items, split);
+        const int slots = rowwise_work_list(row_ptr_host, mb, p->cuts, dense.data(), items, split);
         p->n_items_dense = (int)items.size();
         rowwise_costs(items, p->deal_dense);
         p->n_split_dense = (int)split.size();
@@ -1315,7 +1355,7 @@ extern "C" int smat_plan_values_current(const smat_plan *p, const uint16_t *vals
 extern "C" int smat_plan_info(const smat_plan *p, int64_t *info)
 {
     if (!p || !info) return set_error(SMAT_ERR_INVALID, "plan and info must not be NULL");
-    info[0] = p->kernel; info[1] = p->n_items; info[2] = p->n_split_rows; info[3] = p->chunk;
+    info[0] = p->kernel; info[1] = p->n_items; info[2] = p->n_split_rows; info[3] = p->cuts.piece;
     info[4] = (int64_t)p->workspace_bytes;
     info[5] = p->kernel == SMAT_KERNEL_SWEEP ? 16 * SWEEP_TN : 16 * p->panel_tiles;
     info[6] = p->sweep.n_ops + p->sweep_dense.n_ops + p->sweep_blocks.n_ops;

@@ -9,7 +9,8 @@ from smat_amd import generators as gen
 pytestmark = pytest.mark.gpu
 
 LENGTHS = {"short": list(range(11)) * 2, "shared": list(range(12, 76)), "whole": list(range(1, 71)) * 10,
-           "split": [1, 300, 0, 2, 32, 33, 34, 35, 500, 0] + [3] * 60}  # chunks of 32 blocks, and what they leave
+           "split": [1, 300, 0, 2, 32, 33, 34, 35, 500, 0] + [3] * 60,  # pieces of at most 32 blocks
+          "outlier": [34, 60, 1] * 120 + [200]}                        # N = 136: one row is cut, and whole ones are longer than its pieces
 
 
 @pytest.mark.parametrize("rows", sorted(LENGTHS))
@@ -25,7 +26,7 @@ def test_every_remainder(smat, cuda, oracle, rows, N, packed):
     vals, rp, ci, Bd = dev(A["b_val"]), dev(A["b_row_ptr"].astype(np.int32)), dev(A["b_col_idx"].astype(np.int32)), dev(B)
     kernel = smat.KERNEL_ROWWISE_PACKED if packed else smat.KERNEL_ROWWISE_DIRECT
     plan = smat.Plan(A["b_row_ptr"], M, K, nnzb, N, col_idx_host=A["b_col_idx"], kernel=kernel)
-    assert (plan.info()["split_rows"] > 0) == (rows == "split")
+    assert (plan.info()["split_rows"] > 0) == (rows in ("split", "outlier"))
     C = torch.full((M, N), float("nan"), dtype=torch.float32, device=cuda)
     smat.spmm(vals, rp, ci, Bd, C, M, N, K, nnzb, plan=plan, kernel=kernel, c_f32=True)
     torch.cuda.synchronize()
