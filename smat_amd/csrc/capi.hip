@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -324,7 +325,7 @@ static bool windows_beat(const smat_plan &p, const WindowPlan &shape, const Wind
 
 // Whether a launch of the row-wise kernel reads a row-major B in place: always but for large products on a repacked B, which are 5 to 35 % slower for it (13696 x 6768, 19 %,
 // N = 2384 287 -> 391 us, 8160 x 9536, 24 %, N = 336 61 -> 72; 120 drawn products otherwise 0.44 to 0.93 of the time: a launch less, and loads of whole lines instead of 32
-// pieces), and but for windows that are estimated to be faster, the pass over B before them included.
+// pieces).  Windows are decided on before (rowwise_windows).
 static bool rowwise_stays_row_major(size_t M, size_t K, size_t N, size_t nnzb, size_t n_items, RowLengths lengths, bool packed)
 {
     // from 128 columns on a column-major launch takes wider panels, on B in place as well as repacked, and fits where this one does not
@@ -333,7 +334,6 @@ static bool rowwise_stays_row_major(size_t M, size_t K, size_t N, size_t nnzb, s
 }
 static bool rowwise_stays_row_major(const smat_plan &p, const SpmmArgs &a)
 {
-    if (p.window && rowwise_row_major_us(a.M, a.N, a.nnzb) > window_launch(a, *p.window).us + to_col_major_us(a.K, a.N)) return false;
     return rowwise_stays_row_major(a.M, a.K, a.N, a.nnzb, (size_t)p.n_items, p.n_split_rows ? RowLengths::SPLIT : RowLengths::EVEN, a.b_packed != nullptr);
 }
 // Test hook (not part of smat.h): whether a launch over whole block rows reads a row-major B in place, windows aside.
@@ -341,6 +341,26 @@ extern "C" int smat_internal_rowwise_stays_row_major(size_t M, size_t K, size_t 
 {
     return rowwise_stays_row_major(M, K, N, nnzb, n_items, RowLengths::EVEN, packed != 0);
 }
+
+// The launch from windows in the place of the row-wise kernel, or none, where the choice is the plan's; on a row-major B where they are faster than that kernel on B in place, the
+// pass over B before them included.
+static WindowLaunch rowwise_windows(const smat_plan &p, const SpmmArgs &a, bool b_row_major)
+{
+    const bool shares = rowwise_shares_items(a.N, (size_t)p.n_items, p.nnzb / (size_t)p.n_items);
+    const double in_place = a.N == p.n_cap || window_forced() || shares || a.b_packed ? SHORT_US : rowwise_in_place_us(p, a.N, p.window->share4);
+    WindowLaunch l;
+    if (in_place < SHORT_US) {
+        l = window_launch(a, *p.window);
+        if (!windows_beat(p, *p.window, l, a.N, in_place)) return WindowLaunch();
+    } else {
+        l = window_or_not(a, p, [&] { return shares ? 0.0 : rowwise_estimate_us(a.M, a.K, a.N, a.nnzb, (size_t)p.n_items, RowLengths::EVEN, a.b_packed != nullptr); });
+    }
+    if (b_row_major && rowwise_row_major_fits((size_t)a.n_items, a.N) && rowwise_row_major_us(a.M, a.N, a.nnzb) <= l.us + to_col_major_us(a.K, a.N)) return WindowLaunch();
+    return l;
+}
+
+static std::atomic<int64_t> g_turned{0}; // test hook: launches that brought a row-major B into column-major order
+extern "C" int64_t smat_internal_turned_launches(void) { return g_turned.load(std::memory_order_relaxed); }
 
 extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_ptr,
                                       const int32_t *col_idx, const uint16_t *B, void *C, size_t M,
@@ -405,6 +425,11 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
     }
     const uint16_t *B_as_given = B;
     bool sweep_row_major = false;
+    // Launches that leave the choice to the plan: windows of B or columns of B in LDS, which were weighed when the plan was made, or, for another width than
+    // its own, where they are estimated to be faster.
+    WindowLaunch windows;
+    ResidentLaunch columns;
+    const bool plans_choice = plan && o.kernel == SMAT_KERNEL_AUTO, column_major = o.b_layout == SMAT_B_COL_MAJOR;
     if (kernel == SMAT_KERNEL_MIXED && (!plan || !plan->compact || (!plan->d_items_dense && !plan->sweep_dense.d_ops && !plan->sweep_blocks.d_ops) || !plan->d_bt || N > plan->n_cap))
         return set_error(SMAT_ERR_INVALID, "SMAT_KERNEL_MIXED needs a plan that split the block rows when the values were "
                                            "attached (smat_plan_attach_values) and n_hint >= N");
@@ -421,35 +446,23 @@ extern "C" int smat_spmm_bcsr_f16_ex(const uint16_t *vals, const int32_t *row_pt
                                          : plan->sweep_dense.d_ops     ? &plan->sweep_dense
                                                                        : nullptr;
         sweep_row_major = sweep && sweep->d_ops_row_major && sweep_takes_row_major(N, K, sweep->n_rg);
-        a.b_row_major = !sweep && rowwise_stays_row_major(*plan, a);
+        if (kernel == SMAT_KERNEL_ROWWISE && plans_choice && plan->window) windows = rowwise_windows(*plan, a, true);
+        a.b_row_major = !sweep && !windows.tiles && rowwise_stays_row_major(*plan, a);
         if (!sweep_row_major && !a.b_row_major) {
+            g_turned.fetch_add(1, std::memory_order_relaxed);
             e = launch_b_to_col_major(B, plan->d_bcol, N, K, static_cast<hipStream_t>(o.stream));
             if (e != hipSuccess) return set_error(SMAT_ERR_HIP, "SpMM launch failed: %s", hipGetErrorString(e));
             a.B = B = plan->d_bcol;
         }
     }
-    // Launches that leave the choice to the plan: windows of B or columns of B in LDS, which were weighed when the plan was made, or, for another width than
-    // its own, where they are estimated to be faster.
-    WindowLaunch windows;
-    ResidentLaunch columns;
-    if (plan && o.kernel == SMAT_KERNEL_AUTO && (plan->window || plan->resident)) {
-        const bool column_major = o.b_layout == SMAT_B_COL_MAJOR;
-        if (kernel == SMAT_KERNEL_ROWWISE && plan->window && !a.b_row_major) { // a row-major B lies in column-major order by now
-            const bool shares = rowwise_shares_items(N, (size_t)plan->n_items, nnzb / (size_t)plan->n_items);
-            const double in_place = N == plan->n_cap || window_forced() || shares || a.b_packed ? SHORT_US : rowwise_in_place_us(*plan, N, plan->window->share4);
-            if (in_place < SHORT_US) {
-                windows = window_launch(a, *plan->window);
-                if (!windows_beat(*plan, *plan->window, windows, N, in_place)) windows = WindowLaunch();
-            } else {
-                windows = window_or_not(a, *plan, [&] {
-                    return shares ? 0.0 : rowwise_estimate_us(M, K, N, nnzb, (size_t)plan->n_items, RowLengths::EVEN, a.b_packed != nullptr);
-                });
-            }
-        } else if (kernel == SMAT_KERNEL_SWEEP && plan->window && column_major) {
+    if (plans_choice && column_major && (plan->window || plan->resident)) {
+        if (kernel == SMAT_KERNEL_ROWWISE && plan->window) {
+            windows = rowwise_windows(*plan, a, false);
+        } else if (kernel == SMAT_KERNEL_SWEEP && plan->window) {
             windows = window_or_not(a, *plan, [&] { return sweep_estimate_us((size_t)plan->sweep.n_rg, plan->sweep_chunks, nnzb, M, N); });
-        } else if (kernel == SMAT_KERNEL_COMPACT && plan->window && column_major && N <= plan->n_cap) {
+        } else if (kernel == SMAT_KERNEL_COMPACT && plan->window && N <= plan->n_cap) {
             windows = window_or_not(a, *plan, [&] { return compact_estimate_us(*plan->compact, M, K, N); });
-        } else if (kernel == SMAT_KERNEL_COMPACT && plan->resident && column_major && N <= plan->n_cap) {
+        } else if (kernel == SMAT_KERNEL_COMPACT && plan->resident && N <= plan->n_cap) {
             columns = resident_launch(*plan->resident, K, N);
             if (N != plan->n_cap && !resident_forced() && columns.us >= 0.9 * compact_estimate_us(*plan->compact, M, K, N)) columns = ResidentLaunch();
         }

@@ -536,3 +536,37 @@ def test_infinities_under_the_first_octet_of_a_row(smat, cuda, oracle, force, ro
     smat.spmm(d[0], d[1], d[2], d[3], C, M, N, K, nnzb, plan=plan)
     assert np.array_equal(C.cpu().numpy(), want, equal_nan=True)
     plan.close()
+
+
+def test_row_major_b_is_turned_only_for_windows_that_are_taken(smat, cuda, oracle, force):
+    """A launch that names the row-wise kernel takes no windows, and one without windows reads B in place: no pass over B before either."""
+    import torch
+    counts = smat.lib.smat_internal_window_launches, smat.lib.smat_internal_turned_launches
+    counts[1].restype = ctypes.c_int64
+    rng = np.random.default_rng(9)
+    groups = [rng.choice(1000, 10, replace=False) for _ in range(250)]  # the block columns of 16 block rows, all over B: not for the sweep kernel
+    ci = np.concatenate([np.sort(rng.permutation(groups[i // 16])[:8]) for i in range(4000)]).astype(np.int32) * 16
+    rp = np.arange(0, len(ci) + 1, 8, dtype=np.int32)
+    vals = rng.integers(-3, 4, len(ci) * 256).astype(np.float16).view(np.uint16)
+    M, K, n_hint, nnzb = 64000, 16000, 256, len(ci)
+    d = [to_dev(torch, x, cuda) for x in (vals, rp, ci)]
+    force(16, 0)
+    plan = smat.Plan(rp, M, K, nnzb, n_hint, col_idx_host=ci, b_row_major=True)
+    plan.attach_values(*d)
+    assert smat.lib.smat_internal_plan_window_rows(plan.handle) == 16
+    force(0, 0)
+    taken = set()
+    for kernel in (smat.KERNEL_AUTO, smat.KERNEL_ROWWISE_DIRECT):
+        for N in (256, 200, 136, 64, 24, 8):
+            B = whole_b(K, N, seed=N)
+            want = oracle.spmm_bcsr(M, N, K, rp, ci, vals, B, threads=8).astype(np.float16)
+            rows = to_dev(torch, np.ascontiguousarray(B.reshape(N, K).T), cuda)
+            C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+            before = [count() for count in counts]
+            smat.spmm(*d, rows, C, M, N, K, nnzb, plan=plan, kernel=kernel, b_row_major=True)
+            windows, turned = (count() - b for count, b in zip(counts, before))
+            assert np.array_equal(C.cpu().numpy(), want), N
+            assert turned == windows, N
+            taken.add((kernel, windows))
+    assert taken == {(smat.KERNEL_AUTO, 0), (smat.KERNEL_AUTO, 1), (smat.KERNEL_ROWWISE_DIRECT, 0)}
+    plan.close()
