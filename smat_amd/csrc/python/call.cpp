@@ -117,9 +117,12 @@ PyObject *bind(PyObject *, PyObject *args)
     if (!PyArg_ParseTuple(args, "KKOOO", &launch, &drop_in, &in_python, &check, &plan_type)) return nullptr;
     g_launch = reinterpret_cast<decltype(g_launch)>(launch);
     g_launch_drop_in = reinterpret_cast<decltype(g_launch_drop_in)>(drop_in);
-    Py_XSETREF(g_in_python, Py_NewRef(in_python));
-    Py_XSETREF(g_check, Py_NewRef(check));
-    Py_XSETREF(g_plan_type, Py_NewRef(plan_type));
+    Py_INCREF(in_python);
+    Py_INCREF(check);
+    Py_INCREF(plan_type);
+    Py_XSETREF(g_in_python, in_python);
+    Py_XSETREF(g_check, check);
+    Py_XSETREF(g_plan_type, plan_type);
     Py_RETURN_NONE;
 }
 
