@@ -902,6 +902,24 @@ static size_t even_rows(size_t mb, size_t group_rows)
     const size_t n_rg = (mb + group_rows - 1) / group_rows;
     return (mb + n_rg - 1) / n_rg;
 }
+// The row groups that the plan builds for candidates of up to `rows` block rows: as many in each where the streams are light, others take as long or longer for it (2768 x 8000, 20 %,
+// N = 3488, fp32 75.6 -> 76.9).
+struct SweepGroups {
+    size_t rows, listed; // block rows of a group; chunks that the groups list together
+    bool light;
+};
+static SweepGroups sweep_groups(const int32_t *row_ptr, const int32_t *col_idx, size_t mb, size_t kb, size_t nnzb, size_t rows)
+{
+    const size_t even = even_rows(mb, rows), listed = sweep_listed_chunks(row_ptr, col_idx, mb, kb, even);
+    if (sweep_light(listed, nnzb)) return {even, listed, true};
+    return {rows, even == rows ? listed : sweep_listed_chunks(row_ptr, col_idx, mb, kb, rows), false};
+}
+// Test hook (not part of smat.h): out[0..2] = block rows of a group, chunks listed, light.
+extern "C" void smat_internal_sweep_groups(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t rows, int64_t *out)
+{
+    const SweepGroups g = sweep_groups(row_ptr, col_idx, M / 16, K / 16, nnzb, rows);
+    out[0] = (int64_t)g.rows; out[1] = (int64_t)g.listed; out[2] = g.light;
+}
 static int g_force_group_rows = 0; // test hook: 64, 32 or 16 whatever the estimates say
 static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, size_t n_items,
                                RowLengths lengths, bool packed, bool b_row_major, double *us = nullptr)
@@ -917,7 +935,7 @@ static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, s
     size_t group_rows = 0;
     for (size_t rows : {(size_t)SWEEP_G, (size_t)SWEEP_G / 2, (size_t)SWEEP_G / 4}) {
         const size_t n_rg = (mb + rows - 1) / rows;
-        const double sweep = sweep_estimate_us(n_rg, sweep_listed_chunks(row_ptr, col_idx, mb, kb, even_rows(mb, rows)), nnzb, M, N);
+        const double sweep = sweep_estimate_us(n_rg, sweep_groups(row_ptr, col_idx, mb, kb, nnzb, rows).listed, nnzb, M, N);
         const bool in_place = b_row_major && sweep_takes_row_major(N, K, (int)n_rg);
         const double t = in_place ? sweep_in_place_factor(N) * sweep : sweep + to_col_major;
         if (t < best) best = t, group_rows = rows;
@@ -947,10 +965,8 @@ static hipError_t sweep_small_groups(smat_plan &p, size_t group_rows)
     const size_t mb = p.M / 16, kb = p.K / 16, nnzb = p.nnzb;
     const int32_t *row_ptr = p.row_ptr_host.data(), *col_idx = p.col_idx_host.data();
     SweepPlanHost h;
-    const size_t even = even_rows(mb, group_rows);
-    const bool light = sweep_light(sweep_listed_chunks(row_ptr, col_idx, mb, kb, even), nnzb);
-    if (light) group_rows = even; // others take as long or longer for it (2768 x 8000, 20 %, N = 3488, fp32 75.6 -> 76.9)
-    build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, group_rows, 16.0 * (double)nnzb, light);
+    const SweepGroups groups = sweep_groups(row_ptr, col_idx, mb, kb, nnzb, group_rows);
+    build_sweep_plan(row_ptr, col_idx, mb, kb, h, nullptr, 0, groups.rows, 16.0 * (double)nnzb, groups.light);
     const hipError_t e = p.sweep.upload(h, p.d_bcol != nullptr);
     if (e != hipSuccess) {
         p.sweep.release();

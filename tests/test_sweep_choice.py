@@ -67,3 +67,23 @@ def test_row_wise_where_the_streams_cannot_help(m, k, n, nnzb):
     rp = np.concatenate([[0], np.cumsum(np.bincount(cells // (k // 16), minlength=m // 16))]).astype(np.int32)
     ci = (cells % (k // 16) * 16).astype(np.int32)
     assert _fn(rp.ctypes.data, ci.ctypes.data, m, k, nnzb, n, 1) == 0
+
+
+@pytest.mark.parametrize("mb, kb, share", [(193, 257, 0.15), (33, 400, 0.30), (65, 120, 0.60), (70, 300, 0.02), (129, 96, 0.9), (64, 200, 0.25)])
+@pytest.mark.parametrize("rows", [64, 32, 16])
+def test_what_is_estimated_is_what_is_built(mb, kb, share, rows):
+    """The chunks that the choice counts are those that the streams of its row groups list, and light where the kernel's streams are."""
+    rng = np.random.default_rng(mb + rows)
+    mask = rng.random((mb, kb)) < share
+    rp = np.concatenate([[0], np.cumsum(mask.sum(1))]).astype(np.int32)
+    ci = (np.nonzero(mask)[1] * 16).astype(np.int32)
+    out = (C.c_int64 * 3)()
+    ptr = lambda a: C.c_void_p(a.ctypes.data)  # noqa: E731
+    lib.smat_internal_sweep_groups(ptr(rp), ptr(ci), C.c_size_t(16 * mb), C.c_size_t(16 * kb), C.c_size_t(len(ci)), C.c_size_t(rows), out)
+    group, listed, light = out
+    chunks = np.nonzero(mask)[1] // 16
+    in_groups = lambda g: len(np.unique(np.nonzero(mask)[0] // g * kb + chunks))  # noqa: E731
+    n_rg = -(-mb // rows)
+    even = -(-mb // n_rg)
+    assert light == (len(ci) <= 8 * 8 * in_groups(even))
+    assert group == (even if light else rows) and listed == in_groups(group)
