@@ -34,6 +34,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <type_traits>
 #include <vector>
@@ -52,8 +53,7 @@ namespace {
 
 int g_force_run = 0;
 int g_tune = 1; // test hook: 0 = attaching values measures nothing, the estimate decides the deal
-int g_last_share = 1; // test hook: wavefronts a task of the latest launch
-int g_last_run = 0; // test hook: the run length of the latest launch
+std::atomic<int> g_last_share{1}, g_last_run{0}; // test hooks: wavefronts a task and the run length of the latest launch, of any thread
 int g_force_list = 0; // test hook: 1 = lists of whole columns, 2 = of nonzeros, 0 = compact_build decides
 int g_force_staged = 0; // test hook: 1 = entries go through LDS in blocks wherever they may, 2 = nowhere, 0 = the launcher decides
 int g_force_order = 0; // test hook: 1 = tasks of lists with split rows in the order of their items, 0 = order_tasks
@@ -889,11 +889,12 @@ hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
     if (a.xcd_run > 0) xcd_run = a.xcd_run;
     if (g_force_run > 0) xcd_run = g_force_run;
     xcd_run = std::min<long>((wgs + 7) / 8, xcd_run);
-    g_last_run = (int)xcd_run;
+    g_last_run.store((int)xcd_run, std::memory_order_relaxed);
     // A workgroup of four tasks keeps its place until the longest is done; one task each is up to 12 % faster (4864 x 6496, 12 % of full blocks and 15 more a row, N =
     // 400 30.5 -> 26.6 us, 40000 x 60000, 10 a row, N = 64, row-major 9.7 -> 9.3, R-MAT scale 18, N = 64 63.9 -> 62.7).  Where a place has many steps to do the end of a launch
     // matters less than the lines that neighbouring tasks find of each other's in their L1: four (R-MAT scale 20, N = 128, row-major 366, one each 378; 19, N = 256 362 and 365, 40000 x 60000, 30 a row, N = 256 73.8 and 74.6).
-    const int share = g_last_share = !p.may_share ? 1 : g_force_share ? g_force_share : compact_share(p, total);
+    const int share = !p.may_share ? 1 : g_force_share ? g_force_share : compact_share(p, total);
+    g_last_share.store(share, std::memory_order_relaxed);
     const int waves = share > 1 ? share : (double)p.n_steps * n_panels >= 32.0 * 16.0 * 256.0 ? 4 : 1;
     xcd_run *= share > 1 ? 4 : 4 / waves;
     wgs = share > 1 ? total : (total + waves - 1) / waves;
@@ -1559,14 +1560,14 @@ extern "C" void smat_internal_compact_staged(int what) { smat::g_force_staged = 
 extern "C" void smat_internal_compact_order(int what) { smat::g_force_order = what; }
 // Test hook: 1, 2 or 4 = wavefronts of a launch that share a task, where tasks are of one item, 0 = as the sizes say (the default).
 extern "C" void smat_internal_compact_share(int what) { smat::g_force_share = what; }
-extern "C" int smat_internal_compact_last_share(void) { return smat::g_last_share; }
+extern "C" int smat_internal_compact_last_share(void) { return smat::g_last_share.load(); }
 // Test hook (host only): steps of the chunks of split rows.
 extern "C" long smat_internal_compact_chunk(long steps, size_t rows, long longest, size_t n_cap) { return smat::split_chunk_steps(steps, rows, longest, n_cap); }
 // Test hooks for the deal of the compact kernel's workgroups to the XCDs: a run length that every launch uses
 // (0 = chosen per plan and number of panels), the run length of the latest launch, and the choice itself for a list
 // of item costs (host only).
 extern "C" void smat_internal_compact_run(int run) { smat::g_force_run = run; }
-extern "C" int smat_internal_compact_last_run(void) { return smat::g_last_run; }
+extern "C" int smat_internal_compact_last_run(void) { return smat::g_last_run.load(); }
 extern "C" void smat_internal_compact_tune(int on) { smat::g_tune = on; }
 extern "C" unsigned smat_internal_choose_xcd_run(const uint64_t *cost_prefix, uint64_t n_items, int n_panels)
 {
