@@ -847,10 +847,10 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
 // wavefronts are enough.  Alone / two / four, us, the copy of B among them: 3584 x 4112, 8 % of full blocks and 10 more a row, N = 96 (448 tasks and panels of 15 steps) 10.5 / 8.7 / 8.6,
 // 4416 x 8160, 8 % and 3, N = 72 (552 of 22) 13.4 / 11.0 / 11.4, 2832 x 2144, 32 a row, N = 48 (177 of 14) 5.65 / 4.37 / 4.07, 6992 x 7616, 7 % and 4, N = 80 (874 of 18) 12.7 / 11.4 / 12.0;
 // 5776 x 6752, 5 % and 3, N = 192 (1083 of 12) 12.2 / 12.2 / 12.5, 4288 x 1088, 8 a row, N = 48 (268 of 4) 3.88 / 4.06 / 4.11.
-int compact_share(const CompactPlan &p, long total)
+int compact_share(bool by_name, int64_t n_steps, int64_t n_tasks, long total)
 {
-    if (p.by_name || total > 900 || p.n_steps < 6 * (int64_t)p.n_tasks) return 1;
-    return total > 400 || p.n_steps < 12 * (int64_t)p.n_tasks ? 2 : 4;
+    if (by_name || total > 900 || n_steps < 6 * n_tasks) return 1;
+    return total > 400 || n_steps < 12 * n_tasks ? 2 : 4;
 }
 
 // Halves from row to row of the copy's last panel: 8, 16, 32, .. as many as hold the columns that are left, so that what is gathered at random lies on as few lines as may be.
@@ -893,7 +893,7 @@ hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
     // A workgroup of four tasks keeps its place until the longest is done; one task each is up to 12 % faster (4864 x 6496, 12 % of full blocks and 15 more a row, N =
     // 400 30.5 -> 26.6 us, 40000 x 60000, 10 a row, N = 64, row-major 9.7 -> 9.3, R-MAT scale 18, N = 64 63.9 -> 62.7).  Where a place has many steps to do the end of a launch
     // matters less than the lines that neighbouring tasks find of each other's in their L1: four (R-MAT scale 20, N = 128, row-major 366, one each 378; 19, N = 256 362 and 365, 40000 x 60000, 30 a row, N = 256 73.8 and 74.6).
-    const int share = !p.may_share ? 1 : g_force_share ? g_force_share : compact_share(p, total);
+    const int share = !p.may_share ? 1 : g_force_share ? g_force_share : compact_share(p.by_name, p.n_steps, p.n_tasks, total);
     g_last_share.store(share, std::memory_order_relaxed);
     const int waves = share > 1 ? share : (double)p.n_steps * n_panels >= 32.0 * 16.0 * 256.0 ? 4 : 1;
     xcd_run *= share > 1 ? 4 : 4 / waves;
@@ -1560,6 +1560,8 @@ extern "C" void smat_internal_compact_staged(int what) { smat::g_force_staged = 
 extern "C" void smat_internal_compact_order(int what) { smat::g_force_order = what; }
 // Test hook: 1, 2 or 4 = wavefronts of a launch that share a task, where tasks are of one item, 0 = as the sizes say (the default).
 extern "C" void smat_internal_compact_share(int what) { smat::g_force_share = what; }
+// Test hook (host only): the rule for such a list, total tasks x panels.
+extern "C" int smat_internal_compact_share_rule(int by_name, int64_t n_steps, int64_t n_tasks, int64_t total) { return smat::compact_share(by_name != 0, n_steps, n_tasks, total); }
 extern "C" int smat_internal_compact_last_share(void) { return smat::g_last_share.load(); }
 // Test hook (host only): steps of the chunks of split rows.
 extern "C" long smat_internal_compact_chunk(long steps, size_t rows, long longest, size_t n_cap) { return smat::split_chunk_steps(steps, rows, longest, n_cap); }

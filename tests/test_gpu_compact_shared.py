@@ -66,3 +66,45 @@ def test_shared_tasks_match_the_oracle(smat, cuda, oracle, hooks, lengths, N, pa
         assert hooks.smat_internal_compact_last_share() == (share if may else 1)
         assert np.array_equal(C.cpu().numpy(), want)
     plan.close()
+
+
+def full_blocks_and_pairs(mb, kb, keep, per_row, seed):
+    """BCSR of full blocks, and between them nonzeros in pairs, one below the other, small whole numbers."""
+    rng = np.random.default_rng(seed)
+    blocks = np.zeros((mb, kb, 16, 16), np.float16)
+    full = rng.random((mb, kb)) < keep
+    blocks[full] = rng.integers(1, 3, (full.sum(), 16, 16))
+    row = np.repeat(np.arange(16 * mb), per_row)
+    col = rng.integers(0, 16 * kb, row.size)
+    for r in (row, row ^ 1):
+        blocks[r // 16, col // 16, r % 16, col % 16] = 1
+    there = blocks.any((2, 3))
+    rp = np.concatenate([[0], np.cumsum(there.sum(1))]).astype(np.int32)
+    return rp, (np.nonzero(there)[1] * 16).astype(np.int32), np.ascontiguousarray(blocks[there]).reshape(-1).view(np.uint16)
+
+
+# One kernel for all blocks, as the rule says by itself; and the list added to what the sweep kernel wrote of the full blocks, where a plan asks for that by name and only the hook
+# shares tasks.
+@pytest.mark.parametrize("mb,kb,keep,per_row,N,kernel,share", [(224, 257, 0.08, 5, 96, 0, 2), (100, 2600, 0.0, 32, 48, 0, 4), (2, 256, 0.30, 12, 16384, 6, 1)])
+@pytest.mark.parametrize("row_major", [False, True])
+def test_plans_that_attach_values_share_tasks(smat, cuda, oracle, hooks, mb, kb, keep, per_row, N, kernel, share, row_major):
+    import torch
+    M, K = 16 * mb, 16 * kb
+    rp, ci, val = full_blocks_and_pairs(mb, kb, keep, per_row, seed=N)
+    nnzb = len(ci)
+    b = np.random.default_rng(N).integers(-1, 2, (N, K)).astype(np.float16)
+    want = oracle.spmm_bcsr(M, N, K, rp, ci, val, b.reshape(-1).view(np.uint16), threads=8)
+    assert np.abs(want).max() <= 2048  # whole numbers in fp16
+    vals, brp, bci = to_dev(torch, val, cuda), to_dev(torch, rp, cuda), to_dev(torch, ci, cuda)
+    Bd = to_dev(torch, (np.ascontiguousarray(b.T) if row_major else b).reshape(-1).view(np.uint16), cuda)
+    plan = smat.Plan(rp, M, K, nnzb, N, col_idx_host=ci, kernel=kernel, b_row_major=row_major)
+    plan.attach_values(vals, brp, bci)
+    assert plan.info()["kernel"] == (kernel or smat.KERNEL_COMPACT)
+    for forced in (0, 2, 4, 1):
+        hooks.smat_internal_compact_share(forced)
+        for c_f32 in (False, True):
+            C = torch.full((M, N), float("nan"), dtype=torch.float32 if c_f32 else torch.float16, device=cuda)
+            smat.spmm(vals, brp, bci, Bd, C, M, N, K, nnzb, plan=plan, c_f32=c_f32, b_row_major=row_major, kernel=kernel)
+            assert np.array_equal(C.cpu().numpy(), want if c_f32 else want.astype(np.float16)), forced
+            assert hooks.smat_internal_compact_last_share() == (forced or share)
+    plan.close()
