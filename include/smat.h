@@ -80,9 +80,9 @@ int smat_plan_cache_clear(void);
 #define SMAT_B_COL_MAJOR 0 /* B[n*K + k]: the reference layout               */
 #define SMAT_B_ROW_MAJOR 1 /* B[k*N + n].  The compact kernel reads rows of B and takes this layout in place
                             * (column-major B is first copied row-major into plan scratch on every launch).
-                            * So does the sweep kernel, unless many row groups share a large B.  The
-                            * row-wise kernel feeds the MFMA 8 consecutive k of one column per lane: for it
-                            * a row-major B is first transposed into the reference layout in plan scratch
+                            * So do the row-wise kernel, but for large products on a repacked B and for
+                            * windows of B, and the sweep kernel, unless many row groups share a large B;
+                            * these transpose B into the reference layout in plan scratch first
                             * (one read and one write of B per launch).  Both need a plan created with
                             * b_layout = SMAT_B_ROW_MAJOR and n_hint >= N; C has the same bits as for
                             * column-major B through that plan */

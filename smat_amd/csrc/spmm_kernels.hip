@@ -107,10 +107,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 4))) void
     const uint16_t *abase = vals + i16 * 16 + kh * 8;
     const f16x8 zero8 = zero_f16x8();
 
-    // Every load below is unconditional (indices are clamped instead of branching): loads
-    // inside branches cannot be counted by the compiler's vmcnt bookkeeping, which then
-    // waits for everything in flight and serialises load and MFMA phases.
-    // Two register sets: the operands of pair j+1 are in flight while pair j is multiplied.
+    // Two register sets: the operands of pair j+1 are in flight while pair j is multiplied.  The loads of a
+    // trip are without conditions: loads inside branches cannot be counted by the compiler's vmcnt bookkeeping,
+    // which then waits for everything in flight and serialises load and MFMA phases.  The branch is behind the
+    // loop, where one or two pairs are left.
     for (int pb = p0; pb < p1; pb += 64) {
         const int cnt = (p1 - pb) < 64 ? (p1 - pb) : 64;
         const int npair = (cnt + 1) >> 1;
@@ -118,12 +118,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 4))) void
         const int myc = col_idx[pb + (lane < cnt ? lane : cnt - 1)];
 
         auto issue = [&](int j, f16x8 &a, f16x8 (&b)[TN]) {
-            const int jj = j < npair ? j : npair - 1; // past the end: reload the last pair (unused)
-            const int second = (2 * jj + 1 < cnt) ? 2 * jj + 1 : 2 * jj; // a single block pairs with itself
-            const int c0 = __builtin_amdgcn_readlane(myc, 2 * jj);
+            const int second = (2 * j + 1 < cnt) ? 2 * j + 1 : 2 * j; // a single block pairs with itself
+            const int c0 = __builtin_amdgcn_readlane(myc, 2 * j);
             const int c1 = __builtin_amdgcn_readlane(myc, second);
             const int bc = sel ? c1 : c0;
-            const long pp = (long)pb + (sel ? second : 2 * jj);
+            const long pp = (long)pb + (sel ? second : 2 * j);
             a = load_f16x8(abase + pp * 256);
             // column-major: + first column of the block; packed: + slab of the block column
             const long boffs = PACKED ? (long)bc * N : (long)bc;
