@@ -56,7 +56,7 @@ int g_tune = 1; // test hook: 0 = attaching values measures nothing, the estimat
 std::atomic<int> g_last_share{1}, g_last_run{0}; // test hooks: wavefronts a task and the run length of the latest launch, of any thread
 int g_force_list = 0; // test hook: 1 = lists of whole columns, 2 = of nonzeros, 0 = compact_build decides
 int g_force_staged = 0; // test hook: 1 = entries go through LDS in blocks wherever they may, 2 = nowhere, 0 = the launcher decides
-int g_force_order = 0; // test hook: 1 = tasks of lists with split rows in the order of their items, 0 = order_tasks
+int g_force_order = 0; // test hook: 1 = tasks of lists with split rows in the order of their items, 2 = as order_tasks says, 0 = orders_tasks decides
 int g_force_share = 0; // test hook: 1, 2 or 4 = wavefronts that share a task where they may, 0 = the launcher decides
 int g_force_tq = 0; // test hook: 1 or 2 = panels of 64 or 128 columns whatever the sizes say, 0 = the launcher decides
 
@@ -1272,6 +1272,14 @@ static long split_chunk_steps(long steps, size_t rows, long longest, size_t n_ca
 // 64 228 -> 190; 18, 22 a row, N = 64, row-major 63 -> 55; 18, 16, N = 128 111 -> 107; 15, 16, N = 256 33.6 -> 31.3; 15, N = 24, 14, 13 and 12 within 1 %.
 // Classes are octaves; two of them where a column-major B has more than two panels (18, 10 a row, N = 256 159.1, with octaves 161.9, with two 157.9; 19, 22 a row, N = 200 513, 513,
 // 517; with two panels or fewer two octaves are 1 to 5 % slower).
+// Not where a row-major B has more than two panels and an eighth to a half of the memory-side cache's 256 MiB; in the order of the block rows -> ordered, us: 17, 16 a row, N = 184 96.0 -> 99.9, N =
+// 256 98.4 -> 103.3; 17, 20, N = 160 79.3 -> 81.3; 18, 16, N = 256 186.4 -> 190.6; smaller and larger ones gain: 16, 20, N = 256 52.2 -> 51.4, 16, 9, N = 184 32.9 -> 31.0; 19, 16, N = 136, fp32 397 -> 380,
+// 19, 10, N = 200 358 -> 337; two panels: 17, 16, N = 128 46.0 -> 43.9.
+static bool orders_tasks(size_t K, size_t n_cap, bool b_row_major)
+{
+    const size_t b = 2 * K * n_cap;
+    return !(b_row_major && n_cap > 128 && b > ((size_t)32 << 20) && b <= ((size_t)128 << 20));
+}
 static void order_tasks(std::vector<int4> &tasks, std::vector<uint32_t> &costs, const std::vector<WorkItem> &items, const std::vector<int32_t> &row_first, int octaves)
 {
     uint64_t total = 0, total_chunks = 0;
@@ -1507,7 +1515,7 @@ hipError_t compact_build(CompactCensus &s, const uint16_t *vals, const int32_t *
         costs.push_back((uint32_t)steps + 2 + (uint32_t)(j - i));
         i = j;
     }
-    p->ordered = !split.empty() && g_force_order != 1;
+    p->ordered = !split.empty() && g_force_order != 1 && (g_force_order == 2 || orders_tasks(K, n_cap, b_row_major));
     if (p->ordered) order_tasks(tasks, costs, items, cc_host, n_cap > 128 && !b_row_major ? 2 : 1);
     std::vector<uint64_t> cost_prefix(costs.size() + 1, 0);
     for (size_t i = 0; i < costs.size(); i++) cost_prefix[i + 1] = cost_prefix[i] + costs[i];
@@ -1556,7 +1564,8 @@ extern "C" void smat_internal_compact_panel(int tq) { smat::g_force_tq = tq; }
 extern "C" void smat_internal_compact_list(int what) { smat::g_force_list = what; }
 // Test hook: 1 = entries go through LDS in blocks of 256 wherever they may, 2 = nowhere, 0 = as the sizes say (the default).
 extern "C" void smat_internal_compact_staged(int what) { smat::g_force_staged = what; }
-// Test hook: 1 = tasks of lists with split rows in the order of their items, 0 = as order_tasks says (the default).
+// Test hooks: 1 = tasks of lists with split rows in the order of their items, 2 = as order_tasks says, 0 = as the sizes say (the default); and the rule (host only).
+extern "C" int smat_internal_compact_orders(size_t K, size_t n_cap, int b_row_major) { return smat::orders_tasks(K, n_cap, b_row_major != 0); }
 extern "C" void smat_internal_compact_order(int what) { smat::g_force_order = what; }
 // Test hook: 1, 2 or 4 = wavefronts of a launch that share a task, where tasks are of one item, 0 = as the sizes say (the default).
 extern "C" void smat_internal_compact_share(int what) { smat::g_force_share = what; }
