@@ -747,6 +747,9 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
                 it = tk.y;
                 return;
             }
+            // Not unrolled: the parts of several wavefronts in registers at once were 30 to 60 more of them for all launches, and panels of 16 and 32 columns ran four to six wavefronts a SIMD
+            // instead of eight and seven (stencil 59 x 32 x 62, N = 8, row-major 9.42 -> 8.05 us, N = 32 11.9 -> 10.8, 64^3, N = 16 21.4 -> 19.8).
+#pragma unroll 1
             for (int v = 1; v < wavefronts; v++)
 #pragma unroll
                 for (int t = 0; t < TQ * T; t++) acc[t / T][t % T] += *reinterpret_cast<const f32x4 *>(lds_of_workgroup + v * OWN + t * 1024 + lane * 16);
@@ -1569,6 +1572,21 @@ extern "C" int smat_internal_compact_orders(size_t K, size_t n_cap, int b_row_ma
 extern "C" void smat_internal_compact_order(int what) { smat::g_force_order = what; }
 // Test hook: 1, 2 or 4 = wavefronts of a launch that share a task, where tasks are of one item, 0 = as the sizes say (the default).
 extern "C" void smat_internal_compact_share(int what) { smat::g_force_share = what; }
+// Test hook: registers of a product from entries, panels of 16, 32, 64 or 128 columns; 0 = not known.
+extern "C" int smat_internal_compact_registers(int width, int c_f32)
+{
+    using namespace smat;
+    const auto of = [](auto kernel) {
+        hipFuncAttributes a = {};
+        return hipFuncGetAttributes(&a, reinterpret_cast<const void *>(kernel)) == hipSuccess ? a.numRegs : 0;
+    };
+    switch (width) {
+    case 16: return c_f32 ? of(spmm_compact_kernel<16, true, false, 2, false, false>) : of(spmm_compact_kernel<16, false, false, 2, false, false>);
+    case 32: return c_f32 ? of(spmm_compact_kernel<32, true, false, 2, false, false>) : of(spmm_compact_kernel<32, false, false, 2, false, false>);
+    case 64: return c_f32 ? of(spmm_compact_kernel<64, true, false, 2, false, false>) : of(spmm_compact_kernel<64, false, false, 2, false, false>);
+    default: return c_f32 ? of(spmm_compact_kernel<128, true, false, 2, false, false>) : of(spmm_compact_kernel<128, false, false, 2, false, false>);
+    }
+}
 // Test hook (host only): the rule for such a list, total tasks x panels.
 extern "C" int smat_internal_compact_share_rule(int by_name, int64_t n_steps, int64_t n_tasks, int64_t total) { return smat::compact_share(by_name != 0, n_steps, n_tasks, total); }
 extern "C" int smat_internal_compact_last_share(void) { return smat::g_last_share.load(); }

@@ -60,3 +60,11 @@ def test_narrow_panels_match_the_oracle(smat, cuda, oracle, hooks, M, K, per_row
         smat.spmm(vals, brp, bci, Bd, C, M, N, K, A.nnzb, plan=plan, c_f32=c_f32, kernel=smat.KERNEL_COMPACT, b_row_major=row_major)
         assert np.array_equal(C.cpu().numpy(), want)
     plan.close()
+
+
+@pytest.mark.parametrize("width,most", [(16, 64), (32, 72), (64, 128), (128, 168)])
+@pytest.mark.parametrize("c_f32", [0, 1])
+def test_registers_leave_room_for_the_wavefronts(smat, cuda, width, most, c_f32):
+    """512 registers a SIMD: eight wavefronts of panels of 16 columns, seven of 32, four of 64 and three of 128."""
+    registers = smat.lib.smat_internal_compact_registers(width, c_f32)
+    assert 0 < registers <= most
