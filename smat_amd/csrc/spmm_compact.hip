@@ -540,7 +540,7 @@ template <int W, bool C_F32, bool C_ACC, int AF, bool STAGED, bool BIG>
 __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const uint16_t *__restrict__ acol, const uint32_t *__restrict__ entries, const int2 *__restrict__ step_range, const int32_t *__restrict__ cols,
     const uint16_t *__restrict__ Bt, void *__restrict__ Cout, float *__restrict__ workspace, const WorkItem *__restrict__ items,
-    const int4 *__restrict__ tasks, int n_tasks, int N, int n_panels, long panel_stride, long row_stride_of_most, long last_row_stride, unsigned xcd_run, bool shared)
+    const int4 *__restrict__ tasks, int n_tasks, int N, int n_panels, long panel_stride, long row_stride_of_most, long last_row_stride, unsigned xcd_run, int tasks_of_workgroup, int share_log2)
 {
     constexpr int TQ = W > 64 ? 2 : 1, PW = W / TQ, T = PW / 16; // a row of PW columns is gathered by PW / 8 lanes, 32 rows by T instructions
     constexpr int A_BYTES = 1024, B_BYTES = 64 * W, I_BYTES = 2048;
@@ -559,27 +559,37 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
     const unsigned slot = blockIdx.x >> 3;
     const unsigned run = __builtin_amdgcn_readfirstlane(slot / xcd_run);
     const long wg = ((long)run * 8 + (blockIdx.x & 7)) * xcd_run + (slot - run * xcd_run);
-    const int wavefronts = blockDim.x >> 6;
-    const long w = shared ? wg : wg * wavefronts + wave;
+    const bool shared = share_log2 > 0; // a task of one workgroup, between 2 or 4 wavefronts; else 1 or 4 tasks, one each
+    const long w = wg * tasks_of_workgroup + (wave & (tasks_of_workgroup - 1));
     if (w >= total) return;
     const int panel = __builtin_amdgcn_readfirstlane((int)(w / n_tasks));
     const int task = __builtin_amdgcn_readfirstlane((int)(w - (long)panel * n_tasks));
+    asm volatile("" ::"s"(items), "s"(step_range), "s"(cols), "s"(Bt)); // here with the arguments above, not one wait after the other below
     const int4 tk = tasks[task]; // first item, items (at most 64), first and last column of the stream
-    if (tk.y == 0) return;       // a place that order_tasks left empty
     int e = tk.z, e_last = tk.w;
     if (shared) { // tasks of one item: this wavefront's steps of it
-        const int steps = ((e_last - e) / 32 + wavefronts - 1) / wavefronts;
+        const int steps = (((e_last - e) >> 5) + (1 << share_log2) - 1) >> share_log2;
         e = min(e + wave * steps * 32, e_last);
         e_last = min(e + steps * 32, e_last);
     }
     const int begin = e;
     // Scalar loads share a counter with the LDS operations below, which would wait for them at every step: the items of
     // the task and the entry ranges of its steps come in through vector loads, one per lane, and are read from the lanes.
-    const WorkItem mine = items[tk.x + (lane < tk.y ? lane : tk.y - 1)];
+    // Both are asked for before one is waited for, which the shortest launches notice (16384^2, 16 a row, N = 16, row-major 4.11 -> 4.00 us, 64 6.99 -> 6.88; stencil 40 x 49 x 32,
+    // N = 16, fp32 5.85 -> 5.73).
+    const WorkItem mine = items[tk.x + min(lane, max(tk.y, 1) - 1)];
+    const int first_step = e >> 5;
+    int range_from = first_step;
+    int2 ranges = {0, 0}; // AF > 0: entries of the step range_from + lane
+    if constexpr (AF > 0) ranges = step_range[range_from + lane];
+    int tasks_items = tk.y;
+    asm volatile("" : "+s"(tasks_items)::"memory"); // the loads above stay above
+    if (tasks_items == 0) return;                   // a place that order_tasks left empty
     int it = 0, item_end, br, dst;
     auto enter = [&] {
         br = __builtin_amdgcn_readlane(mine.block_row, it);
-        item_end = shared ? e_last : __builtin_amdgcn_readlane(mine.end, it);
+        const int own_end = __builtin_amdgcn_readlane(mine.end, it);
+        item_end = shared ? e_last : own_end;
         dst = __builtin_amdgcn_readlane(mine.dst, it);
     };
     enter();
@@ -619,13 +629,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
         int n;                     // the step's entries
         u32x4 L[TQ][T];
     };
-    int2 ranges = {0, 0}; // entries of the step range_from + lane
-    const int first_step = e >> 5;
-    int range_from = first_step;
-    if constexpr (AF > 0) {
-        *reinterpret_cast<u32x4 *>(a_tile + lane * 16) = (u32x4){0u, 0u, 0u, 0u};
-        ranges = step_range[range_from + lane];
-    }
+    if constexpr (AF > 0) *reinterpret_cast<u32x4 *>(a_tile + lane * 16) = (u32x4){0u, 0u, 0u, 0u};
     // The indices of 8 steps are 1 KiB, one load, and go to one half of 2 KiB of LDS, from where each lane takes the four of
     // its octet (an instruction that brings 128 bytes costs the vector memory path as much as one that brings 1 KiB).
     unsigned char *const i_tile = lds + A_BYTES + B_BYTES;
@@ -750,7 +754,7 @@ __global__ __launch_bounds__(256, 2) void spmm_compact_kernel(
             // Not unrolled: the parts of several wavefronts in registers at once were 30 to 60 more of them for all launches, and panels of 16 and 32 columns ran four to six wavefronts a SIMD
             // instead of eight and seven (stencil 59 x 32 x 62, N = 8, row-major 9.42 -> 8.05 us, N = 32 11.9 -> 10.8, 64^3, N = 16 21.4 -> 19.8).
 #pragma unroll 1
-            for (int v = 1; v < wavefronts; v++)
+            for (int v = 1; v < 1 << share_log2; v++)
 #pragma unroll
                 for (int t = 0; t < TQ * T; t++) acc[t / T][t % T] += *reinterpret_cast<const f32x4 *>(lds_of_workgroup + v * OWN + t * 1024 + lane * 16);
         }
@@ -909,7 +913,7 @@ hipError_t launch_compact_as(const CompactArgs &a, hipStream_t st)
     auto launch = [&](auto af, auto staged, auto f32, auto acc, auto wide) {
         hipLaunchKernelGGL((spmm_compact_kernel<W, decltype(f32)::value, decltype(acc)::value, decltype(af)::value, decltype(staged)::value, decltype(wide)::value>),
                            dim3((unsigned)wgs), dim3(64 * waves), (size_t)(waves * compact_lds_bytes(W, decltype(staged)::value)), st, p.d_acol, p.d_entries, p.d_step_range, cols, a.Bt, a.C, p.d_workspace,
-                           p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, last_row_stride, (unsigned)xcd_run, share > 1);
+                           p.d_items, p.d_tasks, p.n_tasks, (int)a.N, n_panels, panel_stride, row_stride, last_row_stride, (unsigned)xcd_run, share > 1 ? 1 : waves, share == 4 ? 2 : share - 1);
     };
     using std::false_type;
     using std::true_type;
