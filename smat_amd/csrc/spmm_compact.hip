@@ -1281,11 +1281,13 @@ static long split_chunk_steps(long steps, size_t rows, long longest, size_t n_ca
 // 517; with two panels or fewer two octaves are 1 to 5 % slower).
 // Not where a row-major B has more than two panels and an eighth to a half of the memory-side cache's 256 MiB; in the order of the block rows -> ordered, us: 17, 16 a row, N = 184 96.0 -> 99.9, N =
 // 256 98.4 -> 103.3; 17, 20, N = 160 79.3 -> 81.3; 18, 16, N = 256 186.4 -> 190.6; smaller and larger ones gain: 16, 20, N = 256 52.2 -> 51.4, 16, 9, N = 184 32.9 -> 31.0; 19, 16, N = 136, fp32 397 -> 380,
-// 19, 10, N = 200 358 -> 337; two panels: 17, 16, N = 128 46.0 -> 43.9.
+// 19, 10, N = 200 358 -> 337; two panels: 17, 16, N = 128 46.0 -> 43.9.  Nor where one panel of it is less than an L2's 4 MiB, which all XCDs hold whole: 15, 17 a row, N = 16 10.0 -> 11.1, N = 32 11.7 -> 12.3;
+// 16, 20, N = 8 13.8 -> 14.3; 42 such products 1.6 % in the mean (14, 20, N = 32 9.6 -> 9.3); from 4 MiB on 18, 12, N = 8 25.1 -> 23.7; several panels 12, 16, N = 256 9.9 -> 9.2.
 static bool orders_tasks(size_t K, size_t n_cap, bool b_row_major)
 {
     const size_t b = 2 * K * n_cap;
-    return !(b_row_major && n_cap > 128 && b > ((size_t)32 << 20) && b <= ((size_t)128 << 20));
+    if (!b_row_major) return true;
+    return n_cap <= 64 ? b >= ((size_t)4 << 20) : n_cap <= 128 || b <= ((size_t)32 << 20) || b > ((size_t)128 << 20);
 }
 static void order_tasks(std::vector<int4> &tasks, std::vector<uint32_t> &costs, const std::vector<WorkItem> &items, const std::vector<int32_t> &row_first, int octaves)
 {
