@@ -1274,8 +1274,8 @@ static long split_chunk_steps(long steps, size_t rows, long longest, size_t n_ca
 //   * whole rows come by classes of length, the longest first: what runs at the same time advances through B at about the same pace.  256 tasks of a class,
 //     or what is a 256th of the launch, go to the XCD that has least to do so far, which makes the XCDs even where runs of the deal left up to 4 %.  Inside
 //     a class rows keep their order.
-// A model of the caches finds 67 % of what is asked for in them, 55 % in the order before, 61 with exact lengths in runs of 16 tasks, 73 with rows from 1000 columns on cut
-// in eighths too, whose partial tiles would be ten times as many.  In the order of the block rows -> so, us: R-MAT scale 20, 16 a row, N = 128 456 -> 428, row-major 449 -> 377, N =
+// Counted on R-MAT scale 20, N = 128: 58.5 % of the requests to the L2s found, 53.0 in the order before, and 1.85 GB fetched from beyond them, 2.17.  (A model of the gathers alone finds 67 and 55 %, 61
+// with exact lengths in runs of 16 tasks, 73 with rows from 1000 columns on cut in eighths too, whose partial tiles would be ten times as many.)  In the order of the block rows -> so, us: R-MAT scale 20, 16 a row, N = 128 456 -> 428, row-major 449 -> 377, N =
 // 64 228 -> 190; 18, 22 a row, N = 64, row-major 63 -> 55; 18, 16, N = 128 111 -> 107; 15, 16, N = 256 33.6 -> 31.3; 15, N = 24, 14, 13 and 12 within 1 %.
 // Classes are octaves; two of them where a column-major B has more than two panels (18, 10 a row, N = 256 159.1, with octaves 161.9, with two 157.9; 19, 22 a row, N = 200 513, 513,
 // 517; with two panels or fewer two octaves are 1 to 5 % slower).
