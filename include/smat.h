@@ -98,7 +98,8 @@ int smat_plan_cache_clear(void);
                                * 5% of the blocks exist and (M/1024) x (N/64) workgroups fill the 256 CUs, or
                                * once the attached values are mostly full blocks and an estimate finds it
                                * a quarter faster (on groups of 64, 32 or 16 block rows; 0.11 us of host time
-                               * a block for its streams, which a thousand products have to make up for).
+                               * a block for its streams, which a thousand products,
+                               * 1,500 on a row-major B, have to make up for).
                                * It works from the plan's op list, NOT from the row_ptr / col_idx passed at
                                * launch: the plan must have been made from the same block pattern
                                * (smat_plan_check verifies that on request)                                 */

@@ -889,7 +889,7 @@ extern "C" int smat_plan_create(smat_plan **out, const int32_t *row_ptr_host,
 //     239 products that creation leaves to the choice (random blocks 768^2 to 16384^2 at 3 to 36 %, bands; N = 64 to 4096) it
 //     takes 96, all but a band of 8192 rows (8.7 -> 9.1 us) faster than row-wise with fp16 results (by up to 60 %; what the rule
 //     leaves would gain another 1.7 % in the mean), seven up to 10 % slower with fp32 ones, whose stores cost the sweep kernel more;
-//   * a thousand products make up for the building, 0.11 us a block (one core).  The products that it took to do so, as
+//   * a thousand products (1,500 on a row-major B) make up for the building, 0.11 us a block (one core).  The products that it took to do so, as
 //     measured: 109 in the middle, 958 for 2336 x 2192, 20 %, N = 896 (12.9 -> 12.4 us), 1,740 for a band of 16384 rows and 250,
 //     N = 128 (12.4 -> 10.3), and that band of 8192 rows never does.
 // Measured, us, before and after: 8192^2, 10 %, N = 640: 41.7 -> 28.9, N = 1536: 71.4 -> 41.9; 3088 x 4112, 15 %, N = 2000:
@@ -930,8 +930,12 @@ static size_t sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, s
     const double to_col_major = b_row_major ? to_col_major_us(K, N) : 0.0;
     double row_wise = rowwise_estimate_us(M, K, N, nnzb, n_items, lengths, packed, true) + to_col_major;
     if (b_row_major) row_wise = std::min(row_wise, rowwise_row_major_us(M, N, nnzb));
-    // (the estimate on a row-major B in place errs to either side)
-    double best = std::min(row_wise / (b_row_major ? 1.05 : packed ? 1.1 : 1.2), row_wise - 0.11e-3 * (double)nnzb);
+    // On a row-major B in place, whose estimate errs to either side, 1,500 products have to pay.  With a thousand, long bands of few columns, which the
+    // sweep kernel takes 5 to 20 % less time for, went row-wise for what is left of the gain without the pass over B (rows, bandwidth, N, row-wise and sweep,
+    // us: 53232, 172, 40 13.5 and 11.3; 63760, 173, 48 15.3 and 12.8; 12672, 225, 88 11.4 and 9.8).  Of 640 products (bands, random blocks) that moves seven:
+    // five gain, two lose 3 and 4 %; 2,000 move five more: one gains 8 %, one loses 8.
+    const double build = 0.11e-3 * (double)nnzb / (b_row_major ? 1.5 : 1.0);
+    double best = std::min(row_wise / (b_row_major ? 1.05 : packed ? 1.1 : 1.2), row_wise - build);
     size_t group_rows = 0;
     for (size_t rows : {(size_t)SWEEP_G, (size_t)SWEEP_G / 2, (size_t)SWEEP_G / 4}) {
         const size_t n_rg = (mb + rows - 1) / rows;
@@ -955,6 +959,11 @@ extern "C" void smat_internal_sweep_force_light(int what) { g_force_light = what
 extern "C" int smat_internal_sweep_group_rows(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N, int packed)
 {
     return (int)sweep_group_rows(row_ptr, col_idx, M, K, nnzb, N, M / 16, RowLengths::EVEN, packed != 0, false);
+}
+// Test hook (not part of smat.h): the same for plans made for a row-major B.
+extern "C" int smat_internal_sweep_group_rows_row_major(const int32_t *row_ptr, const int32_t *col_idx, size_t M, size_t K, size_t nnzb, size_t N)
+{
+    return (int)sweep_group_rows(row_ptr, col_idx, M, K, nnzb, N, M / 16, RowLengths::EVEN, true, true);
 }
 
 // The streams are built once the values are known to be dense.  The search for a better deal of the rows to the wavefronts

@@ -60,6 +60,29 @@ def test_choice_is_worth_its_building(m, k, n, share, packed, row_wise, t64, t32
     assert times[group] <= 1.15 * min(worth)
 
 
+# rows, bandwidth, n, times of the row-wise kernel on a row-major B in place and of the sweep kernel on row groups of 64, 32, 16,
+# fp16 results, and whether the sweep kernel is taken
+ROW_MAJOR = [
+    (12672, 225, 88, 11.39, 21.43, 13.74, 9.82, True),
+    (20608, 60, 96, 7.97, 13.41, 9.43, 7.57, True),
+    (37520, 233, 40, 12.44, 21.25, 14.14, 11.05, True),
+    (63760, 173, 48, 15.31, 19.11, 13.87, 12.83, True),
+    (57296, 65, 56, 9.70, 14.18, 10.80, 9.86, False),
+    (21936, 44, 88, 9.20, 18.08, 12.63, 9.95, False),
+]
+
+
+@pytest.mark.parametrize("m,bandwidth,n,row_wise,t64,t32,t16,sweep", ROW_MAJOR)
+def test_row_major_choice_pays_for_its_building(m, bandwidth, n, row_wise, t64, t32, t16, sweep):
+    fn = lib.smat_internal_sweep_group_rows_row_major
+    fn.restype, fn.argtypes = C.c_int, [C.c_void_p, C.c_void_p] + [C.c_size_t] * 4
+    rp, ci, K = pattern(m, bandwidth, "band")
+    group = fn(rp.ctypes.data, ci.ctypes.data, m, K, ci.size, n)
+    times = {0: row_wise, 64: t64, 32: t32, 16: t16}
+    assert bool(group) == sweep
+    assert times[group] == min(times.values())
+
+
 @pytest.mark.parametrize("m,k,n,nnzb", [(1024, 512, 4096, 600), (1024, 256, 4096, 300), (64, 1024, 4096, 1), (8192, 8192, 8, 26000)])
 def test_row_wise_where_the_streams_cannot_help(m, k, n, nnzb):
     rng = np.random.default_rng(2)
